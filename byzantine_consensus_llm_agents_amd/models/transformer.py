@@ -435,7 +435,8 @@ class DecoderModel:
             down     : residual <- residual + h Wd^T          (+ plain RMSNorm of the next layer)
 
         so the residual stream never takes a separate add pass and the [T, 2I]
-        gate_up activation is never written to HBM.
+        gate_up activation is never written to HBM.  Steps of a few rows take the norms
+        into the GEMMs that read them (``norm_linear`` / ``norm_linear_silu``).
         """
         ops, c = self.ops, self.cfg
         residual = None
@@ -443,15 +444,13 @@ class DecoderModel:
         for li, L in enumerate(self.layers):
             if li == 0:  # embedding gather fused with the first input norm
                 h, residual = ops.embed_rmsnorm(tokens, self.embed, L["ln1"], c.rms_eps)
+                qkv = ops.linear(h, L["qkv"], L.get("qkv_bias"))
             else:
-                h = ops.rmsnorm(residual, L["ln1"], c.rms_eps)
-            qkv = ops.linear(h, L["qkv"], L.get("qkv_bias"))
+                qkv = ops.norm_linear(residual, L["ln1"], c.rms_eps, L["qkv"], L.get("qkv_bias"))
             attn = self._attention(li, L, qkv, meta, k_cache, v_cache)
             if li == last and meta.logits_idx is not None:  # see _last_layer_rows
                 attn, residual = self._last_layer_rows(meta, attn, residual)
             residual = ops.linear_residual(attn, L["o"], residual)
-            h = ops.rmsnorm(residual, L["ln2"], c.rms_eps)
-            act = ops.linear_silu(h, L["gate_up"])
+            act = ops.norm_linear_silu(residual, L["ln2"], c.rms_eps, L["gate_up"])
             residual = ops.linear_residual(act, L["down"], residual)
-        h = ops.rmsnorm(residual, self.final_norm, c.rms_eps)
-        return ops.linear(h, self.lm_head)
+        return ops.norm_linear(residual, self.final_norm, c.rms_eps, self.lm_head)

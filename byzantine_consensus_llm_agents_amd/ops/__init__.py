@@ -83,6 +83,8 @@ def _torch_ops() -> SimpleNamespace:
         prefill_tile_rows=lambda hd, kv_fp8=False, max_blocks=0: 64,
         silu_mul=_ref.silu_mul,
         linear_silu=_ref.linear_silu,
+        norm_linear=_ref.norm_linear,
+        norm_linear_silu=_ref.norm_linear_silu,
         linear_residual=_ref.linear_residual,
         sample_step=_ref.sample_step,
         quant_fp8=_ref.quant_fp8,

@@ -20,6 +20,8 @@ _LIB = None
 PREFILL_TILE_ROWS = 128
 PREFILL32_MAX_BLOCKS = 1024  # csrc/kernels/attention.hip: the 32x32 kernel's LDS block-id table
 
+SKINNY_ROWS, SKINNY_MAX_K = 16, 12288  # csrc/kernels/gemm_skinny.hip
+
 c_int, c_float, c_void_p, c_uint32, c_int64 = ctypes.c_int, ctypes.c_float, ctypes.c_void_p, ctypes.c_uint32, ctypes.c_int64
 
 
@@ -90,6 +92,8 @@ def load_library(path: str = None) -> ctypes.CDLL:
                         c_int, c_int, c_int, c_int, c_int, c_void_p],
         "bcg_gemm_nt_fp8": [c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                             c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
+        "bcg_gemm_skinny": [c_int, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
+                            c_void_p],
         "bcg_gemm_tile": [c_int, ctypes.POINTER(c_int), ctypes.POINTER(c_int)],
         "bcg_gemm_num_cfgs": [],
         "bcg_embed_scale_rmsnorm": [c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_float, c_float, c_void_p, c_void_p,
@@ -364,10 +368,36 @@ def hip_ops() -> SimpleNamespace:
             key = (M, N, K, epi, dtype, "lib" if choice is None else f"{choice[0]}x{choice[1]}")
             dispatch_log.calls[key] = dispatch_log.calls.get(key, 0) + 1
 
-    def linear(x, w, bias=None, _epi_log=0):
-        """y = x W^T (+b): hand MFMA GEMM where the plan says it beats hipBLASLt, hipBLASLt otherwise."""
+    def _skinny(x, w, epi):
+        """Whether the few-row kernel takes x W^T: every shape of up to SKINNY_ROWS rows whose rows are whole 128-byte
+        lines (csrc/kernels/gemm_skinny.hip holds both sides' times); table and library keep the others."""
         M, K = x.shape
         N = w.shape[0]
+        return (plan.mode == "1" and 1 <= M <= SKINNY_ROWS and x.dtype == w.dtype == torch.bfloat16 and w.dim() == 2
+                and w.shape[1] == K and K % 64 == 0 and 64 <= K <= SKINNY_MAX_K and N >= 8 and N % (8 if epi == 1 else 4) == 0
+                and x.is_contiguous() and w.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+
+    def _gemm_skinny(x, w, epi=0, bias=None, residual=None, norm_w=None, eps=0.0):
+        M, K = x.shape
+        N = w.shape[0]
+        _log(M, N, K, epi, ("skinny", 1))
+        out = residual if epi == 2 else torch.empty(M, N // 2 if epi == 1 else N, dtype=x.dtype, device=x.device)
+        _check(lib.bcg_gemm_skinny(epi, _p(x), _p(w), None if norm_w is None else _p(norm_w), eps,
+                                   None if bias is None else _p(bias), None if residual is None else _p(residual), _p(out),
+                                   M, N, K, _stream()), "gemm_skinny")
+        return out
+
+    def _few_row_bias(bias, N):
+        return bias is None or (bias.dtype == torch.bfloat16 and bias.shape == (N,) and bias.is_contiguous()
+                                and bias.data_ptr() % 8 == 0)
+
+    def linear(x, w, bias=None, _epi_log=0):
+        """y = x W^T (+b): the few-row kernel, the hand MFMA GEMM where the plan says it beats hipBLASLt, hipBLASLt
+        otherwise."""
+        M, K = x.shape
+        N = w.shape[0]
+        if _skinny(x, w, 0) and _few_row_bias(bias, N):
+            return _gemm_skinny(x, w, 0, bias)
         cfg = None
         if x.is_contiguous() and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16:
             cfg = plan.choose(M, N, K, 0)
@@ -466,11 +496,29 @@ def hip_ops() -> SimpleNamespace:
     def linear_silu(x, w):
         """silu(x Wg^T) * (x Wu^T), W = [gate; up] -- K-ACT fused into the gate_up GEMM."""
         M, K = x.shape
+        if _skinny(x, w, 1):
+            return _gemm_skinny(x, w, 1)
         cfg = plan.choose(M, w.shape[0], K, 1) if x.is_contiguous() and x.dtype == torch.bfloat16 else None
         if cfg is None:
             return silu_mul(linear(x, w, _epi_log=1))
         _log(M, w.shape[0], K, 1, cfg)
         return gemm_nt(x, w, cfg, 1)
+
+    def _norm_fusable(x, w_norm):
+        return (x.shape[1] <= 8192 and w_norm.shape == (x.shape[1],) and w_norm.dtype == torch.bfloat16 and w_norm.is_contiguous()
+                and w_norm.data_ptr() % 16 == 0)
+
+    def norm_linear(x, w_norm, eps, w, bias=None):
+        """linear(rmsnorm(x, w_norm, eps), w, bias), one kernel for a few rows."""
+        if x.dim() == 2 and _skinny(x, w, 0) and _norm_fusable(x, w_norm) and _few_row_bias(bias, w.shape[0]):
+            return _gemm_skinny(x, w, 0, bias, norm_w=w_norm, eps=eps)
+        return linear(rmsnorm(x, w_norm, eps), w, bias)
+
+    def norm_linear_silu(x, w_norm, eps, w):
+        """linear_silu(rmsnorm(x, w_norm, eps), w), one kernel for a few rows."""
+        if x.dim() == 2 and _skinny(x, w, 1) and _norm_fusable(x, w_norm):
+            return _gemm_skinny(x, w, 1, norm_w=w_norm, eps=eps)
+        return linear_silu(rmsnorm(x, w_norm, eps), w)
 
     residual_addmm = os.environ.get("BCG_RESIDUAL_ADDMM", "1") == "1"
 
@@ -478,6 +526,9 @@ def hip_ops() -> SimpleNamespace:
         """residual <- residual + x W^T (in place; the o/down projection fused with the
         residual-stream update of the next add+RMSNorm).  Returns `residual`."""
         M, K = x.shape
+        if (_skinny(x, w, 2) and residual.shape == (M, w.shape[0]) and residual.dtype == torch.bfloat16
+                and residual.is_contiguous() and residual.data_ptr() % 8 == 0):
+            return _gemm_skinny(x, w, 2, residual=residual)
         cfg = plan.choose(M, w.shape[0], K, 2) if x.is_contiguous() and x.dtype == torch.bfloat16 else None
         _log(M, w.shape[0], K, 2, cfg)
         if cfg is None:
@@ -643,7 +694,7 @@ def hip_ops() -> SimpleNamespace:
     extra.update(seqhyper_ops(lib))
 
     return SimpleNamespace(name="hip", **extra, rmsnorm_fp8=rmsnorm_fp8, embed_rmsnorm_fp8=embed_rmsnorm_fp8,
-                           linear_fp8_residual=linear_fp8_residual, linear=linear, linear_silu=linear_silu, linear_residual=linear_residual,
+                           linear_fp8_residual=linear_fp8_residual, linear=linear, norm_linear=norm_linear, norm_linear_silu=norm_linear_silu, linear_silu=linear_silu, linear_residual=linear_residual,
                            gemm_nt=gemm_nt, gemm_plan=plan, prepare_device=prepare_device,
                            register_stream=register_stream, quant_fp8=quant_fp8, add_rmsnorm_fp8=add_rmsnorm_fp8,
                            silu_mul_fp8=silu_mul_fp8, linear_fp8=linear_fp8, gemm_nt_fp8=gemm_nt_fp8, fp8_cfg=fp8_cfg, rmsnorm=rmsnorm, add_rmsnorm=add_rmsnorm, silu_mul=silu_mul,

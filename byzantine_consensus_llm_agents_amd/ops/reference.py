@@ -187,6 +187,16 @@ def linear_silu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return (torch.nn.functional.silu(gu[:, :inter]) * gu[:, inter:]).to(x.dtype)
 
 
+def norm_linear(x, w_norm, eps, w, bias=None):
+    """linear(rmsnorm(x, w_norm, eps), w, bias)."""
+    return torch.nn.functional.linear(rmsnorm(x, w_norm, eps), w, bias)
+
+
+def norm_linear_silu(x, w_norm, eps, w):
+    """linear_silu(rmsnorm(x, w_norm, eps), w)."""
+    return linear_silu(rmsnorm(x, w_norm, eps), w)
+
+
 def linear_residual(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor) -> torch.Tensor:
     """residual <- residual + x W^T, rounded once (the fused o/down GEMM epilogue); in place."""
     residual.copy_((residual.float() + x.float() @ w.float().t()).to(residual.dtype))
