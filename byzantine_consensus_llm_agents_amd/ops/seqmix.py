@@ -40,6 +40,9 @@ def _act(t):
 ACT_CODES = {"gelu_tanh": 0, "relu2": 1, "silu": 2, "clamped_glu": 3}
 EXPERT_ACTS = {"silu_gated": "silu", "clamped_glu": "clamped_glu"}   # gated experts -> activation of their hidden values
 
+WIDE_ROWS = 256    # rows of a position tile of the 256 x 256 expert products
+WIDE_SLOTS = 64    # ... taken from this many routed rows per expert on (see `_wide_experts`)
+
 
 def seqmix_ops(lib, linear):
     split_keys = lib.bcg_multimap_split_keys()
@@ -257,6 +260,18 @@ def seqmix_ops(lib, linear):
             return torch.cat([gate, up])
         return torch.stack([gate.reshape(ff // 16, 16, W), up.reshape(ff // 16, 16, W)], 1).reshape(2 * ff, W)
 
+    def _wide_experts(n_slots, E, W, ff, kind, h, up, down):
+        """Whether the products run on position tiles of 256 rows: from WIDE_SLOTS routed rows per expert on.  Two gated
+        products of 8 experts, top 2, 64-row tiles -> 256-row tiles, us: width 2048, ff 2048: 32 rows per expert 93 -> 112,
+        64: 115 -> 112, 256: 211 -> 133, 2046: 836 -> 509; width 4096, ff 3072: 32: 186 -> 197, 64: 297 -> 208, 256: 629 ->
+        306, 2046: 2274 -> 1210 (1.02 PFLOP/s of 0.54)."""
+        if h.dtype != torch.bfloat16 or W % 64 or ff % 64 or (kind in EXPERT_ACTS and ff % 128) or n_slots < WIDE_SLOTS * E:
+            return False
+        rows = n_slots + E * (WIDE_ROWS - 1) + 2 * WIDE_ROWS    # (with a tile to spare: the kernel's offsets are 32-bit)
+        n_up = up.shape[1]
+        return (2 * rows * max(W, n_up) < 1 << 31 and 2 * (max(W, n_up) + 256) * max(W, ff) < 1 << 31
+                and all(t.data_ptr() % 16 == 0 for t in (h, up, down)))
+
     def moe_experts(h, up, down, idx, weights, kind="relu2", limit=0.0):
         T, W = h.shape
         E, n_up, _ = up.shape
@@ -271,12 +286,31 @@ def seqmix_ops(lib, linear):
         _req(idx.dtype == torch.int32 and idx.shape == (T, top) and idx.is_contiguous() and weights.dtype == torch.float32
              and weights.shape == (T, top) and weights.is_contiguous(), "routing tables [T, top]")
         n_slots = T * top
-        n_tiles = (n_slots + E * (tile_rows - 1) + tile_rows - 1) // tile_rows
-        cap = n_tiles * tile_rows
         dev, f32 = h.device, _act(h)
+        wide = _wide_experts(n_slots, E, W, ff, kind, h, up, down)
+        rows = WIDE_ROWS if wide else tile_rows
+        n_tiles = (n_slots + E * (rows - 1) + rows - 1) // rows
+        cap = n_tiles * rows
         sorted_ = torch.empty(cap, dtype=torch.int32, device=dev)
         tile_e = torch.empty(n_tiles, dtype=torch.int32, device=dev)
-        _check(lib.bcg_moe_align(_p(idx), n_slots, E, _p(sorted_), cap, _p(tile_e), n_tiles, _stream()), "moe_align")
+        out = torch.empty(T, W, dtype=torch.float32, device=dev)
+        if wide:
+            place = torch.empty(n_slots + 1, dtype=torch.int32, device=dev)   # every slot's position; the tiles in use
+            pos, used = place[:n_slots], place[n_slots:]
+            _check(lib.bcg_moe_align(_p(idx), n_slots, E, _p(sorted_), cap, _p(tile_e), n_tiles, rows, _p(pos), _p(used),
+                                     _stream()), "moe_align")
+            a = torch.empty(cap, W, dtype=h.dtype, device=dev)
+            _check(lib.bcg_moe_gather(_p(h), _p(sorted_), _p(a), cap, 2 * W, top, _stream()), "moe_gather")
+            hidden = torch.empty(cap, ff, dtype=h.dtype, device=dev)
+            _check(lib.bcg_gemm_w4_grouped(3 if gated else 4, _p(a), _p(up), _p(hidden), _p(tile_e), _p(used), n_tiles, n_up, W,
+                                           limit if kind == "clamped_glu" else 0.0, _stream()), "moe gate / up")
+            y = a   # the down product's rows replace the gathered ones
+            _check(lib.bcg_gemm_w4_grouped(0, _p(hidden), _p(down), _p(y), _p(tile_e), _p(used), n_tiles, W, ff, 0.0, _stream()),
+                   "moe down")
+            _check(lib.bcg_moe_combine(_p(y), _p(weights), _p(pos), _p(out), T, W, top, f32, _stream()), "moe_combine")
+            return out
+        _check(lib.bcg_moe_align(_p(idx), n_slots, E, _p(sorted_), cap, _p(tile_e), n_tiles, rows, None, None, _stream()),
+               "moe_align")
         code = ACT_CODES[EXPERT_ACTS[kind]] if gated else 1
         if gated and ff % 16 == 0:   # rows paired by `moe_pair_rows`: the hidden values in the product's epilogue
             hidden = torch.empty(cap, ff, dtype=h.dtype, device=dev)
@@ -295,8 +329,7 @@ def seqmix_ops(lib, linear):
         y = torch.empty(n_slots, W, dtype=h.dtype, device=dev)
         _check(lib.bcg_moe_gemm(_p(hidden), ff, _p(down), _p(y), W, _p(sorted_), _p(tile_e), n_tiles, W, ff, top, 0, 1, 0,
                                 0.0, f32, _stream()), "moe down")
-        out = torch.empty(T, W, dtype=torch.float32, device=dev)
-        _check(lib.bcg_moe_combine(_p(y), _p(weights), _p(out), T, W, top, f32, _stream()), "moe_combine")
+        _check(lib.bcg_moe_combine(_p(y), _p(weights), None, _p(out), T, W, top, f32, _stream()), "moe_combine")
         return out
 
     return dict(embed_scale_rmsnorm=embed_scale_rmsnorm, embed_position=embed_position, residual_add_rmsnorm32=residual_add_rmsnorm32,

@@ -84,7 +84,8 @@ namespace {
 constexpr int BM = 256, BN = 256, BK = 64;
 constexpr int W4_COUNTERS = 65536;  // the caller's arrival-counter array (one per tile)
 constexpr int A_BYTES = BM * 128;  // one operand's K-tile: 256 rows of 128 B
-enum Epilogue { EPI_STORE = 0, EPI_SILU_MUL = 1, EPI_RESIDUAL = 2 };
+// EPI_GATED: W's rows alternate 16 gate and 16 up rows as they lie in memory (bcg_gemm_w4_grouped)
+enum Epilogue { EPI_STORE = 0, EPI_SILU_MUL = 1, EPI_RESIDUAL = 2, EPI_GATED = 3, EPI_RELU2 = 4 };
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -152,13 +153,22 @@ __device__ uint64_t w4_stamps[1 << 17];
 
 // F8: e4m3 operands with v_mfma_scale_f32_32x32x64_f8f6f4 (unit E8M0 block scales; x_scale[m] *
 // w_scale[n] applied in the epilogue)
-template <int EPI, bool F8 = false>
+// GROUPED: rows 256 t .. of X meet the weight group[t] of a stack [groups, N, K]; only the first used[0] tiles of
+// 256 rows hold work (the row counts of the groups are known on the device only)
+template <int EPI, bool F8 = false, bool GROUPED = false>
 __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_w4_kernel(
     const void* __restrict__ Xv, const void* __restrict__ Wv, const bf16_t* __restrict__ bias,
     const bf16_t* __restrict__ residual, bf16_t* __restrict__ C, float* __restrict__ ws,
     int* __restrict__ counters, int M, int N, int K, int ldc, int inter, int m_tiles, int n_tiles,
-    int split_k, const float* __restrict__ x_scale, const float* __restrict__ w_scale) {
-  static_assert(!F8 || EPI != EPI_SILU_MUL, "fp8: store / residual epilogues");
+    int split_k, const float* __restrict__ x_scale, const float* __restrict__ w_scale,
+    const int* __restrict__ group, const int* __restrict__ used, float limit) {
+  static_assert(!F8 || EPI == EPI_STORE || EPI == EPI_RESIDUAL, "fp8: store / residual epilogues");
+  static_assert(GROUPED || (EPI != EPI_GATED && EPI != EPI_RELU2), "grouped epilogues");
+  if constexpr (GROUPED) {
+    m_tiles = min(m_tiles, used[0]);
+    split_k = 1;
+    if (static_cast<int>(blockIdx.x) >= m_tiles * n_tiles) return;
+  }
   constexpr bool L32 = F8;                             // 32x32 accumulator layout
   constexpr int SLOTS = F8 ? 16 : W4_SLOTS;            // MFMAs per phase
   constexpr int ESZ = F8 ? 1 : 2;                      // bytes per element
@@ -250,7 +260,8 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
   auto item_srd = [&](const Geo& g, i32x4& sX, i32x4& sW) {
     const int wr0 = EPI == EPI_SILU_MUL ? (g.n0 >> 1) : g.n0;
     sX = make_srd(X + static_cast<size_t>(g.m0) * row_bytes, static_cast<uint32_t>(M - g.m0) * row_bytes);
-    sW = make_srd(W + static_cast<size_t>(wr0) * row_bytes, static_cast<uint32_t>(w_rows - wr0) * row_bytes);
+    const size_t w_first = (GROUPED ? static_cast<size_t>(group[g.m0 / BM]) * N : 0) + wr0;
+    sW = make_srd(W + w_first * row_bytes, static_cast<uint32_t>(w_rows - wr0) * row_bytes);
   };
   const uint32_t voffX = static_cast<uint32_t>(prow) * row_bytes + pch;
   // SILU: 16-row blocks of the tile alternate gate / up of the same 16 features, so stage row
@@ -405,7 +416,7 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
       // offset (m-block j's rows included) rides in the VGPR: only that part is range-checked (an
       // SGPR offset is added after the check), and the host bounds (M + 256) * ldc * 2 below
       // 2^31 so a masked column's 0x80000000 + offset never wraps into range.
-      constexpr bool SILU = EPI == EPI_SILU_MUL;
+      constexpr bool SILU = EPI == EPI_SILU_MUL || EPI == EPI_GATED;
       constexpr int NP = SILU ? NB / 4 : NB / 2;  // 8-column groups per m-block per lane
       constexpr int JG = 1;                       // m-blocks per residual batch
       const uint32_t ldb = static_cast<uint32_t>(ldc) * 2;
@@ -447,8 +458,16 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
 #pragma unroll
             for (int k = 0; k < 2; ++k) {
               const auto g = value(4 * p + 2 * k, j), u = value(4 * p + 2 * k + 1, j);
+              if (EPI == EPI_GATED && limit > 0.f) {  // clamped unit: min(g, limit), u within +-limit
 #pragma unroll
-              for (int e = 0; e < 4; ++e) h[k][e] = silu(g[e]) * u[e];
+                for (int e = 0; e < 4; ++e) {
+                  const float gc = fminf(g[e], limit), uc = fminf(fmaxf(u[e], -limit), limit);
+                  h[k][e] = gc * __builtin_amdgcn_rcpf(1.f + __expf(-1.702f * gc)) * (uc + 1.f);
+                }
+              } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) h[k][e] = silu(g[e]) * u[e];
+              }
             }
             float o[8];
             swap8(h[0], h[1], o);
@@ -499,6 +518,10 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
                 swap8(fa, fb, o);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
+                  if constexpr (EPI == EPI_RELU2) {
+                    const float v = fmaxf(o[e], 0.f);
+                    o[e] = v * v;
+                  }
                   if constexpr (HB) {
                     const uint32_t w = bq[p][e >> 1];
                     o[e] += __uint_as_float((e & 1) ? (w & 0xffff0000u) : (w << 16));
@@ -1030,7 +1053,20 @@ int launch_w4(const void* x, const void* w, const void* bias, const void* res, v
                    : W4_PERSIST && split_k == 1 ? std::min(nwg, w4_cus()) : nwg;
   hipLaunchKernelGGL((gemm_w4_kernel<EPI, F8>), dim3(grid), dim3(256),
                      0, stream, x, w, static_cast<const bf16_t*>(bias), static_cast<const bf16_t*>(res),
-                     static_cast<bf16_t*>(c), ws, cnt, M, N, K, ldc, inter, m_tiles, n_tiles, split_k, xs, wsc);
+                     static_cast<bf16_t*>(c), ws, cnt, M, N, K, ldc, inter, m_tiles, n_tiles, split_k, xs, wsc,
+                     static_cast<const int*>(nullptr), static_cast<const int*>(nullptr), 0.f);
+  return BCG_CHECK_LAUNCH();
+}
+
+template <int EPI>
+int launch_w4_grouped(const void* x, const void* w, void* c, const int* group, const int* used, int m_tiles, int N, int K,
+                      float limit, hipStream_t stream) {
+  const int n_tiles = (N + BN - 1) / BN, inter = N / 2, ldc = EPI == EPI_GATED ? inter : N;
+  const int grid = static_cast<int>(std::min<long long>(1ll * m_tiles * n_tiles, w4_cus()));
+  hipLaunchKernelGGL((gemm_w4_kernel<EPI, false, true>), dim3(grid), dim3(256), 0, stream, x, w, static_cast<const bf16_t*>(nullptr),
+                     static_cast<const bf16_t*>(nullptr), static_cast<bf16_t*>(c), static_cast<float*>(nullptr),
+                     static_cast<int*>(nullptr), m_tiles * BM, N, K, ldc, inter, m_tiles, n_tiles, 1,
+                     static_cast<const float*>(nullptr), static_cast<const float*>(nullptr), group, used, limit);
   return BCG_CHECK_LAUNCH();
 }
 
@@ -1075,6 +1111,25 @@ BCG_API int bcg_gemm_w4(int epi, const void* x, const void* w, const void* bias,
     case EPI_RESIDUAL:
       if (!residual) return -2;
       return launch_w4<EPI_RESIDUAL>(x, w, bias, residual, c, wsf, cnt, M, N, K, inter, split_k, stream);
+    default: return -2;
+  }
+}
+
+// Grouped product (experts): rows 256 t .. 256 t + 255 of x [256 m_tiles, K] times w[group[t]] [N, K], for the first
+// used[0] <= m_tiles row tiles; c rows past them stay as they are.  epi: 0 = store, 3 = gated unit of rows that
+// alternate 16 gate / 16 up (c [*, N / 2]; limit > 0: the clamped unit, else silu(gate) * up), 4 = relu squared.  group
+// and used are read on the device.  K % 64 == 0; N % 16 == 0, epi 3: N % 256 == 0.
+BCG_API int bcg_gemm_w4_grouped(int epi, const void* x, const void* w, void* c, const int* group, const int* used, int m_tiles,
+                                int N, int K, float limit, hipStream_t stream) {
+  if (m_tiles <= 0 || N <= 0 || N % 16 || K % BK || K <= 0 || m_tiles > (1 << 20)) return -2;
+  const unsigned long long M = 1ull * m_tiles * BM;
+  if (2 * (M + BM) * K >= (1ull << 31) || 2ull * (N + BN) * K >= (1ull << 31) || 2 * (M + BM) * N >= (1ull << 31)) return -2;
+  switch (epi) {
+    case EPI_STORE: return launch_w4_grouped<EPI_STORE>(x, w, c, group, used, m_tiles, N, K, 0.f, stream);
+    case EPI_GATED:
+      if (N % 256) return -2;
+      return launch_w4_grouped<EPI_GATED>(x, w, c, group, used, m_tiles, N, K, limit, stream);
+    case EPI_RELU2: return launch_w4_grouped<EPI_RELU2>(x, w, c, group, used, m_tiles, N, K, 0.f, stream);
     default: return -2;
   }
 }

@@ -10,7 +10,10 @@
 //             rows and applies the activation, "down" scatters rows back to their slots
 //   combine : out32[t] = sum_j weight[t, j] * y[slot(t, j)]   (fp32, fixed order)
 //
-// Position tiles are TM rows; a tile belongs to one expert (tile_expert, -1 = unused).
+// Position tiles are TM rows; a tile belongs to one expert (tile_expert, -1 = unused).  Steps with many slots per
+// expert (`moe_experts` in ops/seqmix.py has the rule) take position tiles of 256 rows instead: `gather` copies the
+// token rows into position order, the products run on the 256 x 256 kernel of the dense projections
+// (bcg_gemm_w4_grouped) and `combine` reads the rows where they are.
 #include <algorithm>
 
 #include "seqmix_common.h"
@@ -103,7 +106,7 @@ __global__ __launch_bounds__(256) void route_kernel(const T* __restrict__ h, con
 
 __global__ __launch_bounds__(1024) void align_kernel(const int* __restrict__ idx, int n_slots, int E,
                                                      int* __restrict__ sorted, int cap, int* __restrict__ tile_expert,
-                                                     int n_tiles) {
+                                                     int n_tiles, int tm, int* __restrict__ pos, int* __restrict__ used) {
   __shared__ int cnt[MAX_E], off[MAX_E + 1];
   for (int e = threadIdx.x; e < E; e += blockDim.x) cnt[e] = 0;
   __syncthreads();
@@ -115,21 +118,39 @@ __global__ __launch_bounds__(1024) void align_kernel(const int* __restrict__ idx
   __syncthreads();
   if (threadIdx.x == 0) {
     off[0] = 0;
-    for (int e = 0; e < E; ++e) off[e + 1] = off[e] + (cnt[e] + TM - 1) / TM * TM;
+    for (int e = 0; e < E; ++e) off[e + 1] = off[e] + (cnt[e] + tm - 1) / tm * tm;
+    if (used != nullptr) *used = off[E] / tm;
   }
   __syncthreads();
   for (int t = threadIdx.x; t < n_tiles; t += blockDim.x) {
     int who = -1;
     for (int e = 0; e < E; ++e)
-      if (t * TM >= off[e] && t * TM < off[e + 1]) who = e;
+      if (t * tm >= off[e] && t * tm < off[e + 1]) who = e;
     tile_expert[t] = who;
   }
   for (int e = threadIdx.x; e < E; e += blockDim.x) cnt[e] = 0;
   __syncthreads();
   for (int i = threadIdx.x; i < n_slots; i += blockDim.x) {
     const int e = idx[i];
-    if (e >= 0 && e < E) sorted[off[e] + atomicAdd(&cnt[e], 1)] = i;
+    if (e >= 0 && e < E) {
+      const int p = off[e] + atomicAdd(&cnt[e], 1);
+      sorted[p] = i;
+      if (pos != nullptr) pos[i] = p;
+    } else if (pos != nullptr) {
+      pos[i] = -1;
+    }
   }
+}
+
+// Rows of the positions, for the 256-row products: out[p] = a[sorted[p] / top].  Padding positions stay as they
+// are: nothing reads what the products make of them.
+__global__ __launch_bounds__(256) void gather_rows_kernel(const uint4* __restrict__ a, const int* __restrict__ sorted,
+                                                          uint4* __restrict__ out, int row_vecs, int top) {
+  const int slot = sorted[blockIdx.x];
+  if (slot < 0) return;
+  const uint4* src = a + static_cast<size_t>(slot / top) * row_vecs;
+  uint4* dst = out + static_cast<size_t>(blockIdx.x) * row_vecs;
+  for (int i = threadIdx.x; i < row_vecs; i += 256) dst[i] = src[i];
 }
 
 // Hidden value of a gated expert from its two products (rounded to T like a projection's output):
@@ -438,14 +459,27 @@ __global__ __launch_bounds__(256) void moe_gemm_lds_narrow_kernel(const T* __res
     }
 }
 
-template <typename T>
+// out32[t] = sum_j weight[t, j] * y[row(t, j)], j in order; row: the slot, or its position where y is in position
+// order (an unplaced slot adds nothing).  VEC columns per thread: 16-byte loads of the rows, bound by memory.
+template <typename T, int VEC>
 __global__ __launch_bounds__(256) void combine_kernel(const T* __restrict__ y, const float* __restrict__ wts,
-                                                      float* __restrict__ out, int W, int top) {
+                                                      const int* __restrict__ pos, float* __restrict__ out, int W, int top) {
+  typedef T Row __attribute__((ext_vector_type(VEC)));
+  typedef float Sum __attribute__((ext_vector_type(VEC)));
   const int t = blockIdx.x;
-  for (int c = threadIdx.x; c < W; c += 256) {
-    float s = 0.f;
-    for (int j = 0; j < top; ++j) s += wts[t * top + j] * Elem<T>::ld(y[(static_cast<size_t>(t) * top + j) * W + c]);
-    out[static_cast<size_t>(t) * W + c] = s;
+  for (int c = VEC * threadIdx.x; c < W; c += 256 * VEC) {
+    Sum s;
+#pragma unroll
+    for (int q = 0; q < VEC; ++q) s[q] = 0.f;
+    for (int j = 0; j < top; ++j) {
+      const int64_t row = pos != nullptr ? pos[t * top + j] : static_cast<int64_t>(t) * top + j;
+      if (row < 0) continue;
+      const float w = wts[t * top + j];
+      const Row v = *reinterpret_cast<const Row*>(y + row * W + c);
+#pragma unroll
+      for (int q = 0; q < VEC; ++q) s[q] += w * Elem<T>::ld(v[q]);
+    }
+    *reinterpret_cast<Sum*>(out + static_cast<size_t>(t) * W + c) = s;
   }
 }
 
@@ -486,14 +520,25 @@ BCG_API int bcg_moe_route(const void* h, const void* rw, const void* rb, const v
   return BCG_CHECK_LAUNCH();
 }
 
-// sorted: [cap] with cap = n_tiles * TM >= n_slots + E (TM - 1); tile_expert: [n_tiles].
-BCG_API int bcg_moe_align(const void* idx, int n_slots, int E, void* sorted, int cap, void* tile_expert, int n_tiles,
-                          void* stream) {
+// Position tiles of `tm` rows.  sorted: [cap] with cap = n_tiles * tm >= n_slots + E (tm - 1); tile_expert: [n_tiles];
+// pos (may be null): [n_slots], every slot's position; used (may be null): [1], the tiles that hold slots.
+BCG_API int bcg_moe_align(const void* idx, int n_slots, int E, void* sorted, int cap, void* tile_expert, int n_tiles, int tm,
+                          void* pos, void* used, void* stream) {
   if (n_slots <= 0) return 0;
-  if (E < 1 || E > MAX_E || cap != n_tiles * TM || cap < n_slots + E * (TM - 1)) return -2;
+  if (E < 1 || E > MAX_E || tm < 1 || cap != n_tiles * tm || cap < n_slots + E * (tm - 1)) return -2;
   align_kernel<<<1, 1024, 0, static_cast<hipStream_t>(stream)>>>(static_cast<const int*>(idx), n_slots, E,
                                                                  static_cast<int*>(sorted), cap,
-                                                                 static_cast<int*>(tile_expert), n_tiles);
+                                                                 static_cast<int*>(tile_expert), n_tiles, tm,
+                                                                 static_cast<int*>(pos), static_cast<int*>(used));
+  return BCG_CHECK_LAUNCH();
+}
+
+// out[p] = a[sorted[p] / top] for the placed positions p < cap; rows of row_bytes (a multiple of 16), 16-byte aligned.
+BCG_API int bcg_moe_gather(const void* a, const void* sorted, void* out, int cap, int row_bytes, int top, void* stream) {
+  if (cap <= 0) return 0;
+  if (row_bytes <= 0 || row_bytes % 16 || top < 1) return -2;
+  gather_rows_kernel<<<cap, 256, 0, static_cast<hipStream_t>(stream)>>>(static_cast<const uint4*>(a), static_cast<const int*>(sorted),
+                                                                      static_cast<uint4*>(out), row_bytes / 16, top);
   return BCG_CHECK_LAUNCH();
 }
 
@@ -543,12 +588,19 @@ BCG_API int bcg_moe_gemm(const void* a, int64_t a_stride, const void* w, void* o
   return BCG_CHECK_LAUNCH();
 }
 
-BCG_API int bcg_moe_combine(const void* y, const void* wts, void* out, int T_, int W, int top, int is_f32, void* stream) {
+BCG_API int bcg_moe_combine(const void* y, const void* wts, const void* pos, void* out, int T_, int W, int top, int is_f32,
+                            void* stream) {
   if (T_ <= 0) return 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (is_f32)
-    combine_kernel<float><<<T_, 256, 0, s>>>(static_cast<const float*>(y), static_cast<const float*>(wts), static_cast<float*>(out), W, top);
-  else
-    combine_kernel<bf16_t><<<T_, 256, 0, s>>>(static_cast<const bf16_t*>(y), static_cast<const float*>(wts), static_cast<float*>(out), W, top);
+  const bool vec = (reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(out)) % 16 == 0;
+#define BCG_COMBINE(TYPE, VEC_)                                                                                          \
+  combine_kernel<TYPE, VEC_><<<T_, 256, 0, s>>>(static_cast<const TYPE*>(y), static_cast<const float*>(wts), \
+                                                static_cast<const int*>(pos), static_cast<float*>(out), W, top)
+  if (is_f32) {
+    if (vec && W % 4 == 0) BCG_COMBINE(float, 4); else BCG_COMBINE(float, 1);
+  } else {
+    if (vec && W % 8 == 0) BCG_COMBINE(bf16_t, 8); else BCG_COMBINE(bf16_t, 1);
+  }
+#undef BCG_COMBINE
   return BCG_CHECK_LAUNCH();
 }
