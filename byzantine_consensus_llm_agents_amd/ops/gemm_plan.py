@@ -15,10 +15,11 @@ simple rule (hand kernel up to ``max_m`` rows).
 
 """
 
+import bisect
 import ctypes
 import json
 import os
-from typing import Dict, Optional, Tuple
+from typing import Dict, List, Optional, Tuple
 
 TABLE = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "engine", "tuned",
                      "hand_gemm.json")
@@ -29,6 +30,9 @@ W4_CFG = 11  # csrc/kernels/gemm_w4.hip: 256 x 256, four 128 x 128 waves (one pe
 BIG_CFGS = (PP_CFG, W4_CFG)  # 256 x 256 tiles (the register-staged form lost its A/B: csrc/experimental/gemm_rs.hip)
 N_CFGS = len(TILES)
 SPLITS = (1, 2, 3, 4, 6, 8)
+CUS = 256
+LARGE_M = 2048    # `pieces`: from here on the row count is a prefill step's
+W4_KTILE_US = 1.46   # one wave of 256 x 256 tiles: microseconds per 64 of K (512 tiles, K = 4096 .. 17408)
 STREAM_K = 0  # split_k value of the W4 kernel's stream-K launch (one workgroup per CU over tiles x K-tiles)
 
 
@@ -37,6 +41,7 @@ class GemmPlan:
         self.mode = os.environ.get("BCG_HAND_GEMM", "1")
         self.force_split = int(os.environ.get("BCG_HAND_GEMM_SPLIT", "1"))  # split-K in "force" mode (tests)
         self.max_m = max_m
+        self.rows: Dict[Tuple[int, int, int], List[int]] = {}
         self.timings: Dict[Tuple[int, int, int, int], Dict[str, float]] = {}
         self.tiles = {}
         for cfg in range(N_CFGS):
@@ -52,6 +57,8 @@ class GemmPlan:
             for key, choice in data.get("choice", {}).items():
                 m, n, k, e = map(int, key.split(","))
                 self.table[(m, n, k, e)] = tuple(choice) if isinstance(choice, list) else (int(choice), 1)
+            for (m, n, k, e) in sorted(self.table):     # measured row counts of every shape, in order
+                self.rows.setdefault((n, k, e), []).append(m)
             for key, times in data.get("timings_us", {}).items():
                 self.timings[tuple(map(int, key.split(",")))] = times
 
@@ -83,12 +90,11 @@ class GemmPlan:
 
     def _lookup(self, M: int, N: int, K: int, epi: int) -> Optional[Tuple[int, int]]:
         """Table choice at M, else at the nearest measured M above (same projection shape)."""
-        choice = self.table.get((M, N, K, epi))
-        if choice is None and self.table:
-            above = [m for (m, n, k, e) in self.table if (n, k, e) == (N, K, epi) and m >= M]
-            if above:
-                choice = self.table[(min(above), N, K, epi)]
-        return choice
+        ms = self.rows.get((N, K, epi))
+        if not ms:
+            return None
+        at = bisect.bisect_left(ms, M)
+        return self.table[(ms[at], N, K, epi)] if at < len(ms) else None
 
     def choose(self, M: int, N: int, K: int, epi: int) -> Optional[Tuple[int, int]]:
         """(tile configuration, split-K) of the hand kernel, or None for the library path."""
@@ -112,6 +118,41 @@ class GemmPlan:
             return None
         cfg = self.default_cfg(M)
         return (cfg, 1) if self.supported(cfg, M, N, K, epi) else None
+
+    def pieces(self, M: int, N: int, K: int, epi: int) -> List[Tuple[int, Optional[Tuple[int, int]]]]:
+        """[(rows, choice)]: how the M rows run, one choice for all of them or two runs of rows.
+
+        A prefill step has any number of rows, the table a few, and 256 x 256 tiles come in rounds of 256 (one per CU):
+        288 tiles cost two rounds.  At row counts that the table does not hold, from LARGE_M on:
+        * a last round that is short goes to the rows it is made of: whole rounds for the first M1 rows, and the
+          rest as a GEMM of its own, where that is estimated below 0.6 of a round (4449 x 4096 x 12288, us: library
+          658, one 256 x 256 launch 470, split here 345; 4449 x 4096 x 4096: 138, 172, 117);
+        * whole rounds, or a last one filled to 0.88, stay on the library, which is 3 to 15 % faster there (8183 x 16384 x
+          2048: 373 us against 440; 16098 x 7168 x 5120 and 16098 x 5120 x 17408: 3 % and 6 %);
+        * otherwise the library is erratic and the 256 x 256 kernel is not: taken from 0.82 of its rounds filled on (one
+          full round and a second: 0.88): 8183 x 11264 x 2048: 346 -> 284 us, 8183 x 5056 x 4096: 384 -> 257, 11111 x 4096
+          x 4096: 389 -> 275, 2900 x 24576 x 4096: 544 -> 451; the worst of 14 shapes by 10 row counts: 368 -> 398; and with the gated epilogue, which saves the library a pass, from 0.55
+          (2039 x 9728 x 896: 67 -> 47)."""
+        choice = self.choose(M, N, K, epi)
+        if self.mode != "1" or M < LARGE_M or (M, N, K, epi) in self.table or not self.supported(W4_CFG, M, N, K, epi):
+            return [(M, choice)]
+        n_t, m_t = -(-N // 256), -(-M // 256)
+        tiles = m_t * n_t
+        rounds, rest = divmod(tiles, CUS)
+        if rounds and rest:
+            m1 = rounds * CUS // n_t
+            M1, M2 = 256 * m1, M - 256 * m1
+            if (0 < m1 < m_t and m1 * n_t >= 0.94 * rounds * CUS
+                    and 12 + 2e-6 * M2 * N * K / 0.8e3 < 0.6 * W4_KTILE_US * K / 64):
+                main = (W4_CFG, 1) if epi == 1 or (m1 * n_t) % CUS else None
+                if (M1, N, K, epi) in self.table:
+                    main = self.choose(M1, N, K, epi)
+                return [(M1, main), (M2, self.choose(M2, N, K, epi))]
+        filled = tiles / (CUS * (rounds + (rest > 0)))
+        whole = rest == 0 or rest >= 0.88 * CUS
+        if choice is None and (filled >= 0.55 if epi == 1 else rounds and not whole and filled >= (0.88 if rounds == 1 else 0.82)):
+            choice = (W4_CFG, 1)
+        return [(M, choice)]
 
 
 FP8_TABLE = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "engine", "tuned",

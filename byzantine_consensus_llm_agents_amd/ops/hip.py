@@ -370,14 +370,35 @@ def hip_ops() -> SimpleNamespace:
             key = (M, N, K, epi, dtype, "lib" if choice is None else f"{choice[0]}x{choice[1]}")
             dispatch_log.calls[key] = dispatch_log.calls.get(key, 0) + 1
 
+    def _plain(x, w):
+        """Operands that the kernels of this file take as they lie: bf16, rows contiguous, 16-byte aligned, and no
+        gradient asked of them (the library's products carry one, these do not)."""
+        return (x.dtype == w.dtype == torch.bfloat16 and w.dim() == 2 and w.shape[1] == x.shape[1] and x.is_contiguous()
+                and w.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+                and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)))
+
+    def _plain_bias(bias, N):
+        return bias is None or (bias.dtype == torch.bfloat16 and bias.shape == (N,) and bias.is_contiguous()
+                                and bias.data_ptr() % 16 == 0)
+
+    def _plain_residual(residual, M, N):
+        return (residual.shape == (M, N) and residual.dtype == torch.bfloat16 and residual.is_contiguous()
+                and residual.data_ptr() % 16 == 0)
+
+    def _pieces(x, w, epi, others=True):
+        """Runs of rows and their choices (`GemmPlan.pieces`); others: whether the bias / residual lies as the kernels want."""
+        M, K = x.shape
+        if others and _plain(x, w):
+            return plan.pieces(M, w.shape[0], K, epi)
+        return [(M, plan.choose(M, w.shape[0], K, epi))]
+
     def _skinny(x, w, epi):
         """Whether the few-row kernel takes x W^T: every shape of up to SKINNY_ROWS rows whose rows are whole 128-byte
         lines (csrc/kernels/gemm_skinny.hip holds both sides' times); table and library keep the others."""
         M, K = x.shape
         N = w.shape[0]
-        return (plan.mode == "1" and 1 <= M <= SKINNY_ROWS and x.dtype == w.dtype == torch.bfloat16 and w.dim() == 2
-                and w.shape[1] == K and K % 64 == 0 and 64 <= K <= SKINNY_MAX_K and N >= 8 and N % (8 if epi == 1 else 4) == 0
-                and x.is_contiguous() and w.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+        return (plan.mode == "1" and 1 <= M <= SKINNY_ROWS and K % 64 == 0 and 64 <= K <= SKINNY_MAX_K
+                and N >= 8 and N % (8 if epi == 1 else 4) == 0 and _plain(x, w))
 
     def _gemm_skinny(x, w, epi=0, bias=None, residual=None, norm_w=None, eps=0.0):
         M, K = x.shape
@@ -389,24 +410,32 @@ def hip_ops() -> SimpleNamespace:
                                    M, N, K, _stream()), "gemm_skinny")
         return out
 
-    def _few_row_bias(bias, N):
-        return bias is None or (bias.dtype == torch.bfloat16 and bias.shape == (N,) and bias.is_contiguous()
-                                and bias.data_ptr() % 8 == 0)
-
     def linear(x, w, bias=None, _epi_log=0):
         """y = x W^T (+b): the few-row kernel, the hand MFMA GEMM where the plan says it beats hipBLASLt, hipBLASLt
         otherwise."""
         M, K = x.shape
         N = w.shape[0]
-        if _skinny(x, w, 0) and _few_row_bias(bias, N):
+        if _skinny(x, w, 0) and _plain_bias(bias, N):
             return _gemm_skinny(x, w, 0, bias)
-        cfg = None
-        if x.is_contiguous() and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16:
-            cfg = plan.choose(M, N, K, 0)
-        _log(M, N, K, _epi_log, cfg)
+        if not (x.is_contiguous() and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16):
+            _log(M, N, K, _epi_log, None)
+            return torch.nn.functional.linear(x, w, bias)
+        parts = _pieces(x, w, 0, _plain_bias(bias, N))
+        if len(parts) == 1:
+            return _linear_rows(x, w, bias, parts[0][1], None, _epi_log)
+        out, at = torch.empty(M, N, dtype=x.dtype, device=x.device), 0
+        for rows, cfg in parts:
+            _linear_rows(x[at:at + rows], w, bias, cfg, out[at:at + rows], _epi_log)
+            at += rows
+        return out
+
+    def _linear_rows(x, w, bias, cfg, out, epi_log):
+        _log(x.shape[0], w.shape[0], x.shape[1], epi_log, cfg)
         if cfg is not None:
-            return gemm_nt(x, w, cfg, 0, bias=bias)
-        return torch.nn.functional.linear(x, w, bias)
+            return gemm_nt(x, w, cfg, 0, bias=bias, out=out)
+        if out is None:
+            return torch.nn.functional.linear(x, w, bias)
+        return torch.mm(x, w.t(), out=out) if bias is None else torch.addmm(bias, x, w.t(), out=out)
 
     from .gemm_plan import PP_CFG, W4_CFG, GemmPlan
     plan = GemmPlan(lib)
@@ -500,11 +529,21 @@ def hip_ops() -> SimpleNamespace:
         M, K = x.shape
         if _skinny(x, w, 1):
             return _gemm_skinny(x, w, 1)
-        cfg = plan.choose(M, w.shape[0], K, 1) if x.is_contiguous() and x.dtype == torch.bfloat16 else None
-        if cfg is None:
+        if not (x.is_contiguous() and x.dtype == torch.bfloat16):
             return silu_mul(linear(x, w, _epi_log=1))
-        _log(M, w.shape[0], K, 1, cfg)
-        return gemm_nt(x, w, cfg, 1)
+        parts, N = _pieces(x, w, 1), w.shape[0]
+        if len(parts) == 1 and parts[0][1] is None:
+            return silu_mul(linear(x, w, _epi_log=1))
+        out, at = torch.empty(M, N // 2, dtype=x.dtype, device=x.device), 0
+        for rows, cfg in parts:
+            xr, dst = x[at:at + rows], out[at:at + rows]
+            at += rows
+            if cfg is None:
+                dst.copy_(silu_mul(linear(xr, w, _epi_log=1)))
+            else:
+                _log(rows, N, K, 1, cfg)
+                gemm_nt(xr, w, cfg, 1, out=dst)
+        return out
 
     def _norm_fusable(x, w_norm):
         return (x.shape[1] <= 8192 and w_norm.shape == (x.shape[1],) and w_norm.dtype == torch.bfloat16 and w_norm.is_contiguous()
@@ -512,7 +551,7 @@ def hip_ops() -> SimpleNamespace:
 
     def norm_linear(x, w_norm, eps, w, bias=None):
         """linear(rmsnorm(x, w_norm, eps), w, bias), one kernel for a few rows."""
-        if x.dim() == 2 and _skinny(x, w, 0) and _norm_fusable(x, w_norm) and _few_row_bias(bias, w.shape[0]):
+        if x.dim() == 2 and _skinny(x, w, 0) and _norm_fusable(x, w_norm) and _plain_bias(bias, w.shape[0]):
             return _gemm_skinny(x, w, 0, bias, norm_w=w_norm, eps=eps)
         return linear(rmsnorm(x, w_norm, eps), w, bias)
 
@@ -528,20 +567,30 @@ def hip_ops() -> SimpleNamespace:
         """residual <- residual + x W^T (in place; the o/down projection fused with the
         residual-stream update of the next add+RMSNorm).  Returns `residual`."""
         M, K = x.shape
-        if (_skinny(x, w, 2) and residual.shape == (M, w.shape[0]) and residual.dtype == torch.bfloat16
-                and residual.is_contiguous() and residual.data_ptr() % 8 == 0):
+        if _skinny(x, w, 2) and _plain_residual(residual, M, w.shape[0]):
             return _gemm_skinny(x, w, 2, residual=residual)
-        cfg = plan.choose(M, w.shape[0], K, 2) if x.is_contiguous() and x.dtype == torch.bfloat16 else None
+        parts = [(M, None)]
+        if x.is_contiguous() and x.dtype == torch.bfloat16:
+            parts = _pieces(x, w, 2, _plain_residual(residual, M, w.shape[0]))
+        at = 0
+        for rows, cfg in parts:
+            whole = rows == M
+            _residual_rows(x if whole else x[at:at + rows], w, residual if whole else residual[at:at + rows], cfg)
+            at += rows
+        return residual
+
+    def _residual_rows(x, w, residual, cfg):
+        M, K = x.shape
         _log(M, w.shape[0], K, 2, cfg)
-        if cfg is None:
-            if (residual_addmm and residual.is_contiguous() and residual.dtype == x.dtype == w.dtype
-                    and residual.shape == (M, w.shape[0])):
-                # hipBLASLt with beta = 1: the residual add rides in the GEMM epilogue (one read
-                # of the residual, no separate elementwise pass over three [M, H] tensors)
-                return residual.addmm_(x, w.t())
+        if cfg is not None:
+            gemm_nt(x, w, cfg, 2, residual=residual, out=residual)
+        elif (residual_addmm and residual.is_contiguous() and residual.dtype == x.dtype == w.dtype
+                and residual.shape == (M, w.shape[0])):
+            # hipBLASLt with beta = 1: the residual add rides in the GEMM epilogue (one read
+            # of the residual, no separate elementwise pass over three [M, H] tensors)
+            residual.addmm_(x, w.t())
+        else:
             residual.add_(torch.nn.functional.linear(x, w))
-            return residual
-        return gemm_nt(x, w, cfg, 2, residual=residual, out=residual)
 
     def sample_step(logits, fsm_next, fsm_dist, fsm_base, fsm_state, gen_count, max_new, temperature,
                     row_keys, done, seq_lens, out_tokens, next_tokens, seed, budget_aware, n_text_tokens,
