@@ -20,6 +20,8 @@
 // The bf16 instance for heads up to 64 / 128 wide takes 32 keys per iteration and prefetches
 // the next iteration's K fragments in registers.
 //
+// prefill_staged_kernel: the same tiles for exact shapes with 16-token pages, K and V through LDS.
+//
 // decode_mfma_kernel: single-token rows.  The 16 MFMA columns hold the query heads that share
 // one KV head (GQA packing), so the cache is read once per KV head; one wave per 128-key split.
 // The split size is fixed, so a row's result does not depend on what else is in the batch.
@@ -68,6 +70,31 @@ struct AttnArgs {
   const float* slopes;      // [H] or null: slope_h (i - j) is taken off the score (SHAPED instances)
   int swz;                  // fragment-major slabs (see the top of the file)
 };
+
+// Maximum / sum over the four lanes that share a column (lanes col, col + 16, col + 32, col + 48): register swaps, no LDS
+// round trip.
+__device__ __forceinline__ float column_max(float x) {
+  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float column_sum(float x) {
+  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// Two neighbouring 16-deep operands in one 32-deep product (bf16): the lanes' 4 + 4 elements of both operands pair up the
+// same way, so the order of k inside the instruction is free.  An odd last operand is paired with zeros: a 16-deep product
+// behind 32-deep ones on the same accumulator gave wrong sums.
+__device__ __forceinline__ f32x4 mma32(s16x4 a0, s16x4 a1, s16x4 b0, s16x4 b1, f32x4 c) {
+  typedef short s16x8 __attribute__((ext_vector_type(8)));
+  const s16x8 a = __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7), b = __builtin_shufflevector(b0, b1, 0, 1, 2, 3, 4, 5, 6, 7);
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4 mma32(f32x4 a0, f32x4 a1, f32x4 b0, f32x4 b1, f32x4 c) { return mma16(a1, b1, mma16(a0, b0, c)); }
 
 // First key that a query at position `pos` sees: the window's or the chunk's first, else 0.
 __device__ __forceinline__ int first_key(const AttnArgs& a, int pos) {
@@ -224,10 +251,13 @@ __device__ __forceinline__ void attend_range(const AttnArgs& a_, int g, const ty
 #pragma unroll
       for (int m = 0; m < NM; ++m) {
         s[u][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (m < a.maps) {
+        if (m < a.maps) {   // (fragments past kc are zero)
 #pragma unroll
-          for (int c = 0; c < KC; ++c)
-            if (c < kc) s[u][m] = mma16(kf[u][m][c], qf[m][c], s[u][m]);
+          for (int c = 0; c + 1 < KC; c += 2)
+            if (c < kc) s[u][m] = mma32(kf[u][m][c], kf[u][m][c + 1], qf[m][c], qf[m][c + 1], s[u][m]);
+          if constexpr (KC & 1) {
+            if (KC - 1 < kc) s[u][m] = mma32(kf[u][m][KC - 1], zero_frag<T>(), qf[m][KC - 1], zero_frag<T>(), s[u][m]);
+          }
         }
       }
     // the K fragments are spent: the next iteration's go into the same registers, under the
@@ -258,9 +288,7 @@ __device__ __forceinline__ void attend_range(const AttnArgs& a_, int g, const ty
           if (masked && (key > limit || (key < lo && !(MODE == KEEP && key < keep)))) v[u][i] = -INFINITY;
           bm = fmaxf(bm, v[u][i]);
         }
-      bm = fmaxf(bm, __shfl_xor(bm, 16, WAVE));
-      bm = fmaxf(bm, __shfl_xor(bm, 32, WAVE));
-      const float m_new = fmaxf(mx[m], bm);                 // finite: the running maximum starts finite
+      const float m_new = fmaxf(mx[m], column_max(bm));     // finite: the running maximum starts finite
       float ps = 0.f;
 #pragma unroll
       for (int u = 0; u < KT; ++u)
@@ -269,8 +297,6 @@ __device__ __forceinline__ void attend_range(const AttnArgs& a_, int g, const ty
           v[u][i] = __builtin_amdgcn_exp2f(v[u][i] - m_new);
           ps += v[u][i];
         }
-      ps += __shfl_xor(ps, 16, WAVE);
-      ps += __shfl_xor(ps, 32, WAVE);
       if (__any(m_new > mx[m])) {                           // (wave-uniform) the running maximum moved
         const float alpha = __builtin_amdgcn_exp2f(mx[m] - m_new);
         den[m] *= alpha;
@@ -284,19 +310,25 @@ __device__ __forceinline__ void attend_range(const AttnArgs& a_, int g, const ty
       for (int u = 0; u < KT; ++u) pf[u][m] = Elem<T>::pack(v[u][0], v[u][1], v[u][2], v[u][3]);
     }
     // ---- O^T += V^T P^T ----
+    static_assert(KT <= 2, "one 32-deep product per 32 keys");
 #pragma unroll
-    for (int u = 0; u < KT; ++u)
+    for (int t = 0; t < VT; ++t)
+      if (t < vt) {
+        F x[KT];
 #pragma unroll
-      for (int t = 0; t < VT; ++t)
-        if (t < vt) {
-          F x;
-          if constexpr (PF) x = vf[u][t]; else x = load_v(u, t);
-          acc[0][t] = mma16(x, pf[u][0], acc[0][t]);
-          if constexpr (NM > 1) {
-            if (a.maps > 1) acc[1][t] = mma16(x, pf[u][1], acc[1][t]);
-          }
+        for (int u = 0; u < KT; ++u) {
+          if constexpr (PF) x[u] = vf[u][t]; else x[u] = load_v(u, t);
         }
+#pragma unroll
+        for (int m = 0; m < NM; ++m)
+          if (m < a.maps) {
+            if constexpr (KT == 2) acc[m][t] = mma32(x[0], x[1], pf[0][m], pf[1][m], acc[m][t]);
+            else acc[m][t] = mma16(x[0], pf[0][m], acc[m][t]);
+          }
+      }
   }
+#pragma unroll
+  for (int m = 0; m < NM; ++m) den[m] = column_sum(den[m]);
 }
 
 template <typename T, int KC, int VT, int KT, bool PF, bool FULL, int OCC, int EXACT = 0, int NM = 2, int MODE = PLAIN>
@@ -338,7 +370,7 @@ __global__ __launch_bounds__(256, OCC) void prefill_kernel(AttnArgs a) {
   }
   if (a.sink != nullptr) {   // the sink starts the softmax: weight 1 at its own logit
     mx[0] = a.sink[h] * LOG2E;
-    den[0] = 1.0f;
+    den[0] = grp == 0 ? 1.0f : 0.0f;   // (a column's denominator is summed over its lanes at the end)
   }
   const int lo = first_key(a, pos), lo_max = first_key(a, pos_max);   // (both masks: the first key grows with the position)
   const int k_win = first_key(a, pos_min) & ~15, k_begin = MODE == KEEP ? 0 : k_win;
@@ -366,8 +398,7 @@ __global__ __launch_bounds__(256, OCC) void prefill_kernel(AttnArgs a) {
         ss += o * o;   // rows >= vdim are zero (their V^T fragments were zero)
       }
     }
-  ss += __shfl_xor(ss, 16, WAVE);
-  ss += __shfl_xor(ss, 32, WAVE);
+  ss = column_sum(ss);
   const float r = (a.head_eps >= 0.f ? 1.0f / sqrtf(ss / a.vdim + a.head_eps) : 1.0f) * a.out_scale;
   if (col < n_rows) {
     T* orow = static_cast<T*>(a.out) + (static_cast<size_t>(row) * a.H + h) * a.vdim;
@@ -375,12 +406,225 @@ __global__ __launch_bounds__(256, OCC) void prefill_kernel(AttnArgs a) {
     for (int t = 0; t < VT; ++t)
       if (t < vt) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int e = 16 * t + 4 * grp + i;
-          if (e < a.vdim) orow[e] = Elem<T>::st(acc[0][t][i] * r);
+        for (int i = 0; i < 4; ++i) acc[0][t][i] *= r;
+        const int e = 16 * t + 4 * grp;
+        if (EXACT) {   // whole tiles, aligned rows
+          *reinterpret_cast<F*>(orow + e) = Elem<T>::pack(acc[0][t][0], acc[0][t][1], acc[0][t][2], acc[0][t][3]);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (e + i < a.vdim) orow[e + i] = Elem<T>::st(acc[0][t][i]);
         }
       }
   }
+}
+
+// Prefill tiles of exact shapes (bf16, 16-token pages, fragment-major slabs), the pages staged through LDS.
+//
+// What bounded the form above: each of its waves loads every K / V fragment for 16 query rows alone and waits for it,
+// with registers for one block in flight.  Here the 4 waves of a tile read one copy: a chunk of 32 keys is two pages,
+// each a contiguous run of K and of V, copied as it lies (16 bytes per thread and access; the next chunk is in flight
+// in registers while this one is multiplied, the page numbers one chunk further ahead; two buffers, one barrier per
+// chunk).  The fragments come from LDS at the offsets they have in the slab, the 4-key rows of V moved apart by 128
+// bytes so that the lane groups read different banks.  All waves walk the tile's key range; a wave skips chunks that
+// hold no key it sees.  Tiles with the most keys start first, the heads of a tile side by side.
+// Measured, 8 prompts of 1000 tokens: two 64-wide maps over 128-wide values, 16 heads: 226 us (one load per wave, 16-deep
+// products) -> 190 (32-deep products, column statistics by register swaps) -> 148 here; 32 latent heads of 192 / 128:
+// 379 -> 313 -> 168; 3 prompts of 700, 16 heads of 128 with a window: 52 -> 43 -> 29.  Two heads' waves on one copy
+// (512 threads) measured the same at the large sizes and 41 against 36 us at the small one.  What is left: LDS reads
+// (20 KB per 16 rows and chunk, 75 of the 168 us if alone) and softmax arithmetic, at 3 waves per SIMD.
+template <int KC, int VT, int NM, int MODE>
+__global__ __launch_bounds__(256, NM * (KC + 2 * VT) <= 24 ? 4 : KC + VT <= 24 ? 3 : 2) void prefill_staged_kernel(AttnArgs a) {
+  typedef s16x4 F;
+  constexpr int DIM = 16 * KC, VD = 16 * VT, KD = NM * DIM, TH = 256;
+  constexpr int UNITS = 4 * (KD + VD), NU = (UNITS + TH - 1) / TH;   // 16-byte units of a chunk, and per thread
+  constexpr int VROW = VD / 2 + 8, BUF = 4 * KD + 8 * VROW;          // LDS: the 4-key rows of V 128 bytes apart in banks
+  __shared__ __attribute__((aligned(16))) f32x4 chunk_lds[2 * BUF];  // twice K page 0, K page 1, V page 0, V page 1
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 15, grp = lane >> 4;
+  const int h = blockIdx.x % a.H, g = h / (a.H / a.G);
+  const int* item = a.work + 3 * ((gridDim.x - 1 - blockIdx.x) / a.H);
+  const int seq = item[0], first = item[1], row_end = item[2];
+  const int row0 = first + 16 * wave;
+  const bool active = row0 < row_end;
+  const int ctx = a.seq_lens[seq], q_end = a.q_start[seq + 1];
+  const int n_rows = active ? min(16, row_end - row0) : 1;
+  const int row = (active ? row0 : first) + min(col, n_rows - 1);   // columns past the tile repeat its last row (never stored)
+  const int pos = ctx - (q_end - row);
+  const int pos_min = ctx - (q_end - (active ? row0 : first)), pos_max = pos_min + n_rows - 1;
+  const int pos_first = ctx - (q_end - first), pos_last = ctx - (q_end - (row_end - 1));
+  const bf16_t* qrow = static_cast<const bf16_t*>(a.q) + (static_cast<size_t>(row) * a.H + h) * KD;
+  F qf[NM][KC];
+#pragma unroll
+  for (int m = 0; m < NM; ++m)
+#pragma unroll
+    for (int c = 0; c < KC; ++c) qf[m][c] = *reinterpret_cast<const F*>(qrow + m * DIM + 16 * c + 4 * grp);
+  f32x4 acc[NM][VT];
+  float mx[NM], den[NM];
+#pragma unroll
+  for (int m = 0; m < NM; ++m) {
+    mx[m] = MAX_FLOOR;
+    den[m] = 0.f;
+#pragma unroll
+    for (int t = 0; t < VT; ++t) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  if (a.sink != nullptr) {   // the sink starts the softmax: weight 1 at its own logit
+    mx[0] = a.sink[h] * LOG2E;
+    den[0] = grp == 0 ? 1.0f : 0.0f;
+  }
+  const int lo = first_key(a, pos), lo_min = first_key(a, pos_min), lo_max = first_key(a, pos_max);
+  const int k_win = first_key(a, pos_first) & ~15, k_begin = MODE == KEEP ? 0 : k_win, keep = MODE == KEEP ? a.keep : 0;
+  const float sc = a.scale * LOG2E;
+  const float slope = MODE == SHAPED && a.slopes != nullptr ? a.slopes[h] * LOG2E : 0.f;
+  const float cap = MODE == SHAPED ? a.softcap : 0.f;
+  const float cap2 = cap * LOG2E, arg2 = cap > 0.f ? 2.0f * LOG2E * a.scale / cap : 0.f;
+  auto next_key = [&](int key0) {   // KEEP: past the kept keys, on to the window
+    const int n = key0 + 32;
+    if constexpr (MODE == KEEP) return (n >= keep && n < k_win) ? k_win : n;
+    else return n;
+  };
+
+  const int* table = a.block_tables + static_cast<size_t>(seq) * a.max_blocks;
+  const int last_page = min((ctx - 1) >> 4, a.max_blocks - 1);
+  auto page_of = [&](int p) {   // past the sequence: its last page again, every key of it is masked
+    const int page = table[min(p, last_page)];
+    return static_cast<size_t>((page < 0 || page >= a.num_blocks) ? 0 : page) * a.G + g;
+  };
+  f32x4 stage[NU];   // (the threads past the end of a chunk repeat its last unit)
+  auto fetch = [&](size_t s0, size_t s1) {
+#pragma unroll
+    for (int i = 0; i < NU; ++i) {
+      const int u = min(tid + i * TH, UNITS - 1);
+      const bool isv = u >= 4 * KD;
+      const int w = isv ? VD : KD, r = isv ? u - 4 * KD : u, second = r >= 2 * w;
+      const f32x4* base = static_cast<const f32x4*>(isv ? a.v_cache : a.k_cache);
+      stage[i] = base[(second ? s1 : s0) * (2 * w) + (r - second * 2 * w)];
+    }
+  };
+  auto put = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < NU; ++i) {
+      const int u = min(tid + i * TH, UNITS - 1), v = u - 4 * KD;
+      chunk_lds[buf * BUF + (v < 0 ? u : 4 * KD + v + v / (VD / 2) * 8)] = stage[i];
+    }
+  };
+
+  int key0 = k_begin, nxt = next_key(k_begin);
+  fetch(page_of(key0 >> 4), page_of((key0 >> 4) + 1));
+  put(0);
+  fetch(page_of(nxt >> 4), page_of((nxt >> 4) + 1));
+  size_t p0 = page_of(next_key(nxt) >> 4), p1 = page_of((next_key(nxt) >> 4) + 1);   // the pages two chunks ahead
+  __syncthreads();
+  for (int buf = 0; key0 <= pos_last; buf ^= 1) {
+    if (active && key0 <= pos_max && (key0 + 31 >= lo_min || key0 < keep)) {   // (wave-uniform) some key is seen
+      const bf16_t* ks = reinterpret_cast<const bf16_t*>(chunk_lds + buf * BUF);
+      const bf16_t* vs = ks + 32 * KD;
+      f32x4 sm[2][NM];
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+          sm[u][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+          auto frag = [&](int c) { return *reinterpret_cast<const F*>(ks + u * 16 * KD + ((m * DIM + 16 * c) / 4 * 16 + grp * 16 + col) * 4); };
+#pragma unroll
+          for (int c = 0; c + 1 < KC; c += 2) sm[u][m] = mma32(frag(c), frag(c + 1), qf[m][c], qf[m][c + 1], sm[u][m]);
+          if constexpr (KC & 1) sm[u][m] = mma32(frag(KC - 1), zero_frag<bf16_t>(), qf[m][KC - 1], zero_frag<bf16_t>(), sm[u][m]);
+        }
+      const bool masked = key0 + 31 > pos_min || key0 < lo_max;
+      float cap_now = cap;
+      if constexpr (MODE == SHAPED) asm volatile("" : "+v"(cap_now));
+      const bool capped = cap_now > 0.f;
+      F pf[2][NM];
+#pragma unroll
+      for (int m = 0; m < NM; ++m) {
+        float v[2][4], bm = -INFINITY;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int key = key0 + 16 * u + 4 * grp + i;
+            if constexpr (MODE == SHAPED) {
+              float x = sm[u][m][i] * sc;
+              if (capped) x = cap2 - 2.0f * cap2 * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(sm[u][m][i] * arg2) + 1.0f);
+              v[u][i] = x - slope * static_cast<float>(pos - key);
+            } else {
+              v[u][i] = sm[u][m][i] * sc;
+            }
+            if (masked && (key > pos || (key < lo && !(MODE == KEEP && key < keep)))) v[u][i] = -INFINITY;
+            bm = fmaxf(bm, v[u][i]);
+          }
+        const float m_new = fmaxf(mx[m], column_max(bm));
+        float ps = 0.f;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            v[u][i] = __builtin_amdgcn_exp2f(v[u][i] - m_new);
+            ps += v[u][i];
+          }
+        if (__any(m_new > mx[m])) {
+          const float alpha = __builtin_amdgcn_exp2f(mx[m] - m_new);
+          den[m] *= alpha;
+#pragma unroll
+          for (int t = 0; t < VT; ++t) acc[m][t] *= alpha;
+        }
+        den[m] += ps;
+        mx[m] = m_new;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) pf[u][m] = Elem<bf16_t>::pack(v[u][0], v[u][1], v[u][2], v[u][3]);
+      }
+#pragma unroll
+      for (int t = 0; t < VT; ++t) {
+        const F x0 = *reinterpret_cast<const F*>(vs + grp * 8 * VROW + (16 * t + col) * 4);
+        const F x1 = *reinterpret_cast<const F*>(vs + (4 + grp) * 8 * VROW + (16 * t + col) * 4);
+#pragma unroll
+        for (int m = 0; m < NM; ++m) acc[m][t] = mma32(x0, x1, pf[0][m], pf[1][m], acc[m][t]);
+      }
+    }
+    if (nxt <= pos_last) put(buf ^ 1);   // (its readers passed the barrier of the chunk before)
+    key0 = nxt;
+    nxt = next_key(nxt);
+    if (nxt <= pos_last) {
+      fetch(p0, p1);
+      const int n2 = next_key(nxt);
+      p0 = page_of(n2 >> 4);
+      p1 = page_of((n2 >> 4) + 1);
+    }
+    __syncthreads();
+  }
+  if (!active) return;
+  float o_den[NM];
+#pragma unroll
+  for (int m = 0; m < NM; ++m) o_den[m] = (m == 0 ? 1.0f : a.lam) / column_sum(den[m]);
+  float ss = 0.f;
+#pragma unroll
+  for (int t = 0; t < VT; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float o = acc[0][t][i] * o_den[0];
+      if constexpr (NM > 1) o -= acc[1][t][i] * o_den[1];
+      acc[0][t][i] = o;
+      ss += o * o;
+    }
+  ss = column_sum(ss);
+  const float r = (a.head_eps >= 0.f ? 1.0f / sqrtf(ss / VD + a.head_eps) : 1.0f) * a.out_scale;
+  if (col < n_rows) {
+    bf16_t* orow = static_cast<bf16_t*>(a.out) + (static_cast<size_t>(row) * a.H + h) * VD;
+#pragma unroll
+    for (int t = 0; t < VT; ++t)
+      *reinterpret_cast<F*>(orow + 16 * t + 4 * grp) = Elem<bf16_t>::pack(acc[0][t][0] * r, acc[0][t][1] * r, acc[0][t][2] * r, acc[0][t][3] * r);
+  }
+}
+
+// what the copies of whole pages need: one page is a chunk's half, slabs of whole 16-byte units
+inline bool staged_layout(const AttnArgs& a) {
+  return a.swz && a.BS == 16 && ((reinterpret_cast<uintptr_t>(a.k_cache) | reinterpret_cast<uintptr_t>(a.v_cache)) & 15) == 0;
+}
+
+template <int KC, int VT, int NM, int MODE>
+int launch_staged(const AttnArgs& a, int n_tiles, hipStream_t s) {
+  prefill_staged_kernel<KC, VT, NM, MODE><<<n_tiles * a.H, 256, 0, s>>>(a);
+  return BCG_CHECK_LAUNCH();
 }
 
 // Single-token rows, the query heads of one KV head packed into the 16 MFMA columns: column c is
@@ -526,7 +770,7 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(AttnArgs a) {
 
 // Exact one-map instances (bf16): X(KC, VT, keys tiles per iteration, workgroups per CU).
 #define BCG_EXACT1_PLAIN(X) X(8, 8, 2, 2) X(4, 4, 2, 2) X(4, 8, 2, 2) X(2, 2, 2, 2) X(6, 6, 2, 2) X(6, 4, 2, 2) X(12, 8, 2, 2) \
-                            X(12, 12, 2, 1) X(16, 16, 2, 1) X(32, 32, 1, 1)
+                            X(12, 12, 2, 1) X(16, 16, 2, 1)
 #define BCG_EXACT1_KEEP(X) X(8, 8, 2, 2) X(4, 4, 2, 2) X(4, 8, 2, 2) X(2, 2, 2, 2) X(6, 6, 2, 2) X(12, 12, 2, 1) X(16, 16, 2, 1)
 #define BCG_EXACT1_SHAPED(X) X(8, 8, 2, 2) X(4, 4, 2, 2) X(2, 2, 2, 2) X(3, 3, 2, 2) X(6, 6, 2, 2) X(12, 12, 2, 1) X(16, 16, 2, 1)
 
@@ -534,11 +778,10 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(AttnArgs a) {
 template <typename T, int MODE>
 int launch_prefill_mode(const AttnArgs& a, int n_tiles, bool full, hipStream_t s) {
   dim3 grid(n_tiles, a.H);
-  if constexpr (sizeof(T) == 2) if (full && a.swz && a.BS == 16) {
+  if constexpr (sizeof(T) == 2) if (full && staged_layout(a)) {
 #define BCG_X(KC_, VT_, KT_, OCC_)                                                               \
   if (a.dim == 16 * KC_ && a.vdim == 16 * VT_) {                                                 \
-    prefill_kernel<T, KC_, VT_, KT_, true, true, OCC_, 1, 1, MODE><<<grid, 256, 0, s>>>(a);      \
-    return BCG_CHECK_LAUNCH();                                                                   \
+    return launch_staged<KC_, VT_, 1, MODE>(a, n_tiles, s);                                      \
   }
     if constexpr (MODE == SHAPED) { BCG_EXACT1_SHAPED(BCG_X) } else { BCG_EXACT1_KEEP(BCG_X) }
 #undef BCG_X
@@ -573,21 +816,23 @@ int launch_prefill(const AttnArgs& a, int n_tiles, int tile_rows, hipStream_t s)
   if (tile_rows != 64) return -2;
   if (a.softcap > 0.f || a.slopes != nullptr) return launch_prefill_mode<T, SHAPED>(a, n_tiles, full, s);
   if (a.keep > 0) return launch_prefill_mode<T, KEEP>(a, n_tiles, full, s);
-  if constexpr (sizeof(T) == 2) if (full && a.maps == 1 && a.swz && a.BS == 16) {   // one-map heads, exact shapes
+  if constexpr (sizeof(T) == 2) if (full && a.maps == 1 && staged_layout(a)) {   // one-map heads, exact shapes
 #define BCG_X(KC_, VT_, KT_, OCC_)                                                               \
   if (a.dim == 16 * KC_ && a.vdim == 16 * VT_) {                                                 \
-    prefill_kernel<T, KC_, VT_, KT_, true, true, OCC_, 1, 1><<<grid, 256, 0, s>>>(a);            \
-    return BCG_CHECK_LAUNCH();                                                                   \
+    return launch_staged<KC_, VT_, 1, PLAIN>(a, n_tiles, s);                                     \
   }
     BCG_EXACT1_PLAIN(BCG_X)
 #undef BCG_X
+    if (a.dim == 512 && a.vdim == 512) {   // (two chunks of it do not fit the 64 KiB)
+      prefill_kernel<T, 32, 32, 1, true, true, 1, 1, 1><<<grid, 256, 0, s>>>(a);
+      return BCG_CHECK_LAUNCH();
+    }
   }
   if constexpr (sizeof(T) == 2) if (small) {
-    const bool exact = full && a.maps == 2 && a.swz && a.BS == 16;
+    const bool exact = full && a.maps == 2 && staged_layout(a);
 #define BCG_EXACT(KC_, VT_)                                                                      \
   if (exact && a.dim == 16 * KC_ && a.vdim == 16 * VT_) {                                        \
-    prefill_kernel<T, KC_, VT_, 2, true, true, 2, 2><<<grid, 256, 0, s>>>(a);                    \
-    return BCG_CHECK_LAUNCH();                                                                   \
+    return launch_staged<KC_, VT_, 2, PLAIN>(a, n_tiles, s);                                     \
   }
     BCG_EXACT(4, 8) BCG_EXACT(3, 6) BCG_EXACT(2, 4) BCG_EXACT(4, 4) BCG_EXACT(2, 2)
 #undef BCG_EXACT
@@ -626,6 +871,10 @@ int launch_decode(const AttnArgs& a, int n_items, hipStream_t s) {
     decode_mfma_kernel<T, KC_, VT_, KT_, true, true, OCC_, 1, 1><<<grid, 64, 0, s>>>(a);         \
   }
     BCG_EXACT1_PLAIN(BCG_X)
+    if (!done && a.dim == 512 && a.vdim == 512) {
+      done = true;
+      decode_mfma_kernel<T, 32, 32, 1, true, true, 1, 1, 1><<<grid, 64, 0, s>>>(a);
+    }
 #undef BCG_X
   }
   if constexpr (sizeof(T) == 2) if (!done && a.dim <= 64 && a.vdim <= 128) {
