@@ -34,7 +34,7 @@ def _segments(meta, T):
 
 
 def seqstate_ops(lib):
-    min_chunked = lib.bcg_retention_min_len()
+    min_chunked, chunk = lib.bcg_decay_chunks_min_len(), lib.bcg_decay_chunks_tokens()
 
     def embed_hashed_bigram_norm(tokens, meta, prev, table, scale, bigram, hash_mul, eps, gains, out_dtype):
         T, W = tokens.numel(), table.shape[1]
@@ -209,14 +209,15 @@ def seqstate_ops(lib):
             _req(beta.dtype == torch.float32 and beta.is_contiguous() and beta.shape == (T, H), "beta fp32 [T, H]")
         B = _segments(meta, T)
         out = torch.empty(T, H, vdim, dtype=torch.float32, device=g.device)
-        # a fixed decay per head and plain writes: long segments run as chunks of matrix products, the
+        # one decay per head and no correction term: long segments run as chunks of matrix products, the
         # short ones among them (single tokens beside portions) token by token
         skip = 0
-        if g_const and beta is None and not delta and not unit_last and not meta.decode and T - B + 1 >= min_chunked:
+        if gd == 1 and not delta and not unit_last and not meta.decode and T - B + 1 >= min_chunked:
             skip = min_chunked
-            _check(lib.bcg_retention_chunks(_p(q), _p(k), _p(g), _p(v), v.stride(0), _p(meta.positions), _p(meta.q_start),
-                                            _p(meta.state_rows), _p(state), state.shape[0], _p(out), B, H, Gq, dim, vdim, _act(v),
-                                            _stream()), "retention_chunks")
+            scores = torch.empty((T // chunk + B) * Gq * chunk * chunk, dtype=torch.float32, device=g.device)
+            _check(lib.bcg_decay_chunks(_p(q), _p(k), _p(g), 0 if g_const else H, _p(beta), _p(v), v.stride(0), _p(meta.positions),
+                                        _p(meta.q_start), _p(meta.state_rows), _p(state), state.shape[0], _p(out), _p(scores), T, B,
+                                        H, Gq, dim, vdim, _act(v), _stream()), "decay_chunks")
             if B == 1:
                 return out
         _check(lib.bcg_gated_state_scan(_p(q), _p(k), _p(g), _p(v), v.stride(0), _p(beta), _p(meta.positions),

@@ -1,43 +1,62 @@
-// Recurrence with one fixed decay per head over chunks of tokens (retention, long segments):
+// Recurrence with one decay per head over chunks of tokens (retention, scalar-decay state spaces; long segments):
 //
-//   S_t = g S_(t-1) + k_t v_t^T,  o_t = S_t^T q_t        S fp32 [dim, vdim] per head, g in [0, 1]
+//   S_t = g_t S_(t-1) + b_t k_t v_t^T,  o_t = S_t^T q_t        S fp32 [dim, vdim] per head, g in [0, 1]
 //
-// A chunk of CT tokens is one set of matrix products instead of CT steps; with S the state in
-// front of the chunk and r = 0, 1, ... the token's place in it,
+// (g the same for every token or one number per token; b = 1 or one number per token).  A chunk of CT tokens is one
+// set of matrix products instead of CT steps; with S the state in front of the chunk and
+// W(r, s) = g_(s + 1) ... g_r the decay from token s of the chunk to token r,
 //
-//   o_r = g^(r + 1) S^T q_r + sum_(s <= r) g^(r - s) (q_r . k_s) v_s
-//   S  <- g^n S + sum_s g^(n - 1 - s) k_s v_s^T            (n tokens in the chunk)
+//   o_r = (g_0 ... g_r) S^T q_r + sum_(s <= r) W(r, s) b_s (q_r . k_s) v_s
+//   S  <- (g_0 ... g_n-1) S + sum_s W(n - 1, s) b_s k_s v_s^T            (n tokens in the chunk)
 //
-// Everything is fp32 (true-fp32 MFMAs, `mma16`); v is read in the activation type T.  The powers of g
-// come from a table of repeated products (g = 0 gives 1, 0, 0, ...).  The token-by-token form of
-// seqmix_state.hip serves short segments; both leave the same state up to rounding.
+// Everything is fp32 (true-fp32 MFMAs, `mma16`); v is read in the activation type T.  Every W is a product of decays (in
+// double, rounded once), never a quotient (a decay of 0 cuts cleanly): inside a 16-token block directly, across blocks as (from s to the end of
+// its block) x (whole blocks) x (from the start of r's block to r).  The token-by-token form of seqmix_state.hip serves
+// short segments; both leave the same state up to rounding.
 //
-// One workgroup per (segment, head, VT value columns), four waves.  The chunk's keys lie in LDS as
-// rows, its values transposed, the state transposed (value column by value column).  Wave w owns the
-// chunk's queries 16 w .. 16 w + 15 and the state's key-feature tiles w, w + 4, ...  The products are
+// Two launches.  scores_kernel computes the q_r . k_s of all chunks at once (heads that share q and k
+// share them, and so do the workgroups of a head).  chunk_kernel walks a segment's chunks:
+// one workgroup per (segment, head, VT value columns), four waves.  The chunk's values lie in LDS transposed, and so does
+// the state (value column by value column).  Wave w owns the chunk's queries 16 w .. 16 w + 15
+// and the state's key features from 16 ND w on (a lane's ND features are neighbours).  The products are
 // arranged so that a result in C registers is the next product's B operand (no shuffle):
 //   S^T Q^T       [value column x query]   from the state in LDS
-//   K Q^T         [key x query]            weighted by g^(r - s), zero above the diagonal
-//   V^T (K Q^T)   [value column x query]   added to it
-//   V^T K         [value column x key feature], keys weighted by g^(n - 1 - s): the state's update
+//   V^T (K Q^T)   [value column x query]   scores weighted by W b, added to it
+//   V^T K         [value column x key feature], keys weighted by W b: the state's update
+// The walk is a serial chain, so its operands are fetched a chunk ahead into the registers that the phase before has
+// just used up (no wave needs another wave's keys or queries: they do not pass LDS), and VT shrinks where the launch would leave CUs
+// idle.  What bounds it: the fp32 matrix rate (32 cycles per 16 x 16 x 4) where all CUs are busy, else the chain.
+// Measured, both launches: 3 segments of 700 tokens, 8 heads, 128 x 256 states: 89 us (keys, scores and 64-column
+// workgroups in one kernel, 96 workgroups: 202); 8 segments of 1000, 128 heads sharing keys, 128 x 64 states: 494 us (token
+// by token: 1552), of which the matrix rate is 250; 64 segments of 16: 149 (220).
+// Rounding, against float64 (relative rms, token by token -> here): decays about 0.5: 8.4e-8 -> 7.4e-8, 0.9: 1.1e-7 -> 1.0e-7, 0.99:
+// 2.5e-7 -> 1.2e-7, 0.999: 4.6e-7 -> 1.5e-7.  That takes the scores in double (parallel, so nearly free), decay products in
+// double, and short chains in the fp32 accumulators (one chain over all features and keys: 1.5e-7 at decays about 0.5).
 #include <algorithm>
 
 #include "seqmix_common.h"
 
 namespace {
 
-constexpr int CT = 64, VT = 64, NTH = 256;
-constexpr int MIN_LEN = 16;   // shorter segments are faster token by token
+constexpr int CT = 64, NTH = 256;
+// Shorter segments go token by token.  Measured (us, token by token -> here): 64 segments of 16, 128 heads: 220 -> 149; 8 heads: 69 ->
+// 45; 4 heads of 64 x 64: 10 -> 12 (the second launch), 4 segments of 40: 15 -> 11.
+constexpr int MIN_LEN = 16;
 
 struct ChunkArgs {
   const float* q; const float* k;                   // [T, Gq, dim]
-  const float* decay;                               // [H]
+  const float* g; int g_token;                      // [H] (g_token 0) or [T, H]
+  const float* beta;                                // [T, H] or null
   const void* v; int64_t v_stride;                  // [T, >= H vdim]
   const int* positions; const int* q_start; const int* state_rows;
   float* state;                                     // [n_rows, H, dim, vdim]
   float* out;                                       // [T, H, vdim]
-  int n_rows, H, Gq, dim, vdim, vec;                // vec: rows of q / k are 16-byte aligned
+  float* scores;                                    // [chunks, Gq, CT (query), CT (key)]
+  int n_rows, B, H, Gq, dim, vdim, vec;             // vec: rows of q / k are 16-byte aligned
 };
+
+// Segment b's chunk c has the number q_start[b] / CT + b + c: at most T / CT + B numbers, no two chunks alike.
+__device__ __forceinline__ int chunk_base(const int* q_start, int b) { return q_start[b] / CT + b; }
 
 // four fp32 at p[0..3], zero from n_valid on
 __device__ __forceinline__ f32x4 load4(const float* p, int n_valid, bool vec) {
@@ -49,48 +68,147 @@ __device__ __forceinline__ f32x4 load4(const float* p, int n_valid, bool vec) {
   return r;
 }
 
+// FULL: whole aligned tiles (dim = 16 DC): no branch around a load
+template <bool FULL>
+__device__ __forceinline__ f32x4 load4f(const float* p, int n_valid, bool vec) {
+  if constexpr (FULL) return *reinterpret_cast<const f32x4*>(p);
+  else return load4(p, n_valid, vec);
+}
+
+template <int DC, bool FULL>
+__global__ __launch_bounds__(NTH) void scores_kernel(ChunkArgs a) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 15, grp = lane >> 4;
+  const int id = blockIdx.x, gq = blockIdx.y, dim = a.dim;
+  int lo = 0, hi = a.B - 1;   // the last segment whose first number is <= id
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (chunk_base(a.q_start, mid) <= id) lo = mid; else hi = mid - 1;
+  }
+  const int t0 = a.q_start[lo], t1 = a.q_start[lo + 1], first = t0 + (id - chunk_base(a.q_start, lo)) * CT;
+  if (t1 - t0 < MIN_LEN || first < t0 || first >= t1) return;
+  for (int e = wave; e < 10; e += 4) {   // the ten 16 x 16 tiles on and under the diagonal
+    const int rt = e >= 6 ? 3 : e >= 3 ? 2 : e >= 1 ? 1 : 0, st = e - rt * (rt + 1) / 2;
+    if (first + 16 * rt >= t1) continue;
+    const float* qrow = a.q + (static_cast<size_t>(min(first + 16 * rt + col, t1 - 1)) * a.Gq + gq) * dim + 4 * grp;
+    // (register i of a double result holds row grp + 4 i of the first operand: lane `col` supplies the key that makes it 4 grp + i)
+    const int key = 4 * (col & 3) + (col >> 2);
+    const float* krow = a.k + (static_cast<size_t>(min(first + 16 * st + key, t1 - 1)) * a.Gq + gq) * dim + 4 * grp;
+    f32x4 qf[DC], kf[DC];
+#pragma unroll
+    for (int c = 0; c < DC; ++c) {
+      qf[c] = load4f<FULL>(qrow + 16 * c, dim - 16 * c - 4 * grp, a.vec);
+      kf[c] = load4f<FULL>(krow + 16 * c, dim - 16 * c - 4 * grp, a.vec);
+    }
+    typedef double f64x4 __attribute__((ext_vector_type(4)));
+    f64x4 s = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int c = 0; c < DC; ++c)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        s = __builtin_amdgcn_mfma_f64_16x16x4f64(static_cast<double>(kf[c][j]), static_cast<double>(qf[c][j]), s, 0, 0, 0);
+    f32x4 r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = s[i];
+    *reinterpret_cast<f32x4*>(a.scores + ((static_cast<size_t>(id) * a.Gq + gq) * CT + 16 * rt + col) * CT + 16 * st + 4 * grp) = r;
+  }
+}
+
+// the value N lanes away in the row of 16 (1 from outside it)
+template <int CTRL>
+__device__ __forceinline__ double row_move(double x) {
+  const int lo = __builtin_amdgcn_update_dpp(__double2loint(1.0), __double2loint(x), CTRL, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(1.0), __double2hiint(x), CTRL, 0xf, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+template <int CTRL>
+__device__ __forceinline__ double row_mul(double x) { return x * row_move<CTRL>(x); }
+
 // DC: 16-wide tiles of key features (dim <= 16 DC).
-template <typename T, int DC, int OCC>
-__global__ __launch_bounds__(NTH, OCC) void retention_chunk_kernel(ChunkArgs a) {
+template <typename T, int DC, int VT, bool FULL>
+__global__ __launch_bounds__(NTH, DC <= 8 ? 2 : 1) void chunk_kernel(ChunkArgs a) {
   typedef typename Elem<T>::frag F;
-  constexpr int LDK = 16 * DC + 4, LDV = CT + 4, ND = (DC + 3) / 4;
-  __shared__ __attribute__((aligned(16))) float Ks[CT * LDK];   // [token][feature]
+  constexpr int LDK = 16 * DC + 4, LDV = CT + 4, ND = (DC + 3) / 4, NU = VT / 16;
   __shared__ __attribute__((aligned(16))) float Ss[VT * LDK];   // [value column][feature]
   __shared__ __attribute__((aligned(16))) T Vs[VT * LDV];       // [value column][token]
-  __shared__ float pw[CT + 1];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 15, grp = lane >> 4;
+  __shared__ __attribute__((aligned(16))) float gs[CT], bs[CT];
+  __shared__ double pre[CT], post[CT], whole[4];   // decay from a block's start to the token; that behind the token, times b; over a block
+  __shared__ int wild;   // some value was infinite or NaN: it must not reach earlier queries as 0 x value
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 15, grp = lane >> 4;
   const int b = blockIdx.x, h = blockIdx.y, v0 = blockIdx.z * VT;
   const int t0 = a.q_start[b], t1 = a.q_start[b + 1], sr = a.state_rows[b];
   if (t1 - t0 < MIN_LEN || sr < 0 || sr >= a.n_rows) return;
   const int gq = h / (a.H / a.Gq), dim = a.dim, vdim = a.vdim;
-  if (tid <= CT) {
-    const float g = a.decay[h];
-    float p = 1.0f;
-    for (int i = 0; i < tid; ++i) p *= g;
-    pw[tid] = p;
-  }
   float* Sg = a.state + (static_cast<size_t>(sr) * a.H + h) * dim * vdim + v0;
   const bool carry = a.positions[t0] != 0;
   const bool vec_s = (vdim & 3) == 0;
-  f32x4 S[ND][4];   // lane: S^T[value column 16 u + 4 grp + i][feature 16 (wave + 4 m) + col]
+  const int d0 = 16 * ND * wave + ND * col;   // this lane's features of the state: d0 .. d0 + ND - 1
+  const bool vec_k = FULL || (ND > 1 && a.vec && (dim & 3) == 0 && d0 + ND <= dim);
+  f32x4 S[ND][NU];   // lane: S^T[value column 16 u + 4 grp + i][feature d0 + m]
 #pragma unroll
-  for (int m = 0; m < ND; ++m) {
-    const int d = 16 * (wave + 4 * m) + col;
+  for (int m = 0; m < ND; ++m)
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
-      S[m][u] = (carry && d < dim) ? load4(Sg + static_cast<size_t>(d) * vdim + 16 * u + 4 * grp, vdim - v0 - 16 * u - 4 * grp, vec_s)
-                                   : f32x4{0.f, 0.f, 0.f, 0.f};
-  }
-  auto stage_state = [&]() {
+    for (int u = 0; u < NU; ++u)
+      S[m][u] = (carry && d0 + m < dim) ? load4(Sg + static_cast<size_t>(d0 + m) * vdim + 16 * u + 4 * grp, vdim - v0 - 16 * u - 4 * grp, vec_s)
+                                        : f32x4{0.f, 0.f, 0.f, 0.f};
+  const bool owner = 16 * ND * wave < dim;   // (wave-uniform) the wave has features
+  const int place = 16 * wave + col;         // this lane's query in a chunk
+
+  // ---- loads, one chunk ahead; rows past the segment repeat its last one and are masked where they are used ----
+  f32x4 qf[DC];
+  float kf[4][4][ND];
+  f32x4 rf[4];
+  uint32_t vf[NU][4];   // (bits; packed where they are staged: packing waits for the loads)
+  float gf, bf;
+  const T* vbase = static_cast<const T*>(a.v) + static_cast<size_t>(h) * vdim + v0;
+  const int v_col = tid % VT, v_tok = 4 * (tid / VT);
+  const uint32_t v_src = min(v_col, vdim - 1 - v0);   // (columns past the state repeat its last one and are not stored)
+  // (a chunk's rows start at a uniform address; a lane's place in the chunk is a 32-bit offset)
+  const uint32_t row = static_cast<uint32_t>(a.Gq) * dim, v_row = static_cast<uint32_t>(a.v_stride);
+  auto load_q = [&](int first) {
+    const float* base = a.q + static_cast<size_t>(first) * row + gq * dim;
+    const uint32_t o = min(place, t1 - 1 - first) * row + 4 * grp;
 #pragma unroll
-    for (int m = 0; m < ND; ++m) {
-      const int dt = wave + 4 * m;
-      if (dt < DC) {
+    for (int c = 0; c < DC; ++c) qf[c] = load4f<FULL>(base + (o + 16 * c), dim - 16 * c - 4 * grp, a.vec);
+  };
+  auto load_k = [&](int first, int tt) {
+    const float* base = a.k + static_cast<size_t>(first) * row + gq * dim;
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t o = min(16 * tt + 4 * grp + j, t1 - 1 - first) * row + d0;
+      if constexpr (ND > 1) {
+        typedef float fv __attribute__((ext_vector_type(ND)));
+        if (vec_k) {
+          const fv x = *reinterpret_cast<const fv*>(base + o);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) Ss[(16 * u + 4 * grp + i) * LDK + 16 * dt + col] = S[m][u][i];
+          for (int m = 0; m < ND; ++m) kf[tt][j][m] = x[m];
+          continue;
+        }
       }
+#pragma unroll
+      for (int m = 0; m < ND; ++m) kf[tt][j][m] = FULL || d0 + m < dim ? base[o + m] : 0.f;
+    }
+  };
+  auto load_r = [&](int first, int id) {
+    const float* base = a.scores + (static_cast<size_t>(id) * a.Gq + gq) * CT * CT;
+    const uint32_t o = place * CT + 4 * grp;
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt)
+      if (kt <= wave && first + 16 * wave < t1) rf[kt] = *reinterpret_cast<const f32x4*>(base + (o + 16 * kt));
+  };
+  auto load_v = [&](int first) {
+    const T* base = vbase + static_cast<size_t>(first) * a.v_stride;
+#pragma unroll
+    for (int p = 0; p < NU; ++p)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const T x = base[min(v_tok + p * (4 * NTH / VT) + j, t1 - 1 - first) * v_row + v_src];
+        if constexpr (sizeof(T) == 2) vf[p][j] = x; else vf[p][j] = __float_as_uint(x);
+      }
+    gf = 1.0f;
+    bf = 0.0f;
+    if (wave == 0 && first + lane < t1) {
+      gf = a.g[static_cast<size_t>(first + lane) * a.g_token + h];
+      bf = a.beta != nullptr ? a.beta[static_cast<size_t>(first + lane) * a.H + h] : 1.0f;
     }
   };
   auto value_frag = [&](int u, int tok) {   // V^T[value column 16 u + col][tokens tok .. tok + 3] as fp32
@@ -102,71 +220,115 @@ __global__ __launch_bounds__(NTH, OCC) void retention_chunk_kernel(ChunkArgs a) 
     }
     return r;
   };
-  stage_state();
-  const T* vbase = static_cast<const T*>(a.v) + static_cast<size_t>(h) * vdim + v0;
-  for (int first = t0; first < t1; first += CT) {
+  if (tid == 0) wild = 0;
+  __syncthreads();
+  int id = chunk_base(a.q_start, b);
+  load_v(t0);
+  load_q(t0);
+  load_r(t0, id);
+#pragma unroll
+  for (int tt = 0; tt < 4; ++tt) load_k(t0, tt);
+  for (int first = t0; first < t1; first += CT, ++id) {
     const int n = min(CT, t1 - first);
-    // ---- the chunk's keys and values; rows past the segment are zero ----
-    for (int e = tid; e < CT * 4 * DC; e += NTH) {
-      const int r = e / (4 * DC), f = 4 * (e - r * 4 * DC);
-      const f32x4 x = r < n ? load4(a.k + (static_cast<size_t>(first + r) * a.Gq + gq) * dim + f, dim - f, a.vec) : f32x4{0.f, 0.f, 0.f, 0.f};
-      *reinterpret_cast<f32x4*>(&Ks[r * LDK + f]) = x;
+    const bool more = first + CT < t1;
+    // ---- values, state and decays to LDS ----
+#pragma unroll
+    for (int p = 0; p < NU; ++p) {
+      F f;
+      bool odd = false;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t x = first + v_tok + p * (4 * NTH / VT) + j < t1 ? vf[p][j] : 0u;
+        if constexpr (sizeof(T) == 2) { f[j] = static_cast<short>(x); odd |= (x & 0x7F80u) == 0x7F80u; }
+        else { f[j] = __uint_as_float(x); odd |= (x & 0x7F800000u) == 0x7F800000u; }
+      }
+      *reinterpret_cast<F*>(&Vs[v_col * LDV + v_tok + p * (4 * NTH / VT)]) = f;
+      if (odd) wild = 1;
     }
+    if (owner) {
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      const int r = 16 * wave + 4 * p;
-      F f = zero_frag<T>();
+      for (int u = 0; u < NU; ++u)
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (r + j < n && v0 + lane < vdim) {
-          const T x = vbase[static_cast<size_t>(first + r + j) * a.v_stride + lane];
-          if constexpr (sizeof(T) == 2) f[j] = static_cast<short>(x); else f[j] = x;
-        }
-      *reinterpret_cast<F*>(&Vs[lane * LDV + r]) = f;
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int m = 0; m < ND; ++m)
+            if (DC % 4 == 0 || d0 + m < 16 * DC) Ss[(16 * u + 4 * grp + i) * LDK + d0 + m] = S[m][u][i];
     }
-    const int place = 16 * wave + col;   // this lane's query
-    f32x4 qf[DC];
-    {
-      const float* qrow = a.q + (static_cast<size_t>(first + min(place, n - 1)) * a.Gq + gq) * dim;
-#pragma unroll
-      for (int c = 0; c < DC; ++c) qf[c] = load4(qrow + 16 * c + 4 * grp, dim - 16 * c - 4 * grp, a.vec);
+    if (wave == 0) {   // lane = token
+      const double p = row_mul<0x118>(row_mul<0x114>(row_mul<0x112>(row_mul<0x111>(static_cast<double>(gf)))));   // row_shr 1, 2, 4, 8
+      const double s = row_mul<0x108>(row_mul<0x104>(row_mul<0x102>(row_mul<0x101>(static_cast<double>(gf)))));   // row_shl 1, 2, 4, 8
+      gs[lane] = gf;
+      bs[lane] = bf;
+      pre[lane] = p;
+      post[lane] = row_move<0x101>(s) * bf;
+      if (col == 15) whole[grp] = p;
     }
     __syncthreads();
-    const bool live = 16 * wave < n;   // (wave-uniform) some query of the wave
-    f32x4 o[4];
+    if (more) load_v(first + CT);
+    const double wh[4] = {whole[0], whole[1], whole[2], whole[3]};
+    f32x4 o[NU];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) o[u] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (live) {
-      if (carry || first > t0) {
+    for (int u = 0; u < NU; ++u) o[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (16 * wave < n) {
 #pragma unroll
-        for (int c = 0; c < DC; ++c)
+      for (int kt = 0; kt < 3; ++kt) {   // the blocks before the queries' own
+        if (kt < wave) {   // (wave-uniform)
+          double g = pre[place];
+          for (int k = kt + 1; k < wave; ++k) g *= wh[k];
+          f32x4 s;
 #pragma unroll
-          for (int u = 0; u < 4; ++u)
-            o[u] = mma16(*reinterpret_cast<const f32x4*>(&Ss[(16 * u + col) * LDK + 16 * c + 4 * grp]), qf[c], o[u]);
-        const float g = pw[place + 1];
+          for (int i = 0; i < 4; ++i) s[i] = rf[kt][i] * static_cast<float>(post[16 * kt + 4 * grp + i] * g);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) o[u] *= g;
+          for (int u = 0; u < NU; ++u) o[u] += mma16(value_frag(u, 16 * kt + 4 * grp), s, f32x4{0.f, 0.f, 0.f, 0.f});
+        }
       }
-      for (int kt = 0; kt <= wave; ++kt) {
-        f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0;   // (two chains)
+      // their own: the decay over tokens key + 1 .. query of the block
+      f32x4 s = wave == 0 ? rf[0] : wave == 1 ? rf[1] : wave == 2 ? rf[2] : rf[3];
+      {
+        double x = 1.0;
 #pragma unroll
-        for (int c = 0; c < DC; ++c) {
-          const f32x4 kf = *reinterpret_cast<const f32x4*>(&Ks[(16 * kt + col) * LDK + 16 * c + 4 * grp]);
-          if (c & 1) s1 = mma16(kf, qf[c], s1); else s0 = mma16(kf, qf[c], s0);
+        for (int t = 4; t < 16; ++t) x *= static_cast<double>((t >= 4 * grp + 4 && t <= col) ? gs[16 * wave + t] : 1.0f);
+        const f32x4 own = *reinterpret_cast<const f32x4*>(&gs[16 * wave + 4 * grp]);
+        const f32x4 be = *reinterpret_cast<const f32x4*>(&bs[16 * wave + 4 * grp]);
+#pragma unroll
+        for (int i = 3; i >= 0; --i) {
+          s[i] = 4 * grp + i <= col ? s[i] * (x * be[i]) : 0.f;
+          x *= static_cast<double>(4 * grp + i <= col ? own[i] : 1.0f);
         }
-        f32x4 s = s0 + s1;
+      }
+      if (!wild) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int back = place - (16 * kt + 4 * grp + i);
-          s[i] = back >= 0 ? s[i] * pw[back] : 0.f;
+        for (int u = 0; u < NU; ++u) o[u] += mma16(value_frag(u, 16 * wave + 4 * grp), s, f32x4{0.f, 0.f, 0.f, 0.f});
+      } else {   // (rare) key by key, masked
+#pragma unroll 1
+        for (int key = 0; key < 16; ++key) {
+          const float x = __shfl((key & 2) ? ((key & 1) ? s[3] : s[2]) : ((key & 1) ? s[1] : s[0]), (key >> 2) * 16 + col, 64);
+#pragma unroll
+          for (int u = 0; u < NU; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const float y = o[u][i] + x * Elem<T>::ld(Vs[(16 * u + 4 * grp + i) * LDV + 16 * wave + key]);
+              o[u][i] = key <= col ? y : o[u][i];
+            }
         }
+      }
+    }
+    if (more) load_r(first + CT, id + 1);
+    if (16 * wave < n) {
+      if (carry || first > t0) {   // S^T Q^T, in chains of one feature tile (one long chain rounds twice as much)
+        double gd = pre[place];
+        for (int k = 0; k < wave; ++k) gd *= wh[k];
+        const float g = gd;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) o[u] = mma16(value_frag(u, 16 * kt + 4 * grp), s, o[u]);
+        for (int u = 0; u < NU; ++u)
+#pragma unroll
+          for (int c = 0; c < DC; ++c)
+            o[u] += g * mma16(*reinterpret_cast<const f32x4*>(&Ss[(16 * u + col) * LDK + 16 * c + 4 * grp]), qf[c], f32x4{0.f, 0.f, 0.f, 0.f});
       }
       if (place < n) {
         float* orow = a.out + (static_cast<size_t>(first + place) * a.H + h) * vdim + v0;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < NU; ++u) {
           const int e = 16 * u + 4 * grp;
           if (vec_s && v0 + e + 3 < vdim) {
             *reinterpret_cast<f32x4*>(orow + e) = o[u];
@@ -178,42 +340,47 @@ __global__ __launch_bounds__(NTH, OCC) void retention_chunk_kernel(ChunkArgs a) 
         }
       }
     }
+    if (more) load_q(first + CT);
     // ---- the state behind the chunk ----
-    const float gn = pw[n];
+    if (owner) {
+      const float gn = (wh[0] * wh[1]) * (wh[2] * wh[3]);
 #pragma unroll
-    for (int m = 0; m < ND; ++m)
+      for (int m = 0; m < ND; ++m)
 #pragma unroll
-      for (int u = 0; u < 4; ++u) S[m][u] *= gn;
-    for (int tt = 0; 16 * tt < n; ++tt) {
-      f32x4 vf[4];
+        for (int u = 0; u < NU; ++u) S[m][u] *= gn;
 #pragma unroll
-      for (int u = 0; u < 4; ++u) vf[u] = value_frag(u, 16 * tt + 4 * grp);
-      float w[4];
+      for (int tt = 0; tt < 4; ++tt) {
+        if (16 * tt < n) {   // (uniform)
+          double g = 1.0;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) w[j] = pw[max(n - 1 - (16 * tt + 4 * grp + j), 0)];   // (keys past the segment are zero)
+          for (int k = tt + 1; k < 4; ++k) g *= wh[k];
+          float w[4];
 #pragma unroll
-      for (int m = 0; m < ND; ++m) {
-        const int dt = wave + 4 * m;
-        if (dt < DC) {
-          f32x4 kf;
+          for (int j = 0; j < 4; ++j) w[j] = post[16 * tt + 4 * grp + j] * g;
+          f32x4 x[NU];
 #pragma unroll
-          for (int j = 0; j < 4; ++j) kf[j] = Ks[(16 * tt + 4 * grp + j) * LDK + 16 * dt + col] * w[j];
+          for (int u = 0; u < NU; ++u) x[u] = value_frag(u, 16 * tt + 4 * grp);
 #pragma unroll
-          for (int u = 0; u < 4; ++u) S[m][u] = mma16(vf[u], kf, S[m][u]);
+          for (int m = 0; m < ND; ++m) {
+            f32x4 kw;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) kw[j] = 16 * tt + 4 * grp + j < n ? kf[tt][j][m] * w[j] : 0.f;
+#pragma unroll
+            for (int u = 0; u < NU; ++u) S[m][u] += mma16(x[u], kw, f32x4{0.f, 0.f, 0.f, 0.f});
+          }
         }
+        if (more) load_k(first + CT, tt);
       }
     }
     __syncthreads();   // every reader of the chunk and of the old state is done
-    if (first + CT < t1) stage_state();
   }
 #pragma unroll
   for (int m = 0; m < ND; ++m) {
-    const int d = 16 * (wave + 4 * m) + col;
-    if (d >= dim) continue;
+    if (d0 + m >= dim) continue;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
+    for (int u = 0; u < NU; ++u) {
       const int e = 16 * u + 4 * grp;
-      float* p = Sg + static_cast<size_t>(d) * vdim + e;
+      float* p = Sg + static_cast<size_t>(d0 + m) * vdim + e;
       if (vec_s && v0 + e + 3 < vdim) {
         *reinterpret_cast<f32x4*>(p) = S[m][u];
       } else {
@@ -225,36 +392,60 @@ __global__ __launch_bounds__(NTH, OCC) void retention_chunk_kernel(ChunkArgs a) 
   }
 }
 
-template <typename T>
-int launch_chunks(const ChunkArgs& a, int B, hipStream_t s) {
-  const dim3 grid(B, a.H, (a.vdim + VT - 1) / VT);
-  if (a.dim <= 32) retention_chunk_kernel<T, 2, 2><<<grid, NTH, 0, s>>>(a);
-  else if (a.dim <= 64) retention_chunk_kernel<T, 4, 2><<<grid, NTH, 0, s>>>(a);
-  else if (a.dim <= 128) retention_chunk_kernel<T, 8, sizeof(T) == 2 ? 2 : 1><<<grid, NTH, 0, s>>>(a);
-  else retention_chunk_kernel<T, 16, 1><<<grid, NTH, 0, s>>>(a);
+template <typename T, int DC, bool FULL>
+int launch_chunks(const ChunkArgs& a, int n_chunks, hipStream_t s) {
+  scores_kernel<DC, FULL><<<dim3(n_chunks, a.Gq), NTH, 0, s>>>(a);
+  // 64 value columns per workgroup where that gives every CU two, else fewer: the walk is serial, idle CUs cost nothing
+  // (96 workgroups of 64 columns -> 384 of 16: 140 us -> 75, 3 segments of 700)
+  const int64_t wide = static_cast<int64_t>(a.B) * a.H * ((a.vdim + 63) / 64);
+  if (wide >= 512) chunk_kernel<T, DC, 64, FULL><<<dim3(a.B, a.H, (a.vdim + 63) / 64), NTH, 0, s>>>(a);
+  else if (wide >= 256) chunk_kernel<T, DC, 32, FULL><<<dim3(a.B, a.H, (a.vdim + 31) / 32), NTH, 0, s>>>(a);
+  else chunk_kernel<T, DC, 16, FULL><<<dim3(a.B, a.H, (a.vdim + 15) / 16), NTH, 0, s>>>(a);
   return BCG_CHECK_LAUNCH();
+}
+
+template <typename T, int DC>
+int launch_full(const ChunkArgs& a, int n_chunks, hipStream_t s) {
+  if constexpr (sizeof(T) == 2) {
+    if (a.vec && a.dim == 16 * DC) return launch_chunks<T, DC, true>(a, n_chunks, s);
+  }
+  return launch_chunks<T, DC, false>(a, n_chunks, s);
+}
+
+template <typename T>
+int launch_dim(const ChunkArgs& a, int n_chunks, hipStream_t s) {
+  if (a.dim <= 32) return launch_full<T, 2>(a, n_chunks, s);
+  if (a.dim <= 64) return launch_full<T, 4>(a, n_chunks, s);
+  if (a.dim <= 128) return launch_full<T, 8>(a, n_chunks, s);
+  return launch_full<T, 16>(a, n_chunks, s);
 }
 
 }  // namespace
 
-// Segments shorter than this are left alone by `bcg_retention_chunks`.
-BCG_API int bcg_retention_min_len() { return MIN_LEN; }
+// Segments shorter than this are left alone by `bcg_decay_chunks`.
+BCG_API int bcg_decay_chunks_min_len() { return MIN_LEN; }
 
-BCG_API int bcg_retention_chunks(const void* q32, const void* k32, const void* decay, const void* v, int64_t v_stride,
-                                 const void* positions, const void* q_start, const void* state_rows, void* state, int n_rows,
-                                 void* out, int B, int H, int Gq, int dim, int vdim, int is_f32, void* stream) {
-  if (B <= 0) return 0;
-  if (dim < 1 || dim > 256 || vdim < 1 || H <= 0 || Gq <= 0 || H % Gq || H > 65535 || (vdim + VT - 1) / VT > 65535) return -2;
+// `scores` takes (T / tokens + B) Gq tokens^2 fp32 elements
+BCG_API int bcg_decay_chunks_tokens() { return CT; }
+
+// g: [H] (g_token 0) or [T, H] (g_token H); beta [T, H] or null.
+BCG_API int bcg_decay_chunks(const void* q32, const void* k32, const void* g, int g_token, const void* beta, const void* v,
+                             int64_t v_stride, const void* positions, const void* q_start, const void* state_rows, void* state,
+                             int n_rows, void* out, void* scores, int T_, int B, int H, int Gq, int dim, int vdim, int is_f32,
+                             void* stream) {
+  if (B <= 0 || T_ <= 0) return 0;
+  if (dim < 1 || dim > 256 || vdim < 1 || H <= 0 || Gq <= 0 || H % Gq || H > 65535 || (vdim + 15) / 16 > 65535) return -2;
   auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-  if (!al16(state) || !al16(out)) return -2;
+  if (!al16(state) || !al16(out) || !al16(scores) || scores == nullptr || (g_token != 0 && g_token != H)) return -2;
   ChunkArgs a;
-  a.q = static_cast<const float*>(q32); a.k = static_cast<const float*>(k32); a.decay = static_cast<const float*>(decay);
+  a.q = static_cast<const float*>(q32); a.k = static_cast<const float*>(k32);
+  a.g = static_cast<const float*>(g); a.g_token = g_token; a.beta = static_cast<const float*>(beta);
   a.v = v; a.v_stride = v_stride;
   a.positions = static_cast<const int*>(positions); a.q_start = static_cast<const int*>(q_start);
   a.state_rows = static_cast<const int*>(state_rows);
-  a.state = static_cast<float*>(state); a.out = static_cast<float*>(out);
-  a.n_rows = n_rows; a.H = H; a.Gq = Gq; a.dim = dim; a.vdim = vdim;
+  a.state = static_cast<float*>(state); a.out = static_cast<float*>(out); a.scores = static_cast<float*>(scores);
+  a.n_rows = n_rows; a.B = B; a.H = H; a.Gq = Gq; a.dim = dim; a.vdim = vdim;
   a.vec = dim % 4 == 0 && al16(q32) && al16(k32);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  return is_f32 ? launch_chunks<float>(a, B, s) : launch_chunks<bf16_t>(a, B, s);
+  return is_f32 ? launch_dim<float>(a, T_ / CT + B, s) : launch_dim<bf16_t>(a, T_ / CT + B, s);
 }
