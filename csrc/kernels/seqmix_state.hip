@@ -197,7 +197,40 @@ __global__ __launch_bounds__(NT) void short_conv_vec_kernel(const T* __restrict_
     for (int j = 0; j < TAPS; ++j) wr[e][j] = w[static_cast<size_t>(c + e) * TAPS + j];
   }
   const int t_end = min(T_, (static_cast<int>(blockIdx.x) + 1) * rows);
-  for (int t = blockIdx.x * rows; t < t_end; ++t) {
+  const int t_first = blockIdx.x * rows;
+  auto finish = [&](const float (&acc)[VEC], int t) {
+    Vec o;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      const float v = act == 1 ? acc[e] * sigmoidf_(acc[e]) : acc[e];
+      o.e[e] = Elem<T>::st(v);
+    }
+    *reinterpret_cast<Vec*>(out + static_cast<size_t>(t) * C + c) = o;
+  };
+  // CONV_ROWS rows deep inside one segment: every input once, all loads in flight at once (row by row each waits for its
+  // segment's tables; 8183 rows of 8448 channels: 144 -> 103 us)
+  if (t_end - t_first == CONV_ROWS) {
+    const int seg = token_seq[t_first];
+    if (token_seq[t_end - 1] == seg && t_first - q_start[seg] >= TAPS - 1) {
+      Vec u[CONV_ROWS + TAPS - 1];
+#pragma unroll
+      for (int r = 0; r < CONV_ROWS + TAPS - 1; ++r)
+        u[r] = *reinterpret_cast<const Vec*>(y + static_cast<size_t>(t_first + r - (TAPS - 1)) * y_stride + c);
+#pragma unroll
+      for (int r = 0; r < CONV_ROWS; ++r) {
+        float acc[VEC];
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+          acc[e] = br[e];
+#pragma unroll
+          for (int j = 0; j < TAPS; ++j) acc[e] += wr[e][j] * Elem<T>::ld(u[r + j].e[e]);
+        }
+        finish(acc, t_first + r);
+      }
+      return;
+    }
+  }
+  for (int t = t_first; t < t_end; ++t) {
     const int seg = token_seq[t], off = t - q_start[seg], pos = positions[t];
     const int sr = state_rows[seg];
     const bool row_ok = sr >= 0 && sr < n_rows;
@@ -216,13 +249,7 @@ __global__ __launch_bounds__(NT) void short_conv_vec_kernel(const T* __restrict_
         for (int e = 0; e < VEC; ++e) acc[e] += wr[e][j] * Elem<T>::ld(u.e[e]);
       }
     }
-    Vec o;
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) {
-      const float v = act == 1 ? acc[e] * sigmoidf_(acc[e]) : acc[e];
-      o.e[e] = Elem<T>::st(v);
-    }
-    *reinterpret_cast<Vec*>(out + static_cast<size_t>(t) * C + c) = o;
+    finish(acc, t);
   }
 }
 
@@ -601,6 +628,14 @@ __global__ __launch_bounds__(NT) void retention_prepare_kernel(const T* __restri
   }
 }
 
+// Sum over LANES neighbouring lanes (a power of two), the result in each of them.
+template <int LANES>
+__device__ __forceinline__ float lanes_sum(float x) {
+#pragma unroll
+  for (int d = 1; d < LANES; d *= 2) x += __shfl_xor(x, d, 64);
+  return x;
+}
+
 // Gated delta rule.  One block per token: q / k heads (G of them, from the convolved row c) become
 // unit vectors x / sqrt(sum x^2 + 1e-6), q also times dim^-1/2; beta = sigmoid(y[off_beta + h]);
 // decay g[h, i] = exp(-exp(a_log[h]) softplus(a[h, i] + dt_bias[h, i])), i < gd: gd = dim (a decay per
@@ -616,6 +651,24 @@ __global__ __launch_bounds__(NT) void delta_prepare_kernel(const T* __restrict__
   const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const T* crow = c + static_cast<size_t>(t) * c_stride;
   const float qs = 1.0f / sqrtf(static_cast<float>(dim));
+  // whole aligned quads, up to 128 wide: 32 lanes a vector (8183 rows of 16 + 16 vectors of 128: 43 us; a wave a vector, single
+  // columns and two passes: 103)
+  if (dim % 4 == 0 && dim <= 128 && c_stride % 4 == 0 &&
+      ((reinterpret_cast<uintptr_t>(c) | reinterpret_cast<uintptr_t>(q32) | reinterpret_cast<uintptr_t>(k32)) & 15) == 0) {
+    typedef T T4 __attribute__((ext_vector_type(4)));
+    const int l = threadIdx.x & 31, i = 4 * l;
+    for (int v = threadIdx.x >> 5; v < 2 * G; v += NT / 32) {
+      f32x4 x = {0.f, 0.f, 0.f, 0.f};
+      if (i < dim) {
+        const T4 e = *reinterpret_cast<const T4*>(crow + static_cast<size_t>(v) * dim + i);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x[j] = Elem<T>::ld(e[j]);
+      }
+      const float r = (v < G ? qs : 1.0f) / sqrtf(lanes_sum<32>((x[0] * x[0] + x[1] * x[1]) + (x[2] * x[2] + x[3] * x[3])) + 1e-6f);
+      float* o = (v < G ? q32 : k32) + (static_cast<size_t>(t) * G + (v < G ? v : v - G)) * dim;
+      if (i < dim) *reinterpret_cast<f32x4*>(o + i) = x * r;
+    }
+  } else
   for (int v = wave; v < 2 * G; v += NT / 64) {           // vector v: q heads, then k heads
     const T* x = crow + static_cast<size_t>(v) * dim;
     float s = 0.f;
@@ -846,6 +899,74 @@ __global__ __launch_bounds__(NT) void head_norm_gate_kernel(const float* __restr
   }
 }
 
+// The same without a normaliser column, four columns per access and LANES lanes per head (4 LANES >= vdim / NQ), a head's
+// values in registers.  Needs vdim and the gate's stride to be multiples of 4 and every pointer 16-byte aligned.  Bound by
+// memory: 8183 rows of 32 heads of 128: 63 us (160 with a wave per head, single columns and two passes).
+template <typename T, int LANES, int NQ>
+__global__ __launch_bounds__(NT) void head_norm_gate_vec_kernel(const float* __restrict__ o, const float* __restrict__ w, float eps,
+                                                                const T* __restrict__ gate, int64_t gate_stride,
+                                                                T* __restrict__ out, int64_t n_heads_total, int H, int vdim,
+                                                                int gate_kind, int w_head) {
+  typedef T T4 __attribute__((ext_vector_type(4)));
+  const int l = threadIdx.x % LANES;
+  const int64_t th = static_cast<int64_t>(blockIdx.x) * (NT / LANES) + threadIdx.x / LANES;
+  if (th >= n_heads_total) return;   // (whole groups of lanes)
+  const int64_t t = th / H;
+  const int h = static_cast<int>(th - t * H);
+  const T* grow = gate != nullptr ? gate + t * gate_stride + static_cast<int64_t>(h) * vdim : nullptr;
+  f32x4 x[NQ];
+  T4 g[NQ];
+  float s = 0.f;
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    const int e = 4 * (l + q * LANES);
+    x[q] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (e < vdim) {
+      x[q] = *reinterpret_cast<const f32x4*>(o + th * vdim + e);
+      if (gate != nullptr) g[q] = *reinterpret_cast<const T4*>(grow + e);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) s += x[q][j] * x[q][j];
+  }
+  const float r = 1.0f / sqrtf(lanes_sum<LANES>(s) / vdim + eps);
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    const int e = 4 * (l + q * LANES);
+    if (e < vdim) {
+      f32x4 v = x[q] * r;
+      if (w != nullptr) v *= *reinterpret_cast<const f32x4*>(w + h * w_head + e);
+      T4 y;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (gate != nullptr) {
+          const float z = Elem<T>::ld(g[q][j]);
+          v[j] *= gate_kind == 0 ? sigmoidf_(z) : z * sigmoidf_(z);
+        }
+        y[j] = Elem<T>::st(v[j]);
+      }
+      *reinterpret_cast<T4*>(out + th * vdim + e) = y;
+    }
+  }
+}
+
+template <typename T>
+bool launch_head_norm_vec(const float* o, const float* w, float eps, const T* gate, int64_t gate_stride, T* out, int64_t n, int H,
+                          int vdim, int gate_kind, const float* floor_, int w_head, hipStream_t s) {
+  const uintptr_t bits = reinterpret_cast<uintptr_t>(o) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(gate) |
+                         reinterpret_cast<uintptr_t>(out);
+  if (floor_ != nullptr || vdim % 4 || gate_stride % 4 || bits % 16 || vdim > 1024) return false;
+#define BCG_HNG(LANES, NQ)                                                                                                    \
+  head_norm_gate_vec_kernel<T, LANES, NQ><<<static_cast<int>((n + NT / LANES - 1) / (NT / LANES)), NT, 0, s>>>(               \
+      o, w, eps, gate, gate_stride, out, n, H, vdim, gate_kind, w_head)
+  if (vdim <= 64) BCG_HNG(16, 1);
+  else if (vdim <= 128) BCG_HNG(32, 1);
+  else if (vdim <= 256) BCG_HNG(64, 1);
+  else if (vdim <= 512) BCG_HNG(64, 2);
+  else BCG_HNG(64, 4);
+#undef BCG_HNG
+  return true;
+}
+
 template <typename T, bool DELTA>
 int launch_scan(const ScanArgs& a, int B, hipStream_t s) {
   dim3 grid(B, a.H, (a.vdim + 8 * SCAN_WAVES - 1) / (8 * SCAN_WAVES));
@@ -1066,11 +1187,17 @@ BCG_API int bcg_head_norm_gate(const void* o32, const void* w, float eps, const 
   const int64_t n = static_cast<int64_t>(T_) * H;
   const int grid = static_cast<int>((n + NT / 64 - 1) / (NT / 64));
   const float *o = static_cast<const float*>(o32), *wf = static_cast<const float*>(w);
+  const float* fl = static_cast<const float*>(floor_);
+  if (is_f32 ? launch_head_norm_vec<float>(o, wf, eps, static_cast<const float*>(gate), gate_stride, static_cast<float*>(out), n, H, vdim,
+                                           gate_kind, fl, w_head, s)
+             : launch_head_norm_vec<bf16_t>(o, wf, eps, static_cast<const bf16_t*>(gate), gate_stride, static_cast<bf16_t*>(out), n, H,
+                                            vdim, gate_kind, fl, w_head, s))
+    return BCG_CHECK_LAUNCH();
   BCG_BY_TYPE((head_norm_gate_kernel<float><<<grid, NT, 0, s>>>(o, wf, eps, static_cast<const float*>(gate), gate_stride,
                                                                static_cast<float*>(out), n, H, vdim, gate_kind,
-                                                               static_cast<const float*>(floor_), w_head)),
+                                                               fl, w_head)),
               (head_norm_gate_kernel<bf16_t><<<grid, NT, 0, s>>>(o, wf, eps, static_cast<const bf16_t*>(gate), gate_stride,
                                                                 static_cast<bf16_t*>(out), n, H, vdim, gate_kind,
-                                                                static_cast<const float*>(floor_), w_head)));
+                                                                fl, w_head)));
   return BCG_CHECK_LAUNCH();
 }

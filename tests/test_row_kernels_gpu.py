@@ -125,3 +125,64 @@ def test_fp8_rows(ops, T, I):
         torch.testing.assert_close(a[1], b[1], rtol=2 ** -7, atol=0)
         back, want = a[0].float() * a[1][:, None], b[0].float() * b[1][:, None]
         assert ((back - want).norm() / want.norm()).item() < 0.02
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("H,vdim", [(3, 4), (2, 64), (5, 68), (4, 128), (3, 132), (2, 256), (2, 260), (1, 1024), (1, 1028), (3, 66)])
+@pytest.mark.parametrize("form", ["plain", "gated", "offset", "whole-row weight"])
+def test_head_norm_rows(ops, dtype, H, vdim, form):
+    g = torch.Generator(device="cuda").manual_seed(vdim)
+    r = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    T = 7
+    o, w = r(T, H, vdim), r(H * vdim if form == "whole-row weight" else vdim)
+    gate = None if form == "plain" else r(T, H * vdim + 8).to(dtype)[:, (2 if form == "offset" else 8):][:, :H * vdim]
+    for act in ("sigmoid", "silu"):
+        a = (o, None if form == "plain" else w, 1e-5, gate, dtype, act)
+        torch.testing.assert_close(ops.head_norm_gate(*a), ref.head_norm_gate(*a), **_tol(dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("H,vdim,parts", [(2, 4, 2), (16, 64, 1), (17, 64, 1), (33, 64, 1), (65, 64, 1), (129, 64, 1), (4, 66, 2), (130, 64, 2)])
+def test_gated_group_rows(ops, dtype, H, vdim, parts):
+    g = torch.Generator(device="cuda").manual_seed(H)
+    r = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    T, n = 5, H * vdim
+    for off in (0, 2):
+        a = (r(T, H, vdim), r(T, n + 8).to(dtype)[:, off:off + n], r(H), r(T, n + 4).to(dtype)[:, :n], r(n), parts, 1e-5, dtype)
+        torch.testing.assert_close(ops.gated_group_norm(*a), ref.gated_group_norm(*a), **_tol(dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("W", [4, 1020, 2052, 2050])
+def test_embed_dyt_rows(ops, dtype, W):
+    table, w, b = torch.randn(50, W, device="cuda").to(dtype), torch.randn(W, device="cuda"), torch.randn(W, device="cuda")
+    tokens = torch.randint(0, 50, (5,), device="cuda", dtype=torch.int32)
+    a = (tokens, table, 0.7, (0.8, w, b), dtype)
+    for x, y in zip(ops.embed_scale_dyt(*a), ref.embed_scale_dyt(*a)):
+        torch.testing.assert_close(x, y, **_tol(dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("taps", [2, 3, 4])
+def test_short_conv_blocks_of_rows(ops, dtype, taps):
+    """Large steps: blocks of rows inside a segment, over a boundary, at a segment's first rows, a continued segment."""
+    from test_decay_chunks_gpu import _meta
+    lens, starts, C = [1001, 1, 2, 7, 1040, 9], [0, 4, 0, 3, 11, 0], 40
+    meta, T = _meta(lens, starts, "cuda"), sum(lens)
+    y = torch.randn(T, C + 8, device="cuda").to(dtype)
+    w, b = torch.randn(C, taps, device="cuda"), torch.randn(C, device="cuda")
+    sa = torch.randn(len(lens) + 2, taps - 1, C, device="cuda").to(dtype)
+    sb = sa.clone()
+    torch.testing.assert_close(ops.short_conv(y, C, w, meta, sa, "silu", b), ref.short_conv(y, C, w, meta, sb, "silu", b), **_tol(dtype))
+    torch.testing.assert_close(sa, sb, rtol=0, atol=0)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("H,G,dim", [(2, 1, 4), (6, 3, 100), (4, 2, 128), (2, 2, 132), (2, 1, 30)])
+def test_delta_prepare_rows(ops, dtype, H, G, dim):
+    T = 5
+    r = lambda *s: torch.randn(*s, device="cuda")  # noqa: E731
+    c, y, a = r(T, 2 * G * dim + 8).to(dtype), r(T, H + 3).to(dtype), r(T, H).to(dtype)
+    args = (c, y, 2, a, r(H), r(H), H, G, dim)
+    for x, z in zip(ops.delta_prepare(*args), ref.delta_prepare(*args)):
+        torch.testing.assert_close(x, z, rtol=2e-5, atol=1e-5)
