@@ -28,6 +28,7 @@ TILES = ((128, 128), (64, 128), (128, 64), (256, 128), (64, 256), (64, 64), (32,
 PP_CFG = 10  # csrc/kernels/gemm_pp.hip: 256 x 256 ping-pong tile, N only a multiple of 16
 W4_CFG = 11  # csrc/kernels/gemm_w4.hip: 256 x 256, four 128 x 128 waves (one per SIMD), LDS-DMA fed
 BIG_CFGS = (PP_CFG, W4_CFG)  # 256 x 256 tiles (the register-staged form lost its A/B: csrc/experimental/gemm_rs.hip)
+SMALL_CFG = 5  # 64 x 64
 N_CFGS = len(TILES)
 SPLITS = (1, 2, 3, 4, 6, 8)
 CUS = 256
@@ -118,6 +119,27 @@ class GemmPlan:
             return None
         cfg = self.default_cfg(M)
         return (cfg, 1) if self.supported(cfg, M, N, K, epi) else None
+
+    def columns(self, M: int, N: int, K: int) -> int:
+        """Gated projections (epilogue 1) below LARGE_M rows: how many of the N columns run as whole rounds of 256 x 256
+        tiles, the others in 64 x 64 tiles behind them; N: no split.
+
+        A decode step's rows make few tiles, and one round and a sixteenth costs two: 448 x 34816 x 5120 (272 tiles) took 217
+        us, as one round (125) and the last 2048 columns in 224 small tiles (35) 165 to 172; 352 rows 175 -> 162, 512: 195 -> 176;
+        768 x 22528 x 5120: 186 -> 162.  Taken where the rounds are at least 0.94 full, the rest is at most one small
+        tile per CU (0.43 us per 64 of K against 1.46 for a round) and the rows fill 0.65 of their tiles (300 x 33792 x
+        4096: 126 -> 129)."""
+        if self.mode != "1" or not 256 < M < LARGE_M or N % 256 or not self.supported(W4_CFG, M, N, K, 1):
+            return N
+        n_t, m_t = N // 256, -(-M // 256)
+        rounds, rest = divmod(m_t * n_t, CUS)
+        n1 = rounds * CUS // m_t
+        if not (rounds and rest) or n1 * m_t < 0.94 * rounds * CUS or M < 0.65 * 256 * m_t:
+            return N
+        N2 = N - 256 * n1
+        if -(-M // 64) * (N2 // 64) > CUS or not self.supported(SMALL_CFG, M, N2, K, 1):
+            return N
+        return 256 * n1
 
     def pieces(self, M: int, N: int, K: int, epi: int) -> List[Tuple[int, Optional[Tuple[int, int]]]]:
         """[(rows, choice)]: how the M rows run, one choice for all of them or two runs of rows.

@@ -438,7 +438,7 @@ def hip_ops() -> SimpleNamespace:
             return torch.nn.functional.linear(x, w, bias)
         return torch.mm(x, w.t(), out=out) if bias is None else torch.addmm(bias, x, w.t(), out=out)
 
-    from .gemm_plan import PP_CFG, W4_CFG, GemmPlan
+    from .gemm_plan import PP_CFG, SMALL_CFG, W4_CFG, GemmPlan
     plan = GemmPlan(lib)
 
     # Split-K arrival counters (one int per output tile; the last-arriving workgroup of a
@@ -532,7 +532,16 @@ def hip_ops() -> SimpleNamespace:
             return _gemm_skinny(x, w, 1)
         if not (x.is_contiguous() and x.dtype == torch.bfloat16):
             return silu_mul(linear(x, w, _epi_log=1))
-        parts, N = _pieces(x, w, 1), w.shape[0]
+        N = w.shape[0]
+        n1 = plan.columns(M, N, K) if _plain(x, w) else N
+        if n1 < N:
+            out = torch.empty(M, N // 2, dtype=x.dtype, device=x.device)
+            for cfg, at, n in ((W4_CFG, 0, n1), (SMALL_CFG, n1, N - n1)):   # both halves of w from row at / 2 on
+                _log(M, n, K, 1, (cfg, 1))
+                _check(lib.bcg_gemm_nt(cfg, 1, _p(x), w.data_ptr() + at * K, None, None, out.data_ptr() + at, None, None, M, n, K, N // 2,
+                                       1, _stream()), "gemm_nt")   # (at / 2 rows or features of 2 bytes)
+            return out
+        parts = _pieces(x, w, 1)
         if len(parts) == 1 and parts[0][1] is None:
             return silu_mul(linear(x, w, _epi_log=1))
         out, at = torch.empty(M, N // 2, dtype=x.dtype, device=x.device), 0

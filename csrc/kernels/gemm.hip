@@ -412,7 +412,8 @@ BCG_API int bcg_gemm_num_cfgs() { return N_CFG + 2; }
 // split_k > 1: fp32 partial tiles in `ws` (>= m_tiles*n_tiles*split_k*BM*BN floats) and one
 // zero-initialised int counter per output tile in `counters` (left zeroed by every launch).
 // Requirements (checked by the caller): K % 64 == 0, K/64 >= split_k; N % BN == 0; EPI 1:
-// N == 2*inter and inter % (BN/2) == 0; all pointers 16-B aligned, rows contiguous.
+// N <= 2*inter (less: N / 2 features from w's first row on, the up rows inter behind the gate rows, rows of `c` inter
+// apart) and inter % (BN/2) == 0; all pointers 16-B aligned, rows contiguous.
 BCG_API int bcg_gemm_nt(int cfg, int epi, const void* x, const void* w, const void* bias, const void* residual,
                         void* c, void* ws, void* counters, int M, int N, int K, int inter, int split_k,
                         hipStream_t stream) {
@@ -428,7 +429,7 @@ BCG_API int bcg_gemm_nt(int cfg, int epi, const void* x, const void* w, const vo
   switch (epi) {
     case EPI_STORE: return dispatch<EPI_STORE>(cfg, x, w, bias, residual, c, wsf, cnt, M, N, K, inter, split_k, stream);
     case EPI_SILU_MUL:
-      if (N != 2 * inter || inter % (bn / 2)) return -2;
+      if (N > 2 * inter || inter % (bn / 2)) return -2;   // (N < 2 inter: N / 2 features from the first row of w on, up rows still inter behind)
       return dispatch<EPI_SILU_MUL>(cfg, x, w, nullptr, nullptr, c, wsf, cnt, M, N, K, inter, split_k, stream);
     case EPI_RESIDUAL:
       if (!residual) return -2;

@@ -1081,7 +1081,7 @@ BCG_API int bcg_gemm_w4_stamps(void* host, int n) {
 
 // Same contract as bcg_gemm_pp: epi 0 = store (+bias), 1 = silu(gate)*up into [M, inter],
 // 2 = residual + acc.  K % 64 == 0, K/64 >= split_k; N % 16 == 0 (a partial last n-tile is
-// masked); EPI 1: N == 2*inter, inter % 128 == 0.  split_k > 1: `ws` >= m_tiles*n_tiles*
+// masked); EPI 1: N == 2*inter (or less: the first N / 2 features, N % 256 == 0), inter % 128 == 0.  split_k > 1: `ws` >= m_tiles*n_tiles*
 // split_k*65536 floats, `counters` = 65536 ints, zeroed before first use (the last arriver of
 // each tile leaves its counter zeroed).
 // split_k == 0: stream-K (one workgroup per CU over the tiles x K-tiles units): `ws` >=
@@ -1106,7 +1106,7 @@ BCG_API int bcg_gemm_w4(int epi, const void* x, const void* w, const void* bias,
   switch (epi) {
     case EPI_STORE: return launch_w4<EPI_STORE>(x, w, bias, residual, c, wsf, cnt, M, N, K, inter, split_k, stream);
     case EPI_SILU_MUL:
-      if (N != 2 * inter || inter % 128) return -2;
+      if (N > 2 * inter || inter % 128 || (N != 2 * inter && N % BN)) return -2;   // (N < 2 inter: the first N / 2 features)
       return launch_w4<EPI_SILU_MUL>(x, w, nullptr, nullptr, c, wsf, cnt, M, N, K, inter, split_k, stream);
     case EPI_RESIDUAL:
       if (!residual) return -2;

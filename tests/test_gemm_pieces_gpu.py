@@ -56,3 +56,26 @@ def test_operands_that_do_not_lie_so():
     xg = x.clone().requires_grad_()
     ops.linear(xg, w).float().sum().backward()
     assert off(xg.grad, w.float().sum(0).expand(M, K)) < 2 ** -7
+
+
+# M, N, K, columns of the whole rounds (N: one launch)
+COLUMNS = [(448, 34816, 512, 32768), (333, 34816, 64, 32768), (300, 34816, 64, 34816), (512, 33792, 128, 32768), (600, 22528, 256, 21760),
+           (768, 22016, 192, 21760), (448, 32768, 128, 32768), (256, 66048, 64, 66048), (600, 24576, 128, 24576), (448, 34832, 64, 34832)]
+
+
+@pytest.mark.parametrize("M,N,K,n1", COLUMNS)
+def test_columns(M, N, K, n1):
+    from byzantine_consensus_llm_agents_amd.ops import get_ops
+    ops = get_ops("hip")
+    if ops.gemm_plan.mode != "1":
+        pytest.skip("BCG_HAND_GEMM")
+    assert ops.gemm_plan.columns(M, N, K) == n1
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    x = torch.randn(M, K, device="cuda", generator=g).bfloat16()
+    w = (torch.randn(N, K, device="cuda", generator=g) * K ** -0.5).bfloat16()
+    y = (x.float() @ w.float().t()).double()
+    want = torch.nn.functional.silu(y[:, :N // 2]) * y[:, N // 2:]
+    got = ops.linear_silu(x, w)
+    assert ((got.double() - want).norm() / want.norm()).item() < 2 ** -7
+    # the last features alone (the rest's tiles)
+    assert ((got[:, -64:].double() - want[:, -64:]).norm() / want[:, -64:].norm()).item() < 2 ** -7

@@ -1,0 +1,55 @@
+"""The rules that split a projection into runs of rows or columns (`GemmPlan.pieces`, `GemmPlan.columns`), over random
+shapes without a GPU: every row and column is covered once, each run is one that its kernel supports, and
+shapes that the general path takes alone still do."""
+import random
+
+import pytest
+
+from byzantine_consensus_llm_agents_amd.ops.gemm_plan import CUS, LARGE_M, SMALL_CFG, W4_CFG, GemmPlan
+
+
+def _shapes(n):
+    rng = random.Random(3)
+    for _ in range(n):
+        yield (rng.choice([1, 16, 17, 255, 256, 257, 448, 512, 700, 1024, 2047, 2048, 2049, 4449, 8183, 16384, rng.randint(1, 20000)]),
+               rng.choice([16, 64, 1792, 4096, 5056, 22528, 24576, 34816, 16 * rng.randint(1, 3000), 256 * rng.randint(1, 200), rng.randint(1, 40000)]),
+               rng.choice([64, 896, 4096, 5120, 17408, 64 * rng.randint(1, 300), rng.randint(1, 9000)]), rng.choice([0, 1, 2]))
+
+
+def test_runs_of_rows():
+    plan = GemmPlan()
+    plan.mode = "1"
+    split = 0
+    for M, N, K, epi in _shapes(20000):
+        runs = plan.pieces(M, N, K, epi)
+        assert sum(r for r, _ in runs) == M and len(runs) <= 2 and all(r > 0 for r, _ in runs)
+        for r, c in runs:
+            assert c is None or plan.supported(c[0], r, N, K, epi, c[1]), (M, N, K, epi, runs)
+        if M < LARGE_M or (M, N, K, epi) in plan.table:
+            assert runs == [(M, plan.choose(M, N, K, epi))]
+        split += len(runs) > 1
+    assert split
+
+
+def test_columns():
+    plan = GemmPlan()
+    plan.mode = "1"
+    split = 0
+    for M, N, K, _ in _shapes(40000):
+        n1 = plan.columns(M, N, K)
+        assert 0 < n1 <= N
+        if n1 < N:
+            assert 256 < M < LARGE_M and n1 % 256 == 0 and N % 256 == 0
+            assert plan.supported(W4_CFG, M, n1, K, 1) and plan.supported(SMALL_CFG, M, N - n1, K, 1)
+            whole = n1 // 256 * -(-M // 256)
+            assert whole >= 0.94 * CUS * -(-whole // CUS)
+            split += 1
+    assert split
+
+
+@pytest.mark.parametrize("mode", ["0", "force"])
+def test_other_modes_split_nothing(mode):
+    plan = GemmPlan()
+    plan.mode = mode
+    for M, N, K, epi in _shapes(2000):
+        assert plan.columns(M, N, K) == N and plan.pieces(M, N, K, epi) == [(M, plan.choose(M, N, K, epi))]
