@@ -245,7 +245,7 @@ __global__ __launch_bounds__(NTH, DC <= 8 ? 2 : 1) void chunk_kernel(ChunkArgs a
       *reinterpret_cast<F*>(&Vs[v_col * LDV + v_tok + p * (4 * NTH / VT)]) = f;
       if (odd) wild = 1;
     }
-    if (owner) {
+    if (ND * wave < DC) {   // every column of the tiles: what lies past dim is zero, and multiplied
 #pragma unroll
       for (int u = 0; u < NU; ++u)
 #pragma unroll

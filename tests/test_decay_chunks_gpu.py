@@ -78,3 +78,18 @@ def test_values_out_of_range_stay_behind_their_token(ops, dtype):
         keep[70:100, 0, 5] = False
         torch.testing.assert_close(got[keep], clean[keep], rtol=0, atol=1e-4)
         assert not torch.isfinite(got[70:100, 0, 5]).any()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("dim", [1, 12, 16, 33, 48, 65, 80, 96, 130, 176])
+def test_what_lies_past_the_key_features(ops, dtype, dim):
+    """Widths that leave whole 16-feature tiles unused, right after a call that leaves NaN in every workgroup's LDS."""
+    lens, starts = [130, 64], [0, 5]
+    c = lambda *t: [x.to(DEV) for x in t]  # noqa: E731
+    nan = _inputs([64] * 16, 128, 1, 128, 64, dtype, "fixed")
+    q, k, d, v, beta, state = _inputs(lens, 3, 3, dim, 40, dtype, "token", dim)
+    want = ref.gated_state_scan(*(x.double() for x in (q, k, d, v, beta)), _meta(lens, starts, "cpu"), state.double(), False)
+    (nq, nk, nd, nv, ns), (q, k, d, v, beta, state) = c(nan[0], nan[1], nan[2], nan[3], nan[5]), c(q, k, d, v, beta, state)
+    ops.gated_state_scan(nq, nk, nd, nv, None, _meta([64] * 16, [1] * 16, DEV), ns * math.nan, False)
+    got = ops.gated_state_scan(q, k, d, v, beta, _meta(lens, starts, DEV), state, False)
+    torch.testing.assert_close(got.cpu().double(), want.double(), rtol=0, atol=1e-5 * (8 + 4 * math.sqrt(130)))
