@@ -25,7 +25,7 @@
 //            || 16 ds_read_b128 of k-step 0 of tile t+1 -> x0/w0
 // RAW: a piece is waited for by every wave (counted vmcnt) before the barrier that precedes its
 //      first read.  WAR: a slot is refilled only after the barrier that follows its last reads
-//      (lgkmcnt(0) before that barrier).  Odd waves issue their pieces half a stride later.
+//      (lgkmcnt(0) before that barrier).  Two of the waves issue their pieces half a stride later (Sched).
 // One barrier per K-tile, a piece has 1.5 phases (~1500 cycles) to land.
 //
 // LDS: rows of 128 B (64 bf16 of K), the 16-B chunk c of row r at c ^ ((r >> 1) & 7): the
@@ -56,7 +56,7 @@
 #define W4_RAS (W4_SLOTS / 32)
 #endif
 #ifndef W4_DA0
-#define W4_DA0 (W4_SLOTS / 2 + 1)  // RING5 phase A: LDS-DMA pieces of X(t+2)
+#define W4_DA0 (W4_SLOTS / 2)  // phase A: LDS-DMA pieces of X(t+2)
 #endif
 #ifndef W4_DAS
 #define W4_DAS (W4_SLOTS / 16)
@@ -117,21 +117,23 @@ __device__ __forceinline__ i32x4 make_srd(const void* base, uint32_t bytes) {
   return r;
 }
 
-// Staggered schedules (W4_STAGGER): the odd waves issue their pieces half a stride later than
-// the even waves, so the CU's four waves do not send their LDS-DMA in lock step (the same
-// device as the two loop bodies, selected by a SIMD-id bit, of hipBLASLt's MT256x256 kernel).
-struct SchedMain {
-  static constexpr int RA0 = W4_RA0, RAS = W4_RAS, DA0 = W4_DA0, DAS = W4_DAS, DB0 = W4_DB0, DBS = W4_DBS,
-                       RB0 = W4_RB0, RBS = W4_RBS;
-};
-struct SchedAlt {
-  static constexpr int RA0 = W4_RA0, RAS = W4_RAS, DA0 = W4_DA0 + W4_DAS / 2, DAS = W4_DAS,
-                       DB0 = W4_DB0 + W4_DBS / 2, DBS = W4_DBS, RB0 = W4_RB0, RBS = W4_RBS;
-  static_assert(DA0 + 7 * DAS < W4_SLOTS && DB0 + (W4_NPB - 1) * DBS < W4_SLOTS, "staggered schedule");
+// Where a phase's memory operations go.  A phase has W4_SLOTS issue slots, one behind each MFMA.  Phase A: the reads take
+// the even slots of the first half, X's 8 pieces every fourth slot of the second.  Phase B: the reads take slots 2, 6, 10,
+// ..., W's pieces every eighth slot from 0 on.  The four waves leave the barrier together and would send their pieces of
+// one index into the CU's single LDS-DMA path in the same slot; the waves of the second column half (HALF = 1)
+// therefore take the free slots in the middle between the others' pieces (34, 38, ... and 4, 12, ...).  Measured, one
+// schedule for all four waves -> this, us: 16384 x 34816 x 5120 gated 3930 -> 3902, 16384 x 5120 x 17408 2066 -> 2052, 8192 x
+// 5120 x 5120 330 -> 326.5, 448 x 32768 x 5120 131.3 -> 130.5; four schedules, a quarter stride apart: 3940, 2068, 330, 132.
+template <int HALF>
+struct Sched {
+  static constexpr int RA0 = W4_RA0, RAS = W4_RAS, DA0 = W4_DA0 + HALF * W4_DAS / 2, DAS = W4_DAS,
+                       DB0 = W4_DB0 + HALF * W4_DBS / 2, DBS = W4_DBS, RB0 = W4_RB0, RBS = W4_RBS;
+  static_assert(DA0 + 7 * DAS < W4_SLOTS && DB0 + (W4_NPB - 1) * DBS < W4_SLOTS, "each piece has a slot of its phase");
 };
 // fp8 (e4m3) form: a K-tile is 128 elements in the same 128-B rows; each phase = one 64-deep
 // k-step = 16 v_mfma_scale_f32_32x32x64_f8f6f4 (the cycles of 64 bf16 16x16x32), so the same
-// 16 reads and 8 pieces per phase serve twice the FLOPs.
+// 16 reads and 8 pieces per phase serve twice the FLOPs.  One schedule for the four waves: with 16 slots a phase there is none
+// between the pieces to move to (a slot apart measured 16384 x 32768 x 6144: 2423 us, the same for all: 2404).
 #ifndef W4F8_DA0
 #define W4F8_DA0 8
 #endif
@@ -142,10 +144,6 @@ struct SchedF8 {
   static constexpr int RA0 = 0, RAS = 1, DA0 = W4F8_DA0, DAS = 1, DB0 = W4F8_DB0, DBS = 2, RB0 = 0, RBS = 1;
   static_assert(DA0 + 7 * DAS < 16 && DB0 + 7 * DBS < 16, "fp8 schedule");
 };
-struct SchedF8Alt {
-  static constexpr int RA0 = 0, RAS = 1, DA0 = W4F8_DA0 - 1, DAS = 1, DB0 = W4F8_DB0 + 1, DBS = 2, RB0 = 0, RBS = 1;
-};
-
 #ifdef W4_STAMPS
 // [workgroup][wave][phase A, wait, phase B, K-tiles, epilogues, kernel total, items, -]
 __device__ uint64_t w4_stamps[1 << 17];
@@ -904,15 +902,12 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
 #endif
   };
   if constexpr (F8) {
-    if (wave & 1)
-      run(SchedF8Alt{});
-    else
-      run(SchedF8{});
+    run(SchedF8{});
   } else {
-    if (wave & 1)
-      run(SchedAlt{});
+    if (wn)
+      run(Sched<1>{});
     else
-      run(SchedMain{});
+      run(Sched<0>{});
   }
   // every piece (the zero-range ones past the end included) has landed before the wave ends
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
