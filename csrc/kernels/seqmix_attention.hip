@@ -445,6 +445,7 @@ __global__ __launch_bounds__(256, NM * (KC + 2 * VT) <= 24 ? 4 : KC + VT <= 24 ?
   const int h = blockIdx.x % a.H, g = h / (a.H / a.G);
   const int* item = a.work + 3 * ((gridDim.x - 1 - blockIdx.x) / a.H);
   const int seq = item[0], first = item[1], row_end = item[2];
+  if (first >= row_end) return;   // (the whole workgroup) an entry without rows: its sequence and row need not exist
   const int row0 = first + 16 * wave;
   const bool active = row0 < row_end;
   const int ctx = a.seq_lens[seq], q_end = a.q_start[seq + 1];

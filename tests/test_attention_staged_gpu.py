@@ -35,3 +35,14 @@ def test_staged_prefill(ops, maps, dim, vdim, H, G, kind):
     got = ops.multimap_attention(q, *ops.kv_from_logical(k, v), meta, *args, **kw)
     want = ref.multimap_attention(q.float(), k.float(), v.float(), meta.block_tables, meta.q_start, meta.seq_lens, *args, **kw)
     torch.testing.assert_close(got.float(), want.float().reshape(got.shape), rtol=2e-2, atol=2e-2)
+
+
+def test_entries_without_rows(ops):
+    """A tile list padded with entries that hold no row, their sequence and row outside the batch: nothing of them is read."""
+    k, v, meta, T = _paged(SEQ, NEW, 16, 2, 64, 128, torch.bfloat16, seed=3)
+    q = torch.randn(T, 4, 64, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16).to(k.device)
+    args = (0.125, 1, 0.0, -1.0, 1.0, 128)
+    want = ops.multimap_attention(q, *ops.kv_from_logical(k, v), meta, *args)
+    pad = torch.tensor([[-1, T, T], [len(SEQ), 0, 0], [0, 5, 5]], dtype=torch.int32, device=k.device)
+    meta.tiles = torch.cat([pad, meta.tiles, pad])
+    assert torch.equal(ops.multimap_attention(q, *ops.kv_from_logical(k, v), meta, *args), want)
