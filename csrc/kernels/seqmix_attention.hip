@@ -427,12 +427,13 @@ __global__ __launch_bounds__(256, OCC) void prefill_kernel(AttnArgs a) {
 // in registers while this one is multiplied, the page numbers one chunk further ahead; two buffers, one barrier per
 // chunk).  The fragments come from LDS at the offsets they have in the slab, the 4-key rows of V moved apart by 128
 // bytes so that the lane groups read different banks.  All waves walk the tile's key range; a wave skips chunks that
-// hold no key it sees.  Tiles with the most keys start first, the heads of a tile side by side.
+// hold no key it sees.  The tile list is walked as it comes, the heads of a tile side by side: the engine lists the tiles with the
+// most keys first, so the launch ends on short ones (backwards, on the longest: 149, 170, 36.6 and 30 us of the four below).
 // Measured, 8 prompts of 1000 tokens: two 64-wide maps over 128-wide values, 16 heads: 226 us (one load per wave, 16-deep
-// products) -> 190 (32-deep products, column statistics by register swaps) -> 148 here; 32 latent heads of 192 / 128:
-// 379 -> 313 -> 168; 3 prompts of 700, 16 heads of 128 with a window: 52 -> 43 -> 29.  Two heads' waves on one copy
-// (512 threads) measured the same at the large sizes and 41 against 36 us at the small one.  What is left: LDS reads
-// (20 KB per 16 rows and chunk, 75 of the 168 us if alone) and softmax arithmetic, at 3 waves per SIMD.
+// products) -> 190 (32-deep products, column statistics by register swaps) -> 127 here; 32 latent heads of 192 / 128:
+// 379 -> 313 -> 162; 3 prompts of 700, 16 latent heads: 63 -> 35, 16 heads of 128 with a window: 52 -> 43 -> 28.  Two heads'
+// waves on one copy (512 threads) measured the same at the large sizes and 41 against 36 us at the small one.  What is left: LDS
+// reads (20 KB per 16 rows and chunk, 75 of the 162 us if alone) and softmax arithmetic, at 3 waves per SIMD.
 template <int KC, int VT, int NM, int MODE>
 __global__ __launch_bounds__(256, NM * (KC + 2 * VT) <= 24 ? 4 : KC + VT <= 24 ? 3 : 2) void prefill_staged_kernel(AttnArgs a) {
   typedef s16x4 F;
@@ -443,7 +444,7 @@ __global__ __launch_bounds__(256, NM * (KC + 2 * VT) <= 24 ? 4 : KC + VT <= 24 ?
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, grp = lane >> 4;
   const int h = blockIdx.x % a.H, g = h / (a.H / a.G);
-  const int* item = a.work + 3 * ((gridDim.x - 1 - blockIdx.x) / a.H);
+  const int* item = a.work + 3 * (blockIdx.x / a.H);
   const int seq = item[0], first = item[1], row_end = item[2];
   if (first >= row_end) return;   // (the whole workgroup) an entry without rows: its sequence and row need not exist
   const int row0 = first + 16 * wave;
