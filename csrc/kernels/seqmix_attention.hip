@@ -492,6 +492,7 @@ __global__ __launch_bounds__(256, NM * (KC + 2 * VT) <= 24 ? 4 : KC + VT <= 24 ?
     const int page = table[min(p, last_page)];
     return static_cast<size_t>((page < 0 || page >= a.num_blocks) ? 0 : page) * a.G + g;
   };
+  typedef f32x4 Unit __attribute__((aligned(8)));   // (one 16-byte load all the same: global loads need 4-byte alignment)
   f32x4 stage[NU];   // (the threads past the end of a chunk repeat its last unit)
   auto fetch = [&](size_t s0, size_t s1) {
 #pragma unroll
@@ -499,7 +500,7 @@ __global__ __launch_bounds__(256, NM * (KC + 2 * VT) <= 24 ? 4 : KC + VT <= 24 ?
       const int u = min(tid + i * TH, UNITS - 1);
       const bool isv = u >= 4 * KD;
       const int w = isv ? VD : KD, r = isv ? u - 4 * KD : u, second = r >= 2 * w;
-      const f32x4* base = static_cast<const f32x4*>(isv ? a.v_cache : a.k_cache);
+      const Unit* base = static_cast<const Unit*>(isv ? a.v_cache : a.k_cache);
       stage[i] = base[(second ? s1 : s0) * (2 * w) + (r - second * 2 * w)];
     }
   };
@@ -618,9 +619,9 @@ __global__ __launch_bounds__(256, NM * (KC + 2 * VT) <= 24 ? 4 : KC + VT <= 24 ?
   }
 }
 
-// what the copies of whole pages need: one page is a chunk's half, slabs of whole 16-byte units
+// what the copies of whole pages need: one page is a chunk's half, caches on 8 bytes like every 4-element fragment
 inline bool staged_layout(const AttnArgs& a) {
-  return a.swz && a.BS == 16 && ((reinterpret_cast<uintptr_t>(a.k_cache) | reinterpret_cast<uintptr_t>(a.v_cache)) & 15) == 0;
+  return a.swz && a.BS == 16 && ((reinterpret_cast<uintptr_t>(a.k_cache) | reinterpret_cast<uintptr_t>(a.v_cache)) & 7) == 0;
 }
 
 template <int KC, int VT, int NM, int MODE>

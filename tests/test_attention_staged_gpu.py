@@ -46,3 +46,14 @@ def test_entries_without_rows(ops):
     pad = torch.tensor([[-1, T, T], [len(SEQ), 0, 0], [0, 5, 5]], dtype=torch.int32, device=k.device)
     meta.tiles = torch.cat([pad, meta.tiles, pad])
     assert torch.equal(ops.multimap_attention(q, *ops.kv_from_logical(k, v), meta, *args), want)
+
+
+def test_caches_off_16_bytes(ops):
+    """Caches 8 bytes past a 16-byte boundary: the same kernel, the same bits."""
+    k, v, meta, T = _paged(SEQ, NEW, 16, 2, 64, 128, torch.bfloat16, seed=3)
+    q = torch.randn(T, 4, 64, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16).to(k.device)
+    args = (0.125, 1, 0.0, -1.0, 1.0, 128)
+    kl, vl = ops.kv_from_logical(k, v)
+    off = [torch.cat([x.new_zeros(4), x.flatten()])[4:].view(x.shape) for x in (kl, vl)]
+    assert all(x.data_ptr() % 16 == 8 for x in off)
+    assert torch.equal(ops.multimap_attention(q, *off, meta, *args), ops.multimap_attention(q, kl, vl, meta, *args))
