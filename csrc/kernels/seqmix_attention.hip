@@ -87,14 +87,31 @@ __device__ __forceinline__ float column_sum(float x) {
 }
 
 // Two neighbouring 16-deep operands in one 32-deep product (bf16): the lanes' 4 + 4 elements of both operands pair up the
-// same way, so the order of k inside the instruction is free.  An odd last operand is paired with zeros: a 16-deep product
-// behind 32-deep ones on the same accumulator gave wrong sums.
+// same way, so the order of k inside the instruction is free.
 __device__ __forceinline__ f32x4 mma32(s16x4 a0, s16x4 a1, s16x4 b0, s16x4 b1, f32x4 c) {
   typedef short s16x8 __attribute__((ext_vector_type(8)));
   const s16x8 a = __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7), b = __builtin_shufflevector(b0, b1, 0, 1, 2, 3, 4, 5, 6, 7);
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 __device__ __forceinline__ f32x4 mma32(f32x4 a0, f32x4 a1, f32x4 b0, f32x4 b1, f32x4 c) { return mma16(a1, b1, mma16(a0, b0, c)); }
+
+// The product of two rows of N operands, of which the first n_used hold something (the others are zero): every product of one
+// depth, an odd last operand beside zeros.  The depths must not meet on one accumulator: a 16x16x16 product that takes
+// the result of a 16x16x32 one (or the other way round) as its accumulator needs three wait states between the
+// two, which hipcc does not insert when the registers are exactly the same -- it counts on the forwarding that
+// two products of one form have.  Without them the sums are wrong (gfx950, ROCm 7.2: 0, 1 and 2 states wrong in half of the
+// elements, 3 and more right); with the loads of two maps between them it showed at two 48-wide maps and not at one.
+template <typename T, int N, typename FA, typename FB>
+__device__ __forceinline__ f32x4 mma_row(int n_used, FA a, FB b) {
+  f32x4 c = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < N; i += 2)
+    if (i < n_used) {
+      if (i + 1 < N) c = mma32(a(i), a(i + 1), b(i), b(i + 1), c);
+      else c = mma32(a(i), zero_frag<T>(), b(i), zero_frag<T>(), c);
+    }
+  return c;
+}
 
 // First key that a query at position `pos` sees: the window's or the chunk's first, else 0.
 __device__ __forceinline__ int first_key(const AttnArgs& a, int pos) {
@@ -251,14 +268,7 @@ __device__ __forceinline__ void attend_range(const AttnArgs& a_, int g, const ty
 #pragma unroll
       for (int m = 0; m < NM; ++m) {
         s[u][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (m < a.maps) {   // (fragments past kc are zero)
-#pragma unroll
-          for (int c = 0; c + 1 < KC; c += 2)
-            if (c < kc) s[u][m] = mma32(kf[u][m][c], kf[u][m][c + 1], qf[m][c], qf[m][c + 1], s[u][m]);
-          if constexpr (KC & 1) {
-            if (KC - 1 < kc) s[u][m] = mma32(kf[u][m][KC - 1], zero_frag<T>(), qf[m][KC - 1], zero_frag<T>(), s[u][m]);
-          }
-        }
+        if (m < a.maps) s[u][m] = mma_row<T, KC>(kc, [&](int c) { return kf[u][m][c]; }, [&](int c) { return qf[m][c]; });
       }
     // the K fragments are spent: the next iteration's go into the same registers, under the
     // softmax and the second product
@@ -527,11 +537,9 @@ __global__ __launch_bounds__(256, NM * (KC + 2 * VT) <= 24 ? 4 : KC + VT <= 24 ?
       for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int m = 0; m < NM; ++m) {
-          sm[u][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-          auto frag = [&](int c) { return *reinterpret_cast<const F*>(ks + u * 16 * KD + ((m * DIM + 16 * c) / 4 * 16 + grp * 16 + col) * 4); };
-#pragma unroll
-          for (int c = 0; c + 1 < KC; c += 2) sm[u][m] = mma32(frag(c), frag(c + 1), qf[m][c], qf[m][c + 1], sm[u][m]);
-          if constexpr (KC & 1) sm[u][m] = mma32(frag(KC - 1), zero_frag<bf16_t>(), qf[m][KC - 1], zero_frag<bf16_t>(), sm[u][m]);
+          sm[u][m] = mma_row<bf16_t, KC>(
+              KC, [&](int c) { return *reinterpret_cast<const F*>(ks + u * 16 * KD + ((m * DIM + 16 * c) / 4 * 16 + grp * 16 + col) * 4); },
+              [&](int c) { return qf[m][c]; });
         }
       const bool masked = key0 + 31 > pos_min || key0 < lo_max;
       float cap_now = cap;
