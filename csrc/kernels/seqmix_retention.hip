@@ -142,7 +142,8 @@ __global__ __launch_bounds__(NTH, DC <= 8 ? 2 : 1) void chunk_kernel(ChunkArgs a
   const bool carry = a.positions[t0] != 0;
   const bool vec_s = (vdim & 3) == 0;
   const int d0 = 16 * ND * wave + ND * col;   // this lane's features of the state: d0 .. d0 + ND - 1
-  const bool vec_k = FULL || (ND > 1 && a.vec && (dim & 3) == 0 && d0 + ND <= dim);
+  constexpr bool OWNERS = FULL && DC % 4 == 0;   // every wave has features (of 32, two waves have none: they must not read past a row)
+  const bool vec_k = OWNERS || (ND > 1 && a.vec && (dim & 3) == 0 && d0 + ND <= dim);
   f32x4 S[ND][NU];   // lane: S^T[value column 16 u + 4 grp + i][feature d0 + m]
 #pragma unroll
   for (int m = 0; m < ND; ++m)
@@ -185,7 +186,7 @@ __global__ __launch_bounds__(NTH, DC <= 8 ? 2 : 1) void chunk_kernel(ChunkArgs a
         }
       }
 #pragma unroll
-      for (int m = 0; m < ND; ++m) kf[tt][j][m] = FULL || d0 + m < dim ? base[o + m] : 0.f;
+      for (int m = 0; m < ND; ++m) kf[tt][j][m] = OWNERS || d0 + m < dim ? base[o + m] : 0.f;
     }
   };
   auto load_r = [&](int first, int id) {

@@ -93,3 +93,14 @@ def test_what_lies_past_the_key_features(ops, dtype, dim):
     ops.gated_state_scan(nq, nk, nd, nv, None, _meta([64] * 16, [1] * 16, DEV), ns * math.nan, False)
     got = ops.gated_state_scan(q, k, d, v, beta, _meta(lens, starts, DEV), state, False)
     torch.testing.assert_close(got.cpu().double(), want.double(), rtol=0, atol=1e-5 * (8 + 4 * math.sqrt(130)))
+
+
+def test_keys_at_the_end_of_their_memory(ops):
+    """32 key features leave two of a workgroup's four waves without any: nothing is read past the last key."""
+    lens, H, dim, vdim = [64] * 64, 2, 32, 32
+    q, k, d, v, beta, state = _inputs(lens, H, H, dim, vdim, torch.bfloat16, "token")
+    want = ref.gated_state_scan(*(x.double() for x in (q, k, d, v, beta)), _meta(lens, [0] * 64, "cpu"), state.double(), False)
+    whole = torch.empty(12 << 18, device=DEV)     # 12 MiB: a memory block of its own, k its last MiB
+    tail = whole[-k.numel():].view(k.shape).copy_(k)
+    got = ops.gated_state_scan(q.to(DEV), tail, d.to(DEV), v.to(DEV), beta.to(DEV), _meta(lens, [0] * 64, DEV), state.to(DEV), False)
+    torch.testing.assert_close(got.cpu().double(), want.double(), rtol=0, atol=1e-5 * (8 + 4 * math.sqrt(64)))
