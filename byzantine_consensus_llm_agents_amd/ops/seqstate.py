@@ -212,7 +212,8 @@ def seqstate_ops(lib):
         # one decay per head and no correction term: long segments run as chunks of matrix products, the
         # short ones among them (single tokens beside portions) token by token
         skip = 0
-        if gd == 1 and not delta and not unit_last and not meta.decode and T - B + 1 >= min_chunked:
+        if (gd == 1 and not delta and not unit_last and not meta.decode and T - B + 1 >= min_chunked
+                and state.data_ptr() % 16 == 0):   # (the chunks move the state 16 bytes at a time, the other form by elements)
             skip = min_chunked
             scores = torch.empty((T // chunk + B) * Gq * chunk * chunk, dtype=torch.float32, device=g.device)
             _check(lib.bcg_decay_chunks(_p(q), _p(k), _p(g), 0 if g_const else H, _p(beta), _p(v), v.stride(0), _p(meta.positions),

@@ -104,3 +104,21 @@ def test_keys_at_the_end_of_their_memory(ops):
     tail = whole[-k.numel():].view(k.shape).copy_(k)
     got = ops.gated_state_scan(q.to(DEV), tail, d.to(DEV), v.to(DEV), beta.to(DEV), _meta(lens, [0] * 64, DEV), state.to(DEV), False)
     torch.testing.assert_close(got.cpu().double(), want.double(), rtol=0, atol=1e-5 * (8 + 4 * math.sqrt(64)))
+
+
+@pytest.mark.parametrize("decay", ["fixed", "token"])
+def test_state_off_16_bytes(ops, decay):
+    """A state that does not lie on 16 bytes (a slice of a larger table) goes token by token."""
+    lens, starts = [70, 1, 20], [3, 5, 0]
+    q, k, d, v, beta, state = _inputs(lens, 3, 1, 5, 7, torch.bfloat16, decay)
+    table = torch.cat([state.new_zeros(1), state.flatten()])
+    want_state = state.double()
+    want = ref.gated_state_scan(q.double(), k.double(), d.double(), v.double(), None if beta is None else beta.double(),
+                                _meta(lens, starts, "cpu"), want_state, False)
+    c = lambda x: None if x is None else x.to(DEV)  # noqa: E731
+    off = c(table)[1:].view(state.shape)
+    assert off.data_ptr() % 16 == 4
+    got = ops.gated_state_scan(c(q), c(k), c(d), c(v), c(beta), _meta(lens, starts, DEV), off, False)
+    bound = 1e-5 * (8 + 4 * math.sqrt(70))
+    torch.testing.assert_close(got.cpu().double(), want.double(), rtol=0, atol=bound)
+    torch.testing.assert_close(off.cpu().double(), want_state, rtol=0, atol=bound)
