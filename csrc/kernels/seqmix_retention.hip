@@ -396,11 +396,12 @@ __global__ __launch_bounds__(NTH, DC <= 8 ? 2 : 1) void chunk_kernel(ChunkArgs a
 template <typename T, int DC, bool FULL>
 int launch_chunks(const ChunkArgs& a, int n_chunks, hipStream_t s) {
   scores_kernel<DC, FULL><<<dim3(n_chunks, a.Gq), NTH, 0, s>>>(a);
-  // 64 value columns per workgroup where that gives every CU two, else fewer: the walk is serial, idle CUs cost nothing
-  // (96 workgroups of 64 columns -> 384 of 16: 140 us -> 75, 3 segments of 700)
+  // 64 value columns per workgroup from more than one workgroup per CU on, fewer below: the walk is serial, idle CUs cost nothing
+  // (96 workgroups of 64 columns -> 384 of 16: 140 us -> 75, 3 segments of 700).  At one per CU 32 columns win (64 segments of
+  // 200, 4 heads of 64 x 64: 47 us, 64 columns 50), past it their second round loses (100 segments: 74 us, 62).
   const int64_t wide = static_cast<int64_t>(a.B) * a.H * ((a.vdim + 63) / 64);
-  if (wide >= 512) chunk_kernel<T, DC, 64, FULL><<<dim3(a.B, a.H, (a.vdim + 63) / 64), NTH, 0, s>>>(a);
-  else if (wide >= 256) chunk_kernel<T, DC, 32, FULL><<<dim3(a.B, a.H, (a.vdim + 31) / 32), NTH, 0, s>>>(a);
+  if (wide > 256) chunk_kernel<T, DC, 64, FULL><<<dim3(a.B, a.H, (a.vdim + 63) / 64), NTH, 0, s>>>(a);
+  else if (wide == 256) chunk_kernel<T, DC, 32, FULL><<<dim3(a.B, a.H, (a.vdim + 31) / 32), NTH, 0, s>>>(a);
   else chunk_kernel<T, DC, 16, FULL><<<dim3(a.B, a.H, (a.vdim + 15) / 16), NTH, 0, s>>>(a);
   return BCG_CHECK_LAUNCH();
 }
