@@ -33,8 +33,25 @@ def _segments(meta, T):
     return B
 
 
+def chunked_from(B, H, dim, f32):
+    """Tokens of a segment from which the chunks (two launches, and the token-by-token one behind them for the segments
+    that are shorter) are the faster form of a recurrence with one decay per head.
+
+    Token by token -> chunks, us: one segment of 16, 4 heads of 64 x 64: 8.1 -> 7.6 (fp32 activations 6.8 -> 8.4, of 32: 10.1 -> 9.1);
+    16 segments of 16, 16 heads of 64 x 64: 9.8 -> 12.2, of 32: 14.7 -> 13.9; 64 segments of 16 there: 24.2 -> 23.7;
+    128 x 128: 16 segments of 16: 18.9 -> 17.6.  fp32 activations, 64 x 64, 4 heads: 4 segments of 48: 13.5 -> 12.8; 64
+    segments of 100: 28.6 -> 31.4, of 128: 34.6 -> 30.7; 128 x 128, 16 segments of 20: 20.2 -> 23.0, of 24: 23.8 -> 23.8."""
+    if dim > 64:
+        return 24 if f32 and B > 1 and B * H < 1024 else 16
+    if B == 1:
+        return 32 if f32 else 16
+    if f32:
+        return 48 if B * H < 128 else 128
+    return 32 if B * H < 1024 else 16
+
+
 def seqstate_ops(lib):
-    min_chunked, chunk = lib.bcg_decay_chunks_min_len(), lib.bcg_decay_chunks_tokens()
+    chunk = lib.bcg_decay_chunks_tokens()
 
     def embed_hashed_bigram_norm(tokens, meta, prev, table, scale, bigram, hash_mul, eps, gains, out_dtype):
         T, W = tokens.numel(), table.shape[1]
@@ -212,13 +229,17 @@ def seqstate_ops(lib):
         # one decay per head and no correction term: long segments run as chunks of matrix products, the
         # short ones among them (single tokens beside portions) token by token
         skip = 0
-        if (gd == 1 and not delta and not unit_last and not meta.decode and T - B + 1 >= min_chunked
-                and state.data_ptr() % 16 == 0):   # (the chunks move the state 16 bytes at a time, the other form by elements)
-            skip = min_chunked
+        if gd == 1 and not delta and not unit_last and not meta.decode and state.data_ptr() % 16 == 0:   # (16 bytes at a time)
+            longest, skip = T - B + 1, 16   # (at most; a step that says how long its longest segment is knows better)
+            if getattr(meta, "max_q_len", 1) > 1:
+                longest, skip = min(longest, meta.max_q_len), chunked_from(B, H, dim, _act(v))
+            if longest < skip:
+                skip = 0
+        if skip:
             scores = torch.empty((T // chunk + B) * Gq * chunk * chunk, dtype=torch.float32, device=g.device)
             _check(lib.bcg_decay_chunks(_p(q), _p(k), _p(g), 0 if g_const else H, _p(beta), _p(v), v.stride(0), _p(meta.positions),
                                         _p(meta.q_start), _p(meta.state_rows), _p(state), state.shape[0], _p(out), _p(scores), T, B,
-                                        H, Gq, dim, vdim, _act(v), _stream()), "decay_chunks")
+                                        H, Gq, dim, vdim, skip, _act(v), _stream()), "decay_chunks")
             if B == 1:
                 return out
         _check(lib.bcg_gated_state_scan(_p(q), _p(k), _p(g), _p(v), v.stride(0), _p(beta), _p(meta.positions),

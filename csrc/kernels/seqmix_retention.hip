@@ -39,9 +39,6 @@
 namespace {
 
 constexpr int CT = 64, NTH = 256;
-// Shorter segments go token by token.  Measured (us, token by token -> here): 64 segments of 16, 128 heads: 220 -> 149; 8 heads: 69 ->
-// 45; 4 heads of 64 x 64: 10 -> 12 (the second launch), 4 segments of 40: 15 -> 11.
-constexpr int MIN_LEN = 16;
 
 struct ChunkArgs {
   const float* q; const float* k;                   // [T, Gq, dim]
@@ -53,6 +50,7 @@ struct ChunkArgs {
   float* out;                                       // [T, H, vdim]
   float* scores;                                    // [chunks, Gq, CT (query), CT (key)]
   int n_rows, B, H, Gq, dim, vdim, vec;             // vec: rows of q / k are 16-byte aligned
+  int min_len;                                      // shorter segments are the token-by-token kernel's
 };
 
 // Segment b's chunk c has the number q_start[b] / CT + b + c: at most T / CT + B numbers, no two chunks alike.
@@ -85,7 +83,7 @@ __global__ __launch_bounds__(NTH) void scores_kernel(ChunkArgs a) {
     if (chunk_base(a.q_start, mid) <= id) lo = mid; else hi = mid - 1;
   }
   const int t0 = a.q_start[lo], t1 = a.q_start[lo + 1], first = t0 + (id - chunk_base(a.q_start, lo)) * CT;
-  if (t1 - t0 < MIN_LEN || first < t0 || first >= t1) return;
+  if (t1 - t0 < a.min_len || first < t0 || first >= t1) return;
   for (int e = wave; e < 10; e += 4) {   // the ten 16 x 16 tiles on and under the diagonal
     const int rt = e >= 6 ? 3 : e >= 3 ? 2 : e >= 1 ? 1 : 0, st = e - rt * (rt + 1) / 2;
     if (first + 16 * rt >= t1) continue;
@@ -136,7 +134,7 @@ __global__ __launch_bounds__(NTH, DC <= 8 ? 2 : 1) void chunk_kernel(ChunkArgs a
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 15, grp = lane >> 4;
   const int b = blockIdx.x, h = blockIdx.y, v0 = blockIdx.z * VT;
   const int t0 = a.q_start[b], t1 = a.q_start[b + 1], sr = a.state_rows[b];
-  if (t1 - t0 < MIN_LEN || sr < 0 || sr >= a.n_rows) return;
+  if (t1 - t0 < a.min_len || sr < 0 || sr >= a.n_rows) return;
   const int gq = h / (a.H / a.Gq), dim = a.dim, vdim = a.vdim;
   float* Sg = a.state + (static_cast<size_t>(sr) * a.H + h) * dim * vdim + v0;
   const bool carry = a.positions[t0] != 0;
@@ -424,19 +422,16 @@ int launch_dim(const ChunkArgs& a, int n_chunks, hipStream_t s) {
 
 }  // namespace
 
-// Segments shorter than this are left alone by `bcg_decay_chunks`.
-BCG_API int bcg_decay_chunks_min_len() { return MIN_LEN; }
-
 // `scores` takes (T / tokens + B) Gq tokens^2 fp32 elements
 BCG_API int bcg_decay_chunks_tokens() { return CT; }
 
-// g: [H] (g_token 0) or [T, H] (g_token H); beta [T, H] or null.
+// g: [H] (g_token 0) or [T, H] (g_token H); beta [T, H] or null.  Segments of fewer than `min_len` tokens are left alone.
 BCG_API int bcg_decay_chunks(const void* q32, const void* k32, const void* g, int g_token, const void* beta, const void* v,
                              int64_t v_stride, const void* positions, const void* q_start, const void* state_rows, void* state,
-                             int n_rows, void* out, void* scores, int T_, int B, int H, int Gq, int dim, int vdim, int is_f32,
-                             void* stream) {
+                             int n_rows, void* out, void* scores, int T_, int B, int H, int Gq, int dim, int vdim, int min_len,
+                             int is_f32, void* stream) {
   if (B <= 0 || T_ <= 0) return 0;
-  if (dim < 1 || dim > 256 || vdim < 1 || H <= 0 || Gq <= 0 || H % Gq || H > 65535 || (vdim + 15) / 16 > 65535) return -2;
+  if (dim < 1 || dim > 256 || vdim < 1 || H <= 0 || Gq <= 0 || H % Gq || H > 65535 || (vdim + 15) / 16 > 65535 || min_len < 1) return -2;
   auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
   if (!al16(state) || !al16(out) || !al16(scores) || scores == nullptr || (g_token != 0 && g_token != H)) return -2;
   ChunkArgs a;
@@ -448,6 +443,7 @@ BCG_API int bcg_decay_chunks(const void* q32, const void* k32, const void* g, in
   a.state = static_cast<float*>(state); a.out = static_cast<float*>(out); a.scores = static_cast<float*>(scores);
   a.n_rows = n_rows; a.B = B; a.H = H; a.Gq = Gq; a.dim = dim; a.vdim = vdim;
   a.vec = dim % 4 == 0 && al16(q32) && al16(k32);
+  a.min_len = min_len;
   hipStream_t s = static_cast<hipStream_t>(stream);
   return is_f32 ? launch_dim<float>(a, T_ / CT + B, s) : launch_dim<bf16_t>(a, T_ / CT + B, s);
 }
