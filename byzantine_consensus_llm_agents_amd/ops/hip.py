@@ -14,6 +14,7 @@ from types import SimpleNamespace
 import torch
 
 from ..utils.build import kernel_sources, kernels_source_hash, kernels_target
+from .operands import bare
 
 _LIB = None
 # Rows per prefill attention tile unless BCG_PREFILL_TILE_ROWS says otherwise (prefill_tile_rows)
@@ -371,18 +372,17 @@ def hip_ops() -> SimpleNamespace:
             dispatch_log.calls[key] = dispatch_log.calls.get(key, 0) + 1
 
     def _plain(x, w):
-        """Operands that the kernels of this file take as they lie: bf16, rows contiguous, 16-byte aligned, and no
-        gradient asked of them (the library's products carry one, these do not)."""
+        """Operands that the kernels of this file take as they lie: bf16, rows contiguous, 16-byte aligned, and bare
+        (the library's products carry gradients and tangents, these do not)."""
         return (x.dtype == w.dtype == torch.bfloat16 and w.dim() == 2 and w.shape[1] == x.shape[1] and x.is_contiguous()
-                and w.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
-                and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)))
+                and w.is_contiguous() and bare(x) and bare(w) and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
     def _plain_bias(bias, N):
-        return bias is None or (bias.dtype == torch.bfloat16 and bias.shape == (N,) and bias.is_contiguous()
+        return bias is None or (bias.dtype == torch.bfloat16 and bias.shape == (N,) and bias.is_contiguous() and bare(bias)
                                 and bias.data_ptr() % 16 == 0)
 
     def _plain_residual(residual, M, N):
-        return (residual.shape == (M, N) and residual.dtype == torch.bfloat16 and residual.is_contiguous()
+        return (residual.shape == (M, N) and residual.dtype == torch.bfloat16 and residual.is_contiguous() and bare(residual)
                 and residual.data_ptr() % 16 == 0)
 
     def _pieces(x, w, epi, others=True):
@@ -556,7 +556,7 @@ def hip_ops() -> SimpleNamespace:
 
     def _norm_fusable(x, w_norm):
         return (x.shape[1] <= 8192 and w_norm.shape == (x.shape[1],) and w_norm.dtype == torch.bfloat16 and w_norm.is_contiguous()
-                and w_norm.data_ptr() % 16 == 0)
+                and bare(w_norm) and w_norm.data_ptr() % 16 == 0)
 
     def norm_linear(x, w_norm, eps, w, bias=None):
         """linear(rmsnorm(x, w_norm, eps), w, bias), one kernel for a few rows."""
