@@ -372,18 +372,19 @@ def hip_ops() -> SimpleNamespace:
             dispatch_log.calls[key] = dispatch_log.calls.get(key, 0) + 1
 
     def _plain(x, w):
-        """Operands that the kernels of this file take as they lie: bf16, rows contiguous, 16-byte aligned, and bare
+        """Operands that the kernels of this file take as they lie: bf16 on the current GPU, rows contiguous, 16-byte aligned and bare
         (the library's products carry gradients and tangents, these do not)."""
-        return (x.dtype == w.dtype == torch.bfloat16 and w.dim() == 2 and w.shape[1] == x.shape[1] and x.is_contiguous()
+        return (x.dtype == w.dtype == torch.bfloat16 and x.is_cuda and x.device == w.device
+                and x.get_device() == torch.cuda.current_device() and w.dim() == 2 and w.shape[1] == x.shape[1] and x.is_contiguous()
                 and w.is_contiguous() and bare(x) and bare(w) and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
-    def _plain_bias(bias, N):
-        return bias is None or (bias.dtype == torch.bfloat16 and bias.shape == (N,) and bias.is_contiguous() and bare(bias)
-                                and bias.data_ptr() % 16 == 0)
+    def _plain_beside(t, shape, x):
+        """The same for a bias, residual or norm weight beside x."""
+        return (t.dtype == torch.bfloat16 and t.device == x.device and t.shape == shape and t.is_contiguous() and bare(t)
+                and t.data_ptr() % 16 == 0)
 
-    def _plain_residual(residual, M, N):
-        return (residual.shape == (M, N) and residual.dtype == torch.bfloat16 and residual.is_contiguous() and bare(residual)
-                and residual.data_ptr() % 16 == 0)
+    def _plain_bias(bias, N, x):
+        return bias is None or _plain_beside(bias, (N,), x)
 
     def _pieces(x, w, epi, others=True):
         """Runs of rows and their choices (`GemmPlan.pieces`); others: whether the bias / residual lies as the kernels want."""
@@ -415,12 +416,12 @@ def hip_ops() -> SimpleNamespace:
         otherwise."""
         M, K = x.shape
         N = w.shape[0]
-        if _skinny(x, w, 0) and _plain_bias(bias, N):
+        if _skinny(x, w, 0) and _plain_bias(bias, N, x):
             return _gemm_skinny(x, w, 0, bias)
         if not (x.is_contiguous() and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16):
             _log(M, N, K, _epi_log, None)
             return torch.nn.functional.linear(x, w, bias)
-        parts = _pieces(x, w, 0, _plain_bias(bias, N))
+        parts = _pieces(x, w, 0, _plain_bias(bias, N, x))
         if len(parts) == 1:
             return _linear_rows(x, w, bias, parts[0][1], None, _epi_log)
         out, at = torch.empty(M, N, dtype=x.dtype, device=x.device), 0
@@ -555,12 +556,11 @@ def hip_ops() -> SimpleNamespace:
         return out
 
     def _norm_fusable(x, w_norm):
-        return (x.shape[1] <= 8192 and w_norm.shape == (x.shape[1],) and w_norm.dtype == torch.bfloat16 and w_norm.is_contiguous()
-                and bare(w_norm) and w_norm.data_ptr() % 16 == 0)
+        return x.shape[1] <= 8192 and _plain_beside(w_norm, (x.shape[1],), x)
 
     def norm_linear(x, w_norm, eps, w, bias=None):
         """linear(rmsnorm(x, w_norm, eps), w, bias), one kernel for a few rows."""
-        if x.dim() == 2 and _skinny(x, w, 0) and _norm_fusable(x, w_norm) and _plain_bias(bias, w.shape[0]):
+        if x.dim() == 2 and _skinny(x, w, 0) and _norm_fusable(x, w_norm) and _plain_bias(bias, w.shape[0], x):
             return _gemm_skinny(x, w, 0, bias, norm_w=w_norm, eps=eps)
         return linear(rmsnorm(x, w_norm, eps), w, bias)
 
@@ -576,11 +576,11 @@ def hip_ops() -> SimpleNamespace:
         """residual <- residual + x W^T (in place; the o/down projection fused with the
         residual-stream update of the next add+RMSNorm).  Returns `residual`."""
         M, K = x.shape
-        if _skinny(x, w, 2) and _plain_residual(residual, M, w.shape[0]):
+        if _skinny(x, w, 2) and _plain_beside(residual, (M, w.shape[0]), x):
             return _gemm_skinny(x, w, 2, residual=residual)
         parts = [(M, None)]
         if x.is_contiguous() and x.dtype == torch.bfloat16:
-            parts = _pieces(x, w, 2, _plain_residual(residual, M, w.shape[0]))
+            parts = _pieces(x, w, 2, _plain_beside(residual, (M, w.shape[0]), x))
         at = 0
         for rows, cfg in parts:
             whole = rows == M

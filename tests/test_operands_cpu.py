@@ -1,8 +1,13 @@
 """Which operands the kernels without a graph behind them take (ops/operands.py), without a GPU."""
+import os
+
+import pytest
 import torch
 from torch.autograd import forward_ad
 
+from byzantine_consensus_llm_agents_amd.ops import get_ops
 from byzantine_consensus_llm_agents_amd.ops.operands import bare
+from byzantine_consensus_llm_agents_amd.utils.build import kernels_target
 
 
 def test_gradients_and_tangents():
@@ -15,3 +20,29 @@ def test_gradients_and_tangents():
     with forward_ad.dual_level():
         assert bare(x) and not bare(forward_ad.make_dual(x, torch.ones_like(x)))
     assert bare(x)
+
+
+@pytest.fixture(scope="module")
+def ops():
+    if not os.path.exists(kernels_target()):
+        pytest.skip("kernel library not built")
+    ops = get_ops("hip")
+    if ops.gemm_plan.mode != "1":
+        pytest.skip("BCG_HAND_GEMM")
+    return ops
+
+
+def _data():
+    g = torch.Generator().manual_seed(1)
+    return [torch.randn(*s, generator=g).bfloat16() for s in ((5, 3, 128), (36, 128), (36,), (5, 3, 36))]
+
+
+def test_host_memory(ops):
+    """Operands in host memory, or on two devices, never reach a kernel: the library computes them, or says no."""
+    x, w, b, r = _data()
+    want = torch.nn.functional.linear(x[0], w, b)
+    assert torch.equal(ops.linear(x[0], w, b), want)
+    assert torch.equal(ops.linear_residual(x[0], w, r[0].clone()), r[0].addmm(x[0], w.t()))
+    rows, wide = x.reshape(15, 128)[:1].expand(2900, 128).contiguous(), w[:1].expand(24576, 128).contiguous()
+    assert ops.gemm_plan.pieces(2900, 24576, 128, 0)[0][1] is not None     # (a shape of the 256 x 256 kernel)
+    assert torch.equal(ops.linear(rows, wide), torch.nn.functional.linear(rows, wide))

@@ -52,3 +52,13 @@ def test_forward_mode(ops, M, N, K):
         assert _off(out.primal, x.float() @ w.float().t()) < 2 ** -8 and _off(out.tangent, t.float() @ w.float().t()) < 2 ** -8
         out = forward_ad.unpack_dual(ops.linear(x, w, forward_ad.make_dual(b, b)))
         assert _off(out.tangent, b.expand(M, N)) < 2 ** -8
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_two_devices(ops, M, N, K):
+    """One operand in host memory: refused as the library refuses it."""
+    x, w, b, r = _data(M, N, K)
+    for call in (lambda: ops.linear(x, w.cpu()), lambda: ops.linear(x, w, b.cpu()), lambda: ops.linear_residual(x, w, r.cpu()),
+                 lambda: ops.norm_linear(x, torch.ones(K, device="cuda").bfloat16(), 1e-6, w.cpu())):
+        with pytest.raises(RuntimeError):
+            call()
