@@ -14,7 +14,7 @@ from types import SimpleNamespace
 import torch
 
 from ..utils.build import kernel_sources, kernels_source_hash, kernels_target
-from .operands import bare
+from .operands import bare, watched
 
 _LIB = None
 # Rows per prefill attention tile unless BCG_PREFILL_TILE_ROWS says otherwise (prefill_tile_rows)
@@ -372,11 +372,11 @@ def hip_ops() -> SimpleNamespace:
             dispatch_log.calls[key] = dispatch_log.calls.get(key, 0) + 1
 
     def _plain(x, w):
-        """Operands that the kernels of this file take as they lie: bf16 on the current GPU, rows contiguous, 16-byte aligned and bare
-        (the library's products carry gradients and tangents, these do not)."""
+        """Operands that the kernels of this file take as they lie: bf16 on the current GPU, rows contiguous, 16-byte aligned, bare
+        and not watched (the library's products carry gradients, tangents and transforms, these do not)."""
         return (x.dtype == w.dtype == torch.bfloat16 and x.is_cuda and x.device == w.device
                 and x.get_device() == torch.cuda.current_device() and w.dim() == 2 and w.shape[1] == x.shape[1] and x.is_contiguous()
-                and w.is_contiguous() and bare(x) and bare(w) and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+                and w.is_contiguous() and not watched() and bare(x) and bare(w) and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
     def _plain_beside(t, shape, x):
         """The same for a bias, residual or norm weight beside x."""

@@ -3,10 +3,12 @@ import os
 
 import pytest
 import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
 from torch.autograd import forward_ad
+from torch.fx.experimental.proxy_tensor import make_fx
 
 from byzantine_consensus_llm_agents_amd.ops import get_ops
-from byzantine_consensus_llm_agents_amd.ops.operands import bare
+from byzantine_consensus_llm_agents_amd.ops.operands import bare, watched
 from byzantine_consensus_llm_agents_amd.utils.build import kernels_target
 
 
@@ -46,3 +48,31 @@ def test_host_memory(ops):
     rows, wide = x.reshape(15, 128)[:1].expand(2900, 128).contiguous(), w[:1].expand(24576, 128).contiguous()
     assert ops.gemm_plan.pieces(2900, 24576, 128, 0)[0][1] is not None     # (a shape of the 256 x 256 kernel)
     assert torch.equal(ops.linear(rows, wide), torch.nn.functional.linear(rows, wide))
+
+
+def test_transforms(ops):
+    """The few-row kernel's shapes under vmap, functional gradients and tangents, as the library computes them."""
+    lin = torch.nn.functional.linear
+    x, w, b, r = _data()
+    assert torch.equal(torch.vmap(lambda t: ops.linear(t, w, b))(x), torch.vmap(lambda t: lin(t, w, b))(x))
+    two = torch.stack([w, -w])
+    assert torch.equal(torch.vmap(lambda t: ops.linear(x[0], t))(two), torch.vmap(lambda t: lin(x[0], t))(two))
+    got, want = (torch.vmap(f)(x, r.clone()) for f in (lambda t, u: ops.linear_residual(t, w, u), lambda t, u: u.addmm_(t, w.t())))
+    assert torch.equal(got, want)
+    for arg in range(3):
+        a = (x[0], w, b)
+        got = torch.func.grad(lambda t: ops.linear(*a[:arg], t, *a[arg + 1:]).float().sum())(a[arg])
+        assert torch.equal(got, torch.func.grad(lambda t: lin(*a[:arg], t, *a[arg + 1:]).float().sum())(a[arg]))
+    got, want = (torch.func.jvp(lambda t: f(t, w, b), (x[0],), (x[1],)) for f in (ops.linear, lin))
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+def test_traces_and_fakes(ops):
+    x, w, b, _ = _data()
+    x = x[0]
+    f = lambda x, w, b: ops.linear(x, w, b)  # noqa: E731
+    for trace in (make_fx(f)(x, w, b), make_fx(f, tracing_mode="fake")(x, w, b), torch.jit.trace(f, (x, w, b))):
+        assert torch.equal(trace(x * 2, w, b), torch.nn.functional.linear(x * 2, w, b))
+    with FakeTensorMode() as mode:
+        assert watched() and ops.linear(mode.from_tensor(x), mode.from_tensor(w)).shape == (3, 36)
+    assert not watched() and not bare(mode.from_tensor(x))

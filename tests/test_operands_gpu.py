@@ -62,3 +62,12 @@ def test_two_devices(ops, M, N, K):
                  lambda: ops.norm_linear(x, torch.ones(K, device="cuda").bfloat16(), 1e-6, w.cpu())):
         with pytest.raises(RuntimeError):
             call()
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_autocast_and_vmap(ops, M, N, K):
+    x, w, b, _ = _data(M, N, K)
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert ops.linear(x, w, b).dtype == torch.float16
+    y = torch.vmap(lambda t: ops.linear(t, w, b))(x[None])
+    assert _off(y[0], x.float() @ w.float().t() + b.float()) < 2 ** -8
