@@ -1086,8 +1086,10 @@ BCG_API int bcg_gemm_w4_sk_ws_floats() { return 2 * w4_cus() * BM * BN; }
 BCG_API int bcg_gemm_w4(int epi, const void* x, const void* w, const void* bias, const void* residual, void* c,
                         void* ws, void* counters, int M, int N, int K, int inter, int split_k, hipStream_t stream) {
   if (M <= 0 || N <= 0 || N % 16 || K % BK || K <= 0 || split_k < 0 || K / BK < split_k) return -2;
-  // 32-bit buffer offsets, rows up to a whole tile past the end included
-  if (2ull * (M + BM) * K >= (1ull << 31) || 2ull * (N + BN) * K >= (1ull << 31)) return -2;
+  // 32-bit buffer offsets, rows up to a whole tile past the end included (the gated form's up rows lie `inter` rows behind its gate
+  // rows however few of them are asked for)
+  const unsigned long long w_rows = epi == EPI_SILU_MUL ? 2ull * inter : static_cast<unsigned long long>(N);
+  if (2ull * (M + BM) * K >= (1ull << 31) || 2 * (w_rows + BN) * K >= (1ull << 31)) return -2;
   // the output (and residual) offsets, a masked column's 0x80000000 bias included, stay 32-bit
   if (2ull * (M + BM) * (epi == EPI_SILU_MUL ? inter : N) >= (1ull << 31)) return -2;
   if (split_k != 1 && (!ws || !counters)) return -2;

@@ -53,3 +53,16 @@ def test_other_modes_split_nothing(mode):
     plan.mode = mode
     for M, N, K, epi in _shapes(2000):
         assert plan.columns(M, N, K) == N and plan.pieces(M, N, K, epi) == [(M, plan.choose(M, N, K, epi))]
+
+
+def test_gated_columns_of_a_weight_past_32_bits():
+    """A few columns of a gated weight whose up rows lie past the 32-bit offsets are refused before any launch (no GPU)."""
+    import ctypes
+    import os
+    from byzantine_consensus_llm_agents_amd.ops.hip import load_library
+    from byzantine_consensus_llm_agents_amd.utils.build import kernels_target
+    if not os.path.exists(kernels_target()):
+        pytest.skip("kernel library not built")
+    one = ctypes.c_void_p(16)
+    for inter, K in ((1 << 20, 1024), (1 << 19, 2048), ((1 << 20) - 128, 1024), (-128, 64)):     # 2 (2 inter + 256) K bytes: 2^31 and more
+        assert load_library().bcg_gemm_nt(W4_CFG, 1, one, one, None, None, one, None, None, 256, 256, K, inter, 1, None) == -2
