@@ -146,35 +146,66 @@ class GemmPlan:
 
         A prefill step has any number of rows, the table a few, and 256 x 256 tiles come in rounds of 256 (one per CU):
         288 tiles cost two rounds.  At row counts that the table does not hold, from LARGE_M on:
-        * a last round that is short goes to the rows it is made of: whole rounds for the first M1 rows, and the
+        * a last round that is short goes to the rows it is made of: (nearly) whole rounds for the first M1 rows, and the
           rest as a GEMM of its own, where that is estimated below 0.6 of a round (4449 x 4096 x 12288, us: library
-          658, one 256 x 256 launch 470, split here 345; 4449 x 4096 x 4096: 138, 172, 117);
-        * whole rounds, or a last one filled to 0.88, stay on the library, which is 3 to 15 % faster there (8183 x 16384 x
-          2048: 373 us against 440; 16098 x 7168 x 5120 and 16098 x 5120 x 17408: 3 % and 6 %);
-        * otherwise the library is erratic and the 256 x 256 kernel is not: taken from 0.82 of its rounds filled on (one
-          full round and a second: 0.88): 8183 x 11264 x 2048: 346 -> 284 us, 8183 x 5056 x 4096: 384 -> 257, 11111 x 4096
-          x 4096: 389 -> 275, 2900 x 24576 x 4096: 544 -> 451; the worst of 14 shapes by 10 row counts: 368 -> 398; and with the gated epilogue, which saves the library a pass, from 0.55
-          (2039 x 9728 x 896: 67 -> 47)."""
+          658, one 256 x 256 launch 470, split here 345).  `_main` says which kernel takes the rounds;
+        * otherwise the 256 x 256 kernel takes all rows where `_large_tiles` says so."""
         choice = self.choose(M, N, K, epi)
         if self.mode != "1" or M < LARGE_M or (M, N, K, epi) in self.table or not self.supported(W4_CFG, M, N, K, epi):
             return [(M, choice)]
         n_t, m_t = -(-N // 256), -(-M // 256)
-        tiles = m_t * n_t
-        rounds, rest = divmod(tiles, CUS)
+        rounds, rest = divmod(m_t * n_t, CUS)
         if rounds and rest:
             m1 = rounds * CUS // n_t
             M1, M2 = 256 * m1, M - 256 * m1
             if (0 < m1 < m_t and m1 * n_t >= 0.94 * rounds * CUS
                     and 12 + 2e-6 * M2 * N * K / 0.8e3 < 0.6 * W4_KTILE_US * K / 64):
-                main = (W4_CFG, 1) if epi == 1 or (m1 * n_t) % CUS else None
+                split, main = self._main(N, epi, rounds, m1 * n_t)
                 if (M1, N, K, epi) in self.table:
-                    main = self.choose(M1, N, K, epi)
-                return [(M1, main), (M2, self.choose(M2, N, K, epi))]
-        filled = tiles / (CUS * (rounds + (rest > 0)))
-        whole = rest == 0 or rest >= 0.88 * CUS
-        if choice is None and (filled >= 0.55 if epi == 1 else rounds and not whole and filled >= (0.88 if rounds == 1 else 0.82)):
+                    split, main = True, self.choose(M1, N, K, epi)
+                if split:
+                    return [(M1, main), (M2, self.choose(M2, N, K, epi))]
+        if choice is None and self._large_tiles(N, K, epi, rounds, rest):
             choice = (W4_CFG, 1)
         return [(M, choice)]
+
+    @staticmethod
+    def _main(N: int, epi: int, rounds: int, tiles: int) -> Tuple[bool, Optional[Tuple[int, int]]]:
+        """(whether to split, the kernel of the rounds) for `tiles` tiles that fill `rounds` rounds but for a few.
+
+        The library's time jumps by up to 1.5 from one row count to the next.  Over 26 weights (N 2048 to 28672, K 768 to 17408,
+        2048 to 16384 rows, 64 row counts each) its good and bad cases go with the number of rounds.  Library on all rows over
+        the split, geometric mean (points slower by over 3 %):
+        * rounds exactly full: the library, 1.08 to 1.39 (0 of 152);
+        * N a multiple of 256: 1, 2 and 4 rounds the library 1.16, 1.21, 1.16 (1 of 94; the 256 x 256 kernel 1.09, 1.15,
+          1.09 with 18), 3 and 5 the 256 x 256 kernel 1.18 and 1.05 (3 of 41; the library 1.05 and 0.93 with 22); from 6 on
+          neither (0.97, 17 of 41);
+        * other N: the 256 x 256 kernel up to 9 rounds, 1.02 to 1.34 (0 of 43), 0.93 to 0.96 beyond;
+        * the gated epilogue, which saves the library a pass: 1.07 to 1.26 (2 of 127)."""
+        if epi == 1:
+            return True, (W4_CFG, 1)
+        if tiles % CUS == 0:
+            return True, None
+        if N % 256:
+            return rounds <= 9, (W4_CFG, 1)
+        return rounds <= 5, (W4_CFG, 1) if rounds in (3, 5) else None
+
+    @staticmethod
+    def _large_tiles(N: int, K: int, epi: int, rounds: int, rest: int) -> bool:
+        """Whether the 256 x 256 kernel takes the library's place on all rows, `rounds` full rounds of tiles and `rest` tiles.
+
+        The same measurements, library over 256 x 256 kernel (points slower by over 3 %):
+        * the gated epilogue: rounds filled to 0.8 and more 1.08 to 1.48 (0 of 402), to 0.65 up to K = 2048 1.06 to 1.15 (1 of 49), to
+          0.55 up to K = 1024 1.19 to 1.53 (0 of 12), both from a full round on; below that 0.86 to 1.04;
+        * N not a multiple of 256: 1.00 to 1.26 at up to 8 rounds (13 of 70), but for 4 (1.01, 8 of 12); below 1 beyond;
+        * N a multiple of 256: four full rounds and half of one, or five and a half (8183 x 11264 x 2048: 369 -> 301 us): 1.10 (10 of 52,
+          the worst 0.91); everywhere else the library is ahead (0.97; rounds 1 and 3: 0.92)."""
+        filled = (rounds * CUS + rest) / (CUS * (rounds + (rest > 0)))
+        if epi == 1:
+            return filled >= (0.8 if not rounds or K > 2048 else 0.65 if K > 1024 else 0.55)
+        if N % 256:
+            return 0 < rest < 0.88 * CUS and rounds in (1, 2, 3, 5, 6, 7, 8) and filled >= (0.88 if rounds == 1 else 0.82)
+        return (rounds == 4 and rest >= CUS // 2) or (rounds == 5 and CUS // 2 <= rest < 5 * CUS // 8)
 
 
 FP8_TABLE = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "engine", "tuned",

@@ -13,7 +13,8 @@ CASES = [(4449, 4096, 12288, 2, [4096, 353]),      # one whole round of tiles, t
          (4449, 4096, 12288, 0, [4096, 353]), (2049, 8192, 4096, 0, [2048, 1]),
          (2560, 32768, 1024, 0, [2560]),           # whole rounds: one run, the library
          (8183, 11264, 2048, 0, [8183]), (2900, 24576, 512, 0, [2900]),
-         (2048, 1792, 1024, 1, [2048]), (2177, 9728, 896, 1, [2177])]
+         (2048, 1792, 1024, 1, [2048]), (2177, 9728, 896, 1, [2177]),
+         (2565, 12800, 896, 0, [2560, 5]), (8706, 7680, 896, 2, [8704, 2])]   # rounds full but for a few tiles on the library
 
 
 @pytest.mark.parametrize("M,N,K,epi,rows", CASES)
