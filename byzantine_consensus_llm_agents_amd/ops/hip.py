@@ -386,12 +386,14 @@ def hip_ops() -> SimpleNamespace:
     def _plain_bias(bias, N, x):
         return bias is None or _plain_beside(bias, (N,), x)
 
-    def _pieces(x, w, epi, others=True):
-        """Runs of rows and their choices (`GemmPlan.pieces`); others: whether the bias / residual lies as the kernels want."""
+    def _pieces(x, w, epi, beside=None, shape=None):
+        """Runs of rows and their choices (`GemmPlan.pieces`); beside: the bias or residual, of this shape.  Fewer rows than LARGE_M are
+        one run whatever the operands are, so nothing is looked at there: a small eager step is bound by the host (24 layers of
+        width 896, 456 rows: 4408 us with the look, 3810 without)."""
         M, K = x.shape
-        if others and _plain(x, w):
-            return plan.pieces(M, w.shape[0], K, epi)
-        return [(M, plan.choose(M, w.shape[0], K, epi))]
+        if M < LARGE_M or not (_plain(x, w) and (beside is None or _plain_beside(beside, shape, x))):
+            return [(M, plan.choose(M, w.shape[0], K, epi))]
+        return plan.pieces(M, w.shape[0], K, epi)
 
     def _skinny(x, w, epi):
         """Whether the few-row kernel takes x W^T: every shape of up to SKINNY_ROWS rows whose rows are whole 128-byte
@@ -421,7 +423,7 @@ def hip_ops() -> SimpleNamespace:
         if not (x.is_contiguous() and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16):
             _log(M, N, K, _epi_log, None)
             return torch.nn.functional.linear(x, w, bias)
-        parts = _pieces(x, w, 0, _plain_bias(bias, N, x))
+        parts = _pieces(x, w, 0, bias, (N,))
         if len(parts) == 1:
             return _linear_rows(x, w, bias, parts[0][1], None, _epi_log)
         out, at = torch.empty(M, N, dtype=x.dtype, device=x.device), 0
@@ -438,7 +440,7 @@ def hip_ops() -> SimpleNamespace:
             return torch.nn.functional.linear(x, w, bias)
         return torch.mm(x, w.t(), out=out) if bias is None else torch.addmm(bias, x, w.t(), out=out)
 
-    from .gemm_plan import PP_CFG, SMALL_CFG, W4_CFG, GemmPlan
+    from .gemm_plan import LARGE_M, PP_CFG, SMALL_CFG, W4_CFG, GemmPlan
     plan = GemmPlan(lib)
 
     # Split-K arrival counters (one int per output tile; the last-arriving workgroup of a
@@ -533,8 +535,8 @@ def hip_ops() -> SimpleNamespace:
         if not (x.is_contiguous() and x.dtype == torch.bfloat16):
             return silu_mul(linear(x, w, _epi_log=1))
         N = w.shape[0]
-        n1 = plan.columns(M, N, K) if _plain(x, w) else N
-        if n1 < N:
+        n1 = plan.columns(M, N, K)
+        if n1 < N and _plain(x, w):
             out = torch.empty(M, N // 2, dtype=x.dtype, device=x.device)
             for cfg, at, n in ((W4_CFG, 0, n1), (SMALL_CFG, n1, N - n1)):   # both halves of w from row at / 2 on
                 _log(M, n, K, 1, (cfg, 1))
@@ -580,7 +582,7 @@ def hip_ops() -> SimpleNamespace:
             return _gemm_skinny(x, w, 2, residual=residual)
         parts = [(M, None)]
         if x.is_contiguous() and x.dtype == torch.bfloat16:
-            parts = _pieces(x, w, 2, _plain_beside(residual, (M, w.shape[0]), x))
+            parts = _pieces(x, w, 2, residual, (M, w.shape[0]))
         at = 0
         for rows, cfg in parts:
             whole = rows == M

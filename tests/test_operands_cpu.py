@@ -76,3 +76,17 @@ def test_traces_and_fakes(ops):
     with FakeTensorMode() as mode:
         assert watched() and ops.linear(mode.from_tensor(x), mode.from_tensor(w)).shape == (3, 36)
     assert not watched() and not bare(mode.from_tensor(x))
+
+
+def test_small_steps_are_not_looked_at(ops, monkeypatch):
+    """From 17 rows to LARGE_M a projection is one run whatever its operands are: no check is paid for there."""
+    from byzantine_consensus_llm_agents_amd.ops import hip
+    from byzantine_consensus_llm_agents_amd.ops.gemm_plan import LARGE_M
+    seen = []
+    monkeypatch.setattr(hip, "bare", lambda t: seen.append(t) or bare(t))
+    w, b = torch.ones(36, 128).bfloat16(), torch.ones(36).bfloat16()
+    for M in (17, 100, LARGE_M - 1):
+        x, r = torch.ones(M, 128).bfloat16(), torch.zeros(M, 36).bfloat16()
+        ops.linear(x, w, b)
+        ops.linear_residual(x, w, r)
+    assert not seen
