@@ -33,6 +33,7 @@ N_CFGS = len(TILES)
 SPLITS = (1, 2, 3, 4, 6, 8)
 CUS = 256
 LARGE_M = 2048    # `pieces`: from here on the row count is a prefill step's
+LONG_K = 10240    # from here on the library's rate follows the rounds less
 W4_KTILE_US = 1.46   # one wave of 256 x 256 tiles: microseconds per 64 of K (512 tiles, K = 4096 .. 17408)
 STREAM_K = 0  # split_k value of the W4 kernel's stream-K launch (one workgroup per CU over tiles x K-tiles)
 
@@ -149,63 +150,76 @@ class GemmPlan:
         * a last round that is short goes to the rows it is made of: (nearly) whole rounds for the first M1 rows, and the
           rest as a GEMM of its own, where that is estimated below 0.6 of a round (4449 x 4096 x 12288, us: library
           658, one 256 x 256 launch 470, split here 345).  `_main` says which kernel takes the rounds;
-        * otherwise the 256 x 256 kernel takes all rows where `_large_tiles` says so."""
+        * otherwise the 256 x 256 kernel takes all rows where `_large_tiles` says so (8183 x 11264 x 2048: library 369 us, here 301;
+          2619 x 16384 x 2048: 167 and 149)."""
         choice = self.choose(M, N, K, epi)
         if self.mode != "1" or M < LARGE_M or (M, N, K, epi) in self.table or not self.supported(W4_CFG, M, N, K, epi):
             return [(M, choice)]
         n_t, m_t = -(-N // 256), -(-M // 256)
-        rounds, rest = divmod(m_t * n_t, CUS)
+        tiles = m_t * n_t
+        rounds, rest = divmod(tiles, CUS)
         if rounds and rest:
             m1 = rounds * CUS // n_t
             M1, M2 = 256 * m1, M - 256 * m1
             if (0 < m1 < m_t and m1 * n_t >= 0.94 * rounds * CUS
                     and 12 + 2e-6 * M2 * N * K / 0.8e3 < 0.6 * W4_KTILE_US * K / 64):
-                split, main = self._main(N, epi, rounds, m1 * n_t)
+                split, main = self._main(N, K, epi, rounds, m1 * n_t, tiles)
                 if (M1, N, K, epi) in self.table:
                     split, main = True, self.choose(M1, N, K, epi)
                 if split:
                     return [(M1, main), (M2, self.choose(M2, N, K, epi))]
-        if choice is None and self._large_tiles(N, K, epi, rounds, rest):
+        if choice is None and self._large_tiles(K, epi, tiles):
             choice = (W4_CFG, 1)
         return [(M, choice)]
 
     @staticmethod
-    def _main(N: int, epi: int, rounds: int, tiles: int) -> Tuple[bool, Optional[Tuple[int, int]]]:
-        """(whether to split, the kernel of the rounds) for `tiles` tiles that fill `rounds` rounds but for a few.
+    def _even(tiles: int) -> bool:
+        """Whether `tiles` tiles of 256 x 256 are the same number for every round that they take.
 
-        The library's time jumps by up to 1.5 from one row count to the next.  Over 26 weights (N 2048 to 28672, K 768 to 17408,
-        2048 to 16384 rows, 64 row counts each) its good and bad cases go with the number of rounds.  Library on all rows over
-        the split, geometric mean (points slower by over 3 %):
-        * rounds exactly full: the library, 1.08 to 1.39 (0 of 152);
-        * N a multiple of 256: 1, 2 and 4 rounds the library 1.16, 1.21, 1.16 (1 of 94; the 256 x 256 kernel 1.09, 1.15,
-          1.09 with 18), 3 and 5 the 256 x 256 kernel 1.18 and 1.05 (3 of 41; the library 1.05 and 0.93 with 22); from 6 on
-          neither (0.97, 17 of 41);
-        * other N: the 256 x 256 kernel up to 9 rounds, 1.02 to 1.34 (0 of 43), 0.93 to 0.96 beyond;
-        * the gated epilogue, which saves the library a pass: 1.07 to 1.26 (2 of 127)."""
-        if epi == 1:
-            return True, (W4_CFG, 1)
-        if tiles % CUS == 0:
-            return True, None
-        if N % 256:
-            return rounds <= 9, (W4_CFG, 1)
-        return rounds <= 5, (W4_CFG, 1) if rounds in (3, 5) else None
+        The library's measured rate has two levels, and this tells them apart up to LONG_K: 6144 x 4096 (N x K), 7678 rows (720
+        tiles, 3 rounds of 240) 1505 TFLOP/s, 4096 x 4096, 11612 rows (736 tiles) 904; the 256 x 256 kernel 1330 and 1415."""
+        return tiles % -(-tiles // CUS) == 0
 
     @staticmethod
-    def _large_tiles(N: int, K: int, epi: int, rounds: int, rest: int) -> bool:
-        """Whether the 256 x 256 kernel takes the library's place on all rows, `rounds` full rounds of tiles and `rest` tiles.
+    def _main(N: int, K: int, epi: int, rounds: int, tiles: int, all_tiles: int) -> Tuple[bool, Optional[Tuple[int, int]]]:
+        """(whether to split, the kernel of the rounds) for `tiles` of `all_tiles` tiles that fill `rounds` rounds but for a few.
 
-        The same measurements, library over 256 x 256 kernel (points slower by over 3 %):
-        * the gated epilogue: rounds filled to 0.8 and more 1.08 to 1.48 (0 of 402), to 0.65 up to K = 2048 1.06 to 1.15 (1 of 49), to
-          0.55 up to K = 1024 1.19 to 1.53 (0 of 12), both from a full round on; below that 0.86 to 1.04;
-        * N not a multiple of 256: 1.00 to 1.26 at up to 8 rounds (13 of 70), but for 4 (1.01, 8 of 12); below 1 beyond;
-        * N a multiple of 256: four full rounds and half of one, or five and a half (8183 x 11264 x 2048: 369 -> 301 us): 1.10 (10 of 52,
-          the worst 0.91); everywhere else the library is ahead (0.97; rounds 1 and 3: 0.92)."""
-        filled = (rounds * CUS + rest) / (CUS * (rounds + (rest > 0)))
+        Library on all rows over the split, geometric mean (points slower by over 3 %), over 150 weights (N 256 to 20480, K 768 to
+        18000) at 2048 to 12288 rows that the rules were not drawn from, 1591 splits: 1.22 (61), the slowest 0.81:
+        * rounds of the same number of tiles go to the library: 1 round 1.33 (9 of 283), 2: 1.32 (0 of 226), 3: 1.24 (0 of 115), more 1.12
+          (8 of 154), the 256 x 256 kernel 3 to 9 % less; but for one round of N not a multiple of 256 (1.42 against 1.30), and from LONG_K on
+          up to 3 rounds (4 and more that are not exactly full: 0.90 to 1.1);
+        * others go to the 256 x 256 kernel, the library being slow there (0.72 to 0.95): 3 rounds 1.13 (7 of 129), more 1.05 to
+          1.09 (23 of 304); not 2 where all rows are even (1.00, 12 of 26), nor past 7 rounds (LONG_K: 5), 0.92 to 1.00;
+        * the gated epilogue saves the library a pass: 1.07 to 1.26 (2 of 127)."""
         if epi == 1:
-            return filled >= (0.8 if not rounds or K > 2048 else 0.65 if K > 1024 else 0.55)
-        if N % 256:
-            return 0 < rest < 0.88 * CUS and rounds in (1, 2, 3, 5, 6, 7, 8) and filled >= (0.88 if rounds == 1 else 0.82)
-        return (rounds == 4 and rest >= CUS // 2) or (rounds == 5 and CUS // 2 <= rest < 5 * CUS // 8)
+            return True, (W4_CFG, 1)
+        if GemmPlan._even(tiles):
+            if N % 256 and rounds == 1:
+                return True, (W4_CFG, 1)
+            return K < LONG_K or rounds <= 3 or tiles % CUS == 0, None
+        if rounds == 2 and N % 256 == 0 and GemmPlan._even(all_tiles):
+            return False, None
+        return rounds <= (7 if K < LONG_K else 5), (W4_CFG, 1)
+
+    @staticmethod
+    def _large_tiles(K: int, epi: int, tiles: int) -> bool:
+        """Whether the 256 x 256 kernel takes the library's place on all rows.
+
+        Library over 256 x 256 kernel (points slower by over 3 %) over the same held-out points:
+        * tiles that are uneven over their rounds: 2 rounds 1.45 (10 of 204), 3: 1.28 (6 of 538), 4: 1.15 (7 of 337), 5: 1.10 (43 of
+          416), 6 to 8 1.07 (21 of 402); less filled ones and more rounds 0.87 to 1.06;
+        * even ones: the library, 0.75 to 0.96; from LONG_K on its rate follows the rounds less, 2 rounds 1.30 (42 of 206), 3: 1.22 (4
+          of 129), 4: 1.09 (11 of 94) between these fillings;
+        * the gated epilogue: rounds filled to 0.8 and more 1.08 to 1.48 (0 of 402), to 0.65 up to K = 2048 1.06 to 1.15 (1 of 49), to
+          0.55 up to K = 1024 1.19 to 1.53 (0 of 12), both from a full round on; below that 0.86 to 1.04."""
+        rounds = -(-tiles // CUS)
+        filled = tiles / (CUS * rounds)
+        if epi == 1:
+            return filled >= (0.8 if rounds == 1 or K > 2048 else 0.65 if K > 1024 else 0.55)
+        if not GemmPlan._even(tiles):
+            return filled >= (0.76 if rounds <= 3 else 0.8 if rounds <= 5 else 0.9) and rounds <= (8 if K < LONG_K else 6)
+        return K >= LONG_K and 2 <= rounds <= 4 and 0.8 <= filled < (0.9 if K < 12000 else 0.95)
 
 
 FP8_TABLE = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "engine", "tuned",

@@ -54,9 +54,12 @@ LIB, LARGE = None, (W4_CFG, 1)
     (4098, 4096, 896, 2, [(4096, LIB), 2]), (8201, 12288, 960, 0, [(8192, LIB), 9]),          # rounds exactly full
     (2820, 5632, 896, 0, [(2816, LIB), 4]), (2565, 12800, 896, 0, [(2560, LIB), 5]), (8706, 7680, 896, 2, [(8704, LIB), 2]),
     (8723, 5632, 896, 2, [(8704, LARGE), 19]), (5384, 15104, 960, 0, [(5376, LARGE), 8]),     # 3 and 5 rounds but for a few tiles
-    (7172, 13568, 960, 0, [(7172, LIB)]),                                                     # 6
+    (7172, 13568, 960, 0, [(7168, LARGE), 4]),                                                # 6
+    (16098, 7168, 960, 0, [(16098, LIB)]), (7678, 6144, 960, 0, [(7678, LIB)]),               # no split: 7 and 3 even rounds
+    (11612, 4096, 960, 0, [(11612, LARGE)]), (2478, 16384, 960, 0, [(2478, LARGE)]),          # 3 uneven ones
+    (9010, 4608, 10304, 0, [(9010, LARGE)]), (9010, 4608, 10176, 0, [(9010, LIB)]),           # 3 even ones, either side of LONG_K
     (2318, 6784, 896, 0, [(2304, LARGE), 14]), (8195, 11792, 896, 0, [(8192, LARGE), 3]),     # N not a multiple of 256
-    (2617, 10304, 512, 0, [(2617, LARGE)]), (7982, 8016, 512, 2, [(7982, LIB)]), (8796, 9232, 512, 0, [(8796, LARGE)]),
+    (2617, 10304, 512, 0, [(2617, LARGE)]), (7982, 8016, 512, 2, [(7982, LIB)]), (8796, 9232, 512, 0, [(8796, LIB)]),
     (7939, 9216, 512, 0, [(7939, LARGE)]), (8183, 11264, 512, 0, [(8183, LARGE)]), (3858, 12544, 512, 0, [(3858, LIB)]),
     (5409, 3072, 896, 1, [(5376, LARGE), 33]), (4462, 4096, 512, 1, [(4462, LARGE)]), (2300, 9728, 2048, 1, [(2300, LARGE)]),
     (2300, 9728, 2112, 1, [(2300, LIB)]), (2300, 8192, 2048, 1, [(2048, LARGE), 252]), (4365, 2048, 512, 1, [(4365, LIB)])])
