@@ -31,7 +31,7 @@ BIG_CFGS = (PP_CFG, W4_CFG)  # 256 x 256 tiles (the register-staged form lost it
 SMALL_CFG = 5  # 64 x 64
 N_CFGS = len(TILES)
 SPLITS = (1, 2, 3, 4, 6, 8)
-CUS = 256
+CUS = 256       # compute units of an MI355X; on a part of one the rounds would be sized wrongly, the results the same
 LARGE_M = 2048    # `pieces`: from here on the row count is a prefill step's
 LONG_K = 10240    # from here on the library's rate follows the rounds less
 W4_KTILE_US = 1.46   # one wave of 256 x 256 tiles: microseconds per 64 of K (512 tiles, K = 4096 .. 17408)

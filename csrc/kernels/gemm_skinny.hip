@@ -5,22 +5,23 @@
 // stream over W, and a CU takes in no more than about 27 GB/s, weights and activations together (measured
 // over N = 4096 .. 151936, K = 896 .. 17408; all CUs: 6.2 TB/s of HBM).  Hence
 //   * even shares: each of the 256 CUs owns N / 256 rows of W, in groups of 4, whatever that number is (20 rows for
-//     N = 5120: blocks of 16 rows would put 320 workgroups on 256 CUs, 24.4 us where this takes 14.6); a tile of
+//     N = 5120: blocks of 16 rows would put 320 workgroups on 256 CUs, 24.4 us where this takes 14.8); a tile of
 //     the matrix instruction that the share does not fill repeats its last row, which costs no traffic;
 //   * as many rows as fit share one read of X: 2 or 4 blocks of 16 rows per workgroup where N allows it;
 //   * the waves of a workgroup share K, each streams its K range straight into registers, two groups of lines in
 //     flight, no barrier in the loop; the partial tiles meet in LDS once, in wave order: the same inputs
 //     give the same bits;
 //   * one load instruction covers 8 rows x 128 bytes, whole cache lines (64-byte pieces of 16 rows, the order of the
-//     matrix instruction, ran at half the rate: the vocabulary projection 484 us, this 260); a DPP rotation
+//     matrix instruction, ran at half the rate: the vocabulary projection 484 us, this 265); a DPP rotation
 //     by 8 lanes puts the halves of two loads in order;
 //   * NORM: the row factor 1 / rms leaves the sum, y = rstd * sum_k (x w)[k] W[n, k]: each wave squares the
 //     fragments that it loads anyway, and the factor is applied to the finished tile.  x * w is rounded to bf16
 //     once, as the separate norm rounds its output once.
 // 10 rows, before (norm kernel + tile GEMM with split-K, or the library) -> now, us: 7168 x 5120 24.6 -> 16.8,
-// 5120 x 5120 17.6 -> 14.6, gate + up 34816 x 5120 90.6 -> 71, 151936 x 5120 277 -> 260, 18432 x 4096 79 -> 32,
-// 4096 x 4096 13.4 -> 10.3, 4096 x 12288 26.1 -> 23, 896 x 896 5.8 -> 4.3, gate + up 9728 x 896 15.4 -> 9.3,
-// 896 x 4864 13.1 -> 8.4.  Not here: M > 16 (X then takes as much of a CU's intake as W: at 20 rows 5120 x
+// 5120 x 5120 17.6 -> 14.8, gate + up 34816 x 5120 90.6 -> 72, 151936 x 5120 277 -> 265, 18432 x 4096 79 -> 33,
+// 4096 x 4096 13.4 -> 10.3, 4096 x 12288 26.1 -> 23, 896 x 896 5.8 -> 4.4, gate + up 9728 x 896 15.4 -> 8.8,
+// 896 x 4864 13.1 -> 8.4; launches back to back, every one with other weights (within a captured step the profiler has 18.2, 15.4, 74
+// and 265 for the first four).  Not here: M > 16 (X then takes as much of a CU's intake as W: at 20 rows 5120 x
 // 5120 took 18.7 against 17.5), K > 12288 (5120 x 17408: 40 against 36.6).
 #include "common.h"
 

@@ -834,7 +834,7 @@ int launch_prefill(const AttnArgs& a, int n_tiles, int tile_rows, hipStream_t s)
   }
     BCG_EXACT1_PLAIN(BCG_X)
 #undef BCG_X
-    if (a.dim == 512 && a.vdim == 512) {   // (two chunks of it do not fit the 64 KiB)
+    if (a.dim == 512 && a.vdim == 512) {   // (two chunks of it take 130 of the CU's 160 KiB: one workgroup per CU; that form is not built)
       prefill_kernel<T, 32, 32, 1, true, true, 1, 1, 1><<<grid, 256, 0, s>>>(a);
       return BCG_CHECK_LAUNCH();
     }

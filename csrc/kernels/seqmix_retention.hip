@@ -26,9 +26,9 @@
 // The walk is a serial chain, so its operands are fetched a chunk ahead into the registers that the phase before has
 // just used up (no wave needs another wave's keys or queries: they do not pass LDS), and VT shrinks where the launch would leave CUs
 // idle.  What bounds it: the fp32 matrix rate (32 cycles per 16 x 16 x 4) where all CUs are busy, else the chain.
-// Measured, both launches: 3 segments of 700 tokens, 8 heads, 128 x 256 states: 89 us (keys, scores and 64-column
-// workgroups in one kernel, 96 workgroups: 202); 8 segments of 1000, 128 heads sharing keys, 128 x 64 states: 494 us (token
-// by token: 1552), of which the matrix rate is 250; 64 segments of 16: 149 (220).
+// Measured, both launches: 3 segments of 700 tokens, 8 heads, 128 x 256 states: 91 us (keys, scores and 64-column
+// workgroups in one kernel, 96 workgroups: 202); 8 segments of 1000, 128 heads sharing keys, 128 x 64 states: 494 to 524 us (token
+// by token: 1552), of which the matrix rate is 250 (in a whole step, 64 heads of 128 x 128: 690); 64 segments of 16: 149 (220).
 // Rounding, against float64 (relative rms, token by token -> here): decays about 0.5: 8.4e-8 -> 7.4e-8, 0.9: 1.1e-7 -> 1.0e-7, 0.99:
 // 2.5e-7 -> 1.2e-7, 0.999: 4.6e-7 -> 1.5e-7.  That takes the scores in double (parallel, so nearly free), decay products in
 // double, and short chains in the fp32 accumulators (one chain over all features and keys: 1.5e-7 at decays about 0.5).
