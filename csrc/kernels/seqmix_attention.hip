@@ -627,9 +627,10 @@ __global__ __launch_bounds__(256, NM * (KC + 2 * VT) <= 24 ? 4 : KC + VT <= 24 ?
   }
 }
 
-// what the copies of whole pages need: one page is a chunk's half, caches on 8 bytes like every 4-element fragment
-inline bool staged_layout(const AttnArgs& a) {
-  return a.swz && a.BS == 16 && ((reinterpret_cast<uintptr_t>(a.k_cache) | reinterpret_cast<uintptr_t>(a.v_cache)) & 7) == 0;
+// what the copies of whole pages need: one page is a chunk's half, caches on 8 bytes like every 4-element fragment; and what its
+// one-dimensional launch holds: fewer than 2^32 threads
+inline bool staged_layout(const AttnArgs& a, int n_tiles) {
+  return a.swz && a.BS == 16 && static_cast<int64_t>(n_tiles) * a.H < (1 << 24) && ((reinterpret_cast<uintptr_t>(a.k_cache) | reinterpret_cast<uintptr_t>(a.v_cache)) & 7) == 0;
 }
 
 template <int KC, int VT, int NM, int MODE>
@@ -789,7 +790,7 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(AttnArgs a) {
 template <typename T, int MODE>
 int launch_prefill_mode(const AttnArgs& a, int n_tiles, bool full, hipStream_t s) {
   dim3 grid(n_tiles, a.H);
-  if constexpr (sizeof(T) == 2) if (full && staged_layout(a)) {
+  if constexpr (sizeof(T) == 2) if (full && staged_layout(a, n_tiles)) {
 #define BCG_X(KC_, VT_, KT_, OCC_)                                                               \
   if (a.dim == 16 * KC_ && a.vdim == 16 * VT_) {                                                 \
     return launch_staged<KC_, VT_, 1, MODE>(a, n_tiles, s);                                      \
@@ -827,7 +828,7 @@ int launch_prefill(const AttnArgs& a, int n_tiles, int tile_rows, hipStream_t s)
   if (tile_rows != 64) return -2;
   if (a.softcap > 0.f || a.slopes != nullptr) return launch_prefill_mode<T, SHAPED>(a, n_tiles, full, s);
   if (a.keep > 0) return launch_prefill_mode<T, KEEP>(a, n_tiles, full, s);
-  if constexpr (sizeof(T) == 2) if (full && a.maps == 1 && staged_layout(a)) {   // one-map heads, exact shapes
+  if constexpr (sizeof(T) == 2) if (full && a.maps == 1 && staged_layout(a, n_tiles)) {   // one-map heads, exact shapes
 #define BCG_X(KC_, VT_, KT_, OCC_)                                                               \
   if (a.dim == 16 * KC_ && a.vdim == 16 * VT_) {                                                 \
     return launch_staged<KC_, VT_, 1, PLAIN>(a, n_tiles, s);                                     \
@@ -840,7 +841,7 @@ int launch_prefill(const AttnArgs& a, int n_tiles, int tile_rows, hipStream_t s)
     }
   }
   if constexpr (sizeof(T) == 2) if (small) {
-    const bool exact = full && a.maps == 2 && staged_layout(a);
+    const bool exact = full && a.maps == 2 && staged_layout(a, n_tiles);
 #define BCG_EXACT(KC_, VT_)                                                                      \
   if (exact && a.dim == 16 * KC_ && a.vdim == 16 * VT_) {                                        \
     return launch_staged<KC_, VT_, 2, PLAIN>(a, n_tiles, s);                                     \

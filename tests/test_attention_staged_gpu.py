@@ -57,3 +57,15 @@ def test_caches_off_16_bytes(ops):
     off = [torch.cat([x.new_zeros(4), x.flatten()])[4:].view(x.shape) for x in (kl, vl)]
     assert all(x.data_ptr() % 16 == 8 for x in off)
     assert torch.equal(ops.multimap_attention(q, *off, meta, *args), ops.multimap_attention(q, kl, vl, meta, *args))
+
+
+def test_more_workgroups_than_one_dimension_holds(ops):
+    """2^24 tiles x heads of 256 threads do not fit a one-dimensional launch: such calls keep the general instances."""
+    H = 17
+    k, v, meta, T = _paged([16], [16], 16, 1, 32, 32, torch.bfloat16, seed=3)
+    q = torch.randn(T, H, 32, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16).to(k.device)
+    args = (32 ** -0.5, 1, 0.0, -1.0, 1.0, 32)
+    want = ops.multimap_attention(q, *ops.kv_from_logical(k, v), meta, *args)
+    meta.tiles = torch.cat([meta.tiles, torch.tensor([[0, 0, 0]], dtype=torch.int32, device=k.device).expand((1 << 24) // H, 3)]).contiguous()
+    got = ops.multimap_attention(q, *ops.kv_from_logical(k, v), meta, *args)
+    torch.testing.assert_close(got, want, rtol=2e-2, atol=2e-2)
