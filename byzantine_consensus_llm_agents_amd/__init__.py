@@ -1,6 +1,6 @@
 """MI355X-native Byzantine Consensus Game framework.
 
-Layers (see SURVEY.md §1 for the reference's layer map):
+Layers:
   bcg/       simulation layer, API-compatible with the reference
   engine/    in-process inference engine (scheduler, paged KV, JSON FSM, sampler)
   models/    Qwen3 / Qwen2 / Mistral decoders (TP-aware), weight loaders

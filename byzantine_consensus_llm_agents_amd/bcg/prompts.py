@@ -1,6 +1,6 @@
 """Prompt texts and JSON schemas of the BCG agents.
 
-The prompt *bytes* are part of the behavioural contract (SURVEY.md §2.4 item 6):
+The prompt *bytes* are part of the behavioural contract:
 they must match the reference exactly so that consensus-rate experiments are
 comparable.  Sources: honest system prompts ``bcg/bcg_agents.py:361-431``,
 honest round prompt ``:452-471``, honest vote prompts ``:484-571``, Byzantine

@@ -8,7 +8,7 @@ Round structure (reference ``run_round`` :517-658):
   store reasoning -> vote (one batched call, retries) -> game.advance_round ->
   network.advance_round.
 
-Retry ladder (reference :256-478, SURVEY §2.4 item 4): after a batch attempt,
+Retry ladder (reference :256-478): after a batch attempt,
 if the failed fraction is <= 30% and attempts remain, the failed agents run
 their own sequential 3-attempt path and the ladder stops; otherwise the failed
 subset is re-batched (max 3 batch attempts).  Failed decides abstain, failed

@@ -2,7 +2,7 @@
 
 The reference's experiments were cluster sweeps of independent runs driven
 through ``run_simulation`` (``bcg/main.py:1073-1141``; the driver itself is
-not in the repo, SURVEY.md §2.2 "DP over seeds", §7.2 step 6).  Here one
+not in the repo).  Here one
 launch covers the whole sweep:
 
 * one process per GPU (``torchrun``), TP groups of ``--tp`` consecutive ranks
@@ -16,9 +16,9 @@ launch covers the whole sweep:
   ``game.game_over``) with a seeded ``ByzantineConsensusGame``;
 * rank 0 gathers every game's ``get_statistics()`` and writes one JSON: the
   consensus-outcome distribution (valid / invalid / none / timeout -- the
-  BASELINE.md quality-parity metric), mean rounds / quality score, and
+  quality-parity metric), mean rounds / quality score, and
   decisions per second over the node;
-* checkpoint / resume (the reference has neither, SURVEY.md §5.4): every
+* checkpoint / resume (the reference has neither): every
   finished game is appended to ``<out>.rank<R>.jsonl`` as it completes;
   ``--resume`` reloads all those records and only plays the missing seeds.
 

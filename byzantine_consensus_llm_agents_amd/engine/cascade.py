@@ -2,8 +2,8 @@
 
 With prefix caching, every agent's system prompt + chat header is computed once and its
 full KV blocks are handed to every later request with the same prompt prefix -- the same
-agent role in every concurrent game (SURVEY §2.3 K-ATTN-D; ``engine/engine.py`` admission).
-In the driver's bench ~40 % of a decode row's context sits in such shared blocks, and the
+agent role in every concurrent game (``engine/engine.py`` admission).
+In the served benchmark ~40 % of a decode row's context sits in such shared blocks, and the
 per-row decode kernel streams them once per row: the same bytes, ~20-100 times per step.
 
 ``plan_groups`` groups the live rows whose leading physical block ids coincide;

@@ -245,8 +245,7 @@ class InferenceEngine:
         self.graphs = None
         # Prefill runs on the engine's one stream between decode bursts.  (A second prefill
         # stream concurrent with the bursts lost three A/Bs, the last -2.9 % tokens/s: every
-        # 256x256 GEMM holds a CU's whole LDS, so the two streams only time-share the CUs --
-        # PERF.md "Overlapped prefill"; removed in round 5.)
+        # 256x256 GEMM holds a CU's whole LDS, so the two streams only time-share the CUs.)
         if hasattr(self.ops, "prepare_device"):  # split-K counters: allocated before any graph capture
             self.ops.prepare_device(self.device)
         self._skip_done_attn = os.environ.get("BCG_SKIP_DONE_ATTN", "1") != "0"

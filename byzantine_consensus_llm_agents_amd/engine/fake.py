@@ -1,6 +1,6 @@
 """Scripted engine backend: schema-valid JSON without a model.
 
-Used for CPU plumbing runs (BASELINE config 1 without weights) and for the
+Used for CPU plumbing runs (four agents of the smallest model, without weights) and for the
 parity tests, where the *same* function answers both the reference (through a
 stub ``vllm`` package, ``tools/gen_golden.py``) and this framework, so that the
 two simulators can be diffed on identical engine outputs.
@@ -235,7 +235,7 @@ class BurnInLLM:
 class HostModelBackend:
     """Engine stand-in that does the real engine's HOST work and models its GPU time.
 
-    For measuring whether the host keeps up with several DP ranks per node (VERDICT r3 item 8):
+    For measuring whether the host keeps up with several DP ranks per node:
     every call tokenizes its prompts with the model's tokenizer, produces schema-valid outputs
     of the measured mean lengths (:class:`BurnInLLM`; votes drawn by :func:`scripted_object`, so
     games do end), re-tokenizes and detokenizes them (the engine's sampler produces ids, the

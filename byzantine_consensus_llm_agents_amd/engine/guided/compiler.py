@@ -5,7 +5,7 @@ a single ``int16 [rows, vocab]`` device tensor (``table``) plus a per-row
 ``dist`` vector.  A decoding sequence carries ``(fsm_base, fsm_state)``; the
 sampling kernel reads ``table[fsm_base + fsm_state]`` -- so any mix of
 schemas shares one batch (the fix for the reference's batch-size-1
-fallback, SURVEY.md §0).
+fallback).
 """
 
 import hashlib

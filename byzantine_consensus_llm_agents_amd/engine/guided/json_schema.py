@@ -1,6 +1,6 @@
 """JSON Schema -> byte-level regular AST (the language guided decoding enforces).
 
-Covers what the BCG agents use (SURVEY.md §2.4 item 2) and the common rest:
+Covers what the BCG agents use and the common rest:
 objects (properties emitted in schema order, required/optional,
 ``additionalProperties: false``), strings (full JSON escapes, UTF-8
 validated, optional ``enum``/``maxLength``), integers with exact
@@ -70,7 +70,7 @@ def validity_aware(schema: Dict, min_visible: int = 10, ascii_text: bool = False
     multi-byte characters that re-tokenise at several tokens per character once the game
     quotes them in later prompts (reasoning [:200], strategies 5 x 400 chars), and late-game
     prompts run into the context limit -- far outside the reference's bounded prompt sizes
-    (SURVEY 5.7: ~0.6-2.5k tokens).  Idempotent (TP followers re-apply it to the key)."""
+    (~0.6-2.5k tokens).  Idempotent (TP followers re-apply it to the key)."""
     if not isinstance(schema, dict):
         return schema
     out = dict(schema)

@@ -1,7 +1,7 @@
-"""Decoder architectures served by the engine (shapes from SURVEY.md §2.3).
+"""Decoder architectures served by the engine (their published shapes).
 
 One ``ModelConfig`` describes every family the reference can select
-(``bcg/config.py:20-25``) plus the plumbing model of BASELINE config 1:
+(``bcg/config.py:20-25``) plus the plumbing model of the four-agent game:
 
 * Qwen3 8B/14B/32B - GQA, per-head QK-RMSNorm, no QKV bias, untied head;
 * Qwen2.5-0.5B     - QKV bias, tied embeddings, no QK-norm;

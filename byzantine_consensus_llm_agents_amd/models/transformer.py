@@ -7,7 +7,7 @@ One forward serves both phases:
 * decode  - one token per sequence (``T = B``), captured into a HIP graph by
   the engine.
 
-Per layer (SURVEY.md §3.3): fused residual-add+RMSNorm -> QKV GEMM -> fused
+Per layer: fused residual-add+RMSNorm -> QKV GEMM -> fused
 QK-norm+RoPE+paged-KV-write (HIP) -> paged attention (HIP, MFMA) -> o_proj GEMM
 [-> all-reduce fused with the next add+RMSNorm] -> gate_up GEMM with SiLU*mul in its
 epilogue -> down GEMM [-> all-reduce fused with the next add+RMSNorm]; at TP=1 the

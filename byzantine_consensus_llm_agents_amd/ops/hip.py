@@ -3,8 +3,8 @@
 Every wrapper validates dtypes, contiguity and shapes on the host before it
 launches (a kernel that indexes out of bounds can take down every GPU of the
 node), then launches on the current HIP stream -- so the calls are captured
-by ``torch.cuda.graph`` like any PyTorch op.  A missing library raises: on a
-GPU box the engine never silently falls back to the PyTorch references.
+by ``torch.cuda.graph`` like any PyTorch op.  A missing library raises: with a
+GPU the engine never silently falls back to the PyTorch references.
 """
 
 import ctypes
@@ -360,7 +360,7 @@ def hip_ops() -> SimpleNamespace:
         ok = rows in (128, 256) and hd == 128 and not kv_fp8 and max_blocks <= PREFILL32_MAX_BLOCKS
         return rows if ok else 64
 
-    # Per-call GEMM dispatch log (VERDICT r3: which projection shapes reach a hand kernel, also
+    # Per-call GEMM dispatch log (which projection shapes reach a hand kernel, also
     # inside TP worker processes that no profiler sees): (M, N, K, epi, dtype) -> choice -> calls.
     # Off unless enabled (BCG_GEMM_LOG=1 or dispatch_log.enable()); graph-captured calls are
     # logged once, at capture (the replays run the same kernels).
@@ -449,7 +449,7 @@ def hip_ops() -> SimpleNamespace:
     # shared by eager launches and every captured decode graph, which replay on that stream
     # one after another -- and one per registered side stream.  Buffers are allocated eagerly
     # by `prepare_device` / `register_stream`, never inside a graph capture: a zero-fill captured into one bucket's graph would leave the
-    # buffer uninitialised for every other graph (ADVICE r2).
+    # buffer uninitialised for every other graph.
     counters = {}       # device index -> int32 [65536]
     side_counters = {}  # (device index, stream handle) -> int32 [65536]
 

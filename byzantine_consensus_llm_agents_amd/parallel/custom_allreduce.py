@@ -1,7 +1,7 @@
 """One-shot / two-shot all-reduce over xGMI peer memory (``csrc/kernels/allreduce.hip``).
 
 The reference's TP collectives are NCCL all-reduces inside vLLM
-(``bcg/vllm_agent.py:131,139-142``; SURVEY.md §2.2, §2.3 K-COLL).  On an
+(``bcg/vllm_agent.py:131,139-142``).  On an
 MI355X node every GPU has a direct xGMI link to each of the other seven, so a
 ring (RCCL's default) is per-link bound and pays n-1 latency hops.  Decode
 messages are small -- ``[B, hidden]`` bf16, 10-2000 KiB -- so here each rank

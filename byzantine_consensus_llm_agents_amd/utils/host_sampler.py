@@ -1,5 +1,5 @@
 """Where a rank's host CPU goes: a low-rate sampler of the engine thread's Python stack and of
-every OS thread's run state (bench.py, env BCG_HOST_SAMPLE=1; VERDICT r4 item 3).
+every OS thread's run state (bench.py, env BCG_HOST_SAMPLE=1).
 
 `time.thread_time` per thread says how much CPU each thread used, not on what.  This samples,
 every `interval` seconds:

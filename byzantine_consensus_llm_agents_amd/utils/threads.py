@@ -1,4 +1,4 @@
-"""Per-rank host thread budget (VERDICT r4 item 3): bench.py and bcg/sweep.py call it before
+"""Per-rank host thread budget: bench.py and bcg/sweep.py call it before
 torch or the tokenizer start their pools.  No torch import here."""
 
 import os

@@ -1,4 +1,4 @@
-"""Per-phase wall-clock timers and roctx ranges (SURVEY.md §5.1: the reference has none).
+"""Per-phase wall-clock timers and roctx ranges (the reference has none).
 
 ``PhaseTimer.phase(name)`` accumulates host wall time per phase (tokenize,
 fsm_compile, prefill, sample, decode, detokenize ...).  With
