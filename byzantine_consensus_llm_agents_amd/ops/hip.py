@@ -21,7 +21,9 @@ _LIB = None
 PREFILL_TILE_ROWS = 128
 PREFILL32_MAX_BLOCKS = 1024  # csrc/kernels/attention.hip: the 32x32 kernel's LDS block-id table
 
-SKINNY_ROWS, SKINNY_MAX_K = 16, 12288  # csrc/kernels/gemm_skinny.hip
+# csrc/kernels/gemm_skinny.hip: most rows, most rows with a fused norm, longest rows in bytes
+SKINNY_ROWS, SKINNY_NORM_ROWS, SKINNY_ROW_BYTES = 32, 16, 65536
+SKINNY_LONG_K = 12288  # past it: fewer shapes gain (`_few_rows_pay`), logged apart
 
 c_int, c_float, c_void_p, c_uint32, c_int64 = ctypes.c_int, ctypes.c_float, ctypes.c_void_p, ctypes.c_uint32, ctypes.c_int64
 
@@ -95,6 +97,7 @@ def load_library(path: str = None) -> ctypes.CDLL:
                             c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
         "bcg_gemm_skinny": [c_int, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
                             c_void_p],
+        "bcg_gemm_skinny_fp8": [c_int] + [c_void_p] * 7 + [c_int] * 3 + [c_void_p],
         "bcg_gemm_tile": [c_int, ctypes.POINTER(c_int), ctypes.POINTER(c_int)],
         "bcg_gemm_num_cfgs": [],
         "bcg_embed_scale_rmsnorm": [c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_float, c_float, c_void_p, c_void_p,
@@ -395,18 +398,32 @@ def hip_ops() -> SimpleNamespace:
             return [(M, plan.choose(M, w.shape[0], K, epi))]
         return plan.pieces(M, w.shape[0], K, epi)
 
+    def _few_rows_pay(M, N, row_bytes, epi):
+        """Whether M <= SKINNY_ROWS rows gain by the few-row kernel.  Each CU reads all of X for its N / 256 rows of W, so few long
+        rows of W lose to a split of K over the CUs (us, tile kernels or library and this one):
+        * up to 16 rows only the gated form past 12288 columns of bf16 (1024 x 16384 22.2, 25.3; 5120 x 25600 138, 48);
+        * 17 to 32 rows: rows of up to 8192 bytes always gain (256 x 4096 11.2, 8.7; 2048 x 4096 14.7, 9.0), longer ones from 4096
+          rows of W on (4096 x 12288 26.0, 24.9; but 3072 x 16384 28.5, 29.3; 1024 x 6144 10.5, 11.7; 256 x 8192 8.7, 14.6)."""
+        if M <= 16:
+            return epi != 1 or row_bytes <= 2 * SKINNY_LONG_K or N >= 4096
+        return row_bytes <= 8192 or N >= 4096
+
     def _skinny(x, w, epi):
-        """Whether the few-row kernel takes x W^T: every shape of up to SKINNY_ROWS rows whose rows are whole 128-byte
-        lines (csrc/kernels/gemm_skinny.hip holds both sides' times); table and library keep the others."""
+        """Whether the few-row kernel takes x W^T: up to SKINNY_ROWS rows of whole 128-byte lines, where they pay (csrc/kernels/
+        gemm_skinny.hip holds more of both sides' times); table and library keep the others."""
         M, K = x.shape
         N = w.shape[0]
-        return (plan.mode == "1" and 1 <= M <= SKINNY_ROWS and K % 64 == 0 and 64 <= K <= SKINNY_MAX_K
-                and N >= 8 and N % (8 if epi == 1 else 4) == 0 and _plain(x, w))
+        return (plan.mode == "1" and 1 <= M <= SKINNY_ROWS and K % 64 == 0 and 64 <= K <= SKINNY_ROW_BYTES // 2
+                and N >= 8 and N % (8 if epi == 1 else 4) == 0 and _few_rows_pay(M, N, 2 * K, epi) and _plain(x, w))
+
+    def _skinny_name(M, K):
+        """("skinny", blocks of 16 rows) in the dispatch log."""
+        return ("skinny" if K <= SKINNY_LONG_K else "skinny_long", -(-M // 16))
 
     def _gemm_skinny(x, w, epi=0, bias=None, residual=None, norm_w=None, eps=0.0):
         M, K = x.shape
         N = w.shape[0]
-        _log(M, N, K, epi, ("skinny", 1))
+        _log(M, N, K, epi, _skinny_name(M, K))
         out = residual if epi == 2 else torch.empty(M, N // 2 if epi == 1 else N, dtype=x.dtype, device=x.device)
         _check(lib.bcg_gemm_skinny(epi, _p(x), _p(w), None if norm_w is None else _p(norm_w), eps,
                                    None if bias is None else _p(bias), None if residual is None else _p(residual), _p(out),
@@ -558,7 +575,7 @@ def hip_ops() -> SimpleNamespace:
         return out
 
     def _norm_fusable(x, w_norm):
-        return x.shape[1] <= 8192 and _plain_beside(w_norm, (x.shape[1],), x)
+        return x.shape[0] <= SKINNY_NORM_ROWS and x.shape[1] <= 8192 and _plain_beside(w_norm, (x.shape[1],), x)
 
     def norm_linear(x, w_norm, eps, w, bias=None):
         """linear(rmsnorm(x, w_norm, eps), w, bias), one kernel for a few rows."""
@@ -721,10 +738,32 @@ def hip_ops() -> SimpleNamespace:
     fp8_plan = Fp8Plan(plan.tiles)
     fp8_cfg = fp8_plan.choose
 
+    def _skinny_fp8(xq, xs, wq, ws, *beside):
+        """Whether the few-row kernel takes the fp8 product: as `_skinny`; `beside`: [(bias or residual, its shape)]."""
+        M, K = xq.shape
+        N = wq.shape[0]
+        return (plan.mode == "1" and 1 <= M <= SKINNY_ROWS and K % 128 == 0 and 128 <= K <= SKINNY_ROW_BYTES and N >= 16 and N % 16 == 0
+                and _few_rows_pay(M, N, K, 0) and xq.is_cuda and xq.get_device() == torch.cuda.current_device() and xq.is_contiguous() and wq.is_contiguous()
+                and all(t.device == xq.device and t.data_ptr() % 16 == 0 and bare(t) for t in (xq, wq, xs, ws))
+                and xs.dtype == ws.dtype == torch.float32 and xs.numel() == M and ws.numel() == N and xs.is_contiguous()
+                and ws.is_contiguous() and not watched()
+                and all(t is None or _plain_beside(t, shape, xq) for t, shape in beside))
+
+    def _gemm_skinny_fp8(xq, xs, wq, ws, epi=0, bias=None, residual=None):
+        M, K = xq.shape
+        N = wq.shape[0]
+        _log(M, N, K, epi, _skinny_name(M, K), "fp8")
+        out = residual if epi == 2 else torch.empty(M, N, dtype=torch.bfloat16, device=xq.device)
+        _check(lib.bcg_gemm_skinny_fp8(epi, _p(xq), _p(wq), _p(xs), _p(ws), None if bias is None else _p(bias),
+                                       None if residual is None else _p(residual), _p(out), M, N, K, _stream()), "gemm_skinny_fp8")
+        return out
+
     def linear_fp8(xq, xs, wq, ws, bias=None, out_dtype=torch.bfloat16):
         """fp8 projection with row-wise activation and per-channel weight scales: the hand
         fp8 MFMA kernel for decode-sized M, hipBLASLt (torch._scaled_mm) otherwise."""
         _req(xq.dtype == f8 and wq.dtype == f8 and xq.shape[1] == wq.shape[1], "linear_fp8 operands")
+        if out_dtype == torch.bfloat16 and _skinny_fp8(xq, xs, wq, ws, (bias, (wq.shape[0],))):
+            return _gemm_skinny_fp8(xq, xs, wq, ws, 0, bias)
         cfg = None
         if out_dtype == torch.bfloat16 and xq.is_contiguous() and wq.is_contiguous():
             cfg = fp8_cfg(xq.shape[0], wq.shape[0], xq.shape[1])
@@ -739,6 +778,8 @@ def hip_ops() -> SimpleNamespace:
         update in the hand fp8 kernel's epilogue (hipBLASLt + a separate add otherwise)."""
         _req(residual.dtype == torch.bfloat16 and residual.is_contiguous()
              and residual.shape == (xq.shape[0], wq.shape[0]), "linear_fp8_residual: residual [M,N] bf16")
+        if xq.dtype == wq.dtype == f8 and _skinny_fp8(xq, xs, wq, ws, (residual, residual.shape)):
+            return _gemm_skinny_fp8(xq, xs, wq, ws, 2, residual=residual)
         if xq.is_contiguous() and wq.is_contiguous():
             cfg = fp8_cfg(xq.shape[0], wq.shape[0], xq.shape[1])
             if cfg is not None:

@@ -1,28 +1,33 @@
-// Projection GEMM of a few rows: C[M, N] = X[M, K] . W[N, K]^T for M <= 16, with the RMS norm of the input, the
-// gated unit and the residual update fused (a decode step of one game: 4 to 16 agents).
+// Projection GEMM of a few rows: C[M, N] = X[M, K] . W[N, K]^T for M <= 32 in bf16 or fp8 (e4m3, row and column scales), with
+// the RMS norm of the input, the gated unit and the residual update fused (a decode step of one to three games).
 //
-// What bounds it: every weight byte is read once and meets at most 16 activation rows, so the kernel is a
-// stream over W, and a CU takes in no more than about 27 GB/s, weights and activations together (measured
-// over N = 4096 .. 151936, K = 896 .. 17408; all CUs: 6.2 TB/s of HBM).  Hence
-//   * even shares: each of the 256 CUs owns N / 256 rows of W, in groups of 4, whatever that number is (20 rows for
-//     N = 5120: blocks of 16 rows would put 320 workgroups on 256 CUs, 24.4 us where this takes 14.8); a tile of
-//     the matrix instruction that the share does not fill repeats its last row, which costs no traffic;
-//   * as many rows as fit share one read of X: 2 or 4 blocks of 16 rows per workgroup where N allows it;
-//   * the waves of a workgroup share K, each streams its K range straight into registers, two groups of lines in
-//     flight, no barrier in the loop; the partial tiles meet in LDS once, in wave order: the same inputs
-//     give the same bits;
-//   * one load instruction covers 8 rows x 128 bytes, whole cache lines (64-byte pieces of 16 rows, the order of the
-//     matrix instruction, ran at half the rate: the vocabulary projection 484 us, this 265); a DPP rotation
-//     by 8 lanes puts the halves of two loads in order;
+// What bounds it: every weight byte is read once and meets at most 32 activation rows, so the kernel is a stream over W.  Plain
+// streaming loads of such weights reach 6.7 TB/s at 356 MB and 6.1 at 84 MB, launch included; the rest is what a CU takes in:
+// X comes from L2 once per CU, and a CU's load path follows the address quads: four neighbouring lanes that read 64 bytes of
+// one row cost a quarter of four that read 16 bytes of four rows (the order of the matrix instruction): 117 and 36 B/ns per CU
+// out of L2.  Hence
+//   * even shares: each of the 256 CUs owns N / 256 rows of W, in groups of 4, whatever that number is (blocks of 16 rows would
+//     put 320 workgroups on 256 CUs for N = 5120), as one workgroup that streams its rows pass after pass (up to 8 blocks of 16
+//     rows at once): the next pass's loads are in flight while a pass is reduced and written (34816 x 5120 gated, 10 rows:
+//     three workgroups per CU, one after the other, 74 us, so 59; 151936 x 5120 265 -> 234);
+//   * the waves of a workgroup share K in turns, unit by unit: neighbouring waves read neighbouring lines (4 % over
+//     a contiguous part of K per wave); no barrier in the loop, every register is loaded again as soon as it has been
+//     consumed; the partial tiles meet in LDS once per pass, in wave order: the same inputs give the same bits;
+//   * a unit of K is 256 bytes: a load takes 64 bytes of each of 16 (row, segment) pairs, and a 4 x 4 transposition within
+//     quads of lanes makes the operands of four matrix instructions (5120 x 17408 with 10 rows 36.2 -> 31.9 us, fp8 6144 x 16384
+//     with 20 rows 25.2 -> 20.8).  Short rows and shares of 4 columns use units of 128 bytes, 8 rows a load and one rotation by 8
+//     lanes (9728 x 896 gated 8.1 -> 7.3, 896 x 4864 8.6 -> 7.7): with 7 units of 256 bytes a wave has nothing to overlap;
+//   * rows past the share, past M and past K lie outside the buffer descriptors: they read as zeros without traffic;
 //   * NORM: the row factor 1 / rms leaves the sum, y = rstd * sum_k (x w)[k] W[n, k]: each wave squares the
 //     fragments that it loads anyway, and the factor is applied to the finished tile.  x * w is rounded to bf16
 //     once, as the separate norm rounds its output once.
-// 10 rows, before (norm kernel + tile GEMM with split-K, or the library) -> now, us: 7168 x 5120 24.6 -> 16.8,
-// 5120 x 5120 17.6 -> 14.8, gate + up 34816 x 5120 90.6 -> 72, 151936 x 5120 277 -> 265, 18432 x 4096 79 -> 33,
-// 4096 x 4096 13.4 -> 10.3, 4096 x 12288 26.1 -> 23, 896 x 896 5.8 -> 4.4, gate + up 9728 x 896 15.4 -> 8.8,
-// 896 x 4864 13.1 -> 8.4; launches back to back, every one with other weights (within a captured step the profiler has 18.2, 15.4, 74
-// and 265 for the first four).  Not here: M > 16 (X then takes as much of a CU's intake as W: at 20 rows 5120 x
-// 5120 took 18.7 against 17.5), K > 12288 (5120 x 17408: 40 against 36.6).
+// 10 rows, us, one workgroup per pass and 128-byte units -> now: 7168 x 5120 18.1 -> 16.4, 5120 x 5120 14.7 -> 12.4, gate + up 34816 x
+// 5120 74.5 -> 59.8, 151936 x 5120 265 -> 234, 4096 x 4096 10.3 -> 9.2, 4096 x 12288 23 -> 18.7, 5120 x 17408 (tile kernel 36.6) 31.9.
+// 20 rows, tile kernel with split-K -> now: fp8 8192 x 6144 15.4 -> 11.6, 6144 x 6144 14.8 -> 10.5, 32768 x 6144 38.5 -> 35.1, 6144 x
+// 16384 27.4 -> 20.8; bf16 32768 x 6144 75.4 -> 68.6.  Launches in a graph, every one with other weights.  From 33 rows on X takes
+// more of a CU's intake than W (64 rows, 4096 x 4096: 14 to 15 us, the tile kernel 14).
+#include <type_traits>
+
 #include "common.h"
 
 namespace {
@@ -30,9 +35,12 @@ namespace {
 enum Epilogue { EPI_STORE = 0, EPI_SILU_MUL = 1, EPI_RESIDUAL = 2 };
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x8 __attribute__((ext_vector_type(8)));
 
-constexpr int CUS = 256;
-constexpr int MAX_ROWS = 16, MAX_K = 12288;
+constexpr int CUS = 256, NW = 8;             // workgroups, waves of one
+constexpr int MAX_ROWS = 32, MAX_NORM_ROWS = 16, MAX_ROW_BYTES = 65536, MAX_NORM_K = 16384;
+constexpr uint32_t PAST_END = 0x80000000u;   // an offset outside every descriptor
+constexpr int ROUND_KB = 64;                 // LDS of one round of a reduction
 
 struct SkinnyArgs {
   const uint8_t* x;        // [M, K]
@@ -41,14 +49,16 @@ struct SkinnyArgs {
   const bf16_t* bias;      // [N] or null
   const bf16_t* residual;  // [M, N] (EPI_RESIDUAL)
   bf16_t* c;
-  int M, row_bytes, ldc, inter, units;   // units: groups of 4 output columns
+  const float* x_scale;    // [M], [N] (F8)
+  const float* w_scale;
+  int M, row_bytes, ldc, inter, units, passes;   // units: groups of 4 output columns
   float eps, inv_k;
 };
 
 __device__ __forceinline__ float silu(float g) { return g * __builtin_amdgcn_rcpf(1.f + __expf(-g)); }
 
 // (x * w) of 8 bf16, rounded to bf16; the squares of x are added to `ss`.
-__device__ __forceinline__ bf16x8 scale_fragment(u32x4 x, u32x4 w, float& ss) {
+__device__ __forceinline__ u32x4 scale_fragment(u32x4 x, u32x4 w, float& ss) {
   bf16x8 out;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -58,207 +68,389 @@ __device__ __forceinline__ bf16x8 scale_fragment(u32x4 x, u32x4 w, float& ss) {
     out[2 * i] = static_cast<__bf16>(lo * __uint_as_float(w[i] << 16));
     out[2 * i + 1] = static_cast<__bf16>(hi * __uint_as_float(w[i] & 0xffff0000u));
   }
-  return out;
+  return __builtin_bit_cast(u32x4, out);
 }
 
-// Two loads cover 16 rows x 128 bytes, whole lines: `a` rows 0-7, `b` rows 8-15, lanes r and r + 8 of a
-// 16-lane group the two halves of a line.  Swapping lanes r and r ^ 8 leaves the MFMA order: `a` = row r, 16-byte
-// chunk kg, `b` = row r, chunk 4 + kg.
-__device__ __forceinline__ void to_rows(u32x4& a, u32x4& b) {
+// 256-byte units.  Load i of a block takes rows 4 g + i (g = lane bits 2, 3), lane bits 4, 5 the 64-byte segment, the quad
+// its four 16-byte chunks.  out[j] of lane q of a quad = in[q] of the quad's lane j: row 4 g + q = lane & 15, chunk j.
+// One select per dword and stage takes its other side from the neighbour (hipcc makes branches of it).  A VALU result is
+// read through DPP, and by a matrix instruction, two wait states later at the earliest: hipcc knows that of its own
+// instructions only, so the block keeps the distance on both sides.
+__device__ __forceinline__ void to_operand(const u32x4 (&in)[4], u32x4 (&out)[4]) {
+  const uint64_t odd = 0xaaaaaaaaaaaaaaaaull, even = ~odd, hi = 0xccccccccccccccccull, lo = ~hi;
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    uint32_t t0, t1, t2, t3, o0, o1, o2, o3;
+    asm("s_nop 1\n\t"
+        "s_mov_b64 vcc, %[odd]\n\t"
+        "v_cndmask_b32_dpp %[t1], %[a], %[b], vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %[t3], %[c], %[d], vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "s_mov_b64 vcc, %[even]\n\t"
+        "v_cndmask_b32_dpp %[t0], %[b], %[a], vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %[t2], %[d], %[c], vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "s_mov_b64 vcc, %[hi]\n\t"
+        "s_nop 0\n\t"
+        "v_cndmask_b32_dpp %[o3], %[t1], %[t3], vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %[o2], %[t0], %[t2], vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "s_mov_b64 vcc, %[lo]\n\t"
+        "v_cndmask_b32_dpp %[o1], %[t3], %[t1], vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %[o0], %[t2], %[t0], vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\t"
+        : [t0] "=&v"(t0), [t1] "=&v"(t1), [t2] "=&v"(t2), [t3] "=&v"(t3), [o0] "=&v"(o0), [o1] "=&v"(o1), [o2] "=&v"(o2), [o3] "=&v"(o3)
+        : [a] "v"(in[0][d]), [b] "v"(in[1][d]), [c] "v"(in[2][d]), [d] "v"(in[3][d]), [odd] "s"(odd), [even] "s"(even), [hi] "s"(hi),
+          [lo] "s"(lo)
+        : "vcc");
+    out[0][d] = o0, out[1][d] = o1, out[2][d] = o2, out[3][d] = o3;
+  }
+}
+
+// 128-byte units.  The two loads of a block cover 16 rows x 128 bytes: in[0] rows 0-7, in[1] rows 8-15, lanes r and r + 8 of a
+// 16-lane group the two halves of a line.  Swapping lanes r and r ^ 8: out[0] = row r, chunk kg, out[1] = row r, chunk 4 + kg.
+__device__ __forceinline__ void to_operand(const u32x4 (&in)[2], u32x4 (&out)[2]) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const int lo = a[i], hi = b[i];
-    a[i] = __builtin_amdgcn_update_dpp(lo, hi, 0x128 /*row_ror:8*/, 0xf, 0xc, false);
-    b[i] = __builtin_amdgcn_update_dpp(hi, lo, 0x128, 0xf, 0x3, false);
+    const int lo = in[0][i], hi = in[1][i];
+    out[0][i] = __builtin_amdgcn_update_dpp(lo, hi, 0x128 /*row_ror:8*/, 0xf, 0xc, false);
+    out[1][i] = __builtin_amdgcn_update_dpp(hi, lo, 0x128, 0xf, 0x3, false);
   }
 }
 
-__device__ __forceinline__ u32x4 load_w(const uint8_t* p) {
-  return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
+__device__ __forceinline__ i32x8 join(u32x4 a, u32x4 b) {
+  return i32x8{static_cast<int>(a[0]), static_cast<int>(a[1]), static_cast<int>(a[2]), static_cast<int>(a[3]),
+               static_cast<int>(b[0]), static_cast<int>(b[1]), static_cast<int>(b[2]), static_cast<int>(b[3])};
 }
 
-// NW waves share K.  NT: 16-row blocks of W per workgroup (EPI_SILU_MUL: gate and up blocks of the same
-// features alternate).  U: lines per group; two groups are in flight.
-template <int NW, int NT, int U, int EPI, bool NORM>
-__global__ __launch_bounds__(64 * NW, 4) void gemm_skinny_kernel(SkinnyArgs a) {
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
+}
+
+template <int MT, int NT, int EPI>
+struct Reduction {   // of a pass's partial tiles, OB output blocks at a time
+  static constexpr int PAIR = EPI == EPI_SILU_MUL ? 2 : 1;          // accumulators of an output block
+  static constexpr int OUT = NT / PAIR * MT;                        // output blocks of 16 x 16
+  static constexpr int ROUNDS = (NW * OUT * PAIR + ROUND_KB - 1) / ROUND_KB;
+  static constexpr int OB = (OUT + ROUNDS - 1) / ROUNDS;
+  static constexpr int PART = OB * PAIR * 1024;                     // bytes of a wave's share of a round
+  static constexpr int LDS = NW * (PART + MT * 64);
+};
+
+// MT, NT: blocks of 16 rows of X and of W (EPI_SILU_MUL: gate and up blocks of the same features alternate).  UB: bytes of
+// a unit of K.  D: units in flight per wave.
+template <int MT, int NT, int UB, int D, int EPI, bool NORM, bool F8>
+__global__ __launch_bounds__(64 * NW, 2) void gemm_skinny_kernel(SkinnyArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  constexpr int PART = NT * 1024;                                // bytes of a wave's partial tile
-  constexpr int BLKS = EPI == EPI_SILU_MUL ? NT / 2 : NT;        // blocks of output columns
-  float* red_ss = reinterpret_cast<float*>(smem + NW * PART);    // [NW][16]
-  uint8_t* norm_lds = smem + NW * PART + NW * 64;                // [row_bytes]
+  using Red = Reduction<MT, NT, EPI>;
+  constexpr int LB = UB / 64;                                       // loads of a block and unit
+  constexpr int PAIR = Red::PAIR, OUT = Red::OUT, OB = Red::OB, PART = Red::PART;
+  float* red_ss = reinterpret_cast<float*>(smem + NW * PART);       // [NW][MT][16]
+  uint8_t* norm_lds = smem + Red::LDS;                              // [lw * NW * UB], zeros past K
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, kg = lane >> 4;
-  // this workgroup's output columns: an even share of the groups of 4
+  // this workgroup's output columns: an even share of the groups of 4, `per` of them a pass
   const int g = gridDim.x, b = blockIdx.x, q = a.units / g, rem = a.units - q * g;
-  const int n0 = 4 * (b * q + min(b, rem)), cols = 4 * (q + (b < rem));
+  const int n0 = 4 * (b * q + min(b, rem)), share = 4 * (q + (b < rem));
+  const int per = (share / 4 + a.passes - 1) / a.passes * 4;
+  const uint32_t rb = a.row_bytes;
+  const int nu = (rb + UB - 1) / UB, lw = (nu + NW - 1) / NW;       // units of K, a wave's units of a pass
+  const uint32_t vo = UB == 256 ? ((lane >> 2) & 3) * 4 * rb + kg * 64 + (lane & 3) * 16 : (r & 7) * rb + (kg + (r >> 3) * 4) * 16;
+  const uint32_t vs = UB == 256 ? rb : 8 * rb;                      // from load to load of a block
+  const uint32_t vo_tail = UB == 256 && (rb & 255) && kg >= 2 ? PAST_END : vo;   // the last unit may be half a unit
+  const uint8_t* wb = a.w + static_cast<size_t>(n0) * rb;
+  const uint8_t* wb_up = wb + static_cast<size_t>(a.inter) * rb;    // EPI_SILU_MUL
 
-  // this wave's lines of K
-  const int lines = a.row_bytes / 128;
-  const int l0 = lines * wave / NW, l1 = lines * (wave + 1) / NW;
-
-  const uint32_t chunk = (kg + (r >> 3) * 4) * 16;
-  const uint8_t* wb = a.w + static_cast<size_t>(n0) * a.row_bytes;
-  const uint8_t* wb_up = wb + static_cast<size_t>(a.inter) * a.row_bytes;   // EPI_SILU_MUL
-  uint32_t w0[BLKS], w1[BLKS];   // rows past the share: its last row again
-#pragma unroll
-  for (int i = 0; i < BLKS; ++i) {
-    w0[i] = static_cast<uint32_t>(min(i * 16 + (r & 7), cols - 1)) * a.row_bytes + chunk;
-    w1[i] = static_cast<uint32_t>(min(i * 16 + 8 + (r & 7), cols - 1)) * a.row_bytes + chunk;
-  }
-  const uint32_t x0 = static_cast<uint32_t>(min(r & 7, a.M - 1)) * a.row_bytes + chunk;
-  const uint32_t x1 = static_cast<uint32_t>(min(8 + (r & 7), a.M - 1)) * a.row_bytes + chunk;
-
-  u32x4 wf[2][U][2 * NT], xf[2][U][2];
-  auto load = [&](int s, int t) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const uint32_t off = static_cast<uint32_t>(min(t + u, l1 - 1)) * 128;  // past the end: a line that is in cache
-#pragma unroll
-      for (int i = 0; i < NT; ++i) {
-        const uint8_t* base = EPI == EPI_SILU_MUL && (i & 1) ? wb_up : wb;
-        const int blk = EPI == EPI_SILU_MUL ? i >> 1 : i;
-        wf[s][u][2 * i] = load_w(base + off + w0[blk]);
-        wf[s][u][2 * i + 1] = load_w(base + off + w1[blk]);
-      }
-      xf[s][u][0] = *reinterpret_cast<const u32x4*>(a.x + off + x0);
-      xf[s][u][1] = *reinterpret_cast<const u32x4*>(a.x + off + x1);
+  u32x4 wf[D][NT][LB], xf[D][MT][LB];
+  struct Item {
+    int p, j;   // pass, unit of this wave
+  };
+  struct Where {
+    const uint8_t *w, *up, *x;
+    int w_bytes, x_bytes;   // from the unit's first byte to the end of the pass's rows (of X)
+    bool tail;
+  };
+  auto advance = [&](Item& it) {
+    if (++it.j == lw) {
+      it.j = 0;
+      ++it.p;
     }
   };
-
-  f32x4 acc[NT];
+  auto where = [&](Item it) {
+    const int t = wave + it.j * NW;
+    const bool in = t < nu && it.p < a.passes;
+    const int off = in ? t * UB : 0, first = in ? it.p * per : 0;
+    const size_t at = static_cast<size_t>(first) * rb + off;
+    return Where{wb + at, wb_up + at, a.x + off, in ? min(per, share - first) * static_cast<int>(rb) - off : 0,
+                 in ? a.M * static_cast<int>(rb) - off : 0, in && t + 1 == nu};
+  };
+  auto fetch = [&](const uint8_t* base, int bytes, int blk, bool tail, auto aux, u32x4 (&out)[LB]) {
+    const int skip = blk * 16 * static_cast<int>(rb);
+    const __amdgpu_buffer_rsrc_t rs = rsrc(base + skip, max(bytes - skip, 0));
+    const uint32_t v = tail ? vo_tail : vo;
 #pragma unroll
-  for (int i = 0; i < NT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float ss = 0.f;
-  auto line = [&](int s, int u, int t) {
-    u32x4 xa = xf[s][u][0], xb = xf[s][u][1];
-    to_rows(xa, xb);
-    bf16x8 x[2] = {__builtin_bit_cast(bf16x8, xa), __builtin_bit_cast(bf16x8, xb)};
+    for (int i = 0; i < LB; ++i) out[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, v + i * vs, 0, decltype(aux)::value);
+  };
+  using Kept = std::integral_constant<int, 0>;
+  using Streamed = std::integral_constant<int, 2>;   // nt: read once
+  auto load_x = [&](const Where& at, int s, int m) { fetch(at.x, at.x_bytes, m, at.tail, Kept{}, xf[s][m]); };
+  auto load_w = [&](const Where& at, int s, int n) {
+    fetch(PAIR == 2 && (n & 1) ? at.up : at.w, at.w_bytes, n / PAIR, at.tail, Streamed{}, wf[s][n]);
+  };
+
+  f32x4 acc[NT][MT];
+  float ss[MT];
+  auto clear = [&] {
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int j = 0; j < MT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < MT; ++j) ss[j] = 0.f;
+  };
+
+  // output block `ob` of a pass: lane holds D[n = 4 kg + e][m = r]
+  auto write_out = [&](int p, int ob, f32x4 v, f32x4 up) {
+    const int i = ob / MT, j = ob % MT, m = j * 16 + r, c = i * 16 + 4 * kg, n = n0 + p * per + c;
+    if (m >= a.M || c >= min(per, share - p * per)) return;
     if constexpr (NORM) {
-      x[0] = scale_fragment(xa, *reinterpret_cast<const u32x4*>(norm_lds + t * 128 + kg * 16), ss);
-      x[1] = scale_fragment(xb, *reinterpret_cast<const u32x4*>(norm_lds + t * 128 + 64 + kg * 16), ss);
-    }
+      float s = 0.f;
 #pragma unroll
-    for (int i = 0; i < NT; ++i) {
-      u32x4 wa = wf[s][u][2 * i], wc = wf[s][u][2 * i + 1];
-      to_rows(wa, wc);
-      acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wa), x[0], acc[i], 0, 0, 0);
-      acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wc), x[1], acc[i], 0, 0, 0);
+      for (int w = 0; w < NW; ++w) s += red_ss[(w * MT + j) * 16 + r];
+      const float rs = rsqrtf(s * a.inv_k + a.eps);
+      v *= rs;
+      up *= rs;
     }
-  };
-  auto compute = [&](int s, int t) {
+    if constexpr (EPI == EPI_SILU_MUL) {
 #pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (t + u < l1) line(s, u, t + u);
+      for (int e = 0; e < 4; ++e) v[e] = silu(v[e]) * up[e];
+    } else {
+      if constexpr (F8) {
+        const float xs = a.x_scale[m];
+        const f32x4 wsc = *reinterpret_cast<const f32x4*>(a.w_scale + n);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] *= xs * wsc[e];
+      }
+      if (a.bias != nullptr) {
+        const u16x4 bb = *reinterpret_cast<const u16x4*>(a.bias + n);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] += bf2f(bb[e]);
+      }
+      if constexpr (EPI == EPI_RESIDUAL) {
+        const u16x4 rr = *reinterpret_cast<const u16x4*>(a.residual + static_cast<size_t>(m) * a.ldc + n);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] += bf2f(rr[e]);
+      }
+    }
+    u16x4 o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = f2bf(v[e]);
+    *reinterpret_cast<u16x4*>(a.c + static_cast<size_t>(m) * a.ldc + n) = o;
   };
 
-  if constexpr (NORM) {  // the norm weights: the same for every row, through LDS
-    for (int i = threadIdx.x * 16; i < a.row_bytes; i += 64 * NW * 16)
-      *reinterpret_cast<u32x4*>(norm_lds + i) = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint8_t*>(a.norm_w) + i);
-  }
-  if (l0 < l1) load(0, l0);
-  if constexpr (NORM) __syncthreads();
-  for (int t = l0; t < l1; t += 2 * U) {
-    load(1, t + U);
-    compute(0, t);
-    load(0, t + 2 * U);
-    compute(1, t + U);
-  }
-
-  // the waves' partial tiles and squares, summed in wave order
+  // the waves' partial tiles and squares, summed in wave order; loads of the next pass stay in flight
+  auto finish = [&](int p) {
+    if constexpr (NORM) {
 #pragma unroll
-  for (int i = 0; i < NT; ++i) *reinterpret_cast<f32x4*>(smem + wave * PART + i * 1024 + lane * 16) = acc[i];
+      for (int j = 0; j < MT; ++j) {
+        ss[j] += __shfl_xor(ss[j], 16);
+        ss[j] += __shfl_xor(ss[j], 32);
+        if (lane < 16) red_ss[(wave * MT + j) * 16 + lane] = ss[j];
+      }
+    }
+#pragma unroll
+    for (int rd = 0; rd < Red::ROUNDS; ++rd) {
+#pragma unroll
+      for (int o = 0; o < OB; ++o) {
+        const int ob = rd * OB + o;
+        if (ob >= OUT) break;
+#pragma unroll
+        for (int h = 0; h < PAIR; ++h)
+          *reinterpret_cast<f32x4*>(smem + wave * PART + (o * PAIR + h) * 1024 + lane * 16) = acc[ob / MT * PAIR + h][ob % MT];
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      auto total = [&](int blk) {
+        f32x4 v = *reinterpret_cast<const f32x4*>(smem + blk * 1024 + lane * 16);
+#pragma unroll
+        for (int w = 1; w < NW; ++w) v += *reinterpret_cast<const f32x4*>(smem + w * PART + blk * 1024 + lane * 16);
+        return v;
+      };
+      for (int o = wave; o < OB; o += NW)
+        if (rd * OB + o < OUT) write_out(p, rd * OB + o, total(PAIR * o), PAIR == 2 ? total(PAIR * o + PAIR - 1) : f32x4{});
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();   // before the next round's partial tiles
+    }
+  };
+
+  constexpr int NV = 2;   // 16-byte pieces of the norm weights per thread that are asked for before the first units
+  u32x4 nv[NV];
   if constexpr (NORM) {
-    ss += __shfl_xor(ss, 16);
-    ss += __shfl_xor(ss, 32);
-    if (lane < 16) red_ss[wave * 16 + lane] = ss;
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+      nv[i] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint8_t*>(a.norm_w) + min((threadIdx.x + i * 64 * NW) * 16, rb - 16));
   }
-  __syncthreads();
-
-  // lane holds D[n = 4 kg + e][m = r] of a block
-  const int i = wave, n = n0 + i * 16 + 4 * kg;
-  if (i >= BLKS || r >= a.M || i * 16 + 4 * kg >= cols) return;
-  auto total = [&](int blk) {
-    f32x4 v = *reinterpret_cast<const f32x4*>(smem + blk * 1024 + lane * 16);
+  Item now{0, 0}, next{0, 0};   // the unit at hand, the next one to load
 #pragma unroll
-    for (int w = 1; w < NW; ++w) v += *reinterpret_cast<const f32x4*>(smem + w * PART + blk * 1024 + lane * 16);
-    return v;
-  };
-  float rs = 1.f;
-  if constexpr (NORM) {
-    float s = 0.f;
+  for (int s = 0; s < D; ++s) {
+    const Where at = where(next);
+    advance(next);
 #pragma unroll
-    for (int w = 0; w < NW; ++w) s += red_ss[w * 16 + r];
-    rs = rsqrtf(s * a.inv_k + a.eps);
+    for (int m = 0; m < MT; ++m) load_x(at, s, m);
+#pragma unroll
+    for (int n = 0; n < NT; ++n) load_w(at, s, n);
   }
-  f32x4 v;
-  if constexpr (EPI == EPI_SILU_MUL) {
-    const f32x4 gate = total(2 * i) * rs, up = total(2 * i + 1) * rs;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = silu(gate[e]) * up[e];
-  } else {
-    v = total(i) * rs;
-    if (a.bias != nullptr) {
-      const u16x4 bb = *reinterpret_cast<const u16x4*>(a.bias + n);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] += bf2f(bb[e]);
+  if constexpr (NORM) {   // the norm weights: the same for every row, through LDS
+    const uint32_t end = static_cast<uint32_t>(lw) * NW * UB;
+    for (uint32_t i = threadIdx.x * 16, k = 0; i < end; i += 64 * NW * 16, ++k) {
+      u32x4 v = {0, 0, 0, 0};
+      if (i < rb) v = k == 0 ? nv[0] : k == 1 ? nv[1] : *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint8_t*>(a.norm_w) + i);
+      *reinterpret_cast<u32x4*>(norm_lds + i) = v;
     }
-    if constexpr (EPI == EPI_RESIDUAL) {
-      const u16x4 rr = *reinterpret_cast<const u16x4*>(a.residual + static_cast<size_t>(r) * a.ldc + n);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+  }
+  clear();
+  while (true) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] += bf2f(rr[e]);
+    for (int s = 0; s < D; ++s) {
+      const Where at = where(next);
+      advance(next);
+      u32x4 xt[MT][LB];
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        to_operand(xf[s][m], xt[m]);
+        load_x(at, s, m);
+        if constexpr (NORM) {
+          const uint8_t* nw = norm_lds + (wave + now.j * NW) * UB;
+#pragma unroll
+          for (int j = 0; j < LB; ++j)
+            xt[m][j] = scale_fragment(xt[m][j], *reinterpret_cast<const u32x4*>(nw + (UB == 256 ? kg * 64 + j * 16 : j * 64 + kg * 16)), ss[m]);
+        }
+        __builtin_amdgcn_sched_barrier(0);   // a register is loaded again where it was consumed, not later
+      }
+#pragma unroll
+      for (int n = 0; n < NT; ++n) {
+        u32x4 wt[LB];
+        to_operand(wf[s][n], wt);
+        load_w(at, s, n);
+        if constexpr (F8) {   // 32 bytes of a row an operand; formats 0 / 0 = e4m3, scales 127 = 1
+#pragma unroll
+          for (int j = 0; j < LB; j += 2)
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+              acc[n][m] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(join(wt[j], wt[j + 1]), join(xt[m][j], xt[m][j + 1]),
+                                                                            acc[n][m], 0, 0, 0, 127, 0, 127);
+        } else {
+#pragma unroll
+          for (int j = 0; j < LB; ++j)
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+              acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wt[j]), __builtin_bit_cast(bf16x8, xt[m][j]),
+                                                                   acc[n][m], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (now.j + 1 == lw) {
+        finish(now.p);
+        if (now.p + 1 == a.passes) return;
+        clear();
+      }
+      advance(now);
     }
   }
-  u16x4 o;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) o[e] = f2bf(v[e]);
-  *reinterpret_cast<u16x4*>(a.c + static_cast<size_t>(r) * a.ldc + n) = o;
 }
 
-template <int NW, int NT, int U, int EPI, bool NORM>
-int launch(const SkinnyArgs& a, hipStream_t stream) {
-  constexpr int MOST = EPI == EPI_SILU_MUL ? 2 * NT : 4 * NT;        // groups of 4 columns that a workgroup can hold
-  const int passes = (a.units + CUS * MOST - 1) / (CUS * MOST);      // workgroups per CU
-  const int grid = a.units < CUS * passes ? a.units : CUS * passes;
-  const int lds = NW * (NT * 1024 + 64) + (NORM ? a.row_bytes : 0);
-  hipLaunchKernelGGL((gemm_skinny_kernel<NW, NT, U, EPI, NORM>), dim3(grid), dim3(64 * NW), lds, stream, a);
+template <int MT, int NT, int UB, int D, int EPI, bool NORM, bool F8>
+int launch(SkinnyArgs a, int passes, hipStream_t stream) {
+  a.passes = passes;
+  const int nu = (a.row_bytes + UB - 1) / UB;
+  const int lds = Reduction<MT, NT, EPI>::LDS + (NORM ? (nu + NW - 1) / NW * NW * UB : 0);
+  auto kernel = gemm_skinny_kernel<MT, NT, UB, D, EPI, NORM, F8>;
+  if (lds > 65536 && hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
+    return -1;
+  hipLaunchKernelGGL(kernel, dim3(a.units < CUS ? a.units : CUS), dim3(64 * NW), lds, stream, a);
   return BCG_CHECK_LAUNCH();
 }
 
-// The fewest row blocks that hold a CU's share in one workgroup, 4 at most: blocks that stay empty cost matrix
-// instructions (4096 x 4096: 1 block 10.3 us, 2 blocks 12.3), fewer than the share fills cost reads of X
-// (10240 x 5120: 2 blocks 29.4, 4 blocks 26.6).  4 waves where a wave's K range would be short
-// (896 x 4864: 8.4 us against 9.7 with 8), 8 to keep enough lines in flight otherwise (4096 x 12288: 23.0, 24.4).
-template <int EPI, bool NORM>
+// The fewest passes, then the fewest row blocks that hold a pass: blocks that stay empty cost instructions.  Rows of up to
+// 2048 bytes and shares of 4 columns take 128-byte units (see above), the latter two units at once: a wave then has only
+// four loads in flight (896 x 4864: 8.5 us with one, 7.7).
+template <int MT, int EPI, bool NORM, bool F8>
 int pick(const SkinnyArgs& a, hipStream_t s) {
-  const int share = (a.units + CUS - 1) / CUS;
-  if constexpr (EPI == EPI_SILU_MUL) {
-    return share <= 4 ? launch<8, 2, 1, EPI, NORM>(a, s) : launch<8, 4, 1, EPI, NORM>(a, s);
-  } else {
-    if (share <= 4) return a.row_bytes < 16384 ? launch<4, 1, 2, EPI, NORM>(a, s) : launch<8, 1, 2, EPI, NORM>(a, s);
-    return share <= 8 ? launch<8, 2, 1, EPI, NORM>(a, s) : launch<8, 4, 1, EPI, NORM>(a, s);
+  constexpr int PER = EPI == EPI_SILU_MUL ? 2 : 4;                             // groups of 4 columns of a block of W
+  constexpr int MOST = EPI == EPI_SILU_MUL ? (MT == 1 ? 6 : 4) : (MT == 1 ? 8 : 4);   // (registers of two waves per SIMD)
+  const int share = (a.units + CUS - 1) / CUS, passes = (share + MOST * PER - 1) / (MOST * PER);
+  const int blocks = ((share + passes - 1) / passes + PER - 1) / PER;
+  if constexpr (MT == 1 && !F8) {
+    if (a.row_bytes <= 2048) {
+      if constexpr (EPI == EPI_SILU_MUL) {
+        return blocks <= 2 ? launch<1, 2, 128, 1, EPI, NORM, F8>(a, passes, s)
+                           : blocks <= 4 ? launch<1, 4, 128, 1, EPI, NORM, F8>(a, passes, s) : launch<1, 6, 128, 1, EPI, NORM, F8>(a, passes, s);
+      } else {
+        return blocks <= 1   ? launch<1, 1, 128, 1, EPI, NORM, F8>(a, passes, s)
+               : blocks <= 2 ? launch<1, 2, 128, 1, EPI, NORM, F8>(a, passes, s)
+               : blocks <= 4 ? launch<1, 4, 128, 1, EPI, NORM, F8>(a, passes, s) : launch<1, 8, 128, 1, EPI, NORM, F8>(a, passes, s);
+      }
+    }
+    if (share == 1) return launch<1, EPI == EPI_SILU_MUL ? 2 : 1, 128, 2, EPI, NORM, F8>(a, passes, s);
   }
+  if constexpr (EPI == EPI_SILU_MUL) {
+    if (blocks <= 2) return launch<MT, 2, 256, 1, EPI, NORM, F8>(a, passes, s);
+    if constexpr (MT == 1)
+      if (blocks > 4) return launch<MT, 6, 256, 1, EPI, NORM, F8>(a, passes, s);
+    return launch<MT, 4, 256, 1, EPI, NORM, F8>(a, passes, s);
+  } else {
+    if (blocks <= 1) return launch<MT, 1, 256, 1, EPI, NORM, F8>(a, passes, s);
+    if (blocks <= 2) return launch<MT, 2, 256, 1, EPI, NORM, F8>(a, passes, s);
+    if constexpr (MT == 1)
+      if (blocks > 4) return launch<MT, 8, 256, 1, EPI, NORM, F8>(a, passes, s);
+    return launch<MT, 4, 256, 1, EPI, NORM, F8>(a, passes, s);
+  }
+}
+
+bool covered(int M, int row_bytes, int n_out) {
+  return M >= 1 && M <= MAX_ROWS && row_bytes >= 128 && row_bytes <= MAX_ROW_BYTES && row_bytes % 128 == 0 && n_out >= 4 && n_out % 4 == 0;
 }
 
 }  // namespace
 
 // epi: 0 = store (+bias), 1 = silu(gate)*up into [M, N / 2], 2 = residual + acc (+bias).  norm_w: RMS-normalise the rows
-// of x with these weights first (epi 0, 1).  1 <= M <= 16, K % 64 == 0, 64 <= K <= 12288, the output width a multiple
-// of 4; rows contiguous, x and w 16-byte aligned, the others 8-byte aligned.
+// of x with these weights first (epi 0, 1; M <= 16, K <= 16384).  1 <= M <= 32, K % 64 == 0, 64 <= K <= 32768, the output
+// width a multiple of 4; rows contiguous, x and w 16-byte aligned, the others 8-byte aligned.
 BCG_API int bcg_gemm_skinny(int epi, const void* x, const void* w, const void* norm_w, float eps, const void* bias,
                             const void* residual, void* c, int M, int N, int K, hipStream_t stream) {
   const int n_out = epi == EPI_SILU_MUL ? N / 2 : N;
-  if (M < 1 || M > MAX_ROWS || K < 64 || K > MAX_K || K % 64 || n_out < 4 || n_out % 4 || (epi == EPI_SILU_MUL && N % 2)) return -2;
+  if (K < 1 || K > MAX_ROW_BYTES / 2 || !covered(M, 2 * K, n_out) || (epi == EPI_SILU_MUL && N % 2)) return -2;
+  if (norm_w && (M > MAX_NORM_ROWS || K > MAX_NORM_K)) return -2;
   const SkinnyArgs a{static_cast<const uint8_t*>(x), static_cast<const uint8_t*>(w), static_cast<const bf16_t*>(norm_w),
-                     static_cast<const bf16_t*>(bias), static_cast<const bf16_t*>(residual), static_cast<bf16_t*>(c),
-                     M, 2 * K, n_out, N / 2, n_out / 4, eps, 1.f / K};
+                     static_cast<const bf16_t*>(bias), static_cast<const bf16_t*>(residual), static_cast<bf16_t*>(c), nullptr, nullptr,
+                     M, 2 * K, n_out, N / 2, n_out / 4, 1, eps, 1.f / K};
   switch (epi) {
-    case EPI_STORE: return norm_w ? pick<EPI_STORE, true>(a, stream) : pick<EPI_STORE, false>(a, stream);
+    case EPI_STORE:
+      if (norm_w) return pick<1, EPI_STORE, true, false>(a, stream);
+      return M <= 16 ? pick<1, EPI_STORE, false, false>(a, stream) : pick<2, EPI_STORE, false, false>(a, stream);
     case EPI_SILU_MUL:
       if (bias) return -2;
-      return norm_w ? pick<EPI_SILU_MUL, true>(a, stream) : pick<EPI_SILU_MUL, false>(a, stream);
+      if (norm_w) return pick<1, EPI_SILU_MUL, true, false>(a, stream);
+      return M <= 16 ? pick<1, EPI_SILU_MUL, false, false>(a, stream) : pick<2, EPI_SILU_MUL, false, false>(a, stream);
     case EPI_RESIDUAL:
       if (!residual || norm_w) return -2;
-      return pick<EPI_RESIDUAL, false>(a, stream);
+      return M <= 16 ? pick<1, EPI_RESIDUAL, false, false>(a, stream) : pick<2, EPI_RESIDUAL, false, false>(a, stream);
+    default: return -2;
+  }
+}
+
+// fp8 (e4m3fn) form: C = x_scale[m] * w_scale[n] * (Xq . Wq^T) (+ bias) (+ residual); epi 0 or 2.  1 <= M <= 32, K % 128 == 0,
+// K <= 65536, N a multiple of 4; rows contiguous, xq, wq and w_scale 16-byte aligned, the others 8-byte aligned.
+BCG_API int bcg_gemm_skinny_fp8(int epi, const void* xq, const void* wq, const float* x_scale, const float* w_scale, const void* bias,
+                                const void* residual, void* c, int M, int N, int K, hipStream_t stream) {
+  if (!covered(M, K, N) || !x_scale || !w_scale) return -2;
+  const SkinnyArgs a{static_cast<const uint8_t*>(xq), static_cast<const uint8_t*>(wq), nullptr, static_cast<const bf16_t*>(bias),
+                     static_cast<const bf16_t*>(residual), static_cast<bf16_t*>(c), x_scale, w_scale,
+                     M, K, N, 0, N / 4, 1, 0.f, 0.f};
+  switch (epi) {
+    case EPI_STORE: return M <= 16 ? pick<1, EPI_STORE, false, true>(a, stream) : pick<2, EPI_STORE, false, true>(a, stream);
+    case EPI_RESIDUAL:
+      if (!residual) return -2;
+      return M <= 16 ? pick<1, EPI_RESIDUAL, false, true>(a, stream) : pick<2, EPI_RESIDUAL, false, true>(a, stream);
     default: return -2;
   }
 }
