@@ -23,6 +23,9 @@ PREFILL32_MAX_BLOCKS = 1024  # csrc/kernels/attention.hip: the 32x32 kernel's LD
 
 # csrc/kernels/gemm_skinny.hip: most rows, most rows with a fused norm, longest rows in bytes
 SKINNY_ROWS, SKINNY_NORM_ROWS, SKINNY_ROW_BYTES = 32, 16, 65536
+# `decode_attention`: every workgroup of a row rotates its queries again, so with many rows the separate launch wins (a step of
+# 24 layers of 14 / 2 heads of 64, us: 120 rows 2051 separate, 2029 fused; 400 rows 2833, 2871)
+DECODE_FUSED_ROWS = 128
 SKINNY_LONG_K = 12288  # past it: fewer shapes gain (`_few_rows_pay`), logged apart
 
 c_int, c_float, c_void_p, c_uint32, c_int64 = ctypes.c_int, ctypes.c_float, ctypes.c_void_p, ctypes.c_uint32, ctypes.c_int64
@@ -95,6 +98,8 @@ def load_library(path: str = None) -> ctypes.CDLL:
                         c_int, c_int, c_int, c_int, c_int, c_void_p],
         "bcg_gemm_nt_fp8": [c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                             c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
+        "bcg_decode_fused": [c_void_p] * 6 + [c_float, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_void_p, c_int,
+                             c_int, c_int, c_int, c_float, c_void_p, c_int, c_int, c_void_p, c_void_p],
         "bcg_gemm_skinny": [c_int, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
                             c_void_p],
         "bcg_gemm_skinny_fp8": [c_int] + [c_void_p] * 7 + [c_int] * 3 + [c_void_p],
@@ -326,6 +331,33 @@ def hip_ops() -> SimpleNamespace:
             _p(q), _p(k_cache), _p(v_cache), layer, NB, n_kv, _p(block_tables), max_blocks, _p(seq_lens),
             B, n_q, hd, BS, scale, _p(ws), max_splits, split, _p(out), _kv_fp8(k_cache, v_cache), *cas,
             _stream()), "paged_attention_decode")
+        return out
+
+    def decode_attention(qkv, positions, slots, n_q, n_kv, hd, q_norm, k_norm, eps, cos_sin, k_cache, v_cache, layer,
+                         block_tables, seq_lens, scale, workspace=None):
+        """paged_attention_decode(qk_norm_rope_kv_write(...)) for one new token per row of a bf16 cache with heads of 64, without the
+        rotary launch (csrc/kernels/attention.hip, FusedArgs, says why not for others)."""
+        B = qkv.shape[0]
+        L, NB, nkv_c, BS, hdc = k_cache.shape
+        _req(qkv.dtype == torch.bfloat16 and qkv.is_contiguous() and qkv.shape[1] == (n_q + 2 * n_kv) * hd, "decode qkv")
+        _req(nkv_c == n_kv and hdc == hd and hd == 64 and BS == 16 and v_cache.shape == (L, NB, n_kv, hd, BS)
+             and k_cache.dtype == v_cache.dtype == torch.bfloat16, "decode kv cache layout")
+        _req(all(t.dtype == torch.int32 and t.is_contiguous() for t in (positions, slots, seq_lens, block_tables))
+             and positions.numel() == slots.numel() == seq_lens.numel() == B and block_tables.shape[0] == B, "decode tables")
+        _req(cos_sin.dtype == torch.float32 and cos_sin.shape[1] == hd and B <= 2048, "decode cos_sin / rows")
+        max_blocks = block_tables.shape[1]
+        split = lib.bcg_decode_split_tokens(B, n_kv, max_blocks * BS)
+        max_splits = lib.bcg_decode_max_splits(max_blocks * BS, 0)
+        need = B * n_q * max_splits * (hd + 2)
+        if workspace is None:
+            workspace = torch.empty(need, dtype=torch.float32, device=qkv.device)
+        _req(workspace.dtype == torch.float32 and workspace.is_contiguous() and workspace.numel() >= need,
+             "decode attention workspace too small")
+        out = torch.empty(B, n_q * hd, dtype=qkv.dtype, device=qkv.device)
+        _check(lib.bcg_decode_fused(
+            _p(qkv), _p(positions), _p(slots), None if q_norm is None else _p(q_norm), None if k_norm is None else _p(k_norm),
+            _p(cos_sin), eps, _p(k_cache), _p(v_cache), layer, NB, n_kv, _p(block_tables), max_blocks, _p(seq_lens), B, n_q, hd,
+            BS, scale, _p(workspace), max_splits, split, _p(out), _stream()), "decode_attention")
         return out
 
     def paged_attention_prefill(q, k_cache, v_cache, layer, block_tables, q_start, seq_lens, scale,
@@ -804,6 +836,7 @@ def hip_ops() -> SimpleNamespace:
                            embed_rmsnorm=embed_rmsnorm,
                            qk_norm_rope_kv_write=qk_norm_rope_kv_write,
                            paged_attention_decode=paged_attention_decode,
+                           decode_attention=decode_attention, decode_fused_rows=DECODE_FUSED_ROWS,
                            decode_workspace_numel=decode_workspace_numel,
                            decode_max_context=lambda cascade=True: lib.bcg_decode_max_context(int(cascade)),
                            paged_attention_prefill=paged_attention_prefill,

@@ -393,12 +393,74 @@ constexpr int DEC_MAX_B = 2048;
 // 64 columns instead of once per row -- into slots 0 .. split_base-1; this kernel covers
 // [kv_begin, ctx) into the slots after them; the combine merges all slots.
 // kv_begin == nullptr: no cascade (every row from token 0).
-template <int HD, bool F8 = false, int CPW = 1>
+//
+// FUSED (heads of 64, bf16 caches): the kernel takes the projected rows as they come, without a rotary launch and a pass over q
+// before it: every workgroup rotates (and normalises) its own query heads while its K/V loads are in flight; the one with the
+// newest token also stores that token's K/V and puts it into its chunk's registers, where the loads brought what was there
+// before.  24 layers of 14 / 2 heads at 4 rows of 500 tokens: 912 -> 873 us a step.  Heads of 128 take the separate launches:
+// two chunks of K/V and the rotation's operands fill the registers (10 rows of 1100 tokens, 40 / 8 heads, a step of 16 layers: 2561
+// us, 2590 fused; 448 rows 6950, 8110).  Merging the splits in the workgroup that arrives last costs more than the merge
+// launch for both (stores past the L2, a ticket, the reads back: 880 and 2669).
+struct FusedArgs {
+  const bf16_t* qkv;        // [B, n_q + 2 n_kv, HD]
+  const int* positions;     // [B]
+  const int* slots;         // [B]
+  const bf16_t* q_norm;     // [HD] or null
+  const bf16_t* k_norm;
+  const float* cos_sin;     // [positions, HD]: cos, sin
+  float eps;
+};
+
+// One head as a row of an operand fragment: lane group h holds dims 32 kk + 8 h .. + 7, and with them both sides of its rotation
+// pairs (d, d + HD / 2): normalised, rotated and rounded as qk_norm_rope_kv_vec_kernel does.
+template <int HD>
+__device__ __forceinline__ void rope_fragments(bf16x8 (&out)[HD / 32], const u16x8 (&raw)[HD / 32], const u16x8 (&norm)[HD / 32],
+                                               bool normed, const f32x4 (&cs)[HD / 64][2], const f32x4 (&sn)[HD / 64][2], float eps, int h) {
+  constexpr int KK = HD / 32;
+  float x[KK][8];
+#pragma unroll
+  for (int kk = 0; kk < KK; ++kk)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[kk][j] = bf2f(raw[kk][j]);
+  if (normed) {
+    float ss = 0.f;
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) ss += x[kk][j] * x[kk][j];
+    ss = rows_sum(ss);
+    const float inv = rsqrtf(ss / HD + eps);
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[kk][j] *= inv * bf2f(norm[kk][j]);
+  }
+#pragma unroll
+  for (int kk = 0; kk < KK / 2; ++kk) {
+    u16x8 lo, hi;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float c = cs[kk][j >> 2][j & 3], sv = sn[kk][j >> 2][j & 3], x1 = x[kk][j], x2 = x[kk + KK / 2][j];
+      lo[j] = f2bf(x1 * c - x2 * sv);
+      hi[j] = f2bf(x2 * c + x1 * sv);
+    }
+    out[kk] = __builtin_bit_cast(bf16x8, lo);
+    out[kk + KK / 2] = __builtin_bit_cast(bf16x8, hi);
+  }
+}
+
+template <int HD>
+__device__ __forceinline__ void load_head(u16x8 (&raw)[HD / 32], const bf16_t* row, int h) {
+#pragma unroll
+  for (int kk = 0; kk < HD / 32; ++kk) raw[kk] = *reinterpret_cast<const u16x8*>(row + kk * 32 + h * 8);
+}
+template <int HD, bool F8 = false, int CPW = 1, bool FUSED = false>
 __global__ __launch_bounds__(256) void decode_attn_kernel(
     const bf16_t* __restrict__ q, KVGeom g, const int* __restrict__ block_tables, int max_blocks,
     const int* __restrict__ seq_lens, int B, int n_q, float scale_log2, float* __restrict__ part_o,
     float* __restrict__ part_ml, int max_splits, const int* __restrict__ kv_begin,
-    const int* __restrict__ split_base) {
+    const int* __restrict__ split_base, FusedArgs fa) {
+  static_assert(!FUSED || (HD == 64 && !F8), "fused: see FusedArgs");
   // CPW chunks per wave: an item covers DEC_WAVES * CPW * 32 tokens; every chunk's loads of
   // a wave are issued before its first MFMA (CPW x 16 loads in flight per wave), and the
   // split partials / merge traffic shrink by CPW
@@ -407,7 +469,7 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
   __shared__ int s_wsum[DEC_WAVES];
   __shared__ float s_ml[DEC_WAVES][2][16];
   __shared__ float s_o[DEC_WAVES][HD][16 + 1];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, w = FUSED ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
   const int r = lane & 15, h = lane >> 4;
   const int G = n_q / g.n_kv;
 
@@ -421,6 +483,7 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
       const int i = tid * per + j;
       const int own = (j < per && i < B) ? max(0, seq_lens[i] - (kv_begin ? kv_begin[i] : 0)) : 0;
       cnt[j] = (own + DEC_SPLIT - 1) / DEC_SPLIT;
+      if (FUSED && j < per && i < B) cnt[j] = max(cnt[j], 1);   // its K/V is stored and its output cleared all the same
       sum += cnt[j];
     }
     int incl = sum;  // inclusive wave scan
@@ -451,27 +514,111 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
       const int mid = (lo + hi + 1) >> 1;
       if (s_pre[mid] <= pos) lo = mid; else hi = mid - 1;
     }
-    const int b = lo, split = pos - s_pre[b];
+    const int b = FUSED ? __builtin_amdgcn_readfirstlane(lo) : lo, split = pos - s_pre[b];
     const int ctx = seq_lens[b];
     const int start = (kv_begin ? kv_begin[b] : 0) + split * DEC_SPLIT;
     const int slot = (split_base ? split_base[b] : 0) + split;  // after the shared-pass slots
     const int* table = block_tables + static_cast<size_t>(b) * max_blocks;
 
     bf16x8 bq[HD / 32];
-    load_q<HD>(bq, q + (static_cast<size_t>(b) * n_q + kvh * G + (r < G ? r : 0)) * HD, r < G, lane);
+    // FUSED: all of this is asked for before the K/V loads, behind which it would wait for them
+    u16x8 raw_q[HD / 32], raw_k[HD / 32], wq[HD / 32] = {}, wk[HD / 32] = {};
+    f32x4 cs[HD / 64][2], sn[HD / 64][2];
+    bf16_t nv[HD / 16];
+    const int newest = ctx - 1;
+    const bool stores = FUSED && pos + 1 == __builtin_amdgcn_readfirstlane(s_pre[b + 1]) && w == max(newest - start, 0) / (CHUNK * CPW);
+    const bf16_t* heads = nullptr;
+    if constexpr (FUSED) {
+      heads = fa.qkv + static_cast<size_t>(b) * (n_q + 2 * g.n_kv) * HD;
+      load_head<HD>(raw_q, heads + (kvh * G + (r < G ? r : 0)) * HD, h);
+      const float* t = fa.cos_sin + static_cast<size_t>(fa.positions[b]) * HD + 8 * h;
+#pragma unroll
+      for (int kk = 0; kk < HD / 64; ++kk)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          cs[kk][e] = *reinterpret_cast<const f32x4*>(t + kk * 32 + 4 * e);
+          sn[kk][e] = *reinterpret_cast<const f32x4*>(t + HD / 2 + kk * 32 + 4 * e);
+        }
+      if (fa.q_norm != nullptr) load_head<HD>(wq, fa.q_norm, h);
+      if (stores) {   // wave-uniform: the wave that covers the newest token
+        load_head<HD>(raw_k, heads + (n_q + kvh) * HD, h);
+        if (fa.k_norm != nullptr) load_head<HD>(wk, fa.k_norm, h);
+#pragma unroll
+        for (int dt = 0; dt < HD / 16; ++dt) nv[dt] = heads[(n_q + g.n_kv + kvh) * HD + dt * 16 + r];
+      }
+    } else {
+      load_q<HD>(bq, q + (static_cast<size_t>(b) * n_q + kvh * G + (r < G ? r : 0)) * HD, r < G, lane);
+    }
     float m = -INFINITY, l = 0.f;
     f32x4 o[HD / 16];
 #pragma unroll
     for (int dt = 0; dt < HD / 16; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     const int t0 = start + w * CHUNK * CPW;
-    const int last_blk = (ctx - 1) / BS;
+    const int last_blk = (FUSED ? max(ctx - 1, 0) : ctx - 1) / BS;
     Chunk<HD, F8> c[CPW];
+    if constexpr (FUSED) {
+      // wave-uniform addresses through the scalar cache: a vector load of a table entry would be waited for together with
+      // the rotary embedding's operands (loads return in order)
+      int blk[CPW][2];
 #pragma unroll
-    for (int j = 0; j < CPW; ++j) {
-      const int tj = t0 + j * CHUNK;
-      if (tj < ctx)  // wave-uniform
-        load_chunk<HD, F8>(c[j], g, table[tj / BS], table[min(tj / BS + 1, last_blk)], kvh, lane);
+      for (int j = 0; j < CPW; ++j)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) blk[j][e] = table[min((t0 + j * CHUNK) / BS + e, last_blk)];
+#pragma unroll
+      for (int j = 0; j < CPW; ++j)
+        if (t0 + j * CHUNK < ctx) load_chunk<HD, F8>(c[j], g, blk[j][0], blk[j][1], kvh, lane);  // wave-uniform
+    } else {
+#pragma unroll
+      for (int j = 0; j < CPW; ++j) {
+        const int tj = t0 + j * CHUNK;
+        if (tj < ctx)  // wave-uniform
+          load_chunk<HD, F8>(c[j], g, table[tj / BS], table[min(tj / BS + 1, last_blk)], kvh, lane);
+      }
+    }
+    if constexpr (FUSED) {
+      rope_fragments<HD>(bq, raw_q, wq, fa.q_norm != nullptr, cs, sn, fa.eps, h);
+      if (r >= G) {
+#pragma unroll
+        for (int kk = 0; kk < HD / 32; ++kk) bq[kk] = bf16x8{};
+      }
+      if (stores) {
+        bf16x8 bk[HD / 32];
+        rope_fragments<HD>(bk, raw_k, wk, fa.k_norm != nullptr, cs, sn, fa.eps, h);
+        const int slot_of = fa.slots[b];
+        const size_t base = block_base<HD>(g, slot_of / BS, kvh);
+        bf16_t* kd = const_cast<bf16_t*>(g.k) + base + (slot_of % BS) * HD + 8 * h;
+        bf16_t* vd = const_cast<bf16_t*>(g.v) + base + slot_of % BS;
+        if (r == 0) {
+#pragma unroll
+          for (int kk = 0; kk < HD / 32; ++kk) *reinterpret_cast<bf16x8*>(kd + kk * 32) = bk[kk];
+        }
+#pragma unroll
+        for (int dt = 0; dt < HD / 16; ++dt)
+          if (dt % 4 == h) vd[(dt * 16 + r) * BS] = nv[dt];
+        // (a parked row stores elsewhere than it reads: its newest token is what the cache holds)
+        if (ctx > 0 && slot_of == table[newest / BS] * BS + newest % BS) {
+#pragma unroll
+          for (int j = 0; j < CPW; ++j) {
+            const int tj = t0 + j * CHUNK;
+            if (newest < tj || newest >= tj + CHUNK) continue;  // wave-uniform
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+              const bool here = tj + 8 * (r >> 2) + 4 * u + (r & 3) == newest;
+#pragma unroll
+              for (int kk = 0; kk < HD / 32; ++kk) c[j].k[u][kk] = here ? bk[kk] : c[j].k[u][kk];
+            }
+            const int at = newest - tj - 8 * h;   // element of this lane's V^T pieces, if 0 .. 7
+#pragma unroll
+            for (int dt = 0; dt < HD / 16; ++dt) {
+              u16x8 v = __builtin_bit_cast(u16x8, c[j].v[dt]);
+#pragma unroll
+              for (int e = 0; e < 8; ++e) v[e] = e == at ? nv[dt] : v[e];
+              c[j].v[dt] = __builtin_bit_cast(bf16x8, v);
+            }
+          }
+        }
+      }
     }
 #pragma unroll
     for (int j = 0; j < CPW; ++j) {
@@ -698,10 +845,10 @@ struct Cascade {
   int split_tokens;       // shared tokens per item (a multiple of CHUNK)
 };
 
-template <int HD, bool F8 = false, int CPW = 1>
+template <int HD, bool F8 = false, int CPW = 1, bool FUSED = false>
 void launch_decode(const bf16_t* q, KVGeom g, const int* tables, int max_blocks, const int* seq_lens, int B,
                    int n_q, float sl, float* ws, int max_splits, bf16_t* out, const Cascade& cas,
-                   hipStream_t stream) {
+                   hipStream_t stream, const FusedArgs& fa = FusedArgs{}) {
   constexpr int DEC_SPLIT = DEC_WAVES * CHUNK * CPW;
   float* part_o = ws;
   float* part_ml = ws + static_cast<size_t>(B) * n_q * max_splits * HD;
@@ -718,12 +865,12 @@ void launch_decode(const bf16_t* q, KVGeom g, const int* tables, int max_blocks,
     int per_cu = 0, cus = 0, dev = 0;
     hipGetDevice(&dev);
     hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, decode_attn_kernel<HD, F8, CPW>, 256, 0);
+    hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, decode_attn_kernel<HD, F8, CPW, FUSED>, 256, 0);
     resident = std::max(1, per_cu) * std::max(1, cus);
   }
   const int grid = static_cast<int>(std::min<long>(static_cast<long>(B) * g.n_kv * max_splits, resident));
-  hipLaunchKernelGGL((decode_attn_kernel<HD, F8, CPW>), dim3(grid), dim3(256), 0, stream, q, g, tables, max_blocks,
-                     seq_lens, B, n_q, sl, part_o, part_ml, max_splits, cas.kv_begin, cas.split_base);
+  hipLaunchKernelGGL((decode_attn_kernel<HD, F8, CPW, FUSED>), dim3(grid), dim3(256), 0, stream, q, g, tables, max_blocks,
+                     seq_lens, B, n_q, sl, part_o, part_ml, max_splits, cas.kv_begin, cas.split_base, fa);
   const int n_bq = B * n_q;
   hipLaunchKernelGGL(decode_combine_kernel<HD>, dim3((n_bq + COMBINE_WAVES - 1) / COMBINE_WAVES),
                      dim3(64 * COMBINE_WAVES), 0, stream, part_o, part_ml, seq_lens, n_q, max_splits, DEC_SPLIT, n_bq,
@@ -1386,6 +1533,25 @@ BCG_API int bcg_paged_attention_decode(const void* q, const void* k_cache, const
   } else {
     return -2;
   }
+  return BCG_CHECK_LAUNCH();
+}
+
+// Rotary embedding, cache write and attention of a decode step (decode_attn_kernel, FUSED): qkv [B, n_q + 2 n_kv, hd] as projected,
+// one new token per row at `slots`; bf16 caches, hd 64.  workspace, max_splits, split_tokens as
+// bcg_paged_attention_decode without shared prefixes.
+BCG_API int bcg_decode_fused(const void* qkv, const int* positions, const int* slots, const void* q_norm, const void* k_norm,
+                             const float* cos_sin, float eps, void* k_cache, void* v_cache, int layer, int num_blocks, int n_kv,
+                             const int* block_tables, int max_blocks, const int* seq_lens, int B, int n_q, int hd, int block_size,
+                             float scale, float* workspace, int max_splits, int split_tokens, void* out, hipStream_t stream) {
+  if (hd != 64 || block_size != BS || n_kv <= 0 || n_q % n_kv || n_q / n_kv > 16 || B <= 0 || B > DEC_MAX_B) return -2;
+  if (split_tokens != DEC_WAVES * CHUNK * DEC_CPW || max_splits * split_tokens < max_blocks * BS || max_splits > 64) return -3;
+  const KVGeom g{static_cast<const bf16_t*>(k_cache), static_cast<const bf16_t*>(v_cache), layer, num_blocks, n_kv};
+  const FusedArgs fa{static_cast<const bf16_t*>(qkv), positions, slots, static_cast<const bf16_t*>(q_norm),
+                     static_cast<const bf16_t*>(k_norm), cos_sin, eps};
+  const Cascade none{nullptr, nullptr, nullptr, 0, nullptr, 0, nullptr, nullptr, 0, CHUNK};
+  bf16_t* ob = static_cast<bf16_t*>(out);
+  launch_decode<64, false, DEC_CPW, true>(nullptr, g, block_tables, max_blocks, seq_lens, B, n_q, scale * LOG2E, workspace, max_splits, ob,
+                                          none, stream, fa);
   return BCG_CHECK_LAUNCH();
 }
 
