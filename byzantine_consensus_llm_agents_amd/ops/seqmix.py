@@ -43,10 +43,13 @@ EXPERT_ACTS = {"silu_gated": "silu", "clamped_glu": "clamped_glu"}   # gated exp
 WIDE_ROWS = 256    # rows of a position tile of the 256 x 256 expert products
 WIDE_SLOTS = 64    # ... taken from this many routed rows per expert on (see `_wide_experts`)
 
+FEW_SLOTS = 24     # position tiles of 32 rows up to this many routed rows per expert (see `_few_row_experts`)
+
 
 def seqmix_ops(lib, linear):
     split_keys = lib.bcg_multimap_split_keys()
     tile_rows = lib.bcg_moe_tile_rows()
+    few_rows = lib.bcg_moe_rows_tile()
 
     def embed_scale_rmsnorm(tokens, table, scale, w, eps, w_offset, out_dtype, add=None):
         _req(tokens.dtype == torch.int32 and tokens.is_contiguous() and tokens.dim() == 1, "tokens int32 [T]")
@@ -272,6 +275,14 @@ def seqmix_ops(lib, linear):
         return (2 * rows * max(W, n_up) < 1 << 31 and 2 * (max(W, n_up) + 256) * max(W, ff) < 1 << 31
                 and all(t.data_ptr() % 16 == 0 for t in (h, up, down)))
 
+    def _few_row_experts(n_slots, E, W, ff, gated, h, up, down):
+        """Whether the products stream the weights past position tiles of 32 rows (csrc/kernels/moe_rows.hip): up to FEW_SLOTS routed
+        rows per expert, where few experts have a second tile that streams their weight again.  Align, two products and combine, tiles of
+        64 rows -> of 32, us: 8 gated experts of 2048 x 2048, top 2: 4 rows per expert 95 -> 51, 16: 95 -> 60, 25: 95 -> 61, 32: 91 -> 75, 40:
+        97 -> 121; 4096 x 3072: 16: 187 -> 124, 32: 189 -> 180; 32 experts of 2048 x 1024, top 4: 4: 125 -> 101, 25: 130 -> 125, 31: 125 -> 138."""
+        return (h.dtype == torch.bfloat16 and n_slots <= FEW_SLOTS * E and W % 64 == 0 and ff % 64 == 0 and max(W, ff) <= 32768
+                and all(t.data_ptr() % 16 == 0 for t in (h, up, down)))
+
     def moe_experts(h, up, down, idx, weights, kind="relu2", limit=0.0):
         T, W = h.shape
         E, n_up, _ = up.shape
@@ -288,7 +299,8 @@ def seqmix_ops(lib, linear):
         n_slots = T * top
         dev, f32 = h.device, _act(h)
         wide = _wide_experts(n_slots, E, W, ff, kind, h, up, down)
-        rows = WIDE_ROWS if wide else tile_rows
+        few = not wide and _few_row_experts(n_slots, E, W, ff, gated, h, up, down)
+        rows = WIDE_ROWS if wide else few_rows if few else tile_rows
         n_tiles = (n_slots + E * (rows - 1) + rows - 1) // rows
         cap = n_tiles * rows
         sorted_ = torch.empty(cap, dtype=torch.int32, device=dev)
@@ -311,6 +323,17 @@ def seqmix_ops(lib, linear):
             return out
         _check(lib.bcg_moe_align(_p(idx), n_slots, E, _p(sorted_), cap, _p(tile_e), n_tiles, rows, None, None, _stream()),
                "moe_align")
+        if few:
+            code = ACT_CODES[EXPERT_ACTS[kind]] if gated else 1
+            held = min(E, n_slots) + n_slots // (2 * few_rows)     # tiles that are expected to hold rows
+            hidden = torch.empty(cap, ff, dtype=h.dtype, device=dev)
+            _check(lib.bcg_moe_rows(_p(h), T, W, _p(up), _p(hidden), ff, _p(sorted_), _p(tile_e), n_tiles, held, n_up, W, top, 1, 0,
+                                    code, limit, _stream()), "moe up rows")
+            y = torch.empty(n_slots, W, dtype=h.dtype, device=dev)
+            _check(lib.bcg_moe_rows(_p(hidden), cap, ff, _p(down), _p(y), W, _p(sorted_), _p(tile_e), n_tiles, held, W, ff, top, 0, 1,
+                                    0, 0.0, _stream()), "moe down rows")
+            _check(lib.bcg_moe_combine(_p(y), _p(weights), None, _p(out), T, W, top, f32, _stream()), "moe_combine")
+            return out
         code = ACT_CODES[EXPERT_ACTS[kind]] if gated else 1
         if gated and ff % 16 == 0:   # rows paired by `moe_pair_rows`: the hidden values in the product's epilogue
             hidden = torch.empty(cap, ff, dtype=h.dtype, device=dev)

@@ -73,6 +73,15 @@ __device__ __forceinline__ float clamped_glu(float gate, float up, float limit) 
   return g / (1.0f + expf(-1.702f * g)) * (u + 1.0f);
 }
 
+// Hidden value of a gated expert from its two products (rounded to T like a projection's output):
+// act 2 silu(gate) * up, the activation rounded too; act 3 `clamped_glu`, rounded once.
+template <typename T>
+__device__ __forceinline__ T gated_hidden(float gate, float up, int act, float limit) {
+  const float g = Elem<T>::ld(Elem<T>::st(gate)), u = Elem<T>::ld(Elem<T>::st(up));
+  if (act == 3) return Elem<T>::st(clamped_glu(g, u, limit));
+  return Elem<T>::st(Elem<T>::ld(Elem<T>::st(g / (1.0f + expf(-g)))) * u);
+}
+
 template <typename T>
 __device__ __forceinline__ typename Elem<T>::frag zero_frag() {
   typename Elem<T>::frag r;

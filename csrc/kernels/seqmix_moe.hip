@@ -13,7 +13,8 @@
 // Position tiles are TM rows; a tile belongs to one expert (tile_expert, -1 = unused).  Steps with many slots per
 // expert (`moe_experts` in ops/seqmix.py has the rule) take position tiles of 256 rows instead: `gather` copies the
 // token rows into position order, the products run on the 256 x 256 kernel of the dense projections
-// (bcg_gemm_w4_grouped) and `combine` reads the rows where they are.
+// (bcg_gemm_w4_grouped) and `combine` reads the rows where they are.  Steps with few slots per expert take tiles of 32 rows
+// and the streaming products of moe_rows.hip.
 #include <algorithm>
 
 #include "seqmix_common.h"
@@ -151,15 +152,6 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const uint4* __restric
   const uint4* src = a + static_cast<size_t>(slot / top) * row_vecs;
   uint4* dst = out + static_cast<size_t>(blockIdx.x) * row_vecs;
   for (int i = threadIdx.x; i < row_vecs; i += 256) dst[i] = src[i];
-}
-
-// Hidden value of a gated expert from its two products (rounded to T like a projection's output):
-// act 2 silu(gate) * up, the activation rounded too; act 3 `clamped_glu`, rounded once.
-template <typename T>
-__device__ __forceinline__ T gated_hidden(float gate, float up, int act, float limit) {
-  const float g = Elem<T>::ld(Elem<T>::st(gate)), u = Elem<T>::ld(Elem<T>::st(up));
-  if (act == 3) return Elem<T>::st(clamped_glu(g, u, limit));
-  return Elem<T>::st(Elem<T>::ld(Elem<T>::st(g / (1.0f + expf(-g)))) * u);
 }
 
 // Epilogue of a gated expert's first product (act 2, 3).  The N rows of the expert's weight are its
