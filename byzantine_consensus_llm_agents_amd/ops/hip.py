@@ -22,7 +22,7 @@ PREFILL_TILE_ROWS = 128
 PREFILL32_MAX_BLOCKS = 1024  # csrc/kernels/attention.hip: the 32x32 kernel's LDS block-id table
 
 # csrc/kernels/gemm_skinny.hip: most rows, most rows with a fused norm, longest rows in bytes
-SKINNY_ROWS, SKINNY_NORM_ROWS, SKINNY_ROW_BYTES = 32, 16, 65536
+SKINNY_ROWS, SKINNY_NORM_ROWS, SKINNY_ROW_BYTES = 64, 16, 65536
 # `decode_attention`: every workgroup of a row rotates its queries again, so with many rows the separate launch wins (a step of
 # 24 layers of 14 / 2 heads of 64, us: 120 rows 2051 separate, 2029 fused; 400 rows 2833, 2871)
 DECODE_FUSED_ROWS = 128
@@ -438,7 +438,13 @@ def hip_ops() -> SimpleNamespace:
         rows of W lose to a split of K over the CUs (us, tile kernels or library and this one):
         * up to 16 rows only the gated form past 12288 columns of bf16 (1024 x 16384 22.2, 25.3; 5120 x 25600 138, 48);
         * 17 to 32 rows: rows of up to 8192 bytes always gain (256 x 4096 11.2, 8.7; 2048 x 4096 14.7, 9.0), longer ones from 4096
-          rows of W on (4096 x 12288 26.0, 24.9; but 3072 x 16384 28.5, 29.3; 1024 x 6144 10.5, 11.7; 256 x 8192 8.7, 14.6)."""
+          rows of W on (4096 x 12288 26.0, 24.9; but 3072 x 16384 28.5, 29.3; 1024 x 6144 10.5, 11.7; 256 x 8192 8.7, 14.6);
+        * 33 to 48 rows: one pass over W and rows of up to 8192 bytes (4096 x 2048 11.8, 8.0; 4096 x 4096 13.6, 12.5; 256 x 2048 7.5, 7.2;
+          but 8736 x 2048 14.7, 15.1; 2048 x 8192 13.8, 18.7);
+        * 49 to 64 rows: of those rows of up to 4096 bytes, 1024 of them and more (4096 x 2048 12.4, 9.5; 6144 x 768 10.0, 7.4; but 4096 x
+          4096 13.8, 14.9; 768 x 2048 8.1, 8.9)."""
+        if M > 32:
+            return N <= 32 * 256 and (row_bytes <= 8192 if M <= 48 else row_bytes <= 4096 and N >= 1024)
         if M <= 16:
             return epi != 1 or row_bytes <= 2 * SKINNY_LONG_K or N >= 4096
         return row_bytes <= 8192 or N >= 4096
@@ -777,7 +783,7 @@ def hip_ops() -> SimpleNamespace:
         """Whether the few-row kernel takes the fp8 product: as `_skinny`; `beside`: [(bias or residual, its shape)]."""
         M, K = xq.shape
         N = wq.shape[0]
-        return (plan.mode == "1" and 1 <= M <= SKINNY_ROWS and K % 128 == 0 and 128 <= K <= SKINNY_ROW_BYTES and N >= 16 and N % 16 == 0
+        return (plan.mode == "1" and 1 <= M <= 32 and K % 128 == 0 and 128 <= K <= SKINNY_ROW_BYTES and N >= 16 and N % 16 == 0
                 and _few_rows_pay(M, N, K, 0) and xq.is_cuda and xq.get_device() == torch.cuda.current_device() and xq.is_contiguous() and wq.is_contiguous()
                 and all(t.device == xq.device and t.data_ptr() % 16 == 0 and bare(t) for t in (xq, wq, xs, ws))
                 and xs.dtype == ws.dtype == torch.float32 and xs.numel() == M and ws.numel() == N and xs.is_contiguous()

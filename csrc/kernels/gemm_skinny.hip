@@ -1,7 +1,7 @@
-// Projection GEMM of a few rows: C[M, N] = X[M, K] . W[N, K]^T for M <= 32 in bf16 or fp8 (e4m3, row and column scales), with
+// Projection GEMM of a few rows: C[M, N] = X[M, K] . W[N, K]^T for M <= 64 in bf16, <= 32 in fp8 (e4m3, row and column scales), with
 // the RMS norm of the input, the gated unit and the residual update fused (a decode step of one to three games).
 //
-// What bounds it: every weight byte is read once and meets at most 32 activation rows, so the kernel is a stream over W.  Plain
+// What bounds it: every weight byte is read once and meets a few dozen activation rows at most, so the kernel is a stream over W.  Plain
 // streaming loads of such weights reach 6.7 TB/s at 356 MB and 6.1 at 84 MB, launch included; the rest is what a CU takes in:
 // X comes from L2 once per CU, and a CU's load path follows the address quads: four neighbouring lanes that read 64 bytes of
 // one row cost a quarter of four that read 16 bytes of four rows (the order of the matrix instruction): 117 and 36 B/ns per CU
@@ -25,7 +25,8 @@
 // 5120 74.5 -> 59.8, 151936 x 5120 265 -> 234, 4096 x 4096 10.3 -> 9.2, 4096 x 12288 23 -> 18.7, 5120 x 17408 (tile kernel 36.6) 31.9.
 // 20 rows, tile kernel with split-K -> now: fp8 8192 x 6144 15.4 -> 11.6, 6144 x 6144 14.8 -> 10.5, 32768 x 6144 38.5 -> 35.1, 6144 x
 // 16384 27.4 -> 20.8; bf16 32768 x 6144 75.4 -> 68.6.  Launches in a graph, every one with other weights.  From 33 rows on X takes
-// more of a CU's intake than W (64 rows, 4096 x 4096: 14 to 15 us, the tile kernel 14).
+// more of a CU's intake than W, and two blocks of W fill the registers: short rows in one pass only (64 rows, library -> here:
+// 4096 x 2048 12.4 -> 9.5; 4096 x 4096: tile kernel 13.8, here 14.9).
 #include <type_traits>
 
 #include "common.h"
@@ -38,7 +39,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x8 __attribute__((ext_vector_type(8)));
 
 constexpr int CUS = 256, NW = 8;             // workgroups, waves of one
-constexpr int MAX_ROWS = 32, MAX_NORM_ROWS = 16, MAX_ROW_BYTES = 65536, MAX_NORM_K = 16384;
+constexpr int MAX_ROWS = 64, MAX_NORM_ROWS = 16, MAX_ROW_BYTES = 65536, MAX_NORM_K = 16384;
 constexpr uint32_t PAST_END = 0x80000000u;   // an offset outside every descriptor
 constexpr int ROUND_KB = 64;                 // LDS of one round of a reduction
 
@@ -347,7 +348,7 @@ int launch(SkinnyArgs a, int passes, hipStream_t stream) {
 template <int MT, int EPI, bool NORM, bool F8>
 int pick(const SkinnyArgs& a, hipStream_t s) {
   constexpr int PER = EPI == EPI_SILU_MUL ? 2 : 4;                             // groups of 4 columns of a block of W
-  constexpr int MOST = EPI == EPI_SILU_MUL ? (MT == 1 ? 6 : 4) : (MT == 1 ? 8 : 4);   // (registers of two waves per SIMD)
+  constexpr int MOST = MT >= 3 ? 2 : MT == 2 ? 4 : EPI == EPI_SILU_MUL ? 6 : 8;   // (registers of two waves per SIMD)
   const int share = (a.units + CUS - 1) / CUS, passes = (share + MOST * PER - 1) / (MOST * PER);
   const int blocks = ((share + passes - 1) / passes + PER - 1) / PER;
   if constexpr (MT == 1 && !F8) {
@@ -367,14 +368,25 @@ int pick(const SkinnyArgs& a, hipStream_t s) {
     if (blocks <= 2) return launch<MT, 2, 256, 1, EPI, NORM, F8>(a, passes, s);
     if constexpr (MT == 1)
       if (blocks > 4) return launch<MT, 6, 256, 1, EPI, NORM, F8>(a, passes, s);
-    return launch<MT, 4, 256, 1, EPI, NORM, F8>(a, passes, s);
+    if constexpr (MT <= 2) return launch<MT, 4, 256, 1, EPI, NORM, F8>(a, passes, s);
+    return -2;
   } else {
     if (blocks <= 1) return launch<MT, 1, 256, 1, EPI, NORM, F8>(a, passes, s);
     if (blocks <= 2) return launch<MT, 2, 256, 1, EPI, NORM, F8>(a, passes, s);
     if constexpr (MT == 1)
       if (blocks > 4) return launch<MT, 8, 256, 1, EPI, NORM, F8>(a, passes, s);
-    return launch<MT, 4, 256, 1, EPI, NORM, F8>(a, passes, s);
+    if constexpr (MT <= 2) return launch<MT, 4, 256, 1, EPI, NORM, F8>(a, passes, s);
+    return -2;
   }
+}
+
+// by the blocks of 16 rows
+template <int EPI, bool F8>
+int pick_rows(const SkinnyArgs& a, hipStream_t s) {
+  if (a.M <= 16) return pick<1, EPI, false, F8>(a, s);
+  if (a.M <= 32) return pick<2, EPI, false, F8>(a, s);
+  if constexpr (!F8) return a.M <= 48 ? pick<3, EPI, false, false>(a, s) : pick<4, EPI, false, false>(a, s);
+  return -2;
 }
 
 bool covered(int M, int row_bytes, int n_out) {
@@ -384,7 +396,7 @@ bool covered(int M, int row_bytes, int n_out) {
 }  // namespace
 
 // epi: 0 = store (+bias), 1 = silu(gate)*up into [M, N / 2], 2 = residual + acc (+bias).  norm_w: RMS-normalise the rows
-// of x with these weights first (epi 0, 1; M <= 16, K <= 16384).  1 <= M <= 32, K % 64 == 0, 64 <= K <= 32768, the output
+// of x with these weights first (epi 0, 1; M <= 16, K <= 16384).  1 <= M <= 64, K % 64 == 0, 64 <= K <= 32768, the output
 // width a multiple of 4; rows contiguous, x and w 16-byte aligned, the others 8-byte aligned.
 BCG_API int bcg_gemm_skinny(int epi, const void* x, const void* w, const void* norm_w, float eps, const void* bias,
                             const void* residual, void* c, int M, int N, int K, hipStream_t stream) {
@@ -397,14 +409,14 @@ BCG_API int bcg_gemm_skinny(int epi, const void* x, const void* w, const void* n
   switch (epi) {
     case EPI_STORE:
       if (norm_w) return pick<1, EPI_STORE, true, false>(a, stream);
-      return M <= 16 ? pick<1, EPI_STORE, false, false>(a, stream) : pick<2, EPI_STORE, false, false>(a, stream);
+      return pick_rows<EPI_STORE, false>(a, stream);
     case EPI_SILU_MUL:
       if (bias) return -2;
       if (norm_w) return pick<1, EPI_SILU_MUL, true, false>(a, stream);
-      return M <= 16 ? pick<1, EPI_SILU_MUL, false, false>(a, stream) : pick<2, EPI_SILU_MUL, false, false>(a, stream);
+      return pick_rows<EPI_SILU_MUL, false>(a, stream);
     case EPI_RESIDUAL:
       if (!residual || norm_w) return -2;
-      return M <= 16 ? pick<1, EPI_RESIDUAL, false, false>(a, stream) : pick<2, EPI_RESIDUAL, false, false>(a, stream);
+      return pick_rows<EPI_RESIDUAL, false>(a, stream);
     default: return -2;
   }
 }
@@ -413,15 +425,15 @@ BCG_API int bcg_gemm_skinny(int epi, const void* x, const void* w, const void* n
 // K <= 65536, N a multiple of 4; rows contiguous, xq, wq and w_scale 16-byte aligned, the others 8-byte aligned.
 BCG_API int bcg_gemm_skinny_fp8(int epi, const void* xq, const void* wq, const float* x_scale, const float* w_scale, const void* bias,
                                 const void* residual, void* c, int M, int N, int K, hipStream_t stream) {
-  if (!covered(M, K, N) || !x_scale || !w_scale) return -2;
+  if (!covered(M, K, N) || M > 32 || !x_scale || !w_scale) return -2;
   const SkinnyArgs a{static_cast<const uint8_t*>(xq), static_cast<const uint8_t*>(wq), nullptr, static_cast<const bf16_t*>(bias),
                      static_cast<const bf16_t*>(residual), static_cast<bf16_t*>(c), x_scale, w_scale,
                      M, K, N, 0, N / 4, 1, 0.f, 0.f};
   switch (epi) {
-    case EPI_STORE: return M <= 16 ? pick<1, EPI_STORE, false, true>(a, stream) : pick<2, EPI_STORE, false, true>(a, stream);
+    case EPI_STORE: return pick_rows<EPI_STORE, true>(a, stream);
     case EPI_RESIDUAL:
       if (!residual) return -2;
-      return M <= 16 ? pick<1, EPI_RESIDUAL, false, true>(a, stream) : pick<2, EPI_RESIDUAL, false, true>(a, stream);
+      return pick_rows<EPI_RESIDUAL, true>(a, stream);
     default: return -2;
   }
 }

@@ -8,10 +8,10 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-# rows, N, K: 17 and 32 rows; one column group per workgroup; passes (N / 256 > 64 at two blocks, > 128 at one); K of 1, 1.5 and
+# rows, N, K: 17, 32, 33, 48, 49 and 64 rows; one column group per workgroup; passes (N / 256 > 64 at two blocks, > 128 at one); K of 1, 1.5 and
 # an odd number of units; K from 12289 on and the longest
 SHAPES = [(17, 8, 128), (32, 1028, 192), (20, 5120, 5120), (31, 17408, 448), (24, 70000, 320), (32, 4096, 17408), (16, 70000, 1088),
-          (10, 5120, 17408), (3, 256, 32768), (16, 520, 1600), (32, 36864, 576)]
+          (10, 5120, 17408), (3, 256, 32768), (16, 520, 1600), (32, 36864, 576), (33, 8, 64), (48, 8192, 320), (49, 1024, 2048), (64, 8188, 1088)]
 
 
 @pytest.fixture(scope="module")
