@@ -216,9 +216,17 @@ def seqlatent_ops(lib):
 
     def moe_table_route(tokens, table, top):
         _req(tokens.dtype == torch.int32 and tokens.dim() == 1 and table.dtype == torch.int32 and table.dim() == 2
-             and 1 <= top <= table.shape[1], "moe_table_route: tokens int32 [T], table int32 [vocab, >= top]")
-        idx = table.index_select(0, tokens)[:, :top].contiguous()
-        return idx, torch.full(idx.shape, 1.0 / top, dtype=torch.float32, device=idx.device)
+             and tokens.device == table.device and 1 <= top <= table.shape[1], "moe_table_route: tokens int32 [T], table int32 [vocab, >= top]")
+        T = tokens.numel()
+        if T * top >= 1 << 24:
+            idx = table.index_select(0, tokens)[:, :top].contiguous()
+            return idx, torch.full(idx.shape, 1.0 / top, dtype=torch.float32, device=idx.device)
+        tokens, table = tokens.contiguous(), table.contiguous()
+        idx = torch.empty(T, top, dtype=torch.int32, device=table.device)
+        wts = torch.empty(T, top, dtype=torch.float32, device=table.device)
+        _check(lib.bcg_moe_route_table(_p(tokens), _p(table), table.shape[0], table.shape[1], top, T, _p(idx), _p(wts), _stream()),
+               "moe_route_table")
+        return idx, wts
 
     def gelu_gather_mul(z, tokens, table, off):
         _req(z.dim() == 2 and z.is_contiguous() and table.dim() == 2 and table.is_contiguous() and table.dtype == z.dtype

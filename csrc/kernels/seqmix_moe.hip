@@ -105,6 +105,17 @@ __global__ __launch_bounds__(256) void route_kernel(const T* __restrict__ h, con
   }
 }
 
+// Routing by token id: the first `top` entries of the token's table row, every weight 1 / top.  A token outside the table has no
+// expert (-1).
+__global__ __launch_bounds__(256) void route_table_kernel(const int* __restrict__ tokens, const int* __restrict__ table, int vocab,
+                                                          int width, int top, int n, int* __restrict__ idx, float* __restrict__ wts) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const int token = tokens[i / top];
+  idx[i] = token >= 0 && token < vocab ? table[static_cast<size_t>(token) * width + i % top] : -1;
+  wts[i] = 1.0f / top;
+}
+
 __global__ __launch_bounds__(1024) void align_kernel(const int* __restrict__ idx, int n_slots, int E,
                                                      int* __restrict__ sorted, int cap, int* __restrict__ tile_expert,
                                                      int n_tiles, int tm, int* __restrict__ pos, int* __restrict__ used) {
@@ -509,6 +520,17 @@ BCG_API int bcg_moe_route(const void* h, const void* rw, const void* rb, const v
     route_kernel<bf16_t><<<T_, 256, 0, s>>>(static_cast<const bf16_t*>(h), static_cast<const float*>(rw), static_cast<const float*>(rb),
                                           static_cast<const float*>(gw), static_cast<int*>(idx), static_cast<float*>(wts),
                                           static_cast<float*>(gate), W, E, top, 0, nullptr, 1, 1, 1.0f);
+  return BCG_CHECK_LAUNCH();
+}
+
+// idx, wts: [T, top] from table [vocab, width], width >= top.
+BCG_API int bcg_moe_route_table(const void* tokens, const void* table, int vocab, int width, int top, int T_, void* idx, void* wts,
+                                void* stream) {
+  if (T_ <= 0) return 0;
+  if (vocab < 1 || top < 1 || top > width || T_ > (1 << 24) / top) return -2;
+  route_table_kernel<<<(T_ * top + 255) / 256, 256, 0, static_cast<hipStream_t>(stream)>>>(
+      static_cast<const int*>(tokens), static_cast<const int*>(table), vocab, width, top, T_ * top, static_cast<int*>(idx),
+      static_cast<float*>(wts));
   return BCG_CHECK_LAUNCH();
 }
 

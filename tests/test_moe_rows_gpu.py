@@ -29,3 +29,15 @@ def test_few_row_experts(kind, limit, routing, T, E, top, W, ff):
     for _ in range(2):
         out = ops.moe_experts(h, up, down, idx, w, kind, limit)
         assert ((out.double() - want).norm() / want.norm()).item() < 2 ** -7
+
+
+@pytest.mark.parametrize("T,width,top", [(1, 1, 1), (128, 8, 2), (257, 3, 3)])
+def test_table_routing(T, width, top):
+    """The table's entries, also from a table and tokens that are views; a token outside the table has no expert."""
+    from byzantine_consensus_llm_agents_amd.ops import get_ops
+    ops, g = get_ops("hip"), torch.Generator(device="cuda").manual_seed(T)
+    table = torch.randint(0, 99, (50, 2 * width), device="cuda", generator=g, dtype=torch.int32)[:, :width]
+    tokens = torch.randint(0, 50, (2 * T,), device="cuda", generator=g, dtype=torch.int32)[::2]
+    idx, w = ops.moe_table_route(tokens, table, top)
+    assert torch.equal(idx, table[tokens.long(), :top]) and (w == 1.0 / top).all() and w.shape == (T, top)
+    assert (ops.moe_table_route(torch.tensor([-1, 50], dtype=torch.int32, device="cuda"), table, top)[0] == -1).all()
