@@ -170,21 +170,26 @@ class MofidraModel:
         for r, li in enumerate(runs):
             spec, L = c.layers[li], self.layers[li]
             m, f = spec.mixer, spec.mlp
-            y = ops.linear(h, L["fused"])
+            off, last = m.q_width + m.k_width + m.v_width, r == len(runs) - 1
+            hidden, few = None, last and meta.logits_idx is not None   # few: rows that go on past the last attention
+            if f is not None and f.kind == "dense" and not few:
+                y, hidden = ops.linear_tail_gelu(h, L["fused"], off)
+            else:
+                y = ops.linear(h, L["fused"])
             q = ops.rope_multi_kv_write(y, meta.positions, meta.slots, m.heads, m.kv_heads, m.maps, m.dim, m.vdim,
                                         L["inv_freq"], k_cache[r], v_cache[r])
             attn = ops.multimap_attention(q, k_cache[r], v_cache[r], meta, m.scale, m.maps, L["lam"], eps,
                                           1.0 - m.diff, m.vdim)
-            last = r == len(runs) - 1
-            if last and meta.logits_idx is not None:
+            if few:
                 # past the last attention only the rows whose logits are asked for matter
                 idx = meta.logits_idx
                 attn, x, h, y = (t.index_select(0, idx) for t in (attn, x, h, y))
             parts = [ops.linear(attn, L["o"])]
             gate = gated = None
-            off = m.q_width + m.k_width + m.v_width
             if f is not None and f.kind == "dense":
-                parts.append(ops.linear(ops.act_fn(y[:, off:off + f.ff], "gelu_tanh"), L["down"]))
+                if hidden is None:
+                    hidden = ops.act_fn(y[:, off:off + f.ff], "gelu_tanh")
+                parts.append(ops.linear(hidden, L["down"]))
             elif f is not None:
                 idx_e, w_e, gate = ops.moe_route(h, L["router"], L["router_b"], f.top, L.get("s_gate"))
                 parts.append(ops.moe_experts(h, L["e_up"], L["e_down"], idx_e, w_e, "relu2"))

@@ -31,7 +31,7 @@ Kernel plan of one layer run (HIP backend; the torch backend runs the same ops f
                       (W_uk) + rope_tail -> multimap_attention (one KV head) -> head_linear (W_uv) -> o GEMM
     residual_post_norm  x += s * rms(y), the entry of the next pass, and the next reader's RMS norm, one pass
                       over the row
-    feed-forward      [gate | up] GEMM -> gated_act (clamped_glu) -> down GEMM, or
+    feed-forward      [gate | up] GEMM with clamped_glu (linear_clamped_glu) -> down GEMM, or
                       moe_route -> grouped expert GEMMs (clamped_glu in the epilogue) -> combine
 
 No host synchronisation anywhere: a decode step is capturable in a HIP graph.
@@ -262,7 +262,7 @@ class VagozenModel:
     def _feed_forward(self, f, L, h):
         ops = self.ops
         if f.kind == "dense":
-            return ops.linear(ops.gated_act(ops.linear(h, L["up"]), "clamped_glu", f.limit), L["down"])
+            return ops.linear(ops.linear_clamped_glu(h, L["up"], f.limit), L["down"])
         idx, w, _ = ops.moe_route(h, L["router"], L["router_b"], f.top)
         return ops.moe_experts(h, L["e_up"], L["e_down"], idx, w, "clamped_glu", f.limit)
 

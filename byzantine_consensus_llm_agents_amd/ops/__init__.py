@@ -41,6 +41,7 @@ def _torch_ops() -> SimpleNamespace:
         rope_multi_kv_write=_ref.rope_multi_kv_write,
         multimap_attention=multimap_attention,
         act_fn=_ref.act_fn,
+        linear_tail_gelu=_ref.linear_tail_gelu,
         moe_route=_ref.moe_route,
         moe_experts=_ref.moe_experts,
         embed_hashed_bigram_norm=_ref.embed_hashed_bigram_norm,
@@ -65,6 +66,7 @@ def _torch_ops() -> SimpleNamespace:
         moe_table_route=_ref.moe_table_route,
         gelu_gather_mul=_ref.gelu_gather_mul,
         gated_act=_ref.gated_act,
+        linear_clamped_glu=_ref.linear_clamped_glu,
         hyper_embed_norm=_ref.hyper_embed_norm,
         hyper_update_norm=_ref.hyper_update_norm,
         rope_norm_kv_write=_ref.rope_norm_kv_write,

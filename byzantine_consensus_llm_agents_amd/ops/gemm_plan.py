@@ -142,6 +142,26 @@ class GemmPlan:
             return N
         return 256 * n1
 
+    def clamped_tiles(self, M: int, N: int, K: int) -> bool:
+        """Whether the 256 x 256 kernel takes a clamped gated projection, the unit in its epilogue, from 512 rows on.
+
+        The rule of the other gated epilogue, `_large_tiles`.  Product and activation pass over the one launch: filled rounds
+        (0.8 and more) 16384 x 2048 (N x K) 1.13 to 1.29 over 1000 to 12000 rows, 24576 x 4096 1.00 to 1.13, 8192 x 1024 1.30 to 1.40; below
+        that 0.75 (0.56 filled, 24576 x 4096, 640 rows) to 1.16."""
+        return (self.mode == "1" and M >= 512 and self.supported(W4_CFG, M, N, K, 1)
+                and self._large_tiles(K, 1, -(-M // 256) * (N // 256)))
+
+    def tail_tiles(self, M: int, N: int, K: int, at: int) -> bool:
+        """Whether the 256 x 256 kernel takes a projection whose columns from `at` on go through gelu in its epilogue.
+
+        Product (as `pieces` has it) and activation pass over the one launch, from 1024 rows on: rounds filled to 0.9 and more 1.03 to
+        1.18 (18432 x 4096 in 504 tiles: 1.00), to 0.8 up to K = 2048 1.01 to 1.14 (N 6656 and 11264), at K = 4096 0.92 to 1.01; below
+        that 0.79 to 1.19."""
+        if not (self.mode == "1" and M >= 1024 and 0 < at < N and at % 256 == 0 and self.supported(W4_CFG, M, N, K, 0)):
+            return False
+        tiles = -(-M // 256) * -(-N // 256)
+        return tiles >= (0.8 if K <= 2048 else 0.9) * CUS * -(-tiles // CUS)
+
     def pieces(self, M: int, N: int, K: int, epi: int) -> List[Tuple[int, Optional[Tuple[int, int]]]]:
         """[(rows, choice)]: how the M rows run, one choice for all of them or two runs of rows.
 

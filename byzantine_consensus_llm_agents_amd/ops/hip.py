@@ -171,6 +171,7 @@ def load_library(path: str = None) -> ctypes.CDLL:
         "bcg_rope_tail": [c_void_p, c_int, c_int, c_void_p, c_int, c_int, c_void_p, c_void_p, c_int, c_float, c_int, c_int,
                           c_int, c_int, c_void_p],
         "bcg_gate_mul": [c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_int, c_int, c_int, c_int, c_void_p],
+        "bcg_gemm_w4_act": [c_int] + [c_void_p] * 4 + [c_int] * 4 + [c_float, c_void_p],
         "bcg_gated_act": [c_void_p, c_void_p, c_int64, c_int, c_int, c_float, c_int, c_void_p],
         "bcg_ssm_prepare": [c_void_p, c_int64, c_int, c_void_p, c_int64, c_int, c_void_p, c_void_p, c_void_p, c_void_p,
                             c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
@@ -616,6 +617,33 @@ def hip_ops() -> SimpleNamespace:
                 gemm_nt(xr, w, cfg, 1, out=dst)
         return out
 
+    def _w4_act(epi, x, w, c, tail, inter, limit):
+        M, K = x.shape
+        _log(M, w.shape[0], K, epi, (W4_CFG, 1))
+        _check(lib.bcg_gemm_w4_act(epi, _p(x), _p(w), _p(c), None if tail is None else _p(tail), M, w.shape[0], K, inter, limit, _stream()),
+               "gemm_w4_act")
+
+    def linear_clamped_glu(x, w, limit):
+        """gated_act(linear(x, w), "clamped_glu", limit), W = [gate; up]: one launch where `GemmPlan.clamped_tiles` says so."""
+        M, K = x.shape
+        if not (limit > 0 and plan.clamped_tiles(M, w.shape[0], K) and _plain(x, w)):
+            return extra["gated_act"](linear(x, w), "clamped_glu", limit)
+        out = torch.empty(M, w.shape[0] // 2, dtype=x.dtype, device=x.device)
+        _w4_act(5, x, w, out, None, w.shape[0] // 2, float(limit))
+        return out
+
+    def linear_tail_gelu(x, w, at):
+        """(y, hidden): y = linear(x, w) and None, or, where `GemmPlan.tail_tiles` says that one launch gains, the first `at` columns
+        of it and act_fn of the others, "gelu_tanh"."""
+        M, K = x.shape
+        N = w.shape[0]
+        if not (plan.tail_tiles(M, N, K, at) and _plain(x, w)):
+            return linear(x, w), None
+        y = torch.empty(M, at, dtype=x.dtype, device=x.device)
+        hidden = torch.empty(M, N - at, dtype=x.dtype, device=x.device)
+        _w4_act(6, x, w, y, hidden, at, 0.0)
+        return y, hidden
+
     def _norm_fusable(x, w_norm):
         return x.shape[0] <= SKINNY_NORM_ROWS and x.shape[1] <= 8192 and _plain_beside(w_norm, (x.shape[1],), x)
 
@@ -840,6 +868,7 @@ def hip_ops() -> SimpleNamespace:
 
     return SimpleNamespace(name="hip", **extra, rmsnorm_fp8=rmsnorm_fp8, embed_rmsnorm_fp8=embed_rmsnorm_fp8,
                            linear_fp8_residual=linear_fp8_residual, linear=linear, norm_linear=norm_linear, norm_linear_silu=norm_linear_silu, linear_silu=linear_silu, linear_residual=linear_residual,
+                           linear_clamped_glu=linear_clamped_glu, linear_tail_gelu=linear_tail_gelu,
                            gemm_nt=gemm_nt, gemm_plan=plan, prepare_device=prepare_device,
                            register_stream=register_stream, quant_fp8=quant_fp8, add_rmsnorm_fp8=add_rmsnorm_fp8,
                            silu_mul_fp8=silu_mul_fp8, linear_fp8=linear_fp8, gemm_nt_fp8=gemm_nt_fp8, fp8_cfg=fp8_cfg, rmsnorm=rmsnorm, add_rmsnorm=add_rmsnorm, silu_mul=silu_mul,

@@ -488,6 +488,13 @@ def act_fn(x: torch.Tensor, kind: str) -> torch.Tensor:
     return y.to(x.dtype)
 
 
+def linear_tail_gelu(x, w, at: int):
+    """(y, hidden): ``y = x W^T``, of which a backend may leave out the columns from ``at`` on, and "gelu_tanh" of those
+    columns, or None where the caller applies `act_fn` to ``y[:, at:]`` itself."""
+    y = torch.nn.functional.linear(x, w)
+    return y[:, :at], act_fn(y[:, at:], "gelu_tanh")
+
+
 def moe_route(h, router_w, router_b, top: int, gate_w=None):
     """fp32 router: ``z = W h + b``; the ``top`` largest logits (ties: lowest index) and the
     softmax over those only.  Returns (expert ids int32 [T, top], weights fp32 [T, top],
@@ -986,6 +993,11 @@ def gated_act(both, kind: str = "silu", limit: float = 0.0):
         return clamped_glu(both, limit)
     n = both.shape[1] // 2
     return (act_fn(both[:, :n], kind).float() * both[:, n:].float()).to(both.dtype)
+
+
+def linear_clamped_glu(x, w, limit: float):
+    """`gated_act` ("clamped_glu") of ``x W^T``, W = [gate; up]."""
+    return clamped_glu(torch.nn.functional.linear(x, w), limit)
 
 
 # ------------------------------------------------------------------ hyper-connection streams, layer norms, unit-norm rotary

@@ -85,7 +85,9 @@ constexpr int BM = 256, BN = 256, BK = 64;
 constexpr int W4_COUNTERS = 65536;  // the caller's arrival-counter array (one per tile)
 constexpr int A_BYTES = BM * 128;  // one operand's K-tile: 256 rows of 128 B
 // EPI_GATED: W's rows alternate 16 gate and 16 up rows as they lie in memory (bcg_gemm_w4_grouped)
-enum Epilogue { EPI_STORE = 0, EPI_SILU_MUL = 1, EPI_RESIDUAL = 2, EPI_GATED = 3, EPI_RELU2 = 4 };
+// EPI_CLAMPED: the clamped unit of W = [gate; up], EPI_TAIL_GELU: gelu on the columns from `inter` on, which go to an output
+// of their own (bcg_gemm_w4_act)
+enum Epilogue { EPI_STORE = 0, EPI_SILU_MUL = 1, EPI_RESIDUAL = 2, EPI_GATED = 3, EPI_RELU2 = 4, EPI_CLAMPED = 5, EPI_TAIL_GELU = 6 };
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -99,6 +101,11 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 // g * sigmoid(g) with the hardware reciprocal (1 ulp; a true division expands to ~10
 // instructions with mode switches per element in the epilogue)
 __device__ __forceinline__ float silu(float g) { return g * __builtin_amdgcn_rcpf(1.f + __expf(-g)); }
+
+// gelu, tanh form: z sigmoid(2 u) is 0.5 z (1 + tanh(u))
+__device__ __forceinline__ float gelu(float z) {
+  return z * __builtin_amdgcn_rcpf(1.f + __expf(-1.5957691216057308f * (z + 0.044715f * z * z * z)));
+}
 
 __device__ __forceinline__ u16x4 pack4(float a, float b, float c, float d) {
   typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
@@ -162,6 +169,8 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
     const int* __restrict__ group, const int* __restrict__ used, float limit) {
   static_assert(!F8 || EPI == EPI_STORE || EPI == EPI_RESIDUAL, "fp8: store / residual epilogues");
   static_assert(GROUPED || (EPI != EPI_GATED && EPI != EPI_RELU2), "grouped epilogues");
+  constexpr bool STACKED = EPI == EPI_SILU_MUL || EPI == EPI_CLAMPED;   // W = [gate; up]
+  if constexpr (EPI == EPI_CLAMPED || EPI == EPI_TAIL_GELU) split_k = 1;
   if constexpr (GROUPED) {
     m_tiles = min(m_tiles, used[0]);
     split_k = 1;
@@ -254,20 +263,20 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
   const uint32_t row_bytes = static_cast<uint32_t>(K) * ESZ;
   const int prow = 8 * wave + (lane >> 3);
   const int pch = ((lane & 7) ^ ((4 * wave + (lane >> 4)) & 7)) * 16;
-  const int w_rows = EPI == EPI_SILU_MUL ? 2 * inter : N;
+  const int w_rows = STACKED ? 2 * inter : N;
   auto item_srd = [&](const Geo& g, i32x4& sX, i32x4& sW) {
-    const int wr0 = EPI == EPI_SILU_MUL ? (g.n0 >> 1) : g.n0;
+    const int wr0 = STACKED ? (g.n0 >> 1) : g.n0;
     sX = make_srd(X + static_cast<size_t>(g.m0) * row_bytes, static_cast<uint32_t>(M - g.m0) * row_bytes);
     const size_t w_first = (GROUPED ? static_cast<size_t>(group[g.m0 / BM]) * N : 0) + wr0;
     sW = make_srd(W + w_first * row_bytes, static_cast<uint32_t>(w_rows - wr0) * row_bytes);
   };
   const uint32_t voffX = static_cast<uint32_t>(prow) * row_bytes + pch;
-  // SILU: 16-row blocks of the tile alternate gate / up of the same 16 features, so stage row
+  // STACKED: 16-row blocks of the tile alternate gate / up of the same 16 features, so stage row
   // 32 i + r (r < 32) holds W row (r >> 4) * inter + n0/2 + 16 i + (r & 15)
   const uint32_t voffW =
-      static_cast<uint32_t>(EPI == EPI_SILU_MUL ? (wave >> 1) * inter + (prow & 15) : prow) * row_bytes + pch;
+      static_cast<uint32_t>(STACKED ? (wave >> 1) * inter + (prow & 15) : prow) * row_bytes + pch;
   const uint32_t strideX = 32u * row_bytes;
-  const uint32_t strideW = (EPI == EPI_SILU_MUL ? 16u : 32u) * row_bytes;
+  const uint32_t strideW = (STACKED ? 16u : 32u) * row_bytes;
   // the row part of a piece's offset stays in the VGPR offset: only that is range-checked
   // (the SGPR offset carries the K-tile)
   uint32_t vX[8], vW[8];
@@ -414,13 +423,17 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
       // offset (m-block j's rows included) rides in the VGPR: only that part is range-checked (an
       // SGPR offset is added after the check), and the host bounds (M + 256) * ldc * 2 below
       // 2^31 so a masked column's 0x80000000 + offset never wraps into range.
-      constexpr bool SILU = EPI == EPI_SILU_MUL || EPI == EPI_GATED;
+      constexpr bool SILU = STACKED || EPI == EPI_GATED;
       constexpr int NP = SILU ? NB / 4 : NB / 2;  // 8-column groups per m-block per lane
       constexpr int JG = 1;                       // m-blocks per residual batch
-      const uint32_t ldb = static_cast<uint32_t>(ldc) * 2;
-      const int c0 = SILU ? (n0 >> 1) : n0;
+      // (EPI_TAIL_GELU: a tile lies on one side of `inter`, its columns past it in the second output, `residual` here)
+      const bool tail = EPI == EPI_TAIL_GELU && __builtin_amdgcn_readfirstlane(n0) >= inter;
+      const int ld = tail ? N - inter : ldc;
+      const uint32_t ldb = static_cast<uint32_t>(ld) * 2;
+      const int c0 = SILU ? (n0 >> 1) : tail ? n0 - inter : n0;
       const uint32_t range = static_cast<uint32_t>(M - m0) * ldb;
-      const auto rc = __builtin_amdgcn_make_buffer_rsrc(C + static_cast<size_t>(m0) * ldc + c0, 0, range, 0x00020000);
+      const auto rc = __builtin_amdgcn_make_buffer_rsrc((tail ? const_cast<bf16_t*>(residual) : C) + static_cast<size_t>(m0) * ld + c0, 0,
+                                                        range, 0x00020000);
       const uint32_t rowv = static_cast<uint32_t>(wm * 128 + fr) * ldb;
       uint32_t colv[NP];
 #pragma unroll
@@ -456,7 +469,7 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
 #pragma unroll
             for (int k = 0; k < 2; ++k) {
               const auto g = value(4 * p + 2 * k, j), u = value(4 * p + 2 * k + 1, j);
-              if (EPI == EPI_GATED && limit > 0.f) {  // clamped unit: min(g, limit), u within +-limit
+              if (EPI == EPI_CLAMPED || (EPI == EPI_GATED && limit > 0.f)) {  // clamped unit: min(g, limit), u within +-limit
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                   const float gc = fminf(g[e], limit), uc = fminf(fmaxf(u[e], -limit), limit);
@@ -490,10 +503,11 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
                     rr_rs, rowv + colv[p] + static_cast<uint32_t>((j0 + jj) * MB) * ldb, 0, 0);
           }
         };
-        // one body per bias case (a uniform branch here, not one per quad); the bias groups
+        // one body per bias case (a uniform branch here, not one per quad; EPI_TAIL_GELU, without a bias: per side); the bias groups
         // are widened to fp32 once per item
         auto body = [&](auto has_bias) {
-          constexpr bool HB = decltype(has_bias)::value;
+          constexpr bool HB = EPI != EPI_TAIL_GELU && decltype(has_bias)::value;
+          constexpr bool GELU = EPI == EPI_TAIL_GELU && decltype(has_bias)::value;
           u32x4 bq[HB ? NP : 1];  // 8 bf16 per group, widened where used
           if constexpr (HB) {
             const auto rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(bias + n0), 0,
@@ -520,6 +534,7 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
                     const float v = fmaxf(o[e], 0.f);
                     o[e] = v * v;
                   }
+                  if constexpr (GELU) o[e] = gelu(o[e]);
                   if constexpr (HB) {
                     const uint32_t w = bq[p][e >> 1];
                     o[e] += __uint_as_float((e & 1) ? (w & 0xffff0000u) : (w << 16));
@@ -534,14 +549,14 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
             __builtin_amdgcn_sched_barrier(0);
           }
         };
-        if (bias != nullptr)
+        if (EPI == EPI_TAIL_GELU ? tail : bias != nullptr)
           body(std::true_type{});
         else
           body(std::false_type{});
       }
       return;
     }
-    if constexpr (EPI != EPI_SILU_MUL) {  // (the 32x32 layout is fp8's: store / residual only)
+    if constexpr (!STACKED) {  // (the 32x32 layout is fp8's: store / residual only)
       // batches of JG m-blocks; the residual quads of the next batch are loaded before this
       // batch is computed (one HBM round trip per batch, overlapped, instead of one per quad)
       constexpr int JG = L32 ? 1 : 2;
@@ -1038,9 +1053,9 @@ int w4_sk_grid(int tiles, int nk_all) { return static_cast<int>(std::min<long lo
 template <int EPI, bool F8 = false>
 int launch_w4(const void* x, const void* w, const void* bias, const void* res, void* c, float* ws, int* cnt, int M,
               int N, int K, int inter, int split_k, hipStream_t stream, const float* xs = nullptr,
-              const float* wsc = nullptr) {
+              const float* wsc = nullptr, float limit = 0.f) {
   const int m_tiles = (M + BM - 1) / BM, n_tiles = (N + BN - 1) / BN;
-  const int ldc = EPI == EPI_SILU_MUL ? inter : N;
+  const int ldc = EPI == EPI_SILU_MUL || EPI == EPI_CLAMPED || EPI == EPI_TAIL_GELU ? inter : N;
   const int nwg = m_tiles * n_tiles * std::max(split_k, 1);
   // persistent: one workgroup per CU streams its items (split_k == 1), or its range of the
   // tiles x K-tiles units (split_k == 0, stream-K)
@@ -1049,7 +1064,7 @@ int launch_w4(const void* x, const void* w, const void* bias, const void* res, v
   hipLaunchKernelGGL((gemm_w4_kernel<EPI, F8>), dim3(grid), dim3(256),
                      0, stream, x, w, static_cast<const bf16_t*>(bias), static_cast<const bf16_t*>(res),
                      static_cast<bf16_t*>(c), ws, cnt, M, N, K, ldc, inter, m_tiles, n_tiles, split_k, xs, wsc,
-                     static_cast<const int*>(nullptr), static_cast<const int*>(nullptr), 0.f);
+                     static_cast<const int*>(nullptr), static_cast<const int*>(nullptr), limit);
   return BCG_CHECK_LAUNCH();
 }
 
@@ -1127,6 +1142,29 @@ BCG_API int bcg_gemm_w4_grouped(int epi, const void* x, const void* w, void* c, 
       if (N % 256) return -2;
       return launch_w4_grouped<EPI_GATED>(x, w, c, group, used, m_tiles, N, K, limit, stream);
     case EPI_RELU2: return launch_w4_grouped<EPI_RELU2>(x, w, c, group, used, m_tiles, N, K, 0.f, stream);
+    default: return -2;
+  }
+}
+
+// Projection and activation of a feed-forward in one launch, on all rows: bf16 without bias or split of K, and the operand
+// sizes of bcg_gemm_w4.
+// epi 5: c [M, inter] = the clamped gated unit (limit > 0) of w = [gate; up], N = 2 inter, inter % 128 == 0.
+// epi 6: c [M, inter] = the first `inter` columns of the product, tail [M, N - inter] = gelu (tanh form) of the others;
+//        inter % 256 == 0 (a tile is on one side), 0 < inter < N.
+// Bound by the matrix units like the plain product; the activation on the accumulators replaces a pass that read the product
+// and wrote the hidden values (2039 x 16384 x 2048 clamped: product 107 us and pass 24 -> 107; 8183 x 11264 x 2048, gelu on 8192
+// columns: 301 and 66 -> 316), and rounds once.  No split of K: these instances keep 200 registers and spill none.
+BCG_API int bcg_gemm_w4_act(int epi, const void* x, const void* w, void* c, void* tail, int M, int N, int K, int inter, float limit,
+                            hipStream_t stream) {
+  if (M <= 0 || N <= 0 || N % 16 || K % BK || K <= 0 || inter <= 0) return -2;
+  if (2ull * (M + BM) * K >= (1ull << 31) || 2ull * (N + BN) * K >= (1ull << 31) || 2ull * (M + BM) * N >= (1ull << 31)) return -2;
+  switch (epi) {
+    case EPI_CLAMPED:
+      if (N != 2 * inter || inter % 128 || !(limit > 0.f)) return -2;
+      return launch_w4<EPI_CLAMPED>(x, w, nullptr, nullptr, c, nullptr, nullptr, M, N, K, inter, 1, stream, nullptr, nullptr, limit);
+    case EPI_TAIL_GELU:
+      if (!tail || inter >= N || inter % BN) return -2;
+      return launch_w4<EPI_TAIL_GELU>(x, w, nullptr, tail, c, nullptr, nullptr, M, N, K, inter, 1, stream);
     default: return -2;
   }
 }
