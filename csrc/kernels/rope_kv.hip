@@ -178,17 +178,15 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kv_vec_kernel(
                               n_q, n_kv, num_blocks, block_size, eps, skip_v);
 }
 
-// Prefill V (T >= 64): one workgroup per (16 consecutive tokens, kv head), one thread per dim.
-// When the 16 tokens fill one KV block in order (the common case inside a prompt), thread d
-// gathers its 16 values and writes the block's V^T row d as 32 contiguous bytes -- the
-// per-token form writes 2 bytes at a 32-B stride per element (418 -> 286 us per layer at
-// 16k tokens was left mostly in those stores).  Other groups store element by element.
-//
-// The block is 2*HD threads and both sides move 16 B per lane: thread (i = tid / (HD/8),
-// c = tid % (HD/8)) loads dims 8c..8c+7 of token i (one 16-B load; the former one-thread-per-dim
-// form issued 16 two-byte loads per thread, 128 B per wave instruction, and ran at ~1.4 TB/s),
-// the 16 x HD tile is transposed through LDS, and thread (d = tid / 2, half) stores tokens
-// 8*half..8*half+7 of V^T row d as one 16-B store.
+// Prefill V (T >= 64): one workgroup per (16 consecutive tokens, kv head), 2 HD threads, 16 B per lane on both sides (two bytes a
+// lane and load: ~1.4 TB/s).  The tokens of a packed step fall into groups: consecutive slots of one run of 16 (a multiple of
+// 16 and the 15 behind it).  A workgroup writes the groups that BEGIN among its tokens, up to 15 tokens past them included,
+// so a group is written once and whole wherever the prompt's pages lie against the 16 tokens; a prompt's inside is one full
+// group per workgroup: its 16 x HD tile is transposed through LDS and thread (d = tid / 2, half) stores tokens 8 half .. + 7 of
+// V^T row d as one 16-B store.  Other groups (ends of prompts, single tokens): element by element out of the tile.
+// Bound by memory.  16182 tokens, 8 heads of 128, the query and key part (about 90 us) included, us: groups that do not begin at
+// the workgroup's first token, one thread per dim and token after token 147, element by element out of the tile 128, here
+// 114; pages that do begin there 111.  4534 tokens: 37, 29 (aligned 26).
 template <int HD>
 __global__ __launch_bounds__(2 * HD) void v_write_group_kernel(const bf16_t* __restrict__ qkv,
                                                                const int* __restrict__ slots,
@@ -196,38 +194,46 @@ __global__ __launch_bounds__(2 * HD) void v_write_group_kernel(const bf16_t* __r
                                                                int n_q, int n_kv, int num_blocks, int block_size) {
   constexpr int CPT = HD / 8;      // 16-B chunks per token row
   constexpr int LD = HD + 8;       // LDS row pitch (bf16): rows start 16 B apart in the bank map
-  __shared__ __attribute__((aligned(16))) uint16_t tile[16][LD];
+  __shared__ __attribute__((aligned(16))) uint16_t tile[32][LD];
+  __shared__ int slot_of[32], range[3];
   const int t0 = blockIdx.x * 16, h = blockIdx.y, tid = threadIdx.x;
-  const int nt = min(16, T - t0);
   const int n_heads = n_q + 2 * n_kv;
-  const int s0 = slots[t0];
-  const bool mine = tid >= nt || slots[t0 + tid] == s0 + tid;  // thread i < 16 checks token i
-  const bool fast = __syncthreads_and(mine) && nt == 16 && block_size == 16 && s0 % 16 == 0;
-  const bf16_t* head = qkv + static_cast<size_t>(t0) * n_heads * HD + static_cast<size_t>(n_q + n_kv + h) * HD;
-  if (fast) {
-    const int i = tid / CPT, c = tid % CPT;
-    const u16x8 x = *reinterpret_cast<const u16x8*>(head + static_cast<size_t>(i) * n_heads * HD + 8 * c);
-    *reinterpret_cast<u16x8*>(&tile[i][8 * c]) = x;
-    __syncthreads();
-    const int d = tid >> 1, half = tid & 1;
+  if (tid < 64) {
+    const int t = t0 + tid, s = tid < 32 && t < T ? slots[t] : 0;
+    const bool first = tid < 32 && t < T && (t == 0 || (s & 15) == 0 || s != slots[t - 1] + 1);
+    const uint32_t begins = static_cast<uint32_t>(__ballot(first));
+    if (tid < 32) slot_of[tid] = s;
+    if (tid == 0) {  // a group has at most 16 tokens: the last one ends before token 31, where another begins, or at T
+      range[0] = begins & 0xffff ? __builtin_ctz(begins) : 32;
+      range[2] = __builtin_popcount(begins & 0xffff);
+      range[1] = min(T - t0, begins >> 16 ? 16 + __builtin_ctz(begins >> 16) : 31);
+    }
+  }
+  __syncthreads();
+  const int i0 = range[0], n = range[1] - i0;   // the tokens written here, from t0 + i0 on
+  if (n <= 0) return;
+  const bf16_t* head = qkv + static_cast<size_t>(t0 + i0) * n_heads * HD + static_cast<size_t>(n_q + n_kv + h) * HD;
+  const int c = tid % CPT;
+  for (int i = tid / CPT; i < n; i += 16)
+    *reinterpret_cast<u16x8*>(&tile[i][8 * c]) = *reinterpret_cast<const u16x8*>(head + static_cast<size_t>(i) * n_heads * HD + 8 * c);
+  const int s0 = slot_of[i0];
+  const bool full = n == 16 && range[2] == 1 && block_size % 16 == 0;   // (one group of 16 tokens begins at a multiple of 16)
+  __syncthreads();
+  const int d = tid >> 1, half = tid & 1;
+  bf16_t* base = v_cache + (static_cast<size_t>(layer) * num_blocks * n_kv + h) * HD * block_size + static_cast<size_t>(d) * block_size;
+  const size_t blk_stride = static_cast<size_t>(n_kv) * HD * block_size;
+  if (full) {
     uint32_t w[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       w[j] = uint32_t(tile[8 * half + 2 * j][d]) | (uint32_t(tile[8 * half + 2 * j + 1][d]) << 16);
-    const int blk = s0 / 16;
-    uint4* dst = reinterpret_cast<uint4*>(v_cache + ((static_cast<size_t>(layer) * num_blocks + blk) * n_kv + h) * HD * 16 +
-                                          static_cast<size_t>(d) * 16 + 8 * half);
-    *dst = uint4{w[0], w[1], w[2], w[3]};
+    *reinterpret_cast<uint4*>(base + static_cast<size_t>(s0 / block_size) * blk_stride + s0 % block_size + 8 * half) =
+        uint4{w[0], w[1], w[2], w[3]};
     return;
   }
-  if (tid >= HD) return;  // element-wise path: one thread per dim
-  const int d = tid;
-  const bf16_t* src = head + d;
-  for (int i = 0; i < nt; ++i) {
-    const int slot = slots[t0 + i];
-    const int blk = slot / block_size, off = slot % block_size;
-    v_cache[((static_cast<size_t>(layer) * num_blocks + blk) * n_kv + h) * HD * block_size +
-            static_cast<size_t>(d) * block_size + off] = src[static_cast<size_t>(i) * n_heads * HD];
+  for (int i = half; i < n; i += 2) {
+    const int slot = slot_of[i0 + i], blk = slot / block_size;
+    base[static_cast<size_t>(blk) * blk_stride + (slot - blk * block_size)] = tile[i][d];
   }
 }
 
