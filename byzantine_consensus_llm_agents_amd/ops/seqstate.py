@@ -243,7 +243,7 @@ def seqstate_ops(lib):
             if B == 1:
                 return out
         _check(lib.bcg_gated_state_scan(_p(q), _p(k), _p(g), _p(v), v.stride(0), _p(beta), _p(meta.positions),
-                                        _p(meta.q_start), _p(meta.state_rows), _p(state), state.shape[0], _p(out), B, H, Gq, dim,
+                                        _p(meta.q_start), _p(meta.state_rows), _p(state), state.shape[0], _p(out), T, B, H, Gq, dim,
                                         vdim, gd, int(g_const), skip, int(bool(delta)), int(bool(unit_last)), _act(v), _stream()), "gated_state_scan")
         return out
 

@@ -868,6 +868,152 @@ __global__ __launch_bounds__(64 * SCAN_WAVES) void state_scan_kernel(ScanArgs a)
   }
 }
 
+// The same recurrence with DELTA and one decay per head, for segments of several tokens.
+//
+// The kernel above spends a token on waiting: two passes over the state, each with its own reads of the staged vectors and its own
+// lane sums, one behind the other (about 1300 cycles a token with one wave per SIMD; with four, the LDS serves 16 reads of 16 bytes
+// per lane, 2048 cycles).  Here both sums run over the state as the token finds it, S^T q afterwards being g (S^T q) + (k . q) u:
+// one pass and one round of sums, k kept in registers between them.  g, beta and k . q are numbers (the dots of a chunk's eight
+// tokens are taken together, one per column of lanes), and a workgroup stages everything that its tokens need, so whole chunks
+// run without a branch and the next token's reads overlap this one's sums.  Bound by the vector unit (about 95 instructions a
+// token).  32 heads of 128 x 128, bf16 values, us, the kernel above and this one: 8 segments of 700 to 1300 tokens 1138, 840;
+// one of 1000 699, 332; 16 of 100 201, 160; 24 of 20 73, 56; error against 64 bits 1.05e-7 and 1.04e-7 of the outputs, 7.7e-8 and 7.4e-8 of the
+// state.  (Two columns per lane, half the reads: 915 and 0.45 us a token against 0.35 with one wave per SIMD.)
+template <typename T, int DMAX>
+__global__ __launch_bounds__(64 * SCAN_WAVES, 2) void delta_scan_kernel(ScanArgs a) {
+  constexpr int RPL = DMAX / 8;                      // rows per lane
+  constexpr int GP = RPL + 4;                        // a row group's piece of a staged vector, padded
+  constexpr int VP = 8 * GP;                         // one staged vector
+  constexpr int NTH = 64 * SCAN_WAVES;
+  constexpr int CT = DMAX <= 128 ? 8 : 4;            // tokens staged at a time
+  constexpr int NC = 8 * SCAN_WAVES;                 // the workgroup's columns
+  constexpr int NL = CT * 2 * DMAX / NTH;            // staged elements of q and k per thread
+  constexpr int NV = (CT * NC + NTH - 1) / NTH;      // of v
+  static_assert(CT * 2 * DMAX % NTH == 0 && 2 * CT <= NTH, "staging");
+  __shared__ __attribute__((aligned(16))) float vec[2][CT][2 * VP];
+  __shared__ __attribute__((aligned(16))) float vals[2][CT][NC];
+  __shared__ float gb[2][CT][2];
+  const int tid = threadIdx.x, lane = tid & 63, rg = lane & 7;
+  const int b = blockIdx.x, h = blockIdx.y, j0 = blockIdx.z * NC, jl = (tid >> 6) * 8 + (lane >> 3), j = j0 + jl;
+  const int t0 = a.q_start[b], t1 = a.q_start[b + 1];
+  const int sr = a.state_rows[b];
+  if (t1 <= t0 || sr < 0 || sr >= a.n_rows || (a.skip_len > 0 && t1 - t0 >= a.skip_len)) return;
+  const int gq = h / (a.H / a.Gq);
+  const int dim = a.dim, vdim = a.vdim;
+  float* Sp = a.state + (static_cast<size_t>(sr) * a.H + h) * dim * vdim;
+  // every load is unconditional, its address clamped into the tensor, and what lies outside is replaced afterwards
+  float S[RPL];
+  if (a.positions[t0] != 0) {
+#pragma unroll
+    for (int i = 0; i < RPL; ++i) {
+      const int row = min(rg * RPL + i, dim - 1);
+      S[i] = Sp[static_cast<size_t>(row) * vdim + min(j, vdim - 1)];
+    }
+#pragma unroll
+    for (int i = 0; i < RPL; ++i)
+      if (rg * RPL + i >= dim || j >= vdim) S[i] = 0.f;
+  } else {
+#pragma unroll
+    for (int i = 0; i < RPL; ++i) S[i] = 0.f;
+  }
+  struct Chunk { float r[NL], v[NV], s; };
+  const T* vbase = static_cast<const T*>(a.v) + h * vdim;
+  // (tokens past the end read as the last one: a branch around a load makes it wait for the one before, 1.4 times the time)
+  auto load = [&](int first, Chunk& ch) {
+#pragma unroll
+    for (int n = 0; n < NL; ++n) {   // element: token, q or k, row
+      const int e = tid + NTH * n, tt = e / (2 * DMAX), which = e / DMAX % 2, i = e % DMAX;
+      const size_t row = (static_cast<size_t>(min(first + tt, t1 - 1)) * a.Gq + gq) * dim;
+      ch.r[n] = (which == 0 ? a.q : a.k)[row + min(i, dim - 1)];
+    }
+#pragma unroll
+    for (int n = 0; n < NV; ++n) {
+      const int e = min(tid + NTH * n, CT * NC - 1), tt = e / NC, c = e % NC;
+      ch.v[n] = Elem<T>::ld(vbase[static_cast<size_t>(min(first + tt, t1 - 1)) * a.v_stride + min(j0 + c, vdim - 1)]);
+    }
+    const int t = min(first + (tid >> 1) % CT, t1 - 1);
+    ch.s = tid & 1 ? a.beta[static_cast<size_t>(t) * a.H + h] : a.g[static_cast<size_t>(t) * a.g_token + h];
+  };
+  auto stage = [&](int buf, const Chunk& ch) {
+#pragma unroll
+    for (int n = 0; n < NL; ++n) {
+      const int e = tid + NTH * n, tt = e / (2 * DMAX), which = e / DMAX % 2, i = e % DMAX;
+      vec[buf][tt][which * VP + (i / RPL) * GP + (i % RPL)] = i < dim ? ch.r[n] : 0.f;
+    }
+#pragma unroll
+    for (int n = 0; n < NV; ++n) {
+      const int e = tid + NTH * n;
+      if (CT * NC % NTH == 0 || e < CT * NC) (&vals[buf][0][0])[e] = ch.v[n];
+    }
+    if (tid < 2 * CT) gb[buf][tid >> 1][tid & 1] = ch.s;
+  };
+  Chunk nxt;
+  load(t0, nxt);
+  stage(0, nxt);
+  __syncthreads();
+  float keep = 0.f;   // the lane of row group r keeps the chunk's token r
+  int buf = 0;
+  // k . q of the chunk's tokens, token c in the lanes of column c
+  auto dots = [&] {
+    const float* p = &vec[buf][(lane >> 3) % CT][rg * GP];
+    float s4[4] = {};
+#pragma unroll
+    for (int m = 0; m < RPL / 4; ++m) {
+      const f32x4 q4 = *reinterpret_cast<const f32x4*>(p + 4 * m), k4 = *reinterpret_cast<const f32x4*>(p + VP + 4 * m);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s4[i] += q4[i] * k4[i];
+    }
+    return group8_sum((s4[0] + s4[1]) + (s4[2] + s4[3]));
+  };
+  float kqs = 0.f;
+  auto token = [&](int tt) {
+    const f32x4* qv = reinterpret_cast<const f32x4*>(&vec[buf][tt][rg * GP]);
+    const f32x4* kv = reinterpret_cast<const f32x4*>(&vec[buf][tt][VP + rg * GP]);
+    const float g = gb[buf][tt][0], beta = gb[buf][tt][1];
+    const float kq = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(kqs), 8 * tt));
+    f32x4 k4[RPL / 4];
+    float d[4] = {}, o[4] = {};
+#pragma unroll
+    for (int m = 0; m < RPL / 4; ++m) {
+      k4[m] = kv[m];
+      const f32x4 q4 = qv[m];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        d[i] += S[4 * m + i] * k4[m][i];
+        o[i] += S[4 * m + i] * q4[i];
+      }
+    }
+    const float u = beta * (vals[buf][tt][jl] - g * group8_sum((d[0] + d[1]) + (d[2] + d[3])));
+#pragma unroll
+    for (int m = 0; m < RPL / 4; ++m)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) S[4 * m + i] = S[4 * m + i] * g + k4[m][i] * u;
+    const float os = g * group8_sum((o[0] + o[1]) + (o[2] + o[3])) + kq * u;
+    keep = rg == tt ? os : keep;
+  };
+  for (int first = t0; first < t1; first += CT, buf ^= 1) {
+    const bool more = first + CT < t1;
+    if (more) load(first + CT, nxt);
+    kqs = dots();
+    if (first + CT <= t1) {
+#pragma unroll
+      for (int tt = 0; tt < CT; ++tt) token(tt);
+    } else {
+      for (int tt = 0; first + tt < t1; ++tt) token(tt);
+    }
+    if (more) stage(buf ^ 1, nxt);   // (the other buffer: its readers finished before the last barrier)
+    // one store per chunk, after the wait for the next chunk's loads: a store in flight never stands between a load and its use
+    if (rg < CT && first + rg < t1) {
+      float* p = a.out + (static_cast<size_t>(first + rg) * a.H + h) * vdim + j;
+      if (j < vdim) p[0] = keep;
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < RPL; ++i)
+    if (rg * RPL + i < dim && j < vdim) Sp[static_cast<size_t>(rg * RPL + i) * vdim + j] = S[i];
+}
+
 // o fp32 [T, H, vdim] -> out [T, H vdim]: every head over its root mean square, times w [vdim]
 // (w_head = 0) or w [H vdim] (w_head = vdim) (null: no weight), times sigmoid(gate[t, h vdim + e]) (gate_kind 0) or silu
 // of it (1) (gate null: none).  With `floor_` [T, H] a head of o has vdim + 1 columns and is first
@@ -968,8 +1114,19 @@ bool launch_head_norm_vec(const float* o, const float* w, float eps, const T* ga
 }
 
 template <typename T, bool DELTA>
-int launch_scan(const ScanArgs& a, int B, hipStream_t s) {
+int launch_scan(const ScanArgs& a, int tokens, int B, hipStream_t s) {
   dim3 grid(B, a.H, (a.vdim + 8 * SCAN_WAVES - 1) / (8 * SCAN_WAVES));
+  // four tokens and more per segment: below, staging a chunk of eight costs more than the tokens gain (64 segments of one token
+  // 60 us, 66 that way)
+  if constexpr (DELTA) {
+    if (a.gd == 1 && tokens / 4 >= B) {
+      if (a.dim <= 32) delta_scan_kernel<T, 32><<<grid, 64 * SCAN_WAVES, 0, s>>>(a);
+      else if (a.dim <= 64) delta_scan_kernel<T, 64><<<grid, 64 * SCAN_WAVES, 0, s>>>(a);
+      else if (a.dim <= 128) delta_scan_kernel<T, 128><<<grid, 64 * SCAN_WAVES, 0, s>>>(a);
+      else delta_scan_kernel<T, 256><<<grid, 64 * SCAN_WAVES, 0, s>>>(a);
+      return BCG_CHECK_LAUNCH();
+    }
+  }
   if (a.dim <= 32) state_scan_kernel<T, 32, DELTA><<<grid, 64 * SCAN_WAVES, 0, s>>>(a);
   else if (a.dim <= 64) state_scan_kernel<T, 64, DELTA><<<grid, 64 * SCAN_WAVES, 0, s>>>(a);
   else if (a.dim <= 128) state_scan_kernel<T, 128, DELTA><<<grid, 64 * SCAN_WAVES, 0, s>>>(a);
@@ -1161,7 +1318,7 @@ BCG_API int bcg_delta_prepare(const void* c, int64_t c_stride, const void* y, in
 
 BCG_API int bcg_gated_state_scan(const void* q32, const void* k32, const void* g32, const void* v, int64_t v_stride,
                                  const void* beta, const void* positions, const void* q_start, const void* state_rows,
-                                 void* state, int n_rows, void* out, int B, int H, int Gq, int dim, int vdim, int gd, int g_const, int skip_len, int delta,
+                                 void* state, int n_rows, void* out, int T_, int B, int H, int Gq, int dim, int vdim, int gd, int g_const, int skip_len, int delta,
                                  int unit_last, int is_f32, void* stream) {
   if (B <= 0) return 0;
   if (dim < 1 || dim > 256 || H <= 0 || Gq <= 0 || H % Gq || H > 65535 || (delta && beta == nullptr) || (gd != 1 && gd != dim)) return -2;
@@ -1175,8 +1332,8 @@ BCG_API int bcg_gated_state_scan(const void* q32, const void* k32, const void* g
   a.n_rows = n_rows; a.H = H; a.Gq = Gq; a.dim = dim; a.vdim = vdim; a.gd = gd; a.g_token = g_const ? 0 : H * gd;
   a.skip_len = skip_len;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (delta) return is_f32 ? launch_scan<float, true>(a, B, s) : launch_scan<bf16_t, true>(a, B, s);
-  return is_f32 ? launch_scan<float, false>(a, B, s) : launch_scan<bf16_t, false>(a, B, s);
+  if (delta) return is_f32 ? launch_scan<float, true>(a, T_, B, s) : launch_scan<bf16_t, true>(a, T_, B, s);
+  return is_f32 ? launch_scan<float, false>(a, T_, B, s) : launch_scan<bf16_t, false>(a, T_, B, s);
 }
 
 BCG_API int bcg_head_norm_gate(const void* o32, const void* w, float eps, const void* gate, int64_t gate_stride, void* out,
