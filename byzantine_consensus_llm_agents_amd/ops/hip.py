@@ -813,7 +813,8 @@ def hip_ops() -> SimpleNamespace:
         M, K = xq.shape
         N = wq.shape[0]
         return (plan.mode == "1" and 1 <= M <= 32 and K % 128 == 0 and 128 <= K <= SKINNY_ROW_BYTES and N >= 16 and N % 16 == 0
-                and _few_rows_pay(M, N, K, 0) and xq.is_cuda and xq.get_device() == torch.cuda.current_device() and xq.is_contiguous() and wq.is_contiguous()
+                and wq.dim() == 2 and wq.shape[1] == K and _few_rows_pay(M, N, K, 0)
+                and xq.is_cuda and xq.get_device() == torch.cuda.current_device() and xq.is_contiguous() and wq.is_contiguous()
                 and all(t.device == xq.device and t.data_ptr() % 16 == 0 and bare(t) for t in (xq, wq, xs, ws))
                 and xs.dtype == ws.dtype == torch.float32 and xs.numel() == M and ws.numel() == N and xs.is_contiguous()
                 and ws.is_contiguous() and not watched()

@@ -93,3 +93,17 @@ def test_norm_weight_infinities(ops):
     nw = torch.ones(1088, device="cuda", dtype=torch.bfloat16)
     nw[-1] = float("inf")
     assert (ops.norm_linear(x, nw, 1e-6, w) == float("inf")).all()
+
+
+@pytest.mark.parametrize("M,K,N,KW", [(4, 256, 64, 512), (20, 512, 128, 1024), (32, 128, 4096, 256)])
+def test_fp8_operands_of_other_rows_are_refused(ops, M, K, N, KW):
+    """Rows of W that are longer than those of x: an error before any launch, on both entry points."""
+    f8 = torch.float8_e4m3fn
+    xq, wq = torch.zeros(M, K, device="cuda").to(f8), torch.zeros(N, KW, device="cuda").to(f8)
+    xs, ws = torch.ones(M, 1, device="cuda"), torch.ones(N, device="cuda")
+    res = torch.ones(M, N, device="cuda", dtype=torch.bfloat16)
+    with pytest.raises(ValueError):
+        ops.linear_fp8_residual(xq, xs, wq, ws, res)
+    with pytest.raises(ValueError):
+        ops.linear_fp8(xq, xs, wq, ws)
+    assert (res == 1).all()
