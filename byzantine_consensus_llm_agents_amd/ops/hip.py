@@ -341,12 +341,13 @@ def hip_ops() -> SimpleNamespace:
     def decode_attention(qkv, positions, slots, n_q, n_kv, hd, q_norm, k_norm, eps, cos_sin, k_cache, v_cache, layer,
                          block_tables, seq_lens, scale, workspace=None):
         """paged_attention_decode(qk_norm_rope_kv_write(...)) for one new token per row of a bf16 cache with heads of 64, without the
-        rotary launch (csrc/kernels/attention.hip, FusedArgs, says why not for others)."""
+        rotary launch (csrc/kernels/attention.hip, FusedArgs, says why not for others).  Rows are different sequences: no row sees
+        what another one stores in this call."""
         B = qkv.shape[0]
         L, NB, nkv_c, BS, hdc = k_cache.shape
         _req(qkv.dtype == torch.bfloat16 and qkv.is_contiguous() and qkv.shape[1] == (n_q + 2 * n_kv) * hd, "decode qkv")
         _req(nkv_c == n_kv and hdc == hd and hd == 64 and BS == 16 and v_cache.shape == (L, NB, n_kv, hd, BS)
-             and k_cache.dtype == v_cache.dtype == torch.bfloat16, "decode kv cache layout")
+             and not _kv_fp8(k_cache, v_cache), "decode kv cache layout")
         _req(all(t.dtype == torch.int32 and t.is_contiguous() for t in (positions, slots, seq_lens, block_tables))
              and positions.numel() == slots.numel() == seq_lens.numel() == B and block_tables.shape[0] == B, "decode tables")
         _req(cos_sin.dtype == torch.float32 and cos_sin.shape[1] == hd and B <= 2048, "decode cos_sin / rows")

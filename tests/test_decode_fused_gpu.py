@@ -85,3 +85,15 @@ def test_parked_rows_and_graph_replays(ops):
         g.replay()
         torch.cuda.synchronize()
         assert ((out.double() - want.double()).norm() / want.double().norm()).item() < 2 ** -7
+
+
+def test_strided_caches_are_refused(ops):
+    """Caches that are views of larger ones: an error before any launch, as from the separate operations."""
+    c, k, v, table, sl = _case([5, 40], 4, 2, 64, False, seed=1)
+    f8 = torch.float8_e4m3fn
+    for bad in ((k.repeat(2, 1, 1, 1, 1)[::2], v), (k, v.repeat(2, 1, 1, 1, 1)[::2]), (k.to(f8), v.to(f8))):
+        before = [t.float().nan_to_num() for t in bad]
+        for call in (_separate, _fused)[bad[0].dtype == f8:]:   # (fp8 caches are the separate operations' alone)
+            with pytest.raises(ValueError):
+                call(ops, c, *bad, table, sl)
+        assert all(torch.equal(t.float().nan_to_num(), b) for t, b in zip(bad, before))
