@@ -9,6 +9,7 @@ synchronise with the host.  Semantics: the functions of the same names in ``refe
 
 import torch
 
+from .operands import bare, watched
 from .seqmix import ACT_CODES, _act, _check, _p, _req, _stream
 from .seqstate import _f32, _i32
 
@@ -218,13 +219,16 @@ def seqlatent_ops(lib):
         _req(tokens.dtype == torch.int32 and tokens.dim() == 1 and table.dtype == torch.int32 and table.dim() == 2
              and tokens.device == table.device and 1 <= top <= table.shape[1], "moe_table_route: tokens int32 [T], table int32 [vocab, >= top]")
         T = tokens.numel()
-        if T * top >= 1 << 24:
+        # the launch takes plain tensors of the current device, rows of the table as they lie; host tensors, other devices, transforms
+        # and traces keep the gather
+        if not (T * top < 1 << 24 and table.is_cuda and table.get_device() == torch.cuda.current_device() and table.stride(1) == 1
+                and top <= table.stride(0) < 1 << 31 and not watched() and bare(tokens) and bare(table)):
             idx = table.index_select(0, tokens)[:, :top].contiguous()
             return idx, torch.full(idx.shape, 1.0 / top, dtype=torch.float32, device=idx.device)
-        tokens, table = tokens.contiguous(), table.contiguous()
+        tokens = tokens.contiguous()
         idx = torch.empty(T, top, dtype=torch.int32, device=table.device)
         wts = torch.empty(T, top, dtype=torch.float32, device=table.device)
-        _check(lib.bcg_moe_route_table(_p(tokens), _p(table), table.shape[0], table.shape[1], top, T, _p(idx), _p(wts), _stream()),
+        _check(lib.bcg_moe_route_table(_p(tokens), _p(table), table.shape[0], table.stride(0), top, T, _p(idx), _p(wts), _stream()),
                "moe_route_table")
         return idx, wts
 

@@ -523,7 +523,7 @@ BCG_API int bcg_moe_route(const void* h, const void* rw, const void* rb, const v
   return BCG_CHECK_LAUNCH();
 }
 
-// idx, wts: [T, top] from table [vocab, width], width >= top.
+// idx, wts: [T, top] from the first `top` columns of table's vocab rows, which begin `width` >= top entries apart.
 BCG_API int bcg_moe_route_table(const void* tokens, const void* table, int vocab, int width, int top, int T_, void* idx, void* wts,
                                 void* stream) {
   if (T_ <= 0) return 0;
