@@ -319,7 +319,7 @@ def seqmix_ops(lib, linear):
             y = a   # the down product's rows replace the gathered ones
             _check(lib.bcg_gemm_w4_grouped(0, _p(hidden), _p(down), _p(y), _p(tile_e), _p(used), n_tiles, W, ff, 0.0, _stream()),
                    "moe down")
-            _check(lib.bcg_moe_combine(_p(y), _p(weights), _p(pos), _p(out), T, W, top, f32, _stream()), "moe_combine")
+            _check(lib.bcg_moe_combine(_p(y), _p(weights), _p(pos), _p(idx), E, _p(out), T, W, top, f32, _stream()), "moe_combine")
             return out
         _check(lib.bcg_moe_align(_p(idx), n_slots, E, _p(sorted_), cap, _p(tile_e), n_tiles, rows, None, None, _stream()),
                "moe_align")
@@ -332,7 +332,7 @@ def seqmix_ops(lib, linear):
             y = torch.empty(n_slots, W, dtype=h.dtype, device=dev)
             _check(lib.bcg_moe_rows(_p(hidden), cap, ff, _p(down), _p(y), W, _p(sorted_), _p(tile_e), n_tiles, held, W, ff, top, 0, 1,
                                     0, 0.0, _stream()), "moe down rows")
-            _check(lib.bcg_moe_combine(_p(y), _p(weights), None, _p(out), T, W, top, f32, _stream()), "moe_combine")
+            _check(lib.bcg_moe_combine(_p(y), _p(weights), None, _p(idx), E, _p(out), T, W, top, f32, _stream()), "moe_combine")
             return out
         code = ACT_CODES[EXPERT_ACTS[kind]] if gated else 1
         if gated and ff % 16 == 0:   # rows paired by `moe_pair_rows`: the hidden values in the product's epilogue
@@ -352,7 +352,7 @@ def seqmix_ops(lib, linear):
         y = torch.empty(n_slots, W, dtype=h.dtype, device=dev)
         _check(lib.bcg_moe_gemm(_p(hidden), ff, _p(down), _p(y), W, _p(sorted_), _p(tile_e), n_tiles, W, ff, top, 0, 1, 0,
                                 0.0, f32, _stream()), "moe down")
-        _check(lib.bcg_moe_combine(_p(y), _p(weights), None, _p(out), T, W, top, f32, _stream()), "moe_combine")
+        _check(lib.bcg_moe_combine(_p(y), _p(weights), None, _p(idx), E, _p(out), T, W, top, f32, _stream()), "moe_combine")
         return out
 
     return dict(embed_scale_rmsnorm=embed_scale_rmsnorm, embed_position=embed_position, residual_add_rmsnorm32=residual_add_rmsnorm32,

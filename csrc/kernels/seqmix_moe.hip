@@ -466,7 +466,8 @@ __global__ __launch_bounds__(256) void moe_gemm_lds_narrow_kernel(const T* __res
 // order (an unplaced slot adds nothing).  VEC columns per thread: 16-byte loads of the rows, bound by memory.
 template <typename T, int VEC>
 __global__ __launch_bounds__(256) void combine_kernel(const T* __restrict__ y, const float* __restrict__ wts,
-                                                      const int* __restrict__ pos, float* __restrict__ out, int W, int top) {
+                                                      const int* __restrict__ pos, const int* __restrict__ idx, int E,
+                                                      float* __restrict__ out, int W, int top) {
   typedef T Row __attribute__((ext_vector_type(VEC)));
   typedef float Sum __attribute__((ext_vector_type(VEC)));
   const int t = blockIdx.x;
@@ -475,9 +476,11 @@ __global__ __launch_bounds__(256) void combine_kernel(const T* __restrict__ y, c
 #pragma unroll
     for (int q = 0; q < VEC; ++q) s[q] = 0.f;
     for (int j = 0; j < top; ++j) {
-      const int64_t row = pos != nullptr ? pos[t * top + j] : static_cast<int64_t>(t) * top + j;
-      if (row < 0) continue;
-      const float w = wts[t * top + j];
+      const int64_t slot = static_cast<int64_t>(t) * top + j;
+      const int who = idx[slot];
+      if (who < 0 || who >= E) continue;   // no expert: no product wrote a row for this slot
+      const int64_t row = pos != nullptr ? pos[slot] : slot;
+      const float w = wts[slot];
       const Row v = *reinterpret_cast<const Row*>(y + row * W + c);
 #pragma unroll
       for (int q = 0; q < VEC; ++q) s[q] += w * Elem<T>::ld(v[q]);
@@ -602,14 +605,16 @@ BCG_API int bcg_moe_gemm(const void* a, int64_t a_stride, const void* w, void* o
   return BCG_CHECK_LAUNCH();
 }
 
-BCG_API int bcg_moe_combine(const void* y, const void* wts, const void* pos, void* out, int T_, int W, int top, int is_f32,
-                            void* stream) {
+// out[t] = sum over j of wts[t, j] * the row of y of slot (t, j): y[pos[t, j]], or y[t top + j] without pos.  Slots whose expert (idx) is
+// none of 0 .. E - 1 add nothing.
+BCG_API int bcg_moe_combine(const void* y, const void* wts, const void* pos, const void* idx, int E, void* out, int T_, int W, int top,
+                            int is_f32, void* stream) {
   if (T_ <= 0) return 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const bool vec = (reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(out)) % 16 == 0;
 #define BCG_COMBINE(TYPE, VEC_)                                                                                          \
   combine_kernel<TYPE, VEC_><<<T_, 256, 0, s>>>(static_cast<const TYPE*>(y), static_cast<const float*>(wts), \
-                                                static_cast<const int*>(pos), static_cast<float*>(out), W, top)
+                                                static_cast<const int*>(pos), static_cast<const int*>(idx), E, static_cast<float*>(out), W, top)
   if (is_f32) {
     if (vec && W % 4 == 0) BCG_COMBINE(float, 4); else BCG_COMBINE(float, 1);
   } else {
