@@ -1157,7 +1157,8 @@ BCG_API int bcg_gemm_w4_grouped(int epi, const void* x, const void* w, void* c, 
 BCG_API int bcg_gemm_w4_act(int epi, const void* x, const void* w, void* c, void* tail, int M, int N, int K, int inter, float limit,
                             hipStream_t stream) {
   if (M <= 0 || N <= 0 || N % 16 || K % BK || K <= 0 || inter <= 0) return -2;
-  if (2ull * (M + BM) * K >= (1ull << 31) || 2ull * (N + BN) * K >= (1ull << 31) || 2ull * (M + BM) * N >= (1ull << 31)) return -2;
+  const unsigned long long widest = epi == EPI_CLAMPED ? inter : N;   // columns of the widest output
+  if (2ull * (M + BM) * K >= (1ull << 31) || 2ull * (N + BN) * K >= (1ull << 31) || 2ull * (M + BM) * widest >= (1ull << 31)) return -2;
   switch (epi) {
     case EPI_CLAMPED:
       if (N != 2 * inter || inter % 128 || !(limit > 0.f)) return -2;

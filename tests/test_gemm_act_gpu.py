@@ -54,6 +54,21 @@ def test_tail(ops, monkeypatch, M, at, N, K):
     _close(hidden, torch.nn.functional.gelu(tail, approximate="tanh"), 1.13 * dz[:, at:] + 2.0 ** -20 * tail.abs())
 
 
+def test_clamped_wide_output(ops):
+    """Twice the output's columns are past 32-bit offsets, the output is not: 16384 x 32768 of 64."""
+    M, inter, K, limit = 16384, 32768, 64, 4.0
+    assert ops.gemm_plan.clamped_tiles(M, 2 * inter, K)
+    x = torch.randn(M, K, device=DEV, generator=torch.Generator(DEV).manual_seed(1)).to(torch.bfloat16)
+    w = (torch.randn(2 * inter, K, device=DEV, generator=torch.Generator(DEV).manual_seed(2)) * 3 / K ** 0.5).to(torch.bfloat16)
+    out = ops.linear_clamped_glu(x, w, limit)
+    rows = torch.tensor([0, 255, 256, 8191, 16383], device=DEV)
+    z = x[rows].double() @ w.double().t()
+    dz = K * 2.0 ** -24 * (x[rows].double().abs() @ w.double().abs().t())
+    g, u = z[:, :inter].clamp(max=limit), z[:, inter:].clamp(-limit, limit)
+    slack = 1.1 * (limit + 1) * dz[:, :inter] + limit * dz[:, inter:] + 2.0 ** -20 * (limit + 1) * g.abs()
+    _close(out[rows], (g * torch.sigmoid(1.702 * g) * (u + 1)).cpu(), slack.cpu())
+
+
 def test_extremes(ops, monkeypatch):
     """Infinities and values whose exponentials overflow come out as in the passes of their own."""
     for name in ("clamped_tiles", "tail_tiles"):

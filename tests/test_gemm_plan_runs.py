@@ -4,6 +4,7 @@ shapes that the general path takes alone still do."""
 import random
 
 import pytest
+import torch
 
 from byzantine_consensus_llm_agents_amd.ops.gemm_plan import CUS, LARGE_M, SMALL_CFG, W4_CFG, GemmPlan
 
@@ -89,3 +90,24 @@ def test_gated_columns_of_a_weight_past_32_bits():
     one = ctypes.c_void_p(16)
     for inter, K in ((1 << 20, 1024), (1 << 19, 2048), ((1 << 20) - 128, 1024), (-128, 64)):     # 2 (2 inter + 256) K bytes: 2^31 and more
         assert load_library().bcg_gemm_nt(W4_CFG, 1, one, one, None, None, one, None, None, 256, 256, K, inter, 1, None) == -2
+
+
+@pytest.mark.skipif(torch.cuda.device_count() > 0, reason="calls the entry points with addresses of nothing: the launch has to fail")
+def test_activation_rules_take_what_their_kernel_takes():
+    """The rules of the activations in the 256 x 256 kernel's epilogue and the bounds of its entry point at 32-bit offsets: a size
+    that a rule takes is never refused (-2) there, one past the bounds never taken."""
+    import ctypes
+    import os
+    from byzantine_consensus_llm_agents_amd.ops.hip import load_library
+    from byzantine_consensus_llm_agents_amd.utils.build import kernels_target
+    if not os.path.exists(kernels_target()):
+        pytest.skip("kernel library not built")
+    lib, plan, one = load_library(), GemmPlan(), ctypes.c_void_p(16)
+    taken = refused = 0
+    for M in (512, 4096, 16384, 21589, 43700, 65536, 87126, 87125, 131072 - 256):
+        for ff, K in ((8192, 2048), (12288, 2048), (12288, 4096), (32768, 4096), (65536, 1024), (131072, 2048), (524160, 1024)):
+            for N, epi, at, rule in ((2 * ff, 5, ff, plan.clamped_tiles(M, 2 * ff, K)), (ff + 768, 6, 768, plan.tail_tiles(M, ff + 768, K, 768))):
+                got = lib.bcg_gemm_w4_act(epi, one, one, one, one, M, N, K, at, 1.0, None)
+                assert not (rule and got == -2), (M, N, K, epi)
+                taken, refused = taken + rule, refused + (got == -2)
+    assert plan.clamped_tiles(16384, 65536, 4096) and taken > 20 and refused > 20
