@@ -298,6 +298,8 @@ def seqmix_ops(lib, linear):
              and weights.shape == (T, top) and weights.is_contiguous(), "routing tables [T, top]")
         n_slots = T * top
         dev, f32 = h.device, _act(h)
+        if n_slots == 0:
+            return torch.zeros(T, W, dtype=torch.float32, device=dev)
         wide = _wide_experts(n_slots, E, W, ff, kind, h, up, down)
         few = not wide and _few_row_experts(n_slots, E, W, ff, gated, h, up, down)
         rows = WIDE_ROWS if wide else few_rows if few else tile_rows

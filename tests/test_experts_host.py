@@ -1,5 +1,5 @@
-"""Routing by token id (ops.moe_table_route of the HIP backend) on operands that its kernel does not take: host tensors, wrapped
-tensors and traces get the table's entries from a gather, as from the reference.  No GPU."""
+"""Expert layers of the HIP backend where no kernel runs: routing by token id of host tensors, wrapped tensors and traces is a gather, as
+in the reference; a step without tokens or without chosen experts is zeros.  No GPU."""
 import os
 
 import pytest
@@ -33,3 +33,12 @@ def test_batched_by_a_transform(ops):
     table = torch.arange(60, dtype=torch.int32).view(20, 3)
     tokens = torch.tensor([[0, 19, 3], [7, 7, 1]], dtype=torch.int32)
     assert torch.equal(torch.func.vmap(lambda t: ops.moe_table_route(t, table, 2)[0])(tokens), table[tokens.long(), :2])
+
+
+@pytest.mark.parametrize("T,top", [(0, 2), (3, 0)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_no_slots(ops, T, top, dtype):
+    h, up, down = torch.ones(T, 64, dtype=dtype), torch.ones(4, 128, 64, dtype=dtype), torch.ones(4, 64, 64, dtype=dtype)
+    idx, w = torch.zeros(T, top, dtype=torch.int32), torch.zeros(T, top)
+    out = ops.moe_experts(h, up, down, idx, w, "silu_gated")
+    assert torch.equal(out, reference.moe_experts(h, up, down, idx, w, "silu_gated")) and out.shape == (T, 64) and out.dtype == torch.float32
