@@ -8,6 +8,8 @@ allocator).  Semantics: the functions of the same names in ``reference.py``.
 """
 
 import ctypes
+import functools
+import math
 
 import torch
 
@@ -40,10 +42,42 @@ def _act(t):
 ACT_CODES = {"gelu_tanh": 0, "relu2": 1, "silu": 2, "clamped_glu": 3}
 EXPERT_ACTS = {"silu_gated": "silu", "clamped_glu": "clamped_glu"}   # gated experts -> activation of their hidden values
 
+CUS = 256          # compute units of the GPU
 WIDE_ROWS = 256    # rows of a position tile of the 256 x 256 expert products
 WIDE_SLOTS = 64    # ... taken from this many routed rows per expert on (see `_wide_experts`)
 
-FEW_SLOTS = 24     # position tiles of 32 rows up to this many routed rows per expert (see `_few_row_experts`)
+FEW_SLOTS, FEW_WEIGHT = 24, 1 << 18    # position tiles of 32 rows: most routed rows per expert, least weights of a matrix (see `few_row_tiles`)
+
+
+@functools.lru_cache(maxsize=1024)
+def _likely_tiles(n_slots, E, rows):
+    """How many tiles of `rows` rows hold n_slots slots that go to E experts at random (an expert has c slots, Poisson): the experts with
+    a slot, two standard deviations more than their mean, and the mean of their further tiles."""
+    mean, p, below, more = n_slots / E, math.exp(-n_slots / E), 0.0, 0.0
+    some = E * (1.0 - p)
+    for c in range(4 * rows + 1):
+        below, p = below + p, p * mean / (c + 1)
+        if c and c % rows == 0:
+            more += E * max(0.0, 1.0 - below)     # experts of more than c slots
+    return max(1, round(min(E, n_slots, some + 2 * math.sqrt(some * (1.0 - some / E))) + more))
+
+
+def few_row_tiles(n_slots, E, W, ff, rows):
+    """The tiles that are likely to hold rows if an expert layer's products stream the weights past position tiles of 32 rows (csrc/kernels/
+    moe_rows.hip), 0 if they do not: up to FEW_SLOTS routed rows per expert, where few experts have a second tile that streams their
+    weight again.  All four launches, tiles of 64 rows -> of 32, us: 8 gated experts of 2048 x 2048, top 2: 4 rows per expert 95 -> 51,
+    16: 95 -> 60, 25: 95 -> 61, 32: 91 -> 75, 40: 97 -> 121; 4096 x 3072: 16: 187 -> 124, 32: 189 -> 180.
+    Ratios of the times over 2 to 256 experts, widths 512 to 4096, hidden widths 256 to 3072, 1 to 768 tokens, top 2 and 8:
+    * up to 40 tiles 0.24 to 1.03, but up to 1.07 with experts of 512 x 256: most waves have no part of K there;
+    * more tiles get a few workgroups each: 0.61 to 1.04 where these fill the 256 CUs to 0.85 and the experts are
+      1024 wide and have 2^20 weights a matrix and more; less filled 0.95 to 1.31 (128 experts, 128 slots: 92 tiles, 2 workgroups
+      each), smaller experts 0.86 to 1.4 (256 of 1024 x 256)."""
+    if n_slots > FEW_SLOTS * E or W % 64 or ff % 64 or max(W, ff) > 32768 or W * ff < FEW_WEIGHT:
+        return 0
+    held = _likely_tiles(n_slots, E, rows)
+    if held > 40 and (W < 1024 or ff < 512 or W * ff < 1 << 20 or held * (CUS // held) < 0.85 * CUS):
+        return 0
+    return held
 
 
 def seqmix_ops(lib, linear):
@@ -275,14 +309,6 @@ def seqmix_ops(lib, linear):
         return (2 * rows * max(W, n_up) < 1 << 31 and 2 * (max(W, n_up) + 256) * max(W, ff) < 1 << 31
                 and all(t.data_ptr() % 16 == 0 for t in (h, up, down)))
 
-    def _few_row_experts(n_slots, E, W, ff, gated, h, up, down):
-        """Whether the products stream the weights past position tiles of 32 rows (csrc/kernels/moe_rows.hip): up to FEW_SLOTS routed
-        rows per expert, where few experts have a second tile that streams their weight again.  Align, two products and combine, tiles of
-        64 rows -> of 32, us: 8 gated experts of 2048 x 2048, top 2: 4 rows per expert 95 -> 51, 16: 95 -> 60, 25: 95 -> 61, 32: 91 -> 75, 40:
-        97 -> 121; 4096 x 3072: 16: 187 -> 124, 32: 189 -> 180; 32 experts of 2048 x 1024, top 4: 4: 125 -> 101, 25: 130 -> 125, 31: 125 -> 138."""
-        return (h.dtype == torch.bfloat16 and n_slots <= FEW_SLOTS * E and W % 64 == 0 and ff % 64 == 0 and max(W, ff) <= 32768
-                and all(t.data_ptr() % 16 == 0 for t in (h, up, down)))
-
     def moe_experts(h, up, down, idx, weights, kind="relu2", limit=0.0):
         T, W = h.shape
         E, n_up, _ = up.shape
@@ -301,8 +327,10 @@ def seqmix_ops(lib, linear):
         if n_slots == 0:
             return torch.zeros(T, W, dtype=torch.float32, device=dev)
         wide = _wide_experts(n_slots, E, W, ff, kind, h, up, down)
-        few = not wide and _few_row_experts(n_slots, E, W, ff, gated, h, up, down)
-        rows = WIDE_ROWS if wide else few_rows if few else tile_rows
+        held = 0
+        if not wide and h.dtype == torch.bfloat16 and all(t.data_ptr() % 16 == 0 for t in (h, up, down)):
+            held = few_row_tiles(n_slots, E, W, ff, few_rows)
+        rows = WIDE_ROWS if wide else few_rows if held else tile_rows
         n_tiles = (n_slots + E * (rows - 1) + rows - 1) // rows
         cap = n_tiles * rows
         sorted_ = torch.empty(cap, dtype=torch.int32, device=dev)
@@ -325,14 +353,14 @@ def seqmix_ops(lib, linear):
             return out
         _check(lib.bcg_moe_align(_p(idx), n_slots, E, _p(sorted_), cap, _p(tile_e), n_tiles, rows, None, None, _stream()),
                "moe_align")
-        if few:
+        if held:
             code = ACT_CODES[EXPERT_ACTS[kind]] if gated else 1
-            held = min(E, n_slots) + n_slots // (2 * few_rows)     # tiles that are expected to hold rows
+            used = (n_slots + min(E, n_slots) * (rows - 1)) // rows     # `align` packs the tiles in use at the front, this many at most
             hidden = torch.empty(cap, ff, dtype=h.dtype, device=dev)
-            _check(lib.bcg_moe_rows(_p(h), T, W, _p(up), _p(hidden), ff, _p(sorted_), _p(tile_e), n_tiles, held, n_up, W, top, 1, 0,
+            _check(lib.bcg_moe_rows(_p(h), T, W, _p(up), _p(hidden), ff, _p(sorted_), _p(tile_e), used, held, n_up, W, top, 1, 0,
                                     code, limit, _stream()), "moe up rows")
             y = torch.empty(n_slots, W, dtype=h.dtype, device=dev)
-            _check(lib.bcg_moe_rows(_p(hidden), cap, ff, _p(down), _p(y), W, _p(sorted_), _p(tile_e), n_tiles, held, W, ff, top, 0, 1,
+            _check(lib.bcg_moe_rows(_p(hidden), cap, ff, _p(down), _p(y), W, _p(sorted_), _p(tile_e), used, held, W, ff, top, 0, 1,
                                     0, 0.0, _stream()), "moe down rows")
             _check(lib.bcg_moe_combine(_p(y), _p(weights), None, _p(idx), E, _p(out), T, W, top, f32, _stream()), "moe_combine")
             return out

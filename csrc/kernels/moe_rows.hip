@@ -193,7 +193,8 @@ BCG_API int bcg_moe_rows_tile() { return TILE; }
 // One product of `tiles` position tiles of bcg_moe_rows_tile() rows (bcg_moe_align).  a: [a_rows, K] bf16, rows a_stride apart; row of a
 // position: its slot / top (gather) or the position itself; output row: the slot (scatter) or the position.  act 0 none, 1 squared
 // relu, 2 and 3 gated (N rows in pairs, N / 2 output columns).  K % 64 == 0, N % 16 == 0 (gated: 32); 16-byte aligned.
-// experts: how many tiles are expected to hold rows (the launch splits the weights for that many).
+// tiles: no fewer than hold rows (they come first); experts: how many are likely to (the launch splits the weights for that many: all
+// workgroups that have work at once on 256 CUs, one each).
 BCG_API int bcg_moe_rows(const void* a, int64_t a_rows, int64_t a_stride, const void* w, void* out, int64_t out_stride, const void* sorted,
                          const void* tile_expert, int tiles, int experts, int N, int K, int top, int gather, int scatter, int act,
                          float limit, void* stream) {

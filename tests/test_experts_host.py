@@ -1,6 +1,7 @@
 """Expert layers of the HIP backend where no kernel runs: routing by token id of host tensors, wrapped tensors and traces is a gather, as
 in the reference; a step without tokens or without chosen experts is zeros.  No GPU."""
 import os
+import random
 
 import pytest
 import torch
@@ -42,3 +43,25 @@ def test_no_slots(ops, T, top, dtype):
     idx, w = torch.zeros(T, top, dtype=torch.int32), torch.zeros(T, top)
     out = ops.moe_experts(h, up, down, idx, w, "silu_gated")
     assert torch.equal(out, reference.moe_experts(h, up, down, idx, w, "silu_gated")) and out.shape == (T, 64) and out.dtype == torch.float32
+
+
+def test_tiles_of_few_rows():
+    """The rule for position tiles of 32 rows: never past its limits, and what it counts is enough for the tiles that hold slots."""
+    from byzantine_consensus_llm_agents_amd.ops.seqmix import FEW_SLOTS, few_row_tiles
+    rng, over, taken = random.Random(5), 0, 0
+    for _ in range(400):
+        E, top = rng.choice([1, 2, 8, 31, 64, 200, 256]), rng.choice([1, 2, 8])
+        n = rng.randint(1, max(1, FEW_SLOTS * E // top)) * top
+        held = few_row_tiles(n, E, 2048, 1024, 32)
+        if n > FEW_SLOTS * E or held == 0:
+            continue
+        counts = [0] * E
+        for _ in range(n):
+            counts[rng.randrange(E)] += 1
+        tiles = sum(-(-c // 32) for c in counts)
+        assert tiles <= (n + min(E, n) * 31) // 32      # what is launched
+        taken, over = taken + 1, over + (tiles > held + 1 + E // 30)
+    assert taken > 200 and over < 0.06 * taken           # two standard deviations
+    assert few_row_tiles(24 * 8 + 1, 8, 2048, 2048, 32) == 0 and few_row_tiles(128, 8, 2048, 2048, 32) == 8
+    assert few_row_tiles(128, 128, 2048, 1024, 32) == 0 and few_row_tiles(2048, 256, 1024, 256, 32) == 0
+    assert few_row_tiles(1, 256, 4096, 3072, 32) == 1 and few_row_tiles(16, 8, 512, 256, 32) == 0

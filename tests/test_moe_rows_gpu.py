@@ -1,7 +1,7 @@
 """Expert products of small steps (csrc/kernels/moe_rows.hip) against the same equations in float64.  GPU only.
 
 Tiles of 32 rows: one row, 16 and 17, 32 and 33 rows of an expert, all rows on two experts (several tiles of one), experts without
-a row; K of one and a half units of 256 bytes; shares of the weight that are empty, partial and several passes long.  Bound: hidden
+a row, far more experts than slots; K of one and a half units of 256 bytes; shares of the weight that are empty, partial and several passes long.  Bound: hidden
 values and rows are each one bf16 rounding (2^-9) of an fp32 sum; 2-norm of the error 2^-7."""
 import pytest
 import torch
@@ -11,10 +11,18 @@ from test_moe_wide_gpu import _exact, _routing
 pytestmark = pytest.mark.gpu
 
 
+@pytest.fixture(autouse=True)
+def small_experts(monkeypatch):
+    """The kernel's edges are at sizes below those where it is faster."""
+    from byzantine_consensus_llm_agents_amd.ops import seqmix
+    monkeypatch.setattr(seqmix, "FEW_WEIGHT", 0)
+
+
 @pytest.mark.parametrize("kind,limit", [("silu_gated", 0.0), ("clamped_glu", 1.5), ("relu2", 0.0)])
 @pytest.mark.parametrize("routing,T,E,top,W,ff", [("even", 1, 8, 2, 64, 64), ("even", 16, 1, 1, 128, 64), ("even", 17, 1, 1, 192, 320),
                                                   ("two", 32, 4, 2, 256, 128), ("two", 33, 6, 2, 448, 192), ("even", 64, 8, 2, 2048, 2048),
-                                                  ("two", 70, 8, 2, 64, 1024), ("even", 40, 40, 4, 320, 64)])
+                                                  ("two", 70, 8, 2, 64, 1024), ("even", 40, 40, 4, 320, 64),
+                                                  ("even", 1, 64, 2, 128, 64), ("two", 3, 100, 2, 64, 64), ("even", 300, 256, 8, 1024, 1024)])
 def test_few_row_experts(kind, limit, routing, T, E, top, W, ff):
     from byzantine_consensus_llm_agents_amd.ops import get_ops
     from byzantine_consensus_llm_agents_amd.ops.seqmix import FEW_SLOTS
