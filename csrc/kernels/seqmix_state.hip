@@ -1117,9 +1117,13 @@ template <typename T, bool DELTA>
 int launch_scan(const ScanArgs& a, int tokens, int B, hipStream_t s) {
   dim3 grid(B, a.H, (a.vdim + 8 * SCAN_WAVES - 1) / (8 * SCAN_WAVES));
   // four tokens and more per segment: below, staging a chunk of eight costs more than the tokens gain (64 segments of one token
-  // 60 us, 66 that way)
+  // 60 us, 66 that way).  Both kernels over 1 to 200 segments, 4 to 32 heads, this one's time over the other's: up to 64 rows 0.36 to 1.0, 128
+  // rows 0.47 to 1.0 (fp32 values, 100 and more short segments: to 1.07).  Past 128 rows chunks are of four tokens and a wave keeps 32 rows
+  // and as many of k: 0.60 to 1.0 up to three workgroups per CU, then 1.04 to 1.18 (16 heads of 256 x 256, 8 segments of 1000: 1340 us, 1447);
+  // but 0.85 to 1.0 of bf16 values in segments of less than 16
   if constexpr (DELTA) {
-    if (a.gd == 1 && tokens / 4 >= B) {
+    const int64_t groups = static_cast<int64_t>(grid.x) * grid.y * grid.z;
+    if (a.gd == 1 && tokens / 4 >= B && (a.dim <= 128 || groups <= 768 || (sizeof(T) == 2 && tokens / 16 < B))) {
       if (a.dim <= 32) delta_scan_kernel<T, 32><<<grid, 64 * SCAN_WAVES, 0, s>>>(a);
       else if (a.dim <= 64) delta_scan_kernel<T, 64><<<grid, 64 * SCAN_WAVES, 0, s>>>(a);
       else if (a.dim <= 128) delta_scan_kernel<T, 128><<<grid, 64 * SCAN_WAVES, 0, s>>>(a);

@@ -33,7 +33,7 @@ PARTS, ROWS = [(0, 16), (7, 9), (3, 1), (0, 31), (40, 8), (0, 1)], [3, 0, 4, 1, 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("H,Gq,d,e", [(4, 4, 32, 32), (2, 1, 20, 33), (6, 3, 64, 31), (4, 2, 48, 72), (4, 2, 128, 128), (3, 3, 100, 130), (2, 1, 256, 40),
-                                      (1, 1, 1, 1)])
+                                      (1, 1, 1, 1), (64, 1, 130, 65)])   # (the last: more workgroups than the rule takes past 128 rows, in fp32)
 def test_against_64_bits(dtype, H, Gq, d, e):
     from byzantine_consensus_llm_agents_amd.ops import get_ops
     ops = get_ops("hip")
