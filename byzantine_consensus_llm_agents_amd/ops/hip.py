@@ -23,9 +23,6 @@ PREFILL32_MAX_BLOCKS = 1024  # csrc/kernels/attention.hip: the 32x32 kernel's LD
 
 # csrc/kernels/gemm_skinny.hip: most rows, most rows with a fused norm, longest rows in bytes
 SKINNY_ROWS, SKINNY_NORM_ROWS, SKINNY_ROW_BYTES = 64, 16, 65536
-# `decode_attention`: every workgroup of a row rotates its queries again, so with many rows the separate launch wins (a step of
-# 24 layers of 14 / 2 heads of 64, us: 120 rows 2051 separate, 2029 fused; 400 rows 2833, 2871)
-DECODE_FUSED_ROWS = 128
 SKINNY_LONG_K = 12288  # past it: fewer shapes gain (`_few_rows_pay`), logged apart
 
 c_int, c_float, c_void_p, c_uint32, c_int64 = ctypes.c_int, ctypes.c_float, ctypes.c_void_p, ctypes.c_uint32, ctypes.c_int64
@@ -227,6 +224,19 @@ def _kv_fp8(k_cache: torch.Tensor, v_cache: torch.Tensor) -> int:
     _req(k_cache.dtype == v_cache.dtype and k_cache.dtype in (torch.bfloat16, torch.float8_e4m3fn)
          and k_cache.is_contiguous() and v_cache.is_contiguous(), "KV cache: contiguous bf16 or float8_e4m3fn")
     return int(k_cache.dtype == torch.float8_e4m3fn)
+
+
+def decode_fused_pays(B: int, n_kv: int, splits: int) -> bool:
+    """Whether a decode step of B rows with heads of 64 gains by the rotary embedding inside the attention launch; splits: parts of a
+    row's context that the block table has room for (the contexts themselves are on the device).
+
+    The rotation takes registers, so two workgroups of a CU are resident where the separate kernel has three, and every workgroup of a row rotates
+    its queries again.  Rotary launch, attention and merge over the fused pair, 14 / 2, 16 / 4, 32 / 8, 16 / 16 and 16 / 1 heads, contexts
+    of 16 to 16000 tokens, table of their length: 1.03 to 1.19 while all parts are resident (B n_kv splits <= 512), 0.97 to 1.1 at 576
+    (contexts spread by a third to either side: 1.04 to 1.08, a quarter of the parts is empty), past that 0.72 to 1.04 (16 kv heads, 100 rows of 20
+    tokens 16.5 us, 22.8).  Wide tables say nothing of the contexts: up to 16 heads of K and V in all 1.0 to 1.19 up to 16000 tokens, from 32
+    on 0.93 there.  More than 128 rows were not timed in a step."""
+    return B <= 128 and (B * n_kv <= 16 or B * n_kv * splits <= 576)
 
 
 def hip_ops() -> SimpleNamespace:
@@ -877,7 +887,8 @@ def hip_ops() -> SimpleNamespace:
                            embed_rmsnorm=embed_rmsnorm,
                            qk_norm_rope_kv_write=qk_norm_rope_kv_write,
                            paged_attention_decode=paged_attention_decode,
-                           decode_attention=decode_attention, decode_fused_rows=DECODE_FUSED_ROWS,
+                           decode_attention=decode_attention,
+                           decode_fused_pays=lambda B, n_kv, tokens: decode_fused_pays(B, n_kv, -(-tokens // lib.bcg_decode_split_tokens(B, n_kv, tokens))),
                            decode_workspace_numel=decode_workspace_numel,
                            decode_max_context=lambda cascade=True: lib.bcg_decode_max_context(int(cascade)),
                            paged_attention_prefill=paged_attention_prefill,

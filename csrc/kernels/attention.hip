@@ -397,7 +397,8 @@ constexpr int DEC_MAX_B = 2048;
 // FUSED (heads of 64, bf16 caches): the kernel takes the projected rows as they come, without a rotary launch and a pass over q
 // before it: every workgroup rotates (and normalises) its own query heads while its K/V loads are in flight; the one with the
 // newest token also stores that token's K/V and puts it into its chunk's registers, where the loads brought what was there
-// before.  24 layers of 14 / 2 heads at 4 rows of 500 tokens: 912 -> 873 us a step.  Heads of 128 take the separate launches:
+// before.  24 layers of 14 / 2 heads at 4 rows of 500 tokens: 912 -> 873 us a step.  It keeps 189 registers (the separate one 144), so two workgroups
+// of a CU are resident instead of three: `decode_fused_pays` in ops/hip.py has the line.  Heads of 128 take the separate launches:
 // two chunks of K/V and the rotation's operands fill the registers (10 rows of 1100 tokens, 40 / 8 heads, a step of 16 layers: 2561
 // us, 2590 fused; 448 rows 6950, 8110).  Merging the splits in the workgroup that arrives last costs more than the merge
 // launch for both (stores past the L2, a ticket, the reads back: 880 and 2669).
