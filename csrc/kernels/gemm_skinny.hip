@@ -11,7 +11,9 @@
 //     rows at once): the next pass's loads are in flight while a pass is reduced and written (34816 x 5120 gated, 10 rows:
 //     three workgroups per CU, one after the other, 74 us, so 59; 151936 x 5120 265 -> 234);
 //   * the waves of a workgroup share K in turns, unit by unit: neighbouring waves read neighbouring lines (4 % over
-//     a contiguous part of K per wave); no barrier in the loop, every register is loaded again as soon as it has been
+//     a contiguous part of K per wave).  Rows of 8 and 16 KB are shared in contiguous parts: in turns, all waves of the chip read
+//     the same few memory channels at a time (1 to 10 rows, us, in turns and in parts: 8192 x 8192 30.2, 25.5; 4096 x 8192 16.5, 13.5; 8192 x 4096
+//     15.9, 15.2; 4096 x 4096 8.8, 8.0; but rows of 32 KB, 8192 x 16384 58, 83).  No barrier in the loop, every register is loaded again as soon as it has been
 //     consumed; the partial tiles meet in LDS once per pass, in wave order: the same inputs give the same bits;
 //   * a unit of K is 256 bytes: a load takes 64 bytes of each of 16 (row, segment) pairs, and a 4 x 4 transposition within
 //     quads of lanes makes the operands of four matrix instructions (5120 x 17408 with 10 rows 36.2 -> 31.9 us, fp8 6144 x 16384
@@ -23,6 +25,7 @@
 //     once, as the separate norm rounds its output once.
 // 10 rows, us, one workgroup per pass and 128-byte units -> now: 7168 x 5120 18.1 -> 16.4, 5120 x 5120 14.7 -> 12.4, gate + up 34816 x
 // 5120 74.5 -> 59.8, 151936 x 5120 265 -> 234, 4096 x 4096 10.3 -> 9.2, 4096 x 12288 23 -> 18.7, 5120 x 17408 (tile kernel 36.6) 31.9.
+// 1 row, against the same: 2048 x 8192 10.6 -> 10.3, but up to 1024 x 8192 9.3 -> 9.8, 1024 x 12288 12.4 -> 13.6.
 // 20 rows, tile kernel with split-K -> now: fp8 8192 x 6144 15.4 -> 11.6, 6144 x 6144 14.8 -> 10.5, 32768 x 6144 38.5 -> 35.1, 6144 x
 // 16384 27.4 -> 20.8; bf16 32768 x 6144 75.4 -> 68.6.  Launches in a graph, every one with other weights.  From 33 rows on X takes
 // more of a CU's intake than W, and two blocks of W fill the registers: short rows in one pass only (64 rows, library -> here:
@@ -124,6 +127,8 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_skinny_kernel(SkinnyArgs a) {
   const int per = (share / 4 + a.passes - 1) / a.passes * 4;
   const uint32_t rb = a.row_bytes;
   const int nu = (rb + UB - 1) / UB, lw = (nu + NW - 1) / NW;       // units of K, a wave's units of a pass
+  const bool parts = rb == 8192 || rb == 16384;                     // contiguous units of K per wave, not every NW-th
+  const int u0 = parts ? wave * lw : wave, us = parts ? 1 : NW;     // a wave's first unit, from one of its units to the next
   const uint32_t vo = UB == 256 ? ((lane >> 2) & 3) * 4 * rb + kg * 64 + (lane & 3) * 16 : (r & 7) * rb + (kg + (r >> 3) * 4) * 16;
   const uint32_t vs = UB == 256 ? rb : 8 * rb;                      // from load to load of a block
   const uint32_t vo_tail = UB == 256 && (rb & 255) && kg >= 2 ? PAST_END : vo;   // the last unit may be half a unit
@@ -146,7 +151,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_skinny_kernel(SkinnyArgs a) {
     }
   };
   auto where = [&](Item it) {
-    const int t = wave + it.j * NW;
+    const int t = u0 + it.j * us;
     const bool in = t < nu && it.p < a.passes;
     const int off = in ? t * UB : 0, first = in ? it.p * per : 0;
     const size_t at = static_cast<size_t>(first) * rb + off;
@@ -291,7 +296,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_skinny_kernel(SkinnyArgs a) {
         to_operand(xf[s][m], xt[m]);
         load_x(at, s, m);
         if constexpr (NORM) {
-          const uint8_t* nw = norm_lds + (wave + now.j * NW) * UB;
+          const uint8_t* nw = norm_lds + (u0 + now.j * us) * UB;
 #pragma unroll
           for (int j = 0; j < LB; ++j)
             xt[m][j] = scale_fragment(xt[m][j], *reinterpret_cast<const u32x4*>(nw + (UB == 256 ? kg * 64 + j * 16 : j * 64 + kg * 16)), ss[m]);
@@ -344,7 +349,8 @@ int launch(SkinnyArgs a, int passes, hipStream_t stream) {
 
 // The fewest passes, then the fewest row blocks that hold a pass: blocks that stay empty cost instructions.  Rows of up to
 // 2048 bytes and shares of 4 columns take 128-byte units (see above), the latter two units at once: a wave then has only
-// four loads in flight (896 x 4864: 8.5 us with one, 7.7).
+// four loads in flight (896 x 4864: 8.5 us with one, 7.7); up to four rows, whose loads of X are mostly outside, shares of
+// 8 columns too (2048 x 8192: 11.6, 10.3).
 template <int MT, int EPI, bool NORM, bool F8>
 int pick(const SkinnyArgs& a, hipStream_t s) {
   constexpr int PER = EPI == EPI_SILU_MUL ? 2 : 4;                             // groups of 4 columns of a block of W
@@ -362,7 +368,7 @@ int pick(const SkinnyArgs& a, hipStream_t s) {
                : blocks <= 4 ? launch<1, 4, 128, 1, EPI, NORM, F8>(a, passes, s) : launch<1, 8, 128, 1, EPI, NORM, F8>(a, passes, s);
       }
     }
-    if (share == 1) return launch<1, EPI == EPI_SILU_MUL ? 2 : 1, 128, 2, EPI, NORM, F8>(a, passes, s);
+    if (share == 1 || (EPI != EPI_SILU_MUL && share == 2 && a.M <= 4)) return launch<1, EPI == EPI_SILU_MUL ? 2 : 1, 128, 2, EPI, NORM, F8>(a, passes, s);
   }
   if constexpr (EPI == EPI_SILU_MUL) {
     if (blocks <= 2) return launch<MT, 2, 256, 1, EPI, NORM, F8>(a, passes, s);
