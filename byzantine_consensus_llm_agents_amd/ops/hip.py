@@ -23,7 +23,7 @@ PREFILL32_MAX_BLOCKS = 1024  # csrc/kernels/attention.hip: the 32x32 kernel's LD
 
 # csrc/kernels/gemm_skinny.hip: most rows, most rows with a fused norm, longest rows in bytes
 SKINNY_ROWS, SKINNY_NORM_ROWS, SKINNY_ROW_BYTES = 64, 16, 65536
-SKINNY_LONG_K = 12288  # past it: fewer shapes gain (`_few_rows_pay`), logged apart
+SKINNY_LONG_K = 12288  # past it: fewer shapes gain (`few_rows_pay`), logged apart
 
 c_int, c_float, c_void_p, c_uint32, c_int64 = ctypes.c_int, ctypes.c_float, ctypes.c_void_p, ctypes.c_uint32, ctypes.c_int64
 
@@ -224,6 +224,52 @@ def _kv_fp8(k_cache: torch.Tensor, v_cache: torch.Tensor) -> int:
     _req(k_cache.dtype == v_cache.dtype and k_cache.dtype in (torch.bfloat16, torch.float8_e4m3fn)
          and k_cache.is_contiguous() and v_cache.is_contiguous(), "KV cache: contiguous bf16 or float8_e4m3fn")
     return int(k_cache.dtype == torch.float8_e4m3fn)
+
+
+def few_rows_pay(M: int, N: int, row_bytes: int, gated: bool) -> bool:
+    """Whether M <= SKINNY_ROWS rows of bf16 gain by the few-row kernel, W of N rows of row_bytes; gated: the [gate; up] form, which saves the
+    other side a pass over the product.
+
+    Each CU reads all of X for its N / 256 rows of W, so few long rows of W lose to a split of K over the CUs; a turn of a workgroup's
+    waves is 2048 bytes of a row, so rows of one and a half turns leave waves idle; from 33 rows on one pass over W only.  Times of this kernel
+    over those of tile kernels or library (which has a kernel for exactly 32 rows); "but" is what the lines leave to them:
+    * up to 16 rows 0.22 to 1.0 (to 1.1 for one or two rows of up to 1024 x 12288); but 13312 to 16384 long, few of them: 256 1.11 to
+      1.68, with 13 rows and more 512 and 1024 1.02 to 1.13; gated, up to 3072 of them 1.05 to 1.17 against the plain form and a pass;
+    * 17 to 32 rows, up to 8192 bytes 0.45 to 1.03, longer ones from 4096 of them on 0.33 to 1.03; but 512 x 640 to 512 x 896 1.04 to 1.18, 256 x 1536 1.13
+      to 1.22, exactly 32 rows up to 2048 x 2560 or x 3584 1.06 to 1.17, up to 1024 x 3072 or x 4096 0.98 to 1.19;
+    * 33 to 48 rows 0.46 to 1.06; but up to 1024 x 448 and 512 x 768 1.02 to 1.17, 3072 x 1536 1.01 to 1.13, 256 x 1536 1.5, 2048 x 2560 1.09 to 1.39, 1536 x
+      3072 1.17 to 1.26, 8192 x 4096 1.03 to 1.06, longer rows 1.3 and more;
+    * 49 to 64 rows 0.62 to 1.10, with 1024 to 2048 x 2048 1.02 to 1.16 (a store; gated 0.87 to 0.92); but 1024 x 448 1.05 to 1.27, 6144 x 448 1.04 to
+      1.16, 3072 x 1536 1.14 to 1.26, 4096 x 4096 1.08;
+    * gated 0.42 to 1.03; but with 33 to 48 rows 256 x 1536 1.09, 2048 x 2560 1.08 to 1.1, and the longer rows of the lines above."""
+    part = row_bytes % 2048 != 0     # the last turn is not a whole one
+    if M <= 16:
+        if gated:
+            return row_bytes <= 2 * SKINNY_LONG_K or N >= 4096
+        return row_bytes <= 2 * SKINNY_LONG_K or row_bytes > 32768 or N >= (512 if M <= 12 else 1536)
+    if M <= 32:
+        if gated or row_bytes > 8192:
+            return row_bytes <= 8192 or N >= 4096
+        if row_bytes > 4096:
+            return not (M == 32 and N <= (2048 if part else 1024))
+        if row_bytes > 2048:
+            return not part or N > 256
+        return not (1024 < row_bytes < 2048 and 256 < N < 768)
+    if N > 32 * 256 or row_bytes > (8192 if M <= 48 else 4096):
+        return False
+    if M <= 48:
+        if row_bytes > 4096 and part:
+            return N >= 3072
+        if gated:
+            return not (row_bytes > 2048 and part and N < 512)
+        if row_bytes > 4096:
+            return N >= 2048 if row_bytes <= 6144 else N <= 6144
+        if row_bytes > 2048:
+            return not part or N >= 4096
+        return N <= 256 or N >= (1536 if row_bytes < 1024 else 768)
+    if gated or 1536 <= row_bytes <= 2048:
+        return N >= 1024
+    return 1536 <= N <= 4096 if row_bytes < 1536 else N >= (4096 if part else 1024)
 
 
 def decode_fused_pays(B: int, n_kv: int, splits: int) -> bool:
@@ -446,29 +492,13 @@ def hip_ops() -> SimpleNamespace:
             return [(M, plan.choose(M, w.shape[0], K, epi))]
         return plan.pieces(M, w.shape[0], K, epi)
 
-    def _few_rows_pay(M, N, row_bytes, epi):
-        """Whether M <= SKINNY_ROWS rows gain by the few-row kernel.  Each CU reads all of X for its N / 256 rows of W, so few long
-        rows of W lose to a split of K over the CUs (us, tile kernels or library and this one):
-        * up to 16 rows only the gated form past 12288 columns of bf16 (1024 x 16384 22.2, 25.3; 5120 x 25600 138, 48);
-        * 17 to 32 rows: rows of up to 8192 bytes always gain (256 x 4096 11.2, 8.7; 2048 x 4096 14.7, 9.0), longer ones from 4096
-          rows of W on (4096 x 12288 26.0, 24.9; but 3072 x 16384 28.5, 29.3; 1024 x 6144 10.5, 11.7; 256 x 8192 8.7, 14.6);
-        * 33 to 48 rows: one pass over W and rows of up to 8192 bytes (4096 x 2048 11.8, 8.0; 4096 x 4096 13.6, 12.5; 256 x 2048 7.5, 7.2;
-          but 8736 x 2048 14.7, 15.1; 2048 x 8192 13.8, 18.7);
-        * 49 to 64 rows: of those rows of up to 4096 bytes, 1024 of them and more (4096 x 2048 12.4, 9.5; 6144 x 768 10.0, 7.4; but 4096 x
-          4096 13.8, 14.9; 768 x 2048 8.1, 8.9)."""
-        if M > 32:
-            return N <= 32 * 256 and (row_bytes <= 8192 if M <= 48 else row_bytes <= 4096 and N >= 1024)
-        if M <= 16:
-            return epi != 1 or row_bytes <= 2 * SKINNY_LONG_K or N >= 4096
-        return row_bytes <= 8192 or N >= 4096
-
     def _skinny(x, w, epi):
         """Whether the few-row kernel takes x W^T: up to SKINNY_ROWS rows of whole 128-byte lines, where they pay (csrc/kernels/
         gemm_skinny.hip holds more of both sides' times); table and library keep the others."""
         M, K = x.shape
         N = w.shape[0]
         return (plan.mode == "1" and 1 <= M <= SKINNY_ROWS and K % 64 == 0 and 64 <= K <= SKINNY_ROW_BYTES // 2
-                and N >= 8 and N % (8 if epi == 1 else 4) == 0 and _few_rows_pay(M, N, 2 * K, epi) and _plain(x, w))
+                and N >= 8 and N % (8 if epi == 1 else 4) == 0 and few_rows_pay(M, N, 2 * K, epi == 1) and _plain(x, w))
 
     def _skinny_name(M, K):
         """("skinny", blocks of 16 rows) in the dispatch log."""
@@ -820,11 +850,13 @@ def hip_ops() -> SimpleNamespace:
     fp8_cfg = fp8_plan.choose
 
     def _skinny_fp8(xq, xs, wq, ws, *beside):
-        """Whether the few-row kernel takes the fp8 product: as `_skinny`; `beside`: [(bias or residual, its shape)]."""
+        """Whether the few-row kernel takes the fp8 product: as `_skinny`, every size up to 16 rows, past them rows of up to 8192 bytes and
+        many longer ones (N, K of 256 to 16384, 1 to 32 rows, against tile kernels and library: 0.33 to 1.0); `beside`: [(bias or
+        residual, its shape)]."""
         M, K = xq.shape
         N = wq.shape[0]
         return (plan.mode == "1" and 1 <= M <= 32 and K % 128 == 0 and 128 <= K <= SKINNY_ROW_BYTES and N >= 16 and N % 16 == 0
-                and wq.dim() == 2 and wq.shape[1] == K and _few_rows_pay(M, N, K, 0)
+                and wq.dim() == 2 and wq.shape[1] == K and (M <= 16 or K <= 8192 or N >= 4096)
                 and xq.is_cuda and xq.get_device() == torch.cuda.current_device() and xq.is_contiguous() and wq.is_contiguous()
                 and all(t.device == xq.device and t.data_ptr() % 16 == 0 and bare(t) for t in (xq, wq, xs, ws))
                 and xs.dtype == ws.dtype == torch.float32 and xs.numel() == M and ws.numel() == N and xs.is_contiguous()

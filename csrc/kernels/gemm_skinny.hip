@@ -13,7 +13,8 @@
 //   * the waves of a workgroup share K in turns, unit by unit: neighbouring waves read neighbouring lines (4 % over
 //     a contiguous part of K per wave).  Rows of 8 and 16 KB are shared in contiguous parts: in turns, all waves of the chip read
 //     the same few memory channels at a time (1 to 10 rows, us, in turns and in parts: 8192 x 8192 30.2, 25.5; 4096 x 8192 16.5, 13.5; 8192 x 4096
-//     15.9, 15.2; 4096 x 4096 8.8, 8.0; but rows of 32 KB, 8192 x 16384 58, 83).  No barrier in the loop, every register is loaded again as soon as it has been
+//     15.9, 15.2; 4096 x 4096 8.8, 8.0; but rows of 32 KB, 8192 x 16384 58, 83).  Rows of 32 KB are shared in turns, a workgroup
+//     beginning at its own (4096 x 16384 33.5, so 25.5, library 31.3; but 16384 x 4096 25.7, 31).  No barrier in the loop, every register is loaded again as soon as it has been
 //     consumed; the partial tiles meet in LDS once per pass, in wave order: the same inputs give the same bits;
 //   * a unit of K is 256 bytes: a load takes 64 bytes of each of 16 (row, segment) pairs, and a 4 x 4 transposition within
 //     quads of lanes makes the operands of four matrix instructions (5120 x 17408 with 10 rows 36.2 -> 31.9 us, fp8 6144 x 16384
@@ -129,6 +130,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_skinny_kernel(SkinnyArgs a) {
   const int nu = (rb + UB - 1) / UB, lw = (nu + NW - 1) / NW;       // units of K, a wave's units of a pass
   const bool parts = rb == 8192 || rb == 16384;                     // contiguous units of K per wave, not every NW-th
   const int u0 = parts ? wave * lw : wave, us = parts ? 1 : NW;     // a wave's first unit, from one of its units to the next
+  const int j0 = rb == 32768 ? (blockIdx.x >> 3) % lw : 0;          // ... and the one that it begins with
   const uint32_t vo = UB == 256 ? ((lane >> 2) & 3) * 4 * rb + kg * 64 + (lane & 3) * 16 : (r & 7) * rb + (kg + (r >> 3) * 4) * 16;
   const uint32_t vs = UB == 256 ? rb : 8 * rb;                      // from load to load of a block
   const uint32_t vo_tail = UB == 256 && (rb & 255) && kg >= 2 ? PAST_END : vo;   // the last unit may be half a unit
@@ -151,7 +153,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_skinny_kernel(SkinnyArgs a) {
     }
   };
   auto where = [&](Item it) {
-    const int t = u0 + it.j * us;
+    const int j = it.j + j0, t = u0 + (j < lw ? j : j - lw) * us;
     const bool in = t < nu && it.p < a.passes;
     const int off = in ? t * UB : 0, first = in ? it.p * per : 0;
     const size_t at = static_cast<size_t>(first) * rb + off;
@@ -296,7 +298,8 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_skinny_kernel(SkinnyArgs a) {
         to_operand(xf[s][m], xt[m]);
         load_x(at, s, m);
         if constexpr (NORM) {
-          const uint8_t* nw = norm_lds + (u0 + now.j * us) * UB;
+          const int jn = now.j + j0;
+          const uint8_t* nw = norm_lds + (u0 + (jn < lw ? jn : jn - lw) * us) * UB;
 #pragma unroll
           for (int j = 0; j < LB; ++j)
             xt[m][j] = scale_fragment(xt[m][j], *reinterpret_cast<const u32x4*>(nw + (UB == 256 ? kg * 64 + j * 16 : j * 64 + kg * 16)), ss[m]);

@@ -55,6 +55,30 @@ def test_bf16(ops, M, N, K):
         assert _off(ops.linear_silu(x, w), gated) < 2 ** -7
 
 
+# rows of 8, 16 and 32 KB: other orders of K
+@pytest.mark.parametrize("M,N,K", [(1, 256, 4096), (4, 2048, 4096), (16, 1028, 4096), (1, 520, 8192), (5, 8192, 8192), (20, 4096, 8192), (3, 1024, 16384),
+                                   (16, 4096, 16384), (24, 5120, 16384)])
+def test_row_pitches(ops, M, N, K):
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    x = (torch.randn(M, K, device="cuda", generator=g) * 3).to(torch.bfloat16)
+    w = (torch.randn(N, K, device="cuda", generator=g) * K ** -0.5).to(torch.bfloat16)
+    y = x.double() @ w.double().t()
+    out, used = _calls(ops, lambda: ops.linear(x, w))
+    assert all(u.startswith("skinny") for u in used) and _off(out, y) < 2 ** -8 and torch.equal(out, ops.linear(x, w))
+    if M <= 16 and K <= 8192:
+        nw = (1 + 0.3 * torch.randn(K, device="cuda", generator=g)).to(torch.bfloat16)
+        xd = x.double()
+        normed = xd * torch.rsqrt(xd.square().mean(1, keepdim=True) + 1e-6) * nw.double()
+        assert _off(ops.norm_linear(x, nw, 1e-6, w), normed @ w.double().t()) < 2 ** -7   # (the norm rounds its products too)
+    if N % 16 == 0 and (K <= 4096 or N >= 4096):     # (of bytes that are twice as many)
+        f8 = torch.float8_e4m3fn
+        xq, wq = (x * 20).to(f8), (w * 100).to(f8)
+        xq, wq = torch.cat([xq, xq], 1), torch.cat([wq, wq], 1)
+        xs, ws = torch.full((M, 1), 0.05, device="cuda"), torch.full((N,), 0.01, device="cuda")
+        ref = (xq.double() @ wq.double().t()) * 0.05 * 0.01
+        assert _off(ops.linear_fp8(xq, xs, wq, ws), ref) < 2 ** -8
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 16, 128), (16, 1024, 640), (17, 528, 384), (20, 8192, 6144), (32, 36864, 896), (9, 70000, 256),
                                    (32, 6144, 16384)])
 def test_fp8(ops, M, N, K):
