@@ -235,41 +235,43 @@ def few_rows_pay(M: int, N: int, row_bytes: int, gated: bool) -> bool:
     over those of tile kernels or library (which has a kernel for exactly 32 rows); "but" is what the lines leave to them:
     * up to 16 rows 0.22 to 1.0 (to 1.1 for one or two rows of up to 1024 x 12288); but 13312 to 16384 long, few of them: 256 1.11 to
       1.68, with 13 rows and more 512 and 1024 1.02 to 1.13; gated, up to 3072 of them 1.05 to 1.17 against the plain form and a pass;
-    * 17 to 32 rows, up to 8192 bytes 0.45 to 1.03, longer ones from 4096 of them on 0.33 to 1.03; but 512 x 640 to 512 x 896 1.04 to 1.18, 256 x 1536 1.13
-      to 1.22, exactly 32 rows up to 2048 x 2560 or x 3584 1.06 to 1.17, up to 1024 x 3072 or x 4096 0.98 to 1.19;
-    * 33 to 48 rows 0.46 to 1.06; but up to 1024 x 448 and 512 x 768 1.02 to 1.17, 3072 x 1536 1.01 to 1.13, 256 x 1536 1.5, 2048 x 2560 1.09 to 1.39, 1536 x
+    * 17 to 32 rows, up to 8192 bytes 0.45 to 1.03, longer ones from 4096 of them on 0.33 to 1.03; but up to 31 rows 512 x 640 to 512 x 896 1.04 to 1.18, 256 x 1536 1.13 to
+      1.22, exactly 32 rows up to 2048 x 2560 and 1536 x 3584 0.98 to 1.17, up to 1024 x 3072 or x 4096 0.98 to 1.19;
+    * 33 to 48 rows 0.46 to 1.06; but up to 1024 x 448, 640 x 640 and 512 x 768 1.02 to 1.17, 3072 x 1536 1.01 to 1.13, 256 x 1536 1.5, 2048 x 2560 1.09 to 1.39, 1536 x
       3072 1.17 to 1.26, 8192 x 4096 1.03 to 1.06, longer rows 1.3 and more;
     * 49 to 64 rows 0.62 to 1.10, with 1024 to 2048 x 2048 1.02 to 1.16 (a store; gated 0.87 to 0.92); but 1024 x 448 1.05 to 1.27, 6144 x 448 1.04 to
       1.16, 3072 x 1536 1.14 to 1.26, 4096 x 4096 1.08;
     * gated 0.42 to 1.03; but with 33 to 48 rows 256 x 1536 1.09, 2048 x 2560 1.08 to 1.1, and the longer rows of the lines above."""
     part = row_bytes % 2048 != 0     # the last turn is not a whole one
     if M <= 16:
-        if gated:
+        if gated or row_bytes <= 2 * SKINNY_LONG_K:
             return row_bytes <= 2 * SKINNY_LONG_K or N >= 4096
-        return row_bytes <= 2 * SKINNY_LONG_K or row_bytes > 32768 or N >= (512 if M <= 12 else 1536)
+        return row_bytes > 32768 or N >= (1536 if M > 12 else 512 if row_bytes <= 28672 else 384)
     if M <= 32:
         if gated or row_bytes > 8192:
             return row_bytes <= 8192 or N >= 4096
         if row_bytes > 4096:
-            return not (M == 32 and N <= (2048 if part else 1024))
+            return not (M == 32 and N <= (2048 if part and row_bytes <= 6144 else 1024))
         if row_bytes > 2048:
             return not part or N > 256
-        return not (1024 < row_bytes < 2048 and 256 < N < 768)
+        return not (1024 < row_bytes < 2048 and 256 < N <= 512 and M < 32)
     if N > 32 * 256 or row_bytes > (8192 if M <= 48 else 4096):
         return False
     if M <= 48:
-        if row_bytes > 4096 and part:
-            return N >= 3072
-        if gated:
-            return not (row_bytes > 2048 and part and N < 512)
+        if gated and part:
+            return not 1024 < N < 3072 if row_bytes > 4096 else row_bytes < 2048 or N >= 512
+        if gated or row_bytes == 2048:
+            return True
         if row_bytes > 4096:
-            return N >= 2048 if row_bytes <= 6144 else N <= 6144
+            return N >= 3072 if part else N >= 2048 if row_bytes <= 6144 else N <= 6144
         if row_bytes > 2048:
             return not part or N >= 4096
-        return N <= 256 or N >= (1536 if row_bytes < 1024 else 768)
+        return N <= 256 or row_bytes >= 1792 or N >= (1536 if row_bytes < 1024 else 768 if row_bytes < 1536 else 640)
     if gated or 1536 <= row_bytes <= 2048:
         return N >= 1024
-    return 1536 <= N <= 4096 if row_bytes < 1536 else N >= (4096 if part else 1024)
+    if row_bytes < 1536:
+        return (1536 if row_bytes < 1024 else 1024) <= N <= 4096
+    return N >= (4096 if part else 1024)
 
 
 def decode_fused_pays(B: int, n_kv: int, splits: int) -> bool:

@@ -11,11 +11,11 @@
 //     rows at once): the next pass's loads are in flight while a pass is reduced and written (34816 x 5120 gated, 10 rows:
 //     three workgroups per CU, one after the other, 74 us, so 59; 151936 x 5120 265 -> 234);
 //   * the waves of a workgroup share K in turns, unit by unit: neighbouring waves read neighbouring lines (4 % over
-//     a contiguous part of K per wave).  Rows of 8 and 16 KB are shared in contiguous parts: in turns, all waves of the chip read
-//     the same few memory channels at a time (1 to 10 rows, us, in turns and in parts: 8192 x 8192 30.2, 25.5; 4096 x 8192 16.5, 13.5; 8192 x 4096
-//     15.9, 15.2; 4096 x 4096 8.8, 8.0; but rows of 32 KB, 8192 x 16384 58, 83).  Rows of 32 KB are shared in turns, a workgroup
-//     beginning at its own (4096 x 16384 33.5, so 25.5, library 31.3; but 16384 x 4096 25.7, 31).  No barrier in the loop, every register is loaded again as soon as it has been
-//     consumed; the partial tiles meet in LDS once per pass, in wave order: the same inputs give the same bits;
+//     a contiguous part of K per wave).  Rows of 8 and 16 KB may be shared in contiguous parts (`meets_channels`): in turns, all
+//     waves of the chip read the same few memory channels at a time (1 to 10 rows, us, in turns and in parts: 8192 x 8192 30.2, 25.5;
+//     4096 x 8192 16.5, 13.5; 8192 x 4096 15.9, 15.2; 4096 x 4096 8.8, 8.0; but rows of 32 KB, 8192 x 16384 58, 83).  Rows of
+//     32 KB are shared in turns, a workgroup beginning at its own (4096 x 16384 33.5, so 25.5, library 31.3; but 16384 x 4096
+//     25.7, 31).  No barrier in the loop, every register is loaded again as soon as it has been consumed; the partial tiles meet in LDS once per pass, in wave order: the same inputs give the same bits;
 //   * a unit of K is 256 bytes: a load takes 64 bytes of each of 16 (row, segment) pairs, and a 4 x 4 transposition within
 //     quads of lanes makes the operands of four matrix instructions (5120 x 17408 with 10 rows 36.2 -> 31.9 us, fp8 6144 x 16384
 //     with 20 rows 25.2 -> 20.8).  Short rows and shares of 4 columns use units of 128 bytes, 8 rows a load and one rotation by 8
@@ -111,8 +111,9 @@ struct Reduction {   // of a pass's partial tiles, OB output blocks at a time
 };
 
 // MT, NT: blocks of 16 rows of X and of W (EPI_SILU_MUL: gate and up blocks of the same features alternate).  UB: bytes of
-// a unit of K.  D: units in flight per wave.
-template <int MT, int NT, int UB, int D, int EPI, bool NORM, bool F8>
+// a unit of K.  D: units in flight per wave.  ORD: the orders of `meets_channels` (instances of their own: their index arithmetic costs
+// 0.8 % of a step of small launches).
+template <int MT, int NT, int UB, int D, int EPI, bool NORM, bool F8, bool ORD>
 __global__ __launch_bounds__(64 * NW, 2) void gemm_skinny_kernel(SkinnyArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   using Red = Reduction<MT, NT, EPI>;
@@ -128,9 +129,12 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_skinny_kernel(SkinnyArgs a) {
   const int per = (share / 4 + a.passes - 1) / a.passes * 4;
   const uint32_t rb = a.row_bytes;
   const int nu = (rb + UB - 1) / UB, lw = (nu + NW - 1) / NW;       // units of K, a wave's units of a pass
-  const bool parts = rb == 8192 || rb == 16384;                     // contiguous units of K per wave, not every NW-th
-  const int u0 = parts ? wave * lw : wave, us = parts ? 1 : NW;     // a wave's first unit, from one of its units to the next
-  const int j0 = rb == 32768 ? (blockIdx.x >> 3) % lw : 0;          // ... and the one that it begins with
+  auto unit = [&](int j) {                                          // of K, the j-th of this wave
+    if constexpr (!ORD) return wave + j * NW;
+    if (rb != 32768) return wave * lw + j;
+    j += static_cast<int>(blockIdx.x >> 3) % lw;
+    return wave + (j < lw ? j : j - lw) * NW;
+  };
   const uint32_t vo = UB == 256 ? ((lane >> 2) & 3) * 4 * rb + kg * 64 + (lane & 3) * 16 : (r & 7) * rb + (kg + (r >> 3) * 4) * 16;
   const uint32_t vs = UB == 256 ? rb : 8 * rb;                      // from load to load of a block
   const uint32_t vo_tail = UB == 256 && (rb & 255) && kg >= 2 ? PAST_END : vo;   // the last unit may be half a unit
@@ -153,7 +157,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_skinny_kernel(SkinnyArgs a) {
     }
   };
   auto where = [&](Item it) {
-    const int j = it.j + j0, t = u0 + (j < lw ? j : j - lw) * us;
+    const int t = unit(it.j);
     const bool in = t < nu && it.p < a.passes;
     const int off = in ? t * UB : 0, first = in ? it.p * per : 0;
     const size_t at = static_cast<size_t>(first) * rb + off;
@@ -298,8 +302,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_skinny_kernel(SkinnyArgs a) {
         to_operand(xf[s][m], xt[m]);
         load_x(at, s, m);
         if constexpr (NORM) {
-          const int jn = now.j + j0;
-          const uint8_t* nw = norm_lds + (u0 + (jn < lw ? jn : jn - lw) * us) * UB;
+          const uint8_t* nw = norm_lds + unit(now.j) * UB;
 #pragma unroll
           for (int j = 0; j < LB; ++j)
             xt[m][j] = scale_fragment(xt[m][j], *reinterpret_cast<const u32x4*>(nw + (UB == 256 ? kg * 64 + j * 16 : j * 64 + kg * 16)), ss[m]);
@@ -338,12 +341,23 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_skinny_kernel(SkinnyArgs a) {
   }
 }
 
+// Whether the workgroups meet in the same memory channels if all begin at the same unit of K: many rows of 32 KB, and of 8 and 16 KB where the
+// shares are 2^n bytes apart (one part of K per wave instead of turns: 4096 and 8192 rows 0.84 to 0.97 of the time, but fp8 5120 and 6144 x 8192
+// 1.02 to 1.05, 6144 x 16384 0.96 to 1.01).
+bool meets_channels(const SkinnyArgs& a) {
+  if (a.row_bytes == 32768) return a.units >= 2 * CUS;   // (1024 x 16384: 16.6, so 17.9)
+  const int64_t share = static_cast<int64_t>(a.units / CUS) * 4 * a.row_bytes;
+  return (a.row_bytes == 8192 || a.row_bytes == 16384) && a.units % CUS == 0 && share >= 131072 && (share & (share - 1)) == 0;
+}
+
 template <int MT, int NT, int UB, int D, int EPI, bool NORM, bool F8>
 int launch(SkinnyArgs a, int passes, hipStream_t stream) {
   a.passes = passes;
   const int nu = (a.row_bytes + UB - 1) / UB;
   const int lds = Reduction<MT, NT, EPI>::LDS + (NORM ? (nu + NW - 1) / NW * NW * UB : 0);
-  auto kernel = gemm_skinny_kernel<MT, NT, UB, D, EPI, NORM, F8>;
+  auto kernel = gemm_skinny_kernel<MT, NT, UB, D, EPI, NORM, F8, false>;
+  if constexpr (UB == 256 || D == 2)   // (the others are for shorter rows)
+    if (meets_channels(a)) kernel = gemm_skinny_kernel<MT, NT, UB, D, EPI, NORM, F8, true>;
   if (lds > 65536 && hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
     return -1;
   hipLaunchKernelGGL(kernel, dim3(a.units < CUS ? a.units : CUS), dim3(64 * NW), lds, stream, a);
