@@ -35,7 +35,7 @@ class AttnMeta:
     seq_lens: torch.Tensor       # [B] int32, tokens resident after this step
     q_start: Optional[torch.Tensor] = None   # [B+1] int32 (prefill only)
     max_q_len: int = 1
-    decode: bool = False
+    decode: bool = False         # one new token per row, every row another sequence
     logits_idx: Optional[torch.Tensor] = None  # rows whose logits are needed
     tiles: Optional[torch.Tensor] = None       # [n_tiles, 3] int32 prefill work list (HIP kernel)
     tile_rows: int = 64                        # rows per `tiles` entry (ops.prefill_tile_rows)

@@ -65,8 +65,8 @@ def _likely_tiles(n_slots, E, rows):
 def few_row_tiles(n_slots, E, W, ff, rows):
     """The tiles that are likely to hold rows if an expert layer's products stream the weights past position tiles of 32 rows (csrc/kernels/
     moe_rows.hip), 0 if they do not: up to FEW_SLOTS routed rows per expert, where few experts have a second tile that streams their
-    weight again.  All four launches, tiles of 64 rows -> of 32, us: 8 gated experts of 2048 x 2048, top 2: 4 rows per expert 95 -> 51,
-    16: 95 -> 60, 25: 95 -> 61, 32: 91 -> 75, 40: 97 -> 121; 4096 x 3072: 16: 187 -> 124, 32: 189 -> 180.
+    weight again.  All four launches, tiles of 64 rows -> of 32, us: 8 gated experts of 2048 x 2048, top 2: 4 rows per expert 96 -> 53,
+    16: 97 -> 54; past the line 25: 95 -> 61, 32: 91 -> 75, 40: 97 -> 121; 4096 x 3072: 16: 194 -> 118, 32: 189 -> 180.
     Ratios of the times over 2 to 256 experts, widths 512 to 4096, hidden widths 256 to 3072, 1 to 768 tokens, top 2 and 8:
     * up to 40 tiles 0.24 to 1.03, but up to 1.07 with experts of 512 x 256: most waves have no part of K there;
     * more tiles get a few workgroups each: 0.61 to 1.04 where these fill the 256 CUs to 0.85 and the experts are

@@ -1153,7 +1153,8 @@ BCG_API int bcg_gemm_w4_grouped(int epi, const void* x, const void* w, void* c, 
 //        inter % 256 == 0 (a tile is on one side), 0 < inter < N.
 // Bound by the matrix units like the plain product; the activation on the accumulators replaces a pass that read the product
 // and wrote the hidden values (2039 x 16384 x 2048 clamped: product 107 us and pass 24 -> 107; 8183 x 11264 x 2048, gelu on 8192
-// columns: 301 and 66 -> 316), and rounds once.  No split of K: these instances keep 200 registers and spill none.
+// columns: 301 and 66 -> 316), and rounds once.  No split of K: these instances keep 208 and 198 vector registers
+// beside 256 accumulators (a profiler's count is half of the sum) and spill none.
 BCG_API int bcg_gemm_w4_act(int epi, const void* x, const void* w, void* c, void* tail, int M, int N, int K, int inter, float limit,
                             hipStream_t stream) {
   if (M <= 0 || N <= 0 || N % 16 || K % BK || K <= 0 || inter <= 0) return -2;

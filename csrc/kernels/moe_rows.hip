@@ -4,7 +4,8 @@
 // once for few rows and the kernel is the few-row projection (gemm_skinny.hip, which says why its loads and shares are as they are) with two
 // differences: a workgroup belongs to a position tile, S workgroups share the rows of its expert's weight, and rows of A are
 // gathered by the slots of the tile.  8 experts of 4096 (gated pairs) x 2048 and 2048 x 2048, 128 slots: 53 and 40 us with the 64 x 64 tile
-// kernel (2.5 and 1.7 TB/s: 640 and 320 workgroups of short K-loops behind barriers); align, both products and combine 95 -> 60.
+// kernel (2.5 and 1.7 TB/s: 640 and 320 workgroups of short K-loops behind barriers), 30 and 16 here; align, both products and combine
+// 97 -> 54.
 #include <type_traits>
 
 #include "seqmix_common.h"
