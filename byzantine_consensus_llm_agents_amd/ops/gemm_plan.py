@@ -29,6 +29,7 @@ PP_CFG = 10  # csrc/kernels/gemm_pp.hip: 256 x 256 ping-pong tile, N only a mult
 W4_CFG = 11  # csrc/kernels/gemm_w4.hip: 256 x 256, four 128 x 128 waves (one per SIMD), LDS-DMA fed
 BIG_CFGS = (PP_CFG, W4_CFG)  # 256 x 256 tiles (the register-staged form lost its A/B: csrc/experimental/gemm_rs.hip)
 SMALL_CFG = 5  # 64 x 64
+MID_CFG = 12  # csrc/kernels/gemm_mid.hip: a tile of its own for every product, its plan in the place of the split
 N_CFGS = len(TILES)
 SPLITS = (1, 2, 3, 4, 6, 8)
 CUS = 256       # compute units of an MI355X; on a part of one the rounds would be sized wrongly, the results the same
@@ -41,6 +42,7 @@ STREAM_K = 0  # split_k value of the W4 kernel's stream-K launch (one workgroup 
 class GemmPlan:
     def __init__(self, lib=None, table: Optional[str] = TABLE, max_m: int = 1024):
         self.mode = os.environ.get("BCG_HAND_GEMM", "1")
+        self.lib = lib
         self.force_split = int(os.environ.get("BCG_HAND_GEMM_SPLIT", "1"))  # split-K in "force" mode (tests)
         self.max_m = max_m
         self.rows: Dict[Tuple[int, int, int], List[int]] = {}
@@ -121,6 +123,18 @@ class GemmPlan:
         cfg = self.default_cfg(M)
         return (cfg, 1) if self.supported(cfg, M, N, K, epi) else None
 
+    def mid(self, M: int, N: int, K: int, epi: int) -> Optional[int]:
+        """Plan of the kernel for tens to hundreds of rows (csrc/kernels/gemm_mid.hip), None where it is not taken."""
+        if self.mode != "1" or self.lib is None:
+            return None
+        p = self.lib.bcg_gemm_mid_plan(epi, M, N, K, 0)
+        return p if p >= 0 else None
+
+    def _rest(self, M: int, N: int, K: int, epi: int) -> Optional[Tuple[int, int]]:
+        """The choice for the rows behind whole rounds."""
+        p = self.mid(M, N, K, epi)
+        return self.choose(M, N, K, epi) if p is None else (MID_CFG, p)
+
     def columns(self, M: int, N: int, K: int) -> int:
         """Gated projections (epilogue 1) below LARGE_M rows: how many of the N columns run as whole rounds of 256 x 256
         tiles, the others in 64 x 64 tiles behind them; N: no split.
@@ -187,7 +201,7 @@ class GemmPlan:
                 if (M1, N, K, epi) in self.table:
                     split, main = True, self.choose(M1, N, K, epi)
                 if split:
-                    return [(M1, main), (M2, self.choose(M2, N, K, epi))]
+                    return [(M1, main), (M2, self._rest(M2, N, K, epi))]
         if choice is None and self._large_tiles(K, epi, tiles):
             choice = (W4_CFG, 1)
         return [(M, choice)]

@@ -100,6 +100,9 @@ def load_library(path: str = None) -> ctypes.CDLL:
         "bcg_gemm_skinny": [c_int, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
                             c_void_p],
         "bcg_gemm_skinny_fp8": [c_int] + [c_void_p] * 7 + [c_int] * 3 + [c_void_p],
+        "bcg_gemm_mid_plan": [c_int] * 5,
+        "bcg_gemm_mid_parts": [c_int] * 4 + [ctypes.POINTER(c_int)],
+        "bcg_gemm_mid": [c_int, c_int] + [c_void_p] * 9 + [c_int] * 4 + [c_void_p],
         "bcg_gemm_tile": [c_int, ctypes.POINTER(c_int), ctypes.POINTER(c_int)],
         "bcg_gemm_num_cfgs": [],
         "bcg_embed_scale_rmsnorm": [c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_float, c_float, c_void_p, c_void_p,
@@ -196,7 +199,7 @@ def load_library(path: str = None) -> ctypes.CDLL:
     for name, argtypes in sig.items():
         fn = getattr(lib, name)
         fn.argtypes = argtypes
-        fn.restype = c_int
+        fn.restype = c_int64 if name == "bcg_gemm_mid_parts" else c_int
     _LIB = lib
     return lib
 
@@ -485,6 +488,33 @@ def hip_ops() -> SimpleNamespace:
     def _plain_bias(bias, N, x):
         return bias is None or _plain_beside(bias, (N,), x)
 
+    def _mid(x, w, epi):
+        """The plan by which the kernel for tens to hundreds of rows takes x W^T (csrc/kernels/gemm_mid.hip says which it does), else
+        None.  33 to 64 rows that the few-row kernel takes: from 2.7 M elements of W on (times over the few-row kernel's 0.74 to 0.97 on average over
+        sizes, the slowest 1.1: 40 rows, 6144 x 4096); smaller ones stay where the tests of that kernel hold them (0.77 to 0.82)."""
+        M, K = x.shape
+        N = w.shape[0]
+        if not (33 <= M <= 1024 and plan.mode == "1") or (M <= SKINNY_ROWS and N * K < 2700000 and few_rows_pay(M, N, 2 * K, epi == 1)):
+            return None
+        p = plan.mid(M, N, K, epi)
+        return p if p is not None and _plain(x, w) else None
+
+    def _gemm_mid(p, x, w, epi, out, bias=None, residual=None, scales=(None, None), N=None, at=0):
+        """N, at: gated, N / 2 of the features from at / 2 on, into their columns of `out`."""
+        M, K = x.shape
+        inter = w.shape[0] // 2
+        N = w.shape[0] if N is None else N
+        ws = cnt = None
+        if p >> 8 > 1:
+            tiles = c_int()
+            ws = torch.empty(lib.bcg_gemm_mid_parts(p, epi, M, N, ctypes.byref(tiles)), dtype=torch.float32, device=x.device)
+            _req(tiles.value <= 1 << 16, "gemm_mid: too many output tiles for split-K")
+            cnt = _counters(x.device)
+        _check(lib.bcg_gemm_mid(p, epi, _p(x), w.data_ptr() + at * K, *(None if t is None else _p(t) for t in (*scales, bias, residual)),
+                                out.data_ptr() + at, None if ws is None else _p(ws), None if cnt is None else _p(cnt), M, N, K, inter,
+                                _stream()), "gemm_mid")   # (at / 2 rows or features of 2 bytes)
+        return out
+
     def _pieces(x, w, epi, beside=None, shape=None):
         """Runs of rows and their choices (`GemmPlan.pieces`); beside: the bias or residual, of this shape.  Fewer rows than LARGE_M are
         one run whatever the operands are, so nothing is looked at there: a small eager step is bound by the host (24 layers of
@@ -521,6 +551,10 @@ def hip_ops() -> SimpleNamespace:
         otherwise."""
         M, K = x.shape
         N = w.shape[0]
+        p = _mid(x, w, 0)
+        if p is not None and _plain_bias(bias, N, x):
+            _log(M, N, K, _epi_log, (MID_CFG, p))
+            return _gemm_mid(p, x, w, 0, torch.empty(M, N, dtype=x.dtype, device=x.device), bias)
         if _skinny(x, w, 0) and _plain_bias(bias, N, x):
             return _gemm_skinny(x, w, 0, bias)
         if not (x.is_contiguous() and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16):
@@ -543,7 +577,7 @@ def hip_ops() -> SimpleNamespace:
             return torch.nn.functional.linear(x, w, bias)
         return torch.mm(x, w.t(), out=out) if bias is None else torch.addmm(bias, x, w.t(), out=out)
 
-    from .gemm_plan import LARGE_M, PP_CFG, SMALL_CFG, W4_CFG, GemmPlan
+    from .gemm_plan import LARGE_M, MID_CFG, PP_CFG, SMALL_CFG, W4_CFG, GemmPlan
     plan = GemmPlan(lib)
 
     # Split-K arrival counters (one int per output tile; the last-arriving workgroup of a
@@ -604,6 +638,8 @@ def hip_ops() -> SimpleNamespace:
         N = w.shape[0]
         _req(x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_contiguous() and w.is_contiguous()
              and w.shape[1] == K, "gemm_nt: contiguous bf16 x [M,K], w [N,K]")
+        if cfg == MID_CFG:   # (a piece of a call whose operands were looked at: `_pieces`)
+            return _gemm_mid(split_k, x, w, epi, out, bias, residual)
         _req(plan.supported(cfg, M, N, K, epi, split_k),
              f"gemm_nt: shape {M}x{N}x{K} epi {epi} split {split_k} unsupported by tile {cfg}")
         width = N // 2 if epi == 1 else N
@@ -633,6 +669,10 @@ def hip_ops() -> SimpleNamespace:
     def linear_silu(x, w):
         """silu(x Wg^T) * (x Wu^T), W = [gate; up] -- K-ACT fused into the gate_up GEMM."""
         M, K = x.shape
+        p = _mid(x, w, 1)
+        if p is not None:
+            _log(M, w.shape[0], K, 1, (MID_CFG, p))
+            return _gemm_mid(p, x, w, 1, torch.empty(M, w.shape[0] // 2, dtype=x.dtype, device=x.device))
         if _skinny(x, w, 1):
             return _gemm_skinny(x, w, 1)
         if not (x.is_contiguous() and x.dtype == torch.bfloat16):
@@ -641,8 +681,12 @@ def hip_ops() -> SimpleNamespace:
         n1 = plan.columns(M, N, K)
         if n1 < N and _plain(x, w):
             out = torch.empty(M, N // 2, dtype=x.dtype, device=x.device)
-            for cfg, at, n in ((W4_CFG, 0, n1), (SMALL_CFG, n1, N - n1)):   # both halves of w from row at / 2 on
-                _log(M, n, K, 1, (cfg, 1))
+            p = plan.mid(M, N - n1, K, 1)
+            for cfg, at, n in ((W4_CFG, 0, n1), ((MID_CFG, p) if p is not None else SMALL_CFG, n1, N - n1)):   # both halves of w from row at / 2 on
+                _log(M, n, K, 1, cfg if isinstance(cfg, tuple) else (cfg, 1))
+                if isinstance(cfg, tuple):
+                    _gemm_mid(p, x, w, 1, out, N=n, at=at)
+                    continue
                 _check(lib.bcg_gemm_nt(cfg, 1, _p(x), w.data_ptr() + at * K, None, None, out.data_ptr() + at, None, None, M, n, K, N // 2,
                                        1, _stream()), "gemm_nt")   # (at / 2 rows or features of 2 bytes)
             return out
@@ -708,6 +752,10 @@ def hip_ops() -> SimpleNamespace:
         """residual <- residual + x W^T (in place; the o/down projection fused with the
         residual-stream update of the next add+RMSNorm).  Returns `residual`."""
         M, K = x.shape
+        p = _mid(x, w, 2)
+        if p is not None and _plain_beside(residual, (M, w.shape[0]), x):
+            _log(M, w.shape[0], K, 2, (MID_CFG, p))
+            return _gemm_mid(p, x, w, 2, residual, residual=residual)
         if _skinny(x, w, 2) and _plain_beside(residual, (M, w.shape[0]), x):
             return _gemm_skinny(x, w, 2, residual=residual)
         parts = [(M, None)]
@@ -858,12 +906,24 @@ def hip_ops() -> SimpleNamespace:
         M, K = xq.shape
         N = wq.shape[0]
         return (plan.mode == "1" and 1 <= M <= 32 and K % 128 == 0 and 128 <= K <= SKINNY_ROW_BYTES and N >= 16 and N % 16 == 0
-                and wq.dim() == 2 and wq.shape[1] == K and (M <= 16 or K <= 8192 or N >= 4096)
+                and (M <= 16 or K <= 8192 or N >= 4096) and _plain_fp8(xq, xs, wq, ws, beside))
+
+    def _plain_fp8(xq, xs, wq, ws, beside):
+        """`_plain` for the fp8 products: operands, their scales and what stands beside them."""
+        return (wq.dim() == 2 and wq.shape[1] == xq.shape[1]
                 and xq.is_cuda and xq.get_device() == torch.cuda.current_device() and xq.is_contiguous() and wq.is_contiguous()
                 and all(t.device == xq.device and t.data_ptr() % 16 == 0 and bare(t) for t in (xq, wq, xs, ws))
-                and xs.dtype == ws.dtype == torch.float32 and xs.numel() == M and ws.numel() == N and xs.is_contiguous()
+                and xs.dtype == ws.dtype == torch.float32 and xs.numel() == xq.shape[0] and ws.numel() == wq.shape[0] and xs.is_contiguous()
                 and ws.is_contiguous() and not watched()
                 and all(t is None or _plain_beside(t, shape, xq) for t, shape in beside))
+
+    def _mid_fp8(xq, xs, wq, ws, *beside):
+        """`_mid` for the fp8 products."""
+        M, K = xq.shape
+        if not (33 <= M <= 1024 and plan.mode == "1"):
+            return None
+        p = lib.bcg_gemm_mid_plan(0, M, wq.shape[0], K, 1)
+        return p if p >= 0 and _plain_fp8(xq, xs, wq, ws, beside) else None
 
     def _gemm_skinny_fp8(xq, xs, wq, ws, epi=0, bias=None, residual=None):
         M, K = xq.shape
@@ -880,6 +940,10 @@ def hip_ops() -> SimpleNamespace:
         _req(xq.dtype == f8 and wq.dtype == f8 and xq.shape[1] == wq.shape[1], "linear_fp8 operands")
         if out_dtype == torch.bfloat16 and _skinny_fp8(xq, xs, wq, ws, (bias, (wq.shape[0],))):
             return _gemm_skinny_fp8(xq, xs, wq, ws, 0, bias)
+        p = _mid_fp8(xq, xs, wq, ws, (bias, (wq.shape[0],))) if out_dtype == torch.bfloat16 else None
+        if p is not None:
+            _log(xq.shape[0], wq.shape[0], xq.shape[1], 0, (MID_CFG, p), "fp8")
+            return _gemm_mid(p, xq, wq, 0, torch.empty(xq.shape[0], wq.shape[0], dtype=torch.bfloat16, device=xq.device), bias, scales=(xs, ws))
         cfg = None
         if out_dtype == torch.bfloat16 and xq.is_contiguous() and wq.is_contiguous():
             cfg = fp8_cfg(xq.shape[0], wq.shape[0], xq.shape[1])
@@ -896,6 +960,10 @@ def hip_ops() -> SimpleNamespace:
              and residual.shape == (xq.shape[0], wq.shape[0]), "linear_fp8_residual: residual [M,N] bf16")
         if xq.dtype == wq.dtype == f8 and _skinny_fp8(xq, xs, wq, ws, (residual, residual.shape)):
             return _gemm_skinny_fp8(xq, xs, wq, ws, 2, residual=residual)
+        p = _mid_fp8(xq, xs, wq, ws, (residual, residual.shape)) if xq.dtype == wq.dtype == f8 else None
+        if p is not None:
+            _log(xq.shape[0], wq.shape[0], xq.shape[1], 2, (MID_CFG, p), "fp8")
+            return _gemm_mid(p, xq, wq, 2, residual, residual=residual, scales=(xs, ws))
         if xq.is_contiguous() and wq.is_contiguous():
             cfg = fp8_cfg(xq.shape[0], wq.shape[0], xq.shape[1])
             if cfg is not None:

@@ -1,0 +1,103 @@
+// Plan and entry points of gemm_mid.h; each epilogue's kernels are a source of their own (they compile side by side).
+#include "gemm_mid.h"
+
+BCG_API int bcg_gemm_mid_gated(int tile, const void* args, hipStream_t stream);
+BCG_API int bcg_gemm_mid_residual(int tile, const void* args, hipStream_t stream);
+BCG_API int bcg_gemm_mid_fp8(int tile, const void* args, hipStream_t stream);
+BCG_API int bcg_gemm_mid_fp8_residual(int tile, const void* args, hipStream_t stream);
+
+namespace {
+
+struct MidTile {
+  int mt, nt, wm;
+};
+constexpr MidTile TILES[] = {
+#define T(i, m, n, w) {m, n, w},
+    MID_TILES(T)
+#undef T
+};
+constexpr int N_TILES = sizeof(TILES) / sizeof(TILES[0]);
+constexpr int CUS = 256;
+
+// Microseconds of a launch of one round, x_rows rows of X (a row tile's share) and bn of W, kb bytes each, a workgroup: fitted (relative least squares,
+// three ranges of rows) to the times of these tiles at 2300 products and checked at 1600 others: the tile chosen by it is 1.7, 2.3 and
+// 3.2 % slower on average than the best of all 72.
+struct Cost {
+  float launch, x_row, w_row, product, hbm, area, split, part, gated_part;
+};
+constexpr Cost COSTS[] = {{3.1f, 10.f, 11.9f, 75.5f, 29.2f, 1.73f, 2.3f, 7.8f, 15.5f},      // up to 128 rows
+                          {3.0f, 8.5f, 11.6f, 55.5f, 37.1f, 1.77f, 2.65f, 8.5f, 17.3f},     // up to 288
+                          {2.75f, 9.6f, 10.6f, 43.4f, 47.4f, 1.93f, 3.3f, 9.f, 17.8f}};
+float predicted(const Cost& c, float x_rows, int bm, int bn, float kb, float w_bytes, int split, bool gated, bool f8) {
+  const float area = static_cast<float>(bm) * bn;
+  const float t = c.launch + (c.x_row * x_rows + c.w_row * bn) * kb * 1e-6f + c.product * area * kb * (f8 ? 1e-9f : 0.5e-9f) +
+                  c.hbm * w_bytes * (1e-6f / CUS) + c.area * area * 1e-4f;
+  return split == 1 ? t : t + c.split + (gated ? c.gated_part : c.part) * split * area * 1e-5f;
+}
+
+}  // namespace
+
+// How x [M, K] w [N, K]^T runs here: tile | split << 8, or -1 where it does not: the product has to fit one round of workgroups
+// (several rounds lose to the persistent 256 x 256 kernel), and W to hold 0.8 M elements (below, a launch of the library or the few-row kernel
+// is shorter, 4.6 to 5.5 us against 5.7 to 7).  33 to 1024 rows, 900 products of 64 to 40000 columns and K of 256 to 18000, this over what took
+// them before (tile kernels, library, few-row kernel): up to 64 rows 0.65, 128: 0.66, 256: 0.70, 512: 0.73, 1024: 0.84 on average; 12 projections of the
+// served models 0.81 to 0.90, the slowest (40 to 64 rows, 7168 x 5120 and 6144 x 4096) 1.1.  fp8, whose other side has matrix
+// instructions of twice the rate: 0.5 to 0.86, but 0.8 to 1.25 from M N K = 15e9 on; bf16 1.0 to 1.18 from 80e9 on.
+BCG_API int bcg_gemm_mid_plan(int epi, int M, int N, int K, int f8) {
+  const bool gated = epi == EPI_SILU_MUL;
+  const int bytes = f8 ? K : 2 * K, inter = N / 2;
+  if (M < 33 || M > 1024 || K <= 0 || bytes % 128 || N < 16 || N % (gated ? 32 : 16) || N > 1 << 20 || (f8 && gated)) return -1;
+  if (static_cast<int64_t>(N) * K < 800000 || static_cast<int64_t>(N) * bytes >= 1ll << 31 || static_cast<int64_t>(M) * bytes >= 1ll << 31) return -1;
+  const Cost& cost = COSTS[M <= 128 ? 0 : M <= 288 ? 1 : 2];
+  if (static_cast<float>(M) * N * K > (f8 ? 15e9f : 80e9f)) return -1;
+  int best = -1;
+  float time = 0.f;
+  for (int i = 0; i < N_TILES; ++i) {
+    const int bm = TILES[i].mt * 16, bn = TILES[i].nt * 16;
+    if (gated && TILES[i].nt % 2) continue;
+    const int m_tiles = (M + bm - 1) / bm, tiles = m_tiles * (gated ? (inter + bn / 2 - 1) / (bn / 2) : (N + bn - 1) / bn);
+    if (tiles > CUS) continue;
+    for (int split : {1, 2, 3, 4, 6, 8}) {
+      // (four of K's 128-byte blocks a split: fewer are all start and end)
+      if (split > 1 && (tiles * split > CUS || bytes / 128 < 4 * split)) break;
+      const float t = predicted(cost, static_cast<float>(M) / m_tiles, bm, bn, static_cast<float>(bytes) / split, static_cast<float>(N) * bytes, split, gated, f8);
+      if (best < 0 || t < time) best = i | split << 8, time = t;
+    }
+  }
+  return best;
+}
+
+// fp32 parts (floats of `ws`) and arrival counters (ints, 0 before and after every launch) of a plan; 0 and 0 without a split
+BCG_API int64_t bcg_gemm_mid_parts(int plan, int epi, int M, int N, int* tiles) {
+  const MidTile t = TILES[plan & 255];
+  const int bn = t.nt * 16, width = epi == EPI_SILU_MUL ? N / 2 : N, cols = epi == EPI_SILU_MUL ? bn / 2 : bn;
+  *tiles = (M + t.mt * 16 - 1) / (t.mt * 16) * ((width + cols - 1) / cols);
+  return plan >> 8 > 1 ? static_cast<int64_t>(*tiles) * (plan >> 8) * t.mt * 16 * bn : 0;
+}
+
+// plan: of bcg_gemm_mid_plan for the same sizes, or any other tile and split.  epi: 0 store (+ bias), 1 silu(gate) * up of N / 2 features from w's first
+// row on, their up rows `inter` rows behind, into rows of `c` that are `inter` apart, 2 residual + product (residual may be c).  x_scale [M],
+// w_scale [N]: not null for e4m3 operands (epi 0 and 2).  Pointers 16-byte aligned, rows contiguous; ws and counters as
+// bcg_gemm_mid_parts says.
+BCG_API int bcg_gemm_mid(int plan, int epi, const void* x, const void* w, const float* x_scale, const float* w_scale, const void* bias,
+                         const void* residual, void* c, void* ws, void* counters, int M, int N, int K, int inter, hipStream_t stream) {
+  const bool f8 = x_scale != nullptr, gated = epi == EPI_SILU_MUL;
+  const int bytes = f8 ? K : 2 * K, split = plan >> 8, tile = plan & 255;
+  if (plan < 0 || tile >= N_TILES || M <= 0 || K <= 0 || bytes % 128 || N <= 0 || N % (gated ? 32 : 16) || N > 1 << 20) return -2;
+  if (split < 1 || split > bytes / 128 || (split > 1 && (!ws || !counters)) || (f8 && !w_scale)) return -2;
+  if (gated && (inter < N / 2 || inter % 16 || inter > 1 << 20)) return -2;
+  if (static_cast<int64_t>(gated ? 2 * inter : N) * bytes >= 1ll << 31 || static_cast<int64_t>(M) * bytes >= 1ll << 31) return -2;
+  const int bm = TILES[tile].mt * 16, bn = TILES[tile].nt * 16;
+  const MidArgs a = {static_cast<const unsigned char*>(x), static_cast<const unsigned char*>(w), static_cast<const bf16_t*>(bias),
+                     static_cast<const bf16_t*>(residual), static_cast<bf16_t*>(c), static_cast<float*>(ws), static_cast<int*>(counters),
+                     x_scale, w_scale, M, N, inter, bytes / 128, (M + bm - 1) / bm, gated ? (N / 2 + bn / 2 - 1) / (bn / 2) : (N + bn - 1) / bn, split};
+  if (static_cast<int64_t>(a.m_tiles) * a.n_tiles * split > 1 << 24 || static_cast<int64_t>(a.m_tiles) * a.n_tiles > 1 << 16) return -2;
+  switch (epi) {
+    case EPI_STORE: return f8 ? bcg_gemm_mid_fp8(tile, &a, stream) : launch<EPI_STORE, false>(tile, a, stream);
+    case EPI_SILU_MUL: return f8 ? -2 : bcg_gemm_mid_gated(tile, &a, stream);
+    case EPI_RESIDUAL:
+      if (!residual) return -2;
+      return f8 ? bcg_gemm_mid_fp8_residual(tile, &a, stream) : bcg_gemm_mid_residual(tile, &a, stream);
+    default: return -2;
+  }
+}

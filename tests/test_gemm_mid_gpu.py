@@ -1,0 +1,125 @@
+"""The kernel for tens to hundreds of rows (csrc/kernels/gemm_mid.hip): every tile and split at sizes where it can go wrong, against a product in
+float32; the plan over the sizes that it takes (CPU)."""
+
+import ctypes
+import os
+import random
+
+import pytest
+import torch
+
+from byzantine_consensus_llm_agents_amd.ops.gemm_plan import MID_CFG, GemmPlan
+from byzantine_consensus_llm_agents_amd.utils.build import kernels_target
+
+# (row blocks, column blocks) of the tiles, in the kernel's order
+TILES = [(3, 1), (3, 2), (3, 3), (3, 4), (3, 6), (4, 2), (4, 3), (4, 4), (4, 5), (5, 4), (5, 5), (5, 6), (6, 4), (6, 6), (8, 4), (8, 5),
+         (4, 8), (4, 10), (6, 8), (6, 10), (8, 6), (8, 10), (10, 6), (10, 8), (10, 12), (12, 10), (14, 8), (16, 8)]
+TOL = 4e-3   # one rounding to bf16 of the result: 2^-9 relative, 0.58 of it on average; sums of 32 bits add less than 1e-5
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from byzantine_consensus_llm_agents_amd.ops import get_ops
+    return get_ops("hip")
+
+
+def _err(a, b):
+    return ((a.float() - b).norm() / b.norm()).item()
+
+
+def _run(ops, plan, epi, x, w, out, bias=None, residual=None, scales=(None, None)):
+    lib, tiles = ops.library, ctypes.c_int()
+    (M, K), N = x.shape, w.shape[0]
+    ws = torch.empty(max(1, lib.bcg_gemm_mid_parts(plan, epi, M, N, ctypes.byref(tiles))), device="cuda")
+    cnt = torch.zeros(max(1, tiles.value), dtype=torch.int32, device="cuda")
+    ptr = [None if t is None else ctypes.c_void_p(t.data_ptr()) for t in (x, w, *scales, bias, residual, out, ws, cnt)]
+    assert lib.bcg_gemm_mid(plan, epi, *ptr, M, N, K, N // 2, torch.cuda.current_stream().cuda_stream) == 0
+    assert not cnt.any()
+    return out
+
+
+# rows: one, a tile's last, its first of a second one; columns not a multiple of the tile; K: one block, odd numbers of blocks, splits of unequal length
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", range(len(TILES)), ids=[f"{16 * m}x{16 * n}" for m, n in TILES])
+def test_every_tile(ops, tile):
+    mt, nt = TILES[tile]
+    torch.manual_seed(tile)
+    for M, N, K, split in ((1, 16, 64, 1), (16 * mt, 16 * nt, 320, 1), (16 * mt + 1, 32 * nt + 16, 704, 3), (16 * mt - 7, 16 * nt + 32, 1088, 2)):
+        x = torch.randn(M, K, device="cuda").bfloat16()
+        w = (torch.randn(N, K, device="cuda") * K ** -0.5).bfloat16()
+        bias, res = torch.randn(N, device="cuda").bfloat16(), torch.randn(M, N, device="cuda").bfloat16()
+        y = x.float() @ w.float().t()
+        plan = tile | split << 8
+        nan = lambda n: torch.full((M, n), float("nan"), dtype=torch.bfloat16, device="cuda")   # noqa: E731
+        assert _err(_run(ops, plan, 0, x, w, nan(N), bias=bias), y + bias.float()) < TOL
+        assert _err(_run(ops, plan, 2, x, w, res.clone(), residual=res), y + res.float()) < TOL
+        if N % 32 == 0 and nt % 2 == 0:
+            want = torch.nn.functional.silu(y[:, :N // 2]) * y[:, N // 2:]
+            assert _err(_run(ops, plan, 1, x, w, nan(N // 2)), want) < TOL
+        if K % 128 == 0:
+            xq, wq = x.to(torch.float8_e4m3fn), (w * 8).to(torch.float8_e4m3fn)
+            xs, ws = torch.rand(M, device="cuda") + 0.5, (torch.rand(N, device="cuda") + 0.5) / 8
+            y8 = xq.float() @ wq.float().t() * xs[:, None] * ws
+            assert _err(_run(ops, plan, 0, xq, wq, nan(N), bias=bias, scales=(xs, ws)), y8 + bias.float()) < TOL
+            assert _err(_run(ops, plan, 2, xq, wq, res.clone(), residual=res, scales=(xs, ws)), y8 + res.float()) < TOL
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [33, 100, 1024])
+def test_entry_points_take_it_and_replay(ops, M):
+    """A captured sequence of the three entry points, replayed on other inputs with eager calls between, gives what eager calls give; the operands
+    that the library has to see do not come here."""
+    torch.manual_seed(M)
+    K, N = 1152, 2048
+    x, res = torch.randn(M, K, device="cuda").bfloat16(), torch.randn(M, N, device="cuda").bfloat16()
+    w = (torch.randn(N, K, device="cuda") * K ** -0.5).bfloat16()
+    ops.prepare_device("cuda")
+    assert ops.gemm_plan.mid(M, N, K, 0) is not None
+
+    def step(r):
+        return ops.linear(x, w), ops.linear_silu(x, w), ops.linear_residual(x, w, r)
+    step(res.clone())
+    r = res.clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = step(r)
+    for _ in range(3):
+        x.normal_()
+        r.copy_(res)
+        want = [t.clone() for t in step(res.clone())]
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+        assert _err(want[0], x.float() @ w.float().t()) < TOL
+    xg = x.clone().requires_grad_()
+    ops.linear(xg, w).sum().backward()
+    assert xg.grad is not None
+
+
+def test_plan_takes_one_round_and_refuses_the_rest():
+    if not os.path.exists(kernels_target()):
+        pytest.skip("kernels not built")
+    lib = ctypes.CDLL(kernels_target())
+    lib.bcg_gemm_mid_parts.restype = ctypes.c_int64
+    rng, taken = random.Random(0), 0
+    for _ in range(3000):
+        M, N, K, epi, f8 = rng.randint(1, 1500), 8 * rng.randint(1, 5000), 32 * rng.randint(1, 600), rng.randrange(3), rng.randrange(2)
+        p = lib.bcg_gemm_mid_plan(epi, M, N, K, f8)
+        if p < 0:
+            continue
+        taken += 1
+        assert 33 <= M <= 1024 and N % (32 if epi == 1 else 16) == 0 and K % (128 if f8 else 64) == 0 and not (f8 and epi == 1)
+        mt, nt = TILES[p & 255]
+        assert epi != 1 or nt % 2 == 0
+        tiles = ctypes.c_int()
+        floats = lib.bcg_gemm_mid_parts(p, epi, M, N, ctypes.byref(tiles))
+        assert tiles.value == -(-M // (16 * mt)) * -(-N // (16 * nt)) and tiles.value * (p >> 8) <= 256
+        assert floats == (0 if p >> 8 == 1 else tiles.value * (p >> 8) * 256 * mt * nt)
+        assert K * (1 if f8 else 2) // 128 >= (p >> 8)
+    assert taken > 50
+    assert GemmPlan().mid(100, 4096, 4096, 0) is None     # (no library: no plan)
+    plan = GemmPlan(lib)
+    assert plan._rest(300, 4096, 4096, 0)[0] == MID_CFG
+    for bad in ((0, 32, 4096, 4096, 0), (0, 1025, 4096, 4096, 0), (0, 100, 4096, 4100, 0), (0, 100, 4104, 4096, 0), (1, 100, 4112, 4096, 0),
+                (0, 100, 4096, 64, 0), (0, 1024, 151936, 5120, 0), (1, 100, 4096, 4096, 1)):
+        assert lib.bcg_gemm_mid_plan(*bad) == -1, bad
