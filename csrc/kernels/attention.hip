@@ -383,6 +383,7 @@ struct Causal {
 // most of its workgroups reading seq_lens only to exit: 78 % of the launch at
 // B = 160, ctx 1700, max_model_len 8192.
 constexpr int DEC_MAX_B = 2048;
+constexpr int DEC_MAX_SHARED_SPLITS = 16;   // slots of the shared-prefix pass (bcg_decode_max_splits)
 
 //
 // Shared-prefix (cascade) form: rows whose leading blocks are the SAME physical blocks
@@ -455,21 +456,271 @@ __device__ __forceinline__ void load_head(u16x8 (&raw)[HD / 32], const bf16_t* r
 #pragma unroll
   for (int kk = 0; kk < HD / 32; ++kk) raw[kk] = *reinterpret_cast<const u16x8*>(row + kk * 32 + h * 8);
 }
-template <int HD, bool F8 = false, int CPW = 1, bool FUSED = false>
-__global__ __launch_bounds__(256) void decode_attn_kernel(
+// ------------------------------------------------------- decode, streamed
+// What the kernel below does when its items are more than one round of workgroups: every wave takes an even share of ALL chunks of the batch, pairs
+// (row, kv head) in order, their 32-token chunks in order, cut into as many ranges as there are waves.  A wave's K/V comes by LDS-DMA into 16
+// KB of its own: K of the next chunk is fetched when this one's is in registers, V likewise, across pairs, so no fetch waits
+// for a pair's table, queries or merge and no wave for another.  What bounds the items (4.6 TB/s at 448 rows of 1050 tokens, heads of 128): between two
+// of them the chain of table, loads and merge leaves the memory idle, and the registers hold one item's loads.  A page of K or V is 4 KB
+// in one piece, and a pair is cut where a range ends, not every 256 tokens: fewer parts to store and merge.
+// 448 rows of 8 kv heads, us for items -> this: 60 tokens 51 -> 44, 250 121 -> 114, 1050 418 -> 370 to 380 (5.2 TB/s, merge and all), 160 rows of 2500
+// 340 -> 303, 64 rows of 1050 67 -> 62.  Two chunks ahead with one workgroup a CU (32 KB a wave) is level.
+constexpr int STREAM_G = 8;           // query heads of a kv head
+constexpr int STREAM_RING = 16384;    // bytes of a wave's chunk: K, then V
+constexpr int STREAM_Q = STREAM_G * 256;
+constexpr int STREAM_LDS = 4 * (STREAM_RING + 2 * STREAM_Q);   // two workgroups a CU
+
+// The wave that chunk c of the batch falls to, of `waves` that share `total` chunks: wave w has those from w total / waves on
+__device__ __forceinline__ int stream_wave(int c, int total, int waves) {
+  return static_cast<int>(((static_cast<uint64_t>(c) + 1) * waves - 1) / total);
+}
+
+// stream (out, by the first workgroup; read by the merge): [B + 1] chunks of the rows before, [1] waves that share them
+__device__ __forceinline__ void decode_stream(
+    unsigned char* smem, const bf16_t* q, const KVGeom& g, const int* block_tables, int max_blocks, const int* seq_lens, int B, int n_q,
+    float scale_log2, float* part_o, float* part_ml, int max_splits, const int* kv_begin, const int* split_base, int* stream) {
+  constexpr int HD = 128;
+  static_assert(sizeof(int) * (DEC_MAX_B + 1 + 8) <= STREAM_LDS, "the row table lies where the ring is later");
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, h = lane >> 4;
+  const int G = n_q / g.n_kv, slots = max(2, max_splits - (kv_begin ? DEC_MAX_SHARED_SPLITS : 0));
+  auto own_chunks = [&](int b) { return (max(0, seq_lens[b] - (kv_begin ? kv_begin[b] : 0)) + CHUNK - 1) / CHUNK; };
+
+  // ---- chunks of the rows before each row, and this wave's range ----
+  int b, n, kvh, c, left;          // row, its chunks a head; head; chunk in the pair; chunks of the range
+  int part;                        // which part of its pair the wave's first one is
+  int gw;                          // its range
+  {
+    int* pre = reinterpret_cast<int*>(smem);
+    int* wsum = pre + DEC_MAX_B + 1;
+    constexpr int PER_MAX = DEC_MAX_B / 256;
+    const int rows = (B + 255) / 256;
+    int cnt[PER_MAX], sum = 0, longest = 0;
+#pragma unroll
+    for (int j = 0; j < PER_MAX; ++j) {
+      const int i = tid * rows + j;
+      cnt[j] = j < rows && i < B ? own_chunks(i) : 0;
+      sum += cnt[j];
+      longest = max(longest, cnt[j]);
+    }
+    longest = wave_max(longest);
+    int incl = sum;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(incl, o, WAVE);
+      if (lane >= o) incl += v;
+    }
+    if (lane == 63) wsum[w] = incl, wsum[4 + w] = longest;
+    __syncthreads();
+    for (int ww = 0; ww < 4; ++ww) longest = max(longest, wsum[4 + ww]);
+    int base = incl - sum;
+    for (int ww = 0; ww < w; ++ww) base += wsum[ww];
+#pragma unroll
+    for (int j = 0; j < PER_MAX; ++j) {
+      const int i = tid * rows + j;
+      if (j < rows && i < B) pre[i] = base;
+      base += cnt[j];
+    }
+    if (tid == 255) pre[B] = base;
+    __syncthreads();
+    const int total = pre[B] * g.n_kv;
+    // ranges are so long that a pair of n chunks, cut into (n - 2) / shortest + 2 parts at most, has a slot for each
+    const int shortest = max(1, (longest + slots - 2) / (slots - 1));
+    const int waves = max(1, min(static_cast<int>(gridDim.x) * 4, total / shortest));
+    if (blockIdx.x == 0) {
+      for (int i = tid; i <= B; i += 256) stream[i] = pre[i];
+      if (tid == 0) stream[B + 1] = waves;
+    }
+    // (neighbouring ranges to the waves of a workgroup: their pages lie side by side; fewer ranges than waves: spread evenly)
+    const int at = static_cast<int>(blockIdx.x) * 4 + w, all = gridDim.x * 4;
+    gw = at * waves / all;
+    const int start = static_cast<int>(static_cast<uint64_t>(gw) * total / waves);
+    left = at == 0 || (at - 1) * waves / all != gw ? static_cast<int>((static_cast<uint64_t>(gw) + 1) * total / waves) - start : 0;
+    int lo = 0, hi = B - 1;   // the last row that starts at or before `start`
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (pre[mid] * g.n_kv <= start) lo = mid; else hi = mid - 1;
+    }
+    b = lo;
+    n = pre[lo + 1] - pre[lo];
+    const int in = start - pre[lo] * g.n_kv;
+    kvh = n > 0 ? in / n : 0;
+    c = in - kvh * n;
+    part = left > 0 ? gw - stream_wave(start - c, total, waves) : 0;
+    b = __builtin_amdgcn_readfirstlane(b), n = __builtin_amdgcn_readfirstlane(n), kvh = __builtin_amdgcn_readfirstlane(kvh);
+    c = __builtin_amdgcn_readfirstlane(c), part = __builtin_amdgcn_readfirstlane(part);
+    left = __builtin_amdgcn_readfirstlane(left);
+    __syncthreads();          // the table is read: the ring may be filled
+  }
+  if (left <= 0) return;      // (no barrier below)
+
+  // ---- fetches.  K piece i of page e: rows 4 i + lane / 16, their 16-byte chunk x at place x ^ f with f = 8 e + 4 (i / 2) + lane / 16, so that the
+  // 16 rows of a fragment read hit 16 places; V^T piece i: rows 32 i + lane / 2, halves swapped where bit 3 of the row is set.
+  uint32_t off_k[2][4], off_v[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e) off_k[e][i] = (4 * i + h) * 256 + ((r ^ (8 * e + 4 * (i >> 1) + h)) << 4);
+    off_v[i] = i * 1024 + (lane >> 1) * 32 + (((lane ^ (lane >> 4)) & 1) << 4);
+  }
+  const uint32_t lds = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem));
+  const uint32_t ring = lds + w * STREAM_RING, qring = lds + 4 * STREAM_RING + w * 2 * STREAM_Q;
+  auto dma = [&](uint32_t off, const unsigned char* base, uint32_t to) {
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(to) : "memory", "m0");
+  };
+  const unsigned char* kc = reinterpret_cast<const unsigned char*>(g.k);
+  const unsigned char* vc = reinterpret_cast<const unsigned char*>(g.v);
+  auto page = [&](int blk, int head) {
+    return ((static_cast<size_t>(g.layer) * g.num_blocks + blk) * g.n_kv + head) * (BS * HD * 2);
+  };
+  // (constant address space: scalar loads.  Behind the asm of the fetches hipcc takes vector loads for them, whose wait drains the ring.)
+  typedef const __attribute__((address_space(4))) int* Ints;
+  auto ints = [](const int* p) { return reinterpret_cast<Ints>(reinterpret_cast<uintptr_t>(p)); };
+  const Ints lens = ints(seq_lens), begins = ints(kv_begin), tables = ints(block_tables), bases = ints(split_base);
+  struct Row {
+    Ints table;   // from the row's first own block on
+    int ctx, begin, last, n;   // tokens, first own token, last entry of `table`, chunks a head
+  };
+  auto row = [&](int i) {
+    Row x;
+    x.begin = kv_begin ? begins[i] : 0;
+    x.ctx = lens[i];
+    x.table = tables + static_cast<size_t>(i) * max_blocks + x.begin / BS;
+    x.last = (x.ctx - 1) / BS - x.begin / BS;
+    x.n = (max(0, x.ctx - x.begin) + CHUNK - 1) / CHUNK;
+    return x;
+  };
+  struct Cursor {
+    Row x;
+    int b, kvh, c, pair;
+  };
+  auto advance = [&](Cursor& k) {
+    if (++k.c < k.x.n) return;
+    k.c = 0;
+    k.pair ^= 1;
+    if (++k.kvh < g.n_kv) return;
+    k.kvh = 0;
+    do {   // (only called with chunks left: a row that has some follows)
+      ++k.b;
+      k.x = row(k.b);
+    } while (k.x.n == 0 && k.b < B - 1);
+  };
+  Cursor use = {row(b), b, kvh, c, 0}, get = use;
+  int togo = left;            // chunks not yet fetched
+  int blk0 = 0, blk1 = 0;     // pages of the chunk that is fetched next
+  auto look = [&]() {
+    blk0 = get.x.table[2 * get.c];
+    blk1 = get.x.table[min(2 * get.c + 1, get.x.last)];
+  };
+  auto fetch_k = [&](bool fresh) {
+    if (get.c == 0 || fresh) {   // the pair's queries (rows past the heads repeat the last and are not used)
+      const unsigned char* qs = reinterpret_cast<const unsigned char*>(q + (static_cast<size_t>(get.b) * n_q + get.kvh * G) * HD);
+      dma(min(h, G - 1) * 256 + r * 16, qs, qring + get.pair * STREAM_Q);
+      if (G > 4) dma(min(4 + h, G - 1) * 256 + r * 16, qs, qring + get.pair * STREAM_Q + 1024);
+    }
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) dma(off_k[e][i], kc + page(e ? blk1 : blk0, get.kvh), ring + e * 4096 + i * 1024);
+  };
+  auto fetch_v = [&]() {
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) dma(off_v[i], vc + page(e ? blk1 : blk0, get.kvh), ring + 8192 + e * 4096 + i * 1024);
+    --togo;
+    if (togo > 0) {
+      advance(get);
+      look();
+    }
+  };
+
+  look();
+  fetch_k(true);
+  fetch_v();
+
+  const unsigned char* rk = smem + w * STREAM_RING + (8 * (r >> 2) + (r & 3)) * 256;
+  const unsigned char* rv = smem + w * STREAM_RING + 8192 + (h >> 1) * 4096 + r * 32 + (((h ^ (r >> 3)) & 1) << 4);
+  bf16x8 bq[HD / 32];
+  float m = -INFINITY, l = 0.f;
+  f32x4 o[HD / 16];
+  bool fresh = true;
+  for (; left > 0; --left) {
+    Chunk<HD> x;
+    asm volatile("s_waitcnt vmcnt(8)" ::: "memory");   // all but this chunk's V (stores among them only make the wait longer)
+    if (fresh) {
+      const unsigned char* rq = smem + 4 * STREAM_RING + (w * 2 + use.pair) * STREAM_Q + (r & 7) * 256 + h * 16;
+#pragma unroll
+      for (int kk = 0; kk < HD / 32; ++kk) {
+        bf16x8 v = *reinterpret_cast<const bf16x8*>(rq + kk * 64);
+        bq[kk] = r < G ? v : bf16x8{};
+      }
+      m = -INFINITY, l = 0.f;
+#pragma unroll
+      for (int dt = 0; dt < HD / 16; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+      fresh = false;
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int kk = 0; kk < HD / 32; ++kk) x.k[u][kk] = *reinterpret_cast<const bf16x8*>(rk + u * 1024 + (((kk * 4 + h) ^ r) << 4));
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (togo > 0) {
+      fetch_k(false);
+      asm volatile("s_waitcnt vmcnt(8)" ::: "memory");   // all but the next chunk's K
+    } else {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+#pragma unroll
+    for (int dt = 0; dt < HD / 16; ++dt) x.v[dt] = *reinterpret_cast<const bf16x8*>(rv + dt * 512);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (togo > 0) fetch_v();
+    const int tj = use.x.begin + use.c * CHUNK;
+    if (tj + CHUNK <= use.x.ctx)  // wave-uniform: a full chunk needs no tail masking
+      compute_chunk<HD, AllVisible, false>(x, bq, tj, use.x.ctx, AllVisible{}, scale_log2, m, l, o, lane);
+    else
+      compute_chunk<HD, AllVisible, true>(x, bq, tj, use.x.ctx, AllVisible{}, scale_log2, m, l, o, lane);
+    if (left == 1 || use.c + 1 == use.x.n) {   // the pair or the range ends
+      if (r < G) {
+        const size_t at = (static_cast<size_t>(use.b) * n_q + use.kvh * G + r) * max_splits + (split_base ? bases[use.b] : 0) + part;
+#pragma unroll
+        for (int dt = 0; dt < HD / 16; ++dt) *reinterpret_cast<f32x4*>(part_o + at * HD + dt * 16 + 4 * h) = o[dt];
+        if (h == 0) *reinterpret_cast<float2*>(part_ml + at * 2) = float2{m, l};
+      }
+      part = 0;
+      fresh = true;
+    }
+    if (left > 1) advance(use);
+  }
+}
+
+template <int HD>
+struct ItemShared {
+  int pre[DEC_MAX_B + 1];
+  int wsum[DEC_WAVES];
+  float ml[DEC_WAVES][2][16];
+  float o[DEC_WAVES][HD][16 + 1];
+};
+// STREAM: a step of more items than workgroups is streamed (heads of 128 in bf16)
+template <int HD, bool F8 = false, int CPW = 1, bool FUSED = false, bool STREAM = false>
+__global__ __launch_bounds__(256, (STREAM ? 2 : 1)) void decode_attn_kernel(
     const bf16_t* __restrict__ q, KVGeom g, const int* __restrict__ block_tables, int max_blocks,
     const int* __restrict__ seq_lens, int B, int n_q, float scale_log2, float* __restrict__ part_o,
     float* __restrict__ part_ml, int max_splits, const int* __restrict__ kv_begin,
-    const int* __restrict__ split_base, FusedArgs fa) {
+    const int* __restrict__ split_base, FusedArgs fa, int* __restrict__ stream) {
   static_assert(!FUSED || (HD == 64 && !F8), "fused: see FusedArgs");
+  static_assert(!STREAM || (HD == 128 && !F8 && !FUSED), "streamed: decode_stream");
   // CPW chunks per wave: an item covers DEC_WAVES * CPW * 32 tokens; every chunk's loads of
   // a wave are issued before its first MFMA (CPW x 16 loads in flight per wave), and the
   // split partials / merge traffic shrink by CPW
   constexpr int DEC_SPLIT = DEC_WAVES * CHUNK * CPW;
-  __shared__ int s_pre[DEC_MAX_B + 1];
-  __shared__ int s_wsum[DEC_WAVES];
-  __shared__ float s_ml[DEC_WAVES][2][16];
-  __shared__ float s_o[DEC_WAVES][HD][16 + 1];
+  constexpr int LDS = STREAM ? std::max<int>(STREAM_LDS, sizeof(ItemShared<HD>)) : sizeof(ItemShared<HD>);
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[LDS];
+  ItemShared<HD>& shared = *reinterpret_cast<ItemShared<HD>*>(smem);
+  auto &s_pre = shared.pre;
+  auto &s_wsum = shared.wsum;
+  auto &s_ml = shared.ml;
+  auto &s_o = shared.o;
   const int tid = threadIdx.x, lane = tid & 63, w = FUSED ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
   const int r = lane & 15, h = lane >> 4;
   const int G = n_q / g.n_kv;
@@ -507,6 +758,16 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
     __syncthreads();
   }
   const int n_items = s_pre[B] * g.n_kv;
+  if constexpr (STREAM) {
+    // One round of items is shorter (16 rows, 2 kv heads, 250 to 1700 tokens: 11.5 to 14 us, streamed 15 to 18), more than one are not (from 590
+    // items on 0.84 to 0.99 of the time, 480 still 1.1): only the device knows the contexts.
+    if (n_items > static_cast<int>(gridDim.x)) {
+      __syncthreads();
+      decode_stream(smem, q, g, block_tables, max_blocks, seq_lens, B, n_q, scale_log2, part_o, part_ml, max_splits, kv_begin, split_base, stream);
+      return;
+    }
+    if (blockIdx.x == 0 && tid == 0) stream[B + 1] = 0;
+  }
 
   for (int item = blockIdx.x; item < n_items; item += gridDim.x) {
     const int pos = item / g.n_kv, kvh = item - pos * g.n_kv;
@@ -675,17 +936,27 @@ template <int HD>
 __global__ __launch_bounds__(64 * COMBINE_WAVES) void decode_combine_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_ml, const int* __restrict__ seq_lens, int n_q,
     int max_splits, int split_tokens, int n_bq, bf16_t* __restrict__ out, const int* __restrict__ kv_begin,
-    const int* __restrict__ split_base) {
+    const int* __restrict__ split_base, const int* __restrict__ stream, int B, int n_kv) {
   constexpr int PER = HD / 64;  // dims per lane
   const int lane = threadIdx.x & 63;
   const int bq = blockIdx.x * COMBINE_WAVES + (threadIdx.x >> 6);
   if (bq >= n_bq) return;  // wave-uniform
   const int b = bq / n_q;
+  // every slot's (m, l), before the number of parts is known: what the loads below say arrives at the same time
+  float2 mlv = lane < max_splits ? reinterpret_cast<const float2*>(part_ml)[static_cast<size_t>(bq) * max_splits + lane]
+                                 : float2{-INFINITY, 0.f};
   const int own = max(0, seq_lens[b] - (kv_begin ? kv_begin[b] : 0));
   // <= max_splits <= 64 (host check); slots 0 .. split_base[b]-1 hold the shared-prefix partials
-  const int ns = (split_base ? split_base[b] : 0) + (own + split_tokens - 1) / split_tokens;
-  const float2 mlv = lane < ns ? reinterpret_cast<const float2*>(part_ml)[static_cast<size_t>(bq) * max_splits + lane]
-                               : float2{-INFINITY, 0.f};
+  int parts = (own + split_tokens - 1) / split_tokens;
+  int waves = 0, first = 0, next = 0, total = 0;
+  if (stream != nullptr) waves = stream[B + 1], first = stream[b], next = stream[b + 1], total = stream[B] * n_kv;
+  if (waves > 0) {  // decode_stream: how its waves' ranges cut the pair's chunks
+    const int n = next - first;
+    const int c0 = first * n_kv + (bq - b * n_q) / (n_q / n_kv) * n;
+    parts = n > 0 ? stream_wave(c0 + n - 1, total, waves) - stream_wave(c0, total, waves) + 1 : 0;
+  }
+  const int ns = (split_base ? split_base[b] : 0) + parts;
+  if (lane >= ns) mlv = float2{-INFINITY, 0.f};
   float mm = mlv.x;
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) mm = fmaxf(mm, __shfl_xor(mm, o, 64));
@@ -861,21 +1132,34 @@ void launch_decode(const bf16_t* q, KVGeom g, const int* tables, int max_blocks,
                        cas.items, cas.n_items, cas.max_items, cas.split_tokens, part_o, part_ml, max_splits);
   }
   // fixed (graph-safe) grid striding over the live items: one full wave of resident workgroups
-  static int resident = 0;
-  if (resident == 0) {
-    int per_cu = 0, cus = 0, dev = 0;
-    hipGetDevice(&dev);
-    hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, decode_attn_kernel<HD, F8, CPW, FUSED>, 256, 0);
-    resident = std::max(1, per_cu) * std::max(1, cus);
+  auto run = [&](auto stream_c, int* table) {
+    constexpr bool STREAM = decltype(stream_c)::value;
+    static int resident = 0;
+    if (resident == 0) {
+      int per_cu = 0, cus = 0, dev = 0;
+      hipGetDevice(&dev);
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, decode_attn_kernel<HD, F8, CPW, FUSED, STREAM>, 256, 0);
+      resident = std::max(1, per_cu) * std::max(1, cus);
+    }
+    const int grid = static_cast<int>(std::min<long>(static_cast<long>(B) * g.n_kv * max_splits, resident));
+    hipLaunchKernelGGL((decode_attn_kernel<HD, F8, CPW, FUSED, STREAM>), dim3(grid), dim3(256), 0, stream, q, g, tables, max_blocks,
+                       seq_lens, B, n_q, sl, part_o, part_ml, max_splits, cas.kv_begin, cas.split_base, fa, table);
+  };
+  // Streamed from 256 pairs of row and kv head on: below them the items rarely are more than a round, and the merge's look at how the batch was
+  // cut costs 0.4 us (10 rows of 8 kv heads 2 to 5 % of 9 to 25 us; 256 pairs: 60 tokens +0.5 us, 250 +0.5, 1050 -0.9, 2500 -4).
+  int* table = nullptr;
+  if constexpr (HD == 128 && !F8 && !FUSED) {
+    // (its table lies behind the partials; with one slot a row's range could be cut into more parts than there are slots)
+    if (n_q / g.n_kv <= STREAM_G && B * g.n_kv >= 256 && max_splits - (cas.kv_begin ? DEC_MAX_SHARED_SPLITS : 0) >= 2)
+      table = reinterpret_cast<int*>(part_ml + static_cast<size_t>(B) * n_q * max_splits * 2);
+    if (table != nullptr) run(std::true_type{}, table);
   }
-  const int grid = static_cast<int>(std::min<long>(static_cast<long>(B) * g.n_kv * max_splits, resident));
-  hipLaunchKernelGGL((decode_attn_kernel<HD, F8, CPW, FUSED>), dim3(grid), dim3(256), 0, stream, q, g, tables, max_blocks,
-                     seq_lens, B, n_q, sl, part_o, part_ml, max_splits, cas.kv_begin, cas.split_base, fa);
+  if (table == nullptr) run(std::false_type{}, nullptr);
   const int n_bq = B * n_q;
   hipLaunchKernelGGL(decode_combine_kernel<HD>, dim3((n_bq + COMBINE_WAVES - 1) / COMBINE_WAVES),
                      dim3(64 * COMBINE_WAVES), 0, stream, part_o, part_ml, seq_lens, n_q, max_splits, DEC_SPLIT, n_bq,
-                     out, cas.kv_begin, cas.split_base);
+                     out, cas.kv_begin, cas.split_base, table, B, g.n_kv);
 }
 
 // ----------------------------------------------------------------- prefill
@@ -1484,10 +1768,11 @@ BCG_API int bcg_decode_split_tokens(int B, int n_kv, int max_tokens) { return DE
 // shared-prefix pass (engine/cascade.py keeps shared tokens / its split within it).
 // Only calls with the cascade tables reserve the shared slots (cascade = 0: a plain decode keeps
 // the combine kernel's 64-split limit for its own splits, i.e. 16384 tokens of context).
-constexpr int DEC_MAX_SHARED_SPLITS = 16;
 BCG_API int bcg_decode_max_splits(int max_tokens, int cascade) {
-  const int split = DEC_WAVES * CHUNK * DEC_CPW;
-  return (max_tokens + split - 1) / split + (cascade ? DEC_MAX_SHARED_SPLITS : 0);
+  const int split = DEC_WAVES * CHUNK * DEC_CPW, own = (max_tokens + split - 1) / split, most = 64 - (cascade ? DEC_MAX_SHARED_SPLITS : 0);
+  // one more for a row that a range of the streamed kernel cuts off its beat (its ranges are longer than a split: at the limit of 64 it
+  // needs fewer than the splits)
+  return (own < most ? own + 1 : own) + (cascade ? DEC_MAX_SHARED_SPLITS : 0);
 }
 // Longest context a decode call supports (the combine kernel reads at most 64 splits per row).
 BCG_API int bcg_decode_max_context(int cascade) {
