@@ -23,6 +23,7 @@ PREFILL32_MAX_BLOCKS = 1024  # csrc/kernels/attention.hip: the 32x32 kernel's LD
 
 # csrc/kernels/gemm_skinny.hip: most rows, most rows with a fused norm, longest rows in bytes
 SKINNY_ROWS, SKINNY_NORM_ROWS, SKINNY_ROW_BYTES = 64, 16, 65536
+MID_ROWS = 2047  # csrc/kernels/gemm_mid.hip: most rows
 SKINNY_LONG_K = 12288  # past it: fewer shapes gain (`few_rows_pay`), logged apart
 
 c_int, c_float, c_void_p, c_uint32, c_int64 = ctypes.c_int, ctypes.c_float, ctypes.c_void_p, ctypes.c_uint32, ctypes.c_int64
@@ -494,7 +495,7 @@ def hip_ops() -> SimpleNamespace:
         sizes, the slowest 1.1: 40 rows, 6144 x 4096); smaller ones stay where the tests of that kernel hold them (0.77 to 0.82)."""
         M, K = x.shape
         N = w.shape[0]
-        if not (33 <= M <= 1024 and plan.mode == "1") or (M <= SKINNY_ROWS and N * K < 2700000 and few_rows_pay(M, N, 2 * K, epi == 1)):
+        if not (33 <= M <= MID_ROWS and plan.mode == "1") or (M <= SKINNY_ROWS and N * K < 2700000 and few_rows_pay(M, N, 2 * K, epi == 1)):
             return None
         p = plan.mid(M, N, K, epi)
         return p if p is not None and _plain(x, w) else None
@@ -509,7 +510,9 @@ def hip_ops() -> SimpleNamespace:
             tiles = c_int()
             ws = torch.empty(lib.bcg_gemm_mid_parts(p, epi, M, N, ctypes.byref(tiles)), dtype=torch.float32, device=x.device)
             _req(tiles.value <= 1 << 16, "gemm_mid: too many output tiles for split-K")
-            cnt = _counters(x.device)
+            cnt = _stream_counters(x.device)
+            if cnt is None:
+                p = (p & 255) | 256   # (the same tile, one part)
         _check(lib.bcg_gemm_mid(p, epi, _p(x), w.data_ptr() + at * K, *(None if t is None else _p(t) for t in (*scales, bias, residual)),
                                 out.data_ptr() + at, None if ws is None else _p(ws), None if cnt is None else _p(cnt), M, N, K, inter,
                                 _stream()), "gemm_mid")   # (at / 2 rows or features of 2 bytes)
@@ -603,6 +606,7 @@ def hip_ops() -> SimpleNamespace:
             dev = torch.device("cuda", torch.cuda.current_device())
         if dev.index not in counters:
             counters[dev.index] = _new_counters(dev)
+        _spare(dev)
         if dev.index not in sk_ws:  # (128 MiB; allocated outside any graph capture)
             with torch.cuda.device(dev):
                 sk_ws[dev.index] = torch.empty(lib.bcg_gemm_w4_sk_ws_floats(), dtype=torch.float32, device=dev)
@@ -618,6 +622,31 @@ def hip_ops() -> SimpleNamespace:
         key = (stream.device.index, stream.cuda_stream)
         if key not in side_counters:
             side_counters[key] = _new_counters(stream.device)
+
+    capture_counters = {}  # (device index, stream handle) -> int32 [65536]: of the streams that captured, from `spare_counters`
+    spare_counters = {}    # device index -> up to 4 of them, zeroed outside any capture
+
+    def _stream_counters(dev):
+        """Counters for products of any shape, which a caller may launch on any stream, or capture there and replay elsewhere: each stream's own, made
+        at its first product (the pool's 32 streams, 64 at most), and others for what is captured on it.  None past those, and in a
+        capture that nothing was prepared for."""
+        dev = torch.device("cuda", dev.index if dev.index is not None else torch.cuda.current_device())
+        key = (dev.index, torch.cuda.current_stream(dev).cuda_stream)
+        if torch.cuda.is_current_stream_capturing():
+            spare = spare_counters.get(dev.index)
+            if key not in capture_counters and spare:
+                capture_counters[key] = spare.pop()
+            return capture_counters.get(key)
+        _spare(dev)
+        if key[1] == 0:
+            return _counters(dev)
+        if key not in side_counters and len(side_counters) < 64:
+            side_counters[key] = _new_counters(dev)
+        return side_counters.get(key)
+
+    def _spare(dev):
+        if dev.index not in spare_counters:
+            spare_counters[dev.index] = [_new_counters(dev) for _ in range(4)]
 
     def _counters(dev):
         dev = torch.device("cuda", dev.index if dev.index is not None else torch.cuda.current_device())
@@ -920,7 +949,7 @@ def hip_ops() -> SimpleNamespace:
     def _mid_fp8(xq, xs, wq, ws, *beside):
         """`_mid` for the fp8 products."""
         M, K = xq.shape
-        if not (33 <= M <= 1024 and plan.mode == "1"):
+        if not (33 <= M <= MID_ROWS and plan.mode == "1"):
             return None
         p = lib.bcg_gemm_mid_plan(0, M, wq.shape[0], K, 1)
         return p if p >= 0 and _plain_fp8(xq, xs, wq, ws, beside) else None

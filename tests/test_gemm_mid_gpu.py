@@ -65,7 +65,7 @@ def test_every_tile(ops, tile):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M", [33, 100, 1024])
+@pytest.mark.parametrize("M", [33, 100, 1024, 1025, 2047])
 def test_entry_points_take_it_and_replay(ops, M):
     """A captured sequence of the three entry points, replayed on other inputs with eager calls between, gives what eager calls give; the operands
     that the library has to see do not come here."""
@@ -96,6 +96,34 @@ def test_entry_points_take_it_and_replay(ops, M):
     assert xg.grad is not None
 
 
+@pytest.mark.gpu
+def test_streams_and_captures_without_preparation(ops):
+    """Split products on two streams at once don't share arrival counters, and a capture on a device that nothing was prepared on runs the product
+    in one part."""
+    from byzantine_consensus_llm_agents_amd.ops import hip
+    torch.manual_seed(0)
+    M, N, K = 40, 1024, 8192
+    x, w = torch.randn(M, K, device="cuda").bfloat16(), (torch.randn(N, K, device="cuda") * K ** -0.5).bfloat16()
+    own = getattr(hip.hip_ops, "__wrapped__", hip.hip_ops)()     # an instance that holds no counters yet
+    assert own.gemm_plan.mid(M, N, K, 0) >> 8 > 1
+    want = x.float() @ w.float().t()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = own.linear(x, w)
+    for _ in range(2):
+        graph.replay()
+    assert _err(got, want) < TOL
+    streams, outs = [torch.cuda.Stream() for _ in range(2)], []
+    for _ in range(20):
+        for s in streams:
+            with torch.cuda.stream(s):
+                outs.append(own.linear(x, w))
+        outs.append(own.linear(x, w))
+    torch.cuda.synchronize()
+    assert all(torch.equal(o, outs[0]) for o in outs) and _err(outs[0], want) < TOL
+
+
 def test_plan_takes_one_round_and_refuses_the_rest():
     if not os.path.exists(kernels_target()):
         pytest.skip("kernels not built")
@@ -103,12 +131,12 @@ def test_plan_takes_one_round_and_refuses_the_rest():
     lib.bcg_gemm_mid_parts.restype = ctypes.c_int64
     rng, taken = random.Random(0), 0
     for _ in range(3000):
-        M, N, K, epi, f8 = rng.randint(1, 1500), 8 * rng.randint(1, 5000), 32 * rng.randint(1, 600), rng.randrange(3), rng.randrange(2)
+        M, N, K, epi, f8 = rng.randint(1, 2500), 8 * rng.randint(1, 5000), 32 * rng.randint(1, 600), rng.randrange(3), rng.randrange(2)
         p = lib.bcg_gemm_mid_plan(epi, M, N, K, f8)
         if p < 0:
             continue
         taken += 1
-        assert 33 <= M <= 1024 and N % (32 if epi == 1 else 16) == 0 and K % (128 if f8 else 64) == 0 and not (f8 and epi == 1)
+        assert 33 <= M <= (1024 if f8 else 2047) and (M <= 1024 or N > 512) and N % (32 if epi == 1 else 16) == 0 and K % (128 if f8 else 64) == 0 and not (f8 and epi == 1)
         mt, nt = TILES[p & 255]
         assert epi != 1 or nt % 2 == 0
         tiles = ctypes.c_int()
@@ -120,6 +148,6 @@ def test_plan_takes_one_round_and_refuses_the_rest():
     assert GemmPlan().mid(100, 4096, 4096, 0) is None     # (no library: no plan)
     plan = GemmPlan(lib)
     assert plan._rest(300, 4096, 4096, 0)[0] == MID_CFG
-    for bad in ((0, 32, 4096, 4096, 0), (0, 1025, 4096, 4096, 0), (0, 100, 4096, 4100, 0), (0, 100, 4104, 4096, 0), (1, 100, 4112, 4096, 0),
+    for bad in ((0, 32, 4096, 4096, 0), (0, 2048, 4096, 4096, 0), (0, 1025, 4096, 4096, 1), (0, 1025, 512, 4096, 0), (0, 100, 4096, 4100, 0), (0, 100, 4104, 4096, 0), (1, 100, 4112, 4096, 0),
                 (0, 100, 4096, 64, 0), (0, 1024, 151936, 5120, 0), (1, 100, 4096, 4096, 1)):
         assert lib.bcg_gemm_mid_plan(*bad) == -1, bad
