@@ -23,7 +23,7 @@ PREFILL32_MAX_BLOCKS = 1024  # csrc/kernels/attention.hip: the 32x32 kernel's LD
 
 # csrc/kernels/gemm_skinny.hip: most rows, most rows with a fused norm, longest rows in bytes
 SKINNY_ROWS, SKINNY_NORM_ROWS, SKINNY_ROW_BYTES = 64, 16, 65536
-MID_ROWS = 2047  # csrc/kernels/gemm_mid.hip: most rows
+MID_ROWS = 1536  # csrc/kernels/gemm_mid.hip: most rows
 SKINNY_LONG_K = 12288  # past it: fewer shapes gain (`few_rows_pay`), logged apart
 
 c_int, c_float, c_void_p, c_uint32, c_int64 = ctypes.c_int, ctypes.c_float, ctypes.c_void_p, ctypes.c_uint32, ctypes.c_int64

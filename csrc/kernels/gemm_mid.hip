@@ -43,13 +43,14 @@ float predicted(const Cost& c, float x_rows, int bm, int bn, float kb, float w_b
 // them before (tile kernels, library, few-row kernel): up to 64 rows 0.65, 128: 0.66, 256: 0.70, 512: 0.73, 1024: 0.84 on average; 12 projections of the
 // served models 0.81 to 0.90, the slowest (40 to 64 rows, 7168 x 5120 and 6144 x 4096) 1.1.  fp8, whose other side has matrix
 // instructions of twice the rate: 0.5 to 0.86, but 0.8 to 1.25 from M N K = 15e9 on; bf16 1.0 to 1.18 from 80e9 on.
-// 1025 to 2047 rows, 900 products: 0.80 to 0.94 over 512 columns or more, the slowest 1.05 (1565 x 2432 x 2560 1.07); up to 512 columns 0.7, but
-// 1.2 to 1.3 behind the library's own split of 5632 and 6912 columns of K; 2048 rows on, pieces of the 256 x 256 kernel begin.  fp8 0.64
-// to 0.95, but 1.2 to 1.33 at 768 to 1792 columns of K, which nothing here tells apart.
+// 1025 to 1536 rows, 213 products of more than 512 columns: 0.86 on average, the slowest 1.03; then the library's tiles fill the chip as well: 0.87
+// and 1.07 to 1792 rows, 0.93 and 1.05 to 2047, where 2048 x 8192 behind 2039 rows took 80 us for 70.  Up to 512 columns the library's split of a
+// long K wins at times (1508 x 256 x 5632: 22.5 us for 18.3).  fp8 past 1024 rows 0.64 to 0.95 on average, but 1.2 to 1.33 at 768 to 1792
+// columns of K, which nothing here tells apart.
 BCG_API int bcg_gemm_mid_plan(int epi, int M, int N, int K, int f8) {
   const bool gated = epi == EPI_SILU_MUL;
   const int bytes = f8 ? K : 2 * K, inter = N / 2;
-  if (M < 33 || M > (f8 ? 1024 : 2047) || (M > 1024 && N <= 512) || K <= 0 || bytes % 128 || N < 16 || N % (gated ? 32 : 16) || N > 1 << 20 || (f8 && gated)) return -1;
+  if (M < 33 || M > (f8 ? 1024 : 1536) || (M > 1024 && N <= 512) || K <= 0 || bytes % 128 || N < 16 || N % (gated ? 32 : 16) || N > 1 << 20 || (f8 && gated)) return -1;
   if (static_cast<int64_t>(N) * K < 800000 || static_cast<int64_t>(N) * bytes >= 1ll << 31 || static_cast<int64_t>(M) * bytes >= 1ll << 31) return -1;
   const Cost& cost = COSTS[M <= 128 ? 0 : M <= 288 ? 1 : 2];
   if (static_cast<float>(M) * N * K > (f8 ? 15e9f : 80e9f)) return -1;
