@@ -1,13 +1,11 @@
 """Which GEMM runs where: the hand MFMA kernel (csrc/kernels/gemm.hip) or hipBLASLt.
 
-Decode projections are skinny (M = live rows of a decode bucket, 1..768) and
-the hand kernel's tile shapes, fused epilogues and XCD-aware order are built
-for them; prefill chunks (M = 16384) stay on hipBLASLt's tuned kernels.  The
-choice per (M, N, K, epilogue) comes from a table measured on the GPU
-(``tools/tune_hand_gemm.py`` -> ``engine/tuned/hand_gemm.json``: for every
-decode bucket and projection shape, every tile configuration and the library
-are timed and the fastest is kept).  Shapes the table does not cover use a
-simple rule (hand kernel up to ``max_m`` rows).
+Up to 64 rows the few-row kernel (csrc/kernels/gemm_skinny.hip) and 33 to 1536 rows the one-round kernel
+(csrc/kernels/gemm_mid.hip, `GemmPlan.mid`) come before this choice where their own rules take a product.  What they
+leave (decode buckets whose product is more than a round of tiles, operands they refuse) goes by a table per (M, N, K,
+epilogue) measured on the GPU (``tools/tune_hand_gemm.py`` -> ``engine/tuned/hand_gemm.json``: for every decode bucket
+and projection shape, every tile configuration and the library are timed and the fastest is kept), prefill chunks by
+the rules of `GemmPlan.pieces`, and shapes that nothing covers stay on the library.
 
 ``BCG_HAND_GEMM``: ``0`` = library only, ``1`` (default) = table / rule,
 ``force`` = hand kernel wherever the shape is supported (tests; ``BCG_HAND_GEMM_SPLIT``
@@ -137,13 +135,13 @@ class GemmPlan:
 
     def columns(self, M: int, N: int, K: int) -> int:
         """Gated projections (epilogue 1) below LARGE_M rows: how many of the N columns run as whole rounds of 256 x 256
-        tiles, the others in 64 x 64 tiles behind them; N: no split.
+        tiles, the others behind them; N: no split.
 
         A decode step's rows make few tiles, and one round and a sixteenth costs two: 448 x 34816 x 5120 (272 tiles) took 217
-        us, as one round (125) and the last 2048 columns in 224 small tiles (35) 165 to 172; 352 rows 175 -> 162, 512: 195 -> 176;
+        us, as one round (125) and the last 2048 columns in 224 tiles of 64 x 64 (35) 165 to 172; 352 rows 175 -> 162, 512: 195 -> 176;
         768 x 22528 x 5120: 186 -> 162.  Taken where the rounds are at least 0.94 full, the rest is at most one small
         tile per CU (0.43 us per 64 of K against 1.46 for a round) and the rows fill 0.65 of their tiles (300 x 33792 x
-        4096: 126 -> 129)."""
+        4096: 126 -> 129).  The one-round kernel takes the rest where it can (2048 columns of 5120 over 448 rows: 37 -> 27.6 us in the step)."""
         if self.mode != "1" or not 256 < M < LARGE_M or N % 256 or not self.supported(W4_CFG, M, N, K, 1):
             return N
         n_t, m_t = N // 256, -(-M // 256)

@@ -19,8 +19,9 @@
 //   are 16 contiguous bytes of one V^T row (block h>>1, offset 8(h&1)).
 //   K tiles load row r from token 8(r>>2) + 4u + (r&3) (a row gather: free).
 //
-// Decode: one workgroup per (sequence, kv head, 256-token split); the G = n_q/n_kv query
-// heads of the kv head share every K/V byte (GQA packing: 5 for Qwen3-14B);
+// Decode: one workgroup per (sequence, kv head, 256-token split), or, where the batch has more
+// of these than the chip holds, an even share of all chunks per wave (`decode_stream`); the
+// G = n_q/n_kv query heads of the kv head share every K/V byte (GQA packing: 5 for Qwen3-14B);
 // waves are combined through LDS and splits merged by a second kernel
 // (flash-decoding).  Prefill: one workgroup per (64-query tile, query
 // head), causal over cached prefix + new tokens, varlen via a tile table.
