@@ -38,8 +38,10 @@ float predicted(const Cost& c, float x_rows, int bm, int bn, float kb, float w_b
 }  // namespace
 
 // How x [M, K] w [N, K]^T runs here: tile | split << 8, or -1 where it does not: the product has to fit one round of workgroups
-// (several rounds lose to the persistent 256 x 256 kernel), and W to hold 0.8 M elements (below, a launch of the library or the few-row kernel
-// is shorter, 4.6 to 5.5 us against 5.7 to 7).  33 to 1024 rows, 900 products of 64 to 40000 columns and K of 256 to 18000, this over what took
+// (several rounds lose to the persistent 256 x 256 kernel).  W holds 0.1 M elements or more: 603 products of 0.1 to 0.8 M and K >= 192 took 0.67 of
+// the library's or few-row kernel's time on average, the slowest 1.06, 1.10 and 1.14 (92 x 96 x 1536, 182 x 96 x 1152 and 57 x 256 x 2048, 4.7 to
+// 5.5 us), all others up to 1.04; of 64 and 128 columns of K it is 0.8 M (below, up to 1.17 of a library launch of 4 to 5 us), of fp8 0.8 M.
+// 33 to 1024 rows, 900 products of 64 to 40000 columns and K of 256 to 18000, this over what took
 // them before (tile kernels, library, few-row kernel): up to 64 rows 0.65, 128: 0.66, 256: 0.70, 512: 0.73, 1024: 0.84 on average; 12 projections of the
 // served models 0.81 to 0.90, the slowest (40 to 64 rows, 7168 x 5120 and 6144 x 4096) 1.1.  fp8, whose other side has matrix
 // instructions of twice the rate: 0.5 to 0.86, but 0.8 to 1.25 from M N K = 15e9 on; bf16 1.0 to 1.18 from 80e9 on.
@@ -51,7 +53,7 @@ BCG_API int bcg_gemm_mid_plan(int epi, int M, int N, int K, int f8) {
   const bool gated = epi == EPI_SILU_MUL;
   const int bytes = f8 ? K : 2 * K, inter = N / 2;
   if (M < 33 || M > (f8 ? 1024 : 1536) || (M > 1024 && N <= 512) || K <= 0 || bytes % 128 || N < 16 || N % (gated ? 32 : 16) || N > 1 << 20 || (f8 && gated)) return -1;
-  if (static_cast<int64_t>(N) * K < 800000 || static_cast<int64_t>(N) * bytes >= 1ll << 31 || static_cast<int64_t>(M) * bytes >= 1ll << 31) return -1;
+  if (static_cast<int64_t>(N) * K < (f8 || K < 192 ? 800000 : 100000) || static_cast<int64_t>(N) * bytes >= 1ll << 31 || static_cast<int64_t>(M) * bytes >= 1ll << 31) return -1;
   const Cost& cost = COSTS[M <= 128 ? 0 : M <= 288 ? 1 : 2];
   if (static_cast<float>(M) * N * K > (f8 ? 15e9f : 80e9f)) return -1;
   int best = -1;

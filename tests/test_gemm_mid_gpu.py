@@ -65,12 +65,12 @@ def test_every_tile(ops, tile):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M", [33, 100, 1024, 1025, 1536])
-def test_entry_points_take_it_and_replay(ops, M):
+@pytest.mark.parametrize("M,N,K", [(33, 2048, 1152), (100, 2048, 1152), (1024, 2048, 1152), (1025, 2048, 1152), (1536, 2048, 1152),
+                                   (90, 544, 192), (400, 32, 4096)])
+def test_entry_points_take_it_and_replay(ops, M, N, K):
     """A captured sequence of the three entry points, replayed on other inputs with eager calls between, gives what eager calls give; the operands
     that the library has to see do not come here."""
     torch.manual_seed(M)
-    K, N = 1152, 2048
     x, res = torch.randn(M, K, device="cuda").bfloat16(), torch.randn(M, N, device="cuda").bfloat16()
     w = (torch.randn(N, K, device="cuda") * K ** -0.5).bfloat16()
     ops.prepare_device("cuda")
@@ -149,5 +149,5 @@ def test_plan_takes_one_round_and_refuses_the_rest():
     plan = GemmPlan(lib)
     assert plan._rest(300, 4096, 4096, 0)[0] == MID_CFG
     for bad in ((0, 32, 4096, 4096, 0), (0, 1537, 4096, 4096, 0), (0, 1025, 4096, 4096, 1), (0, 1025, 512, 4096, 0), (0, 100, 4096, 4100, 0), (0, 100, 4104, 4096, 0), (1, 100, 4112, 4096, 0),
-                (0, 100, 4096, 64, 0), (0, 1024, 151936, 5120, 0), (1, 100, 4096, 4096, 1)):
+                (0, 100, 4096, 64, 0), (0, 100, 4096, 128, 0), (0, 100, 512, 192, 0), (0, 100, 512, 1024, 1), (0, 1024, 151936, 5120, 0), (1, 100, 4096, 4096, 1)):
         assert lib.bcg_gemm_mid_plan(*bad) == -1, bad
