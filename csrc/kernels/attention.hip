@@ -943,20 +943,24 @@ __global__ __launch_bounds__(64 * COMBINE_WAVES) void decode_combine_kernel(
   const int bq = blockIdx.x * COMBINE_WAVES + (threadIdx.x >> 6);
   if (bq >= n_bq) return;  // wave-uniform
   const int b = bq / n_q;
-  // every slot's (m, l), before the number of parts is known: what the loads below say arrives at the same time
-  float2 mlv = lane < max_splits ? reinterpret_cast<const float2*>(part_ml)[static_cast<size_t>(bq) * max_splits + lane]
-                                 : float2{-INFINITY, 0.f};
+  const float2* ml = reinterpret_cast<const float2*>(part_ml) + static_cast<size_t>(bq) * max_splits + lane;
+  float2 mlv{-INFINITY, 0.f};
+  // heads of 128, the streamed ones: every slot's (m, l) before the number of parts is known, what the loads below say arrives at the same time
+  if (HD == 128 && lane < max_splits) mlv = *ml;
   const int own = max(0, seq_lens[b] - (kv_begin ? kv_begin[b] : 0));
   // <= max_splits <= 64 (host check); slots 0 .. split_base[b]-1 hold the shared-prefix partials
   int parts = (own + split_tokens - 1) / split_tokens;
-  int waves = 0, first = 0, next = 0, total = 0;
-  if (stream != nullptr) waves = stream[B + 1], first = stream[b], next = stream[b + 1], total = stream[B] * n_kv;
-  if (waves > 0) {  // decode_stream: how its waves' ranges cut the pair's chunks
-    const int n = next - first;
-    const int c0 = first * n_kv + (bq - b * n_q) / (n_q / n_kv) * n;
-    parts = n > 0 ? stream_wave(c0 + n - 1, total, waves) - stream_wave(c0, total, waves) + 1 : 0;
+  if constexpr (HD == 128) {
+    int waves = 0, first = 0, next = 0, total = 0;
+    if (stream != nullptr) waves = stream[B + 1], first = stream[b], next = stream[b + 1], total = stream[B] * n_kv;
+    if (waves > 0) {  // decode_stream: how its waves' ranges cut the pair's chunks
+      const int n = next - first;
+      const int c0 = first * n_kv + (bq - b * n_q) / (n_q / n_kv) * n;
+      parts = n > 0 ? stream_wave(c0 + n - 1, total, waves) - stream_wave(c0, total, waves) + 1 : 0;
+    }
   }
   const int ns = (split_base ? split_base[b] : 0) + parts;
+  if (HD != 128 && lane < ns) mlv = *ml;
   if (lane >= ns) mlv = float2{-INFINITY, 0.f};
   float mm = mlv.x;
 #pragma unroll
