@@ -575,7 +575,7 @@ def hip_ops() -> SimpleNamespace:
     def _linear_rows(x, w, bias, cfg, out, epi_log):
         _log(x.shape[0], w.shape[0], x.shape[1], epi_log, cfg)
         if cfg is not None:
-            return gemm_nt(x, w, cfg, 0, bias=bias, out=out)
+            return _hand(x, w, cfg, 0, out, bias=bias)
         if out is None:
             return torch.nn.functional.linear(x, w, bias)
         return torch.mm(x, w.t(), out=out) if bias is None else torch.addmm(bias, x, w.t(), out=out)
@@ -667,8 +667,6 @@ def hip_ops() -> SimpleNamespace:
         N = w.shape[0]
         _req(x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_contiguous() and w.is_contiguous()
              and w.shape[1] == K, "gemm_nt: contiguous bf16 x [M,K], w [N,K]")
-        if cfg == MID_CFG:   # (a piece of a call whose operands were looked at: `_pieces`)
-            return _gemm_mid(split_k, x, w, epi, out, bias, residual)
         _req(plan.supported(cfg, M, N, K, epi, split_k),
              f"gemm_nt: shape {M}x{N}x{K} epi {epi} split {split_k} unsupported by tile {cfg}")
         width = N // 2 if epi == 1 else N
@@ -694,6 +692,13 @@ def hip_ops() -> SimpleNamespace:
                                _p(ws) if ws is not None else None, _p(cnt) if cnt is not None else None,
                                M, N, K, N // 2, split_k, _stream()), "gemm_nt")
         return out
+
+    def _hand(x, w, cfg, epi, out, **beside):
+        """A piece of a product (`_pieces`) by its choice.  The one-round kernel is chosen only where `_pieces` looked at the operands
+        and comes with an `out` of its rows; `gemm_nt`, which anyone may call, refuses it like every configuration that it does not hold."""
+        if cfg[0] == MID_CFG:
+            return _gemm_mid(cfg[1], x, w, epi, out, **beside)
+        return gemm_nt(x, w, cfg, epi, out=out, **beside)
 
     def linear_silu(x, w):
         """silu(x Wg^T) * (x Wu^T), W = [gate; up] -- K-ACT fused into the gate_up GEMM."""
@@ -730,7 +735,7 @@ def hip_ops() -> SimpleNamespace:
                 dst.copy_(silu_mul(linear(xr, w, _epi_log=1)))
             else:
                 _log(rows, N, K, 1, cfg)
-                gemm_nt(xr, w, cfg, 1, out=dst)
+                _hand(xr, w, cfg, 1, dst)
         return out
 
     def _w4_act(epi, x, w, c, tail, inter, limit):
@@ -801,7 +806,7 @@ def hip_ops() -> SimpleNamespace:
         M, K = x.shape
         _log(M, w.shape[0], K, 2, cfg)
         if cfg is not None:
-            gemm_nt(x, w, cfg, 2, residual=residual, out=residual)
+            _hand(x, w, cfg, 2, residual, residual=residual)
         elif (residual_addmm and residual.is_contiguous() and residual.dtype == x.dtype == w.dtype
                 and residual.shape == (M, w.shape[0])):
             # hipBLASLt with beta = 1: the residual add rides in the GEMM epilogue (one read

@@ -23,6 +23,14 @@ def ops():
     return get_ops("hip")
 
 
+@pytest.fixture(scope="module")
+def ops_cpu():
+    if not os.path.exists(kernels_target()):
+        pytest.skip("kernels not built")
+    from byzantine_consensus_llm_agents_amd.ops.hip import hip_ops
+    return hip_ops()
+
+
 def _err(a, b):
     return ((a.float() - b).norm() / b.norm()).item()
 
@@ -151,3 +159,13 @@ def test_plan_takes_one_round_and_refuses_the_rest():
     for bad in ((0, 32, 4096, 4096, 0), (0, 1537, 4096, 4096, 0), (0, 1025, 4096, 4096, 1), (0, 1025, 512, 4096, 0), (0, 100, 4096, 4100, 0), (0, 100, 4104, 4096, 0), (1, 100, 4112, 4096, 0),
                 (0, 100, 4096, 64, 0), (0, 100, 4096, 128, 0), (0, 100, 512, 192, 0), (0, 100, 512, 1024, 1), (0, 1024, 151936, 5120, 0), (1, 100, 4096, 4096, 1)):
         assert lib.bcg_gemm_mid_plan(*bad) == -1, bad
+
+
+def test_gemm_nt_refuses_the_configuration(ops_cpu):
+    """`gemm_nt` takes the tiles that `GemmPlan.supported` knows: the one-round kernel's number is none of them, whatever `out` and `bias` are."""
+    x, w = torch.zeros(100, 4096).bfloat16(), torch.zeros(4096, 4096).bfloat16()
+    plan = ops_cpu.gemm_plan.mid(100, 4096, 4096, 0)
+    assert plan is not None and not ops_cpu.gemm_plan.supported(MID_CFG, 100, 4096, 4096, 0, plan)
+    for kw in ({}, {"out": torch.zeros(1, 4096).bfloat16()}, {"bias": torch.zeros(1).bfloat16(), "out": torch.zeros(100, 4096).bfloat16()}):
+        with pytest.raises(ValueError):
+            ops_cpu.gemm_nt(x, w, (MID_CFG, plan), **kw)
