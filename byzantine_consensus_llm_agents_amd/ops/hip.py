@@ -101,6 +101,7 @@ def load_library(path: str = None) -> ctypes.CDLL:
         "bcg_gemm_skinny": [c_int, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
                             c_void_p],
         "bcg_gemm_skinny_fp8": [c_int] + [c_void_p] * 7 + [c_int] * 3 + [c_void_p],
+        "bcg_capture_id": [c_void_p],
         "bcg_gemm_mid_plan": [c_int] * 5,
         "bcg_gemm_mid_parts": [c_int] * 4 + [ctypes.POINTER(c_int)],
         "bcg_gemm_mid": [c_int, c_int] + [c_void_p] * 9 + [c_int] * 4 + [c_void_p],
@@ -200,7 +201,7 @@ def load_library(path: str = None) -> ctypes.CDLL:
     for name, argtypes in sig.items():
         fn = getattr(lib, name)
         fn.argtypes = argtypes
-        fn.restype = c_int64 if name == "bcg_gemm_mid_parts" else c_int
+        fn.restype = c_int64 if name in ("bcg_gemm_mid_parts", "bcg_capture_id") else c_int
     _LIB = lib
     return lib
 
@@ -509,10 +510,7 @@ def hip_ops() -> SimpleNamespace:
         if p >> 8 > 1:
             tiles = c_int()
             ws = torch.empty(lib.bcg_gemm_mid_parts(p, epi, M, N, ctypes.byref(tiles)), dtype=torch.float32, device=x.device)
-            _req(tiles.value <= 1 << 16, "gemm_mid: too many output tiles for split-K")
-            cnt = _stream_counters(x.device)
-            if cnt is None:
-                p = (p & 255) | 256   # (the same tile, one part)
+            cnt = _counters(x.device)   # (at most 256 tiles: one round)
         _check(lib.bcg_gemm_mid(p, epi, _p(x), w.data_ptr() + at * K, *(None if t is None else _p(t) for t in (*scales, bias, residual)),
                                 out.data_ptr() + at, None if ws is None else _p(ws), None if cnt is None else _p(cnt), M, N, K, inter,
                                 _stream()), "gemm_mid")   # (at / 2 rows or features of 2 bytes)
@@ -585,13 +583,10 @@ def hip_ops() -> SimpleNamespace:
 
     # Split-K arrival counters (one int per output tile; the last-arriving workgroup of a
     # tile resets its counter, so a buffer stays zero between launches).  Kernels that may
-    # run CONCURRENTLY need disjoint buffers: one per device for the engine's main stream --
-    # shared by eager launches and every captured decode graph, which replay on that stream
-    # one after another -- and one per registered side stream.  Buffers are allocated eagerly
-    # by `prepare_device` / `register_stream`, never inside a graph capture: a zero-fill captured into one bucket's graph would leave the
-    # buffer uninitialised for every other graph.
-    counters = {}       # device index -> int32 [65536]
-    side_counters = {}  # (device index, stream handle) -> int32 [65536]
+    # run CONCURRENTLY need disjoint buffers: every stream has its own for what is launched on it, and every
+    # capture its own for what it records, as the graph may be replayed on any stream, beside others that were captured on the same one.
+    counters = {}          # (device index, stream handle) -> int32 [65536]
+    capture_counters = {}  # (device index, stream handle) -> (capture, int32 [65536]) of the last capture on that stream
 
     def _new_counters(dev):
         _req(not torch.cuda.is_current_stream_capturing(),
@@ -604,9 +599,7 @@ def hip_ops() -> SimpleNamespace:
         dev = torch.device(dev)
         if dev.index is None:
             dev = torch.device("cuda", torch.cuda.current_device())
-        if dev.index not in counters:
-            counters[dev.index] = _new_counters(dev)
-        _spare(dev)
+        register_stream(torch.cuda.default_stream(dev))
         if dev.index not in sk_ws:  # (128 MiB; allocated outside any graph capture)
             with torch.cuda.device(dev):
                 sk_ws[dev.index] = torch.empty(lib.bcg_gemm_w4_sk_ws_floats(), dtype=torch.float32, device=dev)
@@ -614,48 +607,41 @@ def hip_ops() -> SimpleNamespace:
     def _sk_workspace(dev):
         dev = torch.device("cuda", dev.index if dev.index is not None else torch.cuda.current_device())
         if dev.index not in sk_ws:
-            prepare_device(dev)  # raises under capture (the counters' check)
+            _req(not torch.cuda.is_current_stream_capturing(), "stream-K parts must be allocated outside graph capture (ops.prepare_device)")
+            prepare_device(dev)
         return sk_ws[dev.index]
 
     def register_stream(stream):
-        """Give `stream` its own split-K counters (its GEMMs may overlap the main stream's)."""
+        """Make `stream`'s split-K counters now, not at its first product."""
         key = (stream.device.index, stream.cuda_stream)
-        if key not in side_counters:
-            side_counters[key] = _new_counters(stream.device)
-
-    capture_counters = {}  # (device index, stream handle) -> int32 [65536]: of the streams that captured, from `spare_counters`
-    spare_counters = {}    # device index -> up to 4 of them, zeroed outside any capture
-
-    def _stream_counters(dev):
-        """Counters for products of any shape, which a caller may launch on any stream, or capture there and replay elsewhere: each stream's own, made
-        at its first product (the pool's 32 streams, 64 at most), and others for what is captured on it.  None past those, and in a
-        capture that nothing was prepared for."""
-        dev = torch.device("cuda", dev.index if dev.index is not None else torch.cuda.current_device())
-        key = (dev.index, torch.cuda.current_stream(dev).cuda_stream)
-        if torch.cuda.is_current_stream_capturing():
-            spare = spare_counters.get(dev.index)
-            if key not in capture_counters and spare:
-                capture_counters[key] = spare.pop()
-            return capture_counters.get(key)
-        _spare(dev)
-        if key[1] == 0:
-            return _counters(dev)
-        if key not in side_counters and len(side_counters) < 64:
-            side_counters[key] = _new_counters(dev)
-        return side_counters.get(key)
-
-    def _spare(dev):
-        if dev.index not in spare_counters:
-            spare_counters[dev.index] = [_new_counters(dev) for _ in range(4)]
+        if key not in counters:
+            with torch.cuda.stream(stream):   # (zeroed there: its products are behind it)
+                counters.setdefault(key, _new_counters(stream.device))
 
     def _counters(dev):
+        """The current stream's counters, made at its first product; past 64 streams (the pool has 32) zeros for this product alone."""
         dev = torch.device("cuda", dev.index if dev.index is not None else torch.cuda.current_device())
-        side = side_counters.get((dev.index, torch.cuda.current_stream(dev).cuda_stream))
-        if side is not None:
-            return side
-        if dev.index not in counters:
-            prepare_device(dev)  # raises under capture
-        return counters[dev.index]
+        stream = torch.cuda.current_stream(dev)
+        key = (dev.index, stream.cuda_stream)
+        if torch.cuda.is_current_stream_capturing():
+            return _capture_counters(dev, key)
+        if key not in counters:
+            if len(counters) >= 64:
+                return _new_counters(dev)
+            register_stream(stream)
+        return counters[key]
+
+    def _capture_counters(dev, key):
+        """Out of the graph's own memory, zeroed where its first product on this stream is: every replay zeroes them before it uses them, and nobody
+        else does.  Held while the capture lasts (after that it is the graph's: no product of another one is given them), until the
+        next on the stream."""
+        capture = lib.bcg_capture_id(key[1])
+        held = capture_counters.get(key)
+        if held is None or held[0] != capture or capture == 0:
+            held = (capture, torch.zeros(1 << 16, dtype=torch.int32, device=dev))
+            if capture != 0 and (key in capture_counters or len(capture_counters) < 64):
+                capture_counters[key] = held
+        return held[1]
 
     def gemm_nt(x, w, cfg, epi=0, bias=None, residual=None, out=None, split_k=1):
         """Hand MFMA GEMM (csrc/kernels/gemm.hip): x [M,K] @ w[N,K]^T with epilogue `epi`

@@ -81,6 +81,17 @@ BCG_API int64_t bcg_gemm_mid_parts(int plan, int epi, int M, int N, int* tiles) 
   return plan >> 8 > 1 ? static_cast<int64_t>(*tiles) * (plan >> 8) * t.mt * 16 * bn : 0;
 }
 
+// Number of the capture that records what is launched on the stream (no two have the same), 0 without one
+BCG_API int64_t bcg_capture_id(hipStream_t stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  if (hipStreamGetCaptureInfo(stream, &status, &id) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  return status == hipStreamCaptureStatusActive ? static_cast<int64_t>(id) : 0;
+}
+
 // plan: of bcg_gemm_mid_plan for the same sizes, or any other tile and split.  epi: 0 store (+ bias), 1 silu(gate) * up of N / 2 features from w's first
 // row on, their up rows `inter` rows behind, into rows of `c` that are `inter` apart, 2 residual + product (residual may be c).  x_scale [M],
 // w_scale [N]: not null for e4m3 operands (epi 0 and 2).  Pointers 16-byte aligned, rows contiguous; ws and counters as

@@ -106,8 +106,7 @@ def test_entry_points_take_it_and_replay(ops, M, N, K):
 
 @pytest.mark.gpu
 def test_streams_and_captures_without_preparation(ops):
-    """Split products on two streams at once don't share arrival counters, and a capture on a device that nothing was prepared on runs the product
-    in one part."""
+    """Split products on two streams at once don't share arrival counters, and a capture needs nothing prepared."""
     from byzantine_consensus_llm_agents_amd.ops import hip
     torch.manual_seed(0)
     M, N, K = 40, 1024, 8192
@@ -130,6 +129,54 @@ def test_streams_and_captures_without_preparation(ops):
         outs.append(own.linear(x, w))
     torch.cuda.synchronize()
     assert all(torch.equal(o, outs[0]) for o in outs) and _err(outs[0], want) < TOL
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pool", [False, True], ids=["own pools", "one pool"])
+def test_graphs_have_counters_of_their_own(ops, monkeypatch, pool):
+    """Graphs captured on one stream (`torch.cuda.graph` takes the same for all) are replayed on several at once: no two may count arrivals in the same
+    place, and none where eager products do.  Graphs that share a pool are replayed in turn.  One product of a graph is on a side stream."""
+    torch.manual_seed(0)
+    M, N, K = 40, 1024, 8192
+    xs = [torch.randn(M, K, device="cuda").bfloat16() for _ in range(3)]
+    w = (torch.randn(N, K, device="cuda") * K ** -0.5).bfloat16()
+    assert ops.gemm_plan.mid(M, N, K, 0) >> 8 > 1
+    counters, launch = [], ops.library.bcg_gemm_mid
+    monkeypatch.setattr(ops.library, "bcg_gemm_mid", lambda *a: counters.append(a[10].value) or launch(*a))
+    want = [ops.linear(x, w) for x in xs]
+    eager, graphs, outs, side = set(counters), [], [], torch.cuda.Stream()
+    assert len(eager) == 1
+    for x in xs:
+        graphs.append(torch.cuda.CUDAGraph())
+        counters.clear()
+        with torch.cuda.graph(graphs[-1], pool=graphs[0].pool() if pool and len(graphs) > 1 else None):
+            y = [ops.linear(x, w) for _ in range(2)]
+            side.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.stream(side):
+                y.append(ops.linear(x, w))
+            torch.cuda.current_stream().wait_stream(side)
+        outs.append(y)
+        assert counters[0] == counters[1] != counters[2]
+        assert pool or not eager & set(counters)
+        eager |= set(counters)
+    monkeypatch.undo()
+    streams = [torch.cuda.Stream() for _ in graphs]
+    for _ in range(10):
+        for y in outs:
+            for t in y:
+                t.fill_(float("nan"))
+        torch.cuda.synchronize()
+        for g, s in zip(graphs, streams):
+            with torch.cuda.stream(s):
+                g.replay()
+                if not pool:
+                    g.replay()
+            if pool:
+                s.synchronize()
+        eagerly = ops.linear(xs[0], w)
+        torch.cuda.synchronize()
+        assert torch.equal(eagerly, want[0])
+        assert all(torch.equal(t, u) for y, u in zip(outs, want) for t in y)
 
 
 def test_plan_takes_one_round_and_refuses_the_rest():
