@@ -360,7 +360,7 @@ def hip_ops() -> SimpleNamespace:
         """fp32 split partials (o, m, l) of the flash-decoding split-K (+ the shared-prefix
         pass's slots when `cascade`)."""
         max_splits = lib.bcg_decode_max_splits(max_blocks * block_size, int(cascade))
-        return B * n_q * max_splits * (hd + 2) + B + 2   # (the last: how the streamed kernel cut the batch)
+        return B * n_q * max_splits * (hd + 2)
 
     def paged_attention_decode(q, k_cache, v_cache, layer, block_tables, seq_lens, scale, workspace=None,
                                cascade=None):
@@ -376,7 +376,7 @@ def hip_ops() -> SimpleNamespace:
         _req(B <= 2048, "decode attention: at most 2048 rows")
         split = lib.bcg_decode_split_tokens(B, n_kv, max_blocks * BS)
         max_splits = lib.bcg_decode_max_splits(max_blocks * BS, int(cascade is not None))
-        need = B * n_q * max_splits * (hd + 2) + B + 2
+        need = B * n_q * max_splits * (hd + 2)
         if workspace is None:
             ws = torch.empty(need, dtype=torch.float32, device=q.device)
         else:

@@ -471,15 +471,20 @@ constexpr int STREAM_RING = 16384;    // bytes of a wave's chunk: K, then V
 constexpr int STREAM_Q = STREAM_G * 256;
 constexpr int STREAM_LDS = 4 * (STREAM_RING + 2 * STREAM_Q);   // two workgroups a CU
 
+// The merge learns how many parts a pair is cut into from the partials it reads anyway: whoever has the last part writes PARTS_END as the m of the
+// slot behind it.  (A table of the cut, or counts beside the partials, cost it another latency: 0.2 us, 2 to 5 % of a step of short contexts.)
+constexpr uint32_t PARTS_END = 0x7fc0e4d1u;   // a NaN that no product of bf16 values makes (their payloads end in 16 zeros)
+__device__ __forceinline__ void end_parts(float* m) { *reinterpret_cast<uint32_t*>(m) = PARTS_END; }
+
 // The wave that chunk c of the batch falls to, of `waves` that share `total` chunks: wave w has those from w total / waves on
 __device__ __forceinline__ int stream_wave(int c, int total, int waves) {
   return static_cast<int>(((static_cast<uint64_t>(c) + 1) * waves - 1) / total);
 }
 
-// stream (out, by the first workgroup; read by the merge): [B + 1] chunks of the rows before, [1] waves that share them
 __device__ __forceinline__ void decode_stream(
     unsigned char* smem, const bf16_t* q, const KVGeom& g, const int* block_tables, int max_blocks, const int* seq_lens, int B, int n_q,
-    float scale_log2, float* part_o, float* part_ml, int max_splits, const int* kv_begin, const int* split_base, int* stream) {
+    float scale_log2, float* part_o, float* part_ml, int max_splits, const int* kv_begin, const int* split_base) {
+  asm("" : "+s"(B));   // the items' row predicates are not kept for the loop below: 8 pairs of scalars that went through vector lanes, 0.2 us of their path
   constexpr int HD = 128;
   static_assert(sizeof(int) * (DEC_MAX_B + 1 + 8) <= STREAM_LDS, "the row table lies where the ring is later");
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -528,10 +533,6 @@ __device__ __forceinline__ void decode_stream(
     // ranges are so long that a pair of n chunks, cut into (n - 2) / shortest + 2 parts at most, has a slot for each
     const int shortest = max(1, (longest + slots - 2) / (slots - 1));
     const int waves = max(1, min(static_cast<int>(gridDim.x) * 4, total / shortest));
-    if (blockIdx.x == 0) {
-      for (int i = tid; i <= B; i += 256) stream[i] = pre[i];
-      if (tid == 0) stream[B + 1] = waves;
-    }
     // (neighbouring ranges to the waves of a workgroup: their pages lie side by side; fewer ranges than waves: spread evenly)
     const int at = static_cast<int>(blockIdx.x) * 4 + w, all = gridDim.x * 4;
     gw = at * waves / all;
@@ -683,10 +684,12 @@ __device__ __forceinline__ void decode_stream(
       compute_chunk<HD, AllVisible, true>(x, bq, tj, use.x.ctx, AllVisible{}, scale_log2, m, l, o, lane);
     if (left == 1 || use.c + 1 == use.x.n) {   // the pair or the range ends
       if (r < G) {
-        const size_t at = (static_cast<size_t>(use.b) * n_q + use.kvh * G + r) * max_splits + (split_base ? bases[use.b] : 0) + part;
+        const int slot = (split_base ? bases[use.b] : 0) + part;
+        const size_t at = (static_cast<size_t>(use.b) * n_q + use.kvh * G + r) * max_splits + slot;
 #pragma unroll
         for (int dt = 0; dt < HD / 16; ++dt) *reinterpret_cast<f32x4*>(part_o + at * HD + dt * 16 + 4 * h) = o[dt];
         if (h == 0) *reinterpret_cast<float2*>(part_ml + at * 2) = float2{m, l};
+        if (h == 0 && use.c + 1 == use.x.n && slot + 1 < max_splits) end_parts(part_ml + (at + 1) * 2);
       }
       part = 0;
       fresh = true;
@@ -708,7 +711,7 @@ __global__ __launch_bounds__(256, (STREAM ? 2 : 1)) void decode_attn_kernel(
     const bf16_t* __restrict__ q, KVGeom g, const int* __restrict__ block_tables, int max_blocks,
     const int* __restrict__ seq_lens, int B, int n_q, float scale_log2, float* __restrict__ part_o,
     float* __restrict__ part_ml, int max_splits, const int* __restrict__ kv_begin,
-    const int* __restrict__ split_base, FusedArgs fa, int* __restrict__ stream) {
+    const int* __restrict__ split_base, FusedArgs fa) {
   static_assert(!FUSED || (HD == 64 && !F8), "fused: see FusedArgs");
   static_assert(!STREAM || (HD == 128 && !F8 && !FUSED), "streamed: decode_stream");
   // CPW chunks per wave: an item covers DEC_WAVES * CPW * 32 tokens; every chunk's loads of
@@ -764,10 +767,9 @@ __global__ __launch_bounds__(256, (STREAM ? 2 : 1)) void decode_attn_kernel(
     // items on 0.84 to 0.99 of the time, 480 still 1.1): only the device knows the contexts.
     if (n_items > static_cast<int>(gridDim.x)) {
       __syncthreads();
-      decode_stream(smem, q, g, block_tables, max_blocks, seq_lens, B, n_q, scale_log2, part_o, part_ml, max_splits, kv_begin, split_base, stream);
+      decode_stream(smem, q, g, block_tables, max_blocks, seq_lens, B, n_q, scale_log2, part_o, part_ml, max_splits, kv_begin, split_base);
       return;
     }
-    if (blockIdx.x == 0 && tid == 0) stream[B + 1] = 0;
   }
 
   for (int item = blockIdx.x; item < n_items; item += gridDim.x) {
@@ -921,6 +923,9 @@ __global__ __launch_bounds__(256, (STREAM ? 2 : 1)) void decode_attn_kernel(
       if (d == 0) {
         part_ml[pidx * 2] = mm;
         part_ml[pidx * 2 + 1] = ll;
+        if constexpr (STREAM) {
+          if (pos + 1 == s_pre[b + 1] && slot + 1 < max_splits) end_parts(part_ml + (pidx + 1) * 2);
+        }
       }
     }
     __syncthreads();  // s_o / s_ml are rewritten by the next item
@@ -933,11 +938,12 @@ __global__ __launch_bounds__(256, (STREAM ? 2 : 1)) void decode_attn_kernel(
 // is weighted by its factor, broadcast with v_readlane.  The former one-thread-per-dim
 // form walked the splits with dependent broadcast loads twice (35 us per layer at B = 616).
 constexpr int COMBINE_WAVES = 4;
-template <int HD>
+// STREAM: the parts of a pair that has any end where the attention says (PARTS_END, items alike), else their number follows from the length.
+template <int HD, bool STREAM>
 __global__ __launch_bounds__(64 * COMBINE_WAVES) void decode_combine_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_ml, const int* __restrict__ seq_lens, int n_q,
     int max_splits, int split_tokens, int n_bq, bf16_t* __restrict__ out, const int* __restrict__ kv_begin,
-    const int* __restrict__ split_base, const int* __restrict__ stream, int B, int n_kv) {
+    const int* __restrict__ split_base) {
   constexpr int PER = HD / 64;  // dims per lane
   const int lane = threadIdx.x & 63;
   const int bq = blockIdx.x * COMBINE_WAVES + (threadIdx.x >> 6);
@@ -945,22 +951,15 @@ __global__ __launch_bounds__(64 * COMBINE_WAVES) void decode_combine_kernel(
   const int b = bq / n_q;
   const float2* ml = reinterpret_cast<const float2*>(part_ml) + static_cast<size_t>(bq) * max_splits + lane;
   float2 mlv{-INFINITY, 0.f};
-  // heads of 128, the streamed ones: every slot's (m, l) before the number of parts is known, what the loads below say arrives at the same time
-  if (HD == 128 && lane < max_splits) mlv = *ml;
+  if (lane < max_splits) mlv = *ml;   // every slot's, before the number of parts is known: what the loads below say arrives at the same time
   const int own = max(0, seq_lens[b] - (kv_begin ? kv_begin[b] : 0));
   // <= max_splits <= 64 (host check); slots 0 .. split_base[b]-1 hold the shared-prefix partials
-  int parts = (own + split_tokens - 1) / split_tokens;
-  if constexpr (HD == 128) {
-    int waves = 0, first = 0, next = 0, total = 0;
-    if (stream != nullptr) waves = stream[B + 1], first = stream[b], next = stream[b + 1], total = stream[B] * n_kv;
-    if (waves > 0) {  // decode_stream: how its waves' ranges cut the pair's chunks
-      const int n = next - first;
-      const int c0 = first * n_kv + (bq - b * n_q) / (n_q / n_kv) * n;
-      parts = n > 0 ? stream_wave(c0 + n - 1, total, waves) - stream_wave(c0, total, waves) + 1 : 0;
-    }
+  const int base = split_base ? split_base[b] : 0;
+  int ns = base + (own + split_tokens - 1) / split_tokens;
+  if constexpr (STREAM) {   // (a row without tokens has no parts and no end)
+    const unsigned long long ends = __ballot(lane >= base && (lane >= max_splits || __builtin_bit_cast(uint32_t, mlv.x) == PARTS_END));
+    ns = own == 0 ? base : ends != 0 ? __ffsll(ends) - 1 : 64;
   }
-  const int ns = (split_base ? split_base[b] : 0) + parts;
-  if (HD != 128 && lane < ns) mlv = *ml;
   if (lane >= ns) mlv = float2{-INFINITY, 0.f};
   float mm = mlv.x;
 #pragma unroll
@@ -1127,6 +1126,13 @@ void launch_decode(const bf16_t* q, KVGeom g, const int* tables, int max_blocks,
                    int n_q, float sl, float* ws, int max_splits, bf16_t* out, const Cascade& cas,
                    hipStream_t stream, const FusedArgs& fa = FusedArgs{}) {
   constexpr int DEC_SPLIT = DEC_WAVES * CHUNK * CPW;
+  const int shared_slots = cas.kv_begin ? DEC_MAX_SHARED_SPLITS : 0;
+  // Streamed from 256 pairs of row and kv head on (8 or 2 kv heads; times over those of the items): 256 pairs 0.99 to 1.01 up to 1050 tokens, 0.92 at 1700,
+  // 0.91 at 8000; 320: 0.99, 0.93, 0.93; 512: 0.95 at 250, 0.94, 0.88.  Below them it varies: 1.01 to 1.03 up to 600 tokens (this instance's items),
+  // 160 pairs 1.03 to 1.05 at 1700 to 4000 and 0.96 at 8000, 192 and 224 0.91 to 0.97 there, 64 to 128 0.94 to 1.05 at 2500 and 4000.
+  // (With one slot a row's range could be cut into more parts than there are slots.)
+  const bool streamed = HD == 128 && !F8 && !FUSED && n_q / g.n_kv <= STREAM_G && B * g.n_kv >= 256 && max_splits - shared_slots >= 2;
+  if (!streamed) max_splits = std::min(max_splits, (max_blocks * BS + DEC_SPLIT - 1) / DEC_SPLIT + shared_slots);   // no slot to spare
   float* part_o = ws;
   float* part_ml = ws + static_cast<size_t>(B) * n_q * max_splits * HD;
   if (cas.kv_begin != nullptr && cas.max_items > 0) {
@@ -1137,7 +1143,7 @@ void launch_decode(const bf16_t* q, KVGeom g, const int* tables, int max_blocks,
                        cas.items, cas.n_items, cas.max_items, cas.split_tokens, part_o, part_ml, max_splits);
   }
   // fixed (graph-safe) grid striding over the live items: one full wave of resident workgroups
-  auto run = [&](auto stream_c, int* table) {
+  auto run = [&](auto stream_c) {
     constexpr bool STREAM = decltype(stream_c)::value;
     static int resident = 0;
     if (resident == 0) {
@@ -1149,22 +1155,23 @@ void launch_decode(const bf16_t* q, KVGeom g, const int* tables, int max_blocks,
     }
     const int grid = static_cast<int>(std::min<long>(static_cast<long>(B) * g.n_kv * max_splits, resident));
     hipLaunchKernelGGL((decode_attn_kernel<HD, F8, CPW, FUSED, STREAM>), dim3(grid), dim3(256), 0, stream, q, g, tables, max_blocks,
-                       seq_lens, B, n_q, sl, part_o, part_ml, max_splits, cas.kv_begin, cas.split_base, fa, table);
+                       seq_lens, B, n_q, sl, part_o, part_ml, max_splits, cas.kv_begin, cas.split_base, fa);
   };
-  // Streamed from 256 pairs of row and kv head on: below them the items rarely are more than a round, and the merge's look at how the batch was
-  // cut costs 0.4 us (10 rows of 8 kv heads 2 to 5 % of 9 to 25 us; 256 pairs: 60 tokens +0.5 us, 250 +0.5, 1050 -0.9, 2500 -4).
-  int* table = nullptr;
-  if constexpr (HD == 128 && !F8 && !FUSED) {
-    // (its table lies behind the partials; with one slot a row's range could be cut into more parts than there are slots)
-    if (n_q / g.n_kv <= STREAM_G && B * g.n_kv >= 256 && max_splits - (cas.kv_begin ? DEC_MAX_SHARED_SPLITS : 0) >= 2)
-      table = reinterpret_cast<int*>(part_ml + static_cast<size_t>(B) * n_q * max_splits * 2);
-    if (table != nullptr) run(std::true_type{}, table);
-  }
-  if (table == nullptr) run(std::false_type{}, nullptr);
   const int n_bq = B * n_q;
-  hipLaunchKernelGGL(decode_combine_kernel<HD>, dim3((n_bq + COMBINE_WAVES - 1) / COMBINE_WAVES),
-                     dim3(64 * COMBINE_WAVES), 0, stream, part_o, part_ml, seq_lens, n_q, max_splits, DEC_SPLIT, n_bq,
-                     out, cas.kv_begin, cas.split_base, table, B, g.n_kv);
+  auto merge = [&](auto stream_c) {
+    hipLaunchKernelGGL((decode_combine_kernel<HD, decltype(stream_c)::value>), dim3((n_bq + COMBINE_WAVES - 1) / COMBINE_WAVES),
+                       dim3(64 * COMBINE_WAVES), 0, stream, part_o, part_ml, seq_lens, n_q, max_splits, DEC_SPLIT, n_bq,
+                       out, cas.kv_begin, cas.split_base);
+  };
+  if constexpr (HD == 128 && !F8 && !FUSED) {
+    if (streamed) {
+      run(std::true_type{});
+      merge(std::true_type{});
+      return;
+    }
+  }
+  run(std::false_type{});
+  merge(std::false_type{});
 }
 
 // ----------------------------------------------------------------- prefill

@@ -9,6 +9,7 @@ from byzantine_consensus_llm_agents_amd.engine.cascade import CascadeTables, pla
 from byzantine_consensus_llm_agents_amd.ops import reference as R
 
 pytestmark = pytest.mark.gpu
+PARTS_END = 0x7fc0e4d1   # csrc/kernels/attention.hip
 
 
 @pytest.fixture(scope="module")
@@ -43,6 +44,35 @@ def _check(ops, q, k, v, tables, seq, *more):
     out = ops.paged_attention_decode(q, k, v, 0, tables, seq, 128 ** -0.5, *more)
     torch.testing.assert_close(out.float(), ref.float(), atol=2e-2, rtol=2e-2)   # (as the other decode tests: P in bf16, one rounding of the result)
     return out
+
+
+def _marks(ops, ws, B, n_q, max_blocks, cascade=False):
+    """[B, n_q] how many parts the merge found behind the shared slots' end, from the marks that the attention left; -1 without one."""
+    slots = ops.library.bcg_decode_max_splits(max_blocks * 16, int(cascade))
+    m = ws[B * n_q * slots * 128:][:B * n_q * slots * 2].view(torch.int32).view(B, n_q, slots, 2)[..., 0]
+    at = (m == PARTS_END).to(torch.int32)
+    return torch.where(at.any(-1), at.argmax(-1), torch.full_like(at[..., 0], -1).to(torch.int64))
+
+
+# workspaces that hold anything: NaN, marks of an end in every slot, the parts of a batch with other lengths.  Items (one round of them) and streamed ranges;
+# rows without tokens; rows at the edges of a split
+@pytest.mark.parametrize("lens", [[0, 1, 255, 256, 257, 30, 0, 12] * 4, [0, 1, 255, 256, 257, 1900, 700, 0] * 8], ids=["items", "streamed"])
+def test_merge_takes_this_calls_parts(ops, lens):
+    n_kv, G, B = 8, 5, len(lens)
+    k, v, tables, seq = _case(lens, n_kv, 5)
+    q = torch.randn(B, G * n_kv, 128, device="cuda").bfloat16()
+    keep = seq > 0
+    ref = R.paged_attention(q[keep], k, v, 0, tables[keep].contiguous(), torch.arange(int(keep.sum()) + 1, dtype=torch.int32, device="cuda"), seq[keep],
+                            128 ** -0.5)
+    n = ops.decode_workspace_numel(B, G * n_kv, 128, tables.shape[1], cascade=False)
+    fills = [torch.full((n,), x, dtype=torch.int32, device="cuda").view(torch.float32) for x in (0x7fc00000, PARTS_END)]
+    other = torch.empty(n, device="cuda")
+    ops.paged_attention_decode(q, k, v, 0, tables, seq.flip(0).clamp(max=200), 128 ** -0.5, other)
+    outs = [ops.paged_attention_decode(q, k, v, 0, tables, seq, 128 ** -0.5, ws) for ws in (*fills, other)]
+    torch.testing.assert_close(outs[0][keep].float(), ref.float(), atol=2e-2, rtol=2e-2)
+    assert not outs[0][~keep].any() and all(torch.equal(outs[0], o) for o in outs[1:])
+    parts, items = _marks(ops, fills[0], B, G * n_kv, tables.shape[1]), (seq + 255) // 256
+    assert torch.equal(parts, items[:, None].expand_as(parts).where(keep[:, None], torch.full_like(parts, -1))) == (int(items.sum()) * n_kv <= 512)
 
 
 # 1 to 8 query heads a kv head; rows of one token, one chunk, one split and their neighbours, rows without tokens at the ends and between; all rows equal
