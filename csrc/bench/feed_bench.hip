@@ -125,12 +125,12 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
             const uint32_t m0v = __builtin_amdgcn_readfirstlane(lds_base + (p & 15) * 4096 + wave * 1024);
             const uint32_t vo = pv + (p & 7) * 32 * row_bytes;
             if (LAYOUT == 0 && (p & 1))
-              asm volatile("s_mov_b32 m0, %3\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
+              asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
                            :
                            : "v"(vo), "s"(sW), "s"(kb), "s"(m0v)
                            : "memory", "m0");
             else
-              asm volatile("s_mov_b32 m0, %3\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
+              asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
                            :
                            : "v"(vo), "s"(sX), "s"(kb), "s"(m0v)
                            : "memory", "m0");

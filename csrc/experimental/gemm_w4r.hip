@@ -151,7 +151,7 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
   auto piece = [&](int slot, int i, int kt, const i32x4& s) {
     const uint32_t m0v = __builtin_amdgcn_readfirstlane(lds_base + slot * XSLOT + i * 4096 + wave * 1024);
     const uint32_t soff = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(kt) * (BK * 2));
-    asm volatile("s_mov_b32 m0, %3\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
                  :
                  : "v"(voffX + i * strideX), "s"(s), "s"(soff), "s"(m0v)
                  : "memory", "m0");

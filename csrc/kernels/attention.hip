@@ -567,8 +567,8 @@ __device__ __forceinline__ void decode_stream(
   }
   const uint32_t lds = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem));
   const uint32_t ring = lds + w * STREAM_RING, qring = lds + 4 * STREAM_RING + w * 2 * STREAM_Q;
-  auto dma = [&](uint32_t off, const unsigned char* base, uint32_t to) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(to) : "memory", "m0");
+  auto dma = [&](uint32_t off, const unsigned char* base, uint32_t to) {   // (s_nop: the wait state of an LDS load behind a scalar write of m0)
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(to) : "memory", "m0");
   };
   const unsigned char* kc = reinterpret_cast<const unsigned char*>(g.k);
   const unsigned char* vc = reinterpret_cast<const unsigned char*>(g.v);
@@ -1681,7 +1681,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
                                         : vc + base + (r4 * 1024 + lane_v);
       const uint32_t m0v = __builtin_amdgcn_readfirstlane(
           static_cast<uint32_t>(reinterpret_cast<uintptr_t>(slot + (i < 16 ? i * 1024 : KBYTES + (i - 16) * 1024))));
-      asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(m0v) : "memory", "m0");
+      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(m0v) : "memory", "m0");
     }
   };
 

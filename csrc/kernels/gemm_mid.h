@@ -122,11 +122,12 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
   auto at = [&](int s) { const int t = s + rot; return t >= n ? t - n : t; };
   auto valid = [&](int s) { return s < n && at(s) * H + half < nb; };
   auto k_offset = [&](int s) { return __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(kb0 + at(s) * H + half) * 128); };
+  // (s_nop: an LDS load needs a wait state behind a scalar write of m0, which hipcc does not put between instructions of one asm statement)
   auto fetch = [&](int u, uint32_t slot, uint32_t ko) {
     if (u < DX)
-      asm volatile("s_add_u32 m0, %3, %4\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(vo[u]), "s"(sX), "s"(ko), "s"(slot), "n"(u * RG * 1024) : "memory", "m0", "scc");
+      asm volatile("s_add_u32 m0, %3, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(vo[u]), "s"(sX), "s"(ko), "s"(slot), "n"(u * RG * 1024) : "memory", "m0", "scc");
     else
-      asm volatile("s_add_u32 m0, %3, %4\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(vo[u]), "s"(sW), "s"(ko), "s"(slot), "n"(u * RG * 1024) : "memory", "m0", "scc");
+      asm volatile("s_add_u32 m0, %3, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(vo[u]), "s"(sW), "s"(ko), "s"(slot), "n"(u * RG * 1024) : "memory", "m0", "scc");
   };
   auto aim = [&](int s) { sX[2] = valid(s) ? range_x : 0, sW[2] = valid(s) ? range_w : 0; };
   auto fetch_stage = [&](int s) {

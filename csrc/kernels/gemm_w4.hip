@@ -289,7 +289,8 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
   };
   // DMA cursor: stream tile t + 2 is K-tile dk0 + ktd of item jd, whose descriptors are dX / dW
   int jd = 0, ktd = 0, dk0 = gc.k0, dnk = gc.nk;
-  // stream tile t = K-tile kt of the DMA cursor's item: M0 write + piece in one statement
+  // stream tile t = K-tile kt of the DMA cursor's item: M0 write + piece in one statement (with the wait state that an LDS load needs behind a scalar
+  // write of M0: hipcc puts it between its own, not between instructions of one asm statement)
   auto dma = [&](int t, int kt, int q, const i32x4& sX, const i32x4& sW) {
     const uint32_t kb = static_cast<uint32_t>(dk0 + kt) * (BK * 2);
     const bool isx = q < 8;
@@ -297,12 +298,12 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
     const uint32_t soff = __builtin_amdgcn_readfirstlane(kb);
     const uint32_t m0v = dma_m0(t, q);
     if (isx) {
-      asm volatile("s_mov_b32 m0, %3\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
+      asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
                    :
                    : "v"(vX[i]), "s"(sX), "s"(soff), "s"(m0v)
                    : "memory", "m0");
     } else {
-      asm volatile("s_mov_b32 m0, %3\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
+      asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
                    :
                    : "v"(vW[i]), "s"(sW), "s"(soff), "s"(m0v)
                    : "memory", "m0");
@@ -749,7 +750,7 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
       for (int q = 0; q < 16; ++q) {
         const uint32_t soff = __builtin_amdgcn_readfirstlane(base + q * 1024);
         const uint32_t m0v = __builtin_amdgcn_readfirstlane(lds_w + b * 65536 + q * 1024);
-        asm volatile("s_mov_b32 m0, %3\n\tbuffer_load_dwordx4 %0, %1, %2 offen sc1 lds"
+        asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen sc1 lds"
                      :
                      : "v"(static_cast<uint32_t>(lane) * 16), "s"(srd), "s"(soff), "s"(m0v)
                      : "memory", "m0");

@@ -96,3 +96,17 @@ def test_built_library_carries_tree_stamp():
 def test_runtime_module_stamp():
     from byzantine_consensus_llm_agents_amd import runtime
     assert runtime._native.source_hash == build.runtime_source_hash()
+
+
+def test_lds_loads_wait_for_m0():
+    """An LDS load reads M0 one wait state after a scalar write of it at the earliest; the compiler does not look into asm statements for that."""
+    import re
+    found = 0
+    for path in glob.glob(os.path.join(build.CSRC, "**", "*.h*"), recursive=True):
+        for asm in re.findall(r'asm volatile\(\s*((?:"[^"]*"\s*)+)', open(path).read()):
+            steps = re.split(r"\\n(?:\\t)?", asm.replace('"', "").strip())
+            for a, b in zip(steps, steps[1:]):
+                if re.match(r"s_\w+ m0,", a):
+                    found += 1
+                    assert b.strip().startswith("s_nop"), (path, asm)
+    assert found >= 8
