@@ -12,7 +12,8 @@
 //     has only so many fetches under way;
 //   * the tile is free in steps of 16 (8 to 2 accumulator blocks a side), so a plan (below) finds one whose tiles x K-splits fill one round;
 //   * the eight XCDs start K an eighth apart: in step, all CUs read the same 256 bytes of every row, a few channels' worth (101 x 24576 x 4096
-//     48 -> 41 us); within an XCD they stay in step, so X and a W shared by several row tiles are fetched into its L2 once;
+//     48 -> 41 us); within an XCD they stay in step, so X and a W shared by several row tiles are fetched into its L2 once (a column tile whose row
+//     tiles lie on two XCDs keeps the first one's start: equal rows stay equal);
 //   * what runs once is kept short: a launch finds the instruction cache cold, and an unrolled epilogue of 10 KB took 4.2 us of fetches, this 2.2.
 // Measured in a captured graph, other weights each call, us, tile kernels or library before -> here: 101 rows 24576 x 4096 gated 55 -> 45, 6144 x 4096
 // 22.3 -> 20.4, 4096 x 4096 21 -> 15, 4096 x 12288 37 -> 35; 448 rows 5120 x 5120 51 -> 39, 5120 x 17408 109 -> 99, 6144 x 4096 47 -> 33;
@@ -117,8 +118,10 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
     vo[u] = v0 + (EPI == EPI_SILU_MUL && u >= DX ? ((r >> 4) & 1) * a.inter + (r >> 5) * 16 + (r & 8) : r) * row_bytes;
   }
   const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem)) + half * U * 2048 + rg0 * 1024;
-  // stage s of the walk is stage (s + rot) mod n of K
-  const int rot = xcd * n / 8;
+  // stage s of the walk is stage (s + rot) mod n of K.  rot: of the XCD that has the column tile's first row tile, so that rows of one call add K in
+  // one order whichever row tile they are in (a column tile's row tiles may lie on two)
+  const int first = rest * a.m_tiles, home = first < rem * (q + 1) ? first / (q + 1) : rem + (first - rem * (q + 1)) / q;
+  const int rot = home * n / 8;
   auto at = [&](int s) { const int t = s + rot; return t >= n ? t - n : t; };
   auto valid = [&](int s) { return s < n && at(s) * H + half < nb; };
   auto k_offset = [&](int s) { return __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(kb0 + at(s) * H + half) * 128); };

@@ -72,6 +72,20 @@ def test_every_tile(ops, tile):
             assert _err(_run(ops, plan, 2, xq, wq, res.clone(), residual=res, scales=(xs, ws)), y8 + res.float()) < TOL
 
 
+# (tile, row tiles, column tiles, parts): row tiles of a column tile on two XCDs in some columns; the last one partly filled; K in parts
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile,m_tiles,n_tiles,split", [(22, 3, 75, 1), (22, 3, 25, 3), (0, 5, 50, 1), (7, 2, 9, 1), (14, 3, 7, 6), (1, 7, 1, 1)])
+def test_equal_rows_have_equal_results(ops, tile, m_tiles, n_tiles, split):
+    (mt, nt), K = TILES[tile], 4096
+    torch.manual_seed(tile)
+    M, N = 16 * mt * m_tiles - 13, 16 * nt * n_tiles
+    x = torch.randn(1, K // 2, device="cuda").bfloat16().repeat(M, 2)
+    w = torch.randn(N, K // 2, device="cuda").bfloat16().repeat(1, 2)
+    w[:, K // 2:].neg_()       # the sums are 0 but for what the order of their terms rounds
+    out = _run(ops, tile | split << 8, 0, x, w, torch.empty(M, N, dtype=torch.bfloat16, device="cuda"))
+    assert (out == out[:1]).all() and 0 < out.abs().max() < 1e-2
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(33, 2048, 1152), (100, 2048, 1152), (1024, 2048, 1152), (1025, 2048, 1152), (1536, 2048, 1152),
                                    (90, 544, 192), (400, 32, 4096)])
