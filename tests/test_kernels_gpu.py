@@ -239,6 +239,30 @@ def test_paged_attention_prefill32(hip, n_q, n_kv, tile_rows):
         _close(out, ref, atol=2e-2)
 
 
+@pytest.mark.parametrize("tile_rows", [64, 128, 256])
+def test_prefill_repeats_itself(hip, tile_rows):
+    """Every launch gives the same bits, and the running maximum is that of the chunk at hand also where each chunk's scores are far above the last
+    one's (keys that grow with their position; 2^127 is 12 chunks away)."""
+    gen = torch.Generator().manual_seed(7)
+    n_q, n_kv, hd, spec = 40, 8, 128, [(0, 700), (300, 500), (64, 257), (0, 129), (500, 1)]
+    ctx = [a + b for a, b in spec]
+    k, v = _caches(1, 256, n_kv, hd)
+    tables = _tables(len(spec), ctx, 256, 64, gen)
+    for b, n in enumerate(ctx):
+        for i in range(-(-n // 16)):
+            k[0, int(tables[b, i])] *= 1 + i // 2
+    q_start = [0]
+    for _, n in spec:
+        q_start.append(q_start[-1] + n)
+    q = torch.randn(q_start[-1], n_q, hd, device="cuda", dtype=torch.bfloat16)
+    qs, seq = (torch.tensor(t, dtype=torch.int32, device="cuda") for t in (q_start, ctx))
+    tiles = torch.tensor([(i, t, min(t + tile_rows, q_start[i + 1])) for i in range(len(spec)) for t in range(q_start[i], q_start[i + 1], tile_rows)],
+                         dtype=torch.int32, device="cuda")
+    outs = [hip.paged_attention_prefill(q, k, v, 0, tables, qs, seq, hd ** -0.5, None, tiles, tile_rows=tile_rows) for _ in range(6)]
+    _close(outs[0], R.paged_attention(q, k, v, 0, tables, qs, seq, hd ** -0.5), atol=2e-2)
+    assert all(torch.equal(o, outs[0]) for o in outs)
+
+
 def _sample_state(B, V, rows, base, maxnew, temp, dev="cuda"):
     return dict(
         fsm_base=torch.tensor(base, dtype=torch.int32, device=dev),
