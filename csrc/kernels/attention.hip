@@ -1530,10 +1530,10 @@ __device__ __forceinline__ void attn32_scores(const unsigned char* slot, int k_l
     s0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka[kk][0], bq[kk], s0, 0, 0, 0);
     s1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka[kk][1], bq[kk], s1, 0, 0, 0);
   }
-  // the maxima below are asm, in front of which hipcc puts no wait states: 20 from a 16-pass product to a vector read of its result.  (Without them
-  // the maximum was taken over what the registers held before, in places: right but for the last bit, another one each time, as long as the
-  // scores of two chunks are alike.)
-  asm volatile("s_nop 15\n\ts_nop 3" : "+v"(s0), "+v"(s1));
+  // the maxima below are asm, in front of which hipcc puts no wait states: 12 from a product of 8 passes to a vector read of its result, what it puts in
+  // front of its own.  (Without them the maximum was taken over what the registers held before, in places: right but for the last bit, another one
+  // each time, as long as the scores of two chunks are alike.)
+  asm volatile("s_nop 11" : "+v"(s0), "+v"(s1));
   // accumulator i of tile u is token 32u + 16(i>>3) + 8h + (i&7)
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
