@@ -94,17 +94,47 @@ def test_ranges(ops, kind, G):
     out = ops.paged_attention_decode(q, k, v, 0, t, seq, 128 ** -0.5)
     torch.testing.assert_close(out[keep].float(), ref.float(), atol=2e-2, rtol=2e-2)
     assert not out[~keep].any()                 # a row without tokens is zeros, as from the items
+    assert int(((seq + 255) // 256).sum()) * n_kv > 512   # (more than a round of items)
     assert torch.equal(out, ops.paged_attention_decode(q, k, v, 0, t, seq, 128 ** -0.5))
 
 
+def _streamed(ops, q, k, v, tables, seq, cascade=None):
+    """The call's result; its parts are not the items': the step was streamed."""
+    B, n_q, _ = q.shape
+    ws = torch.full((ops.decode_workspace_numel(B, n_q, 128, tables.shape[1], cascade=cascade is not None),), float("nan"), device="cuda")
+    out = _check(ops, q, k, v, tables, seq, ws, cascade)
+    parts = _marks(ops, ws, B, n_q, tables.shape[1], cascade is not None)
+    begin = 0 if cascade is None else cascade.kv_begin[:B]
+    base = 0 if cascade is None else cascade.split_base[:B, None]
+    items = (seq - begin + 255) // 256
+    assert int(items.sum()) * k.shape[2] > 512
+    assert not torch.equal(parts - base, items[:, None].expand_as(parts))
+    return out
+
+
 def test_most_rows_and_longest_context(ops):
-    """As many rows as a call takes, and a context of the most slots."""
+    """As many rows as a call takes, and contexts of the most slots (no slot to spare: the ranges are so long that a row's parts fit) among short ones."""
     rng = random.Random(1)
     k, v, tables, seq = _case([rng.randint(1, 70) for _ in range(2048)], 2, 1)
-    _check(ops, torch.randn(2048, 8, 128, device="cuda").bfloat16(), k, v, tables, seq)
+    _streamed(ops, torch.randn(2048, 8, 128, device="cuda").bfloat16(), k, v, tables, seq)
     limit = ops.decode_max_context(False)
-    k, v, tables, seq = _case([limit] + [rng.randint(1, 300) for _ in range(300)], 1, 2, max_blocks=limit // 16)
-    _check(ops, torch.randn(301, 5, 128, device="cuda").bfloat16(), k, v, tables, seq)
+    assert ops.library.bcg_decode_max_splits(limit, 0) == 64
+    for lens in ([limit] + [rng.randint(1, 300) for _ in range(700)], [limit, limit - 1, 5, limit - 255] * 3 + [rng.randint(1, 300) for _ in range(300)]):
+        k, v, tables, seq = _case(lens, 1, 2, max_blocks=limit // 16)
+        _streamed(ops, torch.randn(len(lens), 5, 128, device="cuda").bfloat16(), k, v, tables, seq)
+
+
+def test_longest_context_behind_shared_prefixes(ops):
+    """The slots of the shared pass taken, the own ones at their limit."""
+    rng = random.Random(4)
+    n_kv, G, shared, limit = 2, 5, 23, ops.decode_max_context(True)
+    assert ops.library.bcg_decode_max_splits(limit, 1) == 64
+    lens = [limit, limit - 100] + [shared * 16 + rng.randint(1, 600) for _ in range(250)]
+    k, v, tables, seq = _case(lens, n_kv, 3, shared, max_blocks=limit // 16)
+    t = CascadeTables(len(lens), "cuda")
+    t.upload(plan_groups([(i, tables[i, :-(-n // 16)].tolist()) for i, n in enumerate(lens)]), heads_per_kv=G)
+    assert int(t.split_base[0]) > 0
+    _streamed(ops, torch.randn(len(lens), G * n_kv, 128, device="cuda").bfloat16(), k, v, tables, seq, t)
 
 
 def test_behind_shared_prefixes_and_replayed(ops):
@@ -116,7 +146,7 @@ def test_behind_shared_prefixes_and_replayed(ops):
     q = torch.randn(B, G * n_kv, 128, device="cuda").bfloat16()
     t = CascadeTables(B, "cuda")
     t.upload(plan_groups([(i, tables[i, :-(-n // 16)].tolist()) for i, n in enumerate(lens)]), heads_per_kv=G)
-    _check(ops, q, k, v, tables, seq, None, t)
+    _streamed(ops, q, k, v, tables, seq, t)
     ws = torch.empty(ops.decode_workspace_numel(B, G * n_kv, 128, tables.shape[1]), dtype=torch.float32, device="cuda")
     args = (q, k, v, 0, tables, seq, 128 ** -0.5, ws)
     ops.paged_attention_decode(*args)

@@ -46,30 +46,75 @@ def _run(ops, plan, epi, x, w, out, bias=None, residual=None, scales=(None, None
     return out
 
 
-# rows: one, a tile's last, its first of a second one; columns not a multiple of the tile; K: one block, odd numbers of blocks, splits of unequal length
-@pytest.mark.gpu
-@pytest.mark.parametrize("tile", range(len(TILES)), ids=[f"{16 * m}x{16 * n}" for m, n in TILES])
-def test_every_tile(ops, tile):
+# rows: one, a tile's last, its first of a second one; columns not a multiple of the tile; K in 128-byte blocks of a row: one, odd and even numbers of
+# them, parts of unequal length and of one block, as many parts as a plan may have (the last workgroup adds four at a time)
+def _sizes(tile):
     mt, nt = TILES[tile]
+    return ((1, 16, 1, 1), (16 * mt, 16 * nt, 5, 1), (16 * mt + 1, 32 * nt + 16, 11, 3), (16 * mt - 7, 16 * nt + 32, 17, 2),
+            (16 * mt, 32 * nt, 10, 6), (16 * mt + 3, 16 * nt + 16, 16, 8), (5, 32, 8, 8))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("f8", [False, True], ids=["bf16", "fp8"])
+@pytest.mark.parametrize("tile", range(len(TILES)), ids=[f"{16 * m}x{16 * n}" for m, n in TILES])
+def test_every_tile(ops, tile, f8):
     torch.manual_seed(tile)
-    for M, N, K, split in ((1, 16, 64, 1), (16 * mt, 16 * nt, 320, 1), (16 * mt + 1, 32 * nt + 16, 704, 3), (16 * mt - 7, 16 * nt + 32, 1088, 2)):
+    for M, N, blocks, split in _sizes(tile):
+        K = blocks * (128 if f8 else 64)
         x = torch.randn(M, K, device="cuda").bfloat16()
         w = (torch.randn(N, K, device="cuda") * K ** -0.5).bfloat16()
         bias, res = torch.randn(N, device="cuda").bfloat16(), torch.randn(M, N, device="cuda").bfloat16()
+        scales, plan = (None, None), tile | split << 8
         y = x.float() @ w.float().t()
-        plan = tile | split << 8
+        if f8:
+            x, w = x.to(torch.float8_e4m3fn), (w * 8).to(torch.float8_e4m3fn)
+            scales = torch.rand(M, device="cuda") + 0.5, (torch.rand(N, device="cuda") + 0.5) / 8
+            y = x.float() @ w.float().t() * scales[0][:, None] * scales[1]
         nan = lambda n: torch.full((M, n), float("nan"), dtype=torch.bfloat16, device="cuda")   # noqa: E731
-        assert _err(_run(ops, plan, 0, x, w, nan(N), bias=bias), y + bias.float()) < TOL
-        assert _err(_run(ops, plan, 2, x, w, res.clone(), residual=res), y + res.float()) < TOL
-        if N % 32 == 0 and nt % 2 == 0:
+        assert _err(_run(ops, plan, 0, x, w, nan(N), scales=scales), y) < TOL
+        assert _err(_run(ops, plan, 0, x, w, nan(N), bias=bias, scales=scales), y + bias.float()) < TOL
+        assert _err(_run(ops, plan, 2, x, w, res.clone(), residual=res, scales=scales), y + res.float()) < TOL
+        if N % 32 == 0 and TILES[tile][1] % 2 == 0 and not f8:
             want = torch.nn.functional.silu(y[:, :N // 2]) * y[:, N // 2:]
             assert _err(_run(ops, plan, 1, x, w, nan(N // 2)), want) < TOL
-        if K % 128 == 0:
-            xq, wq = x.to(torch.float8_e4m3fn), (w * 8).to(torch.float8_e4m3fn)
-            xs, ws = torch.rand(M, device="cuda") + 0.5, (torch.rand(N, device="cuda") + 0.5) / 8
-            y8 = xq.float() @ wq.float().t() * xs[:, None] * ws
-            assert _err(_run(ops, plan, 0, xq, wq, nan(N), bias=bias, scales=(xs, ws)), y8 + bias.float()) < TOL
-            assert _err(_run(ops, plan, 2, xq, wq, res.clone(), residual=res, scales=(xs, ws)), y8 + res.float()) < TOL
+
+
+# NaN in the bytes behind every operand's end, infinities and NaN in rows of x: nobody else's result changes
+@pytest.mark.gpu
+@pytest.mark.parametrize("f8", [False, True], ids=["bf16", "fp8"])
+@pytest.mark.parametrize("tile,split", [(0, 1), (2, 3), (7, 1), (13, 8), (16, 2), (24, 1)])
+def test_non_finite(ops, tile, split, f8):
+    (mt, nt), K = TILES[tile], 128 * 9
+    torch.manual_seed(tile)
+    M, N = 16 * mt + 5, 32 * nt + 16
+    dtype = torch.float8_e4m3fn if f8 else torch.bfloat16
+
+    def behind(t):     # a copy that lies in front of NaN
+        whole = torch.full((t.shape[0] + 300, *t.shape[1:]), float("nan"), device="cuda").to(t.dtype)
+        whole[:len(t)] = t
+        return whole[:len(t)]
+    x, w = torch.randn(M, K, device="cuda").to(dtype), torch.randn(N, K, device="cuda").to(dtype)
+    bias, res = torch.randn(N, device="cuda").bfloat16(), torch.randn(M, N, device="cuda").bfloat16()
+    scales = (torch.rand(M, device="cuda"), torch.rand(N, device="cuda")) if f8 else (None, None)
+    bad = [0, 16 * mt - 1, M - 1]
+    xb = x.clone()
+    xb.view(torch.uint8 if f8 else torch.int16)[bad[0], 3] = 0x7f if f8 else 0x7fc0
+    xb.view(torch.uint8 if f8 else torch.int16)[bad[1], K - 1] = 0x7f if f8 else 0x7f80
+    xb.view(torch.uint8 if f8 else torch.int16)[bad[2]] = 0x7f if f8 else 0x7fc0
+    good = torch.ones(M, dtype=torch.bool, device="cuda")
+    good[bad] = False
+    for epi in (0, 1, 2):
+        if epi == 1 and (f8 or nt % 2):
+            continue
+        n = (N - 16) if epi == 1 else N
+        wn = w[:n].contiguous()
+        kw = {0: {"bias": bias}, 1: {}, 2: {"residual": res}}[epi]
+        want = _run(ops, tile | split << 8, epi, x, wn, torch.empty(M, n // 2 if epi == 1 else n, dtype=torch.bfloat16, device="cuda"), scales=scales, **kw)
+        out = torch.full((M + 300, want.shape[1]), 7., dtype=torch.bfloat16, device="cuda")
+        _run(ops, tile | split << 8, epi, behind(xb), behind(wn), out[:M], scales=tuple(s if s is None else behind(s) for s in scales),
+             **{k: behind(v) for k, v in kw.items()})
+        assert torch.equal(out[:M][good], want[good]) and want.isfinite().all()
+        assert not out[:M][~good].isfinite().all(-1).any() and (out[M:] == 7).all()
 
 
 # (tile, row tiles, column tiles, parts): row tiles of a column tile on two XCDs in some columns; the last one partly filled; K in parts
