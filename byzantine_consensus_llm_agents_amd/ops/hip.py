@@ -56,6 +56,19 @@ def check_source_stamp(lib: ctypes.CDLL, path: str):
             "`python -m byzantine_consensus_llm_agents_amd.utils.build --force`")
 
 
+def few_rows_stay(M: int, N: int, K: int, gated: bool) -> bool:
+    """33 to 64 rows that the few-row kernel takes (`few_rows_pay`) and the one-round kernel could: whether the first keeps them.
+
+    Times of the one-round kernel over the few-row kernel's at 1018 products of 2.7 M elements of W and more: 0.84 on average, 34 of 1.03 to 1.14, most of
+    them where its plan is 48 x 32 tiles in one part that leave a quarter of the CUs idle and the few-row kernel's rows are whole turns: up to
+    48 rows, K in steps of 512 from 2048 to 4096, 4097 to 6500 columns (gated 2700 to 6500) 1.01 on average, up to 1.14 (44 rows, 6144 x 4096:
+    16.1 us for 17.5).  14 of the others are 1.03 to 1.07 slower.  Smaller W: 0.77 to 0.82, left where the tests of the few-row
+    kernel hold them."""
+    if N * K < 2700000:
+        return True
+    return M <= 48 and K % 512 == 0 and 2048 <= K <= 4096 and (2700 if gated else 4097) <= N <= 6500
+
+
 def load_library(path: str = None) -> ctypes.CDLL:
     global _LIB
     if _LIB is not None:
@@ -492,11 +505,10 @@ def hip_ops() -> SimpleNamespace:
 
     def _mid(x, w, epi):
         """The plan by which the kernel for tens to hundreds of rows takes x W^T (csrc/kernels/gemm_mid.hip says which it does), else
-        None.  33 to 64 rows that the few-row kernel takes: from 2.7 M elements of W on (times over the few-row kernel's 0.74 to 0.97 on average over
-        sizes, the slowest 1.1: 40 rows, 6144 x 4096); smaller ones stay where the tests of that kernel hold them (0.77 to 0.82)."""
+        None (`few_rows_stay`)."""
         M, K = x.shape
         N = w.shape[0]
-        if not (33 <= M <= MID_ROWS and plan.mode == "1") or (M <= SKINNY_ROWS and N * K < 2700000 and few_rows_pay(M, N, 2 * K, epi == 1)):
+        if not (33 <= M <= MID_ROWS and plan.mode == "1") or (M <= SKINNY_ROWS and few_rows_stay(M, N, K, epi == 1) and few_rows_pay(M, N, 2 * K, epi == 1)):
             return None
         p = plan.mid(M, N, K, epi)
         return p if p is not None and _plain(x, w) else None

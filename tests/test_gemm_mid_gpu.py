@@ -267,6 +267,15 @@ def test_plan_takes_one_round_and_refuses_the_rest():
         assert lib.bcg_gemm_mid_plan(*bad) == -1, bad
 
 
+def test_few_rows_that_stay():
+    """33 to 64 rows: the few-row kernel keeps small W and whole turns past 4096 columns, else the one-round kernel has them."""
+    from byzantine_consensus_llm_agents_amd.ops.hip import few_rows_stay
+    for M, N, K, gated, want in ((40, 1024, 2560, False, True), (40, 6144, 3072, False, True), (48, 6144, 3072, False, True), (49, 6144, 3072, False, False),
+                                 (40, 6144, 4096, False, True), (40, 6144, 4608, True, False), (40, 4096, 3072, False, False), (40, 4096, 3072, True, True),
+                                 (40, 8192, 2048, True, False), (40, 6144, 2176, True, False), (40, 6144, 1536, True, False)):
+        assert few_rows_stay(M, N, K, gated) == want, (M, N, K, gated)
+
+
 def test_gemm_nt_refuses_the_configuration(ops_cpu):
     """`gemm_nt` takes the tiles that `GemmPlan.supported` knows: the one-round kernel's number is none of them, whatever `out` and `bias` are."""
     x, w = torch.zeros(100, 4096).bfloat16(), torch.zeros(4096, 4096).bfloat16()
