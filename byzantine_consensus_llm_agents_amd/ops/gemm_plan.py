@@ -17,7 +17,7 @@ import bisect
 import ctypes
 import json
 import os
-from typing import Dict, List, Optional, Tuple
+from typing import Dict, List, Optional, Set, Tuple
 
 TABLE = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "engine", "tuned",
                      "hand_gemm.json")
@@ -53,6 +53,7 @@ class GemmPlan:
                 if lib.bcg_gemm_tile(cfg, ctypes.byref(bm), ctypes.byref(bn)) == 0:
                     self.tiles[cfg] = (bm.value, bn.value)
         self.table: Dict[Tuple[int, int, int, int], Tuple[int, int]] = {}
+        self.kept: Set[Tuple[int, int, int, int]] = set()   # entries that the one-round kernel does not beat
         if table and os.path.exists(table):
             with open(table) as fh:
                 data = json.load(fh)
@@ -61,6 +62,7 @@ class GemmPlan:
                 self.table[(m, n, k, e)] = tuple(choice) if isinstance(choice, list) else (int(choice), 1)
             for (m, n, k, e) in sorted(self.table):     # measured row counts of every shape, in order
                 self.rows.setdefault((n, k, e), []).append(m)
+            self.kept = {tuple(map(int, key.split(","))) for key in data.get("beats_one_round", [])}
             for key, times in data.get("timings_us", {}).items():
                 self.timings[tuple(map(int, key.split(",")))] = times
 
@@ -122,9 +124,16 @@ class GemmPlan:
         return (cfg, 1) if self.supported(cfg, M, N, K, epi) else None
 
     def mid(self, M: int, N: int, K: int, epi: int) -> Optional[int]:
-        """Plan of the kernel for tens to hundreds of rows (csrc/kernels/gemm_mid.hip), None where it is not taken."""
+        """Plan of the kernel for tens to hundreds of rows (csrc/kernels/gemm_mid.hip), None where it is not taken: by its own rule, which rests on a
+        model of its time, and where the table holds the projection and what stood there is faster at the measured row count from M on
+        (``tools/tune_hand_gemm.py --one-round``; 32 of 292 entries by 2 % and more, 256 x 2560 x 5120 21.4 us against 25.3)."""
         if self.mode != "1" or self.lib is None:
             return None
+        if self.kept:
+            ms = self.rows.get((N, K, epi), [])
+            at = bisect.bisect_left(ms, M)
+            if at < len(ms) and (ms[at], N, K, epi) in self.kept:
+                return None
         p = self.lib.bcg_gemm_mid_plan(epi, M, N, K, 0)
         return p if p >= 0 else None
 

@@ -265,6 +265,11 @@ def test_plan_takes_one_round_and_refuses_the_rest():
     for bad in ((0, 32, 4096, 4096, 0), (0, 1537, 4096, 4096, 0), (0, 1025, 4096, 4096, 1), (0, 1025, 512, 4096, 0), (0, 100, 4096, 4100, 0), (0, 100, 4104, 4096, 0), (1, 100, 4112, 4096, 0),
                 (0, 100, 4096, 64, 0), (0, 100, 4096, 128, 0), (0, 100, 512, 192, 0), (0, 100, 512, 1024, 1), (0, 1024, 151936, 5120, 0), (1, 100, 4096, 4096, 1)):
         assert lib.bcg_gemm_mid_plan(*bad) == -1, bad
+    # what the table holds as faster is left too, up to its row count from the one below on
+    assert plan.kept and all(key in plan.table and lib.bcg_gemm_mid_plan(key[3], *key[:3], 0) >= 0 for key in plan.kept)
+    for M, want in ((64, True), (65, False), (256, False), (257, True), (320, True), (321, False), (512, False), (513, True)):
+        assert (plan.mid(M, 2560, 5120, 0) is not None) == want, M
+    assert plan.mid(256, 2560, 5120, 2) is not None and GemmPlan(lib, table=None).mid(256, 2560, 5120, 0) is not None
 
 
 def test_few_rows_that_stay():

@@ -12,6 +12,12 @@ The library path uses the shipped TunableOp table (what the engine runs).
 Weights rotate over enough copies to exceed the 256 MiB Infinity Cache, so
 every call streams its weights from HBM as in a real decode step.  Median of
 --reps timed calls per candidate (CUDA events), after a correctness check.
+
+  python tools/tune_hand_gemm.py --one-round
+
+times every entry of the shipped table from 33 rows on against the one-round kernel
+(csrc/kernels/gemm_mid.hip), both as the entry points launch them, in captured graphs, and lists
+those that it does not beat (``beats_one_round``, by 2 % and more).
 """
 import argparse
 import json
@@ -49,6 +55,49 @@ def timed(fn, reps):
     return statistics.median(ts)
 
 
+def graph_us(fns, reps=6):
+    """Microseconds a call, the calls captured one behind the other."""
+    for f in fns[:2]:
+        f()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        for f in fns:
+            f()
+    g.replay()
+    return timed(g.replay, reps) / len(fns)
+
+
+def one_round(path):
+    """Which entries stay faster than the one-round kernel: both sides in turn, twice, the faster time of each."""
+    hip = get_ops("hip")
+    plan = hip.gemm_plan
+    with open(TABLE) as fh:
+        table = json.load(fh)
+    plan.kept, taken, kept = set(), plan.mid, {}
+    for key in table["choice"]:
+        M, N, K, epi = map(int, key.split(","))
+        if not 33 <= M or taken(M, N, K, epi) is None:
+            continue
+        torch.manual_seed(0)
+        ws = [torch.randn(N, K, device="cuda", dtype=torch.bfloat16) * K ** -0.5 for _ in range(max(3, min(24, (600 << 20) // (N * K * 2))))]
+        x, r = torch.randn(M, K, device="cuda").bfloat16(), torch.randn(M, N, device="cuda").bfloat16()
+        call = {0: lambda w: hip.linear(x, w), 1: lambda w: hip.linear_silu(x, w), 2: lambda w: hip.linear_residual(x, w, r)}[epi]
+        us = {True: [], False: []}
+        for mid in (True, False) * 2:
+            plan.mid = taken if mid else lambda *a: None
+            us[mid].append(graph_us([lambda w=w: call(w) for w in ws]))
+        plan.mid = taken
+        old, new = min(us[False]), min(us[True])
+        if new > 1.02 * old:
+            kept[key] = (round(old, 2), round(new, 2))
+        print(f"{key:24s} as it stands {old:8.2f}us  one-round {new:8.2f}us  x{old / new:5.3f}", flush=True)
+    table["beats_one_round"] = sorted(kept)
+    with open(path, "w") as fh:
+        json.dump(table, fh, indent=1, sort_keys=True)
+    print(f"{len(kept)} entries stay: {kept}\nwrote {path}")
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--model", default="qwen3-14b")
@@ -60,7 +109,10 @@ def main():
     ap.add_argument("--skip", default="", help="comma list of projections to skip")
     ap.add_argument("--cfgs", default="", help="comma list of tile configurations to time (default: all); "
                     "with --merge the table's previous best configuration is timed again as well")
+    ap.add_argument("--one-round", action="store_true", help="only list the entries that the one-round kernel does not beat")
     args = ap.parse_args()
+    if args.one_round:
+        return one_round(args.out or os.path.join(ROOT, "gpurun_out", "hand_gemm.json"))
     only_cfgs = {int(c) for c in args.cfgs.split(",") if c}
     os.environ["BCG_HAND_GEMM"] = "0"  # the library path of linear() must not dispatch to us
     hip = get_ops("hip")
