@@ -49,13 +49,22 @@ float predicted(const Cost& c, float x_rows, int bm, int bn, float kb, float w_b
 // and 1.07 to 1792 rows, 0.93 and 1.05 to 2047, where 2048 x 8192 behind 2039 rows took 80 us for 70.  Up to 512 columns the library's split of a
 // long K wins at times (1508 x 256 x 5632: 22.5 us for 18.3).  fp8 past 1024 rows 0.64 to 0.95 on average, but 1.2 to 1.33 at 768 to 1792
 // columns of K, which nothing here tells apart.
+// What else is left to the others (times over theirs): bf16, plain, K of 64 or, up to 128 rows, of 128 into a store (67 products of 6000 to 40000
+// columns: 0.72 to 0.96 on average, but 11 of 1.05 to 1.25); plain, up to 128 rows and 144 columns, K below 2304 (37: 0.91, 12 of 1.03 to 1.16; past
+// these lines 0.48 to 0.87 and 1 of 143).  fp8 into a store, where the other side is one library launch (into a residual it is two: 0.49 to 0.77): K of 128
+// (38 products: 0.98, 18 of 1.03 to 1.19), K of 256 with 65 to 256 rows (29: 0.93, 13), and from M N K = 1.5e9 on more than 176 rows with K up to
+// 3600 (0.97, 40 of 1.03 to 1.4, where its 128 x 128 tiles fill the chip, which nothing here tells); the 281 that stay 0.74 on average, 11 of 1.03 to 1.21.
 BCG_API int bcg_gemm_mid_plan(int epi, int M, int N, int K, int f8) {
   const bool gated = epi == EPI_SILU_MUL;
   const int bytes = f8 ? K : 2 * K, inter = N / 2;
   if (M < 33 || M > (f8 ? 1024 : 1536) || (M > 1024 && N <= 512) || K <= 0 || bytes % 128 || N < 16 || N % (gated ? 32 : 16) || N > 1 << 20 || (f8 && gated)) return -1;
   if (static_cast<int64_t>(N) * K < (f8 || K < 192 ? 800000 : 100000) || static_cast<int64_t>(N) * bytes >= 1ll << 31 || static_cast<int64_t>(M) * bytes >= 1ll << 31) return -1;
   const Cost& cost = COSTS[M <= 128 ? 0 : M <= 288 ? 1 : 2];
-  if (static_cast<float>(M) * N * K > (f8 ? 15e9f : 80e9f)) return -1;
+  const float products = static_cast<float>(M) * N * K;
+  if (products > (f8 ? 15e9f : 80e9f)) return -1;
+  if (f8 && epi == EPI_STORE && (K == 128 || (K == 256 && M > 64 && M <= 256) || (M > 176 && K <= 3600 && products >= 1.5e9f))) return -1;
+  if (!f8 && epi == EPI_STORE && (K == 64 || (K == 128 && M <= 128))) return -1;
+  if (!f8 && !gated && M <= 128 && N <= 144 && K < 2304) return -1;
   int best = -1;
   float time = 0.f;
   for (int i = 0; i < N_TILES; ++i) {

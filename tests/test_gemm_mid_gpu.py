@@ -265,6 +265,15 @@ def test_plan_takes_one_round_and_refuses_the_rest():
     for bad in ((0, 32, 4096, 4096, 0), (0, 1537, 4096, 4096, 0), (0, 1025, 4096, 4096, 1), (0, 1025, 512, 4096, 0), (0, 100, 4096, 4100, 0), (0, 100, 4104, 4096, 0), (1, 100, 4112, 4096, 0),
                 (0, 100, 4096, 64, 0), (0, 100, 4096, 128, 0), (0, 100, 512, 192, 0), (0, 100, 512, 1024, 1), (0, 1024, 151936, 5120, 0), (1, 100, 4096, 4096, 1)):
         assert lib.bcg_gemm_mid_plan(*bad) == -1, bad
+    # where the others are faster: both sides of each line
+    for left, taken in (((0, 100, 16384, 64, 0), (1, 100, 16384, 64, 0)), ((0, 128, 16384, 128, 0), (0, 129, 16384, 128, 0)),
+                        ((0, 300, 16384, 64, 0), (2, 300, 16384, 64, 0)), ((2, 128, 144, 2240, 0), (2, 129, 144, 2240, 0)),
+                        ((0, 128, 144, 2240, 0), (0, 128, 144, 2304, 0)), ((0, 100, 128, 2240, 0), (0, 100, 160, 2240, 0)),
+                        ((0, 100, 128, 2240, 0), (1, 100, 128, 2240, 0)), ((0, 300, 8192, 128, 1), (2, 300, 8192, 128, 1)),
+                        ((0, 65, 8192, 256, 1), (0, 64, 8192, 256, 1)), ((0, 256, 4096, 256, 1), (0, 257, 4096, 256, 1)),
+                        ((0, 200, 15360, 2048, 1), (0, 176, 15360, 2048, 1)), ((0, 200, 15360, 2048, 1), (2, 200, 15360, 2048, 1)),
+                        ((0, 300, 4096, 3584, 1), (0, 300, 4096, 3712, 1)), ((0, 178, 4096, 2176, 1), (0, 178, 3968, 2048, 1))):
+        assert lib.bcg_gemm_mid_plan(*left) == -1 and lib.bcg_gemm_mid_plan(*taken) >= 0, (left, taken)
     # what the table holds as faster is left too, up to its row count from the one below on
     assert plan.kept and all(key in plan.table and lib.bcg_gemm_mid_plan(key[3], *key[:3], 0) >= 0 for key in plan.kept)
     for M, want in ((64, True), (65, False), (256, False), (257, True), (320, True), (321, False), (512, False), (513, True)):
