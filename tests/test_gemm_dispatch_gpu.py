@@ -1,10 +1,10 @@
 """The SHIPPED GEMM dispatch at real model shapes against fp32 references.  GPU only.
 
-* every entry of ``engine/tuned/hand_gemm.json`` -- each (M, N, K, epilogue) with the
-  (tile, split-K) the table picked, or the library path (``F.linear`` / the
-  ``residual.addmm_`` epilogue) where it kept hipBLASLt -- through the same ops the
-  decoder calls (``linear`` / ``linear_silu`` / ``linear_residual``), compared with
-  fp32 ``F.linear`` (+ SiLU*mul / + residual);
+* every entry of ``engine/tuned/hand_gemm.json`` -- each (M, N, K, epilogue) -- through
+  the same ops the decoder calls (``linear`` / ``linear_silu`` / ``linear_residual``),
+  whose rules for few rows and for one round come before the table, and, where the table
+  picked a (tile, split-K), on that configuration (operands that those rules refuse run
+  it), compared with fp32 ``F.linear`` (+ SiLU*mul / + residual);
 * split-K hand GEMMs captured into HIP graphs of several buckets, replayed smallest
   first (the order the engine's ramp-up replays them) against the fp32 reference;
 * a 2-layer decoder with Qwen3-14B's real dimensions (random weights): the HIP
@@ -60,11 +60,12 @@ def test_shipped_table_entries(hip, shape):
     N, K, epi = shape
     gen = torch.Generator(device="cuda").manual_seed(N + K + epi)
     w = (torch.randn(N, K, device="cuda", generator=gen) * K ** -0.5).to(torch.bfloat16)
-    touched = []
+    touched, log = [], hip.dispatch_log
     for M, choice in ENTRIES[shape]:
         x = torch.randn(M, K, device="cuda", generator=gen).to(torch.bfloat16)
         assert hip.gemm_plan.choose(M, N, K, epi) == (choice if choice[0] >= 0 else None) or choice[0] < 0
         ref = x.float() @ w.float().t()
+        log.enabled, log.calls, was = True, {}, (log.enabled, log.calls)
         if epi == 0:
             out = hip.linear(x, w)
         elif epi == 1:
@@ -73,15 +74,22 @@ def test_shipped_table_entries(hip, shape):
             ref = torch.nn.functional.silu(ref[:, :I]) * ref[:, I:]
         else:
             res = torch.randn(M, N, device="cuda", generator=gen).to(torch.bfloat16)
+            before = res.clone()
             ref = ref + res.float()
             out = hip.linear_residual(x, w, res)
             assert out.data_ptr() == res.data_ptr()  # in place
         torch.cuda.synchronize()
+        ran = "+".join(key[5] for key in log.calls)
+        log.enabled, log.calls = was
         e = _err(out, ref)
-        touched.append(f"{M}:{'lib' if choice[0] < 0 else '%dx%d' % choice}:{e:.1e}")
-        assert e < 2e-2, (M, choice, e)
+        touched.append(f"{M}:{ran}:{e:.1e}")
+        assert e < 2e-2, (M, ran, e)
+        if choice[0] >= 0:
+            e = _err(hip.gemm_nt(x, w, choice, epi, residual=before if epi == 2 else None), ref)
+            touched.append(f"{M}:{'%dx%d' % choice}:{e:.1e}")
+            assert e < 2e-2, (M, choice, e)
         del x, ref, out
-    print(f"[table] N={N} K={K} epi={epi} entries(M:choice:err) " + " ".join(touched))
+    print(f"[table] N={N} K={K} epi={epi} entries(M:what ran:err) " + " ".join(touched))
 
 
 def test_split_k_graphs_replay_small_bucket_first(hip):

@@ -164,6 +164,25 @@ def test_entry_points_take_it_and_replay(ops, M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(33, 1040, 1024), (100, 4096, 1152), (176, 6144, 6144), (1000, 1024, 4096), (40, 2048, 8192)])
+def test_fp8_entry_points_take_it(ops, M, N, K):
+    torch.manual_seed(M)
+    xq, wq = (torch.randn(n, K, device="cuda").to(torch.float8_e4m3fn) for n in (M, N))
+    xs, ws = torch.rand(M, 1, device="cuda") + 0.5, (torch.rand(N, device="cuda") + 0.5) * K ** -0.5
+    bias, res = torch.randn(N, device="cuda").bfloat16(), torch.randn(M, N, device="cuda").bfloat16()
+    y = xq.float() @ wq.float().t() * xs * ws
+    log = ops.dispatch_log
+    log.enabled, log.calls, was = True, {}, (log.enabled, log.calls)
+    try:
+        got = ops.linear_fp8(xq, xs, wq, ws, bias), ops.linear_fp8(xq, xs, wq, ws), ops.linear_fp8_residual(xq, xs, wq, ws, res.clone())
+        assert {(key[3], key[5].split("x")[0]) for key in log.calls} == {(0, str(MID_CFG)), (2, str(MID_CFG))}
+    finally:
+        log.enabled, log.calls = was
+    for a, b in zip(got, (y + bias.float(), y, y + res.float())):
+        assert _err(a, b) < TOL
+
+
+@pytest.mark.gpu
 def test_streams_and_captures_without_preparation(ops):
     """Split products on two streams at once don't share arrival counters, and a capture needs nothing prepared."""
     from byzantine_consensus_llm_agents_amd.ops import hip
