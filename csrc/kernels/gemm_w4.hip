@@ -344,13 +344,14 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
   // "memory" keeps the MFMAs in source order with the LDS reads and DMA issued between them;
   // the builtin form lets hipcc cycle the accumulators through a few AGPRs (gemm_rs.hip)
   const int e8m0_one = 127;  // E8M0 block scale 1.0 (VGPR operand of the scaled MFMA)
+  auto pair = [](const bf16x8 (&f)[8], int b) {
+    const i32x8 v = __builtin_shufflevector(__builtin_bit_cast(i32x4, f[2 * b]), __builtin_bit_cast(i32x4, f[2 * b + 1]), 0, 1, 2, 3, 4, 5, 6, 7);
+    return v;
+  };
   auto mf = [&](int idx, const bf16x8 (&xf)[8], const bf16x8 (&wf)[8]) {
     if constexpr (F8) {  // idx = nb * 4 + mb; a block's operand = its two 16-B chunks
       const int nb = idx >> 2, mb = idx & 3;
-      const i32x8 a = __builtin_shufflevector(__builtin_bit_cast(i32x4, wf[2 * nb]),
-                                              __builtin_bit_cast(i32x4, wf[2 * nb + 1]), 0, 1, 2, 3, 4, 5, 6, 7);
-      const i32x8 b = __builtin_shufflevector(__builtin_bit_cast(i32x4, xf[2 * mb]),
-                                              __builtin_bit_cast(i32x4, xf[2 * mb + 1]), 0, 1, 2, 3, 4, 5, 6, 7);
+      const i32x8 a = pair(wf, nb), b = pair(xf, mb);
       asm volatile("v_mfma_scale_f32_32x32x64_f8f6f4 %0, %1, %2, %0, %3, %3 op_sel_hi:[0,0,0]"
                    : "+a"(acc[nb][mb])
                    : "v"(a), "v"(b), "v"(e8m0_one)
@@ -360,6 +361,28 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
                    : "+a"(acc[idx >> 3][idx & 7])
                    : "v"(wf[idx >> 3]), "v"(xf[idx & 7])
                    : "memory");
+    }
+  };
+
+  // product idx and, behind it, piece q of stream tile t + 2 (K-tile kt), in one statement: the product is the wait state between the write of M0
+  // and the load.  16098 x 34816 x 5120 gated, us: 3590 with the write directly in front of the load, 3585 to 3630 with an s_nop between (1.0 % over
+  // the former in one run, the residual form 1.7 %), 3551 so.
+  auto mf_dma = [&](int idx, const bf16x8 (&xf)[8], const bf16x8 (&wf)[8], int t, int kt, int q, const i32x4& srd) {
+    const uint32_t soff = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(dk0 + kt) * (BK * 2));
+    const uint32_t m0v = dma_m0(t, q), off = q < 8 ? vX[q & 7] : vW[q & 7];
+    if constexpr (F8) {
+      const int nb = idx >> 2, mb = idx & 3;
+      const i32x8 a = pair(wf, nb), b = pair(xf, mb);
+      asm volatile("s_mov_b32 m0, %7\n\tv_mfma_scale_f32_32x32x64_f8f6f4 %0, %1, %2, %0, %3, %3 op_sel_hi:[0,0,0]\n\t"
+                   "buffer_load_dwordx4 %4, %5, %6 offen lds"
+                   : "+a"(acc[nb][mb])
+                   : "v"(a), "v"(b), "v"(e8m0_one), "v"(off), "s"(srd), "s"(soff), "s"(m0v)
+                   : "memory", "m0");
+    } else {
+      asm volatile("s_mov_b32 m0, %6\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0\n\tbuffer_load_dwordx4 %3, %4, %5 offen lds"
+                   : "+a"(acc[idx >> 3][idx & 7])
+                   : "v"(wf[idx >> 3]), "v"(xf[idx & 7]), "v"(off), "s"(srd), "s"(soff), "s"(m0v)
+                   : "memory", "m0");
     }
   };
 
@@ -835,13 +858,14 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
   // tile the pieces go through a zero-range descriptor: no memory traffic, the zeros land in a
   // stage nobody reads -- branch-free, one body (a branch around the pieces, or two copies of
   // the phase, made hipcc spill the accumulators)
-  auto phase_b = [&](int t, int kt2, const i32x4& sX, const i32x4& sW, auto sch) {
+  auto phase_b = [&](int t, int kt2, const i32x4& sW, auto sch) {
     using Sch = decltype(sch);
 #pragma clang loop unroll(full)
     for (int idx = 0; idx < SLOTS; ++idx) {
-      mf(idx, x1, w1);
       if (idx >= Sch::DB0 && (idx - Sch::DB0) % Sch::DBS == 0 && (idx - Sch::DB0) / Sch::DBS < W4_NPB)
-        dma(t + 2, kt2, (idx - Sch::DB0) / Sch::DBS + 8, sX, sW);
+        mf_dma(idx, x1, w1, t + 2, kt2, (idx - Sch::DB0) / Sch::DBS + 8, sW);
+      else
+        mf(idx, x1, w1);
       if (idx >= Sch::RB0 && (idx - Sch::RB0) % Sch::RBS == 0 && (idx - Sch::RB0) / Sch::RBS < 16)
         read_frag(t + 1, 0, (idx - Sch::RB0) / Sch::RBS, x0, w0);  // tile t+1 (garbage after the last)
     }
@@ -863,9 +887,10 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
         sW[e] = __builtin_amdgcn_readfirstlane(more ? dW[e] : nullW[e]);
 #pragma clang loop unroll(full)
       for (int idx = 0; idx < SLOTS; ++idx) {  // phase A
-        mf(idx, x0, w0);
         if (idx >= Sch::DA0 && (idx - Sch::DA0) % Sch::DAS == 0 && (idx - Sch::DA0) / Sch::DAS < 8)
-          dma(t + 2, ktd, (idx - Sch::DA0) / Sch::DAS, sX, sX);
+          mf_dma(idx, x0, w0, t + 2, ktd, (idx - Sch::DA0) / Sch::DAS, sX);
+        else
+          mf(idx, x0, w0);
         if (idx >= Sch::RA0 && (idx - Sch::RA0) % Sch::RAS == 0 && (idx - Sch::RA0) / Sch::RAS < 16)
           read_frag(t, 1, (idx - Sch::RA0) / Sch::RAS, x1, w1);
       }
@@ -877,7 +902,7 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
       const uint64_t t_w = __builtin_amdgcn_s_memtime();
       cyc_a += t_a - t_end, cyc_w += t_w - t_a;
 #endif
-      phase_b(t, ktd, sX, sW, sch);
+      phase_b(t, ktd, sW, sch);
       // the MFMA D -> read wait states at the end of every K-tile, inside the loop: whatever
       // hipcc then does with the accumulators -- the item-end block's reads, its register
       // shuffles on the loop exit (a copy of a just-written block there read 16-lane rows not

@@ -108,5 +108,5 @@ def test_lds_loads_wait_for_m0():
             for a, b in zip(steps, steps[1:]):
                 if re.match(r"s_\w+ m0,", a):
                     found += 1
-                    assert b.strip().startswith("s_nop"), (path, asm)
+                    assert b.strip().startswith(("s_nop", "v_mfma")), (path, asm)
     assert found >= 8
