@@ -7,10 +7,12 @@
 // takes 114 B/ns where an instruction reads 128 bytes of a row and 77 where it reads 64 (1 KB each, L2 hits; 256 bytes: 112).  So:
 //   * the waves split K, not the tile (WK = 4: a stage is 128 deep, wave w takes its w-th 32): every fragment is read out of LDS once,
 //     (BM + BN) x 64 bytes a 32-deep step instead of the 1.5 times of 2 x 2 waves, which bound the 128 x 128 tiles of gemm.hip at 0.43 us per 64
-//     of K.  Tiles of more than 128 rows would need too many registers (BM BN / 64 accumulators a lane): there WM = 2 halves of the rows, K in two;
+//     of K.  Tiles of more than 40 blocks of 16 x 16 would need too many registers (four accumulators a block and lane): there, and where the
+//     tile is wide from 32 on, WM = 2 halves of the rows, K in two;
 //   * all four waves fetch an even share of X and W.  Two waves for X and two for W, with a deeper ring for W, took 1.3 times as long: a wave
 //     has only so many fetches under way;
-//   * the tile is free in steps of 16 (8 to 2 accumulator blocks a side), so a plan (below) finds one whose tiles x K-splits fill one round;
+//   * the tile is free in steps of 16 (MID_TILES below: 3 to 16 blocks of rows by 1 to 12 of columns), so a plan (gemm_mid.hip) finds one whose
+//     tiles x K-splits fill one round;
 //   * the eight XCDs start K an eighth apart: in step, all CUs read the same 256 bytes of every row, a few channels' worth (101 x 24576 x 4096
 //     48 -> 41 us); within an XCD they stay in step, so X and a W shared by several row tiles are fetched into its L2 once (a column tile whose row
 //     tiles lie on two XCDs keeps the first one's start: equal rows stay equal);
