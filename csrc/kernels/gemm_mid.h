@@ -121,8 +121,9 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
   }
   const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem)) + half * U * 2048 + rg0 * 1024;
   // stage s of the walk is stage (s + rot) mod n of K.  rot: of the XCD that has the column tile's first row tile, so that rows of one call add K in
-  // one order whichever row tile they are in (a column tile's row tiles may lie on two)
-  const int first = rest * a.m_tiles, home = first < rem * (q + 1) ? first / (q + 1) : rem + (first - rem * (q + 1)) / q;
+  // one order whichever row tile they are in (a column tile's row tiles may lie on two and more)
+  int home = xcd;
+  for (int from = r_id - (bid >> 3); r_id - m_tile < from; from -= home < rem ? q + 1 : q) --home;   // from: the first workgroup of `home`
   const int rot = home * n / 8;
   auto at = [&](int s) { const int t = s + rot; return t >= n ? t - n : t; };
   auto valid = [&](int s) { return s < n && at(s) * H + half < nb; };
@@ -165,6 +166,26 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
       asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(f[MW + i]), "v"(f[j]) : "memory");
     }
   };
+  // product p and fetch u behind it, in one statement: the (first) product is the wait state between the write of m0 and the load.  Over 76
+  // products 1.002 of the time with the write directly in front of the load, an s_nop between them 1.011 (up to 1.06 where a launch is short).
+  auto product_fetch = [&](int p, const bf16x8 (&f)[F], int u, uint32_t slot, uint32_t ko) {
+    const int i = p / MW, j = p % MW;
+    const i32x4 srd = u < DX ? sX : sW;
+    if constexpr (F8) {
+      const i64x2 w = __builtin_bit_cast(i64x2, f[MW + i]), x = __builtin_bit_cast(i64x2, f[j]);
+      const long w0 = w[0], w1 = w[1], x0 = x[0], x1 = x[1];
+      asm volatile("s_add_u32 m0, %8, %9\n\tv_mfma_f32_16x16x32_fp8_fp8 %0, %1, %2, %0\n\tbuffer_load_dwordx4 %5, %6, %7 offen lds\n\t"
+                   "v_mfma_f32_16x16x32_fp8_fp8 %0, %3, %4, %0"
+                   : "+a"(acc[i][j])
+                   : "v"(w0), "v"(x0), "v"(w1), "v"(x1), "v"(vo[u]), "s"(srd), "s"(ko), "s"(slot), "n"(u * RG * 1024)
+                   : "memory", "m0", "scc");
+    } else {
+      asm volatile("s_add_u32 m0, %6, %7\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0\n\tbuffer_load_dwordx4 %3, %4, %5 offen lds"
+                   : "+a"(acc[i][j])
+                   : "v"(f[MW + i]), "v"(f[j]), "v"(vo[u]), "s"(srd), "s"(ko), "s"(slot), "n"(u * RG * 1024)
+                   : "memory", "m0", "scc");
+    }
+  };
 
 #pragma unroll
   for (int s = 0; s < R - 1; ++s) fetch_stage(s);
@@ -187,19 +208,23 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
     auto walk = [&](auto self, auto pp) {
       constexpr int p = decltype(pp)::value;
       if constexpr (p < NB) {
+        constexpr int next = ((p + 1) * EV + PE - 1) / PE, last = (next < EV ? next : EV) - 1;   // the last operation in front of this product
         auto ops = [&](auto self2, auto ee) {
           constexpr int e = decltype(ee)::value;
           if constexpr (e < EV && e * PE / EV <= p) {
             if constexpr (e * PE / EV == p) {
               if constexpr (e < F) nxt[e] = read(from, e);
-              if constexpr (e < D) fetch(e, slot, ko);
+              if constexpr (e < D && e != last) fetch(e, slot, ko);
               __builtin_amdgcn_sched_barrier(0);
             }
             self2(self2, std::integral_constant<int, e + 1>{});
           }
         };
         ops(ops, std::integral_constant<int, (p * EV + PE - 1) / PE>{});
-        product(p, cur);
+        if constexpr (last * PE / EV == p && last < D)
+          product_fetch(p, cur, last, slot, ko);
+        else
+          product(p, cur);
         __builtin_amdgcn_sched_barrier(0);
         self(self, std::integral_constant<int, p + 1>{});
       }
