@@ -17,7 +17,7 @@ import bisect
 import ctypes
 import json
 import os
-from typing import Dict, List, Optional, Set, Tuple
+from typing import Dict, List, Optional, Tuple
 
 TABLE = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "engine", "tuned",
                      "hand_gemm.json")
@@ -53,7 +53,7 @@ class GemmPlan:
                 if lib.bcg_gemm_tile(cfg, ctypes.byref(bm), ctypes.byref(bn)) == 0:
                     self.tiles[cfg] = (bm.value, bn.value)
         self.table: Dict[Tuple[int, int, int, int], Tuple[int, int]] = {}
-        self.kept: Set[Tuple[int, int, int, int]] = set()   # entries that the one-round kernel does not beat
+        self.kept: Dict[Tuple[int, int, int, int], int] = {}   # entries that the one-round kernel does not beat: from which row count on
         if table and os.path.exists(table):
             with open(table) as fh:
                 data = json.load(fh)
@@ -62,7 +62,7 @@ class GemmPlan:
                 self.table[(m, n, k, e)] = tuple(choice) if isinstance(choice, list) else (int(choice), 1)
             for (m, n, k, e) in sorted(self.table):     # measured row counts of every shape, in order
                 self.rows.setdefault((n, k, e), []).append(m)
-            self.kept = {tuple(map(int, key.split(","))) for key in data.get("beats_one_round", [])}
+            self.kept = {tuple(map(int, key.split(","))): rows for key, rows in data.get("beats_one_round", {}).items()}
             for key, times in data.get("timings_us", {}).items():
                 self.timings[tuple(map(int, key.split(",")))] = times
 
@@ -125,14 +125,17 @@ class GemmPlan:
 
     def mid(self, M: int, N: int, K: int, epi: int) -> Optional[int]:
         """Plan of the kernel for tens to hundreds of rows (csrc/kernels/gemm_mid.hip), None where it is not taken: by its own rule, which rests on a
-        model of its time, and where the table holds the projection and what stood there is faster at the measured row count from M on
-        (``tools/tune_hand_gemm.py --one-round``; 32 of 292 entries by 2 % and more, 256 x 2560 x 5120 21.4 us against 25.3)."""
+        model of its time, and where the table holds the projection and what stood there is faster from a row count up to the entry's
+        (``tools/tune_hand_gemm.py --one-round``, up to seven row counts of each of 302 entries; 15 are listed, by 5 to 15 %: 256 x 2560 x 5120 21.0
+        us against 25.2, but 193 rows 20.4 against 18.4, so from 214 on).  Decode steps of the 8b and 14b models bear out 7168 x 5120 at 49 to 64
+        rows (0.5 to 2 us a layer) and 4096 x 12288 at 161 to 192 (3 to 6 us); not 7168 x 5120 at 33 to 40 and 97 to 128 (1.03 of the table's time
+        alone, in steps 2.5 to 5 us a layer faster) and past 352, nor 4096 x 4096 and 5120 x 5120 into a residual past 640 (level)."""
         if self.mode != "1" or self.lib is None:
             return None
         if self.kept:
             ms = self.rows.get((N, K, epi), [])
             at = bisect.bisect_left(ms, M)
-            if at < len(ms) and (ms[at], N, K, epi) in self.kept:
+            if at < len(ms) and M >= self.kept.get((ms[at], N, K, epi), M + 1):
                 return None
         p = self.lib.bcg_gemm_mid_plan(epi, M, N, K, 0)
         return p if p >= 0 else None

@@ -293,9 +293,11 @@ def test_plan_takes_one_round_and_refuses_the_rest():
                         ((0, 200, 15360, 2048, 1), (0, 176, 15360, 2048, 1)), ((0, 200, 15360, 2048, 1), (2, 200, 15360, 2048, 1)),
                         ((0, 300, 4096, 3584, 1), (0, 300, 4096, 3712, 1)), ((0, 178, 4096, 2176, 1), (0, 178, 3968, 2048, 1))):
         assert lib.bcg_gemm_mid_plan(*left) == -1 and lib.bcg_gemm_mid_plan(*taken) >= 0, (left, taken)
-    # what the table holds as faster is left too, up to its row count from the one below on
-    assert plan.kept and all(key in plan.table and lib.bcg_gemm_mid_plan(key[3], *key[:3], 0) >= 0 for key in plan.kept)
-    for M, want in ((64, True), (65, False), (256, False), (257, True), (320, True), (321, False), (512, False), (513, True)):
+    # what the table holds as faster is left too, from the row count that it says on up to its own
+    assert plan.kept and all(key in plan.table and lib.bcg_gemm_mid_plan(key[3], rows, *key[1:3], 0) >= 0 and rows <= key[0] and
+                             not any(rows <= m < key[0] for m in plan.rows[key[1:]]) for key, rows in plan.kept.items())
+    for M, want in ((64, True), (65, True), (213, True), (214, False), (256, False), (257, True), (266, True), (267, False), (320, False),
+                    (321, True), (458, True), (459, False), (512, False), (513, True)):
         assert (plan.mid(M, 2560, 5120, 0) is not None) == want, M
     assert plan.mid(256, 2560, 5120, 2) is not None and GemmPlan(lib, table=None).mid(256, 2560, 5120, 0) is not None
 
