@@ -6,6 +6,7 @@ leave (decode buckets whose product is more than a round of tiles, operands they
 epilogue) measured on the GPU (``tools/tune_hand_gemm.py`` -> ``engine/tuned/hand_gemm.json``: for every decode bucket
 and projection shape, every tile configuration and the library are timed and the fastest is kept), prefill chunks by
 the rules of `GemmPlan.pieces`, and shapes that nothing covers stay on the library.
+Most entries of 33 to 1536 rows serve only operands that the one-round kernel refuses (not contiguous, not on 16 bytes, watched by autograd).
 
 ``BCG_HAND_GEMM``: ``0`` = library only, ``1`` (default) = table / rule,
 ``force`` = hand kernel wherever the shape is supported (tests; ``BCG_HAND_GEMM_SPLIT``

@@ -62,8 +62,8 @@ def few_rows_stay(M: int, N: int, K: int, gated: bool) -> bool:
     Times of the one-round kernel over the few-row kernel's at 1018 products of 2.7 M elements of W and more: 0.84 on average, 34 of 1.03 to 1.14, most of
     them where its plan is 48 x 32 tiles in one part that leave a quarter of the CUs idle and the few-row kernel's rows are whole turns: up to
     48 rows, K in steps of 512 from 2048 to 4096, 4097 to 6500 columns (gated 2700 to 6500) 1.01 on average, up to 1.14 (44 rows, 6144 x 4096:
-    16.1 us for 17.5).  14 of the others are 1.03 to 1.07 slower.  Smaller W: 0.77 to 0.82, left where the tests of the few-row
-    kernel hold them."""
+    16.1 us for 17.5).  14 of the others are 1.03 to 1.07 slower.  Smaller W: 0.77 to 0.82, a gain that
+    this line still leaves to the few-row kernel."""
     if N * K < 2700000:
         return True
     return M <= 48 and K % 512 == 0 and 2048 <= K <= 4096 and (2700 if gated else 4097) <= N <= 6500

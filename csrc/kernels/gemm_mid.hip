@@ -21,7 +21,8 @@ constexpr int CUS = 256;
 
 // Microseconds of a launch of one round, x_rows rows of X (a row tile's share) and bn of W, kb bytes each, a workgroup: fitted (relative least squares,
 // three ranges of rows) to the times of these tiles at 2300 products and checked at 1600 others: the tile chosen by it is 1.7, 2.3 and
-// 3.2 % slower on average than the best of all 72.
+// 3.2 % slower on average than the best of all 72.  (The times are not kept: for another compiler or card, time bcg_gemm_mid with every tile and
+// split of random products, weights changed each call, and fit the nine terms of `predicted` again.)
 struct Cost {
   float launch, x_row, w_row, product, hbm, area, split, part, gated_part;
 };
