@@ -352,13 +352,19 @@ class DecoderModel:
     def _attention(self, li, L, qkv, meta, k_cache, v_cache):
         ops, c = self.ops, self.cfg
         # (not with shared-prefix tables, which the engine passes with every decode step unless `cascade_decode` is off)
-        if (meta.decode and meta.cascade is None and self.hd == 64 and hasattr(ops, "decode_attention") and qkv.is_contiguous()
-                and k_cache.dtype == v_cache.dtype == qkv.dtype == torch.bfloat16 and k_cache.shape[-2] == 16
-                and ops.decode_fused_pays(qkv.shape[0], self.n_kv, meta.block_tables.shape[1] * 16)):
-            lens = meta.seq_lens if meta.attn_seq_lens is None else meta.attn_seq_lens
-            return ops.decode_attention(qkv, meta.positions, meta.slots, self.n_q, self.n_kv, self.hd, L.get("q_norm"),
-                                        L.get("k_norm"), c.rms_eps, self.cos_sin, k_cache, v_cache, li, meta.block_tables,
-                                        lens, self.scale, meta.workspace)
+        if (meta.decode and meta.cascade is None and qkv.is_contiguous() and k_cache.dtype == v_cache.dtype == qkv.dtype == torch.bfloat16
+                and k_cache.shape[-2] == 16):
+            attend = None
+            if hasattr(ops, "decode_attention_pairs"):   # (its fetches are 16 bytes a lane)
+                if self.hd in (64, 128) and (k_cache.data_ptr() | v_cache.data_ptr() | qkv.data_ptr()) % 16 == 0:
+                    attend = ops.decode_attention_pairs
+            elif (self.hd == 64 and hasattr(ops, "decode_attention")
+                  and ops.decode_fused_pays(qkv.shape[0], self.n_kv, meta.block_tables.shape[1] * 16)):
+                attend = ops.decode_attention
+            if attend is not None:
+                lens = meta.seq_lens if meta.attn_seq_lens is None else meta.attn_seq_lens
+                return attend(qkv, meta.positions, meta.slots, self.n_q, self.n_kv, self.hd, L.get("q_norm"), L.get("k_norm"), c.rms_eps,
+                              self.cos_sin, k_cache, v_cache, li, meta.block_tables, lens, self.scale, meta.workspace)
         q = ops.qk_norm_rope_kv_write(qkv, meta.positions, meta.slots, self.n_q, self.n_kv, self.hd,
                                       L.get("q_norm"), L.get("k_norm"), c.rms_eps, self.cos_sin,
                                       k_cache, v_cache, li, contiguous=not meta.decode)

@@ -109,8 +109,8 @@ def load_library(path: str = None) -> ctypes.CDLL:
                         c_int, c_int, c_int, c_int, c_int, c_void_p],
         "bcg_gemm_nt_fp8": [c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                             c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
-        "bcg_decode_fused": [c_void_p] * 6 + [c_float, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_void_p, c_int,
-                             c_int, c_int, c_int, c_float, c_void_p, c_int, c_int, c_void_p, c_void_p],
+        "bcg_decode_pairs": [c_void_p] * 6 + [c_float, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_void_p, c_int,
+                             c_int, c_int, c_int, c_float, c_int, c_void_p, c_void_p, c_void_p],
         "bcg_gemm_skinny": [c_int, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
                             c_void_p],
         "bcg_gemm_skinny_fp8": [c_int] + [c_void_p] * 7 + [c_int] * 3 + [c_void_p],
@@ -292,9 +292,23 @@ def few_rows_pay(M: int, N: int, row_bytes: int, gated: bool) -> bool:
     return N >= (4096 if part else 1024)
 
 
+def decode_parts(B: int, n_kv: int, hd: int, tokens: int) -> int:
+    """Workgroups that share a (row, kv head) pair of a decode step (csrc/kernels/attention.hip, decode_pair_kernel); tokens: context that the block table
+    has room for (the contexts themselves are on the device).
+
+    One, whose merge is its own, up to 448 KB of K/V of a pair, or where the pairs fill the CUs; else as many as there are CUs, up to one
+    for each 128 KB (us for 1, 2, 3, 4, 8 parts): heads of 128, 80 pairs of 400 tokens 9.4, 12.3, 12.5, of 1000 19.5, 17.9, 16.7, of 2500 38.6, 29.1,
+    27.3; 160 pairs of 1000 22.8, 28.6; 8 pairs of 400 8.1, 9.8, 10, 9.5, of 1000 11, 11.8, 11.5, 10.4, 10.1, of 6000 36, 24, 20, 16.7, 13.5; heads of 64, 8 pairs of
+    1000 7.3, 9, 9.1, 8.2, 8.4, of 2500 12.3, 11.9, 11.1, 9.7, 9.3; 128 pairs of 4000 34.8, 31.4."""
+    pair = tokens * hd * 4
+    if pair <= 448 * 1024:
+        return 1
+    return max(1, min(256 // (B * n_kv), -(-pair // (128 * 1024)), 16))
+
+
 def decode_fused_pays(B: int, n_kv: int, splits: int) -> bool:
-    """Whether a decode step of B rows with heads of 64 gains by the rotary embedding inside the attention launch; splits: parts of a
-    row's context that the block table has room for (the contexts themselves are on the device).
+    """Whether a decode step of B rows with heads of 64 gains by `decode_attention` with a backend that has no `decode_attention_pairs`: one whose
+    workgroups take a part of a row's context each and all rotate its queries; splits: parts that the block table has room for.
 
     The rotation takes registers, so two workgroups of a CU are resident where the separate kernel has three, and every workgroup of a row rotates
     its queries again.  Rotary launch, attention and merge over the fused pair, 14 / 2, 16 / 4, 32 / 8, 16 / 16 and 16 / 1 heads, contexts
@@ -417,29 +431,39 @@ def hip_ops() -> SimpleNamespace:
     def decode_attention(qkv, positions, slots, n_q, n_kv, hd, q_norm, k_norm, eps, cos_sin, k_cache, v_cache, layer,
                          block_tables, seq_lens, scale, workspace=None):
         """paged_attention_decode(qk_norm_rope_kv_write(...)) for one new token per row of a bf16 cache with heads of 64, without the
-        rotary launch (csrc/kernels/attention.hip, FusedArgs, says why not for others).  Rows are different sequences: no row sees
-        what another one stores in this call."""
+        rotary launch.  Rows are different sequences: no row sees what another one stores in this call.  `workspace`: as
+        paged_attention_decode."""
+        _req(hd == 64, "decode kv cache layout")
+        B, tokens = qkv.shape[0], block_tables.shape[1] * 16
+        if workspace is not None:
+            _req(workspace.numel() >= B * n_q * lib.bcg_decode_max_splits(tokens, 0) * (hd + 2), "decode attention workspace too small")
+        return decode_attention_pairs(qkv, positions, slots, n_q, n_kv, hd, q_norm, k_norm, eps, cos_sin, k_cache, v_cache, layer,
+                                      block_tables, seq_lens, scale, workspace)
+
+    def decode_attention_pairs(qkv, positions, slots, n_q, n_kv, hd, q_norm, k_norm, eps, cos_sin, k_cache, v_cache, layer,
+                               block_tables, seq_lens, scale, workspace=None, parts=None):
+        """The same for heads of 64 or 128: a workgroup for each of `parts` parts of a (row, kv head) pair (default: `decode_parts`);
+        past one a second launch merges them, out of `workspace` where it holds B n_q parts (hd + 2) floats."""
         B = qkv.shape[0]
         L, NB, nkv_c, BS, hdc = k_cache.shape
         _req(qkv.dtype == torch.bfloat16 and qkv.is_contiguous() and qkv.shape[1] == (n_q + 2 * n_kv) * hd, "decode qkv")
-        _req(nkv_c == n_kv and hdc == hd and hd == 64 and BS == 16 and v_cache.shape == (L, NB, n_kv, hd, BS)
+        _req(nkv_c == n_kv and hdc == hd and hd in (64, 128) and BS == 16 and v_cache.shape == (L, NB, n_kv, hd, BS)
              and not _kv_fp8(k_cache, v_cache), "decode kv cache layout")
         _req(all(t.dtype == torch.int32 and t.is_contiguous() for t in (positions, slots, seq_lens, block_tables))
              and positions.numel() == slots.numel() == seq_lens.numel() == B and block_tables.shape[0] == B, "decode tables")
         _req(cos_sin.dtype == torch.float32 and cos_sin.shape[1] == hd and B <= 2048, "decode cos_sin / rows")
-        max_blocks = block_tables.shape[1]
-        split = lib.bcg_decode_split_tokens(B, n_kv, max_blocks * BS)
-        max_splits = lib.bcg_decode_max_splits(max_blocks * BS, 0)
-        need = B * n_q * max_splits * (hd + 2)
-        if workspace is None:
+        if parts is None:
+            parts = decode_parts(B, n_kv, hd, block_tables.shape[1] * BS)
+        need = 0 if parts == 1 else B * n_q * parts * (hd + 2)
+        if workspace is not None:
+            _req(workspace.dtype == torch.float32 and workspace.is_contiguous(), "decode attention workspace")
+        if need and (workspace is None or workspace.numel() < need):
             workspace = torch.empty(need, dtype=torch.float32, device=qkv.device)
-        _req(workspace.dtype == torch.float32 and workspace.is_contiguous() and workspace.numel() >= need,
-             "decode attention workspace too small")
         out = torch.empty(B, n_q * hd, dtype=qkv.dtype, device=qkv.device)
-        _check(lib.bcg_decode_fused(
+        _check(lib.bcg_decode_pairs(
             _p(qkv), _p(positions), _p(slots), None if q_norm is None else _p(q_norm), None if k_norm is None else _p(k_norm),
-            _p(cos_sin), eps, _p(k_cache), _p(v_cache), layer, NB, n_kv, _p(block_tables), max_blocks, _p(seq_lens), B, n_q, hd,
-            BS, scale, _p(workspace), max_splits, split, _p(out), _stream()), "decode_attention")
+            _p(cos_sin), eps, _p(k_cache), _p(v_cache), layer, NB, n_kv, _p(block_tables), block_tables.shape[1], _p(seq_lens), B, n_q, hd,
+            BS, scale, parts, _p(workspace) if need else None, _p(out), _stream()), "decode_attention_pairs")
         return out
 
     def paged_attention_prefill(q, k_cache, v_cache, layer, block_tables, q_start, seq_lens, scale,
@@ -1021,8 +1045,7 @@ def hip_ops() -> SimpleNamespace:
                            embed_rmsnorm=embed_rmsnorm,
                            qk_norm_rope_kv_write=qk_norm_rope_kv_write,
                            paged_attention_decode=paged_attention_decode,
-                           decode_attention=decode_attention,
-                           decode_fused_pays=lambda B, n_kv, tokens: decode_fused_pays(B, n_kv, -(-tokens // lib.bcg_decode_split_tokens(B, n_kv, tokens))),
+                           decode_attention=decode_attention, decode_attention_pairs=decode_attention_pairs,
                            decode_workspace_numel=decode_workspace_numel,
                            decode_max_context=lambda cascade=True: lib.bcg_decode_max_context(int(cascade)),
                            paged_attention_prefill=paged_attention_prefill,

@@ -395,15 +395,8 @@ constexpr int DEC_MAX_SHARED_SPLITS = 16;   // slots of the shared-prefix pass (
 // 64 columns instead of once per row -- into slots 0 .. split_base-1; this kernel covers
 // [kv_begin, ctx) into the slots after them; the combine merges all slots.
 // kv_begin == nullptr: no cascade (every row from token 0).
-//
-// FUSED (heads of 64, bf16 caches): the kernel takes the projected rows as they come, without a rotary launch and a pass over q
-// before it: every workgroup rotates (and normalises) its own query heads while its K/V loads are in flight; the one with the
-// newest token also stores that token's K/V and puts it into its chunk's registers, where the loads brought what was there
-// before.  24 layers of 14 / 2 heads at 4 rows of 500 tokens: 912 -> 873 us a step.  It keeps 189 registers (the separate one 144), so two workgroups
-// of a CU are resident instead of three: `decode_fused_pays` in ops/hip.py has the line.  Heads of 128 take the separate launches:
-// two chunks of K/V and the rotation's operands fill the registers (10 rows of 1100 tokens, 40 / 8 heads, a step of 16 layers: 2561
-// us, 2590 fused; 448 rows 6950, 8110).  Merging the splits in the workgroup that arrives last costs more than the merge
-// launch for both (stores past the L2, a ticket, the reads back: 880 and 2669).
+
+// The projected rows of a step and what its rotary embedding needs (decode_pair_kernel).
 struct FusedArgs {
   const bf16_t* qkv;        // [B, n_q + 2 n_kv, HD]
   const int* positions;     // [B]
@@ -706,14 +699,13 @@ struct ItemShared {
   float o[DEC_WAVES][HD][16 + 1];
 };
 // STREAM: a step of more items than workgroups is streamed (heads of 128 in bf16)
-template <int HD, bool F8 = false, int CPW = 1, bool FUSED = false, bool STREAM = false>
+template <int HD, bool F8 = false, int CPW = 1, bool STREAM = false>
 __global__ __launch_bounds__(256, (STREAM ? 2 : 1)) void decode_attn_kernel(
     const bf16_t* __restrict__ q, KVGeom g, const int* __restrict__ block_tables, int max_blocks,
     const int* __restrict__ seq_lens, int B, int n_q, float scale_log2, float* __restrict__ part_o,
     float* __restrict__ part_ml, int max_splits, const int* __restrict__ kv_begin,
-    const int* __restrict__ split_base, FusedArgs fa) {
-  static_assert(!FUSED || (HD == 64 && !F8), "fused: see FusedArgs");
-  static_assert(!STREAM || (HD == 128 && !F8 && !FUSED), "streamed: decode_stream");
+    const int* __restrict__ split_base) {
+  static_assert(!STREAM || (HD == 128 && !F8), "streamed: decode_stream");
   // CPW chunks per wave: an item covers DEC_WAVES * CPW * 32 tokens; every chunk's loads of
   // a wave are issued before its first MFMA (CPW x 16 loads in flight per wave), and the
   // split partials / merge traffic shrink by CPW
@@ -725,7 +717,7 @@ __global__ __launch_bounds__(256, (STREAM ? 2 : 1)) void decode_attn_kernel(
   auto &s_wsum = shared.wsum;
   auto &s_ml = shared.ml;
   auto &s_o = shared.o;
-  const int tid = threadIdx.x, lane = tid & 63, w = FUSED ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int r = lane & 15, h = lane >> 4;
   const int G = n_q / g.n_kv;
 
@@ -739,7 +731,6 @@ __global__ __launch_bounds__(256, (STREAM ? 2 : 1)) void decode_attn_kernel(
       const int i = tid * per + j;
       const int own = (j < per && i < B) ? max(0, seq_lens[i] - (kv_begin ? kv_begin[i] : 0)) : 0;
       cnt[j] = (own + DEC_SPLIT - 1) / DEC_SPLIT;
-      if (FUSED && j < per && i < B) cnt[j] = max(cnt[j], 1);   // its K/V is stored and its output cleared all the same
       sum += cnt[j];
     }
     int incl = sum;  // inclusive wave scan
@@ -779,111 +770,27 @@ __global__ __launch_bounds__(256, (STREAM ? 2 : 1)) void decode_attn_kernel(
       const int mid = (lo + hi + 1) >> 1;
       if (s_pre[mid] <= pos) lo = mid; else hi = mid - 1;
     }
-    const int b = FUSED ? __builtin_amdgcn_readfirstlane(lo) : lo, split = pos - s_pre[b];
+    const int b = lo, split = pos - s_pre[b];
     const int ctx = seq_lens[b];
     const int start = (kv_begin ? kv_begin[b] : 0) + split * DEC_SPLIT;
     const int slot = (split_base ? split_base[b] : 0) + split;  // after the shared-pass slots
     const int* table = block_tables + static_cast<size_t>(b) * max_blocks;
 
     bf16x8 bq[HD / 32];
-    // FUSED: all of this is asked for before the K/V loads, behind which it would wait for them
-    u16x8 raw_q[HD / 32], raw_k[HD / 32], wq[HD / 32] = {}, wk[HD / 32] = {};
-    f32x4 cs[HD / 64][2], sn[HD / 64][2];
-    bf16_t nv[HD / 16];
-    const int newest = ctx - 1;
-    const bool stores = FUSED && pos + 1 == __builtin_amdgcn_readfirstlane(s_pre[b + 1]) && w == max(newest - start, 0) / (CHUNK * CPW);
-    const bf16_t* heads = nullptr;
-    if constexpr (FUSED) {
-      heads = fa.qkv + static_cast<size_t>(b) * (n_q + 2 * g.n_kv) * HD;
-      load_head<HD>(raw_q, heads + (kvh * G + (r < G ? r : 0)) * HD, h);
-      const float* t = fa.cos_sin + static_cast<size_t>(fa.positions[b]) * HD + 8 * h;
-#pragma unroll
-      for (int kk = 0; kk < HD / 64; ++kk)
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          cs[kk][e] = *reinterpret_cast<const f32x4*>(t + kk * 32 + 4 * e);
-          sn[kk][e] = *reinterpret_cast<const f32x4*>(t + HD / 2 + kk * 32 + 4 * e);
-        }
-      if (fa.q_norm != nullptr) load_head<HD>(wq, fa.q_norm, h);
-      if (stores) {   // wave-uniform: the wave that covers the newest token
-        load_head<HD>(raw_k, heads + (n_q + kvh) * HD, h);
-        if (fa.k_norm != nullptr) load_head<HD>(wk, fa.k_norm, h);
-#pragma unroll
-        for (int dt = 0; dt < HD / 16; ++dt) nv[dt] = heads[(n_q + g.n_kv + kvh) * HD + dt * 16 + r];
-      }
-    } else {
-      load_q<HD>(bq, q + (static_cast<size_t>(b) * n_q + kvh * G + (r < G ? r : 0)) * HD, r < G, lane);
-    }
+    load_q<HD>(bq, q + (static_cast<size_t>(b) * n_q + kvh * G + (r < G ? r : 0)) * HD, r < G, lane);
     float m = -INFINITY, l = 0.f;
     f32x4 o[HD / 16];
 #pragma unroll
     for (int dt = 0; dt < HD / 16; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     const int t0 = start + w * CHUNK * CPW;
-    const int last_blk = (FUSED ? max(ctx - 1, 0) : ctx - 1) / BS;
+    const int last_blk = (ctx - 1) / BS;
     Chunk<HD, F8> c[CPW];
-    if constexpr (FUSED) {
-      // wave-uniform addresses through the scalar cache: a vector load of a table entry would be waited for together with
-      // the rotary embedding's operands (loads return in order)
-      int blk[CPW][2];
 #pragma unroll
-      for (int j = 0; j < CPW; ++j)
-#pragma unroll
-        for (int e = 0; e < 2; ++e) blk[j][e] = table[min((t0 + j * CHUNK) / BS + e, last_blk)];
-#pragma unroll
-      for (int j = 0; j < CPW; ++j)
-        if (t0 + j * CHUNK < ctx) load_chunk<HD, F8>(c[j], g, blk[j][0], blk[j][1], kvh, lane);  // wave-uniform
-    } else {
-#pragma unroll
-      for (int j = 0; j < CPW; ++j) {
-        const int tj = t0 + j * CHUNK;
-        if (tj < ctx)  // wave-uniform
-          load_chunk<HD, F8>(c[j], g, table[tj / BS], table[min(tj / BS + 1, last_blk)], kvh, lane);
-      }
-    }
-    if constexpr (FUSED) {
-      rope_fragments<HD>(bq, raw_q, wq, fa.q_norm != nullptr, cs, sn, fa.eps, h);
-      if (r >= G) {
-#pragma unroll
-        for (int kk = 0; kk < HD / 32; ++kk) bq[kk] = bf16x8{};
-      }
-      if (stores) {
-        bf16x8 bk[HD / 32];
-        rope_fragments<HD>(bk, raw_k, wk, fa.k_norm != nullptr, cs, sn, fa.eps, h);
-        const int slot_of = fa.slots[b];
-        const size_t base = block_base<HD>(g, slot_of / BS, kvh);
-        bf16_t* kd = const_cast<bf16_t*>(g.k) + base + (slot_of % BS) * HD + 8 * h;
-        bf16_t* vd = const_cast<bf16_t*>(g.v) + base + slot_of % BS;
-        if (r == 0) {
-#pragma unroll
-          for (int kk = 0; kk < HD / 32; ++kk) *reinterpret_cast<bf16x8*>(kd + kk * 32) = bk[kk];
-        }
-#pragma unroll
-        for (int dt = 0; dt < HD / 16; ++dt)
-          if (dt % 4 == h) vd[(dt * 16 + r) * BS] = nv[dt];
-        // (a parked row stores elsewhere than it reads: its newest token is what the cache holds)
-        if (ctx > 0 && slot_of == table[newest / BS] * BS + newest % BS) {
-#pragma unroll
-          for (int j = 0; j < CPW; ++j) {
-            const int tj = t0 + j * CHUNK;
-            if (newest < tj || newest >= tj + CHUNK) continue;  // wave-uniform
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-              const bool here = tj + 8 * (r >> 2) + 4 * u + (r & 3) == newest;
-#pragma unroll
-              for (int kk = 0; kk < HD / 32; ++kk) c[j].k[u][kk] = here ? bk[kk] : c[j].k[u][kk];
-            }
-            const int at = newest - tj - 8 * h;   // element of this lane's V^T pieces, if 0 .. 7
-#pragma unroll
-            for (int dt = 0; dt < HD / 16; ++dt) {
-              u16x8 v = __builtin_bit_cast(u16x8, c[j].v[dt]);
-#pragma unroll
-              for (int e = 0; e < 8; ++e) v[e] = e == at ? nv[dt] : v[e];
-              c[j].v[dt] = __builtin_bit_cast(bf16x8, v);
-            }
-          }
-        }
-      }
+    for (int j = 0; j < CPW; ++j) {
+      const int tj = t0 + j * CHUNK;
+      if (tj < ctx)  // wave-uniform
+        load_chunk<HD, F8>(c[j], g, table[tj / BS], table[min(tj / BS + 1, last_blk)], kvh, lane);
     }
 #pragma unroll
     for (int j = 0; j < CPW; ++j) {
@@ -932,6 +839,224 @@ __global__ __launch_bounds__(256, (STREAM ? 2 : 1)) void decode_attn_kernel(
   }
 }
 
+// ------------------------------------------------------- decode, a workgroup per pair
+// Rotary embedding, cache write, attention and merge of a (row, kv head) pair in ONE workgroup: its waves take the pair's 32-token chunks in
+// turns and meet in LDS once.  Against rotary launch, items and merge launch it saves two launches (2.5 to 3 us each), the parts' way through
+// memory and the items' search for their row (scan, table and loads in a chain).  K/V come by LDS-DMA, a KB in one piece (fragments that
+// lanes load from the pages themselves are 16 bytes of a row each, 36 B/ns of a CU; this way 100 where the lines are in a cache), each wave's into
+// a chunk of its own, fetched again as soon as it is in registers.  The newest token is a chunk of its own, made of the projected row while
+// the first fetches are in flight: the cache counts up to the token before it.  What bounds it: up to 256 pairs the 64 KB that a CU has in flight
+// against the memory's latency, past that the memory (5.3 to 5.6 TB/s).
+// us, rotary + items or stream + merge -> this (spread lengths, heads of 128 / groups of 4 to 6): 10 rows of 1100 tokens, 8 kv heads 21.7 -> 17.5
+// (3 parts; 1: 21), 20 of 1500 37.5 -> 30.3, 32 of 400 26.9 -> 16, 101 of 1000 96 -> 86, 448 of 1050 390 -> 362, 400 of 60 47 -> 38; heads of 64, 2 kv heads (items
+// that rotate by themselves, merge): 4 of 500 10.5 -> 6.1, 512 of 1000 73 -> 55.
+// Waves of a workgroup, chunks of a CU the same throughout (128 KB): fewer for many pairs, whose prologues then hide behind other pairs.  Heads of 128, 4 and
+// 2 waves: 800 pairs of 1000 tokens 85.7, 88.9, of 60 16.1, 11.9; 1600 of 2000 307, 311, of 60 31, 22.8.  Heads of 64, 8 and 4: 512 pairs of 1000
+// 29.4, 30.1, of 60 7.0, 6.5; 1024 of 1000 55.9, 54.8, of 60 12.1, 9.0.  Twice the waves in one workgroup a CU were level and 1 to 3 us slower for short contexts.
+template <int HD, int WAVES>
+struct Pair {
+  static constexpr int PIECES = HD / 32;               // KB of a page of K or of V
+  static constexpr int RING = 4 * PIECES * 1024;       // bytes of a wave's chunk: two pages of K, two of V
+  static constexpr int QUERIES = 16 * HD * 2;
+  static constexpr int LDS = WAVES * RING + QUERIES;
+  static_assert((HD * 17 + 32) * 4 <= RING, "the parts of the waves lie where the chunks were");
+};
+
+template <int HD, int NW>
+__global__ __launch_bounds__(64 * NW, HD == 64 ? 4 : 2) void decode_pair_kernel(
+    KVGeom g, const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ seq_lens, int n_q, float scale_log2, int parts,
+    float* __restrict__ part_o, float* __restrict__ part_ml, bf16_t* __restrict__ out, FusedArgs fa) {
+  constexpr int KP = Pair<HD, NW>::PIECES, RING = Pair<HD, NW>::RING, PAGE = HD * BS * 2;
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[Pair<HD, NW>::LDS];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, h = lane >> 4;
+  const int pair = blockIdx.x / parts, part = blockIdx.x - pair * parts;
+  const int b = pair / g.n_kv, kvh = pair - b * g.n_kv, G = n_q / g.n_kv;
+  // (constant address space: scalar loads, whose wait is not one for the fetches)
+  typedef const __attribute__((address_space(4))) int* Ints;
+  auto ints = [](const int* p) { return reinterpret_cast<Ints>(reinterpret_cast<uintptr_t>(p)); };
+  const Ints table = ints(block_tables) + static_cast<size_t>(b) * max_blocks;
+  const int ctx = min(ints(seq_lens)[b], max_blocks * BS), slot = ints(fa.slots)[b];
+  const int all = (ctx + CHUNK - 1) / CHUNK, last = max(ctx - 1, 0) / BS;
+  const int start = part * all / parts, nchunk = (part + 1) * all / parts;   // the part's chunks
+  const int first = start + (w + NW - 2) % NW;   // (the two waves that rotate begin later: theirs are the last chunks of a turn)
+  int at0 = table[min(2 * first, last)], at1 = table[min(2 * first + 1, last)];
+
+  // ---- fetches.  A row of K lies in LDS with its 16-byte pieces permuted so that the 16 rows of a fragment read hit 16 places: piece x of fragment row
+  // r at place x ^ r (heads of 128: rows of 16 places) or x ^ (r / 2) (heads of 64: rows of 8, neighbours in the other half); V^T: the
+  // halves of a row swapped where bit 3 of it is set.
+  uint32_t off_k[2][KP], off_v[KP];
+#pragma unroll
+  for (int i = 0; i < KP; ++i) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+      off_k[e][i] = HD == 128 ? (4 * i + h) * 256 + ((r ^ (8 * e + 4 * (i >> 1) + h)) << 4)
+                              : (8 * i + (lane >> 3)) * 128 + (((lane & 7) ^ (4 * e + 2 * i + (h & 1))) << 4);
+    off_v[i] = i * 1024 + (lane >> 1) * 32 + (((lane ^ (lane >> 4)) & 1) << 4);
+  }
+  const uint32_t ring = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem)) + w * RING;
+  auto dma = [&](uint32_t off, const unsigned char* base, uint32_t to) {   // (s_nop: the wait state of an LDS load behind a scalar write of m0)
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(to) : "memory", "m0");
+  };
+  const unsigned char* kc = reinterpret_cast<const unsigned char*>(g.k);
+  const unsigned char* vc = reinterpret_cast<const unsigned char*>(g.v);
+  auto page = [&](int blk) { return block_base<HD>(g, blk, kvh) * 2; };
+  auto fetch_k = [&](int blk0, int blk1) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+      for (int i = 0; i < KP; ++i) dma(off_k[e][i], kc + page(e ? blk1 : blk0), ring + e * PAGE + i * 1024);
+  };
+  auto fetch_v = [&](int blk0, int blk1) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+      for (int i = 0; i < KP; ++i) dma(off_v[i], vc + page(e ? blk1 : blk0), ring + (2 + e) * PAGE + i * 1024);
+  };
+  auto begin = [&]() {
+    if (first < nchunk) {
+      fetch_k(at0, at1);   // (a chunk of one page reads it twice)
+      fetch_v(at0, at1);
+    }
+  };
+  if (w >= 2) begin();
+
+  // ---- the first wave rotates the queries, the second of the last part the new key, which it stores with the value
+  bf16_t* queries = reinterpret_cast<bf16_t*>(smem + NW * RING);   // [16][HD]
+  bool own = false;    // (a parked row stores elsewhere than it reads: its newest token is what the cache holds)
+  const int newest = max(ctx - 1, 0);
+  if (ctx > 0) own = slot == table[newest / BS] * BS + newest % BS;
+  const int cached = own ? newest : ctx;
+  const bool adds = w == 1 && part == parts - 1;
+  Chunk<HD> x;
+  if (w == 0 || adds) {
+    const bf16_t* heads = fa.qkv + static_cast<size_t>(b) * (n_q + 2 * g.n_kv) * HD;
+    const bf16_t* nw = w == 0 ? fa.q_norm : fa.k_norm;
+    u16x8 raw[HD / 32], wn[HD / 32] = {};
+    f32x4 cs[HD / 64][2], sn[HD / 64][2];
+    bf16_t nv[HD / 16];
+    load_head<HD>(raw, heads + (w == 0 ? kvh * G + (r < G ? r : 0) : n_q + kvh) * HD, h);
+    if (nw != nullptr) load_head<HD>(wn, nw, h);
+    if (w == 1) {
+#pragma unroll
+      for (int dt = 0; dt < HD / 16; ++dt) nv[dt] = heads[(n_q + g.n_kv + kvh) * HD + dt * 16 + r];
+    }
+    const float* t = fa.cos_sin + static_cast<size_t>(ints(fa.positions)[b]) * HD + 8 * h;
+#pragma unroll
+    for (int kk = 0; kk < HD / 64; ++kk)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        cs[kk][e] = *reinterpret_cast<const f32x4*>(t + kk * 32 + 4 * e);
+        sn[kk][e] = *reinterpret_cast<const f32x4*>(t + HD / 2 + kk * 32 + 4 * e);
+      }
+    bf16x8 turned[HD / 32];
+    rope_fragments<HD>(turned, raw, wn, nw != nullptr, cs, sn, fa.eps, h);
+    if (w == 0) {
+#pragma unroll
+      for (int kk = 0; kk < HD / 32; ++kk)
+        *reinterpret_cast<bf16x8*>(queries + r * HD + kk * 32 + h * 8) = r < G ? turned[kk] : bf16x8{};
+    } else {
+      const size_t base = block_base<HD>(g, slot / BS, kvh);
+      bf16_t* kd = const_cast<bf16_t*>(g.k) + base + (slot % BS) * HD + 8 * h;
+      bf16_t* vd = const_cast<bf16_t*>(g.v) + base + slot % BS;
+      if (r == 0) {
+#pragma unroll
+        for (int kk = 0; kk < HD / 32; ++kk) *reinterpret_cast<bf16x8*>(kd + kk * 32) = turned[kk];
+      }
+#pragma unroll
+      for (int dt = 0; dt < HD / 16; ++dt)
+        if (dt % 4 == h) vd[(dt * 16 + r) * BS] = nv[dt];
+      // token 0 of a chunk whose others are masked
+#pragma unroll
+      for (int kk = 0; kk < HD / 32; ++kk) x.k[0][kk] = r == 0 ? turned[kk] : bf16x8{}, x.k[1][kk] = bf16x8{};
+#pragma unroll
+      for (int dt = 0; dt < HD / 16; ++dt) {
+        u16x8 v = {};
+        v[0] = nv[dt];
+        x.v[dt] = __builtin_bit_cast(bf16x8, v);
+      }
+    }
+  }
+  if (w < 2) begin();
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  bf16x8 bq[HD / 32];
+#pragma unroll
+  for (int kk = 0; kk < HD / 32; ++kk) bq[kk] = *reinterpret_cast<const bf16x8*>(queries + r * HD + kk * 32 + h * 8);
+  float m = -INFINITY, l = 0.f;
+  f32x4 o[HD / 16];
+#pragma unroll
+  for (int dt = 0; dt < HD / 16; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (adds && own) compute_chunk<HD, AllVisible, true>(x, bq, 0, 1, AllVisible{}, scale_log2, m, l, o, lane);
+
+  constexpr int K_ROW = HD * 2;
+  const unsigned char* rk = smem + w * RING + (8 * (r >> 2) + (r & 3)) * K_ROW;
+  const unsigned char* rv = smem + w * RING + 2 * PAGE + (h >> 1) * PAGE + r * 32 + (((h ^ (r >> 3)) & 1) << 4);
+  const int swap = HD == 128 ? r : r >> 1;
+  for (int j = first; j < nchunk; j += NW) {
+    const int next = j + NW;
+    at0 = table[min(2 * next, last)];
+    at1 = table[min(2 * next + 1, last)];
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * KP) : "memory");   // all but this chunk's V
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int kk = 0; kk < HD / 32; ++kk) x.k[u][kk] = *reinterpret_cast<const bf16x8*>(rk + u * 4 * K_ROW + (((kk * 4 + h) ^ swap) << 4));
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (next < nchunk) {
+      fetch_k(at0, at1);
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * KP) : "memory");   // all but the next chunk's K
+    } else {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+#pragma unroll
+    for (int dt = 0; dt < HD / 16; ++dt) x.v[dt] = *reinterpret_cast<const bf16x8*>(rv + dt * 512);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (next < nchunk) fetch_v(at0, at1);
+    const int tj = j * CHUNK;
+    if (tj + CHUNK <= cached)   // wave-uniform: a full chunk needs no tail masking
+      compute_chunk<HD, AllVisible, false>(x, bq, tj, cached, AllVisible{}, scale_log2, m, l, o, lane);
+    else if (tj < cached)
+      compute_chunk<HD, AllVisible, true>(x, bq, tj, cached, AllVisible{}, scale_log2, m, l, o, lane);
+  }
+
+  // ---- the waves' parts meet (every fetch has landed: the last chunk of a wave waits for all of its own)
+  __syncthreads();
+  float* ml = reinterpret_cast<float*>(smem);             // [NW][2][16]
+  float* po = ml + NW * 32;                               // [NW][HD][17]
+  if (h == 0) {
+    ml[w * 32 + r] = m;
+    ml[w * 32 + 16 + r] = l;
+  }
+#pragma unroll
+  for (int dt = 0; dt < HD / 16; ++dt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) po[(w * HD + dt * 16 + 4 * h + i) * 17 + r] = o[dt][i];
+  __syncthreads();
+  for (int idx = tid; idx < G * HD; idx += 64 * NW) {
+    const int qi = idx / HD, d = idx % HD;
+    float mm = -INFINITY;
+#pragma unroll
+    for (int ww = 0; ww < NW; ++ww) mm = fmaxf(mm, ml[ww * 32 + qi]);
+    float ll = 0.f, oo = 0.f;
+#pragma unroll
+    for (int ww = 0; ww < NW; ++ww) {
+      const float mw = ml[ww * 32 + qi];
+      const float f = mw == -INFINITY ? 0.f : exp2f(mw - mm);
+      ll += ml[ww * 32 + 16 + qi] * f;
+      oo += po[(ww * HD + d) * 17 + qi] * f;
+    }
+    const size_t head = static_cast<size_t>(b) * n_q + kvh * G + qi;
+    if (parts == 1) {
+      out[head * HD + d] = f2bf(ll > 0.f ? oo / ll : 0.f);
+    } else {
+      part_o[(head * parts + part) * HD + d] = oo;
+      if (d == 0) *reinterpret_cast<float2*>(part_ml + (head * parts + part) * 2) = float2{mm, ll};
+    }
+  }
+}
+
 // Split merge: one wave per (row, query head), four per workgroup.  Lane s holds split s's
 // (m, l) -- all of them fetched by ONE load instruction, reduced with cross-lane ops --
 // then every split's O partial (HD floats, one coalesced load per split, HD / 64 per lane)
@@ -955,7 +1080,7 @@ __global__ __launch_bounds__(64 * COMBINE_WAVES) void decode_combine_kernel(
   const int own = max(0, seq_lens[b] - (kv_begin ? kv_begin[b] : 0));
   // <= max_splits <= 64 (host check); slots 0 .. split_base[b]-1 hold the shared-prefix partials
   const int base = split_base ? split_base[b] : 0;
-  int ns = base + (own + split_tokens - 1) / split_tokens;
+  int ns = split_tokens == 0 ? max_splits : base + (own + split_tokens - 1) / split_tokens;   // (0: all slots are parts)
   if constexpr (STREAM) {   // (a row without tokens has no parts and no end)
     const unsigned long long ends = __ballot(lane >= base && (lane >= max_splits || __builtin_bit_cast(uint32_t, mlv.x) == PARTS_END));
     ns = own == 0 ? base : ends != 0 ? __ffsll(ends) - 1 : 64;
@@ -1121,17 +1246,17 @@ struct Cascade {
   int split_tokens;       // shared tokens per item (a multiple of CHUNK)
 };
 
-template <int HD, bool F8 = false, int CPW = 1, bool FUSED = false>
+template <int HD, bool F8 = false, int CPW = 1>
 void launch_decode(const bf16_t* q, KVGeom g, const int* tables, int max_blocks, const int* seq_lens, int B,
                    int n_q, float sl, float* ws, int max_splits, bf16_t* out, const Cascade& cas,
-                   hipStream_t stream, const FusedArgs& fa = FusedArgs{}) {
+                   hipStream_t stream) {
   constexpr int DEC_SPLIT = DEC_WAVES * CHUNK * CPW;
   const int shared_slots = cas.kv_begin ? DEC_MAX_SHARED_SPLITS : 0;
   // Streamed from 256 pairs of row and kv head on (8 or 2 kv heads; times over those of the items): 256 pairs 0.99 to 1.01 up to 1050 tokens, 0.92 at 1700,
   // 0.91 at 8000; 320: 0.99, 0.93, 0.93; 512: 0.95 at 250, 0.94, 0.88.  Below them it varies: 1.01 to 1.03 up to 600 tokens (this instance's items),
   // 160 pairs 1.03 to 1.05 at 1700 to 4000 and 0.96 at 8000, 192 and 224 0.91 to 0.97 there, 64 to 128 0.94 to 1.05 at 2500 and 4000.
   // (With one slot a row's range could be cut into more parts than there are slots.)
-  const bool streamed = HD == 128 && !F8 && !FUSED && n_q / g.n_kv <= STREAM_G && B * g.n_kv >= 256 && max_splits - shared_slots >= 2;
+  const bool streamed = HD == 128 && !F8 && n_q / g.n_kv <= STREAM_G && B * g.n_kv >= 256 && max_splits - shared_slots >= 2;
   if (!streamed) max_splits = std::min(max_splits, (max_blocks * BS + DEC_SPLIT - 1) / DEC_SPLIT + shared_slots);   // no slot to spare
   float* part_o = ws;
   float* part_ml = ws + static_cast<size_t>(B) * n_q * max_splits * HD;
@@ -1150,12 +1275,12 @@ void launch_decode(const bf16_t* q, KVGeom g, const int* tables, int max_blocks,
       int per_cu = 0, cus = 0, dev = 0;
       hipGetDevice(&dev);
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, decode_attn_kernel<HD, F8, CPW, FUSED, STREAM>, 256, 0);
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, decode_attn_kernel<HD, F8, CPW, STREAM>, 256, 0);
       resident = std::max(1, per_cu) * std::max(1, cus);
     }
     const int grid = static_cast<int>(std::min<long>(static_cast<long>(B) * g.n_kv * max_splits, resident));
-    hipLaunchKernelGGL((decode_attn_kernel<HD, F8, CPW, FUSED, STREAM>), dim3(grid), dim3(256), 0, stream, q, g, tables, max_blocks,
-                       seq_lens, B, n_q, sl, part_o, part_ml, max_splits, cas.kv_begin, cas.split_base, fa);
+    hipLaunchKernelGGL((decode_attn_kernel<HD, F8, CPW, STREAM>), dim3(grid), dim3(256), 0, stream, q, g, tables, max_blocks,
+                       seq_lens, B, n_q, sl, part_o, part_ml, max_splits, cas.kv_begin, cas.split_base);
   };
   const int n_bq = B * n_q;
   auto merge = [&](auto stream_c) {
@@ -1163,7 +1288,7 @@ void launch_decode(const bf16_t* q, KVGeom g, const int* tables, int max_blocks,
                        dim3(64 * COMBINE_WAVES), 0, stream, part_o, part_ml, seq_lens, n_q, max_splits, DEC_SPLIT, n_bq,
                        out, cas.kv_begin, cas.split_base);
   };
-  if constexpr (HD == 128 && !F8 && !FUSED) {
+  if constexpr (HD == 128 && !F8) {
     if (streamed) {
       run(std::true_type{});
       merge(std::true_type{});
@@ -1838,22 +1963,34 @@ BCG_API int bcg_paged_attention_decode(const void* q, const void* k_cache, const
   return BCG_CHECK_LAUNCH();
 }
 
-// Rotary embedding, cache write and attention of a decode step (decode_attn_kernel, FUSED): qkv [B, n_q + 2 n_kv, hd] as projected,
-// one new token per row at `slots`; bf16 caches, hd 64.  workspace, max_splits, split_tokens as
-// bcg_paged_attention_decode without shared prefixes.
-BCG_API int bcg_decode_fused(const void* qkv, const int* positions, const int* slots, const void* q_norm, const void* k_norm,
+// Rotary embedding, cache write and attention of a decode step (decode_pair_kernel): qkv [B, n_q + 2 n_kv, hd] as projected, one new token per row
+// at `slots`; bf16 caches, hd 64 or 128.  `parts` workgroups take a (row, kv head) pair; workspace: B n_q parts (hd + 2) floats, of one part
+// none.
+BCG_API int bcg_decode_pairs(const void* qkv, const int* positions, const int* slots, const void* q_norm, const void* k_norm,
                              const float* cos_sin, float eps, void* k_cache, void* v_cache, int layer, int num_blocks, int n_kv,
                              const int* block_tables, int max_blocks, const int* seq_lens, int B, int n_q, int hd, int block_size,
-                             float scale, float* workspace, int max_splits, int split_tokens, void* out, hipStream_t stream) {
-  if (hd != 64 || block_size != BS || n_kv <= 0 || n_q % n_kv || n_q / n_kv > 16 || B <= 0 || B > DEC_MAX_B) return -2;
-  if (split_tokens != DEC_WAVES * CHUNK * DEC_CPW || max_splits * split_tokens < max_blocks * BS || max_splits > 64) return -3;
+                             float scale, int parts, float* workspace, void* out, hipStream_t stream) {
+  if ((hd != 64 && hd != 128) || block_size != BS || n_kv <= 0 || n_q % n_kv || n_q / n_kv > 16 || B <= 0 || B > DEC_MAX_B || max_blocks <= 0) return -2;
+  if (parts < 1 || parts > 64 || (parts > 1 && !workspace) || max_blocks * BS > bcg_decode_max_context(0)) return -3;
   const KVGeom g{static_cast<const bf16_t*>(k_cache), static_cast<const bf16_t*>(v_cache), layer, num_blocks, n_kv};
   const FusedArgs fa{static_cast<const bf16_t*>(qkv), positions, slots, static_cast<const bf16_t*>(q_norm),
                      static_cast<const bf16_t*>(k_norm), cos_sin, eps};
-  const Cascade none{nullptr, nullptr, nullptr, 0, nullptr, 0, nullptr, nullptr, 0, CHUNK};
-  bf16_t* ob = static_cast<bf16_t*>(out);
-  launch_decode<64, false, DEC_CPW, true>(nullptr, g, block_tables, max_blocks, seq_lens, B, n_q, scale * LOG2E, workspace, max_splits, ob,
-                                          none, stream, fa);
+  auto run = [&](auto hd_c, auto waves_c) {
+    constexpr int HD = decltype(hd_c)::value, NW = decltype(waves_c)::value;
+    float* part_ml = workspace + static_cast<size_t>(B) * n_q * parts * HD;
+    bf16_t* o = static_cast<bf16_t*>(out);
+    hipLaunchKernelGGL((decode_pair_kernel<HD, NW>), dim3(B * n_kv * parts), dim3(64 * NW), 0, stream, g, block_tables, max_blocks, seq_lens,
+                       n_q, scale * LOG2E, parts, workspace, part_ml, o, fa);
+    if (parts > 1)
+      hipLaunchKernelGGL((decode_combine_kernel<HD, false>), dim3((B * n_q + COMBINE_WAVES - 1) / COMBINE_WAVES), dim3(64 * COMBINE_WAVES), 0, stream,
+                         workspace, part_ml, seq_lens, n_q, parts, 0, B * n_q, o, nullptr, nullptr);
+  };
+  const bool many = static_cast<int64_t>(B) * n_kv * parts > (hd == 64 ? 512 : 1024);   // (see Pair)
+  using std::integral_constant;
+  if (hd == 64)
+    many ? run(integral_constant<int, 64>{}, integral_constant<int, 4>{}) : run(integral_constant<int, 64>{}, integral_constant<int, 8>{});
+  else
+    many ? run(integral_constant<int, 128>{}, integral_constant<int, 2>{}) : run(integral_constant<int, 128>{}, integral_constant<int, 4>{});
   return BCG_CHECK_LAUNCH();
 }
 
