@@ -128,6 +128,7 @@ def load_library(path: str = None) -> ctypes.CDLL:
         "bcg_rope_multi_kv_write": [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
                                     c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
         "bcg_multimap_split_keys": [],
+        "bcg_multimap_pairs": [c_int] * 5,
         "bcg_multimap_attention": [c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p,
                                    c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
                                    c_float, c_float, c_float, c_float, c_int, c_int, c_int, c_int, c_void_p, c_float,
@@ -294,16 +295,20 @@ def few_rows_pay(M: int, N: int, row_bytes: int, gated: bool) -> bool:
 
 def decode_parts(B: int, n_kv: int, hd: int, tokens: int) -> int:
     """Workgroups that share a (row, kv head) pair of a decode step (csrc/kernels/attention.hip, decode_pair_kernel); tokens: context that the block table
-    has room for (the contexts themselves are on the device).
+    has room for (the contexts themselves are on the device)."""
+    return pair_parts(B * n_kv, tokens * hd * 4)
+
+
+def pair_parts(pairs: int, pair: int) -> int:
+    """The same of `pairs` pairs that read up to `pair` bytes each.
 
     One, whose merge is its own, up to 448 KB of K/V of a pair, or where the pairs fill the CUs; else as many as there are CUs, up to one
     for each 128 KB (us for 1, 2, 3, 4, 8 parts): heads of 128, 80 pairs of 400 tokens 9.4, 12.3, 12.5, of 1000 19.5, 17.9, 16.7, of 2500 38.6, 29.1,
     27.3; 160 pairs of 1000 22.8, 28.6; 8 pairs of 400 8.1, 9.8, 10, 9.5, of 1000 11, 11.8, 11.5, 10.4, 10.1, of 6000 36, 24, 20, 16.7, 13.5; heads of 64, 8 pairs of
     1000 7.3, 9, 9.1, 8.2, 8.4, of 2500 12.3, 11.9, 11.1, 9.7, 9.3; 128 pairs of 4000 34.8, 31.4."""
-    pair = tokens * hd * 4
     if pair <= 448 * 1024:
         return 1
-    return max(1, min(256 // (B * n_kv), -(-pair // (128 * 1024)), 16))
+    return max(1, min(256 // pairs, -(-pair // (128 * 1024)), 16))
 
 
 def decode_fused_pays(B: int, n_kv: int, splits: int) -> bool:

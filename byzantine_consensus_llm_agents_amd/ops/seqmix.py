@@ -81,6 +81,8 @@ def few_row_tiles(n_slots, E, W, ff, rows):
 
 
 def seqmix_ops(lib, linear):
+    from .hip import pair_parts
+
     split_keys = lib.bcg_multimap_split_keys()
     tile_rows = lib.bcg_moe_tile_rows()
     few_rows = lib.bcg_moe_rows_tile()
@@ -234,6 +236,16 @@ def seqmix_ops(lib, linear):
                   _p(slopes), keep, _stream())
 
         def decode(work, n_items):
+            if (not f32 and BS == 16 and n_items <= 65535 and (k_cache.data_ptr() | v_cache.data_ptr()) % 16 == 0
+                    and lib.bcg_multimap_pairs(maps, dim, vdim, int(softcap > 0 or slopes is not None), keep)):
+                span = bt.shape[1] * BS
+                if window or chunk:   # (whole chunks of 32 keys, of the kept ones too)
+                    span = min(span, keep + max(window, chunk) + 64)
+                parts = pair_parts(n_items * G * -(-(H // G) // 16), span * (maps * dim + vdim) * 2)
+                ws = torch.empty(n_items * H * parts * (2 * maps + maps * vdim), dtype=torch.float32, device=q.device) if parts > 1 else None
+                _check(lib.bcg_multimap_attention(2, _p(q), _p(k_cache), _p(v_cache), _p(bt), bt.shape[1], None, _p(lens),
+                                                  _p(work), n_items, _p(out), _p(ws), parts, *common), "multimap decode")
+                return
             n_splits = max(1, (bt.shape[1] * BS + split_keys - 1) // split_keys)
             if window or chunk:  # splits are counted from the window's (chunk's) first: it touches this many at most
                 n_splits = min(n_splits, (keep + split_keys - 1) // split_keys + (max(window, chunk) + split_keys - 1) // split_keys + 1)

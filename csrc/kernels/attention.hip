@@ -859,7 +859,7 @@ struct Pair {
   static constexpr int RING = 4 * PIECES * 1024;       // bytes of a wave's chunk: two pages of K, two of V
   static constexpr int QUERIES = 16 * HD * 2;
   static constexpr int LDS = WAVES * RING + QUERIES;
-  static_assert((HD * 17 + 32) * 4 <= RING, "the parts of the waves lie where the chunks were");
+  static_assert((HD * 17 + 64) * 4 <= RING, "the parts of the waves lie where the chunks were");
 };
 
 template <int HD, int NW>
@@ -1024,7 +1024,8 @@ __global__ __launch_bounds__(64 * NW, HD == 64 ? 4 : 2) void decode_pair_kernel(
   // ---- the waves' parts meet (every fetch has landed: the last chunk of a wave waits for all of its own)
   __syncthreads();
   float* ml = reinterpret_cast<float*>(smem);             // [NW][2][16]
-  float* po = ml + NW * 32;                               // [NW][HD][17]
+  float* fac = ml + NW * 32;                              // [NW][16] factors of the waves' parts, [16] of their sum
+  float* po = fac + NW * 32;                              // [NW][HD][17]
   if (h == 0) {
     ml[w * 32 + r] = m;
     ml[w * 32 + 16 + r] = l;
@@ -1034,26 +1035,30 @@ __global__ __launch_bounds__(64 * NW, HD == 64 ? 4 : 2) void decode_pair_kernel(
 #pragma unroll
     for (int i = 0; i < 4; ++i) po[(w * HD + dt * 16 + 4 * h + i) * 17 + r] = o[dt][i];
   __syncthreads();
-  for (int idx = tid; idx < G * HD; idx += 64 * NW) {
-    const int qi = idx / HD, d = idx % HD;
+  if (tid < G) {
     float mm = -INFINITY;
 #pragma unroll
-    for (int ww = 0; ww < NW; ++ww) mm = fmaxf(mm, ml[ww * 32 + qi]);
-    float ll = 0.f, oo = 0.f;
+    for (int ww = 0; ww < NW; ++ww) mm = fmaxf(mm, ml[ww * 32 + tid]);
+    float ll = 0.f;
 #pragma unroll
     for (int ww = 0; ww < NW; ++ww) {
-      const float mw = ml[ww * 32 + qi];
+      const float mw = ml[ww * 32 + tid];
       const float f = mw == -INFINITY ? 0.f : exp2f(mw - mm);
-      ll += ml[ww * 32 + 16 + qi] * f;
-      oo += po[(ww * HD + d) * 17 + qi] * f;
+      fac[ww * 16 + tid] = f;
+      ll += ml[ww * 32 + 16 + tid] * f;
     }
+    fac[NW * 16 + tid] = ll > 0.f ? 1.f / ll : 0.f;
+    if (parts > 1) *reinterpret_cast<float2*>(part_ml + ((static_cast<size_t>(b) * n_q + kvh * G + tid) * parts + part) * 2) = float2{mm, ll};
+  }
+  __syncthreads();
+  for (int idx = tid; idx < G * HD; idx += 64 * NW) {
+    const int qi = idx / HD, d = idx % HD;
+    float oo = 0.f;
+#pragma unroll
+    for (int ww = 0; ww < NW; ++ww) oo += po[(ww * HD + d) * 17 + qi] * fac[ww * 16 + qi];
     const size_t head = static_cast<size_t>(b) * n_q + kvh * G + qi;
-    if (parts == 1) {
-      out[head * HD + d] = f2bf(ll > 0.f ? oo / ll : 0.f);
-    } else {
-      part_o[(head * parts + part) * HD + d] = oo;
-      if (d == 0) *reinterpret_cast<float2*>(part_ml + (head * parts + part) * 2) = float2{mm, ll};
-    }
+    if (parts == 1) out[head * HD + d] = f2bf(oo * fac[NW * 16 + qi]);
+    else part_o[(head * parts + part) * HD + d] = oo;
   }
 }
 

@@ -24,8 +24,10 @@
 //
 // decode_mfma_kernel: single-token rows.  The 16 MFMA columns hold the query heads that share
 // one KV head (GQA packing), so the cache is read once per KV head; one wave per 128-key split.
-// The split size is fixed, so a row's result does not depend on what else is in the batch.
 // decode_merge_kernel merges the splits and applies the map combination + head norm.
+//
+// decode_pair_kernel: single-token rows of exact shapes with 16-token pages, a workgroup per (row, KV head x column group),
+// or for each of a few parts of one.
 //
 // Optional, for one-map heads: a sliding window (a query at position i sees keys j with
 // i - j < window) or a chunk mask (position i sees j <= i of its own chunk, floor(i / chunk) ==
@@ -69,6 +71,7 @@ struct AttnArgs {
   float softcap;            // > 0: scaled scores are capped, cap tanh(s / cap)   (SHAPED instances)
   const float* slopes;      // [H] or null: slope_h (i - j) is taken off the score (SHAPED instances)
   int swz;                  // fragment-major slabs (see the top of the file)
+  int parts;                // decode: 0: n_splits is the most splits of SPLIT_KEYS keys that a row has; else every row has n_splits parts
 };
 
 // Maximum / sum over the four lanes that share a column (lanes col, col + 16, col + 32, col + 48): register swaps, no LDS
@@ -712,6 +715,272 @@ __global__ __launch_bounds__(64, OCC) void decode_mfma_kernel(AttnArgs a) {
       }
 }
 
+// The same rows for exact shapes (bf16, 16-token pages, fragment-major slabs), a workgroup per part of an (item, KV head x column group) pair.
+//
+// Its waves take the pair's 32-key chunks in turns and meet in LDS.  A page's slab is contiguous, so K and V come by LDS-DMA, 1 KB
+// of a slab in one piece, each wave's into a chunk of its own, fetched again as soon as its fragments are in registers (V's 4-key groups with
+// their 128-byte halves swapped in every other one, so that the lane groups of a fragment read differ in banks).  One part is merged, combined
+// and normed here; more are merged by decode_merge_kernel.  Against a wave per split of 128 keys and the merge of all splits it saves a
+// launch and the splits' way through memory, and its loads are 16 bytes a lane instead of 8.  What bounds it: memory from some 256 pairs on (4.8 to
+// 5.1 TB/s), below that a CU's intake and the chain of table, fetch, sums and merge.
+// us, splits and merge -> this (spread lengths): two 64-wide maps over 128-wide values, 32 heads on 8, 64 rows of 1000 74 -> 54, 1 of 40 11 -> 6.2, 1 of 2000 23.5 ->
+// 16.5 (8 parts), 200 of 500 114 -> 80; 16 latent heads of 192 / 128 behind a window of 512, 64 rows 14.8 -> 11.4, 1 row of 500 11.0 -> 9.0; 32 heads on 8 of
+// 128 behind a window of 512, 16 rows 14.7 -> 11.1.  Two waves from 1025 pairs on, whose prologues hide behind more pairs: 200 rows of 40 tokens, 8 KV
+// heads, two maps 25 -> 18 (splits 21), one 128-wide map 21 -> 15 (16.7); of 500 tokens 80.4, 80 and 76, 80.
+template <int KC, int VT, int NM, int MODE, int NW>
+__global__ __launch_bounds__(64 * NW, NM * KC + VT > 24 ? 1 : 2) void decode_pair_kernel(AttnArgs a) {
+  typedef s16x4 F;
+  constexpr int DIM = 16 * KC, VD = 16 * VT, KD = NM * DIM;
+  constexpr int KB = KD * 32, VB = VD * 32, KP = KB / 1024, VP = VB / 1024, RING = 2 * (KB + VB);   // bytes of a page of K and of V, KB, of a wave's chunk
+  static_assert(KB % 1024 == 0 && VB % 1024 == 0, "whole pieces");
+  static_assert((VD * 17 + 64) * 4 <= RING && 16 * VD * 4 <= NW * RING, "the parts of the waves lie where the chunks were");
+  constexpr int SWAP = VD % 32 == 0 ? 128 : 0;
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[NW * RING];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 15, grp = lane >> 4;
+  const int parts = a.n_splits, part = blockIdx.x % parts, pair = blockIdx.x / parts;
+  const int per = a.H / a.G, g = pair % a.G, cg = pair / a.G, item = blockIdx.y;
+  // (constant address space: scalar loads, whose wait is not one for the fetches)
+  typedef const __attribute__((address_space(4))) int* Ints;
+  auto ints = [](const int* p) { return reinterpret_cast<Ints>(reinterpret_cast<uintptr_t>(p)); };
+  const int row = a.work ? ints(a.work)[2 * item] : item, seq = a.work ? ints(a.work)[2 * item + 1] : item;
+  const int ctx = ints(a.seq_lens)[seq], pos = ctx - 1;
+  const Ints table = ints(a.block_tables) + static_cast<size_t>(seq) * a.max_blocks;
+  // this part's chunks: those that hold kept keys come before the window's
+  const int lo = first_key(a, pos), win = lo / 32, keep = MODE == KEEP ? a.keep : 0;
+  const int kept = MODE == KEEP ? min((keep + 31) / 32, win) : 0;
+  const int all = ctx > 0 ? kept + (ctx + 31) / 32 - win : 0, begin = part * all / parts, end = (part + 1) * all / parts;
+  const int last_page = min(max(ctx - 1, 0) / 16, a.max_blocks - 1);
+  auto key_of = [&](int j) { return 32 * (MODE != KEEP || j >= kept ? win + j - kept : j); };
+  auto page_of = [&](int p) {   // past the sequence: its last page again, every key of it is masked
+    const int page = table[min(p, last_page)];
+    return static_cast<size_t>((page < 0 || page >= a.num_blocks) ? 0 : page) * a.G + g;
+  };
+  const uint32_t ring = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem)) + w * RING;
+  auto dma = [&](uint32_t off, const unsigned char* base, uint32_t to) {   // (s_nop: the wait state of an LDS load behind a scalar write of m0)
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(to) : "memory", "m0");
+  };
+  const unsigned char* kc_base = static_cast<const unsigned char*>(a.k_cache);
+  const unsigned char* vc_base = static_cast<const unsigned char*>(a.v_cache);
+  auto fetch_k = [&](size_t s0, size_t s1) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+      for (int i = 0; i < KP; ++i) dma(i * 1024 + lane * 16, kc_base + (e ? s1 : s0) * KB, ring + e * KB + i * 1024);
+  };
+  auto fetch_v = [&](size_t s0, size_t s1) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+      for (int i = 0; i < VP; ++i) {
+        const uint32_t at = i * 1024 + lane * 16;
+        dma(SWAP ? at ^ ((at / (VD * 8) & 1) * SWAP) : at, vc_base + (e ? s1 : s0) * VB, ring + 2 * KB + e * VB + i * 1024);
+      }
+  };
+  size_t s0 = 0, s1 = 0;
+  auto look = [&](int j) {
+    const int p = key_of(j) / 16;
+    s0 = page_of(p);
+    s1 = page_of(p + 1);
+  };
+  const int h = g * per + min(16 * cg + col, per - 1);
+  const bf16_t* qrow = static_cast<const bf16_t*>(a.q) + (static_cast<size_t>(row) * a.H + h) * KD;
+  F qf[NM][KC];
+#pragma unroll
+  for (int m = 0; m < NM; ++m)
+#pragma unroll
+    for (int c = 0; c < KC; ++c) qf[m][c] = *reinterpret_cast<const F*>(qrow + m * DIM + 16 * c + 4 * grp);
+  const float slope = MODE == SHAPED && a.slopes != nullptr ? a.slopes[h] * LOG2E : 0.f;
+  // (all of these are here before the first fetch: a wait for them behind it would be one for the chunk)
+#pragma unroll
+  for (int m = 0; m < NM; ++m)
+#pragma unroll
+    for (int c = 0; c < KC; ++c) asm volatile("" : "+v"(qf[m][c]));
+  if (begin + w < end) {
+    look(begin + w);
+    fetch_k(s0, s1);
+    fetch_v(s0, s1);
+  }
+  f32x4 acc[NM][VT];
+  float mx[NM], den[NM];
+#pragma unroll
+  for (int m = 0; m < NM; ++m) {
+    mx[m] = MAX_FLOOR;
+    den[m] = 0.f;
+#pragma unroll
+    for (int t = 0; t < VT; ++t) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  const float sc = a.scale * LOG2E;
+  const float cap = MODE == SHAPED ? a.softcap : 0.f;
+  const float cap2 = cap * LOG2E, arg2 = cap > 0.f ? 2.0f * LOG2E * a.scale / cap : 0.f;
+  const bf16_t* ks = reinterpret_cast<const bf16_t*>(smem + w * RING);
+  const unsigned char* vs = smem + w * RING + 2 * KB;
+  const uint32_t v_lane = grp * VD * 8 + ((col * 8) ^ ((grp & 1) * SWAP));   // (a feature tile is 128 bytes: tiles alternate between the halves)
+
+  for (int j = begin + w; j < end; j += NW) {
+    const bool more = j + NW < end;
+    if (more) look(j + NW);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * VP) : "memory");   // all but this chunk's V
+    F kf[2][NM][KC];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int m = 0; m < NM; ++m)
+#pragma unroll
+        for (int c = 0; c < KC; ++c) kf[u][m][c] = *reinterpret_cast<const F*>(ks + u * 16 * KD + ((m * DIM + 16 * c) / 4 * 16 + grp * 16 + col) * 4);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (more) {
+      fetch_k(s0, s1);
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * KP) : "memory");   // all but the next chunk's K
+    } else {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    F vf[2][VT];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int t = 0; t < VT; ++t) {
+        const uint32_t at = SWAP ? (v_lane ^ (t % 2 * 128)) + t / 2 * 256 : v_lane + t * 128;
+        vf[u][t] = *reinterpret_cast<const F*>(vs + u * VB + at);
+      }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (more) fetch_v(s0, s1);
+    f32x4 sm[2][NM];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int m = 0; m < NM; ++m) sm[u][m] = mma_row<bf16_t, KC>(KC, [&](int c) { return kf[u][m][c]; }, [&](int c) { return qf[m][c]; });
+    const int key0 = key_of(j);
+    const bool masked = key0 + 31 > pos || key0 < lo;
+    float cap_now = cap;
+    if constexpr (MODE == SHAPED) asm volatile("" : "+v"(cap_now));
+    const bool capped = cap_now > 0.f;
+    F pf[2][NM];
+#pragma unroll
+    for (int m = 0; m < NM; ++m) {
+      float v[2][4], bm = -INFINITY;
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int key = key0 + 16 * u + 4 * grp + i;
+          if constexpr (MODE == SHAPED) {
+            float y = sm[u][m][i] * sc;
+            if (capped) y = cap2 - 2.0f * cap2 * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(sm[u][m][i] * arg2) + 1.0f);
+            v[u][i] = y - slope * static_cast<float>(pos - key);
+          } else {
+            v[u][i] = sm[u][m][i] * sc;
+          }
+          if (masked && (key > pos || (key < lo && !(MODE == KEEP && key < keep)))) v[u][i] = -INFINITY;
+          bm = fmaxf(bm, v[u][i]);
+        }
+      const float m_new = fmaxf(mx[m], column_max(bm));
+      float ps = 0.f;
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          v[u][i] = __builtin_amdgcn_exp2f(v[u][i] - m_new);
+          ps += v[u][i];
+        }
+      if (__any(m_new > mx[m])) {
+        const float alpha = __builtin_amdgcn_exp2f(mx[m] - m_new);
+        den[m] *= alpha;
+#pragma unroll
+        for (int t = 0; t < VT; ++t) acc[m][t] *= alpha;
+      }
+      den[m] += ps;
+      mx[m] = m_new;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) pf[u][m] = Elem<bf16_t>::pack(v[u][0], v[u][1], v[u][2], v[u][3]);
+    }
+#pragma unroll
+    for (int t = 0; t < VT; ++t)
+#pragma unroll
+      for (int m = 0; m < NM; ++m) acc[m][t] = mma32(vf[0][t], vf[1][t], pf[0][m], pf[1][m], acc[m][t]);
+  }
+
+  // ---- the waves' parts meet, map after map (every fetch has landed: the last chunk of a wave waits for all of its own)
+  constexpr int TH = 64 * NW, N_OUT = 16 * VD / TH;    // elements of the heads' outputs per thread
+  float* ml = reinterpret_cast<float*>(smem);          // [NW][2][16]
+  float* fac = ml + NW * 32;                           // [NW][16] factors of the waves' parts, [16] of their sum
+  float* po = fac + NW * 32;                           // [NW][VD][17]
+  const int heads = min(16, per - 16 * cg), h0 = g * per + 16 * cg;
+  float res[N_OUT];                                    // element tid + TH i: head, value feature
+#pragma unroll
+  for (int m = 0; m < NM; ++m) {
+    const float d = column_sum(den[m]);
+    __syncthreads();
+    if (grp == 0) {
+      ml[w * 32 + col] = mx[m];
+      ml[w * 32 + 16 + col] = d;
+    }
+#pragma unroll
+    for (int t = 0; t < VT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) po[(w * VD + 16 * t + 4 * grp + i) * 17 + col] = acc[m][t][i];
+    __syncthreads();
+    if (tid < 16) {
+      const bool sinks = m == 0 && parts == 1 && a.sink != nullptr && tid < heads;
+      const float sink = sinks ? a.sink[h0 + tid] * LOG2E : MAX_FLOOR;
+      float mm = sink;
+#pragma unroll
+      for (int x = 0; x < NW; ++x) mm = fmaxf(mm, ml[x * 32 + tid]);
+      float ll = sinks ? exp2f(sink - mm) : 0.f;
+#pragma unroll
+      for (int x = 0; x < NW; ++x) {
+        const float f = exp2f(ml[x * 32 + tid] - mm);
+        fac[x * 16 + tid] = f;
+        ll += ml[x * 32 + 16 + tid] * f;
+      }
+      fac[NW * 16 + tid] = (m == 0 ? 1.0f : -a.lam) / ll;
+      if (parts > 1 && tid < heads) {
+        float* ws = a.ws + ((static_cast<size_t>(item) * a.H + h0 + tid) * parts + part) * (2 * NM + NM * VD);
+        ws[m] = mm, ws[NM + m] = ll;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < N_OUT; ++i) {
+      const int idx = tid + TH * i, hh = idx / VD, e = idx % VD;
+      if (hh >= heads) break;
+      float oo = 0.f;
+#pragma unroll
+      for (int x = 0; x < NW; ++x) oo += po[(x * VD + e) * 17 + hh] * fac[x * 16 + hh];
+      if (parts > 1) {
+        a.ws[((static_cast<size_t>(item) * a.H + h0 + hh) * parts + part) * (2 * NM + NM * VD) + 2 * NM + m * VD + e] = oo;
+      } else {
+        const float c = fac[NW * 16 + hh];
+        res[i] = m == 0 ? oo * c : res[i] + oo * c;
+      }
+    }
+  }
+  if (parts > 1) return;
+  bf16_t* rows = static_cast<bf16_t*>(a.out) + (static_cast<size_t>(row) * a.H + h0) * VD;
+  if (a.head_eps < 0.f) {   // no norm
+#pragma unroll
+    for (int i = 0; i < N_OUT; ++i) {
+      if ((tid + TH * i) / VD >= heads) break;
+      rows[tid + TH * i] = f2bf(res[i] * a.out_scale);
+    }
+    return;
+  }
+  __syncthreads();
+  float* out = reinterpret_cast<float*>(smem);         // [16][VD]
+#pragma unroll
+  for (int i = 0; i < N_OUT; ++i) {
+    if ((tid + TH * i) / VD >= heads) break;
+    out[tid + TH * i] = res[i];
+  }
+  __syncthreads();
+  for (int hh = w; hh < heads; hh += NW) {
+    float ss = 0.f;
+    for (int e = lane; e < VD; e += 64) ss += out[hh * VD + e] * out[hh * VD + e];
+    ss = wave_sum(ss);
+    const float r = 1.0f / sqrtf(ss / VD + a.head_eps) * a.out_scale;
+    for (int e = lane; e < VD; e += 64) rows[hh * VD + e] = f2bf(out[hh * VD + e] * r);
+  }
+}
+
 // ws layout per (item, head, split): [maps] max, [maps] denominator, [maps][vdim] numerators.  A wave per head: the
 // lanes take the splits' maxima and denominators side by side, then the splits' numerators, four in flight (a split after
 // the other, each behind the load of its maximum, cost 20.5 us at 64 rows x 32 heads x 8 splits of two 128-wide maps;
@@ -721,7 +990,7 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(AttnArgs a) {
   const int lane = threadIdx.x, h = blockIdx.x, item = blockIdx.y;
   const int row = a.work ? a.work[2 * item] : item, seq = a.work ? a.work[2 * item + 1] : item;
   const int ctx = a.seq_lens[seq];
-  const int n = min(a.n_splits, split_count(a, first_key(a, ctx - 1), ctx));
+  const int n = a.parts ? a.n_splits : min(a.n_splits, split_count(a, first_key(a, ctx - 1), ctx));
   const float sink = a.sink != nullptr ? a.sink[h] * LOG2E : MAX_FLOOR;
   const int stride = 2 * a.maps + a.maps * a.vdim;
   const float* w = a.ws + (static_cast<size_t>(item) * a.H + h) * a.n_splits * stride;
@@ -805,16 +1074,7 @@ int launch_prefill_mode(const AttnArgs& a, int n_tiles, bool full, hipStream_t s
 }
 
 template <typename T, int MODE>
-void launch_decode_mode(const AttnArgs& a, dim3 grid, bool full, hipStream_t s) {
-  if constexpr (sizeof(T) == 2) if (full && a.swz && a.BS == 16) {
-#define BCG_X(KC_, VT_, KT_, OCC_)                                                               \
-  if (a.dim == 16 * KC_ && a.vdim == 16 * VT_) {                                                 \
-    decode_mfma_kernel<T, KC_, VT_, KT_, true, true, OCC_, 1, 1, MODE><<<grid, 64, 0, s>>>(a);   \
-    return;                                                                                      \
-  }
-    if constexpr (MODE == SHAPED) { BCG_EXACT1_SHAPED(BCG_X) } else { BCG_EXACT1_KEEP(BCG_X) }
-#undef BCG_X
-  }
+void launch_decode_mode(const AttnArgs& a, dim3 grid, hipStream_t s) {
   if (a.dim <= 64 && a.vdim <= 128) decode_mfma_kernel<T, 4, 8, 1, false, false, 1, 0, 1, MODE><<<grid, 64, 0, s>>>(a);
   else if (a.dim <= 256 && a.vdim <= 256) decode_mfma_kernel<T, 16, 16, 1, false, false, 1, 0, 1, MODE><<<grid, 64, 0, s>>>(a);
   else decode_mfma_kernel<T, 32, 32, 1, false, false, 1, 0, 1, MODE><<<grid, 64, 0, s>>>(a);
@@ -868,40 +1128,65 @@ int launch_prefill(const AttnArgs& a, int n_tiles, int tile_rows, hipStream_t s)
 }
 
 template <typename T>
+void launch_merge(const AttnArgs& a, int n_items, hipStream_t s) {
+  if (a.vdim <= 128) decode_merge_kernel<T, 2><<<dim3(a.H, n_items), 64, 0, s>>>(a);
+  else if (a.vdim <= 256) decode_merge_kernel<T, 4><<<dim3(a.H, n_items), 64, 0, s>>>(a);
+  else decode_merge_kernel<T, 8><<<dim3(a.H, n_items), 64, 0, s>>>(a);
+}
+
+// Pairs of a decode step in a.n_splits parts each (decode_pair_kernel); -2: not these heads.  n_items 0: only says whether.
+int launch_pairs(const AttnArgs& a, int n_items, hipStream_t s) {
+  const dim3 grid(a.G * ((a.H / a.G + 15) / 16) * a.n_splits, n_items);
+  const bool many = static_cast<int64_t>(grid.x) * n_items > 1024;   // (see decode_pair_kernel)
+  auto run = [&](auto kernel4, auto kernel2) {
+    if (n_items == 0) return 0;
+    if (many) kernel2<<<grid, 128, 0, s>>>(a);
+    else kernel4<<<grid, 256, 0, s>>>(a);
+    if (a.n_splits > 1) launch_merge<bf16_t>(a, n_items, s);
+    return BCG_CHECK_LAUNCH();
+  };
+#define BCG_X(KC_, VT_, KT_, OCC_)                                                               \
+  if constexpr ((KC_) % 2 == 0) if (a.dim == 16 * KC_ && a.vdim == 16 * VT_) return run(decode_pair_kernel<KC_, VT_, 1, BCG_MODE, 4>, decode_pair_kernel<KC_, VT_, 1, BCG_MODE, 2>);
+  if (a.maps == 1 && (a.softcap > 0.f || a.slopes != nullptr)) {
+#define BCG_MODE SHAPED
+    BCG_EXACT1_SHAPED(BCG_X)
+#undef BCG_MODE
+    return -2;
+  }
+  if (a.maps == 1 && a.keep > 0) {
+#define BCG_MODE KEEP
+    BCG_EXACT1_KEEP(BCG_X)
+#undef BCG_MODE
+    return -2;
+  }
+  if (a.maps == 1) {
+#define BCG_MODE PLAIN
+    BCG_EXACT1_PLAIN(BCG_X)
+#undef BCG_MODE
+    return -2;
+  }
+#undef BCG_X
+#define BCG_X(KC_, VT_) if (a.dim == 16 * KC_ && a.vdim == 16 * VT_) return run(decode_pair_kernel<KC_, VT_, 2, PLAIN, 4>, decode_pair_kernel<KC_, VT_, 2, PLAIN, 2>);
+  BCG_X(4, 8) BCG_X(3, 6) BCG_X(2, 4) BCG_X(4, 4) BCG_X(2, 2)
+#undef BCG_X
+  return -2;
+}
+
+template <typename T>
 int launch_decode(const AttnArgs& a, int n_items, hipStream_t s) {
   const int per = a.H / a.G;
   dim3 grid(a.G * ((per + 15) / 16), a.n_splits, n_items);
   const bool full = a.dim % 16 == 0 && a.vdim % 16 == 0 && a.vec_k && a.vec_v;
   const bool shaped = a.softcap > 0.f || a.slopes != nullptr;
   bool done = shaped || a.keep > 0;
-  if (shaped) launch_decode_mode<T, SHAPED>(a, grid, full, s);
-  else if (done) launch_decode_mode<T, KEEP>(a, grid, full, s);
-  if constexpr (sizeof(T) == 2) if (!done && full && a.maps == 1 && a.swz && a.BS == 16) {   // one-map heads, exact shapes
-#define BCG_X(KC_, VT_, KT_, OCC_)                                                               \
-  if (!done && a.dim == 16 * KC_ && a.vdim == 16 * VT_) {                                        \
-    done = true;                                                                                 \
-    decode_mfma_kernel<T, KC_, VT_, KT_, true, true, OCC_, 1, 1><<<grid, 64, 0, s>>>(a);         \
-  }
-    BCG_EXACT1_PLAIN(BCG_X)
-    if (!done && a.dim == 512 && a.vdim == 512) {
-      done = true;
-      decode_mfma_kernel<T, 32, 32, 1, true, true, 1, 1, 1><<<grid, 64, 0, s>>>(a);
-    }
-#undef BCG_X
+  if (shaped) launch_decode_mode<T, SHAPED>(a, grid, s);
+  else if (done) launch_decode_mode<T, KEEP>(a, grid, s);
+  if constexpr (sizeof(T) == 2) if (!done && full && a.maps == 1 && a.swz && a.BS == 16 && a.dim == 512 && a.vdim == 512) {
+    done = true;
+    decode_mfma_kernel<T, 32, 32, 1, true, true, 1, 1, 1><<<grid, 64, 0, s>>>(a);
   }
   if constexpr (sizeof(T) == 2) if (!done && a.dim <= 64 && a.vdim <= 128) {
     done = true;
-    const bool exact = full && a.maps == 2 && a.swz && a.BS == 16;
-    bool hit = false;
-#define BCG_EXACT(KC_, VT_)                                                                      \
-  if (!hit && exact && a.dim == 16 * KC_ && a.vdim == 16 * VT_) {                                \
-    hit = true;                                                                                  \
-    decode_mfma_kernel<T, KC_, VT_, 2, true, true, 2, 2><<<grid, 64, 0, s>>>(a);                 \
-  }
-    BCG_EXACT(4, 8) BCG_EXACT(3, 6) BCG_EXACT(2, 4) BCG_EXACT(4, 4) BCG_EXACT(2, 2)
-#undef BCG_EXACT
-    if (hit) {
-    } else
     if (full) decode_mfma_kernel<T, 4, 8, 2, true, true, 2><<<grid, 64, 0, s>>>(a);
     else decode_mfma_kernel<T, 4, 8, 2, true, false, 2><<<grid, 64, 0, s>>>(a);
   }
@@ -918,9 +1203,7 @@ int launch_decode(const AttnArgs& a, int n_items, hipStream_t s) {
   } else {
     decode_mfma_kernel<T, 32, 16, 1, false, false, 1, 0, 1><<<grid, 64, 0, s>>>(a);
   }
-  if (a.vdim <= 128) decode_merge_kernel<T, 2><<<dim3(a.H, n_items), 64, 0, s>>>(a);
-  else if (a.vdim <= 256) decode_merge_kernel<T, 4><<<dim3(a.H, n_items), 64, 0, s>>>(a);
-  else decode_merge_kernel<T, 8><<<dim3(a.H, n_items), 64, 0, s>>>(a);
+  launch_merge<T>(a, n_items, s);
   return BCG_CHECK_LAUNCH();
 }
 
@@ -929,7 +1212,8 @@ int launch_decode(const AttnArgs& a, int n_items, hipStream_t s) {
 BCG_API int bcg_multimap_split_keys() { return SPLIT_KEYS; }
 
 // mode 0: prefill tiles (work = tiles [n_work, 3]); mode 1: single-token items (work = [n_work, 2]
-// {row, sequence}, or null: item i is row i of sequence i).
+// {row, sequence}, or null: item i is row i of sequence i), n_splits the most splits of a row; mode 2: the same where bcg_multimap_pairs says
+// so, every row in n_splits parts (ws is read and written if there are two or more).
 BCG_API int bcg_multimap_attention(int mode, const void* q, const void* k_cache, const void* v_cache,
                                    const void* block_tables, int max_blocks, const void* q_start, const void* seq_lens,
                                    const void* work, int n_work, void* out, void* ws, int n_splits, int H, int G, int maps,
@@ -955,7 +1239,21 @@ BCG_API int bcg_multimap_attention(int mode, const void* q, const void* k_cache,
   a.window = window; a.keep = keep; a.chunk = chunk; a.sink = static_cast<const float*>(sink);
   a.softcap = softcap; a.slopes = static_cast<const float*>(slopes);
   hipStream_t s = static_cast<hipStream_t>(stream);
+  a.parts = mode == 2;
+  if (mode == 2) {
+    if (is_f32 || BS != 16 || !a.swz || n_splits < 1 || n_splits > 64 || H > 65535 || n_work > 65535 || max_blocks < 1 ||
+        ((reinterpret_cast<uintptr_t>(k_cache) | reinterpret_cast<uintptr_t>(v_cache)) & 15) || (n_splits > 1 && !ws))
+      return -2;
+    return launch_pairs(a, n_work, s);
+  }
   if (mode == 0) return is_f32 ? launch_prefill<float>(a, n_work, tile_rows, s) : launch_prefill<bf16_t>(a, n_work, tile_rows, s);
   if (n_splits < 1 || H > 65535 || n_splits > 65535 || n_work > 65535) return -2;
   return is_f32 ? launch_decode<float>(a, n_work, s) : launch_decode<bf16_t>(a, n_work, s);
+}
+
+// Whether mode 2 takes the decode steps of these heads (bf16, 16-token pages, caches on 16 bytes).
+BCG_API int bcg_multimap_pairs(int maps, int dim, int vdim, int shaped, int keep) {
+  AttnArgs a{};
+  a.maps = maps, a.dim = dim, a.vdim = vdim, a.softcap = shaped ? 1.f : 0.f, a.keep = keep, a.H = a.G = a.n_splits = 1;
+  return (maps == 1 || maps == 2) && launch_pairs(a, 0, nullptr) == 0;
 }

@@ -1,0 +1,95 @@
+"""Single-token rows of exact head sizes by a workgroup per (row, KV head) pair (csrc/kernels/seqmix_attention.hip, decode_pair_kernel) against the
+float32 reference.  GPU only.
+
+bf16 operands, fp32 sums; probabilities and outputs are rounded to bf16 (2^-9 each) before and after sums over keys of both signs: an output is off by
+2^-8 of its head's size a few times over at most, as in test_seqmix_kernels_gpu.py."""
+import pytest
+import torch
+
+from byzantine_consensus_llm_agents_amd.models.transformer import AttnMeta
+from byzantine_consensus_llm_agents_amd.ops import reference as ref
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+# contexts at the edges of pages (16), chunks (32) and turns of 2 and 4 waves (64, 128)
+LENS = [1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 127, 128, 129, 300, 513, 1025]
+KINDS = {"plain": {}, "window": dict(window=37), "long window": dict(window=300), "chunk": dict(chunk=50), "keep": dict(window=40, keep=5), "keep far": dict(window=70, keep=140),
+         "sink": dict(sink=True, window=100), "shaped": dict(softcap=3.0, slopes=True)}
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from byzantine_consensus_llm_agents_amd.ops import get_ops
+    return get_ops("hip")
+
+
+def _case(H, G, maps, dim, vdim, kind, rows, wide, eps, seed):
+    lens = (LENS * rows)[:rows]
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    per = [-(-n // 16) for n in lens]
+    blocks = sum(per) + 1
+    ids = torch.randperm(blocks - 1, generator=torch.Generator().manual_seed(seed)) + 1
+    bt, at = torch.full((rows, max(per) + wide), 1 << 28, dtype=torch.int32), 0   # (no pages behind the contexts)
+    for b, n in enumerate(per):
+        bt[b, :n] = ids[at:at + n].to(torch.int32)
+        at += n
+    k = torch.randn(blocks, G, 16, maps * dim, device=DEV, generator=g).to(torch.bfloat16)
+    v = torch.randn(blocks, G, vdim, 16, device=DEV, generator=g).to(torch.bfloat16)
+    kw = dict(KINDS[kind])
+    if kw.get("sink"):
+        kw["sink"] = torch.randn(H, device=DEV, generator=g)
+    if kw.get("slopes"):
+        kw["slopes"] = torch.rand(H, device=DEV, generator=g) * 0.1
+    q = torch.randn(rows, H, maps * dim, device=DEV, generator=g).to(torch.bfloat16)
+    lens = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    return q, k, v, bt.to(DEV), lens, (dim ** -0.5, maps, 0.35, eps, 0.4, vdim), kw
+
+
+# wide: pages that the table has room for besides (enough of them: several parts)
+@pytest.mark.parametrize("H,G,maps,dim,vdim,kind,rows,wide,eps", [
+    (32, 8, 2, 64, 128, "plain", 16, 0, 1e-5), (16, 4, 2, 64, 128, "plain", 3, 900, 1e-5), (16, 16, 2, 32, 32, "plain", 80, 0, 1e-5), (6, 2, 2, 48, 96, "plain", 16, 0, -1.0),
+    (40, 1, 1, 192, 128, "window", 16, 0, -1.0), (17, 1, 1, 192, 128, "long window", 2, 900, -1.0), (4, 2, 1, 96, 64, "plain", 16, 0, 1e-5),
+    (8, 4, 1, 128, 128, "keep", 16, 0, -1.0), (8, 4, 1, 64, 64, "keep far", 16, 900, -1.0), (64, 64, 1, 128, 128, "keep", 20, 0, 1e-5), (4, 2, 1, 64, 128, "chunk", 16, 0, 1e-5),
+    (4, 2, 1, 128, 128, "sink", 16, 0, -1.0), (4, 1, 1, 128, 128, "sink", 2, 4000, -1.0), (4, 2, 1, 192, 192, "shaped", 16, 0, -1.0), (4, 2, 1, 256, 256, "plain", 16, 0, -1.0),
+    (4, 2, 1, 256, 256, "shaped", 600, 0, -1.0), (16, 16, 1, 192, 128, "plain", 70, 0, -1.0)])
+def test_against_reference(ops, H, G, maps, dim, vdim, kind, rows, wide, eps):
+    q, k, v, bt, lens, args, kw = _case(H, G, maps, dim, vdim, kind, rows, wide, eps, seed=dim + rows)
+    assert ops.library.bcg_multimap_pairs(maps, dim, vdim, int(kind == "shaped"), kw.get("keep", 0))
+    kp, vp = ops.kv_from_logical(k, v)
+    got = ops.multimap_attention(q, kp, vp, AttnMeta(positions=None, slots=None, block_tables=bt, seq_lens=lens, decode=True), *args, **kw)
+    want = ref.multimap_attention(q, k, v, bt, torch.arange(rows + 1, dtype=torch.int32, device=DEV), lens, *args, **kw)
+    torch.testing.assert_close(got.float(), want.float(), atol=3e-2, rtol=3e-2)
+
+
+def test_single_rows_and_graph_replays(ops):
+    """Rows of a packed step in an order of their own, several parts, replayed."""
+    q, k, v, bt, lens, args, _ = _case(16, 4, 2, 64, 128, "plain", 6, 1500, 1e-5, seed=9)
+    kp, vp = ops.kv_from_logical(k, v)
+    order = torch.tensor([4, 0, 5, 2], device=DEV)
+    single = torch.stack([order, order.flip(0)], 1).to(torch.int32).contiguous()   # row order[i] is sequence order[-1 - i]'s
+    meta = AttnMeta(positions=None, slots=None, block_tables=bt, seq_lens=lens, q_start=torch.zeros(7, dtype=torch.int32, device=DEV), decode=False, tile_rows=64,
+                    tiles=torch.zeros(0, 3, dtype=torch.int32, device=DEV), single=single)
+    seqs = order.flip(0)
+    want = ref.multimap_attention(q[order], k, v, bt[seqs], torch.arange(5, dtype=torch.int32, device=DEV), lens[seqs], *args)
+    ops.multimap_attention(q, kp, vp, meta, *args)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = ops.multimap_attention(q, kp, vp, meta, *args)
+    for _ in range(3):
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        torch.testing.assert_close(out[order].float(), want.float(), atol=3e-2, rtol=3e-2)
+
+
+def test_caches_off_16_bytes(ops):
+    """Views that begin 8 bytes into their memory take the splits."""
+    q, k, v, bt, lens, args, _ = _case(8, 2, 2, 64, 128, "plain", 5, 0, 1e-5, seed=2)
+    moved = []
+    for t in ops.kv_from_logical(k, v):
+        room = torch.empty(t.numel() + 4, dtype=t.dtype, device=DEV)[4:].view(t.shape)
+        room.copy_(t)
+        moved.append(room)
+    got = ops.multimap_attention(q, *moved, AttnMeta(positions=None, slots=None, block_tables=bt, seq_lens=lens, decode=True), *args)
+    want = ref.multimap_attention(q, k, v, bt, torch.arange(6, dtype=torch.int32, device=DEV), lens, *args)
+    torch.testing.assert_close(got.float(), want.float(), atol=3e-2, rtol=3e-2)
