@@ -31,6 +31,34 @@ template <> struct Elem<float> {
   }
 };
 
+// Grids of the recurrences over segments: heads, segments, column blocks.  A workgroup's XCD is its index modulo 8: with the segments first, 8 of them
+// put all heads of one on one XCD, and the launch ends with the longest (8 segments of 700 to 1300 tokens took as long as 8 of 1300).  The
+// segments come longest first where workgroups wait for a place; where all of them run at once (`at_once`) every CU gets long and short ones instead: the heads of an
+// XCD begin at different segments, every other column block walks them backwards.  (Past 64 segments in the order of the batch.)
+// us, segments first and this: decays in chunks, 64 heads of 128 x 128, 8 segments of 700 to 1300 tokens 657, 560 (8 of 1000: 500), 24 of 210 to 390
+// 580, 470; delta rule, 32 heads, the same 828, 760 (8 of 1000: 685) and 668, 612.
+inline dim3 segment_grid(int H, int B, int Z) { return B <= 65535 ? dim3(H, B, Z) : dim3(B, H, Z); }   // (the second dimension's limit)
+__device__ __forceinline__ int segment_by_length(const int* q_start, int B, int at, bool back) {
+  if (back) at = B - 1 - at;
+  if (B > 64) return at;
+  const int lane = threadIdx.x & 63, len = lane < B ? q_start[lane + 1] - q_start[lane] : -1;
+  int rank = 0;
+  for (int i = 0; i < B; ++i) {
+    const int other = __builtin_amdgcn_readlane(len, i);
+    rank += other > len || (other == len && i < lane);
+  }
+  return __builtin_amdgcn_readfirstlane(__ffsll(__ballot(lane < B && rank == at)) - 1);
+}
+__device__ __forceinline__ void segment_of(const int* q_start, int B, bool at_once, int& b, int& h) {
+  if (B <= 65535) {
+    b = segment_by_length(q_start, B, at_once ? (blockIdx.y + (blockIdx.x >> 3)) % B : blockIdx.y, at_once && (blockIdx.z & 1));
+    h = blockIdx.x;
+  } else {
+    b = blockIdx.x;
+    h = blockIdx.y;
+  }
+}
+
 // C[16 x 16] += A[16 x 16] B[16 x 16].  Lane l holds A[m = l % 16][k = 4 (l / 16) + j],
 // B[k = 4 (l / 16) + j][n = l % 16] (j = 0..3) and C[m = 4 (l / 16) + i][n = l % 16].
 // bf16: one v_mfma_f32_16x16x16_bf16.  fp32: four v_mfma_f32_16x16x4_f32 (true fp32), step j

@@ -132,7 +132,9 @@ __global__ __launch_bounds__(NTH, DC <= 8 ? 2 : 1) void chunk_kernel(ChunkArgs a
   __shared__ double pre[CT], post[CT], whole[4];   // decay from a block's start to the token; that behind the token, times b; over a block
   __shared__ int wild;   // some value was infinite or NaN: it must not reach earlier queries as 0 x value
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 15, grp = lane >> 4;
-  const int b = blockIdx.x, h = blockIdx.y, v0 = blockIdx.z * VT;
+  int b = blockIdx.x, h = blockIdx.y;
+  if constexpr (VT == 64) segment_of(a.q_start, a.B, false, b, h);   // (fewer columns: fewer workgroups than places, where the order costs 2 to 3 us)
+  const int v0 = blockIdx.z * VT;
   const int t0 = a.q_start[b], t1 = a.q_start[b + 1], sr = a.state_rows[b];
   if (t1 - t0 < a.min_len || sr < 0 || sr >= a.n_rows) return;
   const int gq = h / (a.H / a.Gq), dim = a.dim, vdim = a.vdim;
@@ -398,7 +400,7 @@ int launch_chunks(const ChunkArgs& a, int n_chunks, hipStream_t s) {
   // (96 workgroups of 64 columns -> 384 of 16: 140 us -> 75, 3 segments of 700).  At one per CU 32 columns win (64 segments of
   // 200, 4 heads of 64 x 64: 47 us, 64 columns 50), past it their second round loses (100 segments: 74 us, 62).
   const int64_t wide = static_cast<int64_t>(a.B) * a.H * ((a.vdim + 63) / 64);
-  if (wide > 256) chunk_kernel<T, DC, 64, FULL><<<dim3(a.B, a.H, (a.vdim + 63) / 64), NTH, 0, s>>>(a);
+  if (wide > 256) chunk_kernel<T, DC, 64, FULL><<<segment_grid(a.H, a.B, (a.vdim + 63) / 64), NTH, 0, s>>>(a);
   else if (wide == 256) chunk_kernel<T, DC, 32, FULL><<<dim3(a.B, a.H, (a.vdim + 31) / 32), NTH, 0, s>>>(a);
   else chunk_kernel<T, DC, 16, FULL><<<dim3(a.B, a.H, (a.vdim + 15) / 16), NTH, 0, s>>>(a);
   return BCG_CHECK_LAUNCH();

@@ -712,7 +712,7 @@ struct ScanArgs {
   const int* positions; const int* q_start; const int* state_rows;
   float* state;                                     // [n_rows, H, dim, vdim]
   float* out;                                       // [T, H, vdim]
-  int n_rows, H, Gq, dim, vdim, gd, g_token;        // g_token: elements of g per token, H gd or 0
+  int n_rows, B, H, Gq, dim, vdim, gd, g_token;     // g_token: elements of g per token, H gd or 0
   int skip_len;                                     // > 0: segments of at least this length are another kernel's
 };
 
@@ -894,7 +894,9 @@ __global__ __launch_bounds__(64 * SCAN_WAVES, 2) void delta_scan_kernel(ScanArgs
   __shared__ __attribute__((aligned(16))) float vals[2][CT][NC];
   __shared__ float gb[2][CT][2];
   const int tid = threadIdx.x, lane = tid & 63, rg = lane & 7;
-  const int b = blockIdx.x, h = blockIdx.y, j0 = blockIdx.z * NC, jl = (tid >> 6) * 8 + (lane >> 3), j = j0 + jl;
+  int b, h;
+  segment_of(a.q_start, a.B, true, b, h);
+  const int j0 = blockIdx.z * NC, jl = (tid >> 6) * 8 + (lane >> 3), j = j0 + jl;
   const int t0 = a.q_start[b], t1 = a.q_start[b + 1];
   const int sr = a.state_rows[b];
   if (t1 <= t0 || sr < 0 || sr >= a.n_rows || (a.skip_len > 0 && t1 - t0 >= a.skip_len)) return;
@@ -1124,10 +1126,11 @@ int launch_scan(const ScanArgs& a, int tokens, int B, hipStream_t s) {
   if constexpr (DELTA) {
     const int64_t groups = static_cast<int64_t>(grid.x) * grid.y * grid.z;
     if (a.gd == 1 && tokens / 4 >= B && (a.dim <= 128 || groups <= 768 || (sizeof(T) == 2 && tokens / 16 < B))) {
-      if (a.dim <= 32) delta_scan_kernel<T, 32><<<grid, 64 * SCAN_WAVES, 0, s>>>(a);
-      else if (a.dim <= 64) delta_scan_kernel<T, 64><<<grid, 64 * SCAN_WAVES, 0, s>>>(a);
-      else if (a.dim <= 128) delta_scan_kernel<T, 128><<<grid, 64 * SCAN_WAVES, 0, s>>>(a);
-      else delta_scan_kernel<T, 256><<<grid, 64 * SCAN_WAVES, 0, s>>>(a);
+      const dim3 heads_first = segment_grid(a.H, B, grid.z);
+      if (a.dim <= 32) delta_scan_kernel<T, 32><<<heads_first, 64 * SCAN_WAVES, 0, s>>>(a);
+      else if (a.dim <= 64) delta_scan_kernel<T, 64><<<heads_first, 64 * SCAN_WAVES, 0, s>>>(a);
+      else if (a.dim <= 128) delta_scan_kernel<T, 128><<<heads_first, 64 * SCAN_WAVES, 0, s>>>(a);
+      else delta_scan_kernel<T, 256><<<heads_first, 64 * SCAN_WAVES, 0, s>>>(a);
       return BCG_CHECK_LAUNCH();
     }
   }
@@ -1333,7 +1336,7 @@ BCG_API int bcg_gated_state_scan(const void* q32, const void* k32, const void* g
   a.positions = static_cast<const int*>(positions); a.q_start = static_cast<const int*>(q_start);
   a.state_rows = static_cast<const int*>(state_rows);
   a.state = static_cast<float*>(state); a.out = static_cast<float*>(out);
-  a.n_rows = n_rows; a.H = H; a.Gq = Gq; a.dim = dim; a.vdim = vdim; a.gd = gd; a.g_token = g_const ? 0 : H * gd;
+  a.n_rows = n_rows; a.B = B; a.H = H; a.Gq = Gq; a.dim = dim; a.vdim = vdim; a.gd = gd; a.g_token = g_const ? 0 : H * gd;
   a.skip_len = skip_len;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (delta) return is_f32 ? launch_scan<float, true>(a, T_, B, s) : launch_scan<bf16_t, true>(a, T_, B, s);
