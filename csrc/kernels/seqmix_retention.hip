@@ -25,14 +25,17 @@
 //   V^T K         [value column x key feature], keys weighted by W b: the state's update
 // The walk is a serial chain, so its operands are fetched a chunk ahead into the registers that the phase before has
 // just used up (no wave needs another wave's keys or queries: they do not pass LDS), and VT shrinks where the launch would leave CUs
-// idle.  What bounds it: the fp32 matrix rate (32 cycles per 16 x 16 x 4) where all CUs are busy, else the chain.
-// Measured, both launches: 3 segments of 700 tokens, 8 heads, 128 x 256 states: 91 us (keys, scores and 64-column
-// workgroups in one kernel, 96 workgroups: 202); 8 segments of 1000, 128 heads sharing keys, 128 x 64 states: 494 to 524 us (token
-// by token: 1552), of which the matrix rate is 250 (in a whole step, 64 heads of 128 x 128: 690); 64 segments of 16: 149 (220).
+// idle.  What bounds it: the fp32 matrix rate (32 cycles per 16 x 16 x 4) where all CUs are busy, else the chain; of a chunk's 9500 cycles
+// in workgroups of 16 columns 2900 are the state's update, 2300 the scores' products, 1500 the old state's, 1400 staging.  A chunk's
+// decays are made once, by two waves, and read by all; no load stands behind a branch.  Measured, both launches, before and now:
+// 3 segments of 700 tokens, 8 heads, 128 x 256 states: 91 -> 82 us; 64 heads of 128 x 128 that share keys: 8 segments of 1000 502 -> 465 (token by
+// token: 1552; the matrix rate alone: 250), 8 segments of 600 to 1400 540 -> 510, 24 of 300 469 -> 441, one of 2000 207 -> 181.  Adding up the states
+// of all chunks at once, carrying them along and reading them in three more launches: 73 us in the first case, up to twice as long in the others.
 // Rounding, against float64 (relative rms, token by token -> here): decays about 0.5: 8.4e-8 -> 7.4e-8, 0.9: 1.1e-7 -> 1.0e-7, 0.99:
 // 2.5e-7 -> 1.2e-7, 0.999: 4.6e-7 -> 1.5e-7.  That takes the scores in double (parallel, so nearly free), decay products in
 // double, and short chains in the fp32 accumulators (one chain over all features and keys: 1.5e-7 at decays about 0.5).
 #include <algorithm>
+#include <type_traits>
 
 #include "seqmix_common.h"
 
@@ -130,6 +133,7 @@ __global__ __launch_bounds__(NTH, DC <= 8 ? 2 : 1) void chunk_kernel(ChunkArgs a
   __shared__ __attribute__((aligned(16))) T Vs[VT * LDV];       // [value column][token]
   __shared__ __attribute__((aligned(16))) float gs[CT], bs[CT];
   __shared__ double pre[CT], post[CT], whole[4];   // decay from a block's start to the token; that behind the token, times b; over a block
+  __shared__ __attribute__((aligned(16))) float front[CT], tail[CT];   // decay from the chunk's start to the token; that to its end behind the token, times b
   __shared__ int wild;   // some value was infinite or NaN: it must not reach earlier queries as 0 x value
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 15, grp = lane >> 4;
   int b = blockIdx.x, h = blockIdx.y;
@@ -154,7 +158,8 @@ __global__ __launch_bounds__(NTH, DC <= 8 ? 2 : 1) void chunk_kernel(ChunkArgs a
   const bool owner = 16 * ND * wave < dim;   // (wave-uniform) the wave has features
   const int place = 16 * wave + col;         // this lane's query in a chunk
 
-  // ---- loads, one chunk ahead; rows past the segment repeat its last one and are masked where they are used ----
+  // ---- loads, one chunk ahead; rows past the segment repeat its last one and are masked where they are used.  No branch around a load (the last
+  // chunk loads itself again): behind one hipcc waits for every load in flight, the youngest too ----
   f32x4 qf[DC];
   float kf[4][4][ND];
   f32x4 rf[4];
@@ -165,11 +170,17 @@ __global__ __launch_bounds__(NTH, DC <= 8 ? 2 : 1) void chunk_kernel(ChunkArgs a
   const uint32_t v_src = min(v_col, vdim - 1 - v0);   // (columns past the state repeat its last one and are not stored)
   // (a chunk's rows start at a uniform address; a lane's place in the chunk is a 32-bit offset)
   const uint32_t row = static_cast<uint32_t>(a.Gq) * dim, v_row = static_cast<uint32_t>(a.v_stride);
+  auto at = [](const auto* base, uint32_t o) {   // (32 bits of bytes: one register beside a uniform base)
+    typedef std::remove_pointer_t<decltype(base)> E;
+    return reinterpret_cast<E*>(reinterpret_cast<const char*>(base) + static_cast<uint32_t>(o * sizeof(E)));
+  };
+  const float* betas = a.beta != nullptr ? a.beta : a.g;
+  const size_t beta_token = a.beta != nullptr ? a.H : a.g_token;
   auto load_q = [&](int first) {
     const float* base = a.q + static_cast<size_t>(first) * row + gq * dim;
     const uint32_t o = min(place, t1 - 1 - first) * row + 4 * grp;
 #pragma unroll
-    for (int c = 0; c < DC; ++c) qf[c] = load4f<FULL>(base + (o + 16 * c), dim - 16 * c - 4 * grp, a.vec);
+    for (int c = 0; c < DC; ++c) qf[c] = load4f<FULL>(at(base, o + 16 * c), dim - 16 * c - 4 * grp, a.vec);
   };
   auto load_k = [&](int first, int tt) {
     const float* base = a.k + static_cast<size_t>(first) * row + gq * dim;
@@ -179,14 +190,14 @@ __global__ __launch_bounds__(NTH, DC <= 8 ? 2 : 1) void chunk_kernel(ChunkArgs a
       if constexpr (ND > 1) {
         typedef float fv __attribute__((ext_vector_type(ND)));
         if (vec_k) {
-          const fv x = *reinterpret_cast<const fv*>(base + o);
+          const fv x = *reinterpret_cast<const fv*>(at(base, o));
 #pragma unroll
           for (int m = 0; m < ND; ++m) kf[tt][j][m] = x[m];
           continue;
         }
       }
 #pragma unroll
-      for (int m = 0; m < ND; ++m) kf[tt][j][m] = OWNERS || d0 + m < dim ? base[o + m] : 0.f;
+      for (int m = 0; m < ND; ++m) kf[tt][j][m] = OWNERS || d0 + m < dim ? *at(base, o + m) : 0.f;
     }
   };
   auto load_r = [&](int first, int id) {
@@ -194,7 +205,7 @@ __global__ __launch_bounds__(NTH, DC <= 8 ? 2 : 1) void chunk_kernel(ChunkArgs a
     const uint32_t o = place * CT + 4 * grp;
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt)
-      if (kt <= wave && first + 16 * wave < t1) rf[kt] = *reinterpret_cast<const f32x4*>(base + (o + 16 * kt));
+      rf[kt] = *reinterpret_cast<const f32x4*>(at(base, o + 16 * min(kt, wave)));
   };
   auto load_v = [&](int first) {
     const T* base = vbase + static_cast<size_t>(first) * a.v_stride;
@@ -202,15 +213,12 @@ __global__ __launch_bounds__(NTH, DC <= 8 ? 2 : 1) void chunk_kernel(ChunkArgs a
     for (int p = 0; p < NU; ++p)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const T x = base[min(v_tok + p * (4 * NTH / VT) + j, t1 - 1 - first) * v_row + v_src];
+        const T x = *at(base, min(v_tok + p * (4 * NTH / VT) + j, t1 - 1 - first) * v_row + v_src);
         if constexpr (sizeof(T) == 2) vf[p][j] = x; else vf[p][j] = __float_as_uint(x);
       }
-    gf = 1.0f;
-    bf = 0.0f;
-    if (wave == 0 && first + lane < t1) {
-      gf = a.g[static_cast<size_t>(first + lane) * a.g_token + h];
-      bf = a.beta != nullptr ? a.beta[static_cast<size_t>(first + lane) * a.H + h] : 1.0f;
-    }
+    const size_t t = min(first + lane, t1 - 1);
+    gf = a.g[t * a.g_token + h];
+    bf = betas[t * beta_token + h];
   };
   auto value_frag = [&](int u, int tok) {   // V^T[value column 16 u + col][tokens tok .. tok + 3] as fp32
     const F f = *reinterpret_cast<const F*>(&Vs[(16 * u + col) * LDV + tok]);
@@ -231,7 +239,7 @@ __global__ __launch_bounds__(NTH, DC <= 8 ? 2 : 1) void chunk_kernel(ChunkArgs a
   for (int tt = 0; tt < 4; ++tt) load_k(t0, tt);
   for (int first = t0; first < t1; first += CT, ++id) {
     const int n = min(CT, t1 - first);
-    const bool more = first + CT < t1;
+    const int ahead = first + CT < t1 ? first + CT : first, id_ahead = first + CT < t1 ? id + 1 : id;
     // ---- values, state and decays to LDS ----
 #pragma unroll
     for (int p = 0; p < NU; ++p) {
@@ -255,40 +263,64 @@ __global__ __launch_bounds__(NTH, DC <= 8 ? 2 : 1) void chunk_kernel(ChunkArgs a
           for (int m = 0; m < ND; ++m)
             if (DC % 4 == 0 || d0 + m < 16 * DC) Ss[(16 * u + 4 * grp + i) * LDK + d0 + m] = S[m][u][i];
     }
-    if (wave == 0) {   // lane = token
+    if (wave <= 1) {   // lane = token
+      const bool in = first + lane < t1;
+      gf = in ? gf : 1.0f;
+      bf = in ? (a.beta != nullptr ? bf : 1.0f) : 0.0f;
       const double p = row_mul<0x118>(row_mul<0x114>(row_mul<0x112>(row_mul<0x111>(static_cast<double>(gf)))));   // row_shr 1, 2, 4, 8
-      const double s = row_mul<0x108>(row_mul<0x104>(row_mul<0x102>(row_mul<0x101>(static_cast<double>(gf)))));   // row_shl 1, 2, 4, 8
-      gs[lane] = gf;
-      bs[lane] = bf;
-      pre[lane] = p;
-      post[lane] = row_move<0x101>(s) * bf;
-      if (col == 15) whole[grp] = p;
+      auto block = [&](int k) {
+        return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(p), 16 * k + 15), __builtin_amdgcn_readlane(__double2loint(p), 16 * k + 15));
+      };
+      if (wave == 0) {
+        const double w0 = block(0), w1 = block(1), w2 = block(2);
+        gs[lane] = gf;
+        bs[lane] = bf;
+        pre[lane] = p;
+        front[lane] = p * (grp == 0 ? 1.0 : grp == 1 ? w0 : grp == 2 ? w0 * w1 : w0 * w1 * w2);
+        if (col == 15) whole[grp] = p;
+      } else {
+        const double s = row_mul<0x108>(row_mul<0x104>(row_mul<0x102>(row_mul<0x101>(static_cast<double>(gf)))));   // row_shl 1, 2, 4, 8
+        const double after = row_move<0x101>(s) * bf, w1 = block(1), w2 = block(2), w3 = block(3);
+        post[lane] = after;
+        tail[lane] = after * (grp == 3 ? 1.0 : grp == 2 ? w3 : grp == 1 ? w2 * w3 : w1 * w2 * w3);
+      }
     }
     __syncthreads();
-    if (more) load_v(first + CT);
+    load_v(ahead);
     const double wh[4] = {whole[0], whole[1], whole[2], whole[3]};
+    // few columns: the walk's length counts and not its products: nothing of a chunk stands behind a branch, so one step's reads and weights
+    // fly under the products of the one before (blocks of keys that a wave does not see have weights of zero)
+    constexpr bool FEW = VT == 16;
     f32x4 o[NU];
 #pragma unroll
     for (int u = 0; u < NU; ++u) o[u] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (16 * wave < n) {
+    if (FEW || 16 * wave < n) {
+      const double here = pre[place];
 #pragma unroll
       for (int kt = 0; kt < 3; ++kt) {   // the blocks before the queries' own
-        if (kt < wave) {   // (wave-uniform)
-          double g = pre[place];
-          for (int k = kt + 1; k < wave; ++k) g *= wh[k];
+        if (FEW || kt < wave) {   // (wave-uniform)
+          double g = here;
+#pragma unroll
+          for (int k = 1; k < 3; ++k) g *= k > kt && k < wave ? wh[k] : 1.0;
           f32x4 s;
 #pragma unroll
-          for (int i = 0; i < 4; ++i) s[i] = rf[kt][i] * static_cast<float>(post[16 * kt + 4 * grp + i] * g);
+          for (int i = 0; i < 4; ++i) {
+            s[i] = rf[kt][i] * static_cast<float>(post[16 * kt + 4 * grp + i] * g);
+            if (FEW && kt >= wave) s[i] = 0.f;
+          }
 #pragma unroll
-          for (int u = 0; u < NU; ++u) o[u] += mma16(value_frag(u, 16 * kt + 4 * grp), s, f32x4{0.f, 0.f, 0.f, 0.f});
+          for (int u = 0; u < NU; ++u) {
+            f32x4 x = value_frag(u, 16 * kt + 4 * grp);
+            if (FEW && kt >= wave) x = f32x4{0.f, 0.f, 0.f, 0.f};   // (a later value may be infinite)
+            o[u] += mma16(x, s, f32x4{0.f, 0.f, 0.f, 0.f});
+          }
         }
       }
       // their own: the decay over tokens key + 1 .. query of the block
       f32x4 s = wave == 0 ? rf[0] : wave == 1 ? rf[1] : wave == 2 ? rf[2] : rf[3];
       {
-        double x = 1.0;
-#pragma unroll
-        for (int t = 4; t < 16; ++t) x *= static_cast<double>((t >= 4 * grp + 4 && t <= col) ? gs[16 * wave + t] : 1.0f);
+        // (a product along the lanes of a row: lane = token)
+        double x = row_mul<0x118>(row_mul<0x114>(row_mul<0x112>(row_mul<0x111>(static_cast<double>(col >= 4 * grp + 4 ? gs[16 * wave + col] : 1.0f)))));
         const f32x4 own = *reinterpret_cast<const f32x4*>(&gs[16 * wave + 4 * grp]);
         const f32x4 be = *reinterpret_cast<const f32x4*>(&bs[16 * wave + 4 * grp]);
 #pragma unroll
@@ -314,12 +346,10 @@ __global__ __launch_bounds__(NTH, DC <= 8 ? 2 : 1) void chunk_kernel(ChunkArgs a
         }
       }
     }
-    if (more) load_r(first + CT, id + 1);
-    if (16 * wave < n) {
+    load_r(ahead, id_ahead);
+    if (FEW || 16 * wave < n) {
       if (carry || first > t0) {   // S^T Q^T, in chains of one feature tile (one long chain rounds twice as much)
-        double gd = pre[place];
-        for (int k = 0; k < wave; ++k) gd *= wh[k];
-        const float g = gd;
+        const float g = front[place];
 #pragma unroll
         for (int u = 0; u < NU; ++u)
 #pragma unroll
@@ -341,9 +371,17 @@ __global__ __launch_bounds__(NTH, DC <= 8 ? 2 : 1) void chunk_kernel(ChunkArgs a
         }
       }
     }
-    if (more) load_q(first + CT);
+    load_q(ahead);
     // ---- the state behind the chunk ----
-    if (owner) {
+    if (OWNERS || owner) {
+      if (n < CT) {   // (no key past the segment, not even against a weight of zero: it may be infinite)
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int m = 0; m < ND; ++m) kf[tt][j][m] = 16 * tt + 4 * grp + j < n ? kf[tt][j][m] : 0.f;
+      }
       const float gn = (wh[0] * wh[1]) * (wh[2] * wh[3]);
 #pragma unroll
       for (int m = 0; m < ND; ++m)
@@ -351,13 +389,8 @@ __global__ __launch_bounds__(NTH, DC <= 8 ? 2 : 1) void chunk_kernel(ChunkArgs a
         for (int u = 0; u < NU; ++u) S[m][u] *= gn;
 #pragma unroll
       for (int tt = 0; tt < 4; ++tt) {
-        if (16 * tt < n) {   // (uniform)
-          double g = 1.0;
-#pragma unroll
-          for (int k = tt + 1; k < 4; ++k) g *= wh[k];
-          float w[4];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) w[j] = post[16 * tt + 4 * grp + j] * g;
+        if (FEW || 16 * tt < n) {   // (uniform)
+          const f32x4 w = *reinterpret_cast<const f32x4*>(&tail[16 * tt + 4 * grp]);
           f32x4 x[NU];
 #pragma unroll
           for (int u = 0; u < NU; ++u) x[u] = value_frag(u, 16 * tt + 4 * grp);
@@ -365,12 +398,12 @@ __global__ __launch_bounds__(NTH, DC <= 8 ? 2 : 1) void chunk_kernel(ChunkArgs a
           for (int m = 0; m < ND; ++m) {
             f32x4 kw;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) kw[j] = 16 * tt + 4 * grp + j < n ? kf[tt][j][m] * w[j] : 0.f;
+            for (int j = 0; j < 4; ++j) kw[j] = kf[tt][j][m] * w[j];
 #pragma unroll
             for (int u = 0; u < NU; ++u) S[m][u] += mma16(x[u], kw, f32x4{0.f, 0.f, 0.f, 0.f});
           }
         }
-        if (more) load_k(first + CT, tt);
+        load_k(ahead, tt);
       }
     }
     __syncthreads();   // every reader of the chunk and of the old state is done
@@ -396,12 +429,13 @@ __global__ __launch_bounds__(NTH, DC <= 8 ? 2 : 1) void chunk_kernel(ChunkArgs a
 template <typename T, int DC, bool FULL>
 int launch_chunks(const ChunkArgs& a, int n_chunks, hipStream_t s) {
   scores_kernel<DC, FULL><<<dim3(n_chunks, a.Gq), NTH, 0, s>>>(a);
-  // 64 value columns per workgroup from more than one workgroup per CU on, fewer below: the walk is serial, idle CUs cost nothing
-  // (96 workgroups of 64 columns -> 384 of 16: 140 us -> 75, 3 segments of 700).  At one per CU 32 columns win (64 segments of
-  // 200, 4 heads of 64 x 64: 47 us, 64 columns 50), past it their second round loses (100 segments: 74 us, 62).
+  // Value columns per workgroup: 16 while these keep to two workgroups per CU, the walk is serial and idle CUs cost nothing (3 segments of 700,
+  // 8 heads of 128 x 256: 16 columns 83 us, 32 88, 64 139; one of 2000, 64 heads of 128 x 128: 181, 185, 313); 32 up to two workgroups per CU, of keys
+  // wider than 64 up to three (6 segments of 700: 16 columns 166, 32 131, 64 163; 3 of 2000: 507, 415, 450; 64 of 200, 4 heads of 64 x 64: 54, 46, 52); 64
+  // past them (4 of 2000: 672, 501, 458; 100 of 200: 77, 68, 60).
   const int64_t wide = static_cast<int64_t>(a.B) * a.H * ((a.vdim + 63) / 64);
-  if (wide > 256) chunk_kernel<T, DC, 64, FULL><<<segment_grid(a.H, a.B, (a.vdim + 63) / 64), NTH, 0, s>>>(a);
-  else if (wide == 256) chunk_kernel<T, DC, 32, FULL><<<dim3(a.B, a.H, (a.vdim + 31) / 32), NTH, 0, s>>>(a);
+  if (wide > (DC > 4 ? 384 : 256)) chunk_kernel<T, DC, 64, FULL><<<segment_grid(a.H, a.B, (a.vdim + 63) / 64), NTH, 0, s>>>(a);
+  else if (wide > 128) chunk_kernel<T, DC, 32, FULL><<<dim3(a.B, a.H, (a.vdim + 31) / 32), NTH, 0, s>>>(a);
   else chunk_kernel<T, DC, 16, FULL><<<dim3(a.B, a.H, (a.vdim + 15) / 16), NTH, 0, s>>>(a);
   return BCG_CHECK_LAUNCH();
 }
