@@ -199,8 +199,8 @@ def load_library(path: str = None) -> ctypes.CDLL:
         "bcg_moe_route": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
                           c_int, c_int, c_void_p],
         "bcg_moe_align": [c_void_p, c_int, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p],
-        "bcg_moe_gather": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p],
-        "bcg_gemm_w4_grouped": [c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_float, c_void_p],
+        "bcg_gemm_w4_grouped": [c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_float, c_void_p, c_int,
+                                c_int, c_void_p],
         "bcg_moe_route_table": [c_void_p, c_void_p] + [c_int] * 4 + [c_void_p] * 3,
         "bcg_moe_rows_tile": [],
         "bcg_moe_rows": [c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_int64, c_void_p, c_void_p] + [c_int] * 8

@@ -311,9 +311,9 @@ def seqmix_ops(lib, linear):
 
     def _wide_experts(n_slots, E, W, ff, kind, h, up, down):
         """Whether the products run on position tiles of 256 rows: from WIDE_SLOTS routed rows per expert on.  Two gated
-        products of 8 experts, top 2, 64-row tiles -> 256-row tiles, us: width 2048, ff 2048: 32 rows per expert 93 -> 112,
-        64: 115 -> 112, 256: 211 -> 133, 2046: 836 -> 509; width 4096, ff 3072: 32: 186 -> 197, 64: 297 -> 208, 256: 629 ->
-        306, 2046: 2274 -> 1210 (1.02 PFLOP/s of 0.54)."""
+        products of 8 experts, top 2, 64-row tiles -> 256-row tiles, us: width 2048, ff 2048: 32 rows per expert 71 -> 97,
+        64: 89 -> 98, 256: 211 -> 103, 2046: 818 -> 424; width 4096, ff 3072: 32: 190 -> 192, 64: 294 -> 194, 256: 629 ->
+        271, 2046: 2285 -> 1063 (1.16 PFLOP/s of 0.54)."""
         if h.dtype != torch.bfloat16 or W % 64 or ff % 64 or (kind in EXPERT_ACTS and ff % 128) or n_slots < WIDE_SLOTS * E:
             return False
         rows = n_slots + E * (WIDE_ROWS - 1) + 2 * WIDE_ROWS    # (with a tile to spare: the kernel's offsets are 32-bit)
@@ -353,14 +353,12 @@ def seqmix_ops(lib, linear):
             pos, used = place[:n_slots], place[n_slots:]
             _check(lib.bcg_moe_align(_p(idx), n_slots, E, _p(sorted_), cap, _p(tile_e), n_tiles, rows, _p(pos), _p(used),
                                      _stream()), "moe_align")
-            a = torch.empty(cap, W, dtype=h.dtype, device=dev)
-            _check(lib.bcg_moe_gather(_p(h), _p(sorted_), _p(a), cap, 2 * W, top, _stream()), "moe_gather")
             hidden = torch.empty(cap, ff, dtype=h.dtype, device=dev)
-            _check(lib.bcg_gemm_w4_grouped(3 if gated else 4, _p(a), _p(up), _p(hidden), _p(tile_e), _p(used), n_tiles, n_up, W,
-                                           limit if kind == "clamped_glu" else 0.0, _stream()), "moe gate / up")
-            y = a   # the down product's rows replace the gathered ones
-            _check(lib.bcg_gemm_w4_grouped(0, _p(hidden), _p(down), _p(y), _p(tile_e), _p(used), n_tiles, W, ff, 0.0, _stream()),
-                   "moe down")
+            _check(lib.bcg_gemm_w4_grouped(3 if gated else 4, _p(h), _p(up), _p(hidden), _p(tile_e), _p(used), n_tiles, n_up, W,
+                                           limit if kind == "clamped_glu" else 0.0, _p(sorted_), top, T, _stream()), "moe gate / up")
+            y = torch.empty(cap, W, dtype=h.dtype, device=dev)
+            _check(lib.bcg_gemm_w4_grouped(0, _p(hidden), _p(down), _p(y), _p(tile_e), _p(used), n_tiles, W, ff, 0.0, None, 1, 0,
+                                           _stream()), "moe down")
             _check(lib.bcg_moe_combine(_p(y), _p(weights), _p(pos), _p(idx), E, _p(out), T, W, top, f32, _stream()), "moe_combine")
             return out
         _check(lib.bcg_moe_align(_p(idx), n_slots, E, _p(sorted_), cap, _p(tile_e), n_tiles, rows, None, None, _stream()),

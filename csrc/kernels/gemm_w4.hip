@@ -160,15 +160,17 @@ __device__ uint64_t w4_stamps[1 << 17];
 // w_scale[n] applied in the epilogue)
 // GROUPED: rows 256 t .. of X meet the weight group[t] of a stack [groups, N, K]; only the first used[0] tiles of
 // 256 rows hold work (the row counts of the groups are known on the device only)
-template <int EPI, bool F8 = false, bool GROUPED = false>
+// GATHER: row p of X is row slots[p] / top of x [x_rows, K] (slots[p] < 0: zeros)
+template <int EPI, bool F8 = false, bool GROUPED = false, bool GATHER = false>
 __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_w4_kernel(
     const void* __restrict__ Xv, const void* __restrict__ Wv, const bf16_t* __restrict__ bias,
     const bf16_t* __restrict__ residual, bf16_t* __restrict__ C, float* __restrict__ ws,
     int* __restrict__ counters, int M, int N, int K, int ldc, int inter, int m_tiles, int n_tiles,
     int split_k, const float* __restrict__ x_scale, const float* __restrict__ w_scale,
-    const int* __restrict__ group, const int* __restrict__ used, float limit) {
+    const int* __restrict__ group, const int* __restrict__ used, float limit, const int* __restrict__ slots, int top, int x_rows) {
   static_assert(!F8 || EPI == EPI_STORE || EPI == EPI_RESIDUAL, "fp8: store / residual epilogues");
   static_assert(GROUPED || (EPI != EPI_GATED && EPI != EPI_RELU2), "grouped epilogues");
+  static_assert(GROUPED || !GATHER, "rows are gathered for groups");
   constexpr bool STACKED = EPI == EPI_SILU_MUL || EPI == EPI_CLAMPED;   // W = [gate; up]
   if constexpr (EPI == EPI_CLAMPED || EPI == EPI_TAIL_GELU) split_k = 1;
   if constexpr (GROUPED) {
@@ -266,7 +268,8 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
   const int w_rows = STACKED ? 2 * inter : N;
   auto item_srd = [&](const Geo& g, i32x4& sX, i32x4& sW) {
     const int wr0 = STACKED ? (g.n0 >> 1) : g.n0;
-    sX = make_srd(X + static_cast<size_t>(g.m0) * row_bytes, static_cast<uint32_t>(M - g.m0) * row_bytes);
+    sX = GATHER ? make_srd(X, static_cast<uint32_t>(x_rows) * row_bytes)
+                : make_srd(X + static_cast<size_t>(g.m0) * row_bytes, static_cast<uint32_t>(M - g.m0) * row_bytes);
     const size_t w_first = (GROUPED ? static_cast<size_t>(group[g.m0 / BM]) * N : 0) + wr0;
     sW = make_srd(W + w_first * row_bytes, static_cast<uint32_t>(w_rows - wr0) * row_bytes);
   };
@@ -282,6 +285,18 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
   uint32_t vX[8], vW[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) vX[i] = voffX + i * strideX, vW[i] = voffW + i * strideW;
+  // GATHER: the rows that this lane's pieces of an item read, asked for where the DMA cursor enters it (used at once: a load that is
+  // pending at the K-loop's back edge would make hipcc wait for every piece there); an offset past the range reads zeros
+  auto item_rows = [&](const Geo& g) {
+    if constexpr (GATHER) {
+      int slot[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) slot[i] = slots[g.m0 + prow + 32 * i];
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        vX[i] = slot[i] < 0 ? 0x80000000u : static_cast<uint32_t>(slot[i]) / static_cast<uint32_t>(top) * row_bytes + pch;
+    }
+  };
   const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem));
   // piece q (0..15) of stream tile t: q < 8 X piece q, else W piece q - 8
   auto dma_m0 = [&](int t, int q) {
@@ -389,6 +404,7 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
   bf16x8 x0[8], w0[8], x1[8], w1[8];
   i32x4 dX, dW;
   item_srd(gc, dX, dW);
+  item_rows(gc);
   i32x4 nullX = dX, nullW = dW;  // zero-range descriptors: pieces past the stream's last tile
   nullX[2] = 0, nullW[2] = 0;
   auto advance = [&]() {
@@ -397,6 +413,7 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
       if (++jd < n_items) {
         const Geo g = geo(jd);
         item_srd(g, dX, dW);
+        item_rows(g);
         dk0 = g.k0, dnk = g.nk;
       }
     }
@@ -1090,19 +1107,19 @@ int launch_w4(const void* x, const void* w, const void* bias, const void* res, v
   hipLaunchKernelGGL((gemm_w4_kernel<EPI, F8>), dim3(grid), dim3(256),
                      0, stream, x, w, static_cast<const bf16_t*>(bias), static_cast<const bf16_t*>(res),
                      static_cast<bf16_t*>(c), ws, cnt, M, N, K, ldc, inter, m_tiles, n_tiles, split_k, xs, wsc,
-                     static_cast<const int*>(nullptr), static_cast<const int*>(nullptr), limit);
+                     static_cast<const int*>(nullptr), static_cast<const int*>(nullptr), limit, static_cast<const int*>(nullptr), 1, 0);
   return BCG_CHECK_LAUNCH();
 }
 
-template <int EPI>
+template <int EPI, bool GATHER>
 int launch_w4_grouped(const void* x, const void* w, void* c, const int* group, const int* used, int m_tiles, int N, int K,
-                      float limit, hipStream_t stream) {
+                      float limit, const int* slots, int top, int x_rows, hipStream_t stream) {
   const int n_tiles = (N + BN - 1) / BN, inter = N / 2, ldc = EPI == EPI_GATED ? inter : N;
   const int grid = static_cast<int>(std::min<long long>(1ll * m_tiles * n_tiles, w4_cus()));
-  hipLaunchKernelGGL((gemm_w4_kernel<EPI, false, true>), dim3(grid), dim3(256), 0, stream, x, w, static_cast<const bf16_t*>(nullptr),
+  hipLaunchKernelGGL((gemm_w4_kernel<EPI, false, true, GATHER>), dim3(grid), dim3(256), 0, stream, x, w, static_cast<const bf16_t*>(nullptr),
                      static_cast<const bf16_t*>(nullptr), static_cast<bf16_t*>(c), static_cast<float*>(nullptr),
                      static_cast<int*>(nullptr), m_tiles * BM, N, K, ldc, inter, m_tiles, n_tiles, 1,
-                     static_cast<const float*>(nullptr), static_cast<const float*>(nullptr), group, used, limit);
+                     static_cast<const float*>(nullptr), static_cast<const float*>(nullptr), group, used, limit, slots, top, x_rows);
   return BCG_CHECK_LAUNCH();
 }
 
@@ -1153,21 +1170,25 @@ BCG_API int bcg_gemm_w4(int epi, const void* x, const void* w, const void* bias,
   }
 }
 
-// Grouped product (experts): rows 256 t .. 256 t + 255 of x [256 m_tiles, K] times w[group[t]] [N, K], for the first
-// used[0] <= m_tiles row tiles; c rows past them stay as they are.  epi: 0 = store, 3 = gated unit of rows that
-// alternate 16 gate / 16 up (c [*, N / 2]; limit > 0: the clamped unit, else silu(gate) * up), 4 = relu squared.  group
-// and used are read on the device.  K % 64 == 0; N % 16 == 0, epi 3: N % 256 == 0.
+// Grouped product (experts): rows 256 t .. 256 t + 255 of X [256 m_tiles, K] times w[group[t]] [N, K], for the first
+// used[0] <= m_tiles row tiles; c rows past them stay as they are.  epi 0: X = x (slots, top and x_rows unused), c = the product.  Epilogues of
+// gathered rows, X row p = x [x_rows, K] row slots[p] / top (slots[p] < 0: zeros): 3 = gated unit of weight rows that
+// alternate 16 gate / 16 up (c [*, N / 2]; limit > 0: the clamped unit, else silu(gate) * up), 4 = relu squared.  group, used
+// and slots are read on the device.  K % 64 == 0; N % 16 == 0, epi 3: N % 256 == 0.
+// Gathering by the address of the LDS-DMA pieces takes eight loads and a wait per tile; a launch of its own wrote the rows and read
+// them back (all launches of 8 experts, top 2, width 4096, 8183 rows: 1113 -> 1065 us; 1000 rows 291 -> 279; width 2048, 8183 rows 444 -> 423).
 BCG_API int bcg_gemm_w4_grouped(int epi, const void* x, const void* w, void* c, const int* group, const int* used, int m_tiles,
-                                int N, int K, float limit, hipStream_t stream) {
+                                int N, int K, float limit, const int* slots, int top, int x_rows, hipStream_t stream) {
   if (m_tiles <= 0 || N <= 0 || N % 16 || K % BK || K <= 0 || m_tiles > (1 << 20)) return -2;
   const unsigned long long M = 1ull * m_tiles * BM;
   if (2 * (M + BM) * K >= (1ull << 31) || 2ull * (N + BN) * K >= (1ull << 31) || 2 * (M + BM) * N >= (1ull << 31)) return -2;
+  if (epi != EPI_STORE && (slots == nullptr || top < 1 || x_rows < 1 || 2ull * (x_rows + 1ull) * K >= (1ull << 31))) return -2;
   switch (epi) {
-    case EPI_STORE: return launch_w4_grouped<EPI_STORE>(x, w, c, group, used, m_tiles, N, K, 0.f, stream);
+    case EPI_STORE: return launch_w4_grouped<EPI_STORE, false>(x, w, c, group, used, m_tiles, N, K, 0.f, nullptr, 1, 0, stream);
     case EPI_GATED:
       if (N % 256) return -2;
-      return launch_w4_grouped<EPI_GATED>(x, w, c, group, used, m_tiles, N, K, limit, stream);
-    case EPI_RELU2: return launch_w4_grouped<EPI_RELU2>(x, w, c, group, used, m_tiles, N, K, 0.f, stream);
+      return launch_w4_grouped<EPI_GATED, true>(x, w, c, group, used, m_tiles, N, K, limit, slots, top, x_rows, stream);
+    case EPI_RELU2: return launch_w4_grouped<EPI_RELU2, true>(x, w, c, group, used, m_tiles, N, K, 0.f, slots, top, x_rows, stream);
     default: return -2;
   }
 }

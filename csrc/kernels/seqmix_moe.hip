@@ -154,17 +154,6 @@ __global__ __launch_bounds__(1024) void align_kernel(const int* __restrict__ idx
   }
 }
 
-// Rows of the positions, for the 256-row products: out[p] = a[sorted[p] / top].  Padding positions stay as they
-// are: nothing reads what the products make of them.
-__global__ __launch_bounds__(256) void gather_rows_kernel(const uint4* __restrict__ a, const int* __restrict__ sorted,
-                                                          uint4* __restrict__ out, int row_vecs, int top) {
-  const int slot = sorted[blockIdx.x];
-  if (slot < 0) return;
-  const uint4* src = a + static_cast<size_t>(slot / top) * row_vecs;
-  uint4* dst = out + static_cast<size_t>(blockIdx.x) * row_vecs;
-  for (int i = threadIdx.x; i < row_vecs; i += 256) dst[i] = src[i];
-}
-
 // Epilogue of a gated expert's first product (act 2, 3).  The N rows of the expert's weight are its
 // gate and up rows in alternating groups of 16 ([gate 0..15 | up 0..15 | gate 16..31 | ...]), so a
 // wave's n tiles 0 / 2 hold gate columns and tiles 1 / 3 the up columns of the SAME features:
@@ -547,15 +536,6 @@ BCG_API int bcg_moe_align(const void* idx, int n_slots, int E, void* sorted, int
                                                                  static_cast<int*>(sorted), cap,
                                                                  static_cast<int*>(tile_expert), n_tiles, tm,
                                                                  static_cast<int*>(pos), static_cast<int*>(used));
-  return BCG_CHECK_LAUNCH();
-}
-
-// out[p] = a[sorted[p] / top] for the placed positions p < cap; rows of row_bytes (a multiple of 16), 16-byte aligned.
-BCG_API int bcg_moe_gather(const void* a, const void* sorted, void* out, int cap, int row_bytes, int top, void* stream) {
-  if (cap <= 0) return 0;
-  if (row_bytes <= 0 || row_bytes % 16 || top < 1) return -2;
-  gather_rows_kernel<<<cap, 256, 0, static_cast<hipStream_t>(stream)>>>(static_cast<const uint4*>(a), static_cast<const int*>(sorted),
-                                                                      static_cast<uint4*>(out), row_bytes / 16, top);
   return BCG_CHECK_LAUNCH();
 }
 
