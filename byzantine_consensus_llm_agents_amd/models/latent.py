@@ -63,14 +63,17 @@ def latent_mixer(ops, m, L, h, meta, k_cache, v_cache, sel, eps: float):
         q = y[:, :m.q_width]
     q = q.view(T, m.heads, m.dim + m.rot_dim)
     qf = torch.empty(T, m.heads, m.key_width, dtype=dt, device=h.device)
-    ops.head_linear(q[:, :, :m.dim], L["uk"], qf[:, :, :m.kv_rank])
     if m.rot_dim:
-        ops.rope_tail(q, m.dim, qf, m.kv_rank, meta.positions, L["inv_freq"], L["amp"], m.rot_pairs)
+        ops.head_linear_turned(q, m.dim, L["uk"], qf, meta.positions, L["inv_freq"], L["amp"], m.rot_pairs)
+    else:
+        ops.head_linear(q, L["uk"], qf)
     lat = ops.multimap_attention(qf, k_cache, v_cache, meta, m.scale, 1, 0.0, -1.0, 1.0, m.kv_rank, m.window, None)
     if sel is not None:
         lat = lat.index_select(0, sel)
-    att = ops.head_linear(lat.view(-1, m.heads, m.kv_rank), L["uv_t"]).view(-1, m.heads * m.vdim)
+    lat = lat.view(-1, m.heads, m.kv_rank)
     if m.gated:
         gate = y[:, off_g:off_g + m.gate_width]
-        att = ops.gate_mul(att, gate if sel is None else gate.index_select(0, sel), "sigmoid", m.heads * m.vdim // m.gate_width)
+        att = ops.head_linear_gated(lat, L["uv_t"], gate if sel is None else gate.index_select(0, sel))
+    else:
+        att = ops.head_linear(lat, L["uv_t"]).view(-1, m.heads * m.vdim)
     return ops.linear(att, L["o"])

@@ -28,9 +28,9 @@ Kernel plan of one layer (HIP backend; the torch backend runs the same ops from
 ``ops/reference.py``):
 
     latent_attention  fused GEMM [dq | dkv | g] -> rmsnorm_cols (query latent) -> uq GEMM ->
-                      head_linear (W_uk^T q per head, straight into the packed query) + rope_tail;
+                      head_linear_turned (W_uk^T q per head and the rotated tail, into the packed query);
                       latent_kv_write (norm, rotary, paged write) -> multimap_attention (one map,
-                      one KV head, window) -> head_linear (W_uv) -> gate_mul -> o GEMM
+                      one KV head, window) -> head_linear_gated (W_uv, gate) -> o GEMM
     delta             fused GEMM [q | k | v | beta | a | g] -> short_conv (silu) -> delta_prepare ->
                       gated_state_scan -> head_norm_gate (silu) -> o GEMM
     mamba2            in GEMM [z | x | B | C | dt] -> short_conv (bias, silu) -> ssm_prepare ->

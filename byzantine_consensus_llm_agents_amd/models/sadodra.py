@@ -22,7 +22,7 @@ Kernel plan of one layer (HIP backend; the torch backend runs the same ops from
     attention         fused GEMM [q | k] -> rope_pairs_kv_write (norms, temperature, paged K and V from
                       the k part) -> multimap_attention (one map, window, cap, slopes) -> o GEMM
     latent_attention  fused GEMM [q | dkv | g] -> latent_kv_write; head_linear (W_uk) ->
-                      multimap_attention (one KV head) -> head_linear (W_uv) -> gate_mul -> o GEMM
+                      multimap_attention (one KV head) -> head_linear_gated (W_uv, gate) -> o GEMM
     residual_post_norm  x += layer_norm(y), and a rounded copy of x for the next reader
     feed-forward      [gate | up] GEMM -> gated_act (gelu) -> down GEMM -> residual_post_norm
 

@@ -27,8 +27,8 @@ Kernel plan of one layer run (HIP backend; the torch backend runs the same ops f
                       window, kept keys) -> o GEMM
     retention         fused GEMM [q | k | v | g] -> retention_prepare -> gated_state_scan (constant decay)
                       -> head_norm_gate (silu) -> o GEMM
-    latent_attention  fused GEMM [dq | dkv] -> latent_kv_write; rmsnorm_cols -> uq GEMM -> head_linear
-                      (W_uk) + rope_tail -> multimap_attention (one KV head) -> head_linear (W_uv) -> o GEMM
+    latent_attention  fused GEMM [dq | dkv] -> latent_kv_write; rmsnorm_cols -> uq GEMM -> head_linear_turned
+                      (W_uk, tail) -> multimap_attention (one KV head) -> head_linear (W_uv) -> o GEMM
     residual_post_norm  x += s * rms(y), the entry of the next pass, and the next reader's RMS norm, one pass
                       over the row
     feed-forward      [gate | up] GEMM with clamped_glu (linear_clamped_glu) -> down GEMM, or

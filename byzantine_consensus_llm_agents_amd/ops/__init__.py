@@ -60,6 +60,8 @@ def _torch_ops() -> SimpleNamespace:
         latent_kv_write=_ref.latent_kv_write,
         rope_tail=_ref.rope_tail,
         head_linear=_ref.head_linear,
+        head_linear_turned=_ref.head_linear_turned,
+        head_linear_gated=_ref.head_linear_gated,
         gate_mul=_ref.gate_mul,
         ssm_prepare=_ref.ssm_prepare,
         gated_group_norm=_ref.gated_group_norm,

@@ -186,6 +186,8 @@ def load_library(path: str = None) -> ctypes.CDLL:
                                 c_int, c_float, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
         "bcg_rope_tail": [c_void_p, c_int, c_int, c_void_p, c_int, c_int, c_void_p, c_void_p, c_int, c_float, c_int, c_int,
                           c_int, c_int, c_void_p],
+        "bcg_head_linear": [c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_int64, c_int64] + [c_int] * 4 + [c_void_p, c_void_p]
+        + [c_int] * 3 + [c_float, c_void_p, c_int64, c_int, c_void_p],
         "bcg_gate_mul": [c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_int, c_int, c_int, c_int, c_void_p],
         "bcg_gemm_w4_act": [c_int] + [c_void_p] * 4 + [c_int] * 4 + [c_float, c_void_p],
         "bcg_gated_act": [c_void_p, c_void_p, c_int64, c_int, c_int, c_float, c_int, c_void_p],

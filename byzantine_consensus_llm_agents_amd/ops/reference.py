@@ -933,6 +933,18 @@ def head_linear(x3, w, out3=None):
     return out3
 
 
+def head_linear_turned(q, dim: int, w, dst, positions, inv_freq, amp: float, pairs: bool = False):
+    """`head_linear` of ``q[:, :, :dim]`` into the first columns of ``dst``, `rope_tail` of the rest behind them."""
+    head_linear(q[:, :, :dim], w, dst[:, :, :w.shape[2]])
+    return rope_tail(q, dim, dst, w.shape[2], positions, inv_freq, amp, pairs)
+
+
+def head_linear_gated(x3, w, gate):
+    """``gate_mul(head_linear(x3, w), gate, "sigmoid")`` as [T, H N]; gate [T, H N / group]."""
+    n = x3.shape[1] * w.shape[2]
+    return gate_mul(head_linear(x3, w).view(x3.shape[0], n), gate, "sigmoid", n // gate.shape[1])
+
+
 def gate_mul(x, gate, kind: str, group: int = 1):
     """``x * sigmoid(gate)`` or ``x * silu(gate)`` (fp32, rounded once); gate [T, n / group] with any
     row stride: one gate column serves ``group`` neighbouring columns of x (one gate per head)."""

@@ -1,5 +1,5 @@
 """HIP bindings of the dynamic-tanh norm, latent-attention, selective-state-space and token-input
-kernels (csrc/kernels/seqmix_latent.hip).
+kernels (csrc/kernels/seqmix_latent.hip, seqmix_heads.hip).
 
 Same conventions as ``seqmix.py`` / ``seqstate.py``: bf16 or fp32 activations (one template
 instance each), fp32 residual stream, norms, angles, decays and step sizes; shapes, dtypes and
@@ -154,8 +154,51 @@ def seqlatent_ops(lib):
                                  int(pairs), T, H, _act(src), _stream()), "rope_tail")
         return dst
 
+    def _own_heads(x3, w, out3, *more):
+        """Whether csrc/kernels/seqmix_heads.hip takes the product as its operands lie: bf16, inputs of 32, 64, 128 or 256, columns in
+        sixteens, 16-byte aligned rows.  Elsewhere (fp32, other widths, transforms and traces) the vendor's batched product."""
+        return (x3.dtype == torch.bfloat16 and w.shape[1] in (32, 64, 128, 256) and w.shape[2] % 16 == 0 and w.shape[2] > 0 and w.shape[0] > 0
+                and all(t.is_cuda and t.get_device() == torch.cuda.current_device() and t.data_ptr() % 16 == 0 for t in (x3, w, out3))
+                and all(s % 8 == 0 for t in (x3, out3) for s in t.stride()[:2]) and not watched() and all(bare(t) for t in (x3, w, out3, *more)))
+
+    def _head_linear(x3, w, out3, tail=None, gate=None, group=1):
+        T, H, K = x3.shape
+        pos, freq, n, pairs, amp = tail or (None, None, 0, False, 1.0)
+        _check(lib.bcg_head_linear(_p(x3), x3.stride(0), x3.stride(1), _p(w), _p(out3), out3.stride(0), out3.stride(1), T, H, K, w.shape[2],
+                                   _p(pos), _p(freq), n, 0 if freq is None else freq.numel(), int(pairs), float(amp), _p(gate),
+                                   0 if gate is None else gate.stride(0), group, _stream()), "head_linear")
+
+    def head_linear_turned(q, dim, w, dst, positions, inv_freq, amp, pairs=False):
+        """`head_linear` of the first ``dim`` features into ``dst`` and `rope_tail` of the others behind it, in one launch where the
+        kernel takes the operands."""
+        N = w.shape[2]
+        if (q.dim() == 3 and dst.dim() == 3 and q.is_contiguous() and dst.is_contiguous() and q.dtype == dst.dtype and q.shape[:2] == dst.shape[:2]
+                and 0 < dim < q.shape[2] and w.shape[:2] == (q.shape[1], dim) and w.is_contiguous() and w.dtype == q.dtype
+                and q.shape[2] - dim == dst.shape[2] - N and 2 * inv_freq.numel() <= q.shape[2] - dim and q.shape[0] > 0
+                and _own_heads(q[:, :, :dim], w, dst[:, :, :N], q, dst, positions, inv_freq)):
+            _i32(positions, q.shape[0], "positions")
+            _f32(inv_freq, inv_freq.numel(), "inv_freq")
+            _head_linear(q[:, :, :dim], w, dst[:, :, :N], (positions, inv_freq, q.shape[2] - dim, pairs, amp))
+            return dst
+        head_linear(q[:, :, :dim], w, dst[:, :, :N])
+        return rope_tail(q, dim, dst, N, positions, inv_freq, amp, pairs)
+
+    def head_linear_gated(x3, w, gate):
+        """``gate_mul(head_linear(x3, w), gate, "sigmoid")`` as [T, H N] (gate [T, H N / group]), in one launch where the kernel takes the operands."""
+        T, H, _ = x3.shape
+        n = H * w.shape[2]
+        group = n // gate.shape[1] if gate.dim() == 2 and gate.shape[1] > 0 and n % gate.shape[1] == 0 else 0
+        if (T > 0 and w.dim() == 3 and x3.shape[1] == w.shape[0] and x3.shape[2] == w.shape[1] and x3.stride(2) == 1 and x3.dtype == w.dtype
+                and w.is_contiguous() and gate.shape[0] == T and gate.stride(1) == 1 and gate.dtype == x3.dtype and gate.device == x3.device
+                and (gate.stride(0) % 8 == 0 and gate.data_ptr() % 16 == 0 if group == 1 else group > 0 and group % 8 == 0 and w.shape[2] % group == 0)):
+            out = torch.empty(T, H, w.shape[2], dtype=x3.dtype, device=x3.device)
+            if _own_heads(x3, w, out, gate):
+                _head_linear(x3, w, out, None, gate, group)
+                return out.view(T, n)
+        return gate_mul(head_linear(x3, w).view(T, n), gate, "sigmoid", max(group, 1))
+
     def head_linear(x3, w, out3=None):
-        """Per-head products on the vendor's batched GEMM (fp32 accumulation; true fp32 for fp32 operands).
+        """Per-head products (fp32 accumulation; true fp32 for fp32 operands), own kernel or vendor's batched GEMM (`_own_heads`).
         The weight is the right operand as it lies, [H, K, N]: the batched bf16 product has faulted the
         GPU with a transposed view there."""
         _req(x3.dim() == 3 and w.dim() == 3 and x3.shape[1] == w.shape[0] and x3.shape[2] == w.shape[1] and x3.stride(2) == 1
@@ -164,7 +207,9 @@ def seqlatent_ops(lib):
             out3 = torch.empty(x3.shape[0], x3.shape[1], w.shape[2], dtype=x3.dtype, device=x3.device)
         _req(out3.shape == (x3.shape[0], x3.shape[1], w.shape[2]) and out3.stride(2) == 1 and out3.dtype == x3.dtype,
              "head_linear: out [T, H, N]")
-        if x3.shape[0]:
+        if x3.shape[0] and _own_heads(x3, w, out3):
+            _head_linear(x3, w, out3)
+        elif x3.shape[0]:
             torch.bmm(x3.transpose(0, 1), w, out=out3.transpose(0, 1))
         return out3
 
@@ -242,6 +287,7 @@ def seqlatent_ops(lib):
         return out
 
     return dict(embed_scale_dyt=embed_scale_dyt, residual_post_norm=residual_post_norm, rmsnorm_cols=rmsnorm_cols,
-                latent_kv_write=latent_kv_write, rope_tail=rope_tail, head_linear=head_linear, gate_mul=gate_mul,
+                latent_kv_write=latent_kv_write, rope_tail=rope_tail, head_linear=head_linear,
+                head_linear_turned=head_linear_turned, head_linear_gated=head_linear_gated, gate_mul=gate_mul,
                 ssm_prepare=ssm_prepare, gated_group_norm=gated_group_norm, moe_table_route=moe_table_route,
                 gelu_gather_mul=gelu_gather_mul, gated_act=gated_act)
