@@ -35,7 +35,7 @@ Kernel plan of one layer (HIP backend; the torch backend runs the same ops from
                       gated_state_scan -> head_norm_gate (silu) -> o GEMM
     mamba2            in GEMM [z | x | B | C | dt] -> short_conv (bias, silu) -> ssm_prepare ->
                       gated_state_scan -> gated_group_norm -> o GEMM
-    feed-forward      moe_table_route -> grouped expert GEMMs (gated epilogue) -> combine
+    feed-forward      table_experts_post_norm: routes by table, grouped expert GEMMs (gated epilogue), their sum into the stream
     residual_post_norm  x += post(y) fused with the next reader's norm (or a rounded copy of x)
     token input       G GEMM -> gelu_gather_mul -> P GEMM -> residual_post_norm (rms)
 
@@ -341,9 +341,8 @@ class MabivikModel:
             after = ("copy",) if c.side_dim else nxt
             if spec.mlp is not None:
                 h2 = ops.residual_post_norm(x, y, L["post1"], L["pre2"], dt)
-                idx_e, w_e = ops.moe_table_route(tokens, L["table"], spec.mlp.top)
-                h = ops.residual_post_norm(x, ops.moe_experts(h2, L["e_up"], L["e_down"], idx_e, w_e, "silu_gated"),
-                                           L["post2"], after, dt)
+                h = ops.table_experts_post_norm(x, h2, L["e_up"], L["e_down"], tokens, L["table"], spec.mlp.top, "silu_gated",
+                                                L["post2"], after, dt)
             else:
                 h = ops.residual_post_norm(x, y, L["post1"], after, dt)
             if c.side_dim:

@@ -66,6 +66,7 @@ def _torch_ops() -> SimpleNamespace:
         ssm_prepare=_ref.ssm_prepare,
         gated_group_norm=_ref.gated_group_norm,
         moe_table_route=_ref.moe_table_route,
+        table_experts_post_norm=_ref.table_experts_post_norm,
         gelu_gather_mul=_ref.gelu_gather_mul,
         gated_act=_ref.gated_act,
         linear_clamped_glu=_ref.linear_clamped_glu,

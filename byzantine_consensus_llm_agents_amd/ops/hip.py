@@ -200,7 +200,10 @@ def load_library(path: str = None) -> ctypes.CDLL:
         "bcg_moe_tile_rows": [],
         "bcg_moe_route": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
                           c_int, c_int, c_void_p],
-        "bcg_moe_align": [c_void_p, c_int, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p],
+        "bcg_moe_align": [c_void_p, c_int, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int,
+                          c_int, c_void_p],
+        "bcg_experts_post_norm": [c_void_p] * 4 + [c_int] * 3 + [c_float, c_void_p, c_void_p, c_float, c_int, c_float] + [c_void_p] * 3
+        + [c_int, c_int, c_void_p],
         "bcg_gemm_w4_grouped": [c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_float, c_void_p, c_int,
                                 c_int, c_void_p],
         "bcg_moe_route_table": [c_void_p, c_void_p] + [c_int] * 4 + [c_void_p] * 3,
@@ -1039,7 +1042,7 @@ def hip_ops() -> SimpleNamespace:
     extra = seqmix_ops(lib, linear)
     extra.update(seqstate_ops(lib))
     from .seqlatent import seqlatent_ops
-    extra.update(seqlatent_ops(lib))
+    extra.update(seqlatent_ops(lib, extra.pop("_experts")))
     from .seqhyper import seqhyper_ops
     extra.update(seqhyper_ops(lib))
 

@@ -983,6 +983,11 @@ def moe_table_route(tokens, table, top: int):
     return idx, torch.full(idx.shape, 1.0 / top, dtype=torch.float32, device=idx.device)
 
 
+def table_experts_post_norm(x, h, up, down, tokens, table, top: int, kind: str, post, pre, out_dtype):
+    """``x += post(y)``, ``pre(x)`` (`residual_post_norm`) with y = `moe_experts` of h under the routes of `moe_table_route`."""
+    return residual_post_norm(x, moe_experts(h, up, down, *moe_table_route(tokens, table, top), kind), post, pre, out_dtype)
+
+
 def gelu_gather_mul(z, tokens, table, off: int):
     """``gelu_tanh(z) * table[token, off : off + n]`` for z [T, n] (fp32 math, rounded once)."""
     e = table.index_select(0, tokens.long())[:, off:off + z.shape[1]].float()

@@ -24,7 +24,14 @@ def _dyt(norm, W):
 MAX_LN_WIDTH = 16384
 
 
-def seqlatent_ops(lib):
+# most slots that the position kernel's one workgroup also routes by table (8 experts, top 2, us, two launches
+# and one: 128 slots 6.1, 3.4; 2000 6.0, 4.9; 4096 6.6, 6.4; 16366 13.1, 18.8)
+ROUTED_SLOTS = 2048
+
+
+def seqlatent_ops(lib, experts):
+    moe_experts, check_experts, expert_products = experts
+
     def embed_scale_dyt(tokens, table, scale, norm, out_dtype):
         _req(tokens.dtype == torch.int32 and tokens.is_contiguous() and tokens.dim() == 1, "tokens int32 [T]")
         _req(table.dim() == 2 and table.is_contiguous() and table.dtype == out_dtype, "table [V, W] in the activation dtype")
@@ -277,6 +284,36 @@ def seqlatent_ops(lib):
                "moe_route_table")
         return idx, wts
 
+    def table_experts_post_norm(x, h, up, down, tokens, table, top, kind, post, pre, out_dtype):
+        """``residual_post_norm(x, moe_experts(h, up, down, *moe_table_route(tokens, table, top), kind), post, pre, out_dtype)``: the sum of a
+        token's experts goes into the stream where it is made, and a small step's positions are found with its routes."""
+        T, W = h.shape
+        if not (h.dtype == out_dtype == torch.bfloat16 and 0 < T * top < 1 << 24 and 1 <= top <= 8 and W % 4 == 0 and post[0] in ("dyt", "rms")
+                and (pre is None or pre[0] in ("copy", "dyt")) and x.dtype == torch.float32 and x.shape == (T, W) and x.is_contiguous()
+                and tokens.dtype == torch.int32 and tokens.shape == (T,) and tokens.is_contiguous() and table.dtype == torch.int32
+                and table.dim() == 2 and table.stride(1) == 1 and table.shape[0] > 0 and top <= table.shape[1] and table.stride(0) < 1 << 31
+                and all(t.is_cuda and t.get_device() == torch.cuda.current_device() for t in (x, h, up, down, tokens, table))
+                and all(t.data_ptr() % 16 == 0 for t in (x, *(v for n in (post, pre or ()) for v in n if torch.is_tensor(v))))
+                and not watched() and all(bare(t) for t in (x, h, up, down, tokens, table))):
+            return residual_post_norm(x, moe_experts(h, up, down, *moe_table_route(tokens, table, top), kind), post, pre, out_dtype)
+        check_experts(h, up, down, kind, 0.0)
+        if T * top <= ROUTED_SLOTS:
+            idx = torch.empty(T, top, dtype=torch.int32, device=h.device)
+            y, pos = expert_products(h, up, down, idx, kind, 0.0, (tokens, table))
+        else:
+            idx, _ = moe_table_route(tokens, table, top)
+            y, pos = expert_products(h, up, down, idx, kind, 0.0)
+        post_kind, (pa, pw, pb), eps = (0, _dyt(post[1:], W), 0.0) if post[0] == "dyt" else (1, (0.0, _p(post[1]), None), float(post[2]))
+        if post[0] == "rms":
+            _f32(post[1], W, "norm weight")
+        out = None if pre is None else torch.empty(T, W, dtype=out_dtype, device=x.device)
+        pre_kind, (qa, qw, qb) = 0 if pre is None else 1 if pre[0] == "copy" else 2, (0.0, None, None)
+        if pre_kind == 2:
+            qa, qw, qb = _dyt(pre[1:], W)
+        _check(lib.bcg_experts_post_norm(_p(x), _p(y), _p(idx), _p(pos), up.shape[0], top, post_kind, pa, pw, pb, eps, pre_kind, qa, qw, qb,
+                                         _p(out), T, W, _stream()), "experts_post_norm")
+        return out
+
     def gelu_gather_mul(z, tokens, table, off):
         _req(z.dim() == 2 and z.is_contiguous() and table.dim() == 2 and table.is_contiguous() and table.dtype == z.dtype
              and 0 <= off and off + z.shape[1] <= table.shape[1], "gelu_gather_mul: z [T, n], table [vocab, >= off + n]")
@@ -290,4 +327,5 @@ def seqlatent_ops(lib):
                 latent_kv_write=latent_kv_write, rope_tail=rope_tail, head_linear=head_linear,
                 head_linear_turned=head_linear_turned, head_linear_gated=head_linear_gated, gate_mul=gate_mul,
                 ssm_prepare=ssm_prepare, gated_group_norm=gated_group_norm, moe_table_route=moe_table_route,
+                table_experts_post_norm=table_experts_post_norm,
                 gelu_gather_mul=gelu_gather_mul, gated_act=gated_act)

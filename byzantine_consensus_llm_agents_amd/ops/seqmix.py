@@ -321,23 +321,18 @@ def seqmix_ops(lib, linear):
         return (2 * rows * max(W, n_up) < 1 << 31 and 2 * (max(W, n_up) + 256) * max(W, ff) < 1 << 31
                 and all(t.data_ptr() % 16 == 0 for t in (h, up, down)))
 
-    def moe_experts(h, up, down, idx, weights, kind="relu2", limit=0.0):
+    def _expert_products(h, up, down, idx, kind, limit, by_table=None):
+        """Both products of the experts' rows: (y, pos), a slot's row at pos[slot], or at the slot where pos is None.  ``by_table``: (tokens,
+        table) by which `idx` is filled first."""
         T, W = h.shape
         E, n_up, _ = up.shape
         top = idx.shape[1]
-        _req(kind == "relu2" or kind in EXPERT_ACTS, "moe_experts: relu2, silu-gated or clamped gated experts")
-        _req(kind != "clamped_glu" or limit > 0, "clamped experts: a positive limit")
         gated = kind in EXPERT_ACTS
-        _req(not gated or n_up % 2 == 0, "gated experts: [gate; up] rows")
         ff = n_up // 2 if gated else n_up
-        _req(h.is_contiguous() and up.shape == (E, n_up, W) and down.shape == (E, W, ff) and up.is_contiguous()
-             and down.is_contiguous() and up.dtype == h.dtype and down.dtype == h.dtype, "expert weights [E, ff, W] / [E, W, ff]")
-        _req(idx.dtype == torch.int32 and idx.shape == (T, top) and idx.is_contiguous() and weights.dtype == torch.float32
-             and weights.shape == (T, top) and weights.is_contiguous(), "routing tables [T, top]")
         n_slots = T * top
         dev, f32 = h.device, _act(h)
-        if n_slots == 0:
-            return torch.zeros(T, W, dtype=torch.float32, device=dev)
+        tokens, table = by_table or (None, None)
+        route = (_p(tokens), _p(table), 0 if table is None else table.shape[0], 0 if table is None else table.stride(0), top)
         wide = _wide_experts(n_slots, E, W, ff, kind, h, up, down)
         held = 0
         if not wide and h.dtype == torch.bfloat16 and all(t.data_ptr() % 16 == 0 for t in (h, up, down)):
@@ -347,22 +342,20 @@ def seqmix_ops(lib, linear):
         cap = n_tiles * rows
         sorted_ = torch.empty(cap, dtype=torch.int32, device=dev)
         tile_e = torch.empty(n_tiles, dtype=torch.int32, device=dev)
-        out = torch.empty(T, W, dtype=torch.float32, device=dev)
         if wide:
             place = torch.empty(n_slots + 1, dtype=torch.int32, device=dev)   # every slot's position; the tiles in use
             pos, used = place[:n_slots], place[n_slots:]
             _check(lib.bcg_moe_align(_p(idx), n_slots, E, _p(sorted_), cap, _p(tile_e), n_tiles, rows, _p(pos), _p(used),
-                                     _stream()), "moe_align")
+                                     *route, _stream()), "moe_align")
             hidden = torch.empty(cap, ff, dtype=h.dtype, device=dev)
             _check(lib.bcg_gemm_w4_grouped(3 if gated else 4, _p(h), _p(up), _p(hidden), _p(tile_e), _p(used), n_tiles, n_up, W,
                                            limit if kind == "clamped_glu" else 0.0, _p(sorted_), top, T, _stream()), "moe gate / up")
             y = torch.empty(cap, W, dtype=h.dtype, device=dev)
             _check(lib.bcg_gemm_w4_grouped(0, _p(hidden), _p(down), _p(y), _p(tile_e), _p(used), n_tiles, W, ff, 0.0, None, 1, 0,
                                            _stream()), "moe down")
-            _check(lib.bcg_moe_combine(_p(y), _p(weights), _p(pos), _p(idx), E, _p(out), T, W, top, f32, _stream()), "moe_combine")
-            return out
-        _check(lib.bcg_moe_align(_p(idx), n_slots, E, _p(sorted_), cap, _p(tile_e), n_tiles, rows, None, None, _stream()),
-               "moe_align")
+            return y, pos
+        _check(lib.bcg_moe_align(_p(idx), n_slots, E, _p(sorted_), cap, _p(tile_e), n_tiles, rows, None, None, *route,
+                                 _stream()), "moe_align")
         if held:
             code = ACT_CODES[EXPERT_ACTS[kind]] if gated else 1
             used = (n_slots + min(E, n_slots) * (rows - 1)) // rows     # `align` packs the tiles in use at the front, this many at most
@@ -372,8 +365,7 @@ def seqmix_ops(lib, linear):
             y = torch.empty(n_slots, W, dtype=h.dtype, device=dev)
             _check(lib.bcg_moe_rows(_p(hidden), cap, ff, _p(down), _p(y), W, _p(sorted_), _p(tile_e), used, held, W, ff, top, 0, 1,
                                     0, 0.0, _stream()), "moe down rows")
-            _check(lib.bcg_moe_combine(_p(y), _p(weights), None, _p(idx), E, _p(out), T, W, top, f32, _stream()), "moe_combine")
-            return out
+            return y, None
         code = ACT_CODES[EXPERT_ACTS[kind]] if gated else 1
         if gated and ff % 16 == 0:   # rows paired by `moe_pair_rows`: the hidden values in the product's epilogue
             hidden = torch.empty(cap, ff, dtype=h.dtype, device=dev)
@@ -392,11 +384,35 @@ def seqmix_ops(lib, linear):
         y = torch.empty(n_slots, W, dtype=h.dtype, device=dev)
         _check(lib.bcg_moe_gemm(_p(hidden), ff, _p(down), _p(y), W, _p(sorted_), _p(tile_e), n_tiles, W, ff, top, 0, 1, 0,
                                 0.0, f32, _stream()), "moe down")
-        _check(lib.bcg_moe_combine(_p(y), _p(weights), None, _p(idx), E, _p(out), T, W, top, f32, _stream()), "moe_combine")
+        return y, None
+
+    def _check_experts(h, up, down, kind, limit):
+        T, W = h.shape
+        E, n_up, _ = up.shape
+        _req(kind == "relu2" or kind in EXPERT_ACTS, "moe_experts: relu2, silu-gated or clamped gated experts")
+        _req(kind != "clamped_glu" or limit > 0, "clamped experts: a positive limit")
+        gated = kind in EXPERT_ACTS
+        _req(not gated or n_up % 2 == 0, "gated experts: [gate; up] rows")
+        ff = n_up // 2 if gated else n_up
+        _req(h.is_contiguous() and up.shape == (E, n_up, W) and down.shape == (E, W, ff) and up.is_contiguous()
+             and down.is_contiguous() and up.dtype == h.dtype and down.dtype == h.dtype, "expert weights [E, ff, W] / [E, W, ff]")
+
+    def moe_experts(h, up, down, idx, weights, kind="relu2", limit=0.0):
+        T, W = h.shape
+        top = idx.shape[1]
+        _check_experts(h, up, down, kind, limit)
+        _req(idx.dtype == torch.int32 and idx.shape == (T, top) and idx.is_contiguous() and weights.dtype == torch.float32
+             and weights.shape == (T, top) and weights.is_contiguous(), "routing tables [T, top]")
+        if T * top == 0:
+            return torch.zeros(T, W, dtype=torch.float32, device=h.device)
+        y, pos = _expert_products(h, up, down, idx, kind, limit)
+        out = torch.empty(T, W, dtype=torch.float32, device=h.device)
+        _check(lib.bcg_moe_combine(_p(y), _p(weights), _p(pos), _p(idx), up.shape[0], _p(out), T, W, top, _act(h), _stream()), "moe_combine")
         return out
 
     return dict(embed_scale_rmsnorm=embed_scale_rmsnorm, embed_position=embed_position, residual_add_rmsnorm32=residual_add_rmsnorm32,
                 rmsnorm32=rmsnorm32, act_fn=act_fn, rope_multi_kv_write=rope_multi_kv_write,
                 kv_from_logical=kv_from_logical, kv_to_logical=kv_to_logical,
                 multimap_attention=multimap_attention, multimap_tile_rows=multimap_tile_rows, moe_route=moe_route, moe_experts=moe_experts,
+                _experts=(moe_experts, _check_experts, _expert_products),
                 moe_pair_rows=moe_pair_rows, moe_route_scored=moe_route_scored)

@@ -116,36 +116,95 @@ __global__ __launch_bounds__(256) void route_table_kernel(const int* __restrict_
   wts[i] = 1.0f / top;
 }
 
-__global__ __launch_bounds__(1024) void align_kernel(const int* __restrict__ idx, int n_slots, int E,
+// The positions of the routed rows.  `table`: routing by token id as in route_table_kernel, written to idx here (one workgroup: for small steps,
+// where a launch costs more than the reads).
+struct TableRoute {
+  const int* tokens; const int* table;
+  int vocab, width, top;
+};
+template <int HELD>
+__global__ __launch_bounds__(1024) void align_kernel(int* __restrict__ idx, int n_slots, int E,
                                                      int* __restrict__ sorted, int cap, int* __restrict__ tile_expert,
-                                                     int n_tiles, int tm, int* __restrict__ pos, int* __restrict__ used) {
-  __shared__ int cnt[MAX_E], off[MAX_E + 1];
-  for (int e = threadIdx.x; e < E; e += blockDim.x) cnt[e] = 0;
+                                                     int n_tiles, int tm, int* __restrict__ pos, int* __restrict__ used, TableRoute by) {
+  // A thread holds its first HELD slots, asked for at once, with their ranks among those of their expert (what the count was); further
+  // slots, behind the held ones of their expert, are read and counted twice.
+  constexpr int NT = 1024;
+  __shared__ int cnt[MAX_E], more[MAX_E], off[MAX_E + 1];
+  const int tid = threadIdx.x;
+  for (int e = tid; e < E; e += NT) cnt[e] = more[e] = 0;
+  int who[HELD], rank[HELD];
+  if (by.table != nullptr) {
+#pragma unroll
+    for (int k = 0; k < HELD; ++k) {
+      const int i = tid + k * NT;
+      who[k] = i < n_slots ? by.tokens[i / by.top] : -1;
+    }
+#pragma unroll
+    for (int k = 0; k < HELD; ++k) {
+      const int i = tid + k * NT, token = who[k];
+      who[k] = token >= 0 && token < by.vocab ? by.table[static_cast<size_t>(token) * by.width + i % by.top] : -1;
+    }
+#pragma unroll
+    for (int k = 0; k < HELD; ++k)
+      if (tid + k * NT < n_slots) idx[tid + k * NT] = who[k];
+  } else {
+#pragma unroll
+    for (int k = 0; k < HELD; ++k) who[k] = tid + k * NT < n_slots ? idx[tid + k * NT] : -1;
+  }
+  for (int i = tid; i < cap; i += NT) sorted[i] = -1;
   __syncthreads();
-  for (int i = threadIdx.x; i < n_slots; i += blockDim.x) {
+#pragma unroll
+  for (int k = 0; k < HELD; ++k) {
+    if (who[k] >= E) who[k] = -1;
+    rank[k] = who[k] >= 0 ? atomicAdd(&cnt[who[k]], 1) : 0;
+  }
+  for (int i = tid + HELD * NT; i < n_slots; i += NT) {
+    if (by.table != nullptr) {   // (read back below by the thread that wrote it)
+      const int token = by.tokens[i / by.top];
+      idx[i] = token >= 0 && token < by.vocab ? by.table[static_cast<size_t>(token) * by.width + i % by.top] : -1;
+    }
     const int e = idx[i];
-    if (e >= 0 && e < E) atomicAdd(&cnt[e], 1);
-  }
-  for (int i = threadIdx.x; i < cap; i += blockDim.x) sorted[i] = -1;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    off[0] = 0;
-    for (int e = 0; e < E; ++e) off[e + 1] = off[e] + (cnt[e] + tm - 1) / tm * tm;
-    if (used != nullptr) *used = off[E] / tm;
+    if (e >= 0 && e < E) atomicAdd(&more[e], 1);
   }
   __syncthreads();
-  for (int t = threadIdx.x; t < n_tiles; t += blockDim.x) {
-    int who = -1;
-    for (int e = 0; e < E; ++e)
-      if (t * tm >= off[e] && t * tm < off[e + 1]) who = e;
-    tile_expert[t] = who;
+  if (tid < 64) {   // whole tiles per expert, added up by one wave
+    int before = 0;
+    for (int e0 = 0; e0 < E; e0 += 64) {
+      const int e = e0 + tid;
+      int v = e < E ? (cnt[e] + more[e] + tm - 1) / tm * tm : 0;
+      for (int o = 1; o < 64; o <<= 1) {
+        const int u = __shfl_up(v, o, 64);
+        if (tid >= o) v += u;
+      }
+      if (e < E) off[e + 1] = before + v;
+      before += __shfl(v, 63, 64);
+    }
+    if (tid == 0) {
+      off[0] = 0;
+      if (used != nullptr) *used = before / tm;
+    }
   }
-  for (int e = threadIdx.x; e < E; e += blockDim.x) cnt[e] = 0;
   __syncthreads();
-  for (int i = threadIdx.x; i < n_slots; i += blockDim.x) {
+  for (int t = tid; t < n_tiles; t += NT) {
+    int e = -1;
+    for (int k = 0; k < E; ++k)
+      if (t * tm >= off[k] && t * tm < off[k + 1]) e = k;
+    tile_expert[t] = e;
+  }
+#pragma unroll
+  for (int k = 0; k < HELD; ++k) {
+    const int i = tid + k * NT, p = who[k] >= 0 ? off[who[k]] + rank[k] : -1;
+    if (p >= 0) sorted[p] = i;
+    if (pos != nullptr && i < n_slots) pos[i] = p;
+  }
+  if (n_slots <= HELD * NT) return;   // (uniform)
+  __syncthreads();
+  for (int e = tid; e < E; e += NT) more[e] = 0;
+  __syncthreads();
+  for (int i = tid + HELD * NT; i < n_slots; i += NT) {
     const int e = idx[i];
     if (e >= 0 && e < E) {
-      const int p = off[e] + atomicAdd(&cnt[e], 1);
+      const int p = off[e] + cnt[e] + atomicAdd(&more[e], 1);
       sorted[p] = i;
       if (pos != nullptr) pos[i] = p;
     } else if (pos != nullptr) {
@@ -527,15 +586,24 @@ BCG_API int bcg_moe_route_table(const void* tokens, const void* table, int vocab
 }
 
 // Position tiles of `tm` rows.  sorted: [cap] with cap = n_tiles * tm >= n_slots + E (tm - 1); tile_expert: [n_tiles];
-// pos (may be null): [n_slots], every slot's position; used (may be null): [1], the tiles that hold slots.
-BCG_API int bcg_moe_align(const void* idx, int n_slots, int E, void* sorted, int cap, void* tile_expert, int n_tiles, int tm,
-                          void* pos, void* used, void* stream) {
+// pos (may be null): [n_slots], every slot's position; used (may be null): [1], the tiles that hold slots.  table (may be null): idx [n_slots / top,
+// top] is written from its rows `tokens` first (bcg_moe_route_table).
+BCG_API int bcg_moe_align(void* idx, int n_slots, int E, void* sorted, int cap, void* tile_expert, int n_tiles, int tm,
+                          void* pos, void* used, const void* tokens, const void* table, int vocab, int width, int top, void* stream) {
   if (n_slots <= 0) return 0;
   if (E < 1 || E > MAX_E || tm < 1 || cap != n_tiles * tm || cap < n_slots + E * (tm - 1)) return -2;
-  align_kernel<<<1, 1024, 0, static_cast<hipStream_t>(stream)>>>(static_cast<const int*>(idx), n_slots, E,
-                                                                 static_cast<int*>(sorted), cap,
-                                                                 static_cast<int*>(tile_expert), n_tiles, tm,
-                                                                 static_cast<int*>(pos), static_cast<int*>(used));
+  if (table != nullptr && (tokens == nullptr || vocab < 1 || top < 1 || top > width || n_slots % top)) return -2;
+  const TableRoute by{static_cast<const int*>(tokens), static_cast<const int*>(table), vocab, width, top};
+#define BCG_ALIGN(HELD)                                                                                                                        \
+  align_kernel<HELD><<<1, 1024, 0, static_cast<hipStream_t>(stream)>>>(static_cast<int*>(idx), n_slots, E, static_cast<int*>(sorted), cap,      \
+                                                                       static_cast<int*>(tile_expert), n_tiles, tm, static_cast<int*>(pos), \
+                                                                       static_cast<int*>(used), by)
+  // (16 per thread cost 2 us more where one is all.  us, every slot read and counted twice -> held: 128 slots 3.3 -> 3.1, 2000 4.3 -> 3.9, 4096
+  // 5.5 -> 4.4, 16366 12.4 -> 10.9, bound by the counters' atomics)
+  if (n_slots <= 1024) BCG_ALIGN(1);
+  else if (n_slots <= 4096) BCG_ALIGN(4);
+  else BCG_ALIGN(16);
+#undef BCG_ALIGN
   return BCG_CHECK_LAUNCH();
 }
 
