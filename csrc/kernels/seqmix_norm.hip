@@ -73,7 +73,8 @@ __device__ __forceinline__ void narrow4(T* p, f32x4 v) {
 // The two row kernels with the row in registers (W a multiple of 4, at most 1024 CH; aligned rows): one pass over
 // memory, 4 columns per access, instead of scalar accesses and a second read of the stream.  Bound by memory for
 // many rows, by the latency of one row for few.  Measured (8183 rows of 2048, bf16): residual + norm of two parts 80 ->
-// 42 us (14 bytes per element: 5.6 TB/s), embedding 57 -> 31; 64 rows of 4096: 22 -> 7.7, 14.6 -> 6.4.
+// 39 us (14 bytes per element: 6.0 TB/s), embedding 57 -> 31; 64 rows of 4096: 22 -> 5.1, 14.6 -> 6.4.  (With the loads of a group of columns behind the
+// store of the one before, the residual's were 43 and 7.7.)
 template <typename T, int CH>
 __global__ __launch_bounds__(NT) void embed_scale_norm_row_kernel(const int* __restrict__ tokens, const T* __restrict__ table,
                                                                   float scale, const float* __restrict__ add,
@@ -112,33 +113,53 @@ __global__ __launch_bounds__(NT) void residual_norm_row_kernel(float* __restrict
                                                                T* __restrict__ out, int W) {
   __shared__ float red[NT / 64];
   const size_t base = static_cast<size_t>(blockIdx.x) * W;
-  float g = 0.f;
-  if (pg != nullptr) g = 1.0f / (1.0f + expf(-gate[blockIdx.x]));
-  f32x4 v[CH];
+  // All loads of the row are asked for before the first is used (columns past W: the row's last four again, which are not stored).
+  int at[CH];
+#pragma unroll
+  for (int c = 0; c < CH; ++c) at[c] = min(4 * static_cast<int>(threadIdx.x + c * NT), W - 4);
+  f32x4 v[CH], s[CH], wv[CH];
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    v[c] = *reinterpret_cast<const f32x4*>(resid + base + at[c]);
+    s[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  auto add = [&](const auto* p, float f) {
+    f32x4 part[CH];
+#pragma unroll
+    for (int c = 0; c < CH; ++c) part[c] = widen4(p + base + at[c]);
+#pragma unroll
+    for (int c = 0; c < CH; ++c) s[c] += part[c] * f;
+  };
+  if (w != nullptr) {
+#pragma unroll
+    for (int c = 0; c < CH; ++c) wv[c] = *reinterpret_cast<const f32x4*>(w + at[c]);
+  }
+  if (p0 != nullptr && p1 != nullptr) {   // (the usual pair, without a wait between its two)
+    f32x4 part[2][CH];
+#pragma unroll
+    for (int c = 0; c < CH; ++c) part[0][c] = widen4(p0 + base + at[c]), part[1][c] = widen4(p1 + base + at[c]);
+#pragma unroll
+    for (int c = 0; c < CH; ++c) s[c] = part[0][c] + part[1][c];
+  } else {
+    if (p0 != nullptr) add(p0, 1.f);
+    if (p1 != nullptr) add(p1, 1.f);
+  }
+  if (pf != nullptr) add(pf, 1.f);
+  if (pg != nullptr) add(pg, 1.0f / (1.0f + expf(-gate[blockIdx.x])));
   float ss = 0.f;
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
-    const int i = 4 * (threadIdx.x + c * NT);
-    if (i < W) {
-      f32x4 s = {0.f, 0.f, 0.f, 0.f};
-      v[c] = *reinterpret_cast<const f32x4*>(resid + base + i);
-      if (p0 != nullptr) s = widen4<T>(p0 + base + i);
-      if (p1 != nullptr) s += widen4<T>(p1 + base + i);
-      if (pf != nullptr) s += *reinterpret_cast<const f32x4*>(pf + base + i);
-      if (pg != nullptr) s += widen4<T>(pg + base + i) * g;
-      v[c] += s;
-      *reinterpret_cast<f32x4*>(resid + base + i) = v[c];
+    if (4 * (threadIdx.x + c * NT) >= W) break;
+    v[c] += s[c];
+    *reinterpret_cast<f32x4*>(resid + base + at[c]) = v[c];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) ss += v[c][j] * v[c][j];
-    }
+    for (int j = 0; j < 4; ++j) ss += v[c][j] * v[c][j];
   }
   if (w == nullptr) return;
   const float r = 1.0f / sqrtf(block_sum(ss, red) / W + eps);
 #pragma unroll
-  for (int c = 0; c < CH; ++c) {
-    const int i = 4 * (threadIdx.x + c * NT);
-    if (i < W) narrow4<T>(out + base + i, v[c] * r * (*reinterpret_cast<const f32x4*>(w + i) + w_offset));
-  }
+  for (int c = 0; c < CH; ++c)
+    if (4 * (threadIdx.x + c * NT) < W) narrow4<T>(out + base + at[c], v[c] * r * (wv[c] + w_offset));
 }
 
 // x = table[token] + pos_table[position] (both of type T, summed in fp32), out = x rounded to T.
@@ -306,7 +327,9 @@ __global__ __launch_bounds__(NT) void rope_multi_kv_kernel(const T* __restrict__
 // computed once into LDS and serve all its heads and maps (the scalar form computed them per feature); a
 // thread turns a group of four features together with the group `half` further on.  TPB tokens per workgroup: 4 (a
 // wave each; four tokens on consecutive slots of one 4-key group write whole V groups) for large steps, 1 for small
-// ones.  8183 tokens, 16 / 4 heads of two 64-wide maps, bf16: 87 -> 35.5 us; 64 tokens, 32 / 8 heads: 15.9 -> 7.5.
+// ones, whose tokens are cut into slices as long as that makes no more than 512 workgroups: a slice finds the angles again, but has one
+// group of features and one value per thread (64 tokens, 32 / 8 heads of two 64-wide maps, bf16: 7.8 -> 5.9 us in four slices; scalar form
+// 15.9).  8183 tokens, 16 / 4 heads: 87 -> 35 us.
 constexpr int ANGLES = 128;   // pairs of a map in the LDS table
 
 template <typename T, int TPB>
@@ -323,6 +346,20 @@ __global__ __launch_bounds__(NT) void rope_multi_kv_vec_kernel(const T* __restri
   const bool live = t < n_tokens;
   const int tc = live ? t : n_tokens - 1;
   const float pos = static_cast<float>(positions[tc]);
+  const int step = TPB == 1 ? TPT * gridDim.y : TPT, first = tid + (TPB == 1 ? TPT * blockIdx.y : 0);   // this slice's work
+  const T* row = qkv + static_cast<size_t>(tc) * row_stride;
+  const int slot = live ? slots[tc] : -1;
+  const int blk = slot / BS, off = slot - blk * BS;
+  const bool kv_ok = slot >= 0 && blk < num_blocks;
+  const int KD = maps * dim, qw = n_q * KD, kw = n_kv * KD, vw = n_kv * vdim;
+  auto put_values = [&]() {
+    if (!kv_ok) return;
+    for (int idx = first; idx < vw; idx += step) {
+      const int g = idx / vdim, e = idx - g * vdim;
+      v_cache[(static_cast<size_t>(blk) * n_kv + g) * vdim * BS + (static_cast<size_t>(off >> 2) * vdim + e) * 4 + (off & 3)] = row[qw + kw + idx];
+    }
+  };
+  if constexpr (TPB == 1) put_values();   // (nothing to wait for but the slot)
   for (int i = tid; i < half; i += TPT) {
     float s, c;
     sincosf(pos * inv_freq[i], &s, &c);
@@ -330,11 +367,6 @@ __global__ __launch_bounds__(NT) void rope_multi_kv_vec_kernel(const T* __restri
     angle[sub][1][i] = s;
   }
   __syncthreads();
-  const T* row = qkv + static_cast<size_t>(tc) * row_stride;
-  const int slot = live ? slots[tc] : -1;
-  const int blk = slot / BS, off = slot - blk * BS;
-  const bool kv_ok = slot >= 0 && blk < num_blocks;
-  const int KD = maps * dim, qw = n_q * KD, kw = n_kv * KD, vw = n_kv * vdim;
   if (live) {
     const int hg = half >> 2, per = (dim - half) >> 2;   // turned groups, and groups of work, of a map
     const int jobs = (n_q + n_kv) * maps * per;
@@ -346,7 +378,7 @@ __global__ __launch_bounds__(NT) void rope_multi_kv_vec_kernel(const T* __restri
         narrow4<T>(k_cache + (static_cast<size_t>(blk) * n_kv + g) * BS * KD + (static_cast<size_t>(f >> 2) * BS + off) * 4, v);
       }
     };
-    for (int job = tid; job < jobs; job += TPT) {
+    for (int job = first; job < jobs; job += step) {
       const int map = job / per, u = job - map * per;
       if (u < hg) {
         const int idx = map * dim + 4 * u;
@@ -382,12 +414,7 @@ __global__ __launch_bounds__(NT) void rope_multi_kv_vec_kernel(const T* __restri
       }
       return;
     }
-  }
-  if (kv_ok) {
-    for (int idx = tid; idx < vw; idx += TPT) {
-      const int g = idx / vdim, e = idx - g * vdim;
-      v_cache[(static_cast<size_t>(blk) * n_kv + g) * vdim * BS + (static_cast<size_t>(off >> 2) * vdim + e) * 4 + (off & 3)] = row[qw + kw + idx];
-    }
+    put_values();
   }
 }
 
@@ -514,8 +541,11 @@ BCG_API int bcg_rope_multi_kv_write(const void* qkv, int64_t row_stride, const v
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (half >= 0 && half <= ANGLES && 2 * half <= dim && half % 4 == 0 && dim % 4 == 0 && vdim % 4 == 0 && row_stride % 4 == 0 &&
       BS % 4 == 0 && aligned(16, {q_out, k_cache, v_cache}) && aligned(is_f32 ? 16 : 8, {qkv})) {
+    // (groups of four features turned, or the values, of a token over the workgroups that the CUs have room for; see the kernel)
+    const int work = std::max((n_q + n_kv) * maps * ((dim - half) / 4), n_kv * vdim);
+    const int slices = std::max(1, std::min((work + NT - 1) / NT, 512 / T_));
 #define BCG_ROPE_VEC(TYPE, TPB)                                                                                               \
-  rope_multi_kv_vec_kernel<TYPE, TPB><<<(T_ + TPB - 1) / TPB, NT, 0, s>>>(                                                    \
+  rope_multi_kv_vec_kernel<TYPE, TPB><<<dim3((T_ + TPB - 1) / TPB, TPB == 1 ? slices : 1), NT, 0, s>>>(                                                    \
       static_cast<const TYPE*>(qkv), row_stride, static_cast<const int*>(positions), static_cast<const int*>(slots),          \
       static_cast<const float*>(inv_freq), half, static_cast<TYPE*>(q_out), static_cast<TYPE*>(k_cache),                      \
       static_cast<TYPE*>(v_cache), n_q, n_kv, maps, dim, vdim, BS, num_blocks, T_)
