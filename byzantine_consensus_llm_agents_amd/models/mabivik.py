@@ -37,7 +37,7 @@ Kernel plan of one layer (HIP backend; the torch backend runs the same ops from
                       gated_state_scan -> gated_group_norm -> o GEMM
     feed-forward      table_experts_post_norm: routes by table, grouped expert GEMMs (gated epilogue), their sum into the stream
     residual_post_norm  x += post(y) fused with the next reader's norm (or a rounded copy of x)
-    token input       G GEMM -> gelu_gather_mul -> P GEMM -> residual_post_norm (rms)
+    token input       linear_gelu_table (G GEMM, gelu, embedding) -> P GEMM -> residual_post_norm (rms)
 
 No host synchronisation anywhere: a decode step is capturable in a HIP graph.
 """
@@ -346,7 +346,7 @@ class MabivikModel:
             else:
                 h = ops.residual_post_norm(x, y, L["post1"], after, dt)
             if c.side_dim:
-                z = ops.gelu_gather_mul(ops.linear(h, L["side_gate"]), tokens, self.side_embed, i * c.side_dim)
+                z = ops.linear_gelu_table(h, L["side_gate"], tokens, self.side_embed, i * c.side_dim)
                 h = ops.residual_post_norm(x, ops.linear(z, L["side_proj"]), L["side_post"], nxt, dt)
             if trace is not None:
                 trace.append(x.clone())

@@ -68,6 +68,7 @@ def _torch_ops() -> SimpleNamespace:
         moe_table_route=_ref.moe_table_route,
         table_experts_post_norm=_ref.table_experts_post_norm,
         gelu_gather_mul=_ref.gelu_gather_mul,
+        linear_gelu_table=_ref.linear_gelu_table,
         gated_act=_ref.gated_act,
         linear_clamped_glu=_ref.linear_clamped_glu,
         hyper_embed_norm=_ref.hyper_embed_norm,

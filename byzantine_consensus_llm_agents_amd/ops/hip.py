@@ -118,6 +118,7 @@ def load_library(path: str = None) -> ctypes.CDLL:
         "bcg_gemm_mid_plan": [c_int] * 5,
         "bcg_gemm_mid_parts": [c_int] * 4 + [ctypes.POINTER(c_int)],
         "bcg_gemm_mid": [c_int, c_int] + [c_void_p] * 9 + [c_int] * 4 + [c_void_p],
+        "bcg_gemm_mid_act": [c_int] + [c_void_p] * 7 + [c_int] * 6 + [c_void_p],
         "bcg_gemm_tile": [c_int, ctypes.POINTER(c_int), ctypes.POINTER(c_int)],
         "bcg_gemm_num_cfgs": [],
         "bcg_embed_scale_rmsnorm": [c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_float, c_float, c_void_p, c_void_p,
@@ -562,6 +563,21 @@ def hip_ops() -> SimpleNamespace:
                                 _stream()), "gemm_mid")   # (at / 2 rows or features of 2 bytes)
         return out
 
+    def _gemm_mid_act(p, x, w, out, other, at=0, tokens=None, off=0):
+        """bcg_gemm_mid_act: at > 0, `other` takes the columns from `at` on through gelu; else gelu times columns off .. of the rows `tokens` of
+        the table `other`."""
+        M, K = x.shape
+        N = w.shape[0]
+        _log(M, N, K, 0, (MID_CFG, p))
+        ws = cnt = None
+        if p >> 8 > 1:
+            tiles = c_int()
+            ws = torch.empty(lib.bcg_gemm_mid_parts(p, 0, M, N, ctypes.byref(tiles)), dtype=torch.float32, device=x.device)
+            cnt = _counters(x.device)
+        _check(lib.bcg_gemm_mid_act(p, _p(x), _p(w), _p(out), other.data_ptr() + 2 * off, None if tokens is None else _p(tokens),
+                                    None if ws is None else _p(ws), None if cnt is None else _p(cnt), M, N, K, at,
+                                    0 if at else other.shape[1], 0 if at else other.shape[0], _stream()), "gemm_mid_act")
+
     def _pieces(x, w, epi, beside=None, shape=None):
         """Runs of rows and their choices (`GemmPlan.pieces`); beside: the bias or residual, of this shape.  Fewer rows than LARGE_M are
         one run whatever the operands are, so nothing is looked at there: a small eager step is bound by the host (24 layers of
@@ -786,16 +802,34 @@ def hip_ops() -> SimpleNamespace:
         return out
 
     def linear_tail_gelu(x, w, at):
-        """(y, hidden): y = linear(x, w) and None, or, where `GemmPlan.tail_tiles` says that one launch gains, the first `at` columns
-        of it and act_fn of the others, "gelu_tanh"."""
+        """(y, hidden): y = linear(x, w) and None, or, where one launch takes the activation along (`GemmPlan.tail_tiles`, the kernel for
+        tens to hundreds of rows), the first `at` columns of it and act_fn of the others, "gelu_tanh"."""
         M, K = x.shape
         N = w.shape[0]
-        if not (plan.tail_tiles(M, N, K, at) and _plain(x, w)):
+        tiles = plan.tail_tiles(M, N, K, at)
+        p = None if tiles or not (0 < at < N and at % 8 == 0) else _mid(x, w, 0)
+        if p is None and not (tiles and _plain(x, w)):
             return linear(x, w), None
         y = torch.empty(M, at, dtype=x.dtype, device=x.device)
         hidden = torch.empty(M, N - at, dtype=x.dtype, device=x.device)
-        _w4_act(6, x, w, y, hidden, at, 0.0)
+        if p is not None:
+            _gemm_mid_act(p, x, w, y, hidden, at=at)
+        else:
+            _w4_act(6, x, w, y, hidden, at, 0.0)
         return y, hidden
+
+    def linear_gelu_table(x, w, tokens, table, off):
+        """gelu_gather_mul(linear(x, w), tokens, table, off), in one launch where the kernel for tens to hundreds of rows takes the product."""
+        N = w.shape[0]
+        p = _mid(x, w, 0)
+        if p is None or not (table.dim() == 2 and table.dtype == x.dtype and table.device == x.device and table.is_contiguous() and bare(table)
+                             and table.shape[1] % 8 == 0 and off % 8 == 0 and 0 <= off <= table.shape[1] - N and table.data_ptr() % 16 == 0
+                             and tokens.dtype == torch.int32 and tokens.is_contiguous() and tokens.device == x.device
+                             and tokens.numel() == x.shape[0]):
+            return extra["gelu_gather_mul"](linear(x, w), tokens, table, off)
+        out = torch.empty(x.shape[0], N, dtype=x.dtype, device=x.device)
+        _gemm_mid_act(p, x, w, out, table, tokens=tokens, off=off)
+        return out
 
     def _norm_fusable(x, w_norm):
         return x.shape[0] <= SKINNY_NORM_ROWS and x.shape[1] <= 8192 and _plain_beside(w_norm, (x.shape[1],), x)
@@ -1048,7 +1082,7 @@ def hip_ops() -> SimpleNamespace:
 
     return SimpleNamespace(name="hip", **extra, rmsnorm_fp8=rmsnorm_fp8, embed_rmsnorm_fp8=embed_rmsnorm_fp8,
                            linear_fp8_residual=linear_fp8_residual, linear=linear, norm_linear=norm_linear, norm_linear_silu=norm_linear_silu, linear_silu=linear_silu, linear_residual=linear_residual,
-                           linear_clamped_glu=linear_clamped_glu, linear_tail_gelu=linear_tail_gelu,
+                           linear_clamped_glu=linear_clamped_glu, linear_tail_gelu=linear_tail_gelu, linear_gelu_table=linear_gelu_table,
                            gemm_nt=gemm_nt, gemm_plan=plan, prepare_device=prepare_device,
                            register_stream=register_stream, quant_fp8=quant_fp8, add_rmsnorm_fp8=add_rmsnorm_fp8,
                            silu_mul_fp8=silu_mul_fp8, linear_fp8=linear_fp8, gemm_nt_fp8=gemm_nt_fp8, fp8_cfg=fp8_cfg, rmsnorm=rmsnorm, add_rmsnorm=add_rmsnorm, silu_mul=silu_mul,

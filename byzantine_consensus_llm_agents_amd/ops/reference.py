@@ -994,6 +994,11 @@ def gelu_gather_mul(z, tokens, table, off: int):
     return (act_fn(z.float(), "gelu_tanh") * e).to(z.dtype)
 
 
+def linear_gelu_table(x, w, tokens, table, off: int):
+    """`gelu_gather_mul` of ``x W^T``."""
+    return gelu_gather_mul(torch.nn.functional.linear(x, w), tokens, table, off)
+
+
 def clamped_glu(both, limit: float):
     """``g sigmoid(1.702 g) (u + 1)`` for a stacked [gate | up] projection [rows, 2 n], the gate clamped from
     above and the up part from both sides at ``limit``; fp32 math, rounded once."""

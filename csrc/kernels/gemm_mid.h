@@ -33,7 +33,8 @@
 
 namespace {
 
-enum Epilogue { EPI_STORE = 0, EPI_SILU_MUL = 1, EPI_RESIDUAL = 2 };
+// EPI_TAIL_GELU: gelu on the columns from `at` on, which go to an output of their own; EPI_GELU_TABLE: gelu times a row's entry of a table
+enum Epilogue { EPI_STORE = 0, EPI_SILU_MUL = 1, EPI_RESIDUAL = 2, EPI_TAIL_GELU = 3, EPI_GELU_TABLE = 4 };
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef long i64x2 __attribute__((ext_vector_type(2)));
@@ -48,9 +49,18 @@ struct MidArgs {
   int* counters;
   const float *x_scale, *w_scale;
   int M, N, inter, blocks, m_tiles, n_tiles, split;   // inter: W's up rows behind its gate rows; blocks: of 128 bytes in a row of x and w
+  bf16_t* tail;          // EPI_TAIL_GELU: [M, N - at]
+  const bf16_t* table;   // EPI_GELU_TABLE: N columns of row tokens[m] (within 0 .. vocab - 1), rows `table_ld` apart
+  const int* tokens;
+  int at, table_ld, vocab;
 };
 
 __device__ __forceinline__ float silu(float g) { return g * __builtin_amdgcn_rcpf(1.f + __expf(-g)); }
+
+// tanh form: z sigmoid(2 u) is 0.5 z (1 + tanh(u))
+__device__ __forceinline__ float gelu(float z) {
+  return z * __builtin_amdgcn_rcpf(1.f + __expf(-1.5957691216057308f * (z + 0.044715f * z * z * z)));
+}
 
 // buffer descriptor words (base, stride 0, num_records, raw-buffer config), wave-uniform
 __device__ __forceinline__ i32x4 make_srd(const void* base, uint32_t bytes) {
@@ -73,7 +83,7 @@ template <int MT, int NT, int WM, int EPI, bool F8, bool SPLIT>
 __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_mid_kernel(const MidArgs a) {
   constexpr int WK = 4 / WM;
   static_assert(WM == 1 || (WM == 2 && MT % 2 == 0 && NT % 2 == 0), "waves and fetches");
-  static_assert(!F8 || EPI != EPI_SILU_MUL, "fp8: store / residual epilogues");
+  static_assert(!F8 || EPI == EPI_STORE || EPI == EPI_RESIDUAL, "fp8: store / residual epilogues");
   static_assert(EPI != EPI_SILU_MUL || NT % 2 == 0, "gate and up blocks alternate");
   constexpr int U = MT + NT, MW = MT / WM, NB = MW * NT, F = MW + NT;
   static_assert(NB <= 64, "accumulators: the accumulation registers");
@@ -94,7 +104,7 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
   const int r_id = (xcd < rem ? xcd * (q + 1) : rem * (q + 1) + (xcd - rem) * q) + (bid >> 3);
   const int m_tile = r_id % a.m_tiles, rest = r_id / a.m_tiles;
   const int n_tile = rest % a.n_tiles, split = rest / a.n_tiles;
-  const int width = EPI == EPI_SILU_MUL ? a.N / 2 : a.N, ld = EPI == EPI_SILU_MUL ? a.inter : a.N;   // columns written, of a row
+  const int width = EPI == EPI_SILU_MUL ? a.N / 2 : a.N, ld = EPI == EPI_SILU_MUL ? a.inter : EPI == EPI_TAIL_GELU ? a.at : a.N;   // columns written, of a row
   const int m0 = m_tile * MT * 16, n0 = n_tile * NT * (EPI == EPI_SILU_MUL ? 8 : 16);   // gated: the first feature
   const uint32_t row_bytes = static_cast<uint32_t>(a.blocks) * 128;
   const int kb0 = split * a.blocks / a.split, nb = (split + 1) * a.blocks / a.split - kb0;
@@ -261,12 +271,16 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
   const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(a.c + corner, 0, rows * ldb, 0x00020000);
   const __amdgpu_buffer_rsrc_t rr = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(EPI == EPI_RESIDUAL ? a.residual + corner : a.c), 0,
                                                                       EPI == EPI_RESIDUAL ? rows * ldb : 0, 0x00020000);
+  const uint32_t ldt = static_cast<uint32_t>(EPI == EPI_TAIL_GELU ? a.N - a.at : 0) * 2;
+  const __amdgpu_buffer_rsrc_t rt = __builtin_amdgcn_make_buffer_rsrc(EPI == EPI_TAIL_GELU ? a.tail + static_cast<size_t>(m0) * (a.N - a.at) : a.c, 0,
+                                                                      rows * ldt, 0x00020000);
   const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(a.bias), 0, a.bias ? ldb : 0, 0x00020000);
   struct Item {
     uint32_t off, boff;   // bytes from the tile's corner, from the row's start
     bf16x8 r, b;
     float xs;
     f32x4 ws[2];
+    bool tail;
   };
   auto load8 = [&](const __amdgpu_buffer_rsrc_t& rsrc, uint32_t off) { return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, 0, 0)); };
   // (past the rows or the width an offset past every range: stores are dropped, loads are 0)
@@ -274,12 +288,17 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
     Item t;
     const int c = n0 + ci * 8;
     t.boff = c < width ? c * 2 : 0x80000000u;
-    t.off = c < width && row < rows ? row * ldb + c * 2 : 0x80000000u;
+    t.tail = EPI == EPI_TAIL_GELU && c >= a.at;   // (at is a multiple of 8: an item lies on one side)
+    t.off = c < width && row < rows ? t.tail ? row * ldt + (c - a.at) * 2 : row * ldb + c * 2 : 0x80000000u;
     return t;
   };
   auto load = [&](Item& t, int row) {
     if constexpr (EPI == EPI_RESIDUAL) t.r = load8(rr, t.off);
-    if constexpr (EPI != EPI_SILU_MUL) t.b = load8(rb, t.boff);
+    if constexpr (EPI == EPI_GELU_TABLE) {
+      const int token = min(max(a.tokens[m0 + min(row, rows - 1)], 0), a.vocab - 1);
+      t.r = *reinterpret_cast<const bf16x8*>(a.table + static_cast<size_t>(token) * a.table_ld + min(t.boff >> 1, static_cast<uint32_t>(width) - 8));
+    }
+    if constexpr (EPI == EPI_STORE || EPI == EPI_RESIDUAL) t.b = load8(rb, t.boff);
     if constexpr (F8) {
       t.xs = a.x_scale[m0 + min(row, rows - 1)];
       const f32x4* p = reinterpret_cast<const f32x4*>(a.w_scale + min(t.boff >> 1, static_cast<uint32_t>(width) - 8));
@@ -293,6 +312,10 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
       float y = v[e >> 2][e & 3];
       if constexpr (EPI == EPI_SILU_MUL) {
         y = silu(y) * v[2 + (e >> 2)][e & 3];
+      } else if constexpr (EPI == EPI_GELU_TABLE) {
+        y = gelu(y) * static_cast<float>(t.r[e]);
+      } else if constexpr (EPI == EPI_TAIL_GELU) {
+        if (t.tail) y = gelu(y);
       } else {
         if constexpr (F8) y *= t.xs * t.ws[e >> 2][e & 3];
         y += static_cast<float>(t.b[e]);
@@ -300,7 +323,8 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
       }
       o[e] = static_cast<__bf16>(y);
     }
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o), rc, t.off, 0, 0);
+    if (EPI == EPI_TAIL_GELU && t.tail) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o), rt, t.off, 0, 0);
+    else __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o), rc, t.off, 0, 0);
   };
 #pragma unroll
   for (int ph = 0; ph < PH; ++ph) {
