@@ -14,7 +14,7 @@
 // One workgroup per row; the row max is a wave64 shuffle reduction plus one partial per wave in
 // LDS.  Rows are held in registers between the reduction and the store (one pass over memory).  A step of
 // few rows is the latency of one row: 1024 threads per row there (up to WIDE_T rows; 20 rows of 2 x 16384 silu_mul: 18.1
-// -> 6.9 us, 6144-wide norm 7.6 -> 5.1), 256 beyond, where several rows share a CU.
+// -> 6.9 us, 6144-wide norm 7.6 -> 5.0), 256 beyond, where several rows share a CU.
 
 #include "common.h"
 
@@ -89,20 +89,29 @@ __global__ __launch_bounds__(TH) void add_rmsnorm_fp8_kernel(
   const size_t base = static_cast<size_t>(blockIdx.x) * H;
   // x row: the gathered table row (embedding lookup fused in) or this block's row
   const bf16_t* __restrict__ xr = gather ? x + static_cast<size_t>(gather[blockIdx.x]) * H : x + base;
+  // (all loads before the first use, as the bf16 form)
+  u16x8 xv[CHUNKS], rv[CHUNKS], wv[CHUNKS];
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c) {
+    const int at = min(tid + c * TH, nvec - 1) * 8;
+    xv[c] = *reinterpret_cast<const u16x8*>(xr + at);
+    wv[c] = *reinterpret_cast<const u16x8*>(w + at);
+  }
+  if (has_residual == 1) {
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) rv[c] = *reinterpret_cast<const u16x8*>(residual + base + min(tid + c * TH, nvec - 1) * 8);
+  }
   float v[CHUNKS][8];
   float ss = 0.f;
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c) {
     const int vi = tid + c * TH;
     if (vi < nvec) {
-      const u16x8 xv = *reinterpret_cast<const u16x8*>(xr + vi * 8);
-      u16x8 rv;
-      if (has_residual == 1) rv = *reinterpret_cast<const u16x8*>(residual + base + vi * 8);
       u16x8 nr;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        float f = bf2f(xv[j]);
-        if (has_residual == 1) f += bf2f(rv[j]);
+        float f = bf2f(xv[c][j]);
+        if (has_residual == 1) f += bf2f(rv[c][j]);
         nr[j] = f2bf(f);
         f = bf2f(nr[j]);
         v[c][j] = f;
@@ -124,10 +133,9 @@ __global__ __launch_bounds__(TH) void add_rmsnorm_fp8_kernel(
   for (int c = 0; c < CHUNKS; ++c) {
     const int vi = tid + c * TH;
     if (vi < nvec) {
-      const u16x8 wv = *reinterpret_cast<const u16x8*>(w + vi * 8);
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        v[c][j] = bf2f(f2bf(v[c][j] * inv * bf2f(wv[j])));  // the bf16 path's rounding
+        v[c][j] = bf2f(f2bf(v[c][j] * inv * bf2f(wv[c][j])));  // the bf16 path's rounding
         amax = fmaxf(amax, fabsf(v[c][j]));
       }
     }
