@@ -16,12 +16,9 @@ constexpr int WAVE = 64;
 
 __device__ __forceinline__ float bf2f(bf16_t v) { return __uint_as_float(static_cast<uint32_t>(v) << 16); }
 
-__device__ __forceinline__ bf16_t f2bf(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7f800000u) == 0x7f800000u) return static_cast<bf16_t>((u >> 16) | ((u & 0xffff) ? 0x40 : 0));
-  u += 0x7fffu + ((u >> 16) & 1u);  // round to nearest even
-  return static_cast<bf16_t>(u >> 16);
-}
+// round to nearest even by the hardware's conversion (one instruction; in integer arithmetic it was seven, a good part of what a
+// pass over a stream computes).  Infinities and NaN stay what they are, subnormal numbers are zeros as behind every operation of this build.
+__device__ __forceinline__ bf16_t f2bf(float f) { return __builtin_bit_cast(bf16_t, static_cast<__bf16>(f)); }
 
 template <typename T>
 __device__ __forceinline__ T wave_sum(T v) {
