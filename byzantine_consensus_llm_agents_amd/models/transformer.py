@@ -349,22 +349,33 @@ class DecoderModel:
         idx = meta.logits_idx
         return attn.index_select(0, idx), residual.index_select(0, idx)
 
-    def _attention(self, li, L, qkv, meta, k_cache, v_cache):
+    def _decode_order(self, meta, k_cache, v_cache):
+        """`ops.decode_order` for the layers' `decode_attention_pairs`, where more pairs than the CUs hold at once (512) take turns: a layer gains
+        2 to 3 % of its attention, 1 to 13 us, and the launch costs about 4.6 (`decode_order_kernel`)."""
+        if not (meta.decode and meta.cascade is None and hasattr(self.ops, "decode_order") and len(self.layers) >= 8 and self.hd in (64, 128)
+                and k_cache.dtype == v_cache.dtype == torch.bfloat16 and k_cache.shape[-2] == 16):
+            return None
+        lens = meta.seq_lens if meta.attn_seq_lens is None else meta.attn_seq_lens
+        if lens.numel() * self.n_kv <= 512 or lens.numel() > 2048 or lens.dtype != torch.int32 or not lens.is_contiguous():
+            return None
+        return self.ops.decode_order(lens)
+
+    def _attention(self, li, L, qkv, meta, k_cache, v_cache, order=None):
         ops, c = self.ops, self.cfg
         # (not with shared-prefix tables, which the engine passes with every decode step unless `cascade_decode` is off)
         if (meta.decode and meta.cascade is None and qkv.is_contiguous() and k_cache.dtype == v_cache.dtype == qkv.dtype == torch.bfloat16
                 and k_cache.shape[-2] == 16):
-            attend = None
+            attend, extra = None, {}
             if hasattr(ops, "decode_attention_pairs"):   # (its fetches are 16 bytes a lane)
                 if self.hd in (64, 128) and (k_cache.data_ptr() | v_cache.data_ptr() | qkv.data_ptr()) % 16 == 0:
-                    attend = ops.decode_attention_pairs
+                    attend, extra = ops.decode_attention_pairs, {} if order is None else {"order": order}
             elif (self.hd == 64 and hasattr(ops, "decode_attention")
                   and ops.decode_fused_pays(qkv.shape[0], self.n_kv, meta.block_tables.shape[1] * 16)):
                 attend = ops.decode_attention
             if attend is not None:
                 lens = meta.seq_lens if meta.attn_seq_lens is None else meta.attn_seq_lens
                 return attend(qkv, meta.positions, meta.slots, self.n_q, self.n_kv, self.hd, L.get("q_norm"), L.get("k_norm"), c.rms_eps,
-                              self.cos_sin, k_cache, v_cache, li, meta.block_tables, lens, self.scale, meta.workspace)
+                              self.cos_sin, k_cache, v_cache, li, meta.block_tables, lens, self.scale, meta.workspace, **extra)
         q = ops.qk_norm_rope_kv_write(qkv, meta.positions, meta.slots, self.n_q, self.n_kv, self.hd,
                                       L.get("q_norm"), L.get("k_norm"), c.rms_eps, self.cos_sin,
                                       k_cache, v_cache, li, contiguous=not meta.decode)
@@ -397,6 +408,7 @@ class DecoderModel:
         eps = c.rms_eps
         residual = x = h = hq = hs = None
         last = len(self.layers) - 1
+        order = self._decode_order(meta, k_cache, v_cache)
         for li, L in enumerate(self.layers):
             # ---- input norm (the previous layer's down projection is reduced here) ----
             if li == 0:
@@ -412,7 +424,7 @@ class DecoderModel:
                     hq, hs = ops.quant_fp8(h)
             qkv = (ops.linear_fp8(hq, hs, L["qkv"], L["qkv_s"], L.get("qkv_bias")) if fp8
                    else ops.linear(h, L["qkv"], L.get("qkv_bias")))
-            attn = self._attention(li, L, qkv, meta, k_cache, v_cache)
+            attn = self._attention(li, L, qkv, meta, k_cache, v_cache, order)
             if li == last and meta.logits_idx is not None:  # see _last_layer_rows
                 attn, residual = self._last_layer_rows(meta, attn, residual)
             # ---- o_proj, post-attention norm, MLP ----
@@ -455,13 +467,14 @@ class DecoderModel:
         ops, c = self.ops, self.cfg
         residual = None
         last = len(self.layers) - 1
+        order = self._decode_order(meta, k_cache, v_cache)
         for li, L in enumerate(self.layers):
             if li == 0:  # embedding gather fused with the first input norm
                 h, residual = ops.embed_rmsnorm(tokens, self.embed, L["ln1"], c.rms_eps)
                 qkv = ops.linear(h, L["qkv"], L.get("qkv_bias"))
             else:
                 qkv = ops.norm_linear(residual, L["ln1"], c.rms_eps, L["qkv"], L.get("qkv_bias"))
-            attn = self._attention(li, L, qkv, meta, k_cache, v_cache)
+            attn = self._attention(li, L, qkv, meta, k_cache, v_cache, order)
             if li == last and meta.logits_idx is not None:  # see _last_layer_rows
                 attn, residual = self._last_layer_rows(meta, attn, residual)
             residual = ops.linear_residual(attn, L["o"], residual)

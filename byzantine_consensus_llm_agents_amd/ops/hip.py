@@ -110,7 +110,8 @@ def load_library(path: str = None) -> ctypes.CDLL:
         "bcg_gemm_nt_fp8": [c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                             c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
         "bcg_decode_pairs": [c_void_p] * 6 + [c_float, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_void_p, c_int,
-                             c_int, c_int, c_int, c_float, c_int, c_void_p, c_void_p, c_void_p],
+                             c_int, c_int, c_int, c_float, c_int, c_void_p, c_void_p, c_void_p, c_void_p],
+        "bcg_decode_order": [c_void_p, c_int, c_void_p, c_void_p],
         "bcg_gemm_skinny": [c_int, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
                             c_void_p],
         "bcg_gemm_skinny_fp8": [c_int] + [c_void_p] * 7 + [c_int] * 3 + [c_void_p],
@@ -452,9 +453,10 @@ def hip_ops() -> SimpleNamespace:
                                       block_tables, seq_lens, scale, workspace)
 
     def decode_attention_pairs(qkv, positions, slots, n_q, n_kv, hd, q_norm, k_norm, eps, cos_sin, k_cache, v_cache, layer,
-                               block_tables, seq_lens, scale, workspace=None, parts=None):
+                               block_tables, seq_lens, scale, workspace=None, parts=None, order=None):
         """The same for heads of 64 or 128: a workgroup for each of `parts` parts of a (row, kv head) pair (default: `decode_parts`);
-        past one a second launch merges them, out of `workspace` where it holds B n_q parts (hd + 2) floats."""
+        past one a second launch merges them, out of `workspace` where it holds B n_q parts (hd + 2) floats.  order: `decode_order` of
+        seq_lens, the pairs' order over the launch."""
         B = qkv.shape[0]
         L, NB, nkv_c, BS, hdc = k_cache.shape
         _req(qkv.dtype == torch.bfloat16 and qkv.is_contiguous() and qkv.shape[1] == (n_q + 2 * n_kv) * hd, "decode qkv")
@@ -462,6 +464,7 @@ def hip_ops() -> SimpleNamespace:
              and not _kv_fp8(k_cache, v_cache), "decode kv cache layout")
         _req(all(t.dtype == torch.int32 and t.is_contiguous() for t in (positions, slots, seq_lens, block_tables))
              and positions.numel() == slots.numel() == seq_lens.numel() == B and block_tables.shape[0] == B, "decode tables")
+        _req(order is None or (order.dtype == torch.int32 and order.is_contiguous() and order.numel() == B and order.device == qkv.device), "decode order")
         _req(cos_sin.dtype == torch.float32 and cos_sin.shape[1] == hd and B <= 2048, "decode cos_sin / rows")
         if parts is None:
             parts = decode_parts(B, n_kv, hd, block_tables.shape[1] * BS)
@@ -474,8 +477,15 @@ def hip_ops() -> SimpleNamespace:
         _check(lib.bcg_decode_pairs(
             _p(qkv), _p(positions), _p(slots), None if q_norm is None else _p(q_norm), None if k_norm is None else _p(k_norm),
             _p(cos_sin), eps, _p(k_cache), _p(v_cache), layer, NB, n_kv, _p(block_tables), block_tables.shape[1], _p(seq_lens), B, n_q, hd,
-            BS, scale, parts, _p(workspace) if need else None, _p(out), _stream()), "decode_attention_pairs")
+            BS, scale, parts, _p(workspace) if need else None, _p(out), None if order is None else _p(order), _stream()), "decode_attention_pairs")
         return out
+
+    def decode_order(seq_lens):
+        """The rows of a decode step, longest context first (int32): one launch for all layers' `decode_attention_pairs`."""
+        _req(seq_lens.dtype == torch.int32 and seq_lens.is_contiguous() and 0 < seq_lens.numel() <= 2048, "decode order: seq_lens int32 [B]")
+        order = torch.empty_like(seq_lens)
+        _check(lib.bcg_decode_order(_p(seq_lens), seq_lens.numel(), _p(order), _stream()), "decode_order")
+        return order
 
     def paged_attention_prefill(q, k_cache, v_cache, layer, block_tables, q_start, seq_lens, scale,
                                 max_q_len=None, tiles=None, tile_rows=64):
@@ -1089,7 +1099,7 @@ def hip_ops() -> SimpleNamespace:
                            embed_rmsnorm=embed_rmsnorm,
                            qk_norm_rope_kv_write=qk_norm_rope_kv_write,
                            paged_attention_decode=paged_attention_decode,
-                           decode_attention=decode_attention, decode_attention_pairs=decode_attention_pairs,
+                           decode_attention=decode_attention, decode_attention_pairs=decode_attention_pairs, decode_order=decode_order,
                            decode_workspace_numel=decode_workspace_numel,
                            decode_max_context=lambda cascade=True: lib.bcg_decode_max_context(int(cascade)),
                            paged_attention_prefill=paged_attention_prefill,

@@ -865,16 +865,17 @@ struct Pair {
 template <int HD, int NW>
 __global__ __launch_bounds__(64 * NW, HD == 64 ? 4 : 2) void decode_pair_kernel(
     KVGeom g, const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ seq_lens, int n_q, float scale_log2, int parts,
-    float* __restrict__ part_o, float* __restrict__ part_ml, bf16_t* __restrict__ out, FusedArgs fa) {
+    float* __restrict__ part_o, float* __restrict__ part_ml, bf16_t* __restrict__ out, FusedArgs fa, const int* __restrict__ order) {
   constexpr int KP = Pair<HD, NW>::PIECES, RING = Pair<HD, NW>::RING, PAGE = HD * BS * 2;
   __shared__ __attribute__((aligned(1024))) unsigned char smem[Pair<HD, NW>::LDS];
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, h = lane >> 4;
   const int pair = blockIdx.x / parts, part = blockIdx.x - pair * parts;
-  const int b = pair / g.n_kv, kvh = pair - b * g.n_kv, G = n_q / g.n_kv;
   // (constant address space: scalar loads, whose wait is not one for the fetches)
   typedef const __attribute__((address_space(4))) int* Ints;
   auto ints = [](const int* p) { return reinterpret_cast<Ints>(reinterpret_cast<uintptr_t>(p)); };
+  const int at_row = pair / g.n_kv, kvh = pair - at_row * g.n_kv, G = n_q / g.n_kv;
+  const int b = order ? ints(order)[at_row] : at_row;
   const Ints table = ints(block_tables) + static_cast<size_t>(b) * max_blocks;
   const int ctx = min(ints(seq_lens)[b], max_blocks * BS), slot = ints(fa.slots)[b];
   const int all = (ctx + CHUNK - 1) / CHUNK, last = max(ctx - 1, 0) / BS;
@@ -1060,6 +1061,24 @@ __global__ __launch_bounds__(64 * NW, HD == 64 ? 4 : 2) void decode_pair_kernel(
     if (parts == 1) out[head * HD + d] = f2bf(oo * fac[NW * 16 + qi]);
     else part_o[(head * parts + part) * HD + d] = oo;
   }
+}
+
+// Rows by their lengths, longest first (equal ones in their order): where more pairs than the CUs hold at once come in the batch's order, the launch ends
+// with whichever long ones came late.  us, order of the batch and this (spread by 30 % to either side, heads of 128, 8 kv heads): 101 rows
+// of 1000 tokens 86.8, 83.9; 200 of 500 93.2, 91.1; 448 of 1050 375, 362; 64 of 1000, all resident, 55.8, 54.8.  One launch a step, about 4.6 us.
+__global__ __launch_bounds__(256) void decode_order_kernel(const int* __restrict__ seq_lens, int B, int* __restrict__ order) {
+  __shared__ int before[4][64];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), row = blockIdx.x * 64 + lane;
+  const int own = seq_lens[min(row, B - 1)];
+  int n = 0;
+#pragma unroll 8
+  for (int j = w * B / 4; j < (w + 1) * B / 4; ++j) {
+    const int other = seq_lens[j];
+    n += other > own || (other == own && j < row);
+  }
+  before[w][lane] = n;
+  __syncthreads();
+  if (w == 0 && row < B) order[before[0][lane] + before[1][lane] + before[2][lane] + before[3][lane]] = row;
 }
 
 // Split merge: one wave per (row, query head), four per workgroup.  Lane s holds split s's
@@ -1970,11 +1989,11 @@ BCG_API int bcg_paged_attention_decode(const void* q, const void* k_cache, const
 
 // Rotary embedding, cache write and attention of a decode step (decode_pair_kernel): qkv [B, n_q + 2 n_kv, hd] as projected, one new token per row
 // at `slots`; bf16 caches, hd 64 or 128.  `parts` workgroups take a (row, kv head) pair; workspace: B n_q parts (hd + 2) floats, of one part
-// none.
+// none.  order: of the rows over the launch, a permutation (bcg_decode_order), or null.
 BCG_API int bcg_decode_pairs(const void* qkv, const int* positions, const int* slots, const void* q_norm, const void* k_norm,
                              const float* cos_sin, float eps, void* k_cache, void* v_cache, int layer, int num_blocks, int n_kv,
                              const int* block_tables, int max_blocks, const int* seq_lens, int B, int n_q, int hd, int block_size,
-                             float scale, int parts, float* workspace, void* out, hipStream_t stream) {
+                             float scale, int parts, float* workspace, void* out, const int* order, hipStream_t stream) {
   if ((hd != 64 && hd != 128) || block_size != BS || n_kv <= 0 || n_q % n_kv || n_q / n_kv > 16 || B <= 0 || B > DEC_MAX_B || max_blocks <= 0) return -2;
   if (parts < 1 || parts > 64 || (parts > 1 && !workspace) || max_blocks * BS > bcg_decode_max_context(0)) return -3;
   const KVGeom g{static_cast<const bf16_t*>(k_cache), static_cast<const bf16_t*>(v_cache), layer, num_blocks, n_kv};
@@ -1985,7 +2004,7 @@ BCG_API int bcg_decode_pairs(const void* qkv, const int* positions, const int* s
     float* part_ml = workspace + static_cast<size_t>(B) * n_q * parts * HD;
     bf16_t* o = static_cast<bf16_t*>(out);
     hipLaunchKernelGGL((decode_pair_kernel<HD, NW>), dim3(B * n_kv * parts), dim3(64 * NW), 0, stream, g, block_tables, max_blocks, seq_lens,
-                       n_q, scale * LOG2E, parts, workspace, part_ml, o, fa);
+                       n_q, scale * LOG2E, parts, workspace, part_ml, o, fa, order);
     if (parts > 1)
       hipLaunchKernelGGL((decode_combine_kernel<HD, false>), dim3((B * n_q + COMBINE_WAVES - 1) / COMBINE_WAVES), dim3(64 * COMBINE_WAVES), 0, stream,
                          workspace, part_ml, seq_lens, n_q, parts, 0, B * n_q, o, nullptr, nullptr);
@@ -1996,6 +2015,13 @@ BCG_API int bcg_decode_pairs(const void* qkv, const int* positions, const int* s
     many ? run(integral_constant<int, 64>{}, integral_constant<int, 4>{}) : run(integral_constant<int, 64>{}, integral_constant<int, 8>{});
   else
     many ? run(integral_constant<int, 128>{}, integral_constant<int, 2>{}) : run(integral_constant<int, 128>{}, integral_constant<int, 4>{});
+  return BCG_CHECK_LAUNCH();
+}
+
+// order [B] = the rows, longest context first
+BCG_API int bcg_decode_order(const int* seq_lens, int B, int* order, hipStream_t stream) {
+  if (B <= 0 || B > DEC_MAX_B) return -2;
+  hipLaunchKernelGGL(decode_order_kernel, dim3((B + 63) / 64), dim3(256), 0, stream, seq_lens, B, order);
   return BCG_CHECK_LAUNCH();
 }
 
