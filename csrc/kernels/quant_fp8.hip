@@ -45,12 +45,24 @@ __device__ __forceinline__ float block_max(float v, float* red) {
 
 __device__ __forceinline__ float row_scale(float amax) { return fmaxf(amax, 1e-12f) / FP8_MAX; }
 
-// store 8 quantised values (8 bytes); inv: of the row's scale, divided once (a division is ten instructions, and a step of few rows is one
-// workgroup's arithmetic per row; a value within 2^-23 of a tie between two of e4m3's may round the other way)
-__device__ __forceinline__ void store_q8(uint8_t* dst, const float (&y)[8], float inv) {
+// A row's scale and what its values are divided with: a division is ten instructions, and a step of few rows is one workgroup's arithmetic per
+// row, so the row divides once and a value takes the reciprocal and one residual step, three instructions.  The quotient has the
+// division's bits (for every mantissa of a bf16 maximum and value): values and maxima of 8 bits make many
+// quotients exact ties between two of e4m3's values (up to 1 % of a row), which a bare reciprocal rounds either way, a whole e4m3 step apart.
+struct RowScale {
+  float s, inv, back;
+  __device__ explicit RowScale(float amax) : s(row_scale(amax)), inv(1.f / s), back(isinf(s) ? 0.f : s) {}   // (over infinity finite values are 0)
+  __device__ float over(float y) const {
+    const float q = y * inv;
+    return __builtin_fmaf(-__builtin_fmaf(q, back, -y), inv, q);   // (in these signs zeros keep theirs)
+  }
+};
+
+// store 8 quantised values (8 bytes)
+__device__ __forceinline__ void store_q8(uint8_t* dst, const float (&y)[8], const RowScale& r) {
   uint2 p;
-  p.x = pack4_fp8(clampq(y[0] * inv), clampq(y[1] * inv), clampq(y[2] * inv), clampq(y[3] * inv));
-  p.y = pack4_fp8(clampq(y[4] * inv), clampq(y[5] * inv), clampq(y[6] * inv), clampq(y[7] * inv));
+  p.x = pack4_fp8(clampq(r.over(y[0])), clampq(r.over(y[1])), clampq(r.over(y[2])), clampq(r.over(y[3])));
+  p.y = pack4_fp8(clampq(r.over(y[4])), clampq(r.over(y[5])), clampq(r.over(y[6])), clampq(r.over(y[7])));
   *reinterpret_cast<uint2*>(dst) = p;
 }
 
@@ -65,14 +77,14 @@ __global__ __launch_bounds__(QT) void quant_fp8_kernel(const bf16_t* __restrict_
 #pragma unroll
     for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(bf2f(v[j])));
   }
-  const float s = row_scale(block_max(amax, red)), inv = 1.f / s;
-  if (threadIdx.x == 0) scale[blockIdx.x] = s;
+  const RowScale r(block_max(amax, red));
+  if (threadIdx.x == 0) scale[blockIdx.x] = r.s;
   for (int vi = threadIdx.x; vi < nvec; vi += QT) {
     const u16x8 v = *reinterpret_cast<const u16x8*>(x + base + vi * 8);
     float y[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) y[j] = bf2f(v[j]);
-    store_q8(q + base + vi * 8, y, inv);
+    store_q8(q + base + vi * 8, y, r);
   }
 }
 
@@ -141,12 +153,12 @@ __global__ __launch_bounds__(TH) void add_rmsnorm_fp8_kernel(
       }
     }
   }
-  const float s = row_scale(block_max<TH>(amax, red)), inv = 1.f / s;
-  if (tid == 0) scale[blockIdx.x] = s;
+  const RowScale r(block_max<TH>(amax, red));
+  if (tid == 0) scale[blockIdx.x] = r.s;
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c) {
     const int vi = tid + c * TH;
-    if (vi < nvec) store_q8(q + base + vi * 8, v[c], inv);
+    if (vi < nvec) store_q8(q + base + vi * 8, v[c], r);
   }
 }
 
@@ -177,12 +189,12 @@ __global__ __launch_bounds__(TH) void silu_mul_fp8_kernel(const bf16_t* __restri
       for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(y[c][j]));
     }
   }
-  const float s = row_scale(block_max<TH>(amax, red)), inv = 1.f / s;
-  if (threadIdx.x == 0) scale[blockIdx.x] = s;
+  const RowScale r(block_max<TH>(amax, red));
+  if (threadIdx.x == 0) scale[blockIdx.x] = r.s;
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c) {
     const int vi = threadIdx.x + c * TH;
-    if (vi < nvec) store_q8(qrow + vi * 8, y[c], inv);
+    if (vi < nvec) store_q8(qrow + vi * 8, y[c], r);
   }
 }
 
@@ -200,12 +212,12 @@ __global__ __launch_bounds__(QT) void silu_mul_fp8_long_kernel(const bf16_t* __r
 #pragma unroll
     for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(y[j]));
   }
-  const float s = row_scale(block_max(amax, red)), inv = 1.f / s;
-  if (threadIdx.x == 0) scale[blockIdx.x] = s;
+  const RowScale r(block_max(amax, red));
+  if (threadIdx.x == 0) scale[blockIdx.x] = r.s;
   for (int vi = threadIdx.x; vi < nvec; vi += QT) {
     float y[8];
     silu8(row + vi * 8, y, I);
-    store_q8(qrow + vi * 8, y, inv);
+    store_q8(qrow + vi * 8, y, r);
   }
 }
 
