@@ -14,7 +14,7 @@
 // One workgroup per row; the row max is a wave64 shuffle reduction plus one partial per wave in
 // LDS.  Rows are held in registers between the reduction and the store (one pass over memory).  A step of
 // few rows is the latency of one row: 1024 threads per row there (up to WIDE_T rows; 20 rows of 2 x 16384 silu_mul: 18.1
-// -> 5.2 us (7.1 with a division per value), 6144-wide norm 7.6 -> 4.9), 256 beyond, where several rows share a CU.
+// -> 5.0 us (6.7 with a division per value for the quotients too), 6144-wide norm 7.6 -> 4.9), 256 beyond, where several rows share a CU.
 
 #include "common.h"
 
@@ -168,7 +168,7 @@ __device__ __forceinline__ void silu8(const bf16_t* g, float (&y)[8], int I) {
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
     const float a = bf2f(gv[j]);
-    y[j] = bf2f(f2bf(a * __builtin_amdgcn_rcpf(1.f + __expf(-a)) * bf2f(uv[j])));   // (1 ulp of 24 bits, rounded to 8)
+    y[j] = bf2f(f2bf(a / (1.f + __expf(-a)) * bf2f(uv[j])));
   }
 }
 

@@ -69,3 +69,12 @@ def test_infinite_maximum(hip):
     assert not (q.view(torch.uint8).cpu()[1, finite] & 0x7f).any()   # a finite value over infinity is zero
     keep = torch.tensor([0, 2])
     assert torch.equal(q.view(torch.uint8).cpu()[keep], _divided(x[keep])[0])
+
+
+def test_silu_is_divided(hip):
+    """silu(-88) u with u = 2^100: 1 + exp(88) has a reciprocal below the smallest normal number, the quotient has not."""
+    gu = torch.cat([torch.full((2, 64), -88.0), torch.full((2, 64), 2.0 ** 100)], 1).to(torch.bfloat16)
+    q, s = hip.silu_mul_fp8(gu.cuda())
+    want = -88.0 / (1.0 + torch.exp(torch.tensor(88.0, dtype=torch.float64))) * 2.0 ** 100
+    got = q.float().cpu().double() * s.cpu().double()[:, None]
+    assert ((got / want - 1.0).abs() < 2.0 ** -8).all()   # (the row's maximum: one rounding to bf16, 448 in e4m3)
