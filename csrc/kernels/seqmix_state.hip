@@ -35,12 +35,6 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
 }
 
 __device__ __forceinline__ float sigmoidf_(float z) { return 1.0f / (1.0f + expf(-z)); }
-// The same for a result that is rounded to T next: to 8 bits, the hardware's exponential and reciprocal (a few units of the last of 24 bits) instead
-// of the library's and a division, some 20 instructions.
-template <typename T> __device__ __forceinline__ float sigmoid_to(float z) {
-  if constexpr (sizeof(T) == 2) return __builtin_amdgcn_rcpf(1.0f + __expf(-z));
-  else return sigmoidf_(z);
-}
 
 // Factor of the query at position p: 1 + coef ln(floor((p + 1) / every) + 1) (every = 0: 1).
 __device__ __forceinline__ float query_temperature(int p, float coef, int every) {
@@ -209,7 +203,7 @@ __global__ __launch_bounds__(NT) void short_conv_vec_kernel(const T* __restrict_
     Vec o;
 #pragma unroll
     for (int e = 0; e < VEC; ++e) {
-      const float v = act == 1 ? acc[e] * sigmoid_to<T>(acc[e]) : acc[e];
+      const float v = act == 1 ? acc[e] * sigmoidf_(acc[e]) : acc[e];
       o.e[e] = Elem<T>::st(v);
     }
     *reinterpret_cast<Vec*>(out + static_cast<size_t>(t) * C + c) = o;
@@ -236,7 +230,7 @@ __global__ __launch_bounds__(NT) void short_conv_vec_kernel(const T* __restrict_
     finish(acc, t);
   };
   // CONV_ROWS rows deep inside one segment: every input once, all loads in flight at once (row by row each waits for its
-  // segment's tables; 8183 rows of 8704 channels, bf16: 109 us with one run a block, 80 with three: 3.6 TB/s; of 8192 92 and 77)
+  // segment's tables; 8183 rows of 8704 channels, bf16: 95 us, of 8192 91)
   if constexpr (!RUNS) {
     one_row(t_first);   // (a row per workgroup)
     return;
@@ -1113,7 +1107,7 @@ __global__ __launch_bounds__(NT) void head_norm_gate_vec_kernel(const float* __r
       for (int j = 0; j < 4; ++j) {
         if (gate != nullptr) {
           const float z = Elem<T>::ld(g[q][j]);
-          v[j] *= gate_kind == 0 ? sigmoid_to<T>(z) : z * sigmoid_to<T>(z);
+          v[j] *= gate_kind == 0 ? sigmoidf_(z) : z * sigmoidf_(z);
         }
         y[j] = Elem<T>::st(v[j]);
       }
