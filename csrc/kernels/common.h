@@ -17,7 +17,8 @@ constexpr int WAVE = 64;
 __device__ __forceinline__ float bf2f(bf16_t v) { return __uint_as_float(static_cast<uint32_t>(v) << 16); }
 
 // round to nearest even by the hardware's conversion (one instruction; in integer arithmetic it was seven, a good part of what a
-// pass over a stream computes).  Infinities and NaN stay what they are, subnormal numbers are zeros as behind every operation of this build.
+// pass over a stream computes).  Infinities and NaN stay what they are, subnormal numbers are zeros as behind every operation of this build (so a
+// value that is only passed on is copied as it is, not taken through here).
 __device__ __forceinline__ bf16_t f2bf(float f) { return __builtin_bit_cast(bf16_t, static_cast<__bf16>(f)); }
 
 template <typename T>

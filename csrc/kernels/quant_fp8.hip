@@ -125,7 +125,7 @@ __global__ __launch_bounds__(TH) void add_rmsnorm_fp8_kernel(
       for (int j = 0; j < 8; ++j) {
         float f = bf2f(xv[c][j]);
         if (has_residual == 1) f += bf2f(rv[c][j]);
-        nr[j] = f2bf(f);
+        nr[j] = has_residual == 1 ? f2bf(f) : xv[c][j];
         f = bf2f(nr[j]);
         v[c][j] = f;
         ss += f * f;

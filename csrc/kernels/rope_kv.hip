@@ -30,6 +30,13 @@ __device__ __forceinline__ uint8_t to_cache<uint8_t>(float f) {
   return static_cast<uint8_t>(__builtin_amdgcn_cvt_pk_fp8_f32(f, 0.f, 0, false) & 0xff);
 }
 
+// a value as it is (f2bf would make zeros of subnormal numbers)
+template <typename T>
+__device__ __forceinline__ T copy_to_cache(bf16_t v) {
+  if constexpr (sizeof(T) == 2) return v;
+  else return to_cache<T>(bf2f(v));
+}
+
 template <typename CacheT>
 __global__ __launch_bounds__(256) void qk_norm_rope_kv_kernel(
     const bf16_t* __restrict__ qkv, const int* __restrict__ positions, const int* __restrict__ slots,
@@ -55,8 +62,8 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kv_kernel(
     const int h = slot_head - n_q - n_kv;
     const size_t vbase = ((static_cast<size_t>(layer) * num_blocks + blk) * n_kv + h) * hd * block_size;
     if (active) {
-      v_cache[vbase + static_cast<size_t>(lane) * block_size + off] = to_cache<CacheT>(x1);
-      v_cache[vbase + static_cast<size_t>(lane + half) * block_size + off] = to_cache<CacheT>(x2);
+      v_cache[vbase + static_cast<size_t>(lane) * block_size + off] = copy_to_cache<CacheT>(src[lane]);
+      v_cache[vbase + static_cast<size_t>(lane + half) * block_size + off] = copy_to_cache<CacheT>(src[lane + half]);
     }
     return;
   }
@@ -119,8 +126,8 @@ __device__ __forceinline__ void rope_kv_token(
     CacheT* vb = v_cache + ((static_cast<size_t>(layer) * num_blocks + blk) * n_kv + h) * HD * block_size + off;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      vb[static_cast<size_t>(d0 + e) * block_size] = to_cache<CacheT>(x1[e]);
-      vb[static_cast<size_t>(HALF + d0 + e) * block_size] = to_cache<CacheT>(x2[e]);
+      vb[static_cast<size_t>(d0 + e) * block_size] = copy_to_cache<CacheT>(a[e]);
+      vb[static_cast<size_t>(HALF + d0 + e) * block_size] = copy_to_cache<CacheT>(bv[e]);
     }
     return;
   }

@@ -399,28 +399,27 @@ __global__ __launch_bounds__(NT) void latent_kv_write_kernel(const T* __restrict
   T* vs = v_cache + static_cast<size_t>(blk) * R * BS;
   const float pos = static_cast<float>(positions[t]);
   for (int i = lane; i < KD; i += 64) {
-    float val;
+    T c;
     if (i < R) {
-      val = Elem<T>::ld(row[i]) * r * w[i];
-      const T c = Elem<T>::st(val);
+      c = Elem<T>::st(Elem<T>::ld(row[i]) * r * w[i]);
       if (swz) vs[(static_cast<size_t>(o >> 2) * R + i) * 4 + (o & 3)] = c;
       else vs[static_cast<size_t>(i) * BS + o] = c;
     } else {
       const int j = i - R;
-      val = Elem<T>::ld(row[i]);
+      c = row[i];   // (as it is where it is not turned: st would make zeros of subnormal numbers)
       if (j < 2 * half) {
         const bool first = pairs ? (j & 1) == 0 : j < half;   // of the two features that turn together
         const int step = pairs ? 1 : half;
-        float s, c;
-        sincosf(pos * inv_freq[pairs ? j >> 1 : (first ? j : j - half)], &s, &c);
+        float s, cs;
+        sincosf(pos * inv_freq[pairs ? j >> 1 : (first ? j : j - half)], &s, &cs);
         s *= amp;
-        c *= amp;
-        const float other = Elem<T>::ld(row[first ? i + step : i - step]);
-        val = first ? val * c - other * s : val * c + other * s;
+        cs *= amp;
+        const float val = Elem<T>::ld(c), other = Elem<T>::ld(row[first ? i + step : i - step]);
+        c = Elem<T>::st(first ? val * cs - other * s : val * cs + other * s);
       }
     }
-    if (swz) ks[(static_cast<size_t>(i >> 2) * BS + o) * 4 + (i & 3)] = Elem<T>::st(val);
-    else ks[static_cast<size_t>(o) * KD + i] = Elem<T>::st(val);
+    if (swz) ks[(static_cast<size_t>(i >> 2) * BS + o) * 4 + (i & 3)] = c;
+    else ks[static_cast<size_t>(o) * KD + i] = c;
   }
 }
 

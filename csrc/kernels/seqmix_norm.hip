@@ -292,24 +292,25 @@ __global__ __launch_bounds__(NT) void rope_multi_kv_kernel(const T* __restrict__
   const int qw = n_q * maps * dim, kw = n_kv * maps * dim, vw = n_kv * vdim;
   for (int idx = threadIdx.x; idx < qw + kw; idx += NT) {
     const int i = idx % dim;
-    float val = Elem<T>::ld(row[idx]);
+    const float val = Elem<T>::ld(row[idx]);
+    T o = row[idx];   // (as it is where it is not turned: st would make zeros of subnormal numbers)
     if (i < 2 * half) {
       const bool lo = i < half;
       const float other = Elem<T>::ld(row[lo ? idx + half : idx - half]);
       float s, c;
       sincosf(pos * inv_freq[lo ? i : i - half], &s, &c);
-      val = lo ? val * c - other * s : val * c + other * s;
+      o = Elem<T>::st(lo ? val * c - other * s : val * c + other * s);
     }
     if (idx < qw) {
-      q_out[static_cast<size_t>(t) * qw + idx] = Elem<T>::st(val);
+      q_out[static_cast<size_t>(t) * qw + idx] = o;
     } else if (kv_ok) {
       const int kk = idx - qw;
       const int KD = maps * dim;
       const int g = kk / KD, f = kk - g * KD;
       T* slab = k_cache + (static_cast<size_t>(blk) * n_kv + g) * BS * KD;
       // KD % 4 == 0: fragment-major slab [KD / 4][BS][4] (seqmix_attention.hip); else [BS][KD]
-      if ((KD & 3) == 0) slab[(static_cast<size_t>(f >> 2) * BS + off) * 4 + (f & 3)] = Elem<T>::st(val);
-      else slab[static_cast<size_t>(off) * KD + f] = Elem<T>::st(val);
+      if ((KD & 3) == 0) slab[(static_cast<size_t>(f >> 2) * BS + off) * 4 + (f & 3)] = o;
+      else slab[static_cast<size_t>(off) * KD + f] = o;
     }
   }
   if (kv_ok) {
@@ -370,13 +371,13 @@ __global__ __launch_bounds__(NT) void rope_multi_kv_vec_kernel(const T* __restri
   if (live) {
     const int hg = half >> 2, per = (dim - half) >> 2;   // turned groups, and groups of work, of a map
     const int jobs = (n_q + n_kv) * maps * per;
+    auto place = [&](int idx) -> T* {   // (null: a key that no slot takes)
+      if (idx < qw) return q_out + static_cast<size_t>(t) * qw + idx;
+      const int kk = idx - qw, g = kk / KD, f = kk - g * KD;
+      return kv_ok ? k_cache + (static_cast<size_t>(blk) * n_kv + g) * BS * KD + (static_cast<size_t>(f >> 2) * BS + off) * 4 : nullptr;
+    };
     auto put = [&](int idx, f32x4 v) {
-      if (idx < qw) {
-        narrow4<T>(q_out + static_cast<size_t>(t) * qw + idx, v);
-      } else if (kv_ok) {
-        const int kk = idx - qw, g = kk / KD, f = kk - g * KD;
-        narrow4<T>(k_cache + (static_cast<size_t>(blk) * n_kv + g) * BS * KD + (static_cast<size_t>(f >> 2) * BS + off) * 4, v);
-      }
+      if (T* p = place(idx)) narrow4<T>(p, v);
     };
     for (int job = first; job < jobs; job += step) {
       const int map = job / per, u = job - map * per;
@@ -388,7 +389,7 @@ __global__ __launch_bounds__(NT) void rope_multi_kv_vec_kernel(const T* __restri
         put(idx + half, b * c + a * s);
       } else {
         const int idx = map * dim + half + 4 * u;
-        put(idx, widen4<T>(row + idx));
+        if (T* p = place(idx)) *reinterpret_cast<F*>(p) = *reinterpret_cast<const F*>(row + idx);   // (as they are)
       }
     }
   }

@@ -385,16 +385,16 @@ __global__ __launch_bounds__(NT) void rope_pairs_kv_kernel(const T* __restrict__
     const T* vrow = row + v_off;
     for (int idx = threadIdx.x; idx < vw; idx += NT) {
       const int g = idx / vdim, e = idx - g * vdim;
-      float val = Elem<T>::ld(vrow[idx]);
+      T o = vrow[idx];   // (as it is where it is not turned)
       if (v_inv_freq != nullptr) {
-        const float other = Elem<T>::ld(vrow[idx ^ 1]);
+        const float val = Elem<T>::ld(o), other = Elem<T>::ld(vrow[idx ^ 1]);
         float s, c;
         sincosf(pos * v_inv_freq[e >> 1], &s, &c);
-        val = (e & 1) ? val * c + other * s : val * c - other * s;
+        o = Elem<T>::st((e & 1) ? val * c + other * s : val * c - other * s);
       }
       T* slab = v_cache + (static_cast<size_t>(blk) * n_kv + g) * vdim * BS;
-      if (swz) slab[(static_cast<size_t>(off >> 2) * vdim + e) * 4 + (off & 3)] = Elem<T>::st(val);
-      else slab[static_cast<size_t>(e) * BS + off] = Elem<T>::st(val);
+      if (swz) slab[(static_cast<size_t>(off >> 2) * vdim + e) * 4 + (off & 3)] = o;
+      else slab[static_cast<size_t>(e) * BS + off] = o;
     }
   }
 }
