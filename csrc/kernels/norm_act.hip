@@ -86,6 +86,7 @@ __global__ __launch_bounds__(TH) void add_rmsnorm_kernel(
 // A step of few rows is the latency of one row: a vector per thread there; several rows share a CU beyond.
 int launch_norm(const void* x, void* residual, const void* w, void* out, int T, int H, float eps, int has_residual, const int* gather,
                 hipStream_t stream) {
+  if (H == 0) return 0;   // (the kernel reads a row's last vector)
 #define BCG_NORM(TH, CH)                                                                                                    \
   hipLaunchKernelGGL((add_rmsnorm_kernel<TH, CH>), dim3(T), dim3(TH), 0, stream, static_cast<const bf16_t*>(x),              \
                      static_cast<bf16_t*>(residual), static_cast<const bf16_t*>(w), static_cast<bf16_t*>(out), H, eps, has_residual, gather)

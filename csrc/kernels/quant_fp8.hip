@@ -18,6 +18,8 @@
 
 #include "common.h"
 
+BCG_API int bcg_quant_fp8(const void* x, void* q, float* scale, int T, int K, hipStream_t stream);
+
 namespace {
 
 constexpr int QT = 256;
@@ -223,6 +225,7 @@ __global__ __launch_bounds__(QT) void silu_mul_fp8_long_kernel(const bf16_t* __r
 
 int launch_norm(const void* x, void* residual, const void* w, void* q, float* scale, int T, int H, float eps, int has_residual,
                 const int* gather, hipStream_t stream) {
+  if (H == 0) return bcg_quant_fp8(x, q, scale, T, H, stream);   // (scales of nothing; the kernel reads a row's last vector)
 #define BCG_NORM_FP8(TH, CH)                                                                                                  \
   hipLaunchKernelGGL((add_rmsnorm_fp8_kernel<TH, CH>), dim3(T), dim3(TH), 0, stream, static_cast<const bf16_t*>(x),            \
                      static_cast<bf16_t*>(residual), static_cast<const bf16_t*>(w), static_cast<uint8_t*>(q), scale, H, eps,  \

@@ -481,7 +481,7 @@ BCG_API int bcg_residual_add_rmsnorm32(void* resid, const void* p0, const void* 
                                        int W, int is_f32, void* stream) {
   if (T_ <= 0) return 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (W % 4 == 0 && W <= 8192 && aligned(16, {resid, p0, p1, pf, pg, w, out})) {
+  if (W > 0 && W % 4 == 0 && W <= 8192 && aligned(16, {resid, p0, p1, pf, pg, w, out})) {   // (it reads a row's last four)
 #define BCG_RESIDUAL_ROW(TYPE, CH)                                                                                             \
   residual_norm_row_kernel<TYPE, CH><<<T_, NT, 0, s>>>(static_cast<float*>(resid), static_cast<const TYPE*>(p0),               \
                                                        static_cast<const TYPE*>(p1), static_cast<const float*>(pf),            \
