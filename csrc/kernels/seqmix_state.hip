@@ -174,13 +174,12 @@ __global__ __launch_bounds__(NT) void short_conv_kernel(const T* __restrict__ y,
 }
 
 // The same for VEC consecutive channels per thread (one 16-byte load per tap) and `rows`
-// consecutive rows per block (one to four runs of CONV_ROWS in large steps, where a thread's weights are worth keeping: a wave's lie in 512
-// lines, a row's channels in 8; one row in small steps, which need the blocks), the thread's TAPS x VEC weights in registers.  Needs C, the row
+// consecutive rows per block (CONV_ROWS in large steps, where a thread's weights are worth keeping;
+// one in small steps, which need the blocks), the thread's TAPS x VEC weights in registers.  Needs C, the row
 // strides and the base addresses to be multiples of VEC elements.
 constexpr int CONV_ROWS = 8;
 
-// (RUNS: of CONV_ROWS.  A small step's launch reads its code cold: without them 6.0 us for 64 rows of 4096 channels, 6.6 with.)
-template <typename T, int VEC, int TAPS, bool RUNS>
+template <typename T, int VEC, int TAPS>
 __global__ __launch_bounds__(NT) void short_conv_vec_kernel(const T* __restrict__ y, int64_t y_stride, int C,
                                                             const float* __restrict__ w, const int* __restrict__ positions,
                                                             const int* __restrict__ token_seq, const int* __restrict__ q_start,
@@ -208,7 +207,30 @@ __global__ __launch_bounds__(NT) void short_conv_vec_kernel(const T* __restrict_
     }
     *reinterpret_cast<Vec*>(out + static_cast<size_t>(t) * C + c) = o;
   };
-  auto one_row = [&](int t) {
+  // CONV_ROWS rows deep inside one segment: every input once, all loads in flight at once (row by row each waits for its
+  // segment's tables; 8183 rows of 8448 channels: 144 -> 103 us; more runs of them a workgroup, bf16: 8704 channels 92 -> 95, 8192 88 -> 91)
+  if (t_end - t_first == CONV_ROWS) {
+    const int seg = token_seq[t_first];
+    if (token_seq[t_end - 1] == seg && t_first - q_start[seg] >= TAPS - 1) {
+      Vec u[CONV_ROWS + TAPS - 1];
+#pragma unroll
+      for (int r = 0; r < CONV_ROWS + TAPS - 1; ++r)
+        u[r] = *reinterpret_cast<const Vec*>(y + static_cast<size_t>(t_first + r - (TAPS - 1)) * y_stride + c);
+#pragma unroll
+      for (int r = 0; r < CONV_ROWS; ++r) {
+        float acc[VEC];
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+          acc[e] = br[e];
+#pragma unroll
+          for (int j = 0; j < TAPS; ++j) acc[e] += wr[e][j] * Elem<T>::ld(u[r + j].e[e]);
+        }
+        finish(acc, t_first + r);
+      }
+      return;
+    }
+  }
+  for (int t = t_first; t < t_end; ++t) {
     const int seg = token_seq[t], off = t - q_start[seg], pos = positions[t];
     const int sr = state_rows[seg];
     const bool row_ok = sr >= 0 && sr < n_rows;
@@ -228,40 +250,6 @@ __global__ __launch_bounds__(NT) void short_conv_vec_kernel(const T* __restrict_
       }
     }
     finish(acc, t);
-  };
-  // CONV_ROWS rows deep inside one segment: every input once, all loads in flight at once (row by row each waits for its
-  // segment's tables; 8183 rows of 8704 channels, bf16: 95 us, of 8192 91)
-  if constexpr (!RUNS) {
-    one_row(t_first);   // (a row per workgroup)
-    return;
-  }
-#pragma unroll 1
-  for (int t = t_first; t < t_end; t += CONV_ROWS) {
-    bool inside = t_end - t >= CONV_ROWS;
-    if (inside) {
-      const int seg = token_seq[t];
-      inside = token_seq[t + CONV_ROWS - 1] == seg && t - q_start[seg] >= TAPS - 1;
-    }
-    if (!inside) {
-#pragma unroll 1
-      for (int r = t; r < min(t_end, t + CONV_ROWS); ++r) one_row(r);
-    } else {
-      Vec u[CONV_ROWS + TAPS - 1];
-#pragma unroll
-      for (int r = 0; r < CONV_ROWS + TAPS - 1; ++r)
-        u[r] = *reinterpret_cast<const Vec*>(y + static_cast<size_t>(t + r - (TAPS - 1)) * y_stride + c);
-#pragma unroll
-      for (int r = 0; r < CONV_ROWS; ++r) {
-        float acc[VEC];
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) {
-          acc[e] = br[e];
-#pragma unroll
-          for (int j = 0; j < TAPS; ++j) acc[e] += wr[e][j] * Elem<T>::ld(u[r + j].e[e]);
-        }
-        finish(acc, t + r);
-      }
-    }
   }
 }
 
@@ -271,18 +259,11 @@ bool launch_conv_vec(const T* y, int64_t y_stride, int C, const float* w, int ta
   constexpr int VEC = 16 / sizeof(T);
   const uintptr_t bits = reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(state) | reinterpret_cast<uintptr_t>(out);
   if (C % VEC || y_stride % VEC || bits % 16 || taps < 2 || taps > 4) return false;
-  // (a wave's weights are 512 lines, a row's channels 8: as many rows as leave five workgroups per CU)
-  const int cb = (C / VEC + NT - 1) / NT, runs = static_cast<int>(static_cast<int64_t>(T_ / CONV_ROWS) * cb / 1280);
-  const int rows = T_ >= 2048 ? CONV_ROWS * std::min(4, std::max(1, runs)) : 1;
-  dim3 grid((T_ + rows - 1) / rows, cb);
-#define BCG_CONV(TAPS, RUNS) \
-  short_conv_vec_kernel<T, VEC, TAPS, RUNS><<<grid, NT, 0, s>>>(y, y_stride, C, w, ps, ts, qs, sr, state, n_rows, out, act, T_, bias, rows)
-  if (rows == 1) {
-    if (taps == 2) BCG_CONV(2, false); else if (taps == 3) BCG_CONV(3, false); else BCG_CONV(4, false);
-  } else {
-    if (taps == 2) BCG_CONV(2, true); else if (taps == 3) BCG_CONV(3, true); else BCG_CONV(4, true);
-  }
-#undef BCG_CONV
+  const int rows = T_ >= 2048 ? CONV_ROWS : 1;
+  dim3 grid((T_ + rows - 1) / rows, (C / VEC + NT - 1) / NT);
+  if (taps == 2) short_conv_vec_kernel<T, VEC, 2><<<grid, NT, 0, s>>>(y, y_stride, C, w, ps, ts, qs, sr, state, n_rows, out, act, T_, bias, rows);
+  else if (taps == 3) short_conv_vec_kernel<T, VEC, 3><<<grid, NT, 0, s>>>(y, y_stride, C, w, ps, ts, qs, sr, state, n_rows, out, act, T_, bias, rows);
+  else short_conv_vec_kernel<T, VEC, 4><<<grid, NT, 0, s>>>(y, y_stride, C, w, ps, ts, qs, sr, state, n_rows, out, act, T_, bias, rows);
   return true;
 }
 

@@ -1,4 +1,4 @@
-"""Short convolutions of large, wide steps: several runs of rows a workgroup.  GPU only.  Bounds as in test_row_kernels_gpu.py."""
+"""Short convolutions of large, wide steps: runs of rows a workgroup.  GPU only.  Bounds as in test_row_kernels_gpu.py."""
 import pytest
 import torch
 
@@ -9,7 +9,7 @@ from test_row_kernels_gpu import _tol, ops  # noqa: F401
 pytestmark = pytest.mark.gpu
 
 
-# runs of 8 rows: two (bf16) and four (fp32) a workgroup, inside a segment, over its boundaries, behind its first rows, the last run short
+# runs of 8 rows inside a segment, over its boundaries, behind its first rows, the last run short
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("lens,starts", [([1501, 1, 2, 7, 1780, 9], [0, 4, 0, 3, 11, 0]), ([3296], [0]), ([3, 3294], [5, 1])])
 def test_runs_of_rows(ops, dtype, lens, starts):
