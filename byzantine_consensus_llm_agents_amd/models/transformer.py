@@ -353,6 +353,7 @@ class DecoderModel:
         """`ops.decode_order` for the layers' `decode_attention_pairs`, where more pairs than the CUs hold at once (512) take turns: a layer gains
         2 to 3 % of its attention, 1 to 13 us, and the launch costs about 4.6 (`decode_order_kernel`)."""
         if not (meta.decode and meta.cascade is None and hasattr(self.ops, "decode_order") and len(self.layers) >= 8 and self.hd in (64, 128)
+                and self.quant is None
                 and k_cache.dtype == v_cache.dtype == torch.bfloat16 and k_cache.shape[-2] == 16):
             return None
         lens = meta.seq_lens if meta.attn_seq_lens is None else meta.attn_seq_lens
@@ -362,8 +363,11 @@ class DecoderModel:
 
     def _attention(self, li, L, qkv, meta, k_cache, v_cache, order=None):
         ops, c = self.ops, self.cfg
-        # (not with shared-prefix tables, which the engine passes with every decode step unless `cascade_decode` is off)
-        if (meta.decode and meta.cascade is None and qkv.is_contiguous() and k_cache.dtype == v_cache.dtype == qkv.dtype == torch.bfloat16
+        # Not with shared-prefix tables, which the engine passes with every decode step unless `cascade_decode` is off.  Nor with fp8 projections: the
+        # rows behind the attention are quantised, where a value that rounds the other way is off by 6 %, and another order of the
+        # attention's sums moved the logits of steps of a few short rows by up to 4.7 % (their error against float64 is as large with either);
+        # theirs is the separate launches', as with shared-prefix tables.
+        if (meta.decode and meta.cascade is None and "qkv_s" not in L and qkv.is_contiguous() and k_cache.dtype == v_cache.dtype == qkv.dtype == torch.bfloat16
                 and k_cache.shape[-2] == 16):
             attend, extra = None, {}
             if hasattr(ops, "decode_attention_pairs"):   # (its fetches are 16 bytes a lane)

@@ -16,9 +16,10 @@ def test_parts():
 
 @pytest.mark.parametrize("change,paired", [({}, True), ({"hd": 64}, True), ({"hd": 96}, False), ({"cascade": object()}, False), ({"decode": False}, False),
                                            ({"kv": torch.float8_e4m3fn}, False), ({"block": 32}, False), ({"strided": True}, False),
-                                           ({"offset": 4}, False), ({"offset": 8}, True)])
+                                           ({"offset": 4}, False), ({"offset": 8}, True),
+                                           ({"layer": {"qkv_s": None}}, False)])   # (fp8 projections)
 def test_route(change, paired):
-    c = dict(dict(cascade=None, decode=True, rows=60, kv=torch.bfloat16, hd=128, block=16, strided=False, offset=0), **change)
+    c = dict(dict(cascade=None, decode=True, rows=60, kv=torch.bfloat16, hd=128, block=16, strided=False, offset=0, layer={}), **change)
     calls = []
     ops = SimpleNamespace()
     for name in ("decode_attention_pairs", "qk_norm_rope_kv_write", "paged_attention_decode", "paged_attention_prefill"):
@@ -30,6 +31,6 @@ def test_route(change, paired):
     n = 2 * 2 * c["block"] * c["hd"]
     cache = torch.zeros(n + 8).to(c["kv"])[c["offset"]:c["offset"] + n].view(1, 2, 2, c["block"], c["hd"])
     qkv = torch.zeros(c["rows"], 8 * c["hd"], dtype=torch.bfloat16)
-    m._attention(0, {}, qkv.repeat(2, 1)[::2] if c["strided"] else qkv, meta, cache, cache.transpose(3, 4))
+    m._attention(0, c["layer"], qkv.repeat(2, 1)[::2] if c["strided"] else qkv, meta, cache, cache.transpose(3, 4))
     assert calls == (["decode_attention_pairs"] if paired else
                      ["qk_norm_rope_kv_write", "paged_attention_decode" if c["decode"] else "paged_attention_prefill"])
