@@ -110,7 +110,7 @@ def load_library(path: str = None) -> ctypes.CDLL:
         "bcg_gemm_nt_fp8": [c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                             c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
         "bcg_decode_pairs": [c_void_p] * 6 + [c_float, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_void_p, c_int,
-                             c_int, c_int, c_int, c_float, c_int, c_void_p, c_void_p, c_void_p, c_void_p],
+                             c_int, c_int, c_int, c_float, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p],
         "bcg_decode_order": [c_void_p, c_int, c_void_p, c_void_p],
         "bcg_gemm_skinny": [c_int, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
                             c_void_p],
@@ -134,7 +134,7 @@ def load_library(path: str = None) -> ctypes.CDLL:
         "bcg_multimap_attention": [c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p,
                                    c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
                                    c_float, c_float, c_float, c_float, c_int, c_int, c_int, c_int, c_void_p, c_float,
-                                   c_void_p, c_int, c_void_p],
+                                   c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p],
         "bcg_embed_position": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                                c_int, c_void_p],
         "bcg_residual_rms_norm": [c_void_p, c_void_p, c_int, c_void_p, c_float, c_void_p, c_void_p, c_void_p, c_int, c_int,
@@ -300,22 +300,20 @@ def few_rows_pay(M: int, N: int, row_bytes: int, gated: bool) -> bool:
     return N >= (4096 if part else 1024)
 
 
-def decode_parts(B: int, n_kv: int, hd: int, tokens: int) -> int:
-    """Workgroups that share a (row, kv head) pair of a decode step (csrc/kernels/attention.hip, decode_pair_kernel); tokens: context that the block table
-    has room for (the contexts themselves are on the device)."""
-    return pair_parts(B * n_kv, tokens * hd * 4)
+def part_rule(pairs: int, chunk: int, chunks: int):
+    """(parts, one, each, ways, extra) of `PartRule` in csrc/kernels/common.h for `pairs` pairs of a decode step whose block table has room for `chunks`
+    chunks of 32 keys, `chunk` bytes of K and V each (the contexts themselves are on the device).
 
-
-def pair_parts(pairs: int, pair: int) -> int:
-    """The same of `pairs` pairs that read up to `pair` bytes each.
-
-    One, whose merge is its own, up to 448 KB of K/V of a pair, or where the pairs fill the CUs; else as many as there are CUs, up to one
-    for each 128 KB (us for 1, 2, 3, 4, 8 parts): heads of 128, 80 pairs of 400 tokens 9.4, 12.3, 12.5, of 1000 19.5, 17.9, 16.7, of 2500 38.6, 29.1,
-    27.3; 160 pairs of 1000 22.8, 28.6; 8 pairs of 400 8.1, 9.8, 10, 9.5, of 1000 11, 11.8, 11.5, 10.4, 10.1, of 6000 36, 24, 20, 16.7, 13.5; heads of 64, 8 pairs of
-    1000 7.3, 9, 9.1, 8.2, 8.4, of 2500 12.3, 11.9, 11.1, 9.7, 9.3; 128 pairs of 4000 34.8, 31.4."""
-    if pair <= 448 * 1024:
-        return 1
-    return max(1, min(256 // pairs, -(-pair // (128 * 1024)), 16))
+    Rows stay whole up to 448 KB of K/V of a pair (heads of 128, us for 1, 2, 3, 4, 8 parts and a merge launch: 80 pairs of 400 tokens 9.4, 12.3, 12.5, of 1000 19.5, 17.9,
+    16.7, of 2500 38.6, 29.1, 27.3; 8 pairs of 400 8.1, 9.8, 10, 9.5, of 1000 11, 11.8, 11.5, 10.4, 10.1, of 6000 36, 24, 20, 16.7, 13.5), up to 2 MB where
+    the pairs fill the CUs by themselves (160 pairs of 1000 22.8, 28.6): there it is for rows that are long beside the others, 25 us by one workgroup, and with
+    448 KB the look over the rows cost steps of equal ones 2 to 4 % (808 pairs of 1000 tokens 82.5, 85.7).  257 to 352 pairs leave most CUs with one and some
+    with two: cut among 1024 workgroups they even out (320 pairs of 5000 tokens 183 -> 162, 264 of 2000 63 -> 60.5; 384 of 5000 192, 193, 400 194, 197)."""
+    few, uneven = pairs <= 128, 256 < pairs <= 352
+    one, each = (448 if few or uneven else 2048) * 1024 // chunk, max(1, 128 * 1024 // chunk)
+    ways = 1024 if uneven else 256
+    parts = min(16, -(-chunks // each)) if chunks > one else 1
+    return parts, one, each, ways, min(ways, pairs * (parts - 1))
 
 
 def decode_fused_pays(B: int, n_kv: int, splits: int) -> bool:
@@ -454,9 +452,8 @@ def hip_ops() -> SimpleNamespace:
 
     def decode_attention_pairs(qkv, positions, slots, n_q, n_kv, hd, q_norm, k_norm, eps, cos_sin, k_cache, v_cache, layer,
                                block_tables, seq_lens, scale, workspace=None, parts=None, order=None):
-        """The same for heads of 64 or 128: a workgroup for each of `parts` parts of a (row, kv head) pair (default: `decode_parts`);
-        past one a second launch merges them, out of `workspace` where it holds B n_q parts (hd + 2) floats.  order: `decode_order` of
-        seq_lens, the pairs' order over the launch."""
+        """The same for heads of 64 or 128: a workgroup for a (row, kv head) pair, several for one of a long row (`part_rule`; parts: that many
+        for every one).  These meet in `workspace` where it has the room.  order: `decode_order` of seq_lens, the pairs' order over the launch."""
         B = qkv.shape[0]
         L, NB, nkv_c, BS, hdc = k_cache.shape
         _req(qkv.dtype == torch.bfloat16 and qkv.is_contiguous() and qkv.shape[1] == (n_q + 2 * n_kv) * hd, "decode qkv")
@@ -467,8 +464,11 @@ def hip_ops() -> SimpleNamespace:
         _req(order is None or (order.dtype == torch.int32 and order.is_contiguous() and order.numel() == B and order.device == qkv.device), "decode order")
         _req(cos_sin.dtype == torch.float32 and cos_sin.shape[1] == hd and B <= 2048, "decode cos_sin / rows")
         if parts is None:
-            parts = decode_parts(B, n_kv, hd, block_tables.shape[1] * BS)
-        need = 0 if parts == 1 else B * n_q * parts * (hd + 2)
+            rule = part_rule(B * n_kv, 128 * hd, -(-block_tables.shape[1] // 2))
+        else:
+            rule = (parts, 0, 0, 0, B * n_kv * (parts - 1))
+            _req(1 <= parts <= 64 and rule[4] <= 1 << 16, "decode parts")
+        need = 2 * rule[4] * (n_q // n_kv) * (hd + 2)
         if workspace is not None:
             _req(workspace.dtype == torch.float32 and workspace.is_contiguous(), "decode attention workspace")
         if need and (workspace is None or workspace.numel() < need):
@@ -477,7 +477,8 @@ def hip_ops() -> SimpleNamespace:
         _check(lib.bcg_decode_pairs(
             _p(qkv), _p(positions), _p(slots), None if q_norm is None else _p(q_norm), None if k_norm is None else _p(k_norm),
             _p(cos_sin), eps, _p(k_cache), _p(v_cache), layer, NB, n_kv, _p(block_tables), block_tables.shape[1], _p(seq_lens), B, n_q, hd,
-            BS, scale, parts, _p(workspace) if need else None, _p(out), None if order is None else _p(order), _stream()), "decode_attention_pairs")
+            BS, scale, *rule, _p(workspace) if need else None, _p(_counters(qkv.device)) if need else None, _p(out),
+            None if order is None else _p(order), _stream()), "decode_attention_pairs")
         return out
 
     def decode_order(seq_lens):
@@ -1083,7 +1084,7 @@ def hip_ops() -> SimpleNamespace:
 
     from .seqmix import seqmix_ops
     from .seqstate import seqstate_ops
-    extra = seqmix_ops(lib, linear)
+    extra = seqmix_ops(lib, linear, _counters)
     extra.update(seqstate_ops(lib))
     from .seqlatent import seqlatent_ops
     extra.update(seqlatent_ops(lib, extra.pop("_experts")))

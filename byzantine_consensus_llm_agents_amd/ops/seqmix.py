@@ -80,8 +80,8 @@ def few_row_tiles(n_slots, E, W, ff, rows):
     return held
 
 
-def seqmix_ops(lib, linear):
-    from .hip import pair_parts
+def seqmix_ops(lib, linear, counters):
+    from .hip import part_rule
 
     split_keys = lib.bcg_multimap_split_keys()
     tile_rows = lib.bcg_moe_tile_rows()
@@ -198,9 +198,9 @@ def seqmix_ops(lib, linear):
         return 64  # four waves x 16 rows
 
     def multimap_attention(q, k_cache, v_cache, meta, scale, maps, lam, head_eps, out_scale, vdim, window=0, sink=None,
-                           chunk=0, softcap=0.0, slopes=None, keep=0):
+                           chunk=0, softcap=0.0, slopes=None, keep=0, parts=None):
         """Prefill tiles (``meta.tiles``) on the MFMA kernel, one-token rows (``meta.single``, or
-        every row of a decode step) on the split-KV kernel.  ``window`` / ``chunk`` / ``sink``
+        every row of a decode step) by pairs or splits of their keys (``parts``: every pair in that many).  ``window`` / ``chunk`` / ``sink``
         (one-map heads): sliding window in keys, or a chunk mask (a query sees the keys of its own
         ``chunk``-aligned block of positions only); fp32 [H] sink logits of the softmax denominator.
         ``softcap`` / ``slopes`` (one-map heads): scaled scores capped by tanh, then fp32 [H] slopes
@@ -233,7 +233,7 @@ def seqmix_ops(lib, linear):
         keep = int(keep or 0) if window else 0   # (without a window nothing is hidden but the future)
         _req(keep >= 0 and (keep == 0 or (softcap == 0 and slopes is None)), "kept first keys: without softcap / slopes")
         common = (H, G, maps, dim, vdim, BS, NB, scale, lam, head_eps, out_scale, tile_rows, f32, window, chunk, _p(sink), softcap,
-                  _p(slopes), keep, _stream())
+                  _p(slopes), keep)
 
         def decode(work, n_items):
             if (not f32 and BS == 16 and n_items <= 65535 and (k_cache.data_ptr() | v_cache.data_ptr()) % 16 == 0
@@ -241,17 +241,26 @@ def seqmix_ops(lib, linear):
                 span = bt.shape[1] * BS
                 if window or chunk:   # (whole chunks of 32 keys, of the kept ones too)
                     span = min(span, keep + max(window, chunk) + 64)
-                parts = pair_parts(n_items * G * -(-(H // G) // 16), span * (maps * dim + vdim) * 2)
-                ws = torch.empty(n_items * H * parts * (2 * maps + maps * vdim), dtype=torch.float32, device=q.device) if parts > 1 else None
-                _check(lib.bcg_multimap_attention(2, _p(q), _p(k_cache), _p(v_cache), _p(bt), bt.shape[1], None, _p(lens),
-                                                  _p(work), n_items, _p(out), _p(ws), parts, *common), "multimap decode")
+                pairs = n_items * G * -(-(H // G) // 16)
+                if parts is not None:
+                    rule = (parts, 0, 0, 0, pairs * (parts - 1))
+                    _req(1 <= parts <= 16 and rule[4] <= 1 << 16, "decode parts")
+                elif n_items <= 2048:
+                    rule = part_rule(pairs, 64 * (maps * dim + vdim), -(-span // 32))
+                else:   # (every long row's workgroup looks over all of them)
+                    rule = (1, 0, 1, 0, 0)
+                ws = torch.empty(2 * rule[4] * 16 * (2 * maps + maps * vdim), dtype=torch.float32, device=q.device) if rule[4] else None
+                _check(lib.bcg_multimap_attention(2, _p(q), _p(k_cache), _p(v_cache), _p(bt), bt.shape[1], None, _p(lens), _p(work), n_items,
+                                                  _p(out), _p(ws), rule[0], *common, *rule[1:], _p(counters(q.device)) if rule[4] else None,
+                                                  _stream()), "multimap decode")
                 return
+            _req(parts is None, "parts: of the heads that a workgroup takes in pairs")
             n_splits = max(1, (bt.shape[1] * BS + split_keys - 1) // split_keys)
             if window or chunk:  # splits are counted from the window's (chunk's) first: it touches this many at most
                 n_splits = min(n_splits, (keep + split_keys - 1) // split_keys + (max(window, chunk) + split_keys - 1) // split_keys + 1)
             ws = torch.empty(n_items * H * n_splits * (2 * maps + maps * vdim), dtype=torch.float32, device=q.device)
             _check(lib.bcg_multimap_attention(1, _p(q), _p(k_cache), _p(v_cache), _p(bt), bt.shape[1], None, _p(lens),
-                                              _p(work), n_items, _p(out), _p(ws), n_splits, *common), "multimap decode")
+                                              _p(work), n_items, _p(out), _p(ws), n_splits, *common, 0, 0, 0, 0, None, _stream()), "multimap decode")
 
         if meta.decode:
             _req(T == bt.shape[0], "decode step: one row per sequence")
@@ -262,7 +271,7 @@ def seqmix_ops(lib, linear):
              and tiles.is_contiguous() and meta.q_start.dtype == torch.int32, "prefill tiles int32 [n, 3]")
         if tiles.shape[0]:
             _check(lib.bcg_multimap_attention(0, _p(q), _p(k_cache), _p(v_cache), _p(bt), bt.shape[1], _p(meta.q_start),
-                                              _p(lens), _p(tiles), tiles.shape[0], _p(out), None, 0, *common),
+                                              _p(lens), _p(tiles), tiles.shape[0], _p(out), None, 0, *common, 0, 0, 0, 0, None, _stream()),
                    "multimap prefill")
         if single is not None and single.shape[0]:
             _req(single.dtype == torch.int32 and single.dim() == 2 and single.shape[1] == 2 and single.is_contiguous(),

@@ -847,8 +847,8 @@ __global__ __launch_bounds__(256, (STREAM ? 2 : 1)) void decode_attn_kernel(
 // a chunk of its own, fetched again as soon as it is in registers.  The newest token is a chunk of its own, made of the projected row while
 // the first fetches are in flight: the cache counts up to the token before it.  What bounds it: up to 256 pairs the 64 KB that a CU has in flight
 // against the memory's latency, past that the memory (5.3 to 5.6 TB/s).
-// us, rotary + items or stream + merge -> this (spread lengths, heads of 128 / groups of 4 to 6): 10 rows of 1100 tokens, 8 kv heads 21.7 -> 17.5
-// (3 parts; 1: 21), 20 of 1500 37.5 -> 30.3, 32 of 400 26.9 -> 16, 101 of 1000 96 -> 86, 448 of 1050 390 -> 362, 400 of 60 47 -> 38; heads of 64, 2 kv heads (items
+// us, rotary + items or stream + merge -> this (spread lengths, heads of 128 / groups of 4 to 6): 10 rows of 1100 tokens, 8 kv heads 22.2 -> 16.6
+// (rows in 2 to 4 parts; whole: 21), 20 of 1500 37.5 -> 30.3, 32 of 400 26.9 -> 16, 101 of 1000 96 -> 86, 448 of 1050 390 -> 362, 400 of 60 47 -> 38; heads of 64, 2 kv heads (items
 // that rotate by themselves, merge): 4 of 500 10.5 -> 6.1, 512 of 1000 73 -> 55.
 // Waves of a workgroup, chunks of a CU the same throughout (128 KB): fewer for many pairs, whose prologues then hide behind other pairs.  Heads of 128, 4 and
 // 2 waves: 800 pairs of 1000 tokens 85.7, 88.9, of 60 16.1, 11.9; 1600 of 2000 307, 311, of 60 31, 22.8.  Heads of 64, 8 and 4: 512 pairs of 1000
@@ -860,22 +860,30 @@ struct Pair {
   static constexpr int QUERIES = 16 * HD * 2;
   static constexpr int LDS = WAVES * RING + QUERIES;
   static_assert((HD * 17 + 64) * 4 <= RING, "the parts of the waves lie where the chunks were");
+  static_assert((16 + 64 * 48 + 16) * 4 <= LDS, "and the factors of up to 64 parts of a row");
 };
 
 template <int HD, int NW>
 __global__ __launch_bounds__(64 * NW, HD == 64 ? 4 : 2) void decode_pair_kernel(
-    KVGeom g, const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ seq_lens, int n_q, float scale_log2, int parts,
-    float* __restrict__ part_o, float* __restrict__ part_ml, bf16_t* __restrict__ out, FusedArgs fa, const int* __restrict__ order) {
+    KVGeom g, const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ seq_lens, int B, int n_q, float scale_log2,
+    const PartRule rule, float* __restrict__ part_o, int* __restrict__ counters, bf16_t* __restrict__ out, FusedArgs fa, const int* __restrict__ order) {
   constexpr int KP = Pair<HD, NW>::PIECES, RING = Pair<HD, NW>::RING, PAGE = HD * BS * 2;
   __shared__ __attribute__((aligned(1024))) unsigned char smem[Pair<HD, NW>::LDS];
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, h = lane >> 4;
-  const int pair = blockIdx.x / parts, part = blockIdx.x - pair * parts;
   // (constant address space: scalar loads, whose wait is not one for the fetches)
   typedef const __attribute__((address_space(4))) int* Ints;
   auto ints = [](const int* p) { return reinterpret_cast<Ints>(reinterpret_cast<uintptr_t>(p)); };
-  const int at_row = pair / g.n_kv, kvh = pair - at_row * g.n_kv, G = n_q / g.n_kv;
-  const int b = order ? ints(order)[at_row] : at_row;
+  const Place place = place_of(rule, blockIdx.x, B * g.n_kv);
+  const int G = n_q / g.n_kv, at_row = place.at / g.n_kv, kvh = place.at - at_row * g.n_kv;
+  auto chunks_of = [&](int n) { return (min(max(n, 0), max_blocks * BS) + CHUNK - 1) / CHUNK; };
+  auto chunks = [&](int i) { return chunks_of(seq_lens[i]); };
+  Share sh{place.own ? order ? ints(order)[at_row] : at_row : -1, 0, 1, 0};
+  if (__builtin_expect(rule.extra > 0 && (sh.row < 0 || rule.each == 0 || chunks_of(ints(seq_lens)[sh.row]) > rule.one), 0)) {
+    sh = find_share(rule, B, g.n_kv, sh.row, at_row, chunks);
+    if (sh.row < 0) return;   // (the whole workgroup)
+  }
+  const int b = sh.row, part = sh.part, parts = sh.n;
   const Ints table = ints(block_tables) + static_cast<size_t>(b) * max_blocks;
   const int ctx = min(ints(seq_lens)[b], max_blocks * BS), slot = ints(fa.slots)[b];
   const int all = (ctx + CHUNK - 1) / CHUNK, last = max(ctx - 1, 0) / BS;
@@ -1036,6 +1044,10 @@ __global__ __launch_bounds__(64 * NW, HD == 64 ? 4 : 2) void decode_pair_kernel(
 #pragma unroll
     for (int i = 0; i < 4; ++i) po[(w * HD + dt * 16 + 4 * h + i) * 17 + r] = o[dt][i];
   __syncthreads();
+  // where a part of a cut row lies: [2 extra] slots of [G][HD] outputs, then as many of [G][2] maxima and denominators; the first part behind the others
+  auto slot_at = [&](int p) { return p > 0 ? (sh.first + p - 1) * g.n_kv + kvh : rule.extra + sh.first * g.n_kv + kvh; };
+  auto slot_o = [&](int p) { return part_o + static_cast<size_t>(slot_at(p)) * G * HD; };
+  auto slot_ml = [&](int p) { return part_o + (static_cast<size_t>(2 * rule.extra) * HD + 2 * static_cast<size_t>(slot_at(p))) * G; };
   if (tid < G) {
     float mm = -INFINITY;
 #pragma unroll
@@ -1049,17 +1061,64 @@ __global__ __launch_bounds__(64 * NW, HD == 64 ? 4 : 2) void decode_pair_kernel(
       ll += ml[ww * 32 + 16 + tid] * f;
     }
     fac[NW * 16 + tid] = ll > 0.f ? 1.f / ll : 0.f;
-    if (parts > 1) *reinterpret_cast<float2*>(part_ml + ((static_cast<size_t>(b) * n_q + kvh * G + tid) * parts + part) * 2) = float2{mm, ll};
+    if (parts > 1) {
+      store_through(slot_ml(part) + 2 * tid, mm);
+      store_through(slot_ml(part) + 2 * tid + 1, ll);
+    }
   }
   __syncthreads();
+  bf16_t* heads_out = out + (static_cast<size_t>(b) * n_q + kvh * G) * HD;
   for (int idx = tid; idx < G * HD; idx += 64 * NW) {
     const int qi = idx / HD, d = idx % HD;
     float oo = 0.f;
 #pragma unroll
     for (int ww = 0; ww < NW; ++ww) oo += po[(ww * HD + d) * 17 + qi] * fac[ww * 16 + qi];
-    const size_t head = static_cast<size_t>(b) * n_q + kvh * G + qi;
-    if (parts == 1) out[head * HD + d] = f2bf(oo * fac[NW * 16 + qi]);
-    else part_o[(head * parts + part) * HD + d] = oo;
+    if (parts == 1) heads_out[idx] = f2bf(oo * fac[NW * 16 + qi]);
+    else store_through(slot_o(part) + idx, oo);
+  }
+  if (parts == 1) return;
+
+  // ---- the last part of a cut row to arrive adds them up, always in their order
+  if (!last_of(counters + sh.first * g.n_kv + kvh, parts, reinterpret_cast<int*>(smem))) return;
+  const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(part_o, 0, 2 * rule.extra * G * HD * 4, 0x00020000);
+  f32x4 v[8];
+  auto load_eight = [&](int p0, int idx) {   // (past the last part: that one again, which is not added; past the heads: zeros)
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      v[j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rp, idx < G * HD ? (slot_at(min(p0 + j, parts - 1)) * G * HD + idx) * 4 : -16, 0, 16 /*sc1*/));
+  };
+  load_eight(0, 4 * tid);   // (beside the maxima)
+  float* pml = reinterpret_cast<float*>(smem) + 16;       // [parts][2][16]
+  float* pf = pml + parts * 32;                           // [parts][16], [16] of their sum
+  for (int i = tid; i < parts * 32; i += 64 * NW) {
+    const int p = i >> 5, qi = i & 15;
+    if (qi < G) pml[i] = load_through(slot_ml(p) + 2 * qi + ((i >> 4) & 1));
+  }
+  __syncthreads();
+  if (tid < G) {
+    float mm = -INFINITY, ll = 0.f;
+    for (int p = 0; p < parts; ++p) mm = fmaxf(mm, pml[p * 32 + tid]);
+    for (int p = 0; p < parts; ++p) {
+      const float mp = pml[p * 32 + tid], f = mp == -INFINITY ? 0.f : exp2f(mp - mm);
+      pf[p * 16 + tid] = f;
+      ll += pml[p * 32 + 16 + tid] * f;
+    }
+    pf[parts * 16 + tid] = ll > 0.f ? 1.f / ll : 0.f;
+  }
+  __syncthreads();
+  for (int idx = 4 * tid; idx < G * HD; idx += 256 * NW) {
+    const int qi = idx / HD;
+    f32x4 oo = {0.f, 0.f, 0.f, 0.f};
+    for (int p0 = 0; p0 < parts; p0 += 8) {
+      if (p0 > 0 || idx != 4 * tid) load_eight(p0, idx);
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (p0 + j < parts) oo += v[j] * pf[(p0 + j) * 16 + qi];
+    }
+    u16x4 y;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y[e] = f2bf(oo[e] * pf[parts * 16 + qi]);
+    *reinterpret_cast<u16x4*>(heads_out + idx) = y;
   }
 }
 
@@ -1104,7 +1163,7 @@ __global__ __launch_bounds__(64 * COMBINE_WAVES) void decode_combine_kernel(
   const int own = max(0, seq_lens[b] - (kv_begin ? kv_begin[b] : 0));
   // <= max_splits <= 64 (host check); slots 0 .. split_base[b]-1 hold the shared-prefix partials
   const int base = split_base ? split_base[b] : 0;
-  int ns = split_tokens == 0 ? max_splits : base + (own + split_tokens - 1) / split_tokens;   // (0: all slots are parts)
+  int ns = base + (own + split_tokens - 1) / split_tokens;
   if constexpr (STREAM) {   // (a row without tokens has no parts and no end)
     const unsigned long long ends = __ballot(lane >= base && (lane >= max_splits || __builtin_bit_cast(uint32_t, mlv.x) == PARTS_END));
     ns = own == 0 ? base : ends != 0 ? __ffsll(ends) - 1 : 64;
@@ -1988,28 +2047,28 @@ BCG_API int bcg_paged_attention_decode(const void* q, const void* k_cache, const
 }
 
 // Rotary embedding, cache write and attention of a decode step (decode_pair_kernel): qkv [B, n_q + 2 n_kv, hd] as projected, one new token per row
-// at `slots`; bf16 caches, hd 64 or 128.  `parts` workgroups take a (row, kv head) pair; workspace: B n_q parts (hd + 2) floats, of one part
-// none.  order: of the rows over the launch, a permutation (bcg_decode_order), or null.
+// at `slots`; bf16 caches, hd 64 or 128.  parts, one, each, ways, extra: the rule by which several workgroups take a pair of a long row (PartRule; extra >= the parts
+// beyond a pair's first that the rule can make: ways or B n_kv (parts - 1), each 0: the latter); workspace: 2 extra n_q / n_kv (hd + 2) floats, counters: `extra` zeros,
+// left zero; of none null.  order: of the rows over the launch, a permutation (bcg_decode_order), or null.
 BCG_API int bcg_decode_pairs(const void* qkv, const int* positions, const int* slots, const void* q_norm, const void* k_norm,
                              const float* cos_sin, float eps, void* k_cache, void* v_cache, int layer, int num_blocks, int n_kv,
                              const int* block_tables, int max_blocks, const int* seq_lens, int B, int n_q, int hd, int block_size,
-                             float scale, int parts, float* workspace, void* out, const int* order, hipStream_t stream) {
+                             float scale, int parts, int one, int each, int ways, int extra, float* workspace, int* counters, void* out, const int* order,
+                             hipStream_t stream) {
   if ((hd != 64 && hd != 128) || block_size != BS || n_kv <= 0 || n_q % n_kv || n_q / n_kv > 16 || B <= 0 || B > DEC_MAX_B || max_blocks <= 0) return -2;
-  if (parts < 1 || parts > 64 || (parts > 1 && !workspace) || max_blocks * BS > bcg_decode_max_context(0)) return -3;
+  const int64_t most = static_cast<int64_t>(B) * n_kv * (parts - 1);
+  if (parts < 1 || parts > 64 || one < 0 || each < 0 || extra < (each > 0 && most > ways ? ways : most) || extra > 1 << 16 || ways < 0 ||
+      (extra > 0 && (!workspace || !counters)) || max_blocks * BS > bcg_decode_max_context(0)) return -3;
+  const PartRule rule{parts, one, each, ways, extra};
   const KVGeom g{static_cast<const bf16_t*>(k_cache), static_cast<const bf16_t*>(v_cache), layer, num_blocks, n_kv};
   const FusedArgs fa{static_cast<const bf16_t*>(qkv), positions, slots, static_cast<const bf16_t*>(q_norm),
                      static_cast<const bf16_t*>(k_norm), cos_sin, eps};
   auto run = [&](auto hd_c, auto waves_c) {
     constexpr int HD = decltype(hd_c)::value, NW = decltype(waves_c)::value;
-    float* part_ml = workspace + static_cast<size_t>(B) * n_q * parts * HD;
-    bf16_t* o = static_cast<bf16_t*>(out);
-    hipLaunchKernelGGL((decode_pair_kernel<HD, NW>), dim3(B * n_kv * parts), dim3(64 * NW), 0, stream, g, block_tables, max_blocks, seq_lens,
-                       n_q, scale * LOG2E, parts, workspace, part_ml, o, fa, order);
-    if (parts > 1)
-      hipLaunchKernelGGL((decode_combine_kernel<HD, false>), dim3((B * n_q + COMBINE_WAVES - 1) / COMBINE_WAVES), dim3(64 * COMBINE_WAVES), 0, stream,
-                         workspace, part_ml, seq_lens, n_q, parts, 0, B * n_q, o, nullptr, nullptr);
+    hipLaunchKernelGGL((decode_pair_kernel<HD, NW>), dim3(B * n_kv + extra), dim3(64 * NW), 0, stream, g, block_tables, max_blocks, seq_lens, B,
+                       n_q, scale * LOG2E, rule, workspace, counters, static_cast<bf16_t*>(out), fa, order);
   };
-  const bool many = static_cast<int64_t>(B) * n_kv * parts > (hd == 64 ? 512 : 1024);   // (see Pair)
+  const bool many = B * n_kv + (each == 0 ? extra : 0) > (hd == 64 ? 512 : 1024);   // (see Pair)
   using std::integral_constant;
   if (hd == 64)
     many ? run(integral_constant<int, 64>{}, integral_constant<int, 4>{}) : run(integral_constant<int, 64>{}, integral_constant<int, 8>{});

@@ -35,6 +35,92 @@ __device__ __forceinline__ T wave_max(T v) {
   return v;
 }
 
+// Parts that several workgroups leave in memory for the one of them that arrives last, without L2 maintenance (gemm.hip): write-through stores,
+// drained by every wave, one ticket, loads that pass the L2 too.
+__device__ __forceinline__ void store_through(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ float load_through(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
+// Whether this workgroup is the last of n that leave parts under `counter` (zero before and after).  flag: an int in LDS; every thread calls.
+__device__ __forceinline__ bool last_of(int* counter, int n, int* flag) {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const int last = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == n - 1;
+    if (last) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    *flag = last;
+  }
+  __syncthreads();
+  const bool last = *flag != 0;
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");   // (no instruction: keeps the loads behind it)
+  return last;
+}
+
+// Parts of the rows of a decode step whose pairs (row, kv head) are a workgroup each.  A row is cut where it is long by itself and in its step: past `one`
+// chunks into as many parts as its share of the step's chunks is of `ways` workgroups, `parts` and one for `each` chunks at the most.  So rows of equal
+// lengths are cut as far as CUs are idle, and a long row beside short ones is not walked by one workgroup per head while the others are idle; the
+// lengths decide, not the room in the block table.  Those beyond a pair's first are workgroups of their own, `ways` at most in all, which find their row by
+// a scan over the rows (1 to 2 us, also where there is none for them: beside the others' work); a row of up to `one` chunks pays nothing.  The part that
+// arrives last adds them up: as long as a merge launch where rows are cut (1 us longer for one row of 2000 tokens), nothing where none is.
+// us, parts by the number of pairs and the table's width, merged by a launch -> this (before both: rotary launch, items or stream of 256 tokens, merge).  Heads
+// of 128, 8 kv heads: a row of 16000 tokens beside 9 of 400 58 -> 25 (34), beside 32 153 -> 34 (42), beside 447 of 60 222 -> 67 (73); 10 of 400 in a table for
+// 8192 11.6 -> 10.7 (16.7), 10 of 1100 16.9 -> 16.6 (22.2); heads of 64: 4 of 500 in a table for 8192 8.0 -> 6.0 (10.7).  Two 64-wide maps over 128, 8 kv heads: 16000
+// beside 32 of 400 170 -> 37 (117), 1 of 40 in a table for 8192 18.8 -> 6.3 (10.5), 2 of 2000 18.1 -> 15.5 (24.1).
+struct PartRule {
+  int parts, one, each;   // each 0: every row in `parts`
+  int ways;               // workgroups that the step's chunks are shared among
+  int extra;              // workgroups beside the pairs' own
+};
+struct Share {
+  int row, part, n;   // (row < 0: none)
+  int first;          // of the extra workgroups of one of the row's pairs
+};
+// Where workgroup `id` of pairs + extra stands: the pairs' own first where they leave places for others (cut rows' parts then come to idle CUs before the
+// extra ones without a row do: 80 pairs of 6000 tokens 55 us, 68 the other way round), else the extra ones, so that long rows do not begin last.  own: a
+// pair, else an extra one, `at`-th of its kind.
+struct Place { bool own; int at; };
+__device__ __forceinline__ Place place_of(const PartRule& r, int id, int pairs) {
+  if (pairs <= 352) return id < pairs ? Place{true, id} : Place{false, id - pairs};
+  return id < r.extra ? Place{false, id} : Place{true, id - r.extra};
+}
+// The share of row `row`'s own workgroup (part 0), or with row < 0 of extra workgroup `extra` of a pair's column; chunks(i): of row i.  Whole waves call.
+template <typename Chunks>
+__device__ __forceinline__ Share find_share(const PartRule& r, int rows, int pairs_per_row, int row, int extra, Chunks chunks) {
+  const int lane = threadIdx.x & 63;
+  int sum = 0, longest = 0;
+  if (r.each > 0) {
+    for (int i = lane; i < rows; i += WAVE) {
+      const int all = chunks(i);
+      sum += all;
+      longest = max(longest, all);
+    }
+    if (__ballot(longest > r.one) == 0) return Share{-1, 0, 1, 0};   // (an extra workgroup: nothing is cut)
+  }
+  const float per_chunk = r.ways / (static_cast<float>(wave_sum(sum)) * pairs_per_row);
+  int before = 0;
+  for (int i0 = 0; i0 < rows; i0 += WAVE) {
+    int n = 1;
+    if (i0 + lane < rows) {
+      const int all = chunks(i0 + lane);
+      if (r.each == 0) n = r.parts;
+      else if (all > r.one) n = max(1, min(min(r.parts, (all + r.each - 1) / r.each), static_cast<int>(all * per_chunk)));
+    }
+    int end = n - 1;
+#pragma unroll
+    for (int o = 1; o < WAVE; o <<= 1) {
+      const int u = __shfl_up(end, o, WAVE);
+      if (lane >= o) end += u;
+    }
+    end += before;
+    const unsigned long long here = __ballot(row >= 0 ? i0 + lane == row : end - (n - 1) <= extra && extra < end);
+    if (here != 0) {
+      const int at = __ffsll(here) - 1, parts = __builtin_amdgcn_readlane(n, at), first = __builtin_amdgcn_readlane(end, at) - (parts - 1);
+      return Share{i0 + at, row >= 0 ? 0 : extra - first + 1, parts, first};
+    }
+    before = __builtin_amdgcn_readlane(end, WAVE - 1);
+  }
+  return Share{-1, 0, 1, 0};
+}
+
 __device__ __forceinline__ uint32_t fmix32(uint32_t h) {
   h ^= h >> 16;
   h *= 0x85ebca6bu;

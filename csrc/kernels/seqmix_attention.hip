@@ -71,7 +71,9 @@ struct AttnArgs {
   float softcap;            // > 0: scaled scores are capped, cap tanh(s / cap)   (SHAPED instances)
   const float* slopes;      // [H] or null: slope_h (i - j) is taken off the score (SHAPED instances)
   int swz;                  // fragment-major slabs (see the top of the file)
-  int parts;                // decode: 0: n_splits is the most splits of SPLIT_KEYS keys that a row has; else every row has n_splits parts
+  PartRule rule;            // decode by pairs
+  int n_items;
+  int* counters;            // [rule.extra] zeros, left zero
 };
 
 // Maximum / sum over the four lanes that share a column (lanes col, col + 16, col + 32, col + 48): register swaps, no LDS
@@ -719,12 +721,12 @@ __global__ __launch_bounds__(64, OCC) void decode_mfma_kernel(AttnArgs a) {
 //
 // Its waves take the pair's 32-key chunks in turns and meet in LDS.  A page's slab is contiguous, so K and V come by LDS-DMA, 1 KB
 // of a slab in one piece, each wave's into a chunk of its own, fetched again as soon as its fragments are in registers (V's 4-key groups with
-// their 128-byte halves swapped in every other one, so that the lane groups of a fragment read differ in banks).  One part is merged, combined
-// and normed here; more are merged by decode_merge_kernel.  Against a wave per split of 128 keys and the merge of all splits it saves a
+// their 128-byte halves swapped in every other one, so that the lane groups of a fragment read differ in banks).  They are merged, combined and
+// normed here, those of a row in several parts by the part that arrives last.  Against a wave per split of 128 keys and the merge of all splits it saves a
 // launch and the splits' way through memory, and its loads are 16 bytes a lane instead of 8.  What bounds it: memory from some 256 pairs on (4.8 to
 // 5.1 TB/s), below that a CU's intake and the chain of table, fetch, sums and merge.
-// us, splits and merge -> this (spread lengths): two 64-wide maps over 128-wide values, 32 heads on 8, 64 rows of 1000 74 -> 54, 1 of 40 11 -> 6.2, 1 of 2000 23.5 ->
-// 16.5 (8 parts), 200 of 500 114 -> 80; 16 latent heads of 192 / 128 behind a window of 512, 64 rows 14.8 -> 11.4, 1 row of 500 11.0 -> 9.0; 32 heads on 8 of
+// us, splits and merge -> this (spread lengths): two 64-wide maps over 128-wide values, 32 heads on 8, 64 rows of 1000 74 -> 54, 1 of 40 11 -> 6.2, 2 of 2000 24.1 ->
+// 15.5 (8 parts), 200 of 500 114 -> 86; 16 latent heads of 192 / 128 behind a window of 512, 64 rows 14.8 -> 11.4, 1 row of 500 11.0 -> 9.0; 32 heads on 8 of
 // 128 behind a window of 512, 16 rows 14.7 -> 11.1.  Two waves from 1025 pairs on, whose prologues hide behind more pairs: 200 rows of 40 tokens, 8 KV
 // heads, two maps 25 -> 18 (splits 21), one 128-wide map 21 -> 15 (16.7); of 500 tokens 80.4, 80 and 76, 80.
 template <int KC, int VT, int NM, int MODE, int NW>
@@ -734,21 +736,36 @@ __global__ __launch_bounds__(64 * NW, NM * KC + VT > 24 ? 1 : 2) void decode_pai
   constexpr int KB = KD * 32, VB = VD * 32, KP = KB / 1024, VP = VB / 1024, RING = 2 * (KB + VB);   // bytes of a page of K and of V, KB, of a wave's chunk
   static_assert(KB % 1024 == 0 && VB % 1024 == 0, "whole pieces");
   static_assert((VD * 17 + 64) * 4 <= RING && 16 * VD * 4 <= NW * RING, "the parts of the waves lie where the chunks were");
+  static_assert((16 + 16 * 32 + 17 * 16 + 16 * VD) * 4 <= NW * RING, "and the factors of up to 16 parts of a row and their sums");
   constexpr int SWAP = VD % 32 == 0 ? 128 : 0;
   __shared__ __attribute__((aligned(1024))) unsigned char smem[NW * RING];
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 15, grp = lane >> 4;
-  const int parts = a.n_splits, part = blockIdx.x % parts, pair = blockIdx.x / parts;
-  const int per = a.H / a.G, g = pair % a.G, cg = pair / a.G, item = blockIdx.y;
+  const int per = a.H / a.G, columns = a.G * ((per + 15) / 16);
+  const Place place = place_of(a.rule, blockIdx.x, a.n_items * columns);
+  const int at_item = place.at / columns, column = place.at - at_item * columns, g = column % a.G, cg = column / a.G;
   // (constant address space: scalar loads, whose wait is not one for the fetches)
   typedef const __attribute__((address_space(4))) int* Ints;
   auto ints = [](const int* p) { return reinterpret_cast<Ints>(reinterpret_cast<uintptr_t>(p)); };
+  // a row's chunks: those that hold kept keys come before the window's
+  const int keep = MODE == KEEP ? a.keep : 0;
+  auto kept_of = [&](int win_) { return MODE == KEEP ? min((keep + 31) / 32, win_) : 0; };
+  auto chunks_of = [&](int ctx_) {
+    const int win_ = first_key(a, ctx_ - 1) / 32;
+    return ctx_ > 0 ? kept_of(win_) + (ctx_ + 31) / 32 - win_ : 0;
+  };
+  auto chunks = [&](int i) { return chunks_of(a.seq_lens[a.work ? a.work[2 * i + 1] : i]); };
+  Share sh{place.own ? at_item : -1, 0, 1, 0};
+  if (__builtin_expect(a.rule.extra > 0 && (!place.own || a.rule.each == 0 ||
+                                            chunks_of(ints(a.seq_lens)[a.work ? ints(a.work)[2 * at_item + 1] : at_item]) > a.rule.one), 0)) {
+    sh = find_share(a.rule, a.n_items, columns, sh.row, at_item, chunks);
+    if (sh.row < 0) return;   // (the whole workgroup)
+  }
+  const int item = sh.row, part = sh.part, parts = sh.n;
   const int row = a.work ? ints(a.work)[2 * item] : item, seq = a.work ? ints(a.work)[2 * item + 1] : item;
   const int ctx = ints(a.seq_lens)[seq], pos = ctx - 1;
   const Ints table = ints(a.block_tables) + static_cast<size_t>(seq) * a.max_blocks;
-  // this part's chunks: those that hold kept keys come before the window's
-  const int lo = first_key(a, pos), win = lo / 32, keep = MODE == KEEP ? a.keep : 0;
-  const int kept = MODE == KEEP ? min((keep + 31) / 32, win) : 0;
-  const int all = ctx > 0 ? kept + (ctx + 31) / 32 - win : 0, begin = part * all / parts, end = (part + 1) * all / parts;
+  const int lo = first_key(a, pos), win = lo / 32, kept = kept_of(win);
+  const int all = chunks_of(ctx), begin = part * all / parts, end = (part + 1) * all / parts;   // this part's chunks
   const int last_page = min(max(ctx - 1, 0) / 16, a.max_blocks - 1);
   auto key_of = [&](int j) { return 32 * (MODE != KEEP || j >= kept ? win + j - kept : j); };
   auto page_of = [&](int p) {   // past the sequence: its last page again, every key of it is masked
@@ -906,6 +923,10 @@ __global__ __launch_bounds__(64 * NW, NM * KC + VT > 24 ? 1 : 2) void decode_pai
   float* po = fac + NW * 32;                           // [NW][VD][17]
   const int heads = min(16, per - 16 * cg), h0 = g * per + 16 * cg;
   float res[N_OUT];                                    // element tid + TH i: head, value feature
+  // where a part of a cut row lies: [2 extra] slots of [16][NM][VD] numerators, then [16][2][NM] maxima and denominators; the first part behind the others
+  constexpr int SLOT = 16 * (NM * VD + 2 * NM);
+  auto slot_at = [&](int p) { return static_cast<uint32_t>((p > 0 ? (sh.first + p - 1) * columns : a.rule.extra + sh.first * columns) + column) * SLOT; };
+  auto slot_ml = [&](int p, int hh, int den, int m) { return a.ws + slot_at(p) + 16 * NM * VD + (2 * hh + den) * NM + m; };
 #pragma unroll
   for (int m = 0; m < NM; ++m) {
     const float d = column_sum(den[m]);
@@ -934,8 +955,8 @@ __global__ __launch_bounds__(64 * NW, NM * KC + VT > 24 ? 1 : 2) void decode_pai
       }
       fac[NW * 16 + tid] = (m == 0 ? 1.0f : -a.lam) / ll;
       if (parts > 1 && tid < heads) {
-        float* ws = a.ws + ((static_cast<size_t>(item) * a.H + h0 + tid) * parts + part) * (2 * NM + NM * VD);
-        ws[m] = mm, ws[NM + m] = ll;
+        store_through(slot_ml(part, tid, 0, m), mm);
+        store_through(slot_ml(part, tid, 1, m), ll);
       }
     }
     __syncthreads();
@@ -947,14 +968,65 @@ __global__ __launch_bounds__(64 * NW, NM * KC + VT > 24 ? 1 : 2) void decode_pai
 #pragma unroll
       for (int x = 0; x < NW; ++x) oo += po[(x * VD + e) * 17 + hh] * fac[x * 16 + hh];
       if (parts > 1) {
-        a.ws[((static_cast<size_t>(item) * a.H + h0 + hh) * parts + part) * (2 * NM + NM * VD) + 2 * NM + m * VD + e] = oo;
+        store_through(a.ws + slot_at(part) + (hh * NM + m) * VD + e, oo);
       } else {
         const float c = fac[NW * 16 + hh];
         res[i] = m == 0 ? oo * c : res[i] + oo * c;
       }
     }
   }
-  if (parts > 1) return;
+  if (parts > 1) {   // the last part of a cut row to arrive adds them up, always in their order
+    if (!last_of(a.counters + sh.first * columns + column, parts, reinterpret_cast<int*>(smem))) return;
+    const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(a.ws, 0, 2u * a.rule.extra * SLOT * 4, 0x00020000);
+    f32x4 v[8];
+    auto load_eight = [&](int p0, int m, int idx) {    // (past the last part: that one again, which is not added; past the heads: zeros)
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        v[j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                             rp, idx < heads * VD ? (slot_at(min(p0 + j, parts - 1)) + (idx / VD * NM + m) * VD + idx % VD) * 4 : 0xfffffff0u, 0, 16 /*sc1*/));
+    };
+    float* pml = reinterpret_cast<float*>(smem) + 16;  // [16 parts][2][16]
+    float* pf = pml + 16 * 32;                         // [16 parts][16], [16] of their sum
+    float* sum = pf + 17 * 16;                         // [16][VD]
+#pragma unroll
+    for (int m = 0; m < NM; ++m) {
+      if (m > 0) __syncthreads();
+      load_eight(0, m, 4 * tid);                       // (beside the maxima)
+      for (int i = tid; i < parts * 32; i += TH)
+        if ((i & 15) < heads) pml[i] = load_through(slot_ml(i >> 5, i & 15, (i >> 4) & 1, m));
+      __syncthreads();
+      if (tid < heads) {
+        const bool sinks = m == 0 && a.sink != nullptr;
+        const float sink = sinks ? a.sink[h0 + tid] * LOG2E : MAX_FLOOR;
+        float mm = sink;
+        for (int p = 0; p < parts; ++p) mm = fmaxf(mm, pml[p * 32 + tid]);
+        float ll = sinks ? exp2f(sink - mm) : 0.f;
+        for (int p = 0; p < parts; ++p) {
+          const float f = exp2f(pml[p * 32 + tid] - mm);
+          pf[p * 16 + tid] = f;
+          ll += pml[p * 32 + 16 + tid] * f;
+        }
+        pf[16 * 16 + tid] = (m == 0 ? 1.0f : -a.lam) / ll;
+      }
+      __syncthreads();
+      for (int idx = 4 * tid; idx < heads * VD; idx += 4 * TH) {
+        const int hh = idx / VD;
+        f32x4 oo = {0.f, 0.f, 0.f, 0.f};
+        for (int p0 = 0; p0 < parts; p0 += 8) {
+          if (p0 > 0 || idx != 4 * tid) load_eight(p0, m, idx);
+#pragma unroll
+          for (int j = 0; j < 8; ++j)
+            if (p0 + j < parts) oo += v[j] * pf[(p0 + j) * 16 + hh];
+        }
+        oo *= pf[16 * 16 + hh];
+        f32x4* to = reinterpret_cast<f32x4*>(sum + idx);
+        *to = m == 0 ? oo : *to + oo;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < N_OUT; ++i) res[i] = tid + TH * i < heads * VD ? sum[tid + TH * i] : 0.f;
+  }
   bf16_t* rows = static_cast<bf16_t*>(a.out) + (static_cast<size_t>(row) * a.H + h0) * VD;
   if (a.head_eps < 0.f) {   // no norm
 #pragma unroll
@@ -990,7 +1062,7 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(AttnArgs a) {
   const int lane = threadIdx.x, h = blockIdx.x, item = blockIdx.y;
   const int row = a.work ? a.work[2 * item] : item, seq = a.work ? a.work[2 * item + 1] : item;
   const int ctx = a.seq_lens[seq];
-  const int n = a.parts ? a.n_splits : min(a.n_splits, split_count(a, first_key(a, ctx - 1), ctx));
+  const int n = min(a.n_splits, split_count(a, first_key(a, ctx - 1), ctx));
   const float sink = a.sink != nullptr ? a.sink[h] * LOG2E : MAX_FLOOR;
   const int stride = 2 * a.maps + a.maps * a.vdim;
   const float* w = a.ws + (static_cast<size_t>(item) * a.H + h) * a.n_splits * stride;
@@ -1134,15 +1206,14 @@ void launch_merge(const AttnArgs& a, int n_items, hipStream_t s) {
   else decode_merge_kernel<T, 8><<<dim3(a.H, n_items), 64, 0, s>>>(a);
 }
 
-// Pairs of a decode step in a.n_splits parts each (decode_pair_kernel); -2: not these heads.  n_items 0: only says whether.
-int launch_pairs(const AttnArgs& a, int n_items, hipStream_t s) {
-  const dim3 grid(a.G * ((a.H / a.G + 15) / 16) * a.n_splits, n_items);
-  const bool many = static_cast<int64_t>(grid.x) * n_items > 1024;   // (see decode_pair_kernel)
+// Pairs of a decode step by a.rule (decode_pair_kernel); -2: not these heads.  n_items 0: only says whether.
+int launch_pairs(const AttnArgs& a, hipStream_t s) {
+  const int pairs = a.n_items * a.G * ((a.H / a.G + 15) / 16);
+  const bool many = pairs + (a.rule.each == 0 ? a.rule.extra : 0) > 1024;   // (see decode_pair_kernel)
   auto run = [&](auto kernel4, auto kernel2) {
-    if (n_items == 0) return 0;
-    if (many) kernel2<<<grid, 128, 0, s>>>(a);
-    else kernel4<<<grid, 256, 0, s>>>(a);
-    if (a.n_splits > 1) launch_merge<bf16_t>(a, n_items, s);
+    if (a.n_items == 0) return 0;
+    if (many) kernel2<<<pairs + a.rule.extra, 128, 0, s>>>(a);
+    else kernel4<<<pairs + a.rule.extra, 256, 0, s>>>(a);
     return BCG_CHECK_LAUNCH();
   };
 #define BCG_X(KC_, VT_, KT_, OCC_)                                                               \
@@ -1213,13 +1284,14 @@ BCG_API int bcg_multimap_split_keys() { return SPLIT_KEYS; }
 
 // mode 0: prefill tiles (work = tiles [n_work, 3]); mode 1: single-token items (work = [n_work, 2]
 // {row, sequence}, or null: item i is row i of sequence i), n_splits the most splits of a row; mode 2: the same where bcg_multimap_pairs says
-// so, every row in n_splits parts (ws is read and written if there are two or more).
+// so, with n_splits, one, each, ways and extra the rule by which several workgroups take a pair of a long row (PartRule; extra >= the parts beyond a pair's first
+// that the rule can make: ways or pairs (n_splits - 1), each 0: the latter): ws 2 extra 16 (2 maps + maps vdim) floats, counters `extra` zeros, left zero.
 BCG_API int bcg_multimap_attention(int mode, const void* q, const void* k_cache, const void* v_cache,
                                    const void* block_tables, int max_blocks, const void* q_start, const void* seq_lens,
                                    const void* work, int n_work, void* out, void* ws, int n_splits, int H, int G, int maps,
                                    int dim, int vdim, int BS, int num_blocks, float scale, float lam, float head_eps,
                                    float out_scale, int tile_rows, int is_f32, int window, int chunk, const void* sink,
-                                   float softcap, const void* slopes, int keep, void* stream) {
+                                   float softcap, const void* slopes, int keep, int one, int each, int ways, int extra, int* counters, void* stream) {
   if (n_work <= 0) return 0;
   if (keep < 0 || (keep > 0 && (window <= 0 || softcap != 0.f || slopes != nullptr))) return -2;
   if ((window > 0 || chunk > 0 || sink != nullptr || softcap != 0.f || slopes != nullptr) && maps != 1) return -2;
@@ -1239,12 +1311,16 @@ BCG_API int bcg_multimap_attention(int mode, const void* q, const void* k_cache,
   a.window = window; a.keep = keep; a.chunk = chunk; a.sink = static_cast<const float*>(sink);
   a.softcap = softcap; a.slopes = static_cast<const float*>(slopes);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  a.parts = mode == 2;
+  a.n_items = n_work;
+  a.rule = PartRule{n_splits, one, each, ways, extra};
+  a.counters = counters;
   if (mode == 2) {
-    if (is_f32 || BS != 16 || !a.swz || n_splits < 1 || n_splits > 64 || H > 65535 || n_work > 65535 || max_blocks < 1 ||
-        ((reinterpret_cast<uintptr_t>(k_cache) | reinterpret_cast<uintptr_t>(v_cache)) & 15) || (n_splits > 1 && !ws))
+    const int64_t pairs = static_cast<int64_t>(n_work) * G * ((H / G + 15) / 16), most = pairs * (n_splits - 1);
+    if (is_f32 || BS != 16 || !a.swz || n_splits < 1 || n_splits > 16 || H > 65535 || n_work > 65535 || pairs >= 1 << 30 || max_blocks < 1 || one < 0 || each < 0 ||
+        extra < (each > 0 && most > ways ? ways : most) || extra > 1 << 16 || ways < 0 ||
+        ((reinterpret_cast<uintptr_t>(k_cache) | reinterpret_cast<uintptr_t>(v_cache)) & 15) || (extra > 0 && (!ws || !counters)))
       return -2;
-    return launch_pairs(a, n_work, s);
+    return launch_pairs(a, s);
   }
   if (mode == 0) return is_f32 ? launch_prefill<float>(a, n_work, tile_rows, s) : launch_prefill<bf16_t>(a, n_work, tile_rows, s);
   if (n_splits < 1 || H > 65535 || n_splits > 65535 || n_work > 65535) return -2;
@@ -1254,6 +1330,6 @@ BCG_API int bcg_multimap_attention(int mode, const void* q, const void* k_cache,
 // Whether mode 2 takes the decode steps of these heads (bf16, 16-token pages, caches on 16 bytes).
 BCG_API int bcg_multimap_pairs(int maps, int dim, int vdim, int shaped, int keep) {
   AttnArgs a{};
-  a.maps = maps, a.dim = dim, a.vdim = vdim, a.softcap = shaped ? 1.f : 0.f, a.keep = keep, a.H = a.G = a.n_splits = 1;
-  return (maps == 1 || maps == 2) && launch_pairs(a, 0, nullptr) == 0;
+  a.maps = maps, a.dim = dim, a.vdim = vdim, a.softcap = shaped ? 1.f : 0.f, a.keep = keep, a.H = a.G = 1;
+  return (maps == 1 || maps == 2) && launch_pairs(a, nullptr) == 0;
 }

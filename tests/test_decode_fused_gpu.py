@@ -39,7 +39,7 @@ def _case(lens, n_q, n_kv, hd, norm, seed=0, parked=()):
     i32 = dict(dtype=torch.int32, device=dev)
     qkv = torch.randn(B, (n_q + 2 * n_kv) * hd, device=dev, generator=g).to(torch.bfloat16)
     nw = [(1 + 0.2 * torch.randn(hd, device=dev, generator=g)).to(torch.bfloat16) if norm else None for _ in range(2)]
-    ang = torch.rand(4096, hd // 2, device=dev, generator=g) * 6.28
+    ang = torch.rand(max(4096, *lens), hd // 2, device=dev, generator=g) * 6.28   # (a row for every position)
     return dict(qkv=qkv, positions=torch.tensor(pos, **i32), slots=torch.tensor(slots, **i32), n_q=n_q, n_kv=n_kv, hd=hd, q_norm=nw[0],
                 k_norm=nw[1], eps=1e-6, cos_sin=torch.cat([ang.cos(), ang.sin()], 1).contiguous()), k, v, table.to(dev), torch.tensor(lens, **i32)
 

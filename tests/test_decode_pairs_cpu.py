@@ -1,17 +1,20 @@
-"""Which decode steps take a workgroup per (row, kv head) pair, and in how many parts.  No GPU."""
+"""Which decode steps take a workgroup per (row, kv head) pair, and where a long row is cut.  No GPU."""
 from types import SimpleNamespace
 
 import pytest
 import torch
 
 from byzantine_consensus_llm_agents_amd.models.transformer import AttnMeta, DecoderModel
-from byzantine_consensus_llm_agents_amd.ops.hip import decode_parts
+from byzantine_consensus_llm_agents_amd.ops.hip import part_rule
 
 
 def test_parts():
-    assert decode_parts(10, 8, 128, 896) == 1 and decode_parts(10, 8, 128, 912) == 3
-    assert decode_parts(1, 2, 64, 1792) == 1 and decode_parts(1, 2, 64, 1808) == 4 and decode_parts(1, 2, 64, 16384) == 16
-    assert decode_parts(17, 8, 128, 16384) == 1 and decode_parts(2048, 8, 128, 8192) == 1
+    """(parts, one, each, ways, extra): heads of 128 have chunks of 16 KB, of 64 of 8 KB."""
+    assert part_rule(80, 128 * 128, 28) == (1, 28, 8, 256, 0) and part_rule(80, 128 * 128, 29) == (4, 28, 8, 256, 240)
+    assert part_rule(2, 128 * 64, 57) == (4, 56, 16, 256, 6) and part_rule(2, 128 * 64, 512) == (16, 56, 16, 256, 30)
+    assert part_rule(136, 128 * 128, 128) == (1, 128, 8, 256, 0) and part_rule(136, 128 * 128, 512) == (16, 128, 8, 256, 256)
+    assert part_rule(320, 128 * 128, 256) == (16, 28, 8, 1024, 1024) and part_rule(360, 128 * 128, 256)[3] == 256
+    assert part_rule(16384, 128 * 128, 512) == (16, 128, 8, 256, 256) and part_rule(1, 1 << 20, 1) == (1, 0, 1, 256, 0)
 
 
 @pytest.mark.parametrize("change,paired", [({}, True), ({"hd": 64}, True), ({"hd": 96}, False), ({"cascade": object()}, False), ({"decode": False}, False),

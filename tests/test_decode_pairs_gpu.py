@@ -53,3 +53,74 @@ def test_wide_tables_parked_rows_and_graph_replays(ops, parts):
         torch.cuda.synchronize()
         assert ((out.double() - want.double()).norm() / want.double().norm()).item() < 2 ** -7
         _same_cache(c, k0, v0, k, v, k1, v1, True, rows=[1, 3, 4])
+
+
+def _float64(c, k, v, table, lens):
+    """The attention in float64 over what the separate operations rotated and stored."""
+    q = _rotated(c)
+    out = []
+    for b, n in enumerate(lens.tolist()):
+        pages = table[b, :-(-n // 16)].long()
+        kk = k[1, pages].permute(1, 0, 2, 3).reshape(c["n_kv"], -1, c["hd"])[:, :n].double()
+        vv = v[1, pages].permute(1, 0, 3, 2).reshape(c["n_kv"], -1, c["hd"])[:, :n].double()
+        g = c["n_q"] // c["n_kv"]
+        s = torch.softmax(torch.matmul(q[b].view(c["n_kv"], g, c["hd"]), kk.transpose(1, 2).contiguous()) * c["hd"] ** -0.5, -1)
+        out.append(torch.matmul(s, vv).reshape(-1))
+    return torch.stack(out)
+
+
+def _rotated(c):
+    x = c["qkv"].double().view(c["qkv"].shape[0], -1, c["hd"])[:, :c["n_q"]]
+    if c["q_norm"] is not None:
+        x = x / torch.sqrt((x * x).mean(-1, keepdim=True) + c["eps"]) * c["q_norm"].double()
+    cs = c["cos_sin"][c["positions"].long()].double()[:, None]
+    h = c["hd"] // 2
+    cos, sin, a, b = cs[..., :h], cs[..., h:], x[..., :h], x[..., h:]
+    return torch.cat([a * cos - b * sin, b * cos + a * sin], -1).to(torch.bfloat16).double()
+
+
+def _cut(lens, pairs_per_row, rule):
+    """Parts of every row, as find_share of csrc/kernels/common.h has them."""
+    parts, one, each, ways, _ = rule
+    chunks = (lens.cpu() + 31) // 32
+    share = chunks * ways / (int(chunks.sum()) * pairs_per_row)
+    return torch.where(chunks > one, torch.minimum(share.long(), (chunks + each - 1) // each).clamp(1, parts), 1)
+
+
+# long rows beside short ones, few and many pairs, up to the most parts, in tables as wide as they need and wider; (40 rows: the range of pairs that are cut finer)
+@pytest.mark.parametrize("n_q,n_kv,hd,lens,room", [
+    (40, 8, 128, [7000] + [300] * 9, 0), (40, 8, 128, [60] * 20 + [5000] + [90] * 14, 512), (14, 2, 64, [4000, 30, 9000], 0), (10, 2, 128, [3000] * 3, 0),
+    (32, 8, 128, [100] * 130 + [8000], 0), (14, 2, 64, [2500], 512), (40, 8, 128, [1500] * 40, 0)])
+def test_rows_cut_by_the_rule(ops, n_q, n_kv, hd, lens, room):
+    """Outputs in float64's, the parts that the rule says (and no others) in the workspace, on two streams the same bits."""
+    from byzantine_consensus_llm_agents_amd.ops.hip import part_rule
+    c, k, v, table, sl = _case(lens, n_q, n_kv, hd, True, seed=n_q)
+    if room > table.shape[1]:
+        table = torch.cat([table, torch.full((len(lens), room - table.shape[1]), 1 << 28, dtype=torch.int32, device="cuda")], 1).contiguous()
+    rule = part_rule(len(lens) * n_kv, 128 * hd, -(-table.shape[1] // 2))
+    cut = _cut(sl, n_kv, rule)
+    assert cut.max() > 1 and int((cut - 1).sum()) * n_kv <= rule[4]
+    G, extra = n_q // n_kv, rule[4]
+    ws = torch.full((2 * extra * G * (hd + 2),), float("nan"), device="cuda")
+    got = _pairs(ops, c, k, v, table, sl, None, ws)
+    used = (~torch.isnan(ws[:2 * extra * G * hd].view(2 * extra, -1))).all(1)
+    assert int(used[:extra].sum()) == int((cut - 1).sum()) * n_kv and int(used[extra:].sum()) == int((cut > 1).sum()) * n_kv
+    want = _float64(c, k, v, table, sl)
+    off = (got.double() - want).view(len(lens), n_q, hd).norm(dim=-1) / want.view(len(lens), n_q, hd).norm(dim=-1)
+    assert bool((off < 2 ** -7).all()), off.max()
+    streams, outs = [torch.cuda.Stream() for _ in range(2)], [[], []]
+    torch.cuda.synchronize()
+    for _ in range(4):
+        for s, o in zip(streams, outs):
+            with torch.cuda.stream(s):
+                o.append(_pairs(ops, c, k, v, table, sl))
+    torch.cuda.synchronize()
+    assert all(torch.equal(t, got) for o in outs for t in o)
+
+
+def test_short_rows_in_wide_tables_stay_whole(ops):
+    c, k, v, table, sl = _case([500, 300, 800, 40], 14, 2, 64, False, seed=1)
+    narrow = _pairs(ops, c, k, v, table, sl)
+    wide = torch.cat([table, torch.full((4, 1000 - table.shape[1]), 1 << 28, dtype=torch.int32, device="cuda")], 1).contiguous()
+    ws = torch.full((1 << 18,), float("nan"), device="cuda")
+    assert torch.equal(_pairs(ops, c, k, v, wide, sl, None, ws), narrow) and torch.isnan(ws).all()
