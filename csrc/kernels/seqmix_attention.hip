@@ -746,13 +746,11 @@ __global__ __launch_bounds__(64 * NW, NM * KC + VT > 24 ? 1 : 2) void decode_pai
   // (constant address space: scalar loads, whose wait is not one for the fetches)
   typedef const __attribute__((address_space(4))) int* Ints;
   auto ints = [](const int* p) { return reinterpret_cast<Ints>(reinterpret_cast<uintptr_t>(p)); };
-  // a row's chunks: those that hold kept keys come before the window's
-  const int keep = MODE == KEEP ? a.keep : 0;
-  auto kept_of = [&](int win_) { return MODE == KEEP ? min((keep + 31) / 32, win_) : 0; };
-  auto chunks_of = [&](int ctx_) {
-    const int win_ = first_key(a, ctx_ - 1) / 32;
-    return ctx_ > 0 ? kept_of(win_) + (ctx_ + 31) / 32 - win_ : 0;
-  };
+  // a row's chunks: those that hold kept keys come before the window's, which begin with the page of the window's first key (a page in front of it may hold
+  // what are no numbers, and a weight of zero does not take these out)
+  const int keep = MODE == KEEP ? a.keep : 0, kept = (keep + 31) / 32;
+  auto win_of = [&](int ctx_) { return max(first_key(a, ctx_ - 1) & ~15, 32 * kept); };
+  auto chunks_of = [&](int ctx_) { return ctx_ > 0 ? min(kept, (ctx_ + 31) / 32) + max(0, ctx_ - win_of(ctx_) + 31) / 32 : 0; };
   auto chunks = [&](int i) { return chunks_of(a.seq_lens[a.work ? a.work[2 * i + 1] : i]); };
   Share sh{place.own ? at_item : -1, 0, 1, 0};
   if (__builtin_expect(a.rule.extra > 0 && (!place.own || a.rule.each == 0 ||
@@ -764,10 +762,10 @@ __global__ __launch_bounds__(64 * NW, NM * KC + VT > 24 ? 1 : 2) void decode_pai
   const int row = a.work ? ints(a.work)[2 * item] : item, seq = a.work ? ints(a.work)[2 * item + 1] : item;
   const int ctx = ints(a.seq_lens)[seq], pos = ctx - 1;
   const Ints table = ints(a.block_tables) + static_cast<size_t>(seq) * a.max_blocks;
-  const int lo = first_key(a, pos), win = lo / 32, kept = kept_of(win);
+  const int lo = first_key(a, pos), win = win_of(ctx);
   const int all = chunks_of(ctx), begin = part * all / parts, end = (part + 1) * all / parts;   // this part's chunks
   const int last_page = min(max(ctx - 1, 0) / 16, a.max_blocks - 1);
-  auto key_of = [&](int j) { return 32 * (MODE != KEEP || j >= kept ? win + j - kept : j); };
+  auto key_of = [&](int j) { return MODE != KEEP || j >= kept ? win + 32 * (j - kept) : 32 * j; };
   auto page_of = [&](int p) {   // past the sequence: its last page again, every key of it is masked
     const int page = table[min(p, last_page)];
     return static_cast<size_t>((page < 0 || page >= a.num_blocks) ? 0 : page) * a.G + g;

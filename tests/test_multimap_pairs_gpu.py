@@ -14,7 +14,7 @@ DEV = "cuda"
 # contexts at the edges of pages (16), chunks (32) and turns of 2 and 4 waves (64, 128)
 LENS = [1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 127, 128, 129, 300, 513, 1025]
 KINDS = {"plain": {}, "window": dict(window=37), "long window": dict(window=300), "chunk": dict(chunk=50), "keep": dict(window=40, keep=5), "keep far": dict(window=70, keep=140),
-         "sink": dict(sink=True, window=100), "far sink": dict(sink=True, window=700), "shaped": dict(softcap=3.0, slopes=True)}
+         "sink": dict(sink=True, window=100), "far sink": dict(sink=True, window=700), "shaped": dict(softcap=3.0, slopes=True), "shaped window": dict(softcap=3.0, slopes=True, window=100)}
 
 
 @pytest.fixture(scope="module")
@@ -90,6 +90,20 @@ def test_long_rows_beside_short_ones(ops):
                 o.append(ops.multimap_attention(q, kp, vp, meta, *args))
     torch.cuda.synchronize()
     assert all(torch.equal(t, first) for o in outs for t in o)   # (parts are added in their order, whoever comes last)
+
+
+@pytest.mark.parametrize("kind,parts", [("window", None), ("long window", None), ("long window", 5), ("chunk", None), ("keep", None), ("keep far", 2), ("shaped window", None)])
+def test_pages_in_front_of_the_window(ops, kind, parts):
+    """Pages wholly in front of a window (or between it and the kept keys' chunks) hold infinities and NaN: no query sees them."""
+    q, k, v, bt, lens, args, kw = _case(4, 2, 1, 128, 128, kind, 16, 0, -1.0, seed=4)
+    want = ref.multimap_attention(q, k, v, bt, torch.arange(17, dtype=torch.int32, device=DEV), lens, *args, **kw)
+    for b, n in enumerate(lens.tolist()):
+        lo = max(0, n - kw["window"]) if "window" in kw else (n - 1) - (n - 1) % kw["chunk"]
+        for page in range(2 * (-(-kw.get("keep", 0) // 32)), lo // 16):
+            k[bt[b, page]], v[bt[b, page]] = float("nan"), float("inf")
+    kp, vp = ops.kv_from_logical(k, v)
+    got = ops.multimap_attention(q, kp, vp, AttnMeta(positions=None, slots=None, block_tables=bt, seq_lens=lens, decode=True), *args, **kw, parts=parts)
+    _close(got, want, 128)
 
 
 def test_single_rows_and_graph_replays(ops):
