@@ -1144,7 +1144,16 @@ int launch_prefill_mode(const AttnArgs& a, int n_tiles, bool full, hipStream_t s
 }
 
 template <typename T, int MODE>
-void launch_decode_mode(const AttnArgs& a, dim3 grid, hipStream_t s) {
+void launch_decode_mode(const AttnArgs& a, dim3 grid, bool full, hipStream_t s) {
+  if constexpr (sizeof(T) == 2) if (full && a.swz && a.BS == 16) {
+#define BCG_X(KC_, VT_, KT_, OCC_)                                                               \
+  if (a.dim == 16 * KC_ && a.vdim == 16 * VT_) {                                                 \
+    decode_mfma_kernel<T, KC_, VT_, KT_, true, true, OCC_, 1, 1, MODE><<<grid, 64, 0, s>>>(a);   \
+    return;                                                                                      \
+  }
+    if constexpr (MODE == SHAPED) { BCG_EXACT1_SHAPED(BCG_X) } else { BCG_EXACT1_KEEP(BCG_X) }
+#undef BCG_X
+  }
   if (a.dim <= 64 && a.vdim <= 128) decode_mfma_kernel<T, 4, 8, 1, false, false, 1, 0, 1, MODE><<<grid, 64, 0, s>>>(a);
   else if (a.dim <= 256 && a.vdim <= 256) decode_mfma_kernel<T, 16, 16, 1, false, false, 1, 0, 1, MODE><<<grid, 64, 0, s>>>(a);
   else decode_mfma_kernel<T, 32, 32, 1, false, false, 1, 0, 1, MODE><<<grid, 64, 0, s>>>(a);
@@ -1241,6 +1250,10 @@ int launch_pairs(const AttnArgs& a, hipStream_t s) {
   return -2;
 }
 
+// Splits of 128 keys and their merge: fp32, heads or pages of other sizes, and of the exact sizes capped or sloped heads of 48 (a page of them is no whole number
+// of KB) and caches that do not begin on 16 bytes, which the copies of decode_pair_kernel need.
+// us, guarded instances in their place and this: 64 rows of 1000 tokens, heads of 48 capped, 16 on 4, 38.5, 20.1; caches off 16 bytes, 32 heads on 8 of 128 254, 65, two
+// 64-wide maps over 128 84, 75, 16 latent heads of 192 / 128 behind a window of 512 60, 16.6 (on 16 bytes by pairs: 55 with the maps, 13).
 template <typename T>
 int launch_decode(const AttnArgs& a, int n_items, hipStream_t s) {
   const int per = a.H / a.G;
@@ -1248,14 +1261,34 @@ int launch_decode(const AttnArgs& a, int n_items, hipStream_t s) {
   const bool full = a.dim % 16 == 0 && a.vdim % 16 == 0 && a.vec_k && a.vec_v;
   const bool shaped = a.softcap > 0.f || a.slopes != nullptr;
   bool done = shaped || a.keep > 0;
-  if (shaped) launch_decode_mode<T, SHAPED>(a, grid, s);
-  else if (done) launch_decode_mode<T, KEEP>(a, grid, s);
-  if constexpr (sizeof(T) == 2) if (!done && full && a.maps == 1 && a.swz && a.BS == 16 && a.dim == 512 && a.vdim == 512) {
-    done = true;
-    decode_mfma_kernel<T, 32, 32, 1, true, true, 1, 1, 1><<<grid, 64, 0, s>>>(a);
+  if (shaped) launch_decode_mode<T, SHAPED>(a, grid, full, s);
+  else if (done) launch_decode_mode<T, KEEP>(a, grid, full, s);
+  if constexpr (sizeof(T) == 2) if (!done && full && a.maps == 1 && a.swz && a.BS == 16) {   // one-map heads, exact shapes
+#define BCG_X(KC_, VT_, KT_, OCC_)                                                               \
+  if (!done && a.dim == 16 * KC_ && a.vdim == 16 * VT_) {                                        \
+    done = true;                                                                                 \
+    decode_mfma_kernel<T, KC_, VT_, KT_, true, true, OCC_, 1, 1><<<grid, 64, 0, s>>>(a);         \
+  }
+    BCG_EXACT1_PLAIN(BCG_X)
+    if (!done && a.dim == 512 && a.vdim == 512) {
+      done = true;
+      decode_mfma_kernel<T, 32, 32, 1, true, true, 1, 1, 1><<<grid, 64, 0, s>>>(a);
+    }
+#undef BCG_X
   }
   if constexpr (sizeof(T) == 2) if (!done && a.dim <= 64 && a.vdim <= 128) {
     done = true;
+    const bool exact = full && a.maps == 2 && a.swz && a.BS == 16;
+    bool hit = false;
+#define BCG_EXACT(KC_, VT_)                                                                      \
+  if (!hit && exact && a.dim == 16 * KC_ && a.vdim == 16 * VT_) {                                \
+    hit = true;                                                                                  \
+    decode_mfma_kernel<T, KC_, VT_, 2, true, true, 2, 2><<<grid, 64, 0, s>>>(a);                 \
+  }
+    BCG_EXACT(4, 8) BCG_EXACT(3, 6) BCG_EXACT(2, 4) BCG_EXACT(4, 4) BCG_EXACT(2, 2)
+#undef BCG_EXACT
+    if (hit) {
+    } else
     if (full) decode_mfma_kernel<T, 4, 8, 2, true, true, 2><<<grid, 64, 0, s>>>(a);
     else decode_mfma_kernel<T, 4, 8, 2, true, false, 2><<<grid, 64, 0, s>>>(a);
   }

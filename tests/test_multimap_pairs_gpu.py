@@ -130,14 +130,26 @@ def test_single_rows_and_graph_replays(ops):
             _close(out[order], want, 128)
 
 
-def test_caches_off_16_bytes(ops):
+@pytest.mark.parametrize("H,G,maps,dim,vdim,kind,eps", [(8, 2, 2, 64, 128, "plain", 1e-5), (6, 2, 2, 48, 96, "plain", -1.0), (4, 2, 1, 128, 128, "window", -1.0),
+                                                        (4, 2, 1, 192, 128, "plain", -1.0), (8, 4, 1, 64, 64, "keep far", 1e-5), (4, 2, 1, 256, 256, "shaped", -1.0)])
+def test_caches_off_16_bytes(ops, H, G, maps, dim, vdim, kind, eps):
     """Views that begin 8 bytes into their memory take the splits."""
-    q, k, v, bt, lens, args, _ = _case(8, 2, 2, 64, 128, "plain", 5, 0, 1e-5, seed=2)
+    q, k, v, bt, lens, args, kw = _case(H, G, maps, dim, vdim, kind, 16, 0, eps, seed=2)
     moved = []
     for t in ops.kv_from_logical(k, v):
         room = torch.empty(t.numel() + 4, dtype=t.dtype, device=DEV)[4:].view(t.shape)
         room.copy_(t)
         moved.append(room)
-    got = ops.multimap_attention(q, *moved, AttnMeta(positions=None, slots=None, block_tables=bt, seq_lens=lens, decode=True), *args)
-    want = ref.multimap_attention(q, k, v, bt, torch.arange(6, dtype=torch.int32, device=DEV), lens, *args)
-    _close(got, want, 128)
+    got = ops.multimap_attention(q, *moved, AttnMeta(positions=None, slots=None, block_tables=bt, seq_lens=lens, decode=True), *args, **kw)
+    want = ref.multimap_attention(q, k, v, bt, torch.arange(17, dtype=torch.int32, device=DEV), lens, *args, **kw)
+    _close(got, want, vdim)
+
+
+def test_shaped_heads_of_48(ops):
+    """Capped and sloped heads whose pages are no whole number of KB take the splits."""
+    q, k, v, bt, lens, args, kw = _case(4, 2, 1, 48, 48, "shaped", 16, 5, -1.0, seed=3)
+    assert not ops.library.bcg_multimap_pairs(1, 48, 48, 1, 0)
+    kp, vp = ops.kv_from_logical(k, v)
+    got = ops.multimap_attention(q, kp, vp, AttnMeta(positions=None, slots=None, block_tables=bt, seq_lens=lens, decode=True), *args, **kw)
+    want = ref.multimap_attention(q, k, v, bt, torch.arange(17, dtype=torch.int32, device=DEV), lens, *args, **kw)
+    _close(got, want, 48)
