@@ -349,12 +349,20 @@ class DecoderModel:
         idx = meta.logits_idx
         return attn.index_select(0, idx), residual.index_select(0, idx)
 
+    def _by_pairs(self, L, meta, k_cache, v_cache):
+        """Whether `decode_attention_pairs` takes the layers' attention of this step (its fetches are 16 bytes a lane).  Not with shared-prefix
+        tables, which the engine passes with every decode step unless `cascade_decode` is off.  Nor with fp8 projections: the
+        rows behind the attention are quantised, where a value that rounds the other way is off by 6 %, and another order of the
+        attention's sums moved the logits of steps of a few short rows by up to 4.7 % (their error against float64 is as large with either);
+        theirs is the separate launches', as with shared-prefix tables."""
+        return (meta.decode and meta.cascade is None and "qkv_s" not in L and hasattr(self.ops, "decode_attention_pairs") and self.hd in (64, 128)
+                and k_cache.dtype == v_cache.dtype == torch.bfloat16 and k_cache.shape[-2] == 16 and meta.block_tables.shape[1] > 0
+                and (k_cache.data_ptr() | v_cache.data_ptr()) % 16 == 0)
+
     def _decode_order(self, meta, k_cache, v_cache):
         """`ops.decode_order` for the layers' `decode_attention_pairs`, where more pairs than the CUs hold at once (512) take turns: a layer gains
         2 to 3 % of its attention, 1 to 13 us, and the launch costs about 4.6 (`decode_order_kernel`)."""
-        if not (meta.decode and meta.cascade is None and hasattr(self.ops, "decode_order") and len(self.layers) >= 8 and self.hd in (64, 128)
-                and self.quant is None
-                and k_cache.dtype == v_cache.dtype == torch.bfloat16 and k_cache.shape[-2] == 16):
+        if len(self.layers) < 8 or not self._by_pairs(self.layers[0], meta, k_cache, v_cache):
             return None
         lens = meta.seq_lens if meta.attn_seq_lens is None else meta.attn_seq_lens
         if lens.numel() * self.n_kv <= 512 or lens.numel() > 2048 or lens.dtype != torch.int32 or not lens.is_contiguous():
@@ -363,23 +371,10 @@ class DecoderModel:
 
     def _attention(self, li, L, qkv, meta, k_cache, v_cache, order=None):
         ops, c = self.ops, self.cfg
-        # Not with shared-prefix tables, which the engine passes with every decode step unless `cascade_decode` is off.  Nor with fp8 projections: the
-        # rows behind the attention are quantised, where a value that rounds the other way is off by 6 %, and another order of the
-        # attention's sums moved the logits of steps of a few short rows by up to 4.7 % (their error against float64 is as large with either);
-        # theirs is the separate launches', as with shared-prefix tables.
-        if (meta.decode and meta.cascade is None and "qkv_s" not in L and qkv.is_contiguous() and k_cache.dtype == v_cache.dtype == qkv.dtype == torch.bfloat16
-                and k_cache.shape[-2] == 16):
-            attend, extra = None, {}
-            if hasattr(ops, "decode_attention_pairs"):   # (its fetches are 16 bytes a lane)
-                if self.hd in (64, 128) and (k_cache.data_ptr() | v_cache.data_ptr() | qkv.data_ptr()) % 16 == 0:
-                    attend, extra = ops.decode_attention_pairs, {} if order is None else {"order": order}
-            elif (self.hd == 64 and hasattr(ops, "decode_attention")
-                  and ops.decode_fused_pays(qkv.shape[0], self.n_kv, meta.block_tables.shape[1] * 16)):
-                attend = ops.decode_attention
-            if attend is not None:
-                lens = meta.seq_lens if meta.attn_seq_lens is None else meta.attn_seq_lens
-                return attend(qkv, meta.positions, meta.slots, self.n_q, self.n_kv, self.hd, L.get("q_norm"), L.get("k_norm"), c.rms_eps,
-                              self.cos_sin, k_cache, v_cache, li, meta.block_tables, lens, self.scale, meta.workspace, **extra)
+        if (self._by_pairs(L, meta, k_cache, v_cache) and qkv.dtype == torch.bfloat16 and qkv.is_contiguous() and qkv.data_ptr() % 16 == 0):
+            lens = meta.seq_lens if meta.attn_seq_lens is None else meta.attn_seq_lens
+            return ops.decode_attention_pairs(qkv, meta.positions, meta.slots, self.n_q, self.n_kv, self.hd, L.get("q_norm"), L.get("k_norm"), c.rms_eps,
+                                              self.cos_sin, k_cache, v_cache, li, meta.block_tables, lens, self.scale, meta.workspace, order=order)
         q = ops.qk_norm_rope_kv_write(qkv, meta.positions, meta.slots, self.n_q, self.n_kv, self.hd,
                                       L.get("q_norm"), L.get("k_norm"), c.rms_eps, self.cos_sin,
                                       k_cache, v_cache, li, contiguous=not meta.decode)

@@ -316,19 +316,6 @@ def part_rule(pairs: int, chunk: int, chunks: int):
     return parts, one, each, ways, min(ways, pairs * (parts - 1))
 
 
-def decode_fused_pays(B: int, n_kv: int, splits: int) -> bool:
-    """Whether a decode step of B rows with heads of 64 gains by `decode_attention` with a backend that has no `decode_attention_pairs`: one whose
-    workgroups take a part of a row's context each and all rotate its queries; splits: parts that the block table has room for.
-
-    The rotation takes registers, so two workgroups of a CU are resident where the separate kernel has three, and every workgroup of a row rotates
-    its queries again.  Rotary launch, attention and merge over the fused pair, 14 / 2, 16 / 4, 32 / 8, 16 / 16 and 16 / 1 heads, contexts
-    of 16 to 16000 tokens, table of their length: 1.03 to 1.19 while all parts are resident (B n_kv splits <= 512), 0.97 to 1.1 at 576
-    (contexts spread by a third to either side: 1.04 to 1.08, a quarter of the parts is empty), past that 0.72 to 1.04 (16 kv heads, 100 rows of 20
-    tokens 16.5 us, 22.8).  Wide tables say nothing of the contexts: up to 16 heads of K and V in all 1.0 to 1.19 up to 16000 tokens, from 32
-    on 0.93 there.  More than 128 rows were not timed in a step."""
-    return B <= 128 and (B * n_kv <= 16 or B * n_kv * splits <= 576)
-
-
 def hip_ops() -> SimpleNamespace:
     lib = load_library()
 
@@ -438,22 +425,12 @@ def hip_ops() -> SimpleNamespace:
             _stream()), "paged_attention_decode")
         return out
 
-    def decode_attention(qkv, positions, slots, n_q, n_kv, hd, q_norm, k_norm, eps, cos_sin, k_cache, v_cache, layer,
-                         block_tables, seq_lens, scale, workspace=None):
-        """paged_attention_decode(qk_norm_rope_kv_write(...)) for one new token per row of a bf16 cache with heads of 64, without the
-        rotary launch.  Rows are different sequences: no row sees what another one stores in this call.  `workspace`: as
-        paged_attention_decode."""
-        _req(hd == 64, "decode kv cache layout")
-        B, tokens = qkv.shape[0], block_tables.shape[1] * 16
-        if workspace is not None:
-            _req(workspace.numel() >= B * n_q * lib.bcg_decode_max_splits(tokens, 0) * (hd + 2), "decode attention workspace too small")
-        return decode_attention_pairs(qkv, positions, slots, n_q, n_kv, hd, q_norm, k_norm, eps, cos_sin, k_cache, v_cache, layer,
-                                      block_tables, seq_lens, scale, workspace)
-
     def decode_attention_pairs(qkv, positions, slots, n_q, n_kv, hd, q_norm, k_norm, eps, cos_sin, k_cache, v_cache, layer,
                                block_tables, seq_lens, scale, workspace=None, parts=None, order=None):
-        """The same for heads of 64 or 128: a workgroup for a (row, kv head) pair, several for one of a long row (`part_rule`; parts: that many
-        for every one).  These meet in `workspace` where it has the room.  order: `decode_order` of seq_lens, the pairs' order over the launch."""
+        """paged_attention_decode(qk_norm_rope_kv_write(...)) for one new token per row of a bf16 cache with heads of 64 or 128, in one launch.
+        Rows are different sequences: no row sees what another one stores in this call.  A workgroup for a (row, kv head) pair, several for
+        one of a long row (`part_rule`; parts: that many for every one), which meet in `workspace` where it has the room.  order:
+        `decode_order` of seq_lens, the pairs' order over the launch."""
         B = qkv.shape[0]
         L, NB, nkv_c, BS, hdc = k_cache.shape
         _req(qkv.dtype == torch.bfloat16 and qkv.is_contiguous() and qkv.shape[1] == (n_q + 2 * n_kv) * hd, "decode qkv")
@@ -1100,7 +1077,7 @@ def hip_ops() -> SimpleNamespace:
                            embed_rmsnorm=embed_rmsnorm,
                            qk_norm_rope_kv_write=qk_norm_rope_kv_write,
                            paged_attention_decode=paged_attention_decode,
-                           decode_attention=decode_attention, decode_attention_pairs=decode_attention_pairs, decode_order=decode_order,
+                           decode_attention_pairs=decode_attention_pairs, decode_order=decode_order,
                            decode_workspace_numel=decode_workspace_numel,
                            decode_max_context=lambda cascade=True: lib.bcg_decode_max_context(int(cascade)),
                            paged_attention_prefill=paged_attention_prefill,

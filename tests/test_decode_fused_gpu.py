@@ -1,4 +1,4 @@
-"""Rotary embedding, cache write and attention of a decode step without the rotary launch (csrc/kernels/attention.hip, FUSED) against the
+"""Rotary embedding, cache write and attention of a decode step in one launch (csrc/kernels/attention.hip, decode_pair_kernel), heads of 64, against the
 separate operations.  GPU only.
 
 Both round queries and keys to bf16 after the same fp32 arithmetic and store the same bytes (a root mean square summed in
@@ -51,7 +51,7 @@ def _separate(ops, c, k, v, table, lens):
 
 
 def _fused(ops, c, k, v, table, lens):
-    return ops.decode_attention(c["qkv"], c["positions"], c["slots"], c["n_q"], c["n_kv"], c["hd"], c["q_norm"], c["k_norm"], c["eps"],
+    return ops.decode_attention_pairs(c["qkv"], c["positions"], c["slots"], c["n_q"], c["n_kv"], c["hd"], c["q_norm"], c["k_norm"], c["eps"],
                                 c["cos_sin"], k, v, 1, table, lens, c["hd"] ** -0.5)
 
 
