@@ -28,9 +28,6 @@ struct HeadArgs {
   const bf16_t* gate; int64_t gate_row; int group;
 };
 
-// (the hardware's conversion rounds to nearest even and keeps infinities and NaN, as f2bf does in eight instructions)
-__device__ __forceinline__ short round_bf16(float f) { return __builtin_bit_cast(short, static_cast<__bf16>(f)); }
-
 __device__ __forceinline__ float sigmoid(float z) { return 1.0f / (1.0f + expf(-z)); }
 
 // The tails of tokens t_first .. t_end - 1 and heads h0 .. h1 - 1: a thread takes one token's sines once for all of them, V
@@ -60,8 +57,8 @@ __device__ __forceinline__ void turn_tails(const HeadArgs& a, int K, int t_first
 #pragma unroll
         for (int i = 0; i < V; ++i) {
           const float uf = bf2f(static_cast<bf16_t>(u[i])), vf = bf2f(static_cast<bf16_t>(v[i]));
-          p[i] = round_bf16(uf * cs[i] - vf * sn[i]);
-          q[i] = round_bf16(vf * cs[i] + uf * sn[i]);
+          p[i] = static_cast<short>(f2bf(uf * cs[i] - vf * sn[i]));
+          q[i] = static_cast<short>(f2bf(vf * cs[i] + uf * sn[i]));
         }
         *reinterpret_cast<Bits*>(dst + V * j) = p;
         *reinterpret_cast<Bits*>(dst + a.half + V * j) = q;
@@ -170,10 +167,10 @@ __global__ __launch_bounds__(NT, KC <= 4 ? 4 : 2) void heads_kernel(HeadArgs a) 
           for (int i = 0; i < 8; ++i) g[i] = s;
         }
 #pragma unroll
-        for (int i = 0; i < 8; ++i) r[i] = round_bf16(bf2f(static_cast<bf16_t>(round_bf16(o[i]))) * g[i]);
+        for (int i = 0; i < 8; ++i) r[i] = static_cast<short>(f2bf(bf2f(f2bf(o[i])) * g[i]));
       } else {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) r[i] = round_bf16(o[i]);
+        for (int i = 0; i < 8; ++i) r[i] = static_cast<short>(f2bf(o[i]));
       }
       *reinterpret_cast<s16x8*>(a.out + static_cast<int64_t>(t) * a.o_row + h * a.o_head + n) = r;
     }
