@@ -1,5 +1,5 @@
 """Table-routed experts whose sum goes straight into the stream (csrc/kernels/seqmix_latent.hip, experts_post_norm_kernel; routes found by the position
-kernel in small steps) against the separate launches, which the other expert tests hold to float64: one fp32 rounding of the sums apart."""
+kernel in small steps) against the separate launches, one fp32 rounding of the sums apart, and against float64."""
 import pytest
 import torch
 
@@ -29,6 +29,20 @@ def test_against_separate_launches(T, E, top, W, ff, post, pre):
     want = ops.residual_post_norm(x1, ops.moe_experts(h, up, down, *ops.moe_table_route(tokens, table, top), "silu_gated"), norms[post], norms[pre], torch.bfloat16)
     got = ops.table_experts_post_norm(x2, h, up, down, tokens, table, top, "silu_gated", norms[post], norms[pre], torch.bfloat16)
     torch.testing.assert_close(x2, x1, rtol=2 ** -20, atol=2 ** -20)
+    # in float64: y rounded to bf16 behind hidden values rounded up to three times, 2^-9 each
+    u, d = up.double().view(E, ff // 16, 2, 16, W), down.double()
+    gate, lin = u[:, :, 0].reshape(E, ff, W), u[:, :, 1].reshape(E, ff, W)   # (rows in alternating groups of 16)
+    idx = ops.moe_table_route(tokens, table, top)[0].long()
+    y = torch.zeros(T, W, dtype=torch.float64, device=DEV)
+    for e in range(E):
+        rows = (idx == e).any(1).nonzero()[:, 0]
+        z = h[rows].double()
+        y[rows] += (torch.nn.functional.silu(z @ gate[e].T) * (z @ lin[e].T)) @ d[e].T / top
+    if post == "dyt":
+        step = torch.tanh(0.6 * y) * norms[post][2].double() + norms[post][3].double()
+    else:
+        step = y / torch.sqrt((y * y).mean(1, keepdim=True) + 1e-5) * norms[post][1].double()
+    assert (x2.double() - x.double() - step).norm() <= 2 ** -7 * step.norm()   # (both zero where no token has an expert)
     assert (got is None) == (pre is None)
     if pre is not None:
         torch.testing.assert_close(got.float(), want.float(), rtol=2 ** -7, atol=2 ** -7)
