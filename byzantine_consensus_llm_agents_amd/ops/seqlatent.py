@@ -163,8 +163,9 @@ def seqlatent_ops(lib, experts):
 
     def _own_heads(x3, w, out3, *more):
         """Whether csrc/kernels/seqmix_heads.hip takes the product as its operands lie: bf16, inputs of 32, 64, 128 or 256, columns in
-        sixteens, 16-byte aligned rows.  Elsewhere (fp32, other widths, transforms and traces) the vendor's batched product."""
-        return (x3.dtype == torch.bfloat16 and w.shape[1] in (32, 64, 128, 256) and w.shape[2] % 16 == 0 and w.shape[2] > 0 and w.shape[0] > 0
+        sixteens, 16-byte aligned rows, heads that its grid holds beside their tails.  Elsewhere (fp32, other widths, transforms and traces) the
+        vendor's batched product."""
+        return (x3.dtype == torch.bfloat16 and w.shape[1] in (32, 64, 128, 256) and w.shape[2] % 16 == 0 and w.shape[2] > 0 and 0 < w.shape[0] < 1 << 15
                 and all(t.is_cuda and t.get_device() == torch.cuda.current_device() and t.data_ptr() % 16 == 0 for t in (x3, w, out3))
                 and all(s % 8 == 0 for t in (x3, out3) for s in t.stride()[:2]) and not watched() and all(bare(t) for t in (x3, w, out3, *more)))
 

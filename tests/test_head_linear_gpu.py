@@ -65,3 +65,9 @@ def test_other_operands(K, N, dtype, off):
     tol = dict(rtol=2 ** -7, atol=2e-2) if dtype == torch.bfloat16 else dict(rtol=1e-4, atol=1e-4)
     torch.testing.assert_close(ops.head_linear(x, w).float().cpu(), want, **tol)
     torch.testing.assert_close(ops.head_linear_gated(x, w, gate).float().cpu(), want.view(T, H * N) * torch.sigmoid(gate.float().cpu()), **tol)
+
+
+def test_more_heads_than_the_grid_holds():
+    ops, _ = _ops()
+    x, w, _ = _data(2, 1 << 15, 32, 16, 0, 5)
+    torch.testing.assert_close(ops.head_linear(x.to(DEV), w.to(DEV)).float().cpu(), _exact(x, w), rtol=2 ** -8, atol=1e-5)
